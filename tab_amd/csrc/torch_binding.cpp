@@ -5,9 +5,12 @@
 // current HIP stream; all compute is in libtab_amd.so.
 #include <torch/extension.h>
 
+#include <ATen/hip/EmptyTensor.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <c10/hip/HIPCachingAllocator.h>
 
+#include <stdexcept>
 #include <vector>
 
 #include "../../include/tab_amd.h"
@@ -20,29 +23,67 @@
     CHECK_CONTIGUOUS(x)
 // The reference converts dtypes with .toType() on a temporary (TAB_GEMM.cu:279-280,341-347),
 // which dangles whenever a conversion really happens; exact dtypes are required instead.
-#define CHECK_DTYPE(x, t) TORCH_CHECK(x.scalar_type() == t, #x " must have dtype " #t)
+#define CHECK_DTYPE(x, t) \
+    TORCH_CHECK(x.scalar_type() == torch::t, #x " must have dtype ", dtype_name(torch::t), ", got ", dtype_name(x.scalar_type()))
 
 namespace {
 
-void check_status(int status)
+std::string dtype_name(torch::ScalarType t)
 {
-    TORCH_CHECK(status == TAB_OK, tab_status_string(status), ": ", tab_last_error());
+    switch (t) {
+    case torch::kFloat32: return "torch.float32";
+    case torch::kInt64: return "torch.int64";
+    case torch::kInt32: return "torch.int32";
+    default: return std::string("torch.") + c10::toString(t);
+    }
 }
 
-void *current_stream(const torch::Tensor &t)
+// A negative status of a C ABI call; Python sees tab_amd.TabError (a RuntimeError).
+struct StatusError : std::runtime_error {
+    using std::runtime_error::runtime_error;
+};
+
+void check_status(int status)
+{
+    if (status != TAB_OK) throw StatusError(std::string(tab_status_string(status)) + ": " + tab_last_error());
+}
+
+hipStream_t current_stream(const torch::Tensor &t)
 {
     return c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.device().index()).stream();
 }
 
+// Uninitialised device tensor, straight from the caching allocator: torch::empty's way through the dispatcher costs
+// 0.73 us a tensor, this 0.47, beside 2.3 us for a kernel launch.
+torch::Tensor device_empty(c10::IntArrayRef sizes, torch::ScalarType dtype, const torch::Tensor &like)
+{
+    return at::detail::empty_cuda(sizes, dtype, like.device(), c10::nullopt);
+}
+
+// Device scratch of one call (0.2 us, no tensor around it).  Given back when the call returns: the allocator hands the
+// block only to later work of the same stream.
+class Workspace {
+public:
+    Workspace(size_t bytes, hipStream_t stream)
+        : ptr_(c10::hip::HIPCachingAllocator::raw_alloc_with_stream(bytes, stream)) {}
+    ~Workspace() { c10::hip::HIPCachingAllocator::raw_delete(ptr_); }
+    Workspace(const Workspace &) = delete;
+    Workspace &operator=(const Workspace &) = delete;
+    void *get() const { return ptr_; }
+
+private:
+    void *ptr_;
+};
+
 }  // namespace
 
-std::vector<torch::Tensor> TAB_Quantize(torch::Tensor X, torch::Tensor thresholds, int bitwidth, int N,
+std::vector<torch::Tensor> TAB_Quantize(const torch::Tensor &X, const torch::Tensor &thresholds, int bitwidth, int N,
                                         int H, int W, int C)
 {
     CHECK_INPUT(X);
     CHECK_INPUT(thresholds);
-    CHECK_DTYPE(X, torch::kFloat32);
-    CHECK_DTYPE(thresholds, torch::kFloat32);
+    CHECK_DTYPE(X, kFloat32);
+    CHECK_DTYPE(thresholds, kFloat32);
     TORCH_CHECK(bitwidth == 1 || bitwidth == 2, "bitwidth must be 1 or 2, got ", bitwidth);
     TORCH_CHECK(N > 0 && H > 0 && W > 0 && C > 0, "N, H, W, C must be positive");
     TORCH_CHECK(X.numel() == (int64_t)N * H * W * C, "X has ", X.numel(), " elements, expected N*H*W*C = ",
@@ -51,8 +92,8 @@ std::vector<torch::Tensor> TAB_Quantize(torch::Tensor X, torch::Tensor threshold
     TORCH_CHECK(thresholds.device() == X.device(), "X and thresholds must be on the same device");
     const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(X.device());
     const int PC = tab_packed_channels(C);
-    auto QX = torch::empty({N, H, W, PC, bitwidth}, X.options().dtype(torch::kInt64));
-    auto BTN = torch::empty({N}, X.options().dtype(torch::kInt32));
+    auto QX = device_empty({N, H, W, PC, bitwidth}, torch::kInt64, X);
+    auto BTN = device_empty({N}, torch::kInt32, X);
     check_status(tab_quantize(X.data_ptr<float>(), thresholds.data_ptr<float>(), bitwidth, N, H, W, C,
                               QX.data_ptr<int64_t>(), BTN.data_ptr<int32_t>(), current_stream(X)));
     return {QX, BTN};
@@ -80,44 +121,58 @@ std::pair<int, int> check_conv(const torch::Tensor &QW, const torch::Tensor &btn
 
 }  // namespace
 
-torch::Tensor TAB_Conv2d(torch::Tensor X, torch::Tensor QW, torch::Tensor thresholds, torch::Tensor btn, int type,
-                         int padding1, int padding2, int stride1, int stride2, int N, int H, int W, int C, int KN,
-                         int KH, int KW)
+namespace {
+
+// Checks of the calls that take the fp32 activation; returns (OH, OW).
+std::pair<int, int> check_conv_from_floats(const torch::Tensor &X, const torch::Tensor &QW, const torch::Tensor &thresholds,
+                                           const torch::Tensor &btn, int type, int padding1, int padding2, int stride1, int stride2,
+                                           int N, int H, int W, int C, int KN, int KH, int KW)
 {
     CHECK_INPUT(X);
     CHECK_INPUT(QW);
     CHECK_INPUT(thresholds);
     CHECK_INPUT(btn);
-    CHECK_DTYPE(X, torch::kFloat32);
-    CHECK_DTYPE(QW, torch::kInt64);
-    CHECK_DTYPE(thresholds, torch::kFloat32);
-    CHECK_DTYPE(btn, torch::kInt32);
-    const auto [OH, OW] = check_conv(QW, btn, type, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW);
+    CHECK_DTYPE(X, kFloat32);
+    CHECK_DTYPE(QW, kInt64);
+    CHECK_DTYPE(thresholds, kFloat32);
+    CHECK_DTYPE(btn, kInt32);
+    const auto out = check_conv(QW, btn, type, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW);
     TORCH_CHECK(X.numel() == (int64_t)N * H * W * C, "X has ", X.numel(), " elements, expected N*H*W*C = ",
                 (int64_t)N * H * W * C);
     TORCH_CHECK(thresholds.numel() >= N, "thresholds has ", thresholds.numel(), " elements, expected at least N = ", N);
     TORCH_CHECK(QW.device() == X.device() && thresholds.device() == X.device() && btn.device() == X.device(),
                 "X, QW, thresholds and btn must be on the same device");
+    return out;
+}
+
+}  // namespace
+
+torch::Tensor TAB_Conv2d(const torch::Tensor &X, const torch::Tensor &QW, const torch::Tensor &thresholds, const torch::Tensor &btn,
+                         int type, int padding1, int padding2, int stride1, int stride2, int N, int H, int W, int C, int KN,
+                         int KH, int KW)
+{
+    const auto [OH, OW] = check_conv_from_floats(X, QW, thresholds, btn, type, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW);
     const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(X.device());
-    auto Y = torch::empty({N, KN, OH, OW}, X.options());
+    auto Y = device_empty({N, KN, OH, OW}, torch::kFloat32, X);
     const size_t ws_bytes = tab_conv2d_workspace_bytes(type, N, H, W, C);
-    auto ws = torch::empty({(int64_t)ws_bytes}, X.options().dtype(torch::kUInt8));
+    const hipStream_t stream = current_stream(X);
+    const Workspace ws(ws_bytes, stream);
     check_status(tab_conv2d(X.data_ptr<float>(), QW.data_ptr<int64_t>(), thresholds.data_ptr<float>(),
                             btn.data_ptr<int32_t>(), type, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH,
-                            KW, Y.data_ptr<float>(), ws.data_ptr(), ws_bytes, current_stream(X)));
+                            KW, Y.data_ptr<float>(), ws.get(), ws_bytes, stream));
     return Y;
 }
 
 // ---- the entry points beyond the reference's two: same conventions, one C ABI call each -----------------------
 
 // Quantize on an NCHW tensor, the layout and argument order of the reference's CPU binding (TAB_CPU.cpp:20-206, 621).
-std::vector<torch::Tensor> TAB_QuantizeNCHW(torch::Tensor X, torch::Tensor thresholds, int bitwidth, int N, int C,
+std::vector<torch::Tensor> TAB_QuantizeNCHW(const torch::Tensor &X, const torch::Tensor &thresholds, int bitwidth, int N, int C,
                                             int H, int W)
 {
     CHECK_INPUT(X);
     CHECK_INPUT(thresholds);
-    CHECK_DTYPE(X, torch::kFloat32);
-    CHECK_DTYPE(thresholds, torch::kFloat32);
+    CHECK_DTYPE(X, kFloat32);
+    CHECK_DTYPE(thresholds, kFloat32);
     TORCH_CHECK(bitwidth == 1 || bitwidth == 2, "bitwidth must be 1 or 2, got ", bitwidth);
     TORCH_CHECK(N > 0 && H > 0 && W > 0 && C > 0, "N, C, H, W must be positive");
     TORCH_CHECK(X.numel() == (int64_t)N * H * W * C, "X has ", X.numel(), " elements, expected N*C*H*W = ",
@@ -125,20 +180,43 @@ std::vector<torch::Tensor> TAB_QuantizeNCHW(torch::Tensor X, torch::Tensor thres
     TORCH_CHECK(thresholds.numel() >= N, "thresholds has ", thresholds.numel(), " elements, expected at least N = ", N);
     TORCH_CHECK(thresholds.device() == X.device(), "X and thresholds must be on the same device");
     const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(X.device());
-    auto QX = torch::empty({N, H, W, tab_packed_channels(C), bitwidth}, X.options().dtype(torch::kInt64));
-    auto BTN = torch::empty({N}, X.options().dtype(torch::kInt32));
+    auto QX = device_empty({N, H, W, tab_packed_channels(C), bitwidth}, torch::kInt64, X);
+    auto BTN = device_empty({N}, torch::kInt32, X);
     check_status(tab_quantize_nchw(X.data_ptr<float>(), thresholds.data_ptr<float>(), bitwidth, N, C, H, W,
                                    QX.data_ptr<int64_t>(), BTN.data_ptr<int32_t>(), current_stream(X)));
     return {QX, BTN};
 }
 
-// Packer of conv types 4 and 5 (layouts of DRFGEMM_baseline / RTNGEMM_baseline, TAB_CPU.cpp:332-383).
-torch::Tensor TAB_QuantizeFormat(torch::Tensor X, torch::Tensor thresholds, int type, int N, int H, int W, int C)
+// The packed activation alone, NHWC or NCHW: without the BTN vector, which nobody reads of an activation.
+torch::Tensor TAB_QuantizeActivation(const torch::Tensor &X, const torch::Tensor &thresholds, int bitwidth, int N, int H, int W,
+                                     int C, bool nchw)
 {
     CHECK_INPUT(X);
     CHECK_INPUT(thresholds);
-    CHECK_DTYPE(X, torch::kFloat32);
-    CHECK_DTYPE(thresholds, torch::kFloat32);
+    CHECK_DTYPE(X, kFloat32);
+    CHECK_DTYPE(thresholds, kFloat32);
+    TORCH_CHECK(bitwidth == 1 || bitwidth == 2, "bitwidth must be 1 or 2, got ", bitwidth);
+    TORCH_CHECK(N > 0 && H > 0 && W > 0 && C > 0, "N, H, W, C must be positive");
+    TORCH_CHECK(X.numel() == (int64_t)N * H * W * C, "X has ", X.numel(), " elements, expected N*H*W*C = ",
+                (int64_t)N * H * W * C);
+    TORCH_CHECK(thresholds.numel() >= N, "thresholds has ", thresholds.numel(), " elements, expected at least N = ", N);
+    TORCH_CHECK(thresholds.device() == X.device(), "X and thresholds must be on the same device");
+    const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(X.device());
+    auto QX = device_empty({N, H, W, tab_packed_channels(C), bitwidth}, torch::kInt64, X);
+    const float *x = X.data_ptr<float>(), *ths = thresholds.data_ptr<float>();
+    int64_t *q = QX.data_ptr<int64_t>();
+    check_status(nchw ? tab_quantize_nchw(x, ths, bitwidth, N, C, H, W, q, nullptr, current_stream(X))
+                      : tab_quantize(x, ths, bitwidth, N, H, W, C, q, nullptr, current_stream(X)));
+    return QX;
+}
+
+// Packer of conv types 4 and 5 (layouts of DRFGEMM_baseline / RTNGEMM_baseline, TAB_CPU.cpp:332-383).
+torch::Tensor TAB_QuantizeFormat(const torch::Tensor &X, const torch::Tensor &thresholds, int type, int N, int H, int W, int C)
+{
+    CHECK_INPUT(X);
+    CHECK_INPUT(thresholds);
+    CHECK_DTYPE(X, kFloat32);
+    CHECK_DTYPE(thresholds, kFloat32);
     TORCH_CHECK(type == TAB_DRF || type == TAB_RTN, "type must be 4 (DRF) or 5 (RTN), got ", type);
     TORCH_CHECK(N > 0 && H > 0 && W > 0 && C > 0, "N, H, W, C must be positive");
     TORCH_CHECK(X.numel() == (int64_t)N * H * W * C, "X has ", X.numel(), " elements, expected N*H*W*C = ",
@@ -146,63 +224,80 @@ torch::Tensor TAB_QuantizeFormat(torch::Tensor X, torch::Tensor thresholds, int 
     TORCH_CHECK(thresholds.numel() >= N, "thresholds has ", thresholds.numel(), " elements, expected at least N = ", N);
     TORCH_CHECK(thresholds.device() == X.device(), "X and thresholds must be on the same device");
     const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(X.device());
-    auto QX = type == TAB_DRF ? torch::empty({N, H, W, tab_packed_channels(C), 2}, X.options().dtype(torch::kInt64))
-                              : torch::empty({N, H, W, (C + 31) / 32}, X.options().dtype(torch::kInt64));
+    auto QX = type == TAB_DRF ? device_empty({N, H, W, tab_packed_channels(C), 2}, torch::kInt64, X)
+                              : device_empty({N, H, W, (C + 31) / 32}, torch::kInt64, X);
     check_status(tab_quantize_format(X.data_ptr<float>(), thresholds.data_ptr<float>(), type, N, H, W, C,
                                      QX.data_ptr<int64_t>(), current_stream(X)));
     return QX;
 }
 
 // thresholds[n] = scale * mean|X[n]|, the rule README.md:45 leaves to the caller.
-torch::Tensor TAB_Threshold(torch::Tensor X, int N, double scale)
+torch::Tensor TAB_Threshold(const torch::Tensor &X, int N, double scale)
 {
     CHECK_INPUT(X);
-    CHECK_DTYPE(X, torch::kFloat32);
+    CHECK_DTYPE(X, kFloat32);
     TORCH_CHECK(N > 0 && X.numel() > 0 && X.numel() % N == 0, "X has ", X.numel(), " elements, not a positive multiple of N = ", N);
     const long per_item = (long)(X.numel() / N);
     const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(X.device());
-    auto ths = torch::empty({N}, X.options());
+    auto ths = device_empty({N}, torch::kFloat32, X);
     const size_t ws_bytes = tab_threshold_workspace_bytes(N, per_item);
-    auto ws = torch::empty({(int64_t)ws_bytes}, X.options().dtype(torch::kUInt8));
-    check_status(tab_threshold(X.data_ptr<float>(), N, per_item, (float)scale, ths.data_ptr<float>(), ws.data_ptr(), ws_bytes,
-                               current_stream(X)));
+    const hipStream_t stream = current_stream(X);
+    const Workspace ws(ws_bytes, stream);
+    check_status(tab_threshold(X.data_ptr<float>(), N, per_item, (float)scale, ths.data_ptr<float>(), ws.get(), ws_bytes, stream));
     return ths;
 }
 
+// Conv2d with the packed activation in the library's built-in scratch; with `out` given nothing is allocated.
+torch::Tensor TAB_Conv2dStatic(const torch::Tensor &X, const torch::Tensor &QW, const torch::Tensor &thresholds,
+                               const torch::Tensor &btn, int type, int padding1, int padding2, int stride1, int stride2, int N,
+                               int H, int W, int C, int KN, int KH, int KW, const c10::optional<torch::Tensor> &given)
+{
+    const auto [OH, OW] = check_conv_from_floats(X, QW, thresholds, btn, type, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW);
+    const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(X.device());
+    const torch::Tensor out = given ? *given : device_empty({N, KN, OH, OW}, torch::kFloat32, X);
+    CHECK_INPUT(out);
+    CHECK_DTYPE(out, kFloat32);
+    TORCH_CHECK(out.numel() == (int64_t)N * KN * OH * OW, "out has ", out.numel(), " elements, expected ", (int64_t)N * KN * OH * OW);
+    check_status(tab_conv2d_static(X.data_ptr<float>(), QW.data_ptr<int64_t>(), thresholds.data_ptr<float>(), btn.data_ptr<int32_t>(),
+                                   type, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, out.data_ptr<float>(),
+                                   current_stream(X)));
+    return out;
+}
+
 // Conv2d on an activation already packed by Quantize / QuantizeFormat (TAB_GEMM.cu:447-509 only).
-torch::Tensor TAB_Conv2dPacked(torch::Tensor QX, torch::Tensor QW, torch::Tensor btn, int type, int padding1, int padding2,
+torch::Tensor TAB_Conv2dPacked(const torch::Tensor &QX, const torch::Tensor &QW, const torch::Tensor &btn, int type, int padding1, int padding2,
                                int stride1, int stride2, int N, int H, int W, int C, int KN, int KH, int KW)
 {
     CHECK_INPUT(QX);
     CHECK_INPUT(QW);
     CHECK_INPUT(btn);
-    CHECK_DTYPE(QX, torch::kInt64);
-    CHECK_DTYPE(QW, torch::kInt64);
-    CHECK_DTYPE(btn, torch::kInt32);
+    CHECK_DTYPE(QX, kInt64);
+    CHECK_DTYPE(QW, kInt64);
+    CHECK_DTYPE(btn, kInt32);
     const auto [OH, OW] = check_conv(QW, btn, type, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW);
     const int awords = tab_operand_words(type, 0, C);
     TORCH_CHECK(QX.numel() == (int64_t)N * H * W * awords, "QX has ", QX.numel(), " words, type ", type, " expects N*H*W*", awords);
     TORCH_CHECK(QW.device() == QX.device() && btn.device() == QX.device(), "QX, QW and btn must be on the same device");
     const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(QX.device());
-    auto Y = torch::empty({N, KN, OH, OW}, QX.options().dtype(torch::kFloat32));
+    auto Y = device_empty({N, KN, OH, OW}, torch::kFloat32, QX);
     check_status(tab_conv2d_packed(QX.data_ptr<int64_t>(), QW.data_ptr<int64_t>(), btn.data_ptr<int32_t>(), type, padding1,
                                    padding2, stride1, stride2, N, H, W, C, KN, KH, KW, Y.data_ptr<float>(), current_stream(QX)));
     return Y;
 }
 
 // Conv2dPacked with the output thresholded and packed in the epilogue: the next layer's activation, no fp32 Y.
-torch::Tensor TAB_Conv2dPackedOut(torch::Tensor QX, torch::Tensor QW, torch::Tensor btn, int type, int padding1, int padding2,
+torch::Tensor TAB_Conv2dPackedOut(const torch::Tensor &QX, const torch::Tensor &QW, const torch::Tensor &btn, int type, int padding1, int padding2,
                                   int stride1, int stride2, int N, int H, int W, int C, int KN, int KH, int KW,
-                                  torch::Tensor out_thresholds, int out_bitwidth)
+                                  const torch::Tensor &out_thresholds, int out_bitwidth)
 {
     CHECK_INPUT(QX);
     CHECK_INPUT(QW);
     CHECK_INPUT(btn);
     CHECK_INPUT(out_thresholds);
-    CHECK_DTYPE(QX, torch::kInt64);
-    CHECK_DTYPE(QW, torch::kInt64);
-    CHECK_DTYPE(btn, torch::kInt32);
-    CHECK_DTYPE(out_thresholds, torch::kFloat32);
+    CHECK_DTYPE(QX, kInt64);
+    CHECK_DTYPE(QW, kInt64);
+    CHECK_DTYPE(btn, kInt32);
+    CHECK_DTYPE(out_thresholds, kFloat32);
     TORCH_CHECK(out_bitwidth == 1 || out_bitwidth == 2, "out_bitwidth must be 1 or 2, got ", out_bitwidth);
     const auto [OH, OW] = check_conv(QW, btn, type, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW);
     const int awords = tab_operand_words(type, 0, C);
@@ -211,7 +306,7 @@ torch::Tensor TAB_Conv2dPackedOut(torch::Tensor QX, torch::Tensor QW, torch::Ten
     TORCH_CHECK(QW.device() == QX.device() && btn.device() == QX.device() && out_thresholds.device() == QX.device(),
                 "QX, QW, btn and out_thresholds must be on the same device");
     const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(QX.device());
-    auto QY = torch::empty({N, OH, OW, tab_packed_channels(KN), out_bitwidth}, QX.options());
+    auto QY = device_empty({N, OH, OW, tab_packed_channels(KN), out_bitwidth}, torch::kInt64, QX);
     check_status(tab_conv2d_packed_out(QX.data_ptr<int64_t>(), QW.data_ptr<int64_t>(), btn.data_ptr<int32_t>(), type, padding1,
                                        padding2, stride1, stride2, N, H, W, C, KN, KH, KW, out_thresholds.data_ptr<float>(),
                                        out_bitwidth, QY.data_ptr<int64_t>(), current_stream(QX)));
@@ -220,6 +315,13 @@ torch::Tensor TAB_Conv2dPackedOut(torch::Tensor QX, torch::Tensor QW, torch::Ten
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
 {
+    pybind11::register_exception_translator([](std::exception_ptr p) {
+        try {
+            if (p) std::rethrow_exception(p);
+        } catch (const StatusError &e) {
+            PyErr_SetString(pybind11::module_::import("tab_amd._capi").attr("TabError").ptr(), e.what());
+        }
+    });
     m.def("Quantize", &TAB_Quantize, "Ternarization or binarization of NHWC fp32 data, packed 64 channels per int64");
     m.def("Conv2d", &TAB_Conv2d, "Conv2d of all TAB types (0 TNN, 1 TBN, 2 BTN, 3 BNN; 4 DRF and 5 RTN of the CPU path)");
     m.def("TAB_Quantize", &TAB_Quantize, "alias of Quantize");
@@ -228,6 +330,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     m.def("QuantizeFormat", &TAB_QuantizeFormat, "Packer of conv types 4 (DRF) and 5 (RTN)");
     m.def("Threshold", &TAB_Threshold, "thresholds[n] = scale * mean|X[n]|", pybind11::arg("X"), pybind11::arg("N"),
           pybind11::arg("scale") = 0.7);
+    m.def("QuantizeActivation", &TAB_QuantizeActivation, "QX of Quantize or QuantizeNCHW without the BTN vector");
+    m.def("Conv2dStatic", &TAB_Conv2dStatic, "Conv2d with the packed activation in the library's built-in scratch");
     m.def("Conv2dPacked", &TAB_Conv2dPacked, "Conv2d on an already packed activation");
     m.def("Conv2dPackedOut", &TAB_Conv2dPackedOut, "Conv2dPacked with the output quantized and packed in the epilogue");
 }
