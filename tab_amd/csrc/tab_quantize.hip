@@ -24,6 +24,14 @@ __device__ __forceinline__ int wave_sum(int v)
     return v;
 }
 
+// The counts of items 0 .. items - 1 start at zero (for one plane they stay there, TAB_GEMM.cu:283): every quantizer
+// writes them on the side, since a launch of its own for them costs 1.2-4.8 us before the quantizer.  Null: none wanted.
+__device__ __forceinline__ void zero_counts(int32_t *btn, long items)
+{
+    if (btn == nullptr) return;
+    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < items; i += (long)gridDim.x * blockDim.x) btn[i] = 0;
+}
+
 // Fast path, C % 64 == 0 and X 16-byte aligned.
 // Lane layout: a 16-lane DPP row reads one 64-channel row as 16 float4 (256 B contiguous),
 // a wave reads 4 consecutive rows per load (1 KB contiguous) and keeps kLoadsPerLane loads
@@ -34,8 +42,9 @@ template <int BITS, int LOADS = kLoadsPerLane>
 __global__ __launch_bounds__(kThreads) void quantize_rows64(const floatx4 *__restrict__ x,
                                                             const float *__restrict__ ths,
                                                             uint32_t *__restrict__ q, long rows,
-                                                            long rows_per_item, Div32 div_item)
+                                                            long rows_per_item, Div32 div_item, int32_t *btn, long items)
 {
+    zero_counts(btn, items);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // scalar: so are row0 and the item test below
     const int sub = lane >> 4;  // which of the 4 rows of a load
@@ -148,8 +157,9 @@ __device__ __forceinline__ uint32_t or_reduce_group(uint32_t v)
 template <int BITS, int LP>
 __global__ __launch_bounds__(kThreads) void quantize_groups(const float *__restrict__ x, const float *__restrict__ ths,
                                                             uint32_t *__restrict__ q, long rows, long pixels_per_item,
-                                                            int C, int PC)
+                                                            int C, int PC, int32_t *btn, long items)
 {
+    zero_counts(btn, items);
     constexpr int GROUPS = 64 / LP;  // rows per wave-wide load
     constexpr int U = 8;
     const int lane = threadIdx.x & 63;
@@ -226,8 +236,9 @@ template <int BITS>
 __global__ __launch_bounds__(kThreads) void quantize_ballot(const float *__restrict__ x,
                                                             const float *__restrict__ ths,
                                                             uint64_t *__restrict__ q, long pixels,
-                                                            long pixels_per_item, int C, int PC)
+                                                            long pixels_per_item, int C, int PC, int32_t *btn, long items)
 {
+    zero_counts(btn, items);
     const int lane = threadIdx.x & 63;
     const long nwaves = (long)gridDim.x * kWavesPerBlock;
     const long units = pixels * PC;
@@ -308,8 +319,9 @@ __global__ __launch_bounds__(kThreads) void quantize_ballot_format(const float *
 // words of the same pixels run side by side, so their 8- or 16-byte stores meet in L2 as whole lines.
 template <int BITS, int VEC>
 __global__ __launch_bounds__(kThreads) void quantize_nchw(const float *__restrict__ x, const float *__restrict__ ths,
-                                                          uint64_t *__restrict__ q, int N, int C, long HW, int PC)
+                                                          uint64_t *__restrict__ q, int N, int C, long HW, int PC, int32_t *btn)
 {
+    zero_counts(btn, N);
     typedef float vec_t __attribute__((ext_vector_type(VEC)));
     const int pc = blockIdx.x % PC;
     const long g0 = ((long)(blockIdx.x / PC) * kThreads + threadIdx.x) * VEC;  // first pixel, counted through all images
@@ -380,8 +392,9 @@ __global__ __launch_bounds__(kThreads) void quantize_nchw(const float *__restric
 // in WPP / 2 rounds of 64 / rounds lanes each.  grid = ceil(N*H*W / 256) * (PC / U), the word group fastest.
 template <int BITS, int U>
 __global__ __launch_bounds__(64) void quantize_nchw_gather(const float *__restrict__ x, const float *__restrict__ ths,
-                                                                 uint64_t *__restrict__ q, int N, int C, long HW, int PC)
+                                                                 uint64_t *__restrict__ q, int N, int C, long HW, int PC, int32_t *btn)
 {
+    zero_counts(btn, N);
     constexpr int VEC = 4, kInFlight = 8;
     constexpr int WPP = U * BITS;      // words a thread packs per pixel, contiguous in q
     constexpr int ROUNDS = WPP / 2;    // 64 / ROUNDS lanes x 4 pixels x WPP words = 512 words a round
@@ -486,22 +499,22 @@ __global__ __launch_bounds__(64) void quantize_nchw_gather(const float *__restri
     }
 }
 
-__global__ void fill_zero_i32(int32_t *p, long n)
-{
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0;
-}
-
 // btn[n] = sum over item n of popcount(nonzero-plane word) (BTN_Weight, TAB_GEMM.cu:150-160,
 // for every n).  q is the ternary output [items][words_per_item][2]; one workgroup per
 // (item, split) reads its words as 16-byte (sign, nonzero) pairs.  With one split the result
-// is stored directly; with several (very long items) the partial sums are added atomically
-// into btn, which the caller zeroed beforehand.
-__global__ __launch_bounds__(kThreads) void btn_popcount(const ulonglong2 *__restrict__ q,
-                                                         int32_t *__restrict__ btn,
-                                                         long words_per_item, int splits)
+// is stored directly; with several the partial sums are added atomically into btn, which the
+// quantizer zeroed.
+// Bound by reading the packed output back (from the caches, it was just written): four loads in flight a lane and a
+// full CU of waves, in workgroups of 1024 because every workgroup of a split item is one more atomic on the few cache
+// lines of btn.
+constexpr int kCountThreads = 1024;
+constexpr int kCountLoads = 4;
+
+__global__ __launch_bounds__(kCountThreads) void btn_popcount(const ulonglong2 *__restrict__ q,
+                                                              int32_t *__restrict__ btn,
+                                                              long words_per_item, int splits)
 {
-    __shared__ int partial[kWavesPerBlock];
+    __shared__ int partial[kCountThreads / 64];
     const long item = blockIdx.x / splits;
     const int split = blockIdx.x % splits;
     const long per_split = (words_per_item + splits - 1) / splits;
@@ -510,14 +523,22 @@ __global__ __launch_bounds__(kThreads) void btn_popcount(const ulonglong2 *__res
     if (w1 > words_per_item) w1 = words_per_item;
     const ulonglong2 *src = q + item * words_per_item;
     int count = 0;
-    for (long w = w0 + threadIdx.x; w < w1; w += kThreads) count += __popcll(src[w].y);
+    long w = w0 + threadIdx.x;
+    const long step = blockDim.x;
+    for (; w + (kCountLoads - 1) * step < w1; w += kCountLoads * step) {
+        ulonglong2 v[kCountLoads];
+#pragma unroll
+        for (int u = 0; u < kCountLoads; u++) v[u] = src[w + u * step];
+#pragma unroll
+        for (int u = 0; u < kCountLoads; u++) count += __popcll(v[u].y);
+    }
+    for (; w < w1; w += step) count += __popcll(src[w].y);
     count = wave_sum(count);
     if ((threadIdx.x & 63) == 0) partial[threadIdx.x >> 6] = count;
     __syncthreads();
     if (threadIdx.x == 0) {
         int total = 0;
-#pragma unroll
-        for (int w = 0; w < kWavesPerBlock; w++) total += partial[w];
+        for (int i = 0; i < (int)(blockDim.x >> 6); i++) total += partial[i];
         if (splits == 1)
             btn[item] = total;
         else if (total)
@@ -595,28 +616,45 @@ hipError_t launch_threshold(const float *x, long items, long per_item, float sca
     return hipGetLastError();
 }
 
+// Workgroups per item of btn_popcount: enough to fill the chip twice over, none with less than a load a thread.
+int count_splits(long items, long words_per_item)
+{
+    int splits = 1;
+    while (splits < 64 && items * splits < 512 && words_per_item / (splits * 2) >= kCountThreads) splits *= 2;
+    return splits;
+}
+
+void launch_btn_popcount(const uint64_t *qx, int32_t *btn, long items, long words_per_item, int splits, hipStream_t stream)
+{
+    // an item of few words (a filter) takes as many whole waves as it has words for
+    const long per_split = (words_per_item + splits - 1) / splits;
+    const int threads = per_split >= kCountThreads ? kCountThreads : (int)((per_split + 63) / 64) * 64;
+    btn_popcount<<<dim3((unsigned)(items * splits)), dim3(threads), 0, stream>>>(reinterpret_cast<const ulonglong2 *>(qx), btn,
+                                                                               words_per_item, splits);
+}
+
 template <int LP>
 void launch_quantize_groups_of(const float *x, const float *ths, int bitwidth, long rows, long pixels_per_item, int C, int PC,
-                               uint32_t *q, hipStream_t stream)
+                               uint32_t *q, int32_t *btn, long items, hipStream_t stream)
 {
     const long per_block = (long)kWavesPerBlock * (64 / LP) * 8;
     const dim3 grid((unsigned)((rows + per_block - 1) / per_block)), block(kThreads);
     if (bitwidth == 2)
-        quantize_groups<2, LP><<<grid, block, 0, stream>>>(x, ths, q, rows, pixels_per_item, C, PC);
+        quantize_groups<2, LP><<<grid, block, 0, stream>>>(x, ths, q, rows, pixels_per_item, C, PC, btn, items);
     else
-        quantize_groups<1, LP><<<grid, block, 0, stream>>>(x, ths, q, rows, pixels_per_item, C, PC);
+        quantize_groups<1, LP><<<grid, block, 0, stream>>>(x, ths, q, rows, pixels_per_item, C, PC, btn, items);
 }
 
 // The general-path kernel with the smallest group of lanes whose 4 channels a lane cover the widest word.
 void launch_quantize_groups(const float *x, const float *ths, int bitwidth, long rows, long pixels_per_item, int C, int PC,
-                            uint32_t *q, hipStream_t stream)
+                            uint32_t *q, int32_t *btn, long items, hipStream_t stream)
 {
     const int widest = C < kWordBits ? C : kWordBits;
-    if (widest <= 4) launch_quantize_groups_of<1>(x, ths, bitwidth, rows, pixels_per_item, C, PC, q, stream);
-    else if (widest <= 8) launch_quantize_groups_of<2>(x, ths, bitwidth, rows, pixels_per_item, C, PC, q, stream);
-    else if (widest <= 16) launch_quantize_groups_of<4>(x, ths, bitwidth, rows, pixels_per_item, C, PC, q, stream);
-    else if (widest <= 32) launch_quantize_groups_of<8>(x, ths, bitwidth, rows, pixels_per_item, C, PC, q, stream);
-    else launch_quantize_groups_of<16>(x, ths, bitwidth, rows, pixels_per_item, C, PC, q, stream);
+    if (widest <= 4) launch_quantize_groups_of<1>(x, ths, bitwidth, rows, pixels_per_item, C, PC, q, btn, items, stream);
+    else if (widest <= 8) launch_quantize_groups_of<2>(x, ths, bitwidth, rows, pixels_per_item, C, PC, q, btn, items, stream);
+    else if (widest <= 16) launch_quantize_groups_of<4>(x, ths, bitwidth, rows, pixels_per_item, C, PC, q, btn, items, stream);
+    else if (widest <= 32) launch_quantize_groups_of<8>(x, ths, bitwidth, rows, pixels_per_item, C, PC, q, btn, items, stream);
+    else launch_quantize_groups_of<16>(x, ths, bitwidth, rows, pixels_per_item, C, PC, q, btn, items, stream);
 }
 
 // x: fp32 [items][pixels_per_item][C]; qx: [items*pixels_per_item][PC][bitwidth];
@@ -627,16 +665,9 @@ hipError_t launch_quantize(const float *x, const float *ths, int bitwidth, long 
     const int PC = (C + kWordBits - 1) / kWordBits;
     const long pixels = items * pixels_per_item;
     const long words_per_item = pixels_per_item * PC;
-    // very long items are split over several workgroups for the btn pass
-    int splits = 1;
-    if (btn && bitwidth == 2 && items < 512) {
-        while (splits < 64 && items * splits < 512 && words_per_item / (splits * 2) >= 2 * kThreads) splits *= 2;
-    }
-    if (btn && (bitwidth != 2 || splits > 1)) {
-        // zeros for 1-bit (TAB_GEMM.cu:283); a kernel rather than a memset node so that the
-        // call can be captured in a graph
-        fill_zero_i32<<<dim3((unsigned)((items + 255) / 256)), dim3(256), 0, stream>>>(btn, items);
-    }
+    const int splits = btn && bitwidth == 2 ? count_splits(items, words_per_item) : 1;
+    // counts that are not stored whole by btn_popcount start at zero
+    int32_t *zeroed = btn && (bitwidth != 2 || splits > 1) ? btn : nullptr;
     const bool fast = (C % kWordBits == 0) && ((uintptr_t)x % 16 == 0);
     if (fast) {
         const long rows = pixels * PC;
@@ -650,32 +681,29 @@ hipError_t launch_quantize(const float *x, const float *ths, int bitwidth, long 
             // (3.1 MB of fp32: 5.5 -> 4.2 us)
             const dim3 grid((unsigned)((rows + 8 * kWavesPerBlock - 1) / (8 * kWavesPerBlock)));
             if (bitwidth == 2)
-                quantize_rows64<2, 2><<<grid, block, 0, stream>>>(x4, ths, q32, rows, words_per_item, div_item);
+                quantize_rows64<2, 2><<<grid, block, 0, stream>>>(x4, ths, q32, rows, words_per_item, div_item, zeroed, items);
             else
-                quantize_rows64<1, 2><<<grid, block, 0, stream>>>(x4, ths, q32, rows, words_per_item, div_item);
+                quantize_rows64<1, 2><<<grid, block, 0, stream>>>(x4, ths, q32, rows, words_per_item, div_item, zeroed, items);
         } else {
             const dim3 grid((unsigned)blocks);
             if (bitwidth == 2)
-                quantize_rows64<2><<<grid, block, 0, stream>>>(x4, ths, q32, rows, words_per_item, div_item);
+                quantize_rows64<2><<<grid, block, 0, stream>>>(x4, ths, q32, rows, words_per_item, div_item, zeroed, items);
             else
-                quantize_rows64<1><<<grid, block, 0, stream>>>(x4, ths, q32, rows, words_per_item, div_item);
+                quantize_rows64<1><<<grid, block, 0, stream>>>(x4, ths, q32, rows, words_per_item, div_item, zeroed, items);
         }
     } else if (pixels * PC < 0x7fffffffL) {
-        launch_quantize_groups(x, ths, bitwidth, pixels * PC, pixels_per_item, C, PC, reinterpret_cast<uint32_t *>(qx), stream);
+        launch_quantize_groups(x, ths, bitwidth, pixels * PC, pixels_per_item, C, PC, reinterpret_cast<uint32_t *>(qx), zeroed, items, stream);
     } else {
         const long units = pixels * PC;
         long blocks = (units + kWavesPerBlock - 1) / kWavesPerBlock;
         if (blocks > 256 * 32) blocks = 256 * 32;  // grid-stride beyond 32 blocks per CU
         const dim3 grid((unsigned)blocks), block(kThreads);
         if (bitwidth == 2)
-            quantize_ballot<2><<<grid, block, 0, stream>>>(x, ths, qx, pixels, pixels_per_item, C, PC);
+            quantize_ballot<2><<<grid, block, 0, stream>>>(x, ths, qx, pixels, pixels_per_item, C, PC, zeroed, items);
         else
-            quantize_ballot<1><<<grid, block, 0, stream>>>(x, ths, qx, pixels, pixels_per_item, C, PC);
+            quantize_ballot<1><<<grid, block, 0, stream>>>(x, ths, qx, pixels, pixels_per_item, C, PC, zeroed, items);
     }
-    if (btn && bitwidth == 2) {
-        btn_popcount<<<dim3((unsigned)(items * splits)), dim3(kThreads), 0, stream>>>(
-            reinterpret_cast<const ulonglong2 *>(qx), btn, words_per_item, splits);
-    }
+    if (btn && bitwidth == 2) launch_btn_popcount(qx, btn, items, words_per_item, splits, stream);
     return hipGetLastError();
 }
 
@@ -684,12 +712,8 @@ hipError_t launch_quantize_nchw(const float *x, const float *ths, int bitwidth, 
 {
     const int PC = (C + kWordBits - 1) / kWordBits;
     const long words_per_item = HW * PC;
-    int splits = 1;
-    if (btn && bitwidth == 2 && N < 512) {
-        while (splits < 64 && (long)N * splits < 512 && words_per_item / (splits * 2) >= 2 * kThreads) splits *= 2;
-    }
-    if (btn && (bitwidth != 2 || splits > 1))
-        fill_zero_i32<<<dim3((unsigned)((N + 255) / 256)), dim3(256), 0, stream>>>(btn, N);
+    const int splits = btn && bitwidth == 2 ? count_splits(N, words_per_item) : 1;
+    int32_t *zeroed = btn && (bitwidth != 2 || splits > 1) ? btn : nullptr;
     // four pixels per thread when the planes allow aligned 16-byte loads and the launch still fills the chip
     const long pixels = (long)N * HW;
     const bool vec4 = HW % 4 == 0 && (uintptr_t)x % 16 == 0 && ((pixels + 4 * kThreads - 1) / (4 * kThreads)) * PC >= 2048;
@@ -703,21 +727,18 @@ hipError_t launch_quantize_nchw(const float *x, const float *ths, int bitwidth, 
     if (gather_waves > 0x7fffffffL) return hipErrorInvalidValue;
     if (HW % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)qx % 16 == 0 && unit > 1 && gather_waves >= 1024) {
         const dim3 ggrid((unsigned)gather_waves), gblock(64);
-        if (unit == 4 && bitwidth == 2) quantize_nchw_gather<2, 4><<<ggrid, gblock, 0, stream>>>(x, ths, qx, N, C, HW, PC);
-        else if (unit == 4) quantize_nchw_gather<1, 4><<<ggrid, gblock, 0, stream>>>(x, ths, qx, N, C, HW, PC);
-        else if (bitwidth == 2) quantize_nchw_gather<2, 2><<<ggrid, gblock, 0, stream>>>(x, ths, qx, N, C, HW, PC);
-        else quantize_nchw_gather<1, 2><<<ggrid, gblock, 0, stream>>>(x, ths, qx, N, C, HW, PC);
+        if (unit == 4 && bitwidth == 2) quantize_nchw_gather<2, 4><<<ggrid, gblock, 0, stream>>>(x, ths, qx, N, C, HW, PC, zeroed);
+        else if (unit == 4) quantize_nchw_gather<1, 4><<<ggrid, gblock, 0, stream>>>(x, ths, qx, N, C, HW, PC, zeroed);
+        else if (bitwidth == 2) quantize_nchw_gather<2, 2><<<ggrid, gblock, 0, stream>>>(x, ths, qx, N, C, HW, PC, zeroed);
+        else quantize_nchw_gather<1, 2><<<ggrid, gblock, 0, stream>>>(x, ths, qx, N, C, HW, PC, zeroed);
     } else if (vec4) {
-        if (bitwidth == 2) quantize_nchw<2, 4><<<grid, block, 0, stream>>>(x, ths, qx, N, C, HW, PC);
-        else quantize_nchw<1, 4><<<grid, block, 0, stream>>>(x, ths, qx, N, C, HW, PC);
+        if (bitwidth == 2) quantize_nchw<2, 4><<<grid, block, 0, stream>>>(x, ths, qx, N, C, HW, PC, zeroed);
+        else quantize_nchw<1, 4><<<grid, block, 0, stream>>>(x, ths, qx, N, C, HW, PC, zeroed);
     } else {
-        if (bitwidth == 2) quantize_nchw<2, 1><<<grid, block, 0, stream>>>(x, ths, qx, N, C, HW, PC);
-        else quantize_nchw<1, 1><<<grid, block, 0, stream>>>(x, ths, qx, N, C, HW, PC);
+        if (bitwidth == 2) quantize_nchw<2, 1><<<grid, block, 0, stream>>>(x, ths, qx, N, C, HW, PC, zeroed);
+        else quantize_nchw<1, 1><<<grid, block, 0, stream>>>(x, ths, qx, N, C, HW, PC, zeroed);
     }
-    if (btn && bitwidth == 2) {
-        btn_popcount<<<dim3((unsigned)(N * splits)), dim3(kThreads), 0, stream>>>(reinterpret_cast<const ulonglong2 *>(qx), btn,
-                                                                                 words_per_item, splits);
-    }
+    if (btn && bitwidth == 2) launch_btn_popcount(qx, btn, N, words_per_item, splits, stream);
     return hipGetLastError();
 }
 
@@ -739,13 +760,13 @@ hipError_t launch_quantize_format(const float *x, const float *ths, int format, 
         if (blocks <= kSmallLaunchBlocks) {  // too small to fill the chip: 32 rows per workgroup, as in launch_quantize
             const dim3 small((unsigned)((rows + 8 * kWavesPerBlock - 1) / (8 * kWavesPerBlock)));
             if (format == 4)
-                quantize_rows64<4, 2><<<small, block, 0, stream>>>(x4, ths, q32, rows, rows_per_item, div_item);
+                quantize_rows64<4, 2><<<small, block, 0, stream>>>(x4, ths, q32, rows, rows_per_item, div_item, nullptr, 0);
             else
-                quantize_rows64<5, 2><<<small, block, 0, stream>>>(x4, ths, q32, rows, rows_per_item, div_item);
+                quantize_rows64<5, 2><<<small, block, 0, stream>>>(x4, ths, q32, rows, rows_per_item, div_item, nullptr, 0);
         } else if (format == 4) {
-            quantize_rows64<4><<<grid, block, 0, stream>>>(x4, ths, q32, rows, rows_per_item, div_item);
+            quantize_rows64<4><<<grid, block, 0, stream>>>(x4, ths, q32, rows, rows_per_item, div_item, nullptr, 0);
         } else {
-            quantize_rows64<5><<<grid, block, 0, stream>>>(x4, ths, q32, rows, rows_per_item, div_item);
+            quantize_rows64<5><<<grid, block, 0, stream>>>(x4, ths, q32, rows, rows_per_item, div_item, nullptr, 0);
         }
         return hipGetLastError();
     }
