@@ -241,6 +241,7 @@ static int conv_packed(const int64_t *dev_QX, const int64_t *dev_QW, const int32
     a.y = dev_Y;
     a.qy = reinterpret_cast<uint32_t *>(dev_QY);
     a.out_ths = dev_out_ths;
+    a.out_th = 0.f;
     a.out_bits = out_bitwidth;
     a.N = N; a.H = H; a.W = W; a.PC = s.PC;
     a.KN = KN; a.KH = KH; a.KW = KW;

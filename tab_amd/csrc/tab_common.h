@@ -3,6 +3,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <string.h>
+#include <type_traits>
 
 namespace tab {
 
@@ -48,7 +50,7 @@ __host__ __device__ __forceinline__ uint32_t div32(uint32_t x, Div32 f)
     return (uint32_t)(((uint64_t)x * f.mul) >> f.shift);
 }
 
-// Arguments of the fused pad + im2row + popcount-GEMM kernel.
+// Arguments of the fused pad + im2row + GEMM kernels; they travel as ConvParams (below).
 struct ConvArgs {
     const uint64_t *qx;  // packed activation [N][H][W][PC][APL]; PC = words per pixel and plane
     const uint64_t *qw;  // packed weight     [KN][KH][KW][PC][BPL]
@@ -56,7 +58,8 @@ struct ConvArgs {
     float *y;            // [M][KN]
     // packed output instead of y (matrix-core kernel only): 32-bit halves of [M][ceil(KN/64)][out_bits]
     uint32_t *qy;
-    const float *out_ths;  // [N] thresholds applied to the outputs of image n
+    const float *out_ths;  // [N] thresholds applied to the outputs of image n; null: out_th for every image
+    float out_th;
     int out_bits;          // 1 or 2
     int N, H, W, PC;
     int KN, KH, KW;
@@ -79,6 +82,119 @@ struct ConvArgs {
     FastDiv div_pc, div_kw;
     Div32 div_pixels, div_ow;  // by OH*OW and OW: an output row's image and line
 };
+
+// ConvArgs as a kernel receives it.  The host writes kernel arguments into device memory, and from 120 bytes on that costs
+// 0.6-0.8 us a launch (measured launching back to back: 2.8 us up to 112 bytes, 3.4 at 120-128, 3.6-3.9 beyond; ConvArgs
+// itself is 248), a quarter of a small call.  So what a kernel can derive in a few scalar instructions is left out (M and
+// the tile counts), divisors are stored once, and small numbers share a dword: 104 bytes, 112 with packed output or for the
+// mixed launch.  unpack_conv gives the kernels the ConvArgs back; what they do not use of it costs nothing.
+struct ConvParams {
+    const uint64_t *qx, *qw;
+    void *out;             // y or qy
+    uint64_t btn_or_num;   // BTN: btn, otherwise num
+    int N, H, W, KN, OH, OW;
+    int p1, p2, s1, s2;
+    uint32_t pc_kw;        // PC | KW << 16
+    uint32_t g_chunks;     // G | nchunks << 16
+    uint32_t magic_pc, magic_kw, mul_pixels, mul_ow, mul_tiles;
+    uint32_t bits;         // 0-4, 5-9, 10-14: shifts of the three divisors; then the flags below
+};
+struct ConvParamsPacked : ConvParams {
+    const float *out_ths;  // or the bits of out_th (kConvOutConstant)
+};
+struct ConvParamsTail : ConvParams {
+    int tail_big, tail_chunks;
+};
+struct ConvParamsPackedTail : ConvParamsPacked {
+    int tail_big, tail_chunks;
+};
+static_assert(sizeof(ConvParams) == 104 && sizeof(ConvParamsPacked) == 112 && sizeof(ConvParamsTail) == 112, "kernel arguments below 120 bytes");
+constexpr uint32_t kConvOutBits2 = 1u << 15;      // packed output of two planes
+constexpr uint32_t kConvOutConstant = 1u << 16;   // one output threshold for every image
+constexpr uint32_t kConvCachedY = 1u << 17;
+constexpr uint32_t kConvXcdOrder = 1u << 18;      // xcd_share != 0
+constexpr uint32_t kConvRowsOrder = 1u << 19;     // tiles_n != 0
+constexpr int kConvKcwShift = 20;                 // kcw, 6 bits
+
+template <bool PACKED, bool TAIL>
+using ConvParamsOf = typename std::conditional<TAIL, typename std::conditional<PACKED, ConvParamsPackedTail, ConvParamsTail>::type,
+                                               typename std::conditional<PACKED, ConvParamsPacked, ConvParams>::type>::type;
+
+template <int TYPE, bool PACKED, bool TAIL = false>
+ConvParamsOf<PACKED, TAIL> pack_conv(const ConvArgs &a)
+{
+    ConvParamsOf<PACKED, TAIL> k;
+    k.qx = a.qx;
+    k.qw = a.qw;
+    k.out = PACKED ? static_cast<void *>(a.qy) : static_cast<void *>(a.y);
+    k.btn_or_num = TYPE == 2 ? (uint64_t)(uintptr_t)a.btn : (uint64_t)(uint32_t)a.num;
+    k.N = a.N; k.H = a.H; k.W = a.W; k.KN = a.KN; k.OH = a.OH; k.OW = a.OW;
+    k.p1 = a.p1; k.p2 = a.p2; k.s1 = a.s1; k.s2 = a.s2;
+    k.pc_kw = (uint32_t)a.PC | (uint32_t)a.KW << 16;
+    k.g_chunks = (uint32_t)a.G | (uint32_t)a.nchunks << 16;
+    k.magic_pc = a.div_pc.magic;
+    k.magic_kw = a.div_kw.magic;
+    const Div32 tiles = a.xcd_share != 0 || TAIL ? a.div_filter_tiles : a.div_tiles_m;
+    k.mul_pixels = a.div_pixels.mul;
+    k.mul_ow = a.div_ow.mul;
+    k.mul_tiles = tiles.mul;
+    k.bits = (a.div_pixels.shift - 31) | (a.div_ow.shift - 31) << 5 | (tiles.shift - 31) << 10 | (a.y_cached ? kConvCachedY : 0) |
+             (a.xcd_share != 0 ? kConvXcdOrder : 0) | (a.tiles_n != 0 ? kConvRowsOrder : 0) | (uint32_t)a.kcw << kConvKcwShift;
+    if constexpr (PACKED) {
+        k.bits |= (a.out_bits == 2 ? kConvOutBits2 : 0) | (a.out_ths == nullptr ? kConvOutConstant : 0);
+        uint32_t th;
+        memcpy(&th, &a.out_th, sizeof th);
+        k.out_ths = a.out_ths != nullptr ? a.out_ths : reinterpret_cast<const float *>((uintptr_t)th);
+    }
+    if constexpr (TAIL) {
+        k.tail_big = a.tail_big;
+        k.tail_chunks = a.tail_chunks;
+    }
+    return k;
+}
+
+// BM, BN: the workgroup's tile (of a mixed launch: the whole tile).
+template <int TYPE, bool PACKED, int BM, int BN, bool TAIL = false>
+__device__ __forceinline__ ConvArgs unpack_conv(const ConvParamsOf<PACKED, TAIL> &k)
+{
+    ConvArgs a = {};
+    a.qx = k.qx;
+    a.qw = k.qw;
+    if (PACKED) a.qy = static_cast<uint32_t *>(k.out);
+    else a.y = static_cast<float *>(k.out);
+    if (TYPE == 2) a.btn = reinterpret_cast<const int32_t *>((uintptr_t)k.btn_or_num);
+    else a.num = (int)(uint32_t)k.btn_or_num;
+    a.N = k.N; a.H = k.H; a.W = k.W; a.KN = k.KN; a.OH = k.OH; a.OW = k.OW;
+    a.p1 = k.p1; a.p2 = k.p2; a.s1 = k.s1; a.s2 = k.s2;
+    a.PC = (int)(k.pc_kw & 0xffffu);
+    a.KW = (int)(k.pc_kw >> 16);
+    a.G = (int)(k.g_chunks & 0xffffu);
+    a.nchunks = (int)(k.g_chunks >> 16);
+    a.div_pc = FastDiv{k.magic_pc, (uint32_t)a.PC};
+    a.div_kw = FastDiv{k.magic_kw, (uint32_t)a.KW};
+    a.div_pixels = Div32{k.mul_pixels, 31 + (k.bits & 31u)};
+    a.div_ow = Div32{k.mul_ow, 31 + (k.bits >> 5 & 31u)};
+    a.div_tiles_m = a.div_filter_tiles = Div32{k.mul_tiles, 31 + (k.bits >> 10 & 31u)};
+    a.M = k.N * k.OH * k.OW;
+    a.tiles_m = (a.M + BM - 1) / BM;
+    a.filter_tiles = (k.KN + BN - 1) / BN;
+    a.tiles_n = k.bits & kConvRowsOrder ? a.filter_tiles : 0;
+    a.y_cached = (k.bits & kConvCachedY) != 0;
+    a.kcw = (int)(k.bits >> kConvKcwShift & 63u);
+    if constexpr (PACKED) {
+        a.out_bits = k.bits & kConvOutBits2 ? 2 : 1;
+        const bool constant = (k.bits & kConvOutConstant) != 0;
+        a.out_ths = constant ? nullptr : k.out_ths;
+        a.out_th = __uint_as_float((uint32_t)(uintptr_t)k.out_ths);
+    }
+    if constexpr (TAIL) {
+        a.tail_big = k.tail_big;
+        a.tail_chunks = k.tail_chunks;
+    }
+    const int tiles = TAIL ? a.tail_big : a.tiles_m * a.filter_tiles;
+    a.xcd_share = k.bits & kConvXcdOrder ? (int)((uint32_t)tiles / 8u) : 0;
+    return a;
+}
 
 // Compute units of the current device (256 on MI355X), looked up once; 256 if the lookup fails.
 int device_compute_units();

@@ -83,10 +83,11 @@ __device__ __forceinline__ void popcount_acc(int &acc, uint32_t x)
 // PIPE = operand fragments double-buffered in registers (costs APL*TM + BPL*4*NG VGPRs).
 // 256 threads: one wave per SIMD (512-thread workgroups were measured slightly slower).
 template <int TYPE, int TM, int NG, int KCH, bool PIPE>
-__global__ __launch_bounds__(kThreads) void conv_popcount(const ConvArgs p)
+__global__ __launch_bounds__(kThreads) void conv_popcount(const ConvParams k)
 {
     constexpr int APL = Planes<TYPE>::A, BPL = Planes<TYPE>::B;
     constexpr int BM = 16 * TM, BN = 64 * NG, TN = 4 * NG;
+    const ConvArgs p = unpack_conv<TYPE, false, BM, BN>(k);
     using Stager = TileStager<TYPE, BM, BN, KCH>;
     constexpr int kMaxQ = Stager::Q, A_DWORDS = Stager::A_DWORDS, B_DWORDS = Stager::B_DWORDS;
     static_assert(TM % 4 == 0 || TM == 2, "TM is read with 64- or 128-bit LDS loads");
@@ -286,7 +287,7 @@ hipError_t launch_tile(ConvArgs a, hipStream_t stream)
     const long tiles_n = (a.KN + BN - 1) / BN;
     const long blocks = (long)a.tiles_m * tiles_n;
     if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
-    conv_popcount<TYPE, TM, NG, KCH, PIPE><<<dim3((unsigned)blocks), dim3(kThreads), occ.dyn_lds, stream>>>(a);
+    conv_popcount<TYPE, TM, NG, KCH, PIPE><<<dim3((unsigned)blocks), dim3(kThreads), occ.dyn_lds, stream>>>(pack_conv<TYPE, false>(a));
     return hipGetLastError();
 }
 

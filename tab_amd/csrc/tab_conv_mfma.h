@@ -302,7 +302,7 @@ __device__ __forceinline__ void conv_mfma_epilogue_packed(const ConvArgs &p, f32
         for (int mt = 0; mt < TM; mt++) {
             int n = (int)div32((uint32_t)(wave_m0 + mt * 32 + r), p.div_pixels);
             n = n < p.N ? n : p.N - 1;  // rows past M are computed but not stored
-            const float th = p.out_ths[n];
+            const float th = p.out_ths ? p.out_ths[n] : p.out_th;
             uint32_t sign_half[TN], nz_half[TN];
 #pragma unroll
             for (int nt = 0; nt < TN; nt++) {
@@ -429,8 +429,9 @@ constexpr int conv_mfma_lds_bytes()
 // PACKED: packed output (p.qy): the weights are the first MFMA operand and the epilogue packs inside a lane.
 template <int TYPE, int WM, int WN, int TM, int TN, int KCH, bool INTAP, int KS = 1, bool PACKED = false>
 __global__ __launch_bounds__(kConvThreads)
-__attribute__((amdgpu_waves_per_eu(mfma_waves_per_eu(WM, TM, TN, conv_mfma_lds_bytes<TYPE, WM, WN, TM, TN, KCH, INTAP, KS>())))) void conv_mfma(const ConvArgs p)
+__attribute__((amdgpu_waves_per_eu(mfma_waves_per_eu(WM, TM, TN, conv_mfma_lds_bytes<TYPE, WM, WN, TM, TN, KCH, INTAP, KS>())))) void conv_mfma(const ConvParamsOf<PACKED, false> k)
 {
+    const ConvArgs p = unpack_conv<TYPE, PACKED, 32 * WM * TM, 32 * WN * TN>(k);
     static_assert(WM * WN * KS * 64 == kConvThreads, "four waves");
     static_assert(!PACKED || KS == 1, "packed output: whole tiles per wave");
     static_assert(KCH % KS == 0 && (KS == 1 || (TM == 1 && TN == 1)), "k-split waves share one 32x32 tile");
@@ -567,11 +568,11 @@ hipError_t launch_mfma_tile(ConvArgs a, hipStream_t stream)
     if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
     if (a.qy != nullptr) {
         if constexpr (KS == 1)
-            conv_mfma<TYPE, WM, WN, TM, TN, KCH, INTAP, KS, true><<<dim3((unsigned)blocks), dim3(kConvThreads), 0, stream>>>(a);
+            conv_mfma<TYPE, WM, WN, TM, TN, KCH, INTAP, KS, true><<<dim3((unsigned)blocks), dim3(kConvThreads), 0, stream>>>(pack_conv<TYPE, true>(a));
         else
             return hipErrorInvalidValue;  // no packed output from the k-split 32x32 shape
     } else {
-        conv_mfma<TYPE, WM, WN, TM, TN, KCH, INTAP, KS><<<dim3((unsigned)blocks), dim3(kConvThreads), 0, stream>>>(a);
+        conv_mfma<TYPE, WM, WN, TM, TN, KCH, INTAP, KS><<<dim3((unsigned)blocks), dim3(kConvThreads), 0, stream>>>(pack_conv<TYPE, false>(a));
     }
     return hipGetLastError();
 }

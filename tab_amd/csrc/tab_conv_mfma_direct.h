@@ -415,8 +415,9 @@ __device__ __forceinline__ void conv_mfma_direct_tile(const ConvArgs &p, uint32_
 
 template <int TYPE, int WM, int WN, int TM, int TN, int KCH, bool PACKED, int KS = 1, int ARUN = 0>
 __global__ __launch_bounds__(kConvThreads)
-__attribute__((amdgpu_waves_per_eu(mfma_waves_per_eu(KS > 1 ? 1 : WM, TM, TN, 4 * conv_mfma_direct_lds_dwords<TYPE, WM, WN, TM, TN, KCH, KS>())))) void conv_mfma_direct(const ConvArgs p)
+__attribute__((amdgpu_waves_per_eu(mfma_waves_per_eu(KS > 1 ? 1 : WM, TM, TN, 4 * conv_mfma_direct_lds_dwords<TYPE, WM, WN, TM, TN, KCH, KS>())))) void conv_mfma_direct(const ConvParamsOf<PACKED, false> k)
 {
+    const ConvArgs p = unpack_conv<TYPE, PACKED, 32 * WM * TM, 32 * WN * TN>(k);
     __shared__ __attribute__((aligned(16))) uint32_t lds[conv_mfma_direct_lds_dwords<TYPE, WM, WN, TM, TN, KCH, KS>()];
     int tile_m, tile_n;
     if (!tile_of_workgroup(p, tile_m, tile_n)) return;
@@ -433,8 +434,9 @@ __attribute__((amdgpu_waves_per_eu(mfma_waves_per_eu(KS > 1 ? 1 : WM, TM, TN, 4 
 // TNB = 4: the whole tiles are 128x256 (eight MFMA tiles a wave, the pipelined loop, two workgroups a CU) and a remaining tile
 // makes eight quarters.
 template <int TYPE, int KCH, int ARUN, bool PACKED, int TNB = 2>
-__global__ __launch_bounds__(kConvThreads) __attribute__((amdgpu_waves_per_eu(TNB == 4 ? 2 : 4))) void conv_mfma_tail(const ConvArgs p)
+__global__ __launch_bounds__(kConvThreads) __attribute__((amdgpu_waves_per_eu(TNB == 4 ? 2 : 4))) void conv_mfma_tail(const ConvParamsOf<PACKED, true> k)
 {
+    const ConvArgs p = unpack_conv<TYPE, PACKED, 128, 64 * TNB, true>(k);
     constexpr int BIG = conv_mfma_direct_lds_dwords<TYPE, 2, 2, 2, TNB, KCH, 1>(), SMALL = conv_mfma_direct_lds_dwords<TYPE, 1, 1, 2, 2, 8, 4>();
     __shared__ __attribute__((aligned(16))) uint32_t lds[BIG > SMALL ? BIG : SMALL];
     const uint32_t b = blockIdx.x;
@@ -460,9 +462,9 @@ hipError_t launch_mfma_tail_run(ConvArgs a, long blocks, hipStream_t stream)
     a.nchunks = a.G / KCH;
     a.tail_chunks = (a.G + 7) / 8;  // the quarters' chunks of eight words, the last one padded with zeros
     if (a.qy != nullptr) {
-        conv_mfma_tail<TYPE, KCH, ARUN, true, TNB><<<dim3((unsigned)blocks), dim3(kConvThreads), 0, stream>>>(a);
+        conv_mfma_tail<TYPE, KCH, ARUN, true, TNB><<<dim3((unsigned)blocks), dim3(kConvThreads), 0, stream>>>(pack_conv<TYPE, true, true>(a));
     } else {
-        conv_mfma_tail<TYPE, KCH, ARUN, false, TNB><<<dim3((unsigned)blocks), dim3(kConvThreads), 0, stream>>>(a);
+        conv_mfma_tail<TYPE, KCH, ARUN, false, TNB><<<dim3((unsigned)blocks), dim3(kConvThreads), 0, stream>>>(pack_conv<TYPE, false, true>(a));
     }
     return hipGetLastError();
 }
@@ -537,9 +539,9 @@ hipError_t launch_mfma_direct(ConvArgs a, hipStream_t stream)
     const long blocks = order_workgroups<Planes<TYPE>::A>(a, (a.KN + BN - 1) / BN);
     if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
     if (a.qy != nullptr) {
-        conv_mfma_direct<TYPE, WM, WN, TM, TN, KCH, true, KS, ARUN><<<dim3((unsigned)blocks), dim3(kConvThreads), 0, stream>>>(a);
+        conv_mfma_direct<TYPE, WM, WN, TM, TN, KCH, true, KS, ARUN><<<dim3((unsigned)blocks), dim3(kConvThreads), 0, stream>>>(pack_conv<TYPE, true>(a));
     } else {
-        conv_mfma_direct<TYPE, WM, WN, TM, TN, KCH, false, KS, ARUN><<<dim3((unsigned)blocks), dim3(kConvThreads), 0, stream>>>(a);
+        conv_mfma_direct<TYPE, WM, WN, TM, TN, KCH, false, KS, ARUN><<<dim3((unsigned)blocks), dim3(kConvThreads), 0, stream>>>(pack_conv<TYPE, false>(a));
     }
     return hipGetLastError();
 }

@@ -43,11 +43,12 @@ enum RegsOut {
 
 // G: words of K per plane (runtime p.G <= G; missing words are zero on both sides), TN: 32-filter tiles per wave.
 template <int TYPE, int G, int TN, int OUT>
-__global__ __launch_bounds__(kConvThreads) __attribute__((amdgpu_waves_per_eu(2, 3))) void conv_mfma_regs(const ConvArgs p)
+__global__ __launch_bounds__(kConvThreads) __attribute__((amdgpu_waves_per_eu(2, 3))) void conv_mfma_regs(const ConvParamsOf<(OUT >= kOutBits1), false> k)
 {
     constexpr int APL = Planes<TYPE>::A, BPL = Planes<TYPE>::B;
     static_assert(TYPE >= 0 && TYPE <= 3, "types 0..3");
-    constexpr bool PACKED = OUT == kOutBits1 || OUT == kOutBits2;
+    constexpr bool PACKED = OUT >= kOutBits1;
+    const ConvArgs p = unpack_conv<TYPE, PACKED, 32, 32 * TN>(k);
     static_assert(!PACKED || TN % 2 == 0, "packed output writes whole 64-filter words");
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -111,7 +112,7 @@ __global__ __launch_bounds__(kConvThreads) __attribute__((amdgpu_waves_per_eu(2,
                 dst[w][APL - 1] = v[1];
             }
         }
-        if (PACKED) th = p.out_ths[n];
+        if (PACKED) th = p.out_ths ? p.out_ths[n] : p.out_th;
     };
 
     // the first tile's activation is requested before the weights, so that both are in flight together
@@ -347,7 +348,7 @@ hipError_t launch_mfma_regs_tile(ConvArgs a, hipStream_t stream)
     const int cap = (held + tiles_n - 1) / tiles_n;
     a.kcw = G;
     a.nchunks = 1;
-    conv_mfma_regs<TYPE, G, TN, OUT><<<dim3(regs_grid_x(tiles, cap < 1 ? 1 : cap), (unsigned)tiles_n), dim3(kConvThreads), 0, stream>>>(a);
+    conv_mfma_regs<TYPE, G, TN, OUT><<<dim3(regs_grid_x(tiles, cap < 1 ? 1 : cap), (unsigned)tiles_n), dim3(kConvThreads), 0, stream>>>(pack_conv<TYPE, (OUT >= kOutBits1)>(a));
     return hipGetLastError();
 }
 

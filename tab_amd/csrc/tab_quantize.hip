@@ -24,12 +24,16 @@ __device__ __forceinline__ int wave_sum(int v)
     return v;
 }
 
-// The counts of items 0 .. items - 1 start at zero (for one plane they stay there, TAB_GEMM.cu:283): every quantizer
-// writes them on the side, since a launch of its own for them costs 1.2-4.8 us before the quantizer.  Null: none wanted.
-__device__ __forceinline__ void zero_counts(int32_t *btn, long items)
+// The counts of items 0 .. items - 1 start at zero (for one plane they stay there, TAB_GEMM.cu:283).  Every quantizer
+// writes them on the side, since a launch of its own for them costs 1.2-4.8 us before the quantizer: a lane takes the
+// counts with the numbers of `n` rows (or pixels) of its own, of which there are at least as many as items.  At the end of
+// the kernel, so that nothing waits for the argument.  Null: none wanted.
+template <int STRIDE = 1>
+__device__ __forceinline__ void zero_counts(int32_t *btn, long items, long first, int n = 1)
 {
     if (btn == nullptr) return;
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < items; i += (long)gridDim.x * blockDim.x) btn[i] = 0;
+    for (int i = 0; i < n; i++)
+        if (first + i * STRIDE < items) btn[first + i * STRIDE] = 0;
 }
 
 // Fast path, C % 64 == 0 and X 16-byte aligned.
@@ -44,7 +48,6 @@ __global__ __launch_bounds__(kThreads) void quantize_rows64(const floatx4 *__res
                                                             uint32_t *__restrict__ q, long rows,
                                                             long rows_per_item, Div32 div_item, int32_t *btn, long items)
 {
-    zero_counts(btn, items);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // scalar: so are row0 and the item test below
     const int sub = lane >> 4;  // which of the 4 rows of a load
@@ -95,6 +98,7 @@ __global__ __launch_bounds__(kThreads) void quantize_rows64(const floatx4 *__res
             finish(u, ths[(r < rows ? r : rows - 1) / rows_per_item]);
         }
     }
+    if (lane < 4 * LOADS) zero_counts(btn, items, row0 + lane);
 }
 
 // The same row quantizer for a 1x1 convolution with stride and no padding, which reads only the
@@ -159,7 +163,6 @@ __global__ __launch_bounds__(kThreads) void quantize_groups(const float *__restr
                                                             uint32_t *__restrict__ q, long rows, long pixels_per_item,
                                                             int C, int PC, int32_t *btn, long items)
 {
-    zero_counts(btn, items);
     constexpr int GROUPS = 64 / LP;  // rows per wave-wide load
     constexpr int U = 8;
     const int lane = threadIdx.x & 63;
@@ -226,6 +229,7 @@ __global__ __launch_bounds__(kThreads) void quantize_groups(const float *__restr
 #pragma unroll
         for (int u = 0; u < U; u++) finish(u, ths[pixel[u] / pixels_per_item]);
     }
+    if (lane < GROUPS * U) zero_counts<64>(btn, items, row0 + lane, GROUPS * U / 64 > 1 ? GROUPS * U / 64 : 1);
 }
 
 // Fallback of the general path for tensors of 2^31 rows or more: one wave per (pixel, word); lane i tests channel
@@ -238,7 +242,6 @@ __global__ __launch_bounds__(kThreads) void quantize_ballot(const float *__restr
                                                             uint64_t *__restrict__ q, long pixels,
                                                             long pixels_per_item, int C, int PC, int32_t *btn, long items)
 {
-    zero_counts(btn, items);
     const int lane = threadIdx.x & 63;
     const long nwaves = (long)gridDim.x * kWavesPerBlock;
     const long units = pixels * PC;
@@ -263,6 +266,7 @@ __global__ __launch_bounds__(kThreads) void quantize_ballot(const float *__restr
             const uint64_t neg = __ballot(live && (v < t));
             if (lane == 0) q[unit] = neg;
         }
+        if (lane == 0) zero_counts(btn, items, unit);
     }
 }
 
@@ -321,7 +325,6 @@ template <int BITS, int VEC>
 __global__ __launch_bounds__(kThreads) void quantize_nchw(const float *__restrict__ x, const float *__restrict__ ths,
                                                           uint64_t *__restrict__ q, int N, int C, long HW, int PC, int32_t *btn)
 {
-    zero_counts(btn, N);
     typedef float vec_t __attribute__((ext_vector_type(VEC)));
     const int pc = blockIdx.x % PC;
     const long g0 = ((long)(blockIdx.x / PC) * kThreads + threadIdx.x) * VEC;  // first pixel, counted through all images
@@ -380,6 +383,7 @@ __global__ __launch_bounds__(kThreads) void quantize_nchw(const float *__restric
             q[pixel * PC + pc] = sign[e];
         }
     }
+    zero_counts(btn, N, g0, VEC);
 }
 
 // The NCHW quantizer for PC a multiple of U = 2 or 4 and at least one wave of work per SIMD: a thread packs U
@@ -394,7 +398,6 @@ template <int BITS, int U>
 __global__ __launch_bounds__(64) void quantize_nchw_gather(const float *__restrict__ x, const float *__restrict__ ths,
                                                                  uint64_t *__restrict__ q, int N, int C, long HW, int PC, int32_t *btn)
 {
-    zero_counts(btn, N);
     constexpr int VEC = 4, kInFlight = 8;
     constexpr int WPP = U * BITS;      // words a thread packs per pixel, contiguous in q
     constexpr int ROUNDS = WPP / 2;    // 64 / ROUNDS lanes x 4 pixels x WPP words = 512 words a round
@@ -497,6 +500,7 @@ __global__ __launch_bounds__(64) void quantize_nchw_gather(const float *__restri
             if (pixel < total) *reinterpret_cast<ulonglong2 *>(q + (pixel * PC + pc0) * BITS + w % WPP) = pair;
         }
     }
+    zero_counts(btn, N, g0, VEC);
 }
 
 // btn[n] = sum over item n of popcount(nonzero-plane word) (BTN_Weight, TAB_GEMM.cu:150-160,
@@ -512,7 +516,7 @@ constexpr int kCountLoads = 4;
 
 __global__ __launch_bounds__(kCountThreads) void btn_popcount(const ulonglong2 *__restrict__ q,
                                                               int32_t *__restrict__ btn,
-                                                              long words_per_item, int splits)
+                                                              long words_per_item, int splits, int threads)
 {
     __shared__ int partial[kCountThreads / 64];
     const long item = blockIdx.x / splits;
@@ -524,7 +528,7 @@ __global__ __launch_bounds__(kCountThreads) void btn_popcount(const ulonglong2 *
     const ulonglong2 *src = q + item * words_per_item;
     int count = 0;
     long w = w0 + threadIdx.x;
-    const long step = blockDim.x;
+    const long step = threads;  // the workgroup's size, as an argument: blockDim would add 256 bytes of hidden ones
     for (; w + (kCountLoads - 1) * step < w1; w += kCountLoads * step) {
         ulonglong2 v[kCountLoads];
 #pragma unroll
@@ -538,7 +542,7 @@ __global__ __launch_bounds__(kCountThreads) void btn_popcount(const ulonglong2 *
     __syncthreads();
     if (threadIdx.x == 0) {
         int total = 0;
-        for (int i = 0; i < (int)(blockDim.x >> 6); i++) total += partial[i];
+        for (int i = 0; i < threads >> 6; i++) total += partial[i];
         if (splits == 1)
             btn[item] = total;
         else if (total)
@@ -630,7 +634,7 @@ void launch_btn_popcount(const uint64_t *qx, int32_t *btn, long items, long word
     const long per_split = (words_per_item + splits - 1) / splits;
     const int threads = per_split >= kCountThreads ? kCountThreads : (int)((per_split + 63) / 64) * 64;
     btn_popcount<<<dim3((unsigned)(items * splits)), dim3(threads), 0, stream>>>(reinterpret_cast<const ulonglong2 *>(qx), btn,
-                                                                               words_per_item, splits);
+                                                                               words_per_item, splits, threads);
 }
 
 template <int LP>
