@@ -205,6 +205,28 @@ int tab_conv2d_packed_out(const int64_t *dev_QX, const int64_t *dev_QW, const in
                           int out_bitwidth, int64_t *dev_QY, void *stream);
 
 /*
+ * The calls of a layer whose activation thresholds come from the activation itself, as nn.TABConv2d takes them: 0 for a
+ * one-plane activation (types 2, 3), act_scale * mean|X[n]| per image for a two-plane one (types 0, 1; the values of
+ * tab_threshold).  Same results as tab_threshold + tab_quantize[_nchw] + tab_conv2d_packed, in fewer launches: no array of
+ * zeros, and the quantizer adds up an image's partial sums itself.
+ *   nchw       0: dev_X is fp32 [N][H][W][C]; otherwise [N][C][H][W]
+ *   workspace  tab_layer_workspace_bytes(bitwidth of the activation, ...), 16-byte aligned; tab_layer_quantize takes
+ *              tab_threshold_workspace_bytes(N, H*W*C) for two planes and none for one
+ */
+size_t tab_layer_workspace_bytes(int bitwidth, int N, int H, int W, int C);
+int tab_layer_quantize(const float *dev_X, int nchw, int bitwidth, float act_scale, int N, int H, int W, int C,
+                       int64_t *dev_QX, void *workspace, size_t workspace_bytes, void *stream);
+int tab_layer_conv2d(const float *dev_X, int nchw, float act_scale, const int64_t *dev_QW, const int32_t *dev_btn,
+                     int type, int padding1, int padding2, int stride1, int stride2, int N, int H, int W, int C,
+                     int KN, int KH, int KW, float *dev_Y, void *workspace, size_t workspace_bytes, void *stream);
+
+/* tab_conv2d_packed_out with one output threshold for every image. */
+int tab_conv2d_packed_out_const(const int64_t *dev_QX, const int64_t *dev_QW, const int32_t *dev_btn, int type,
+                                int padding1, int padding2, int stride1, int stride2, int N, int H, int W, int C,
+                                int KN, int KH, int KW, float out_threshold, int out_bitwidth, int64_t *dev_QY,
+                                void *stream);
+
+/*
  * Which kernel tab_conv2d / tab_conv2d_packed launch.  Both give bit-identical Y; the switch exists
  * for verification and tuning and has no counterpart in the reference (which has one GEMM kernel
  * per type, TAB_GEMM.cu:25-147).  Process-wide: the choice is one atomic word, a conv call on another

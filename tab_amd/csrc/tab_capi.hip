@@ -135,7 +135,7 @@ int tab_quantize(const float *dev_X, const float *dev_ths, int bitwidth, int N, 
     if (!dev_X || !dev_ths || !dev_QX) return fail(TAB_ERR_BAD_ARGUMENT, "null device pointer");  // dev_BTN may be NULL
     if (((uintptr_t)dev_X % 4) || ((uintptr_t)dev_QX % (8 * bitwidth)))
         return fail(TAB_ERR_BAD_ARGUMENT, "X must be aligned to its floats and QX to a whole packed element (%d bytes)", 8 * bitwidth);
-    hipError_t e = tab::launch_quantize(dev_X, dev_ths, bitwidth, (long)H * W, N, C,
+    hipError_t e = tab::launch_quantize(dev_X, tab::given_thresholds(dev_ths), bitwidth, (long)H * W, N, C,
                                         reinterpret_cast<uint64_t *>(dev_QX), dev_BTN,
                                         static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return device_fail(e, "quantize launch");
@@ -152,7 +152,7 @@ int tab_quantize_nchw(const float *dev_X, const float *dev_ths, int bitwidth, in
         return fail(TAB_ERR_BAD_ARGUMENT, "X must be aligned to its floats and QX to a whole packed element (%d bytes)", 8 * bitwidth);
     if (((long)N * H * W + 255) / 256 * tab_packed_channels(C) > kMaxIndex)
         return fail(TAB_ERR_BAD_SHAPE, "tensor too large for one launch (N*H*W/256 * ceil(C/64) workgroups)");
-    hipError_t e = tab::launch_quantize_nchw(dev_X, dev_ths, bitwidth, N, C, (long)H * W, reinterpret_cast<uint64_t *>(dev_QX),
+    hipError_t e = tab::launch_quantize_nchw(dev_X, tab::given_thresholds(dev_ths), bitwidth, N, C, (long)H * W, reinterpret_cast<uint64_t *>(dev_QX),
                                              dev_BTN, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return device_fail(e, "quantize launch");
     return TAB_OK;
@@ -217,10 +217,11 @@ static int check_conv_pointers(const ConvShape &s, int type, const void *dev_QX,
     return TAB_OK;
 }
 
-/* Shared body of the packed-activation entry points: Y as fp32 (dev_Y) or thresholded and packed (dev_QY). */
+/* Shared body of the packed-activation entry points: Y as fp32 (dev_Y) or thresholded (dev_out_ths per image, or out_th
+ * for all of them) and packed (dev_QY). */
 static int conv_packed(const int64_t *dev_QX, const int64_t *dev_QW, const int32_t *dev_btn, int type, int padding1,
                        int padding2, int stride1, int stride2, int N, int H, int W, int C, int KN, int KH, int KW,
-                       float *dev_Y, const float *dev_out_ths, int out_bitwidth, int64_t *dev_QY, void *stream)
+                       float *dev_Y, const float *dev_out_ths, float out_th, int out_bitwidth, int64_t *dev_QY, void *stream)
 {
     ConvShape s;
     int rc = check_conv(type, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, &s);
@@ -230,7 +231,6 @@ static int conv_packed(const int64_t *dev_QX, const int64_t *dev_QW, const int32
     if (dev_QY) {
         if (out_bitwidth != 1 && out_bitwidth != 2)
             return fail(TAB_ERR_BAD_ARGUMENT, "out_bitwidth must be 1 or 2, got %d", out_bitwidth);
-        if (!dev_out_ths) return fail(TAB_ERR_BAD_ARGUMENT, "null device pointer");
         if ((uintptr_t)dev_QY % (8 * out_bitwidth)) return fail(TAB_ERR_BAD_ARGUMENT, "QY must be aligned to a whole packed element");
     }
 
@@ -241,7 +241,7 @@ static int conv_packed(const int64_t *dev_QX, const int64_t *dev_QW, const int32
     a.y = dev_Y;
     a.qy = reinterpret_cast<uint32_t *>(dev_QY);
     a.out_ths = dev_out_ths;
-    a.out_th = 0.f;
+    a.out_th = out_th;
     a.out_bits = out_bitwidth;
     a.N = N; a.H = H; a.W = W; a.PC = s.PC;
     a.KN = KN; a.KH = KH; a.KW = KW;
@@ -276,7 +276,7 @@ int tab_conv2d_packed(const int64_t *dev_QX, const int64_t *dev_QW, const int32_
 {
     if (!dev_Y) return fail(TAB_ERR_BAD_ARGUMENT, "null device pointer");
     return conv_packed(dev_QX, dev_QW, dev_btn, type, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW,
-                       dev_Y, nullptr, 0, nullptr, stream);
+                       dev_Y, nullptr, 0.f, 0, nullptr, stream);
 }
 
 int tab_conv2d_packed_out(const int64_t *dev_QX, const int64_t *dev_QW, const int32_t *dev_btn,
@@ -284,9 +284,19 @@ int tab_conv2d_packed_out(const int64_t *dev_QX, const int64_t *dev_QW, const in
                           int H, int W, int C, int KN, int KH, int KW, const float *dev_out_ths,
                           int out_bitwidth, int64_t *dev_QY, void *stream)
 {
+    if (!dev_QY || !dev_out_ths) return fail(TAB_ERR_BAD_ARGUMENT, "null device pointer");
+    return conv_packed(dev_QX, dev_QW, dev_btn, type, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW,
+                       nullptr, dev_out_ths, 0.f, out_bitwidth, dev_QY, stream);
+}
+
+int tab_conv2d_packed_out_const(const int64_t *dev_QX, const int64_t *dev_QW, const int32_t *dev_btn,
+                                int type, int padding1, int padding2, int stride1, int stride2, int N,
+                                int H, int W, int C, int KN, int KH, int KW, float out_threshold,
+                                int out_bitwidth, int64_t *dev_QY, void *stream)
+{
     if (!dev_QY) return fail(TAB_ERR_BAD_ARGUMENT, "null device pointer");
     return conv_packed(dev_QX, dev_QW, dev_btn, type, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW,
-                       nullptr, dev_out_ths, out_bitwidth, dev_QY, stream);
+                       nullptr, nullptr, out_threshold, out_bitwidth, dev_QY, stream);
 }
 
 /* Device address of `scratch` on the current device, looked up on the first call made with that device current. */
@@ -311,41 +321,28 @@ static int static_scratch(void **out)
     return TAB_OK;
 }
 
-/* Body of tab_conv2d and tab_conv2d_static (workspace == NULL and builtin: the library's own scratch): quantize
- * into the workspace, then the fused conv kernel. */
-static int conv_from_floats(const float *dev_X, const int64_t *dev_QW, const float *dev_ths, const int32_t *dev_btn, int type,
-                            int padding1, int padding2, int stride1, int stride2, int N, int H, int W, int C, int KN, int KH,
-                            int KW, float *dev_Y, void *workspace, size_t workspace_bytes, bool builtin, void *stream)
+/* Pointer, alignment and size checks of the calls that start from fp32: everything the second stage would reject is
+ * rejected before the quantizer is enqueued. */
+static int check_from_floats(const ConvShape &s, int type, const float *dev_X, const int64_t *dev_QW, const int32_t *dev_btn,
+                             const float *dev_Y, const void *workspace, size_t workspace_bytes, size_t need)
 {
-    ConvShape s;
-    int rc = check_conv(type, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, &s);
-    if (rc != TAB_OK) return rc;
-    if (!dev_X || !dev_ths) return fail(TAB_ERR_BAD_ARGUMENT, "null device pointer");
+    if (!dev_X) return fail(TAB_ERR_BAD_ARGUMENT, "null device pointer");
     if ((uintptr_t)dev_X % 4) return fail(TAB_ERR_BAD_ARGUMENT, "X must be aligned to its floats");
-    const size_t need = tab_conv2d_workspace_bytes(type, N, H, W, C);
-    if (builtin) {
-        if (need > TAB_STATIC_SCRATCH_BYTES)
-            return fail(TAB_ERR_WORKSPACE, "the packed activation needs %zu bytes, the built-in scratch holds %zu; use tab_conv2d with a workspace",
-                        need, (size_t)TAB_STATIC_SCRATCH_BYTES);
-        rc = static_scratch(&workspace);
-        if (rc != TAB_OK) return rc;
-    } else if (!workspace || workspace_bytes < need || ((uintptr_t)workspace % 16)) {
+    if (!workspace || workspace_bytes < need || ((uintptr_t)workspace % 16))
         return fail(TAB_ERR_WORKSPACE, "workspace must be 16-byte aligned and hold %zu bytes (got %zu)", need, workspace_bytes);
-    }
-    // everything the second stage would reject is rejected here, before the quantizer is enqueued
-    rc = check_conv_pointers(s, type, workspace, dev_QW, dev_btn, dev_Y, nullptr);
-    if (rc != TAB_OK) return rc;
-    if (type > 3) {  // the CPU-only types: their own packers, then the same fused kernel
-        hipError_t e = tab::launch_quantize_format(dev_X, dev_ths, type, (long)H * W, N, C, reinterpret_cast<uint64_t *>(workspace),
-                                                   static_cast<hipStream_t>(stream));
-        if (e != hipSuccess) return device_fail(e, "quantize launch");
-        return tab_conv2d_packed(reinterpret_cast<const int64_t *>(workspace), dev_QW, dev_btn, type, padding1, padding2, stride1,
-                                 stride2, N, H, W, C, KN, KH, KW, dev_Y, stream);
-    }
+    return check_conv_pointers(s, type, workspace, dev_QW, dev_btn, dev_Y, nullptr);
+}
+
+/* Quantize an NHWC activation of types 0..3 into the workspace, then the fused conv kernel; small and strided 1x1 layers
+ * take their own ways.  The arguments have been checked. */
+static int conv_from_nhwc(const float *dev_X, const int64_t *dev_QW, const tab::Thresholds &ths, const int32_t *dev_btn, int type,
+                          int padding1, int padding2, int stride1, int stride2, int N, int H, int W, int C, int KN, int KH, int KW,
+                          const ConvShape &s, float *dev_Y, void *workspace, void *stream)
+{
     // A small 1x1 convolution without padding: quantize and multiply in one launch, the packed activation stays in LDS
     // (only under the automatic kernel choice: a forced kernel is what the caller wants to see run)
     if (!tab::conv_kernel_forced() && tab::conv1x1_fused_supported(type, dev_X, C, KH, KW, padding1, padding2, s.M, KN)) {
-        hipError_t e = tab::launch_conv1x1_fused(type, dev_X, dev_ths, reinterpret_cast<const uint64_t *>(dev_QW), dev_btn, dev_Y, N, H,
+        hipError_t e = tab::launch_conv1x1_fused(type, dev_X, ths, reinterpret_cast<const uint64_t *>(dev_QW), dev_btn, dev_Y, N, H,
                                                  W, C, KN, stride1, stride2, s.OH, s.OW, static_cast<hipStream_t>(stream));
         if (e != hipSuccess) return device_fail(e, "conv launch");
         return TAB_OK;
@@ -355,21 +352,131 @@ static int conv_from_floats(const float *dev_X, const int64_t *dev_QW, const flo
     // the reads of X).
     if (KH == 1 && KW == 1 && padding1 == 0 && padding2 == 0 && (stride1 > 1 || stride2 > 1) && N * (long)s.OH < 65536 &&
         tab::quantize_strided_supported(dev_X, H, W, C, s.OH, s.OW)) {
-        hipError_t e = tab::launch_quantize_strided(dev_X, dev_ths, s.abits, N, H, W, C, s.OH, s.OW, stride1, stride2,
+        hipError_t e = tab::launch_quantize_strided(dev_X, ths, s.abits, N, H, W, C, s.OH, s.OW, stride1, stride2,
                                                     reinterpret_cast<uint64_t *>(workspace), static_cast<hipStream_t>(stream));
         if (e != hipSuccess) return device_fail(e, "quantize launch");
         return tab_conv2d_packed(reinterpret_cast<const int64_t *>(workspace), dev_QW, dev_btn, type, 0, 0, 1, 1, N, s.OH,
                                  s.OW, C, KN, 1, 1, dev_Y, stream);
     }
     // stage 1: quantize + pack the activation (TAB_GEMM.cu:419-426); no btn for activations
-    hipError_t e = tab::launch_quantize(dev_X, dev_ths, s.abits, (long)H * W, N, C,
-                                        reinterpret_cast<uint64_t *>(workspace), nullptr,
+    hipError_t e = tab::launch_quantize(dev_X, ths, s.abits, (long)H * W, N, C, reinterpret_cast<uint64_t *>(workspace), nullptr,
                                         static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return device_fail(e, "quantize launch");
     // stage 2: pad + im2row + GEMM, fused
     return tab_conv2d_packed(reinterpret_cast<const int64_t *>(workspace), dev_QW, dev_btn, type,
                              padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, dev_Y,
                              stream);
+}
+
+/* Body of tab_conv2d and tab_conv2d_static (builtin: the library's own scratch). */
+static int conv_from_floats(const float *dev_X, const int64_t *dev_QW, const float *dev_ths, const int32_t *dev_btn, int type,
+                            int padding1, int padding2, int stride1, int stride2, int N, int H, int W, int C, int KN, int KH,
+                            int KW, float *dev_Y, void *workspace, size_t workspace_bytes, bool builtin, void *stream)
+{
+    ConvShape s;
+    int rc = check_conv(type, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, &s);
+    if (rc != TAB_OK) return rc;
+    if (!dev_X || !dev_ths) return fail(TAB_ERR_BAD_ARGUMENT, "null device pointer");
+    const size_t need = tab_conv2d_workspace_bytes(type, N, H, W, C);
+    if (builtin) {
+        if (need > TAB_STATIC_SCRATCH_BYTES)
+            return fail(TAB_ERR_WORKSPACE, "the packed activation needs %zu bytes, the built-in scratch holds %zu; use tab_conv2d with a workspace",
+                        need, (size_t)TAB_STATIC_SCRATCH_BYTES);
+        rc = static_scratch(&workspace);
+        if (rc != TAB_OK) return rc;
+        workspace_bytes = TAB_STATIC_SCRATCH_BYTES;
+    }
+    rc = check_from_floats(s, type, dev_X, dev_QW, dev_btn, dev_Y, workspace, workspace_bytes, need);
+    if (rc != TAB_OK) return rc;
+    if (type > 3) {  // the CPU-only types: their own packers, then the same fused kernel
+        hipError_t e = tab::launch_quantize_format(dev_X, dev_ths, type, (long)H * W, N, C, reinterpret_cast<uint64_t *>(workspace),
+                                                   static_cast<hipStream_t>(stream));
+        if (e != hipSuccess) return device_fail(e, "quantize launch");
+        return tab_conv2d_packed(reinterpret_cast<const int64_t *>(workspace), dev_QW, dev_btn, type, padding1, padding2, stride1,
+                                 stride2, N, H, W, C, KN, KH, KW, dev_Y, stream);
+    }
+    return conv_from_nhwc(dev_X, dev_QW, tab::given_thresholds(dev_ths), dev_btn, type, padding1, padding2, stride1, stride2, N, H, W, C,
+                          KN, KH, KW, s, dev_Y, workspace, stream);
+}
+
+/* Packed activation bytes of a layer call, rounded up so that the partial sums behind them are aligned. */
+static size_t layer_packed_bytes(int bitwidth, int N, int H, int W, int C)
+{
+    return ((size_t)N * H * W * tab_packed_channels(C) * bitwidth * sizeof(int64_t) + 15) & ~(size_t)15;
+}
+
+/* Thresholds of an activation taken from itself: 0 for one plane, act_scale * mean|x| per item for two, whose partial sums
+ * (launched here) go to `sums`. */
+static hipError_t own_thresholds(const float *dev_X, int bitwidth, float act_scale, int N, long per_item, void *sums,
+                                 tab::Thresholds *ths, void *stream)
+{
+    *ths = tab::given_thresholds(nullptr);
+    if (bitwidth == 1) return hipSuccess;
+    return tab::launch_abs_sums(dev_X, N, per_item, act_scale, static_cast<float *>(sums), ths, static_cast<hipStream_t>(stream));
+}
+
+size_t tab_layer_workspace_bytes(int bitwidth, int N, int H, int W, int C)
+{
+    if (bitwidth < 1 || bitwidth > 2 || N < 1 || H < 1 || W < 1 || C < 1) return 0;
+    const size_t sums = tab_threshold_workspace_bytes(N, (long)H * W * C) + (size_t)N * sizeof(float);
+    return layer_packed_bytes(bitwidth, N, H, W, C) + (bitwidth == 2 ? sums : 0);
+}
+
+int tab_layer_quantize(const float *dev_X, int nchw, int bitwidth, float act_scale, int N, int H, int W, int C, int64_t *dev_QX,
+                       void *workspace, size_t workspace_bytes, void *stream)
+{
+    if (bitwidth != 1 && bitwidth != 2) return fail(TAB_ERR_BAD_ARGUMENT, "bitwidth must be 1 or 2, got %d", bitwidth);
+    if (N < 1 || H < 1 || W < 1 || C < 1) return fail(TAB_ERR_BAD_ARGUMENT, "N, H, W, C must be positive");
+    if (!dev_X || !dev_QX) return fail(TAB_ERR_BAD_ARGUMENT, "null device pointer");
+    if (((uintptr_t)dev_X % 4) || ((uintptr_t)dev_QX % (8 * bitwidth)))
+        return fail(TAB_ERR_BAD_ARGUMENT, "X must be aligned to its floats and QX to a whole packed element (%d bytes)", 8 * bitwidth);
+    if (nchw && ((long)N * H * W + 255) / 256 * tab_packed_channels(C) > kMaxIndex)
+        return fail(TAB_ERR_BAD_SHAPE, "tensor too large for one launch (N*H*W/256 * ceil(C/64) workgroups)");
+    const long per_item = (long)H * W * C;
+    const size_t need = bitwidth == 2 ? tab_threshold_workspace_bytes(N, per_item) : 0;
+    if (need && (!workspace || workspace_bytes < need || ((uintptr_t)workspace % 4)))
+        return fail(TAB_ERR_WORKSPACE, "workspace must hold %zu bytes (got %zu)", need, workspace_bytes);
+    tab::Thresholds ths;
+    hipError_t e = own_thresholds(dev_X, bitwidth, act_scale, N, per_item, workspace, &ths, stream);
+    if (e != hipSuccess) return device_fail(e, "threshold launch");
+    uint64_t *q = reinterpret_cast<uint64_t *>(dev_QX);
+    // one pixel per image: NCHW and NHWC are the same memory, and the NHWC quantizers read it along the channels
+    e = nchw && H * W > 1 ? tab::launch_quantize_nchw(dev_X, ths, bitwidth, N, C, (long)H * W, q, nullptr, static_cast<hipStream_t>(stream))
+                          : tab::launch_quantize(dev_X, ths, bitwidth, (long)H * W, N, C, q, nullptr, static_cast<hipStream_t>(stream));
+    if (e != hipSuccess) return device_fail(e, "quantize launch");
+    return TAB_OK;
+}
+
+int tab_layer_conv2d(const float *dev_X, int nchw, float act_scale, const int64_t *dev_QW, const int32_t *dev_btn, int type,
+                     int padding1, int padding2, int stride1, int stride2, int N, int H, int W, int C, int KN, int KH, int KW,
+                     float *dev_Y, void *workspace, size_t workspace_bytes, void *stream)
+{
+    if (type > 3) return fail(TAB_ERR_BAD_ARGUMENT, "type must be 0 (TNN), 1 (TBN), 2 (BTN) or 3 (BNN), got %d", type);
+    ConvShape s;
+    int rc = check_conv(type, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, &s);
+    if (rc != TAB_OK) return rc;
+    rc = check_from_floats(s, type, dev_X, dev_QW, dev_btn, dev_Y, workspace, workspace_bytes, tab_layer_workspace_bytes(s.abits, N, H, W, C));
+    if (rc != TAB_OK) return rc;
+    char *sums = static_cast<char *>(workspace) + layer_packed_bytes(s.abits, N, H, W, C);
+    if (nchw && H * W > 1) {
+        rc = tab_layer_quantize(dev_X, 1, s.abits, act_scale, N, H, W, C, static_cast<int64_t *>(workspace), sums,
+                                workspace_bytes - layer_packed_bytes(s.abits, N, H, W, C), stream);
+        if (rc != TAB_OK) return rc;
+        return tab_conv2d_packed(static_cast<const int64_t *>(workspace), dev_QW, dev_btn, type, padding1, padding2, stride1, stride2,
+                                 N, H, W, C, KN, KH, KW, dev_Y, stream);
+    }
+    tab::Thresholds ths;
+    hipError_t e = own_thresholds(dev_X, s.abits, act_scale, N, (long)H * W * C, sums, &ths, stream);
+    if (e != hipSuccess) return device_fail(e, "threshold launch");
+    if (ths.splits > 4 && tab::conv1x1_fused_supported(type, dev_X, C, KH, KW, padding1, padding2, s.M, KN)) {
+        // the one-launch 1x1 kernel looks thresholds up lane by lane: with many partial sums an item they are added first
+        float *values = reinterpret_cast<float *>(sums + tab_threshold_workspace_bytes(N, (long)H * W * C));
+        e = tab::launch_threshold_values(ths, N, values, static_cast<hipStream_t>(stream));
+        if (e != hipSuccess) return device_fail(e, "threshold launch");
+        ths = tab::given_thresholds(values);
+    }
+    return conv_from_nhwc(dev_X, dev_QW, ths, dev_btn, type, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, s, dev_Y,
+                          workspace, stream);
 }
 
 int tab_conv2d(const float *dev_X, const int64_t *dev_QW, const float *dev_ths,

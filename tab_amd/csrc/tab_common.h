@@ -214,11 +214,22 @@ hipError_t launch_conv_mfma_btn(const ConvArgs &args, int shape, hipStream_t str
 hipError_t launch_conv_mfma_bnn(const ConvArgs &args, int shape, hipStream_t stream);
 hipError_t launch_conv_mfma_drf(const ConvArgs &args, int shape, hipStream_t stream);
 hipError_t launch_conv_mfma_rtn(const ConvArgs &args, int shape, hipStream_t stream);
-hipError_t launch_quantize(const float *x, const float *ths, int bitwidth, long pixels_per_item,
+
+// Where a quantizer finds the threshold of item n: values[n] (splits == 0), the scaled sum of the item's `splits` partial
+// sums of |x| that launch_abs_sums left (values[n * splits ...]; the quantizer adds them up itself, which saves the launch
+// that would), or 0 for every item (values == null).
+struct Thresholds {
+    const float *values;
+    double scale;
+    int splits;
+};
+inline Thresholds given_thresholds(const float *ths) { return Thresholds{ths, 0.0, 0}; }
+
+hipError_t launch_quantize(const float *x, const Thresholds &ths, int bitwidth, long pixels_per_item,
                            long items, int C, uint64_t *qx, int32_t *btn, hipStream_t stream);
 
 // The same quantizer reading x as [N][C][H*W] (the CPU path's input layout, TAB_CPU.cpp:20-206); output as above.
-hipError_t launch_quantize_nchw(const float *x, const float *ths, int bitwidth, int N, int C, long HW, uint64_t *qx,
+hipError_t launch_quantize_nchw(const float *x, const Thresholds &ths, int bitwidth, int N, int C, long HW, uint64_t *qx,
                                 int32_t *btn, hipStream_t stream);
 
 // Packers of the CPU-only conv types: format 4 = DoReFa 2-bit levels, 5 = RTN fields.
@@ -228,18 +239,23 @@ hipError_t launch_quantize_format(const float *x, const float *ths, int format, 
 // Quantize only the pixels (oh*s1, ow*s2) of every image into a compact [N][OH][OW][PC] activation
 // (what a 1x1 convolution with stride and no padding reads).
 bool quantize_strided_supported(const float *x, int H, int W, int C, int OH, int OW);
-hipError_t launch_quantize_strided(const float *x, const float *ths, int bitwidth, int N, int H, int W, int C, int OH,
+hipError_t launch_quantize_strided(const float *x, const Thresholds &ths, int bitwidth, int N, int H, int W, int C, int OH,
                                    int OW, int s1, int s2, uint64_t *qx, hipStream_t stream);
 
 // ths[n] = scale * mean|x[n]| over per_item elements; `partial` holds items * threshold_splits()
 // floats of scratch.
 int threshold_splits(long items, long per_item);
+// The first half of launch_threshold: what a quantizer needs to find the thresholds itself (*source, in `partial`).
+hipError_t launch_abs_sums(const float *x, long items, long per_item, float scale, float *partial, Thresholds *source,
+                           hipStream_t stream);
+// ths[n] from what launch_abs_sums left.
+hipError_t launch_threshold_values(const Thresholds &source, long items, float *ths, hipStream_t stream);
 hipError_t launch_threshold(const float *x, long items, long per_item, float scale, float *ths, float *partial,
                             hipStream_t stream);
 
 // Quantize + 1x1 conv in one launch (tab_conv_fused1x1.hip), for calls that are bound by their launches.
 bool conv1x1_fused_supported(int type, const float *x, int C, int KH, int KW, int p1, int p2, long M, int KN);
-hipError_t launch_conv1x1_fused(int type, const float *x, const float *ths, const uint64_t *qw, const int32_t *btn, float *y, int N,
+hipError_t launch_conv1x1_fused(int type, const float *x, const Thresholds &ths, const uint64_t *qw, const int32_t *btn, float *y, int N,
                                 int H, int W, int C, int KN, int s1, int s2, int OH, int OW, hipStream_t stream);
 
 void force_conv_tile(int tm, int ng);  // tuning hook: 0,0 restores the automatic choice

@@ -21,16 +21,16 @@ namespace {
 
 struct Fused1x1Args {
     const float *x;       // fp32 [N][H][W][C]
-    const float *ths;     // [N]
+    Thresholds ths;       // of the N images
     const uint64_t *qw;   // packed weight [KN][PC][BPL]
     const int32_t *btn;   // [KN] (BTN only)
     float *y;             // [M][KN]
-    int N, H, W, C;
+    int H, W, C;          // (C: also the BNN constant)
     int KN, s1, s2;
     int OH, OW, M;
-    int num;              // C (BNN constant)
     Div32 div_pixels, div_ow;
 };
+static_assert(sizeof(Fused1x1Args) <= 112, "kernel arguments below 120 bytes (see ConvParams)");
 
 // PC: 64-channel words per pixel (1, 2, 4 or 8).
 template <int TYPE, int PC>
@@ -67,7 +67,7 @@ __global__ __launch_bounds__(kConvThreads) void conv1x1_fused(const Fused1x1Args
         const int oh = (int)div32((uint32_t)rem, p.div_ow), ow = rem - oh * p.OW;
         const size_t in_pixel = ((size_t)n * p.H + (size_t)oh * p.s1) * p.W + (size_t)ow * p.s2;
         v[i] = *reinterpret_cast<const floatx4 *>(p.x + in_pixel * p.C + word * 64 + l * 4);
-        th[i] = p.ths[n];
+        th[i] = lane_threshold(p.ths, n);
     }
 
     // ---- weights: filter n0 + r, half kb of every word and plane (filters past KN repeat the last one, never stored) ----
@@ -116,7 +116,7 @@ __global__ __launch_bounds__(kConvThreads) void conv1x1_fused(const Fused1x1Args
     if (TYPE == 0) acc *= 0.25f;  // both operands are +-2: four times the sums
 
     // BTN btn[f] - popcount(b1 of f), BNN NUM - 64 per word (TAB_GEMM.cu:116, 144)
-    float bias = TYPE == 3 ? (float)(p.num - 64 * PC) : 0.f;
+    float bias = TYPE == 3 ? (float)(p.C - 64 * PC) : 0.f;
     if (TYPE == 2) {
         const int f = n0 + r;
         bias = (float)((f < p.KN ? p.btn[f] : 0) - (nonzero + __shfl_xor(nonzero, 32, 64)));
@@ -172,14 +172,13 @@ bool conv1x1_fused_supported(int type, const float *x, int C, int KH, int KW, in
            (M + 31) / 32 * ((KN + 127) / 128) <= kFusedMaxWorkgroups && (KN + 127) / 128 <= 65535;
 }
 
-hipError_t launch_conv1x1_fused(int type, const float *x, const float *ths, const uint64_t *qw, const int32_t *btn, float *y, int N,
+hipError_t launch_conv1x1_fused(int type, const float *x, const Thresholds &ths, const uint64_t *qw, const int32_t *btn, float *y, int N,
                                 int H, int W, int C, int KN, int s1, int s2, int OH, int OW, hipStream_t stream)
 {
     Fused1x1Args a;
     a.x = x; a.ths = ths; a.qw = qw; a.btn = btn; a.y = y;
-    a.N = N; a.H = H; a.W = W; a.C = C; a.KN = KN; a.s1 = s1; a.s2 = s2; a.OH = OH; a.OW = OW;
+    a.H = H; a.W = W; a.C = C; a.KN = KN; a.s1 = s1; a.s2 = s2; a.OH = OH; a.OW = OW;
     a.M = N * OH * OW;
-    a.num = C;
     a.div_pixels = make_div32((uint32_t)(OH * OW));
     a.div_ow = make_div32((uint32_t)OW);
     switch (type) {

@@ -10,6 +10,29 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
 typedef uint32_t uintx2 __attribute__((ext_vector_type(2)));
 
+// Threshold of an item of the lane's own; for partial sums a lane adds them up alone.
+__device__ __forceinline__ float lane_threshold(const Thresholds &t, long item)
+{
+    if (t.values == nullptr) return 0.f;
+    if (t.splits == 0) return t.values[item];
+    double sum = 0.0;
+    for (int i = 0; i < t.splits; i++) sum += (double)t.values[item * t.splits + i];
+    return (float)(sum * t.scale);
+}
+
+// Threshold of one item for a whole wave (every lane active): the lanes share the partial sums.  The order of the sum
+// differs from lane_threshold's; a sum of up to 1024 fp32 values within a factor of 2^19 of each other is exact in fp64.
+__device__ __forceinline__ float wave_threshold(const Thresholds &t, long item)
+{
+    if (t.values == nullptr) return 0.f;
+    if (t.splits == 0) return t.values[item];
+    double sum = 0.0;
+    for (int i = (int)(threadIdx.x & 63); i < t.splits; i += 64) sum += (double)t.values[item * t.splits + i];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+    return __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint((float)(sum * t.scale))));
+}
+
 // OR over the 8 lanes of each half of a 16-lane DPP row; every lane gets the result.
 __device__ __forceinline__ uint32_t or_reduce8(uint32_t v)
 {

@@ -44,7 +44,7 @@ __device__ __forceinline__ void zero_counts(int32_t *btn, long items, long first
 // workgroup) for streaming, 2 for launches too small to fill the chip.
 template <int BITS, int LOADS = kLoadsPerLane>
 __global__ __launch_bounds__(kThreads) void quantize_rows64(const floatx4 *__restrict__ x,
-                                                            const float *__restrict__ ths,
+                                                            const Thresholds ths,
                                                             uint32_t *__restrict__ q, long rows,
                                                             long rows_per_item, Div32 div_item, int32_t *btn, long items)
 {
@@ -73,7 +73,7 @@ __global__ __launch_bounds__(kThreads) void quantize_rows64(const floatx4 *__res
     const long item_first = div_item.mul ? (long)div32((uint32_t)row0, div_item) : row0 / rows_per_item;
     const long item_last = div_item.mul ? (long)div32((uint32_t)row_last, div_item) : row_last / rows_per_item;
     const bool one_item = item_last == item_first;
-    const float t_first = ths[item_first];
+    const float t_first = wave_threshold(ths, item_first);
 
     auto finish = [&](int u, float t) {
         const long r = row0 + u * 4 + sub;
@@ -95,7 +95,7 @@ __global__ __launch_bounds__(kThreads) void quantize_rows64(const floatx4 *__res
 #pragma unroll
         for (int u = 0; u < LOADS; u++) {
             const long r = row0 + u * 4 + sub;
-            finish(u, ths[(r < rows ? r : rows - 1) / rows_per_item]);
+            finish(u, lane_threshold(ths, (r < rows ? r : rows - 1) / rows_per_item));
         }
     }
     if (lane < 4 * LOADS) zero_counts(btn, items, row0 + lane);
@@ -106,7 +106,7 @@ __global__ __launch_bounds__(kThreads) void quantize_rows64(const floatx4 *__res
 // result is the compact [N][OH][OW][PC] activation, i.e. what the conv reads with stride 1.
 // grid = (ceil(OW*PC / (4*LOADS)), N*OH), one wave per workgroup; OW*PC < 65536 (fastdiv range).
 template <int BITS, int LOADS = kLoadsPerLane>
-__global__ __launch_bounds__(64) void quantize_rows64_strided(const floatx4 *__restrict__ x, const float *__restrict__ ths,
+__global__ __launch_bounds__(64) void quantize_rows64_strided(const floatx4 *__restrict__ x, const Thresholds ths,
                                                               uint32_t *__restrict__ q, int H, int W, int PC, int OH,
                                                               int OW, int s1, int s2, FastDiv div_pc)
 {
@@ -117,7 +117,6 @@ __global__ __launch_bounds__(64) void quantize_rows64_strided(const floatx4 *__r
     const long in_line = ((long)n * H + (long)oh * s1) * W;   // first input pixel of the line
     const long out_line = (long)blockIdx.y * line_words;
     const int j0 = blockIdx.x * (4 * LOADS);
-    const float t = ths[n];
 
     floatx4 v[LOADS];
 #pragma unroll
@@ -127,6 +126,7 @@ __global__ __launch_bounds__(64) void quantize_rows64_strided(const floatx4 *__r
         const long r = (in_line + (long)ow * s2) * PC + pc;
         v[u] = LOADS == 2 ? x[r * 16 + l] : __builtin_nontemporal_load(&x[r * 16 + l]);
     }
+    const float t = wave_threshold(ths, n);
 #pragma unroll
     for (int u = 0; u < LOADS; u++) {
         const int j = j0 + u * 4 + sub;
@@ -159,7 +159,7 @@ __device__ __forceinline__ uint32_t or_reduce_group(uint32_t v)
 // smaller groups tensors of few channels (LP = 1: a lane per pixel).  Eight rows per group are in flight.  The
 // lanes' compare bits are ORed over the group; unused high bits of a tail word stay 0 (TAB_GEMM.cu:203-206).
 template <int BITS, int LP>
-__global__ __launch_bounds__(kThreads) void quantize_groups(const float *__restrict__ x, const float *__restrict__ ths,
+__global__ __launch_bounds__(kThreads) void quantize_groups(const float *__restrict__ x, const Thresholds ths,
                                                             uint32_t *__restrict__ q, long rows, long pixels_per_item,
                                                             int C, int PC, int32_t *btn, long items)
 {
@@ -194,7 +194,7 @@ __global__ __launch_bounds__(kThreads) void quantize_groups(const float *__restr
 
     const long item_first = (row0 / PC) / pixels_per_item;
     const bool one_item = ((row_last / PC) / pixels_per_item) == item_first;  // scalar
-    const float t_first = ths[item_first];
+    const float t_first = wave_threshold(ths, item_first);
 
     auto finish = [&](int u, float t) {
         uint32_t w[4] = {0, 0, 0, 0};  // sign low, sign high, nonzero low, nonzero high
@@ -227,7 +227,7 @@ __global__ __launch_bounds__(kThreads) void quantize_groups(const float *__restr
         for (int u = 0; u < U; u++) finish(u, t_first);
     } else {
 #pragma unroll
-        for (int u = 0; u < U; u++) finish(u, ths[pixel[u] / pixels_per_item]);
+        for (int u = 0; u < U; u++) finish(u, lane_threshold(ths, pixel[u] / pixels_per_item));
     }
     if (lane < GROUPS * U) zero_counts<64>(btn, items, row0 + lane, GROUPS * U / 64 > 1 ? GROUPS * U / 64 : 1);
 }
@@ -238,7 +238,7 @@ __global__ __launch_bounds__(kThreads) void quantize_groups(const float *__restr
 // (TAB_GEMM.cu:203-206).
 template <int BITS>
 __global__ __launch_bounds__(kThreads) void quantize_ballot(const float *__restrict__ x,
-                                                            const float *__restrict__ ths,
+                                                            const Thresholds ths,
                                                             uint64_t *__restrict__ q, long pixels,
                                                             long pixels_per_item, int C, int PC, int32_t *btn, long items)
 {
@@ -249,7 +249,7 @@ __global__ __launch_bounds__(kThreads) void quantize_ballot(const float *__restr
         const long pixel = unit / PC;
         const int word = (int)(unit - pixel * PC);
         const long item = pixel / pixels_per_item;
-        const float t = ths[item];
+        const float t = wave_threshold(ths, item);
         const int c = word * kWordBits + lane;
         const bool live = c < C;
         const float v = live ? x[pixel * C + c] : 0.f;
@@ -279,7 +279,7 @@ __global__ __launch_bounds__(kThreads) void quantize_ballot(const float *__restr
 //   [pixel][ceil(C/32)], channel c in word c/32 as the field (bit 2*(c%32) = nonzero, bit 2*(c%32)+1 =
 //   sign) of the ternarizer's value; lane j of the wave tests channel j/2 for bit j.
 template <int FORMAT>
-__global__ __launch_bounds__(kThreads) void quantize_ballot_format(const float *__restrict__ x, const float *__restrict__ ths,
+__global__ __launch_bounds__(kThreads) void quantize_ballot_format(const float *__restrict__ x, const Thresholds ths,
                                                                    uint64_t *__restrict__ q, long pixels,
                                                                    long pixels_per_item, int C, int PC)
 {
@@ -289,7 +289,7 @@ __global__ __launch_bounds__(kThreads) void quantize_ballot_format(const float *
     for (long unit = (long)blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6); unit < units; unit += nwaves) {
         const long pixel = unit / PC;
         const int word = (int)(unit - pixel * PC);
-        const float t = ths[pixel / pixels_per_item];
+        const float t = lane_threshold(ths, pixel / pixels_per_item);
         if (FORMAT == 4) {
             const int c = word * kWordBits + lane;
             const bool live = c < C;
@@ -321,38 +321,44 @@ __global__ __launch_bounds__(kThreads) void quantize_ballot_format(const float *
 // thread's pixels share an image), which keeps every workgroup full whatever H*W is.
 // grid = ceil(N*H*W / (VEC * 256)) * PC workgroups, the word index fastest: the workgroups that write the PC
 // words of the same pixels run side by side, so their 8- or 16-byte stores meet in L2 as whole lines.
+// The form of one pixel a thread serves tensors too small to fill the chip otherwise: bound by the round trip of its
+// loads, it requests the whole word's 64 channels at once (two batches of 32 took one round trip more).
 template <int BITS, int VEC>
-__global__ __launch_bounds__(kThreads) void quantize_nchw(const float *__restrict__ x, const float *__restrict__ ths,
+__global__ __launch_bounds__(kThreads) void quantize_nchw(const float *__restrict__ x, const Thresholds ths,
                                                           uint64_t *__restrict__ q, int N, int C, long HW, int PC, int32_t *btn)
 {
     typedef float vec_t __attribute__((ext_vector_type(VEC)));
+    constexpr int kInFlight = VEC == 1 ? 64 : 8, kTail = VEC == 1 ? 16 : 8;  // loads of a batch; of a batch of a partial word
     const int pc = blockIdx.x % PC;
-    const long g0 = ((long)(blockIdx.x / PC) * kThreads + threadIdx.x) * VEC;  // first pixel, counted through all images
-    if (g0 >= (long)N * HW) return;
+    const long total = (long)N * HW;
+    const long mine = ((long)(blockIdx.x / PC) * kThreads + threadIdx.x) * VEC;  // first pixel, counted through all images
+    const bool live = mine < total;
+    const long g0 = live ? mine : total - VEC;  // lanes past the end repeat the last pixels and store nothing
     const long n = g0 / HW, s0 = g0 - n * HW;
-    const float t = ths[n];
     const int c0 = pc * kWordBits;
     const int channels = C - c0 < kWordBits ? C - c0 : kWordBits;
     const float *src = x + (n * C + c0) * HW + s0;
     uint64_t sign[VEC], nz[VEC];
 #pragma unroll
     for (int e = 0; e < VEC; e++) sign[e] = nz[e] = 0;
-    constexpr int kInFlight = VEC == 1 ? 32 : 8;  // the one-pixel form serves small, latency-bound tensors
-    auto step = [&](const int j0) {
-        float v[kInFlight][VEC];
+    float v[kInFlight][VEC];
+    auto load = [&](const int j0, auto count) {
 #pragma unroll
-        for (int u = 0; u < kInFlight; u++) {
+        for (int u = 0; u < decltype(count)::value; u++) {
             const int j = j0 + u < channels ? j0 + u : channels - 1;  // clamped: the bit is masked below
             if (VEC == 1) {
-                v[u][0] = src[(long)j * HW];  // the one-pixel form serves small tensors, likely cache-resident: plain loads
+                v[u][0] = src[(long)j * HW];  // small tensors, likely cache-resident: plain loads
             } else {
                 const vec_t w = __builtin_nontemporal_load(reinterpret_cast<const vec_t *>(src + (long)j * HW));
 #pragma unroll
                 for (int e = 0; e < VEC; e++) v[u][e] = w[e];
             }
         }
+    };
+    float t = 0.f;
+    auto pack = [&](const int j0, auto count) {
 #pragma unroll
-        for (int u = 0; u < kInFlight; u++) {
+        for (int u = 0; u < decltype(count)::value; u++) {
             const uint64_t bit = j0 + u < channels ? (uint64_t)1 << (j0 + u) : 0;
 #pragma unroll
             for (int e = 0; e < VEC; e++) {
@@ -367,12 +373,32 @@ __global__ __launch_bounds__(kThreads) void quantize_nchw(const float *__restric
             }
         }
     };
+    // the threshold is looked up (or added up) while the first batch is in flight
+    auto threshold = [&]() {
+        const long n_first = (long)__builtin_amdgcn_readfirstlane((int)n);
+        t = __all(n == n_first) ? wave_threshold(ths, n_first) : lane_threshold(ths, n);
+    };
     if (channels == kWordBits) {  // a whole word: unrolled, every bit position a constant
+        using Batch = std::integral_constant<int, kInFlight>;
+        load(0, Batch());
+        threshold();
+        pack(0, Batch());
 #pragma unroll
-        for (int j0 = 0; j0 < kWordBits; j0 += kInFlight) step(j0);
+        for (int j0 = kInFlight; j0 < kWordBits; j0 += kInFlight) {
+            load(j0, Batch());
+            pack(j0, Batch());
+        }
     } else {
-        for (int j0 = 0; j0 < channels; j0 += kInFlight) step(j0);
+        using Batch = std::integral_constant<int, kTail>;
+        load(0, Batch());
+        threshold();
+        pack(0, Batch());
+        for (int j0 = kTail; j0 < channels; j0 += kTail) {
+            load(j0, Batch());
+            pack(j0, Batch());
+        }
     }
+    if (!live) return;
 #pragma unroll
     for (int e = 0; e < VEC; e++) {
         const long pixel = g0 + e;
@@ -395,7 +421,7 @@ __global__ __launch_bounds__(kThreads) void quantize_nchw(const float *__restric
 // One wave per workgroup (with four, the 784 workgroups of that tensor load the CUs 4 : 3), 4 KB of LDS, gone through
 // in WPP / 2 rounds of 64 / rounds lanes each.  grid = ceil(N*H*W / 256) * (PC / U), the word group fastest.
 template <int BITS, int U>
-__global__ __launch_bounds__(64) void quantize_nchw_gather(const float *__restrict__ x, const float *__restrict__ ths,
+__global__ __launch_bounds__(64) void quantize_nchw_gather(const float *__restrict__ x, const Thresholds ths,
                                                                  uint64_t *__restrict__ q, int N, int C, long HW, int PC, int32_t *btn)
 {
     constexpr int VEC = 4, kInFlight = 8;
@@ -413,7 +439,6 @@ __global__ __launch_bounds__(64) void quantize_nchw_gather(const float *__restri
     const long mine = wave_pixel0 + lane * VEC;
     const long g0 = mine < total ? mine : wave_pixel0;  // lanes past the end repeat the wave's first pixels and store nothing
     const long n = g0 / HW, s0 = g0 - n * HW;
-    const float t = ths[n];
     // The U words are U * 64 consecutive channels: batches of kInFlight channels, the next batch's loads issued before
     // the compares of this one (two register buffers), so the memory pipe never waits for the packing.
     const int cbase = pc0 * kWordBits;
@@ -430,6 +455,7 @@ __global__ __launch_bounds__(64) void quantize_nchw_gather(const float *__restri
     };
     uint64_t words[VEC][WPP];
     uint64_t sign[VEC], nz[VEC];
+    float t;
     auto pack = [&](const float (&v)[kInFlight][VEC], const int b) {
         uint32_t s[VEC], z[VEC];
 #pragma unroll
@@ -459,6 +485,8 @@ __global__ __launch_bounds__(64) void quantize_nchw_gather(const float *__restri
     constexpr int kBatches = kWordBits / kInFlight;  // per word
     float v0[kInFlight][VEC], v1[kInFlight][VEC];
     load(v0, 0);
+    const long n_first = (long)__builtin_amdgcn_readfirstlane((int)n);
+    t = __all(n == n_first) ? wave_threshold(ths, n_first) : lane_threshold(ths, n);
 #pragma unroll
     for (int u = 0; u < U; u++) {
 #pragma unroll
@@ -556,9 +584,11 @@ __global__ __launch_bounds__(kCountThreads) void btn_popcount(const ulonglong2 *
 // workgroups per item each reduce a contiguous slice to one fp32 partial (per-thread serial
 // sums of float4, then a tree over lanes and waves), then one thread per item adds the
 // partials in index order in fp64.
-__global__ __launch_bounds__(kThreads) void abs_sum_partial(const float *__restrict__ x, float *__restrict__ partial,
-                                                            long per_item, int splits)
+// An item of one slice is finished here: `out` gets its threshold, not its sum.
+__global__ __launch_bounds__(kThreads) void abs_sum_partial(const float *__restrict__ x, float *__restrict__ out,
+                                                            long per_item, int splits, double scale_over_count)
 {
+    constexpr int kLoads = 4;  // in flight per lane
     __shared__ float wave_part[kWavesPerBlock];
     const long item = blockIdx.x / splits;
     const int split = blockIdx.x % splits;
@@ -571,11 +601,19 @@ __global__ __launch_bounds__(kThreads) void abs_sum_partial(const float *__restr
     if (((uintptr_t)(src + begin) & 15) == 0) {
         const long n4 = begin < end ? (end - begin) / 4 : 0;
         const floatx4 *src4 = reinterpret_cast<const floatx4 *>(src + begin);
-        for (long i = threadIdx.x; i < n4; i += kThreads) {
-            const floatx4 v = __builtin_nontemporal_load(&src4[i]);
+        auto add = [&](const floatx4 v) {
             sum += (__builtin_fabsf(v[0]) + __builtin_fabsf(v[1])) + (__builtin_fabsf(v[2]) + __builtin_fabsf(v[3]));
+        };
+        long i = threadIdx.x;
+        for (; i + (kLoads - 1) * kThreads < n4; i += kLoads * kThreads) {
+            floatx4 v[kLoads];
+#pragma unroll
+            for (int u = 0; u < kLoads; u++) v[u] = __builtin_nontemporal_load(&src4[i + u * kThreads]);
+#pragma unroll
+            for (int u = 0; u < kLoads; u++) add(v[u]);
         }
-        for (long i = begin + n4 * 4 + threadIdx.x; i < end; i += kThreads) sum += __builtin_fabsf(src[i]);
+        for (; i < n4; i += kThreads) add(__builtin_nontemporal_load(&src4[i]));
+        for (i = begin + n4 * 4 + threadIdx.x; i < end; i += kThreads) sum += __builtin_fabsf(src[i]);
     } else {
         for (long i = begin + threadIdx.x; i < end; i += kThreads) sum += __builtin_fabsf(src[i]);
     }
@@ -587,18 +625,16 @@ __global__ __launch_bounds__(kThreads) void abs_sum_partial(const float *__restr
         float total = 0.f;
 #pragma unroll
         for (int w = 0; w < kWavesPerBlock; w++) total += wave_part[w];
-        partial[blockIdx.x] = total;
+        out[blockIdx.x] = splits == 1 ? (float)((double)total * scale_over_count) : total;
     }
 }
 
-__global__ void abs_mean_finish(const float *__restrict__ partial, float *__restrict__ ths, long items, int splits,
-                                double scale_over_count)
+// One wave per item.  (One thread per item, adding its partial sums one dependent load after the other, took 5.8 us for 32
+// items of 64 slices.)
+__global__ __launch_bounds__(64) void abs_mean_finish(const Thresholds source, float *__restrict__ ths)
 {
-    const long n = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= items) return;
-    double total = 0.0;
-    for (int s = 0; s < splits; s++) total += (double)partial[n * splits + s];
-    ths[n] = (float)(total * scale_over_count);
+    const float t = wave_threshold(source, blockIdx.x);
+    if (threadIdx.x == 0) ths[blockIdx.x] = t;
 }
 
 }  // namespace
@@ -610,14 +646,30 @@ int threshold_splits(long items, long per_item)
     return splits;
 }
 
+hipError_t launch_abs_sums(const float *x, long items, long per_item, float scale, float *partial, Thresholds *source,
+                           hipStream_t stream)
+{
+    const int splits = threshold_splits(items, per_item);
+    source->values = partial;
+    source->scale = (double)scale / (double)per_item;
+    source->splits = splits == 1 ? 0 : splits;
+    abs_sum_partial<<<dim3((unsigned)(items * splits)), dim3(kThreads), 0, stream>>>(x, partial, per_item, splits, source->scale);
+    return hipGetLastError();
+}
+
+hipError_t launch_threshold_values(const Thresholds &source, long items, float *ths, hipStream_t stream)
+{
+    abs_mean_finish<<<dim3((unsigned)items), dim3(64), 0, stream>>>(source, ths);
+    return hipGetLastError();
+}
+
 hipError_t launch_threshold(const float *x, long items, long per_item, float scale, float *ths, float *partial,
                             hipStream_t stream)
 {
-    const int splits = threshold_splits(items, per_item);
-    abs_sum_partial<<<dim3((unsigned)(items * splits)), dim3(kThreads), 0, stream>>>(x, partial, per_item, splits);
-    abs_mean_finish<<<dim3((unsigned)((items + 255) / 256)), dim3(256), 0, stream>>>(partial, ths, items, splits,
-                                                                                   (double)scale / (double)per_item);
-    return hipGetLastError();
+    Thresholds source;
+    if (threshold_splits(items, per_item) == 1) return launch_abs_sums(x, items, per_item, scale, ths, &source, stream);
+    const hipError_t e = launch_abs_sums(x, items, per_item, scale, partial, &source, stream);
+    return e != hipSuccess ? e : launch_threshold_values(source, items, ths, stream);
 }
 
 // Workgroups per item of btn_popcount: enough to fill the chip twice over, none with less than a load a thread.
@@ -638,7 +690,7 @@ void launch_btn_popcount(const uint64_t *qx, int32_t *btn, long items, long word
 }
 
 template <int LP>
-void launch_quantize_groups_of(const float *x, const float *ths, int bitwidth, long rows, long pixels_per_item, int C, int PC,
+void launch_quantize_groups_of(const float *x, const Thresholds &ths, int bitwidth, long rows, long pixels_per_item, int C, int PC,
                                uint32_t *q, int32_t *btn, long items, hipStream_t stream)
 {
     const long per_block = (long)kWavesPerBlock * (64 / LP) * 8;
@@ -650,7 +702,7 @@ void launch_quantize_groups_of(const float *x, const float *ths, int bitwidth, l
 }
 
 // The general-path kernel with the smallest group of lanes whose 4 channels a lane cover the widest word.
-void launch_quantize_groups(const float *x, const float *ths, int bitwidth, long rows, long pixels_per_item, int C, int PC,
+void launch_quantize_groups(const float *x, const Thresholds &ths, int bitwidth, long rows, long pixels_per_item, int C, int PC,
                             uint32_t *q, int32_t *btn, long items, hipStream_t stream)
 {
     const int widest = C < kWordBits ? C : kWordBits;
@@ -663,7 +715,7 @@ void launch_quantize_groups(const float *x, const float *ths, int bitwidth, long
 
 // x: fp32 [items][pixels_per_item][C]; qx: [items*pixels_per_item][PC][bitwidth];
 // btn: [items] or nullptr (then no counts are produced).
-hipError_t launch_quantize(const float *x, const float *ths, int bitwidth, long pixels_per_item,
+hipError_t launch_quantize(const float *x, const Thresholds &ths, int bitwidth, long pixels_per_item,
                            long items, int C, uint64_t *qx, int32_t *btn, hipStream_t stream)
 {
     const int PC = (C + kWordBits - 1) / kWordBits;
@@ -711,7 +763,7 @@ hipError_t launch_quantize(const float *x, const float *ths, int bitwidth, long 
     return hipGetLastError();
 }
 
-hipError_t launch_quantize_nchw(const float *x, const float *ths, int bitwidth, int N, int C, long HW, uint64_t *qx,
+hipError_t launch_quantize_nchw(const float *x, const Thresholds &ths, int bitwidth, int N, int C, long HW, uint64_t *qx,
                                 int32_t *btn, hipStream_t stream)
 {
     const int PC = (C + kWordBits - 1) / kWordBits;
@@ -746,9 +798,10 @@ hipError_t launch_quantize_nchw(const float *x, const float *ths, int bitwidth, 
     return hipGetLastError();
 }
 
-hipError_t launch_quantize_format(const float *x, const float *ths, int format, long pixels_per_item, long items, int C,
+hipError_t launch_quantize_format(const float *x, const float *ths_values, int format, long pixels_per_item, long items, int C,
                                   uint64_t *qx, hipStream_t stream)
 {
+    const Thresholds ths = given_thresholds(ths_values);
     const int PC = format == 5 ? (C + 31) / 32 : (C + kWordBits - 1) / kWordBits;
     const long pixels = items * pixels_per_item;
     if (format != 4 && format != 5) return hipErrorInvalidValue;
@@ -793,7 +846,7 @@ bool quantize_strided_supported(const float *x, int H, int W, int C, int OH, int
     return C % kWordBits == 0 && (uintptr_t)x % 16 == 0 && OW * PC < 65536 && PC < 65536;
 }
 
-hipError_t launch_quantize_strided(const float *x, const float *ths, int bitwidth, int N, int H, int W, int C, int OH,
+hipError_t launch_quantize_strided(const float *x, const Thresholds &ths, int bitwidth, int N, int H, int W, int C, int OH,
                                    int OW, int s1, int s2, uint64_t *qx, hipStream_t stream)
 {
     const int PC = C / kWordBits;

@@ -10,7 +10,10 @@
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/hip/HIPCachingAllocator.h>
 
+#include <array>
+#include <memory>
 #include <stdexcept>
+#include <tuple>
 #include <vector>
 
 #include "../../include/tab_amd.h"
@@ -313,8 +316,198 @@ torch::Tensor TAB_Conv2dPackedOut(const torch::Tensor &QX, const torch::Tensor &
     return QY;
 }
 
+// ---- the layers of tab_amd/nn.py: a forward pass is one call from Python ---------------------------------------------
+// Attribute reads, buffer look-ups, a module call, views, an array of zeros and a Python call per operator made some 10 us
+// of host work a layer around kernels of 6-30 us; here the module's attributes are read from its dictionaries (30 ns each).
+
+namespace {
+
+namespace py = pybind11;
+
+// module.<name>, from the module's own dictionary where it is there (nn.Module attributes that are no submodules, parameters
+// or buffers are)
+py::object attribute(py::handle module, py::handle name)
+{
+    PyObject **dict = _PyObject_GetDictPtr(module.ptr());
+    if (dict != nullptr && *dict != nullptr) {
+        PyObject *item = PyDict_GetItemWithError(*dict, name.ptr());
+        if (item != nullptr) return py::reinterpret_borrow<py::object>(item);
+        if (PyErr_Occurred()) throw py::error_already_set();
+    }
+    return py::reinterpret_steal<py::object>(PyObject_GetAttr(module.ptr(), name.ptr()));
+}
+
+PyObject *interned(const char *name) { return PyUnicode_InternFromString(name); }
+
+torch::Tensor buffer(py::handle module, py::handle name)
+{
+    static PyObject *const buffers_name = interned("_buffers");
+    const py::object buffers = attribute(module, buffers_name);
+    PyObject *item = PyDict_Check(buffers.ptr()) ? PyDict_GetItemWithError(buffers.ptr(), name.ptr()) : nullptr;
+    const py::object t = item != nullptr ? py::reinterpret_borrow<py::object>(item)
+                                         : py::reinterpret_steal<py::object>(PyObject_GetAttr(module.ptr(), name.ptr()));
+    return t.cast<torch::Tensor>();
+}
+
+int integer(py::handle module, py::handle name) { return attribute(module, name).cast<int>(); }
+
+std::pair<int, int> pair_of(py::handle module, py::handle name)
+{
+    const py::object v = attribute(module, name);
+    return {v[py::int_(0)].cast<int>(), v[py::int_(1)].cast<int>()};
+}
+
+// What a TABConv2d module holds.
+struct Layer {
+    torch::Tensor QW, btn;
+    int type, C, KN, KH, KW, s1, s2, p1, p2;
+    double act_scale;
+
+    explicit Layer(py::handle m)
+    {
+        static PyObject *const n_qw = interned("QW"), *const n_btn = interned("BTN_W"), *const n_type = interned("conv_type"),
+                               *const n_in = interned("in_channels"), *const n_out = interned("out_channels"),
+                               *const n_kernel = interned("kernel_size"), *const n_stride = interned("stride"),
+                               *const n_padding = interned("padding"), *const n_scale = interned("act_scale");
+        QW = buffer(m, n_qw);
+        btn = buffer(m, n_btn);
+        type = integer(m, n_type);
+        C = integer(m, n_in);
+        KN = integer(m, n_out);
+        std::tie(KH, KW) = pair_of(m, n_kernel);
+        std::tie(s1, s2) = pair_of(m, n_stride);
+        std::tie(p1, p2) = pair_of(m, n_padding);
+        act_scale = attribute(m, n_scale).cast<double>();
+    }
+
+    int act_bits() const { return type < 2 ? 2 : 1; }
+
+    // checks against an activation of N images of H x W on X's device; returns (OH, OW)
+    std::pair<int, int> check(const torch::Tensor &X, int N, int H, int W) const
+    {
+        CHECK_INPUT(QW);
+        CHECK_INPUT(btn);
+        CHECK_DTYPE(QW, kInt64);
+        CHECK_DTYPE(btn, kInt32);
+        TORCH_CHECK(QW.device() == X.device() && btn.device() == X.device(), "X, QW and btn must be on the same device");
+        return check_conv(QW, btn, type, p1, p2, s1, s2, N, H, W, C, KN, KH, KW);
+    }
+};
+
+// The input as contiguous fp32, what the kernels take.
+torch::Tensor plain_input(const torch::Tensor &x)
+{
+    const torch::Tensor X = x.scalar_type() == torch::kFloat32 ? (x.is_contiguous() ? x : x.contiguous()) : x.to(torch::kFloat32).contiguous();
+    CHECK_CUDA(X);
+    return X;
+}
+
+// (N, H, W, C) of a four-dimensional activation; C checked against the layer's.
+std::array<int, 4> activation_sizes(const torch::Tensor &x, bool nchw, int channels)
+{
+    if (x.dim() != 4) throw py::value_error("expected an activation of four dimensions, got " + std::to_string(x.dim()));
+    const std::array<int, 4> s = nchw ? std::array<int, 4>{(int)x.size(0), (int)x.size(2), (int)x.size(3), (int)x.size(1)}
+                                      : std::array<int, 4>{(int)x.size(0), (int)x.size(1), (int)x.size(2), (int)x.size(3)};
+    TORCH_CHECK(s[3] == channels, "expected ", channels, " input channels, got ", s[3]);
+    return s;
+}
+
+// A layer's fp32 output: memory (n, oh, ow, kn) (TAB_GEMM.cu:526), shaped NHWC or, as a strided tensor, NCHW.
+torch::Tensor layer_output(const torch::Tensor &X, bool nchw, int64_t N, int64_t OH, int64_t OW, int64_t KN)
+{
+    if (!nchw) return device_empty({N, OH, OW, KN}, torch::kFloat32, X);
+    return at::detail::empty_strided_cuda({N, KN, OH, OW}, {OH * OW * KN, 1, OW * KN, KN}, torch::kFloat32, X.device());
+}
+
+void run_layer(const Layer &l, const torch::Tensor &X, bool nchw, int N, int H, int W, const torch::Tensor &y)
+{
+    const hipStream_t stream = current_stream(X);
+    const size_t ws_bytes = tab_layer_workspace_bytes(l.act_bits(), N, H, W, l.C);
+    const Workspace ws(ws_bytes, stream);
+    check_status(tab_layer_conv2d(X.data_ptr<float>(), nchw, (float)l.act_scale, l.QW.data_ptr<int64_t>(), l.btn.data_ptr<int32_t>(),
+                                  l.type, l.p1, l.p2, l.s1, l.s2, N, H, W, l.C, l.KN, l.KH, l.KW, y.data_ptr<float>(), ws.get(),
+                                  ws_bytes, stream));
+}
+
+// TABConv2d.forward
+torch::Tensor layer_forward(py::handle module, const torch::Tensor &x, bool nchw)
+{
+    const Layer l(module);
+    const auto [N, H, W, C] = activation_sizes(x, nchw, l.C);
+    const torch::Tensor X = plain_input(x);
+    const auto [OH, OW] = l.check(X, N, H, W);
+    const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(X.device());
+    const torch::Tensor y = layer_output(X, nchw, N, OH, OW, l.KN);
+    run_layer(l, X, nchw, N, H, W, y);
+    return y;
+}
+
+// TABLinear.forward around a TABConv2d: (N, F) as N images of one pixel
+torch::Tensor linear_forward(py::handle conv, const torch::Tensor &x)
+{
+    const Layer l(conv);
+    if (x.dim() != 2) throw py::value_error("expected an input of two dimensions, got " + std::to_string(x.dim()));
+    const int N = (int)x.size(0);
+    TORCH_CHECK(x.size(1) == l.C, "expected ", l.C, " input channels, got ", x.size(1));
+    const torch::Tensor X = plain_input(x);
+    const auto [OH, OW] = l.check(X, N, 1, 1);
+    TORCH_CHECK(OH == 1 && OW == 1, "a linear layer's convolution maps one pixel to one pixel, got ", OH, " x ", OW);
+    const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(X.device());
+    const torch::Tensor y = device_empty({N, l.KN}, torch::kFloat32, X);
+    run_layer(l, X, false, N, 1, 1, y);
+    return y;
+}
+
+// TABPackedChain.forward: packed activations between the layers, in raw blocks of the caching allocator
+torch::Tensor chain_forward(const py::list &modules, const py::dict &ternary_thresholds, bool nchw, const torch::Tensor &x)
+{
+    std::vector<Layer> layers;
+    layers.reserve(modules.size());
+    for (const py::handle m : modules) layers.emplace_back(m);
+    const Layer &first = layers.front();
+    auto [N, H, W, C] = activation_sizes(x, nchw, first.C);
+    const torch::Tensor X = plain_input(x);
+    const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(X.device());
+    const hipStream_t stream = current_stream(X);
+    const auto packed_bytes = [N = N](int H, int W, int C, int bits) { return (size_t)N * H * W * tab_packed_channels(C) * bits * 8; };
+
+    first.check(X, N, H, W);
+    const size_t ws_bytes = first.act_bits() == 2 ? tab_threshold_workspace_bytes(N, (long)H * W * C) : 4;
+    auto q = std::make_unique<Workspace>(packed_bytes(H, W, C, first.act_bits()), stream);
+    {
+        const Workspace ws(ws_bytes, stream);
+        check_status(tab_layer_quantize(X.data_ptr<float>(), nchw, first.act_bits(), (float)first.act_scale, N, H, W, C,
+                                        static_cast<int64_t *>(q->get()), ws.get(), ws_bytes, stream));
+    }
+    for (size_t i = 0;; i++) {
+        const Layer &l = layers[i];
+        const auto [OH, OW] = l.check(X, N, H, W);
+        const int64_t *in = static_cast<const int64_t *>(q->get());
+        if (i + 1 == layers.size()) {
+            const torch::Tensor y = layer_output(X, nchw, N, OH, OW, l.KN);
+            check_status(tab_conv2d_packed(in, l.QW.data_ptr<int64_t>(), l.btn.data_ptr<int32_t>(), l.type, l.p1, l.p2, l.s1, l.s2, N, H,
+                                           W, l.C, l.KN, l.KH, l.KW, y.data_ptr<float>(), stream));
+            return y;
+        }
+        const py::int_ key(i + 1);
+        const float th = ternary_thresholds.contains(key) ? (float)(double)py::float_(py::object(ternary_thresholds[key])) : 0.f;
+        const int bits = layers[i + 1].act_bits();
+        auto out = std::make_unique<Workspace>(packed_bytes(OH, OW, l.KN, bits), stream);
+        check_status(tab_conv2d_packed_out_const(in, l.QW.data_ptr<int64_t>(), l.btn.data_ptr<int32_t>(), l.type, l.p1, l.p2, l.s1, l.s2,
+                                                 N, H, W, l.C, l.KN, l.KH, l.KW, th, bits, static_cast<int64_t *>(out->get()), stream));
+        q = std::move(out);
+        H = OH;
+        W = OW;
+    }
+}
+
+}  // namespace
+
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
 {
+    m.def("layer_forward", &layer_forward, "nn.TABConv2d.forward");
+    m.def("linear_forward", &linear_forward, "nn.TABLinear.forward");
+    m.def("chain_forward", &chain_forward, "nn.TABPackedChain.forward");
     pybind11::register_exception_translator([](std::exception_ptr p) {
         try {
             if (p) std::rethrow_exception(p);

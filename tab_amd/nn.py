@@ -7,12 +7,18 @@ Inference only (the operators have no backward).
 """
 import torch
 from torch import nn
+from torch.nn.modules.module import _has_any_global_hook
 
-from . import (BNN, BTN, TBN, TNN, Conv2d, Conv2dPacked, Conv2dPackedOut, Quantize, QuantizeActivation, Threshold,
-               out_shape)
+from . import _C, BNN, BTN, TBN, TNN, Quantize, Threshold
 
 _ACT_BITS = {TNN: 2, TBN: 2, BTN: 1, BNN: 1}
 _WEIGHT_BITS = {TNN: 2, TBN: 1, BTN: 2, BNN: 1}
+
+
+def _hooked(module):
+    """Whether calling the module would run more than its forward."""
+    return bool(module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
+                or _has_any_global_hook())
 
 
 def _pair(v):
@@ -52,32 +58,9 @@ class TABConv2d(nn.Module):
         return cls(QW, BTN_W, conv_type, C, KN, (KH, KW), stride, padding, act_scale, data_format)
 
     def forward(self, x):
-        nchw = self.data_format == "NCHW"
-        if nchw:
-            N, C, H, W = x.shape
-        else:
-            N, H, W, C = x.shape
-        if C != self.in_channels:
-            raise RuntimeError(f"expected {self.in_channels} input channels, got {C}")
-        x = x.to(torch.float32).contiguous()
-        abits = _ACT_BITS[self.conv_type]
-        if abits == 2:
-            ths = Threshold(x, N, self.act_scale)  # mean|x| per image: the same in either layout
-        else:
-            ths = torch.zeros(N, dtype=torch.float32, device=x.device)
-        (KH, KW), (s1, s2), (p1, p2) = self.kernel_size, self.stride, self.padding
-        if nchw:
-            # quantized straight from NCHW (no transposed fp32 copy), then the packed entry point
-            QX = QuantizeActivation(x, ths, abits, N, H, W, C, nchw=True)  # no BTN vector: nobody reads an activation's
-            y = Conv2dPacked(QX, self.QW, self.BTN_W, self.conv_type, p1, p2, s1, s2, N, H, W, C,
-                             self.out_channels, KH, KW)
-        else:
-            y = Conv2d(x, self.QW, ths, self.BTN_W, self.conv_type, p1, p2, s1, s2, N, H, W, C,
-                       self.out_channels, KH, KW)
-        OH, OW = out_shape(H, W, KH, KW, p1, p2, s1, s2)
-        # the operator's (N,KN,OH,OW)-shaped result is (n,oh,ow,kn) in memory (TAB_GEMM.cu:526)
-        y = y.view(N, OH, OW, self.out_channels)
-        return y.permute(0, 3, 1, 2) if self.data_format == "NCHW" else y
+        # thresholds, quantizer (straight from NCHW where the input is) and convolution; the operator's output is
+        # (n, oh, ow, kn) in memory (TAB_GEMM.cu:526)
+        return _C.layer_forward(self, x, self.data_format == "NCHW")
 
     def extra_repr(self):
         names = {TNN: "TNN", TBN: "TBN", BTN: "BTN", BNN: "BNN"}
@@ -101,8 +84,11 @@ class TABLinear(nn.Module):
         return cls(conv)
 
     def forward(self, x):
+        conv = self.conv
+        if type(conv) is TABConv2d and conv.data_format == "NHWC" and not _hooked(conv):
+            return _C.linear_forward(conv, x)
         N, F = x.shape
-        return self.conv(x.reshape(N, 1, 1, F)).reshape(N, self.conv.out_channels)
+        return conv(x.reshape(N, 1, 1, F)).reshape(N, conv.out_channels)
 
 
 class TABPackedChain(nn.Module):
@@ -134,26 +120,4 @@ class TABPackedChain(nn.Module):
         self.data_format = data_format
 
     def forward(self, x):
-        nchw = self.data_format == "NCHW"
-        if nchw:
-            N, C, H, W = x.shape
-        else:
-            N, H, W, C = x.shape
-        first = self.layers[0]
-        if C != first.in_channels:
-            raise RuntimeError(f"expected {first.in_channels} input channels, got {C}")
-        x = x.to(torch.float32).contiguous()
-        bits = _ACT_BITS[first.conv_type]
-        ths = Threshold(x, N, first.act_scale) if bits == 2 else torch.zeros(N, dtype=torch.float32, device=x.device)
-        q = QuantizeActivation(x, ths, bits, N, H, W, C, nchw=nchw)
-        for i, layer in enumerate(self.layers):
-            (KH, KW), (s1, s2), (p1, p2) = layer.kernel_size, layer.stride, layer.padding
-            args = (layer.conv_type, p1, p2, s1, s2, N, H, W, layer.in_channels, layer.out_channels, KH, KW)
-            OH, OW = out_shape(H, W, KH, KW, p1, p2, s1, s2)
-            if i + 1 == len(self.layers):
-                y = Conv2dPacked(q, layer.QW, layer.BTN_W, *args).view(N, OH, OW, layer.out_channels)
-                return y.permute(0, 3, 1, 2) if self.data_format == "NCHW" else y
-            next_bits = _ACT_BITS[self.layers[i + 1].conv_type]
-            out_ths = torch.full((N,), float(self.ternary_thresholds.get(i + 1, 0.0)), dtype=torch.float32, device=x.device)
-            q = Conv2dPackedOut(q, layer.QW, layer.BTN_W, *args, out_ths, next_bits)
-            H, W = OH, OW
+        return _C.chain_forward(list(self.layers), self.ternary_thresholds, self.data_format == "NCHW", x)
