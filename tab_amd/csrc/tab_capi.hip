@@ -109,6 +109,7 @@ int tab_internal_conv_shape(int type, int M, int KN, int G, int PC, int packed, 
  * round of the chip; 0 = the device's compute units.  Small values let small test shapes mix whole tiles and quarters. */
 void tab_internal_set_tail_round(int workgroups) { tab::set_tail_round(workgroups); }
 
+
 int tab_set_conv_kernel(int kernel, int tile)
 {
     static const int popcount_tm[4] = {7, 8, 4, 2};  // 7: the popcount kernel's own choice
@@ -333,17 +334,31 @@ static int check_from_floats(const ConvShape &s, int type, const float *dev_X, c
     return check_conv_pointers(s, type, workspace, dev_QW, dev_btn, dev_Y, nullptr);
 }
 
+/* Which kernel takes a call from fp32 in one launch: 0 none, 1 conv1x1_fused, 2 conv_small. */
+static int one_launch(int type, const float *dev_X, bool nchw, int padding1, int padding2, int stride1, int stride2, int N, int H, int W,
+                      int C, int KN, int KH, int KW, const ConvShape &s)
+{
+    if (tab::conv_kernel_forced()) return 0;
+    const bool small = tab::conv_small_supported(type, dev_X, nchw, N, H, W, C, KN, KH, KW, padding1, padding2, stride1, stride2, s.OH, s.OW);
+    // of 1x1 layers both take, conv_small is the sooner one from five words a pixel on (N=64 512->1000 4.8 against 5.4 us),
+    // conv1x1_fused below (64->64 3.8 against 3.0)
+    if (!nchw && !(small && s.PC > 4) && tab::conv1x1_fused_supported(type, dev_X, C, KH, KW, padding1, padding2, s.M, KN)) return 1;
+    return small ? 2 : 0;
+}
+
 /* Quantize an NHWC activation of types 0..3 into the workspace, then the fused conv kernel; small and strided 1x1 layers
  * take their own ways.  The arguments have been checked. */
 static int conv_from_nhwc(const float *dev_X, const int64_t *dev_QW, const tab::Thresholds &ths, const int32_t *dev_btn, int type,
                           int padding1, int padding2, int stride1, int stride2, int N, int H, int W, int C, int KN, int KH, int KW,
                           const ConvShape &s, float *dev_Y, void *workspace, void *stream)
 {
-    // A small 1x1 convolution without padding: quantize and multiply in one launch, the packed activation stays in LDS
-    // (only under the automatic kernel choice: a forced kernel is what the caller wants to see run)
-    if (!tab::conv_kernel_forced() && tab::conv1x1_fused_supported(type, dev_X, C, KH, KW, padding1, padding2, s.M, KN)) {
-        hipError_t e = tab::launch_conv1x1_fused(type, dev_X, ths, reinterpret_cast<const uint64_t *>(dev_QW), dev_btn, dev_Y, N, H,
-                                                 W, C, KN, stride1, stride2, s.OH, s.OW, static_cast<hipStream_t>(stream));
+    // One launch where it pays (only under the automatic kernel choice: a forced kernel is what the caller wants to see run):
+    // a 1x1 convolution without padding, the smallest calls of any kernel.  The packed activation stays in LDS.
+    if (const int one = one_launch(type, dev_X, false, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, s)) {
+        hipError_t e = one == 1 ? tab::launch_conv1x1_fused(type, dev_X, ths, reinterpret_cast<const uint64_t *>(dev_QW), dev_btn, dev_Y, N, H, W,
+                                                            C, KN, stride1, stride2, s.OH, s.OW, static_cast<hipStream_t>(stream))
+                                : tab::launch_conv_small(type, dev_X, false, ths, reinterpret_cast<const uint64_t *>(dev_QW), dev_btn, dev_Y, N, H, W,
+                                                         C, KN, KH, KW, padding1, padding2, stride1, stride2, s.OH, s.OW, static_cast<hipStream_t>(stream));
         if (e != hipSuccess) return device_fail(e, "conv launch");
         return TAB_OK;
     }
@@ -458,7 +473,9 @@ int tab_layer_conv2d(const float *dev_X, int nchw, float act_scale, const int64_
     rc = check_from_floats(s, type, dev_X, dev_QW, dev_btn, dev_Y, workspace, workspace_bytes, tab_layer_workspace_bytes(s.abits, N, H, W, C));
     if (rc != TAB_OK) return rc;
     char *sums = static_cast<char *>(workspace) + layer_packed_bytes(s.abits, N, H, W, C);
-    if (nchw && H * W > 1) {
+    const bool planes = nchw && H * W > 1;  // one pixel per image: NCHW and NHWC are the same memory
+    const int one = one_launch(type, dev_X, planes, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, s);
+    if (planes && !one) {
         rc = tab_layer_quantize(dev_X, 1, s.abits, act_scale, N, H, W, C, static_cast<int64_t *>(workspace), sums,
                                 workspace_bytes - layer_packed_bytes(s.abits, N, H, W, C), stream);
         if (rc != TAB_OK) return rc;
@@ -468,12 +485,18 @@ int tab_layer_conv2d(const float *dev_X, int nchw, float act_scale, const int64_
     tab::Thresholds ths;
     hipError_t e = own_thresholds(dev_X, s.abits, act_scale, N, (long)H * W * C, sums, &ths, stream);
     if (e != hipSuccess) return device_fail(e, "threshold launch");
-    if (ths.splits > 4 && tab::conv1x1_fused_supported(type, dev_X, C, KH, KW, padding1, padding2, s.M, KN)) {
-        // the one-launch 1x1 kernel looks thresholds up lane by lane: with many partial sums an item they are added first
+    if (ths.splits > 4 && (one == 1 || (one == 2 && !tab::conv_small_in_one_image(s.OH, s.OW)))) {
+        // these one-launch kernels look thresholds up lane by lane: with many partial sums an item they are added first
         float *values = reinterpret_cast<float *>(sums + tab_threshold_workspace_bytes(N, (long)H * W * C));
         e = tab::launch_threshold_values(ths, N, values, static_cast<hipStream_t>(stream));
         if (e != hipSuccess) return device_fail(e, "threshold launch");
         ths = tab::given_thresholds(values);
+    }
+    if (planes) {
+        e = tab::launch_conv_small(type, dev_X, true, ths, reinterpret_cast<const uint64_t *>(dev_QW), dev_btn, dev_Y, N, H, W, C, KN, KH, KW,
+                                   padding1, padding2, stride1, stride2, s.OH, s.OW, static_cast<hipStream_t>(stream));
+        if (e != hipSuccess) return device_fail(e, "conv launch");
+        return TAB_OK;
     }
     return conv_from_nhwc(dev_X, dev_QW, ths, dev_btn, type, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, s, dev_Y,
                           workspace, stream);
@@ -493,7 +516,7 @@ int tab_conv2d_launches(const float *dev_X, int type, int padding1, int padding2
 {
     ConvShape s;
     if (check_conv(type, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, &s) != TAB_OK) return 0;
-    return !tab::conv_kernel_forced() && tab::conv1x1_fused_supported(type, dev_X, C, KH, KW, padding1, padding2, s.M, KN) ? 1 : 2;
+    return one_launch(type, dev_X, false, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, s) ? 1 : 2;
 }
 
 size_t tab_static_scratch_bytes(void) { return TAB_STATIC_SCRATCH_BYTES; }

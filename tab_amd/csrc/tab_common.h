@@ -86,8 +86,7 @@ struct ConvArgs {
 // ConvArgs as a kernel receives it.  The host writes kernel arguments into device memory, and from 120 bytes on that costs
 // 0.6-0.8 us a launch (measured launching back to back: 2.8 us up to 112 bytes, 3.4 at 120-128, 3.6-3.9 beyond; ConvArgs
 // itself is 248), a quarter of a small call.  So what a kernel can derive in a few scalar instructions is left out (M and
-// the tile counts), divisors are stored once, and small numbers share a dword: 104 bytes, 112 with packed output or for the
-// mixed launch.  unpack_conv gives the kernels the ConvArgs back; what they do not use of it costs nothing.
+// the tile counts), divisors are stored once, and small numbers share a dword: 104 bytes, 112 with packed output.  unpack_conv gives the kernels the ConvArgs back; what they do not use of it costs nothing.
 struct ConvParams {
     const uint64_t *qx, *qw;
     void *out;             // y or qy
@@ -102,13 +101,7 @@ struct ConvParams {
 struct ConvParamsPacked : ConvParams {
     const float *out_ths;  // or the bits of out_th (kConvOutConstant)
 };
-struct ConvParamsTail : ConvParams {
-    int tail_big, tail_chunks;
-};
-struct ConvParamsPackedTail : ConvParamsPacked {
-    int tail_big, tail_chunks;
-};
-static_assert(sizeof(ConvParams) == 104 && sizeof(ConvParamsPacked) == 112 && sizeof(ConvParamsTail) == 112, "kernel arguments below 120 bytes");
+static_assert(sizeof(ConvParams) == 104 && sizeof(ConvParamsPacked) == 112, "kernel arguments below 120 bytes");
 constexpr uint32_t kConvOutBits2 = 1u << 15;      // packed output of two planes
 constexpr uint32_t kConvOutConstant = 1u << 16;   // one output threshold for every image
 constexpr uint32_t kConvCachedY = 1u << 17;
@@ -116,14 +109,13 @@ constexpr uint32_t kConvXcdOrder = 1u << 18;      // xcd_share != 0
 constexpr uint32_t kConvRowsOrder = 1u << 19;     // tiles_n != 0
 constexpr int kConvKcwShift = 20;                 // kcw, 6 bits
 
-template <bool PACKED, bool TAIL>
-using ConvParamsOf = typename std::conditional<TAIL, typename std::conditional<PACKED, ConvParamsPackedTail, ConvParamsTail>::type,
-                                               typename std::conditional<PACKED, ConvParamsPacked, ConvParams>::type>::type;
+template <bool PACKED>
+using ConvParamsOf = typename std::conditional<PACKED, ConvParamsPacked, ConvParams>::type;
 
-template <int TYPE, bool PACKED, bool TAIL = false>
-ConvParamsOf<PACKED, TAIL> pack_conv(const ConvArgs &a)
+template <int TYPE, bool PACKED>
+ConvParamsOf<PACKED> pack_conv(const ConvArgs &a)
 {
-    ConvParamsOf<PACKED, TAIL> k;
+    ConvParamsOf<PACKED> k;
     k.qx = a.qx;
     k.qw = a.qw;
     k.out = PACKED ? static_cast<void *>(a.qy) : static_cast<void *>(a.y);
@@ -134,7 +126,7 @@ ConvParamsOf<PACKED, TAIL> pack_conv(const ConvArgs &a)
     k.g_chunks = (uint32_t)a.G | (uint32_t)a.nchunks << 16;
     k.magic_pc = a.div_pc.magic;
     k.magic_kw = a.div_kw.magic;
-    const Div32 tiles = a.xcd_share != 0 || TAIL ? a.div_filter_tiles : a.div_tiles_m;
+    const Div32 tiles = a.xcd_share != 0 ? a.div_filter_tiles : a.div_tiles_m;
     k.mul_pixels = a.div_pixels.mul;
     k.mul_ow = a.div_ow.mul;
     k.mul_tiles = tiles.mul;
@@ -146,16 +138,12 @@ ConvParamsOf<PACKED, TAIL> pack_conv(const ConvArgs &a)
         memcpy(&th, &a.out_th, sizeof th);
         k.out_ths = a.out_ths != nullptr ? a.out_ths : reinterpret_cast<const float *>((uintptr_t)th);
     }
-    if constexpr (TAIL) {
-        k.tail_big = a.tail_big;
-        k.tail_chunks = a.tail_chunks;
-    }
     return k;
 }
 
-// BM, BN: the workgroup's tile (of a mixed launch: the whole tile).
-template <int TYPE, bool PACKED, int BM, int BN, bool TAIL = false>
-__device__ __forceinline__ ConvArgs unpack_conv(const ConvParamsOf<PACKED, TAIL> &k)
+// BM, BN: the workgroup's tile.
+template <int TYPE, bool PACKED, int BM, int BN>
+__device__ __forceinline__ ConvArgs unpack_conv(const ConvParamsOf<PACKED> &k)
 {
     ConvArgs a = {};
     a.qx = k.qx;
@@ -187,12 +175,7 @@ __device__ __forceinline__ ConvArgs unpack_conv(const ConvParamsOf<PACKED, TAIL>
         a.out_ths = constant ? nullptr : k.out_ths;
         a.out_th = __uint_as_float((uint32_t)(uintptr_t)k.out_ths);
     }
-    if constexpr (TAIL) {
-        a.tail_big = k.tail_big;
-        a.tail_chunks = k.tail_chunks;
-    }
-    const int tiles = TAIL ? a.tail_big : a.tiles_m * a.filter_tiles;
-    a.xcd_share = k.bits & kConvXcdOrder ? (int)((uint32_t)tiles / 8u) : 0;
+    a.xcd_share = k.bits & kConvXcdOrder ? (int)((uint32_t)(a.tiles_m * a.filter_tiles) / 8u) : 0;
     return a;
 }
 
@@ -257,6 +240,14 @@ hipError_t launch_threshold(const float *x, long items, long per_item, float sca
 bool conv1x1_fused_supported(int type, const float *x, int C, int KH, int KW, int p1, int p2, long M, int KN);
 hipError_t launch_conv1x1_fused(int type, const float *x, const Thresholds &ths, const uint64_t *qw, const int32_t *btn, float *y, int N,
                                 int H, int W, int C, int KN, int s1, int s2, int OH, int OW, hipStream_t stream);
+
+// Quantize + convolution in one launch for the smallest calls (tab_conv_small.hip); x NHWC or NCHW.
+bool conv_small_supported(int type, const float *x, bool nchw, int N, int H, int W, int C, int KN, int KH, int KW, int p1, int p2, int s1,
+                          int s2, int OH, int OW);
+bool conv_small_in_one_image(int OH, int OW);
+hipError_t launch_conv_small(int type, const float *x, bool nchw, const Thresholds &ths, const uint64_t *qw, const int32_t *btn, float *y,
+                             int N, int H, int W, int C, int KN, int KH, int KW, int p1, int p2, int s1, int s2, int OH, int OW,
+                             hipStream_t stream);
 
 void force_conv_tile(int tm, int ng);  // tuning hook: 0,0 restores the automatic choice
 void set_tail_round(int workgroups);   // test hook of the mixed launch: workgroups counted as one round of the chip (0: the CUs)

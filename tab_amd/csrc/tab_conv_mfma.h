@@ -429,7 +429,7 @@ constexpr int conv_mfma_lds_bytes()
 // PACKED: packed output (p.qy): the weights are the first MFMA operand and the epilogue packs inside a lane.
 template <int TYPE, int WM, int WN, int TM, int TN, int KCH, bool INTAP, int KS = 1, bool PACKED = false>
 __global__ __launch_bounds__(kConvThreads)
-__attribute__((amdgpu_waves_per_eu(mfma_waves_per_eu(WM, TM, TN, conv_mfma_lds_bytes<TYPE, WM, WN, TM, TN, KCH, INTAP, KS>())))) void conv_mfma(const ConvParamsOf<PACKED, false> k)
+__attribute__((amdgpu_waves_per_eu(mfma_waves_per_eu(WM, TM, TN, conv_mfma_lds_bytes<TYPE, WM, WN, TM, TN, KCH, INTAP, KS>())))) void conv_mfma(const ConvParamsOf<PACKED> k)
 {
     const ConvArgs p = unpack_conv<TYPE, PACKED, 32 * WM * TM, 32 * WN * TN>(k);
     static_assert(WM * WN * KS * 64 == kConvThreads, "four waves");

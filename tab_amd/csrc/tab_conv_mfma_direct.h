@@ -415,7 +415,7 @@ __device__ __forceinline__ void conv_mfma_direct_tile(const ConvArgs &p, uint32_
 
 template <int TYPE, int WM, int WN, int TM, int TN, int KCH, bool PACKED, int KS = 1, int ARUN = 0>
 __global__ __launch_bounds__(kConvThreads)
-__attribute__((amdgpu_waves_per_eu(mfma_waves_per_eu(KS > 1 ? 1 : WM, TM, TN, 4 * conv_mfma_direct_lds_dwords<TYPE, WM, WN, TM, TN, KCH, KS>())))) void conv_mfma_direct(const ConvParamsOf<PACKED, false> k)
+__attribute__((amdgpu_waves_per_eu(mfma_waves_per_eu(KS > 1 ? 1 : WM, TM, TN, 4 * conv_mfma_direct_lds_dwords<TYPE, WM, WN, TM, TN, KCH, KS>())))) void conv_mfma_direct(const ConvParamsOf<PACKED> k)
 {
     const ConvArgs p = unpack_conv<TYPE, PACKED, 32 * WM * TM, 32 * WN * TN>(k);
     __shared__ __attribute__((aligned(16))) uint32_t lds[conv_mfma_direct_lds_dwords<TYPE, WM, WN, TM, TN, KCH, KS>()];
@@ -431,12 +431,13 @@ __attribute__((amdgpu_waves_per_eu(mfma_waves_per_eu(KS > 1 ? 1 : WM, TM, TN, 4 
 // large tile's ratio of expansions to MFMAs): the last, partial round is dealt out in quarters, so the busiest CU carries at
 // most a quarter tile more than the others.  Workgroups are dispatched in index order, whole tiles first.  Needs an even
 // number of words per pixel.
+// (The arguments come unpacked: these launches are longer than the host's work for the next one, and the unpacking at the
+// start of every workgroup cost 1 %.)
 // TNB = 4: the whole tiles are 128x256 (eight MFMA tiles a wave, the pipelined loop, two workgroups a CU) and a remaining tile
 // makes eight quarters.
 template <int TYPE, int KCH, int ARUN, bool PACKED, int TNB = 2>
-__global__ __launch_bounds__(kConvThreads) __attribute__((amdgpu_waves_per_eu(TNB == 4 ? 2 : 4))) void conv_mfma_tail(const ConvParamsOf<PACKED, true> k)
+__global__ __launch_bounds__(kConvThreads) __attribute__((amdgpu_waves_per_eu(TNB == 4 ? 2 : 4))) void conv_mfma_tail(const ConvArgs p)
 {
-    const ConvArgs p = unpack_conv<TYPE, PACKED, 128, 64 * TNB, true>(k);
     constexpr int BIG = conv_mfma_direct_lds_dwords<TYPE, 2, 2, 2, TNB, KCH, 1>(), SMALL = conv_mfma_direct_lds_dwords<TYPE, 1, 1, 2, 2, 8, 4>();
     __shared__ __attribute__((aligned(16))) uint32_t lds[BIG > SMALL ? BIG : SMALL];
     const uint32_t b = blockIdx.x;
@@ -462,9 +463,9 @@ hipError_t launch_mfma_tail_run(ConvArgs a, long blocks, hipStream_t stream)
     a.nchunks = a.G / KCH;
     a.tail_chunks = (a.G + 7) / 8;  // the quarters' chunks of eight words, the last one padded with zeros
     if (a.qy != nullptr) {
-        conv_mfma_tail<TYPE, KCH, ARUN, true, TNB><<<dim3((unsigned)blocks), dim3(kConvThreads), 0, stream>>>(pack_conv<TYPE, true, true>(a));
+        conv_mfma_tail<TYPE, KCH, ARUN, true, TNB><<<dim3((unsigned)blocks), dim3(kConvThreads), 0, stream>>>(a);
     } else {
-        conv_mfma_tail<TYPE, KCH, ARUN, false, TNB><<<dim3((unsigned)blocks), dim3(kConvThreads), 0, stream>>>(pack_conv<TYPE, false, true>(a));
+        conv_mfma_tail<TYPE, KCH, ARUN, false, TNB><<<dim3((unsigned)blocks), dim3(kConvThreads), 0, stream>>>(a);
     }
     return hipGetLastError();
 }

@@ -43,7 +43,7 @@ enum RegsOut {
 
 // G: words of K per plane (runtime p.G <= G; missing words are zero on both sides), TN: 32-filter tiles per wave.
 template <int TYPE, int G, int TN, int OUT>
-__global__ __launch_bounds__(kConvThreads) __attribute__((amdgpu_waves_per_eu(2, 3))) void conv_mfma_regs(const ConvParamsOf<(OUT >= kOutBits1), false> k)
+__global__ __launch_bounds__(kConvThreads) __attribute__((amdgpu_waves_per_eu(2, 3))) void conv_mfma_regs(const ConvParamsOf<(OUT >= kOutBits1)> k)
 {
     constexpr int APL = Planes<TYPE>::A, BPL = Planes<TYPE>::B;
     static_assert(TYPE >= 0 && TYPE <= 3, "types 0..3");

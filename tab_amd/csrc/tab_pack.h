@@ -107,5 +107,46 @@ __device__ __forceinline__ void pack_row(uint32_t sign, uint32_t nz, int l, uint
     }
 }
 
+// OR over the LP lanes (a power of two up to 16, aligned inside a DPP row) of a group; every lane gets the result.
+template <int LP>
+__device__ __forceinline__ uint32_t or_reduce_group(uint32_t v)
+{
+    if (LP >= 2) v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, true);    // quad_perm [1,0,3,2]
+    if (LP >= 4) v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, true);    // quad_perm [2,3,0,1]
+    if (LP >= 8) v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xF, 0xF, true);   // row_half_mirror
+    if (LP >= 16) v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xF, 0xF, true);  // row_mirror
+    return v;
+}
+
+// The packed element of a word of `channels` channels (at least 64 count as 64) from a group of LP lanes, lane l holding the
+// channels l, l + LP, l + 2 LP, l + 3 LP; every lane of the group gets out[0..1] for MODE 1, out[0..3] for MODE 2.  Bits of
+// channels that do not exist stay 0 (TAB_GEMM.cu:203-206).
+template <int MODE, int LP = 16>
+__device__ __forceinline__ void pack_row_strided(const float (&v)[4], float t, int l, int channels, uint32_t (&out)[4])
+{
+    uint32_t w[4] = {0, 0, 0, 0};  // sign low, sign high, nonzero low, nonzero high
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        const int ch = l + LP * e;
+        const bool valid = ch < channels;
+        const int half = LP * e >= 32 ? 1 : 0;             // LP * e is 0, 16, 32, 48 when channels reach 32
+        const int shift = l + (LP * e - 32 * half);
+        if (MODE == 2) {
+            const bool pos = v[e] > t;
+            const bool neg = !pos && (v[e] < -t);
+            w[half] |= (uint32_t)(valid && neg) << shift;
+            w[2 + half] |= (uint32_t)(valid && (pos || neg)) << shift;
+        } else {
+            w[half] |= (uint32_t)(valid && (v[e] < t)) << shift;
+        }
+    }
+    out[0] = or_reduce_group<LP>(w[0]);
+    out[1] = LP == 16 ? or_reduce_group<LP>(w[1]) : 0u;
+    if (MODE == 2) {
+        out[2] = or_reduce_group<LP>(w[2]);
+        out[3] = LP == 16 ? or_reduce_group<LP>(w[3]) : 0u;
+    }
+}
+
 }  // namespace
 }  // namespace tab

@@ -142,17 +142,6 @@ __global__ __launch_bounds__(64) void quantize_rows64_strided(const floatx4 *__r
     }
 }
 
-// OR over the LP lanes (a power of two up to 16, aligned inside a DPP row) of a group; every lane gets the result.
-template <int LP>
-__device__ __forceinline__ uint32_t or_reduce_group(uint32_t v)
-{
-    if (LP >= 2) v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, true);    // quad_perm [1,0,3,2]
-    if (LP >= 4) v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, true);    // quad_perm [2,3,0,1]
-    if (LP >= 8) v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xF, 0xF, true);   // row_half_mirror
-    if (LP >= 16) v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xF, 0xF, true);  // row_mirror
-    return v;
-}
-
 // General path (any C, any alignment of x; pixels * PC < 2^31): a group of LP lanes takes one (pixel, word) row of
 // up to 4 * LP channels, lane l the channels l, l + LP, l + 2 LP, l + 3 LP of the word (so a wave-wide load reads
 // runs of 4 * LP bytes, and neighbouring groups neighbouring rows); LP = 16 serves words of up to 64 channels,
@@ -197,29 +186,13 @@ __global__ __launch_bounds__(kThreads) void quantize_groups(const float *__restr
     const float t_first = wave_threshold(ths, item_first);
 
     auto finish = [&](int u, float t) {
-        uint32_t w[4] = {0, 0, 0, 0};  // sign low, sign high, nonzero low, nonzero high
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const int ch = l + LP * e;
-            const bool valid = ch < channels[u];
-            const int half = LP * e >= 32 ? 1 : 0;             // LP * e is 0, 16, 32, 48 when channels reach 32
-            const int shift = l + (LP * e - 32 * half);
-            if (BITS == 2) {
-                const bool pos = v[u][e] > t;
-                const bool neg = !pos && (v[u][e] < -t);
-                w[half] |= (uint32_t)(valid && neg) << shift;
-                w[2 + half] |= (uint32_t)(valid && (pos || neg)) << shift;
-            } else {
-                w[half] |= (uint32_t)(valid && (v[u][e] < t)) << shift;
-            }
-        }
+        uint32_t out[4];
+        pack_row_strided<BITS, LP>(v[u], t, l, channels[u], out);
         const long r = row0 + u * GROUPS + group;
-        const uint32_t s_lo = or_reduce_group<LP>(w[0]), s_hi = LP == 16 ? or_reduce_group<LP>(w[1]) : 0u;
         if (BITS == 2) {
-            const uint32_t n_lo = or_reduce_group<LP>(w[2]), n_hi = LP == 16 ? or_reduce_group<LP>(w[3]) : 0u;
-            if (r < rows && l == 0) *reinterpret_cast<uintx4 *>(q + r * 4) = uintx4{s_lo, s_hi, n_lo, n_hi};
+            if (r < rows && l == 0) *reinterpret_cast<uintx4 *>(q + r * 4) = uintx4{out[0], out[1], out[2], out[3]};
         } else {
-            if (r < rows && l == 0) *reinterpret_cast<uintx2 *>(q + r * 2) = uintx2{s_lo, s_hi};
+            if (r < rows && l == 0) *reinterpret_cast<uintx2 *>(q + r * 2) = uintx2{out[0], out[1]};
         }
     };
     if (one_item) {
