@@ -483,7 +483,11 @@ int tab_layer_conv2d(const float *dev_X, int nchw, float act_scale, const int64_
                                  N, H, W, C, KN, KH, KW, dev_Y, stream);
     }
     tab::Thresholds ths;
-    hipError_t e = own_thresholds(dev_X, s.abits, act_scale, N, (long)H * W * C, sums, &ths, stream);
+    hipError_t e = hipSuccess;
+    if (one == 2 && s.abits == 2 && tab::conv_small_own_thresholds(dev_X, H, W, C, KH, KW, padding1, padding2))
+        ths = tab::Thresholds{dev_X, (double)act_scale / (double)C, tab::kOwnPixelThresholds};
+    else
+        e = own_thresholds(dev_X, s.abits, act_scale, N, (long)H * W * C, sums, &ths, stream);
     if (e != hipSuccess) return device_fail(e, "threshold launch");
     if (ths.splits > 4 && (one == 1 || (one == 2 && !tab::conv_small_in_one_image(s.OH, s.OW)))) {
         // these one-launch kernels look thresholds up lane by lane: with many partial sums an item they are added first

@@ -206,6 +206,7 @@ struct Thresholds {
     double scale;
     int splits;
 };
+constexpr int kOwnPixelThresholds = -1;  // splits, conv_small only: images of one pixel, the kernel adds up |x| itself
 inline Thresholds given_thresholds(const float *ths) { return Thresholds{ths, 0.0, 0}; }
 
 hipError_t launch_quantize(const float *x, const Thresholds &ths, int bitwidth, long pixels_per_item,
@@ -245,6 +246,8 @@ hipError_t launch_conv1x1_fused(int type, const float *x, const Thresholds &ths,
 bool conv_small_supported(int type, const float *x, bool nchw, int N, int H, int W, int C, int KN, int KH, int KW, int p1, int p2, int s1,
                           int s2, int OH, int OW);
 bool conv_small_in_one_image(int OH, int OW);
+// Images of one pixel (H = W = 1, a 1x1 kernel without padding): conv_small takes kOwnPixelThresholds.
+bool conv_small_own_thresholds(const float *x, int H, int W, int C, int KH, int KW, int p1, int p2);
 hipError_t launch_conv_small(int type, const float *x, bool nchw, const Thresholds &ths, const uint64_t *qw, const int32_t *btn, float *y,
                              int N, int H, int W, int C, int KN, int KH, int KW, int p1, int p2, int s1, int s2, int OH, int OW,
                              hipStream_t stream);

@@ -80,7 +80,7 @@ __device__ __forceinline__ int half_binary_dword(uint32_t w, int d, const Expand
 // v_bitop3_b32 each); a pair is already the two top bits of an E2M1 nibble, sign and the exponent bit of 2, so dwords 2
 // and 3 are one AND of a pair word and dwords 0 and 1 a shift and an AND.  Dword d holds the elements 4i + d of the
 // slice, as in the binary expansions.  Every ternary element is +-2 or (+-)0; a binary partner is +-0.5 throughout
-// (products +-1), and two ternary sides give four times the sum, which the kernels scale back with scale_ternary_sums
+// (products +-1), and two ternary sides give four times the sum, which the kernels scale back with scale_sums
 // (exact: 4 * 64 * G < 2^24 for every G the library takes).  With separate sign and magnitude masks per dword
 // ((s << k) & sign | (z >> j) & bit) the same operand took 12 instructions (activation side) or 14 (weight side).
 // d = 0 and d = 1 make the pair words and leave them in pw for d = 2 and d = 3.
@@ -112,43 +112,66 @@ __device__ __forceinline__ i32x8 expand_ternary(uint32_t s, uint32_t z, const Ex
     return r;
 }
 
-// TNN: both operands are +-2, the accumulators hold four times the sums
-template <int TYPE, int TM, int TN>
-__device__ __forceinline__ void scale_ternary_sums(f32x16 (&acc)[TM][TN])
+// Type 4 (TAB_CPU.cpp:332-358): planes (hi, lo) of a level 0..3 on both sides.  The E2M1 codes 0000, 0001, 0010, 0011 are 0,
+// 0.5, 1 and 1.5, so a level's two bits, hi above lo, are the nibble of half the level: the pair words of the ternary
+// expansion, with (lo, hi) for (nonzero, sign), masked to the low halves of the nibbles (10 instructions; building 1, 2 and 3
+// themselves took 22).  The products are a quarter of the levels' and multiples of 0.25 below 2^22, exact, and the kernels
+// multiply the sums by four.
+// d = 0 and d = 1 make the pair words and leave them in pw for d = 2 and d = 3, as in ternary_dword.
+__device__ __forceinline__ int level_dword(uint32_t hi, uint32_t lo, int d, uint32_t (&pw)[2], const ExpandConsts &c)
 {
-    if (TYPE != 0) return;
+    if (d == 0) {
+        const uint32_t h1 = hi << 1;
+        uint32_t a = ((lo ^ h1) & c.even) ^ h1;  // bit 2j = lo[2j], bit 2j+1 = hi[2j]
+        asm("" : "+v"(a));
+        pw[0] = a;
+        return (int)(a & ~c.pair);
+    }
+    if (d == 1) {
+        const uint32_t l1 = lo >> 1;
+        uint32_t b = ((hi ^ l1) & c.odd) ^ l1;  // bit 2j = lo[2j+1], bit 2j+1 = hi[2j+1]
+        asm("" : "+v"(b));
+        pw[1] = b;
+        return (int)(b & ~c.pair);
+    }
+    return (int)((pw[d - 2] >> 2) & ~c.pair);
+}
+
+__device__ __forceinline__ i32x8 expand_levels(uint32_t hi, uint32_t lo, const ExpandConsts &c)
+{
+    i32x8 r = {0, 0, 0, 0, 0, 0, 0, 0};
+    uint32_t pw[2];
+#pragma unroll
+    for (int d = 0; d < 4; d++) r[d] = level_dword(hi, lo, d, pw, c);
+    return r;
+}
+
+// Type 5 (TAB_CPU.cpp:362-383): a 32-bit slice holds 16 fields (even bit = nonzero, odd bit = sign).  A field is the two top
+// bits of an E2M1 nibble, sign and the exponent bit of 2: the fields at odd positions of the slice are one AND away from an
+// operand dword, those at even positions a shift and an AND (6 instructions a lane's word; +-1 with the nonzero bit moved to
+// its place took 14).  Every element is +-2 or +-0, the sums four times what they should be, as for TNN.  A slice is 16 of
+// the 32 elements a lane feeds, so a lane takes both halves of one word per MFMA and the two half-waves take alternate words.
+__device__ __forceinline__ i32x8 expand_fields(uint32_t lo, uint32_t hi, const ExpandConsts &c)
+{
+    i32x8 r = {0, 0, 0, 0, 0, 0, 0, 0};
+    r[0] = (int)((lo << 2) & c.pair);
+    r[1] = (int)(lo & c.pair);
+    r[2] = (int)((hi << 2) & c.pair);
+    r[3] = (int)(hi & c.pair);
+    return r;
+}
+
+// What the accumulators of a type are multiplied by: both operands +-2 (TNN, RTN) or half a level (DRF).
+template <int TYPE> constexpr float kSumScale = TYPE == 0 || TYPE == 5 ? 0.25f : (TYPE == 4 ? 4.f : 1.f);
+
+template <int TYPE, int TM, int TN>
+__device__ __forceinline__ void scale_sums(f32x16 (&acc)[TM][TN])
+{
+    if (kSumScale<TYPE> == 1.f) return;
 #pragma unroll
     for (int mt = 0; mt < TM; mt++)
 #pragma unroll
-        for (int nt = 0; nt < TN; nt++) acc[mt][nt] *= 0.25f;
-}
-
-// Type 4 (TAB_CPU.cpp:332-358): planes (hi, lo) of a level 0..3 on both sides; E2M1 holds 1 = 0010,
-// 2 = 0100 and 3 = 0101 exactly, so exponent bit 1 = hi, exponent bit 0 = lo & ~hi, mantissa = hi & lo,
-// and the products (at most 9) and their sums stay exact integers.
-__device__ __forceinline__ i32x8 expand_levels(uint32_t hi, uint32_t lo)
-{
-    const uint32_t one = lo & ~hi, three = hi & lo;
-    i32x8 r = {0, 0, 0, 0, 0, 0, 0, 0};
-    r[0] = (int)(((hi & kBit0) << 2) | ((one & kBit0) << 1) | (three & kBit0));
-    r[1] = (int)(((hi & kBit1) << 1) | (one & kBit1) | ((three & kBit1) >> 1));
-    r[2] = (int)((hi & kBit2) | ((one & kBit2) >> 1) | ((three & kBit2) >> 2));
-    r[3] = (int)(((hi & kBit3) >> 1) | ((one & kBit3) >> 2) | ((three & kBit3) >> 3));
-    return r;
-}
-
-// Type 5 (TAB_CPU.cpp:362-383): a 32-bit slice holds 16 fields (even bit = nonzero, odd bit = sign).
-// The fields at even positions of the slice fill one operand dword, those at odd positions the next,
-// each as the nibble (sign, 0, nonzero, 0) = +-1 or +-0.  A slice is 16 of the 32 elements a lane
-// feeds, so a lane takes both halves of one word per MFMA and the two half-waves take alternate words.
-__device__ __forceinline__ i32x8 expand_fields(uint32_t lo, uint32_t hi)
-{
-    i32x8 r = {0, 0, 0, 0, 0, 0, 0, 0};
-    r[0] = (int)(((lo << 1) & kBit1) | ((lo << 2) & kBit3));
-    r[1] = (int)(((lo >> 1) & kBit1) | (lo & kBit3));
-    r[2] = (int)(((hi << 1) & kBit1) | ((hi << 2) & kBit3));
-    r[3] = (int)(((hi >> 1) & kBit1) | (hi & kBit3));
-    return r;
+        for (int nt = 0; nt < TN; nt++) acc[mt][nt] *= kSumScale<TYPE>;
 }
 
 // The FP4 operand of one MFMA: SIDE 0 = activation, 1 = weight; p0, p1 = the lane's 32-bit slice of
@@ -157,8 +180,8 @@ __device__ __forceinline__ i32x8 expand_fields(uint32_t lo, uint32_t hi)
 template <int TYPE, int SIDE>
 __device__ __forceinline__ i32x8 expand_operand(uint32_t p0, uint32_t p1, const ExpandConsts &c)
 {
-    if (TYPE == 4) return expand_levels(p0, p1);
-    if (TYPE == 5) return expand_fields(p0, p1);
+    if (TYPE == 4) return expand_levels(p0, p1, c);
+    if (TYPE == 5) return expand_fields(p0, p1, c);
     constexpr int PL = SIDE ? Planes<TYPE>::B : Planes<TYPE>::A;
     if (PL == 2) return expand_ternary(p0, p1, c);
     if (TYPE == 3) return expand_binary<SIDE>(p0, c);
@@ -538,7 +561,7 @@ __attribute__((amdgpu_waves_per_eu(mfma_waves_per_eu(WM, TM, TN, conv_mfma_lds_b
         __syncthreads();
     }
 
-    scale_ternary_sums<TYPE>(acc);
+    scale_sums<TYPE>(acc);
     if constexpr (PACKED)  // (the chunk loop ends on a barrier: the operand buffers are free for BTN's exchange of biases)
         conv_mfma_epilogue_packed<TYPE, TM, TN, KCH>(p, acc, b_nonzero, wave_m0, wave_n0, lane, lds + wave * (32 * TN), p.nchunks * KCH);
     else

@@ -237,6 +237,8 @@ __device__ __forceinline__ void conv_mfma_direct_tile(const ConvArgs &p, uint32_
             const uint32_t *w = a_w[pair & 1][mt];
             if constexpr (TYPE <= 2)
                 af[set][mt][d] = APL == 2 ? ternary_dword(w[h], w[2 + h], d, pair_words, consts) : half_binary_dword(w[h], d, consts);
+            else if constexpr (TYPE == 4)
+                af[set][mt][d] = level_dword(w[h], w[2 + h], d, pair_words, consts);
             else
                 af[set][mt][d] = expand_operand<TYPE, 0>(w[h], w[2 * (APL - 1) + h], consts)[d];
         } else {
@@ -244,6 +246,8 @@ __device__ __forceinline__ void conv_mfma_direct_tile(const ConvArgs &p, uint32_
             const uint32_t *w = b_w[pair & 1][nt];
             if constexpr (TYPE <= 2)
                 bf[set][nt][d] = BPL == 2 ? ternary_dword(w[h], w[2 + h], d, pair_words, consts) : half_binary_dword(w[h], d, consts);
+            else if constexpr (TYPE == 4)
+                bf[set][nt][d] = level_dword(w[h], w[2 + h], d, pair_words, consts);
             else
                 bf[set][nt][d] = expand_operand<TYPE, 1>(w[h], w[2 * (BPL - 1) + h], consts)[d];
             if (TYPE == 2 && d == 0) b_nonzero[nt] += __builtin_popcount(w[2 + h]);  // (the zeros past the last chunk add nothing)
@@ -354,7 +358,7 @@ __device__ __forceinline__ void conv_mfma_direct_tile(const ConvArgs &p, uint32_
             __syncthreads();
         }
     }
-    scale_ternary_sums<TYPE>(acc);
+    scale_sums<TYPE>(acc);
     if constexpr (KS > 1) {
         // The KS groups hold partial sums of the same tiles.  Rounds of kSplitRoundTiles tiles: every wave deposits its
         // part of the round's tiles (and BTN's partial count of nonzero weight bits), the wave group (round's tile) % KS

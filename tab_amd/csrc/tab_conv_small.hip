@@ -133,7 +133,7 @@ __global__ __launch_bounds__(kConvThreads) void conv_small(const SmallConvArgs p
         const int ih = oh * s1 - p1 + kh, iw = ow * s2 - p2 + kw;
         const bool ok = line < lines && (unsigned)ih < (unsigned)p.H && (unsigned)iw < (unsigned)p.W && n < p.N;
         pixel_of[slot] = ok ? (n * p.H + ih) * p.W + iw : -1;  // < 2^31 (launch check)
-        if (!own_image) th_of[slot] = lane_threshold(p.ths, ok ? n : 0);
+        if (!own_image && p.ths.splits >= 0) th_of[slot] = lane_threshold(p.ths, ok ? n : 0);
     }
     for (int g = tid; g < chunks * PAIRS * 2; g += kConvThreads) {
         const int tap = (int)fastdiv((uint32_t)g, FastDiv{p.magic_pc, (uint32_t)PC}), kh = tap / KW;
@@ -141,6 +141,43 @@ __global__ __launch_bounds__(kConvThreads) void conv_small(const SmallConvArgs p
     }
     const float t_image = own_image ? wave_threshold(p.ths, n0) : 0.f;
     __syncthreads();
+    if constexpr (INPUT == kNhwcWords && APL == 2) {
+        if (p.ths.splits == kOwnPixelThresholds) {
+            // Images of one pixel: a 16-lane row adds up |x| of its slot's image, in the order of abs_sum_partial (whose 256
+            // threads take every 256th float4, i.e. every 16th word: words w, w + 16, ... in turn, then a tree over the four
+            // words of a wave, then the waves), so that the thresholds are the same to the last bit.
+            const int slot = wave * 4 + q;
+            const int pixel = slot < slots ? pixel_of[slot] : -1;
+            const float *src = p.x + (size_t)(uint32_t)(pixel < 0 ? 0 : pixel) * p.C + r * 4;
+            float sum[4][4];
+#pragma unroll
+            for (int b = 0; b < 4; b++)
+#pragma unroll
+                for (int w = 0; w < 4; w++) sum[b][w] = 0.f;
+            for (int w0 = 0; w0 < PC; w0 += 16)
+#pragma unroll
+                for (int b = 0; b < 4; b++) {
+                    if (w0 + 4 * b >= PC) break;  // uniform
+#pragma unroll
+                    for (int w = 0; w < 4; w++) {
+                        const int word = w0 + 4 * b + w;
+                        const floatx4 v = *reinterpret_cast<const floatx4 *>(src + (word < PC ? word : PC - 1) * kWordBits);
+                        const float s = (__builtin_fabsf(v[0]) + __builtin_fabsf(v[1])) + (__builtin_fabsf(v[2]) + __builtin_fabsf(v[3]));
+                        sum[b][w] += word < PC ? s : 0.f;
+                    }
+                }
+            float total = 0.f;
+#pragma unroll
+            for (int b = 0; b < 4; b++) {
+                float s = (sum[b][0] + sum[b][2]) + (sum[b][1] + sum[b][3]);
+#pragma unroll
+                for (int off = 8; off > 0; off >>= 1) s += __shfl_xor(s, off, 16);
+                total += s;
+            }
+            if (r == 0 && slot < slots) th_of[slot] = (float)((double)total * p.ths.scale);
+            __syncthreads();
+        }
+    }
 
     // ---- the patch ----------------------------------------------------------------------------------------------------
     if constexpr (INPUT == kNchw) {
@@ -416,6 +453,13 @@ bool conv_small_in_one_image(int OH, int OW)
     int tl, tc;
     block_of(OW, tl, tc);
     return OH >= tl;
+}
+
+bool conv_small_own_thresholds(const float *x, int H, int W, int C, int KH, int KW, int p1, int p2)
+{
+    // (an image of more than 4096 channels may be summed in several slices)
+    return H == 1 && W == 1 && KH == 1 && KW == 1 && p1 == 0 && p2 == 0 && C <= 4096 && small_input(x, false, C) == kNhwcWords &&
+           threshold_splits(1, C) == 1;
 }
 
 hipError_t launch_conv_small(int type, const float *x, bool nchw, const Thresholds &ths, const uint64_t *qw, const int32_t *btn, float *y,

@@ -339,21 +339,39 @@ py::object attribute(py::handle module, py::handle name)
 
 PyObject *interned(const char *name) { return PyUnicode_InternFromString(name); }
 
+// The item of a dictionary attribute (_buffers, _modules) or, where it is not there, the attribute itself.
+py::object item_or_attribute(py::handle module, py::handle dict_name, py::handle name)
+{
+    const py::object dict = attribute(module, dict_name);
+    PyObject *item = PyDict_Check(dict.ptr()) ? PyDict_GetItemWithError(dict.ptr(), name.ptr()) : nullptr;
+    if (item != nullptr) return py::reinterpret_borrow<py::object>(item);
+    if (PyErr_Occurred()) throw py::error_already_set();
+    return py::reinterpret_steal<py::object>(PyObject_GetAttr(module.ptr(), name.ptr()));
+}
+
 torch::Tensor buffer(py::handle module, py::handle name)
 {
     static PyObject *const buffers_name = interned("_buffers");
-    const py::object buffers = attribute(module, buffers_name);
-    PyObject *item = PyDict_Check(buffers.ptr()) ? PyDict_GetItemWithError(buffers.ptr(), name.ptr()) : nullptr;
-    const py::object t = item != nullptr ? py::reinterpret_borrow<py::object>(item)
-                                         : py::reinterpret_steal<py::object>(PyObject_GetAttr(module.ptr(), name.ptr()));
-    return t.cast<torch::Tensor>();
+    return item_or_attribute(module, buffers_name, name).cast<torch::Tensor>();
 }
 
-int integer(py::handle module, py::handle name) { return attribute(module, name).cast<int>(); }
+int as_int(PyObject *v)
+{
+    if (PyLong_CheckExact(v)) {
+        const long value = PyLong_AsLong(v);
+        if (value == (int)value && !(value == -1 && PyErr_Occurred())) return (int)value;
+        PyErr_Clear();
+    }
+    return py::handle(v).cast<int>();
+}
+
+int integer(py::handle module, py::handle name) { return as_int(attribute(module, name).ptr()); }
 
 std::pair<int, int> pair_of(py::handle module, py::handle name)
 {
     const py::object v = attribute(module, name);
+    if (PyTuple_CheckExact(v.ptr()) && PyTuple_GET_SIZE(v.ptr()) == 2)
+        return {as_int(PyTuple_GET_ITEM(v.ptr(), 0)), as_int(PyTuple_GET_ITEM(v.ptr(), 1))};
     return {v[py::int_(0)].cast<int>(), v[py::int_(1)].cast<int>()};
 }
 
@@ -442,9 +460,39 @@ torch::Tensor layer_forward(py::handle module, const torch::Tensor &x, bool nchw
     return y;
 }
 
-// TABLinear.forward around a TABConv2d: (N, F) as N images of one pixel
-torch::Tensor linear_forward(py::handle conv, const torch::Tensor &x)
+// Whether calling the module would run more than its forward: hooks of its own, hooks of every module, a forward replaced.
+bool plain_call(py::handle module, py::handle type)
 {
+    static PyObject *const hooks[] = {interned("_forward_hooks"), interned("_forward_pre_hooks"), interned("_backward_hooks"),
+                                      interned("_backward_pre_hooks")};
+    static PyObject *const forward_name = interned("forward");
+    static const std::vector<PyObject *> global_hooks = [] {
+        const py::module_ m = py::module_::import("torch.nn.modules.module");
+        std::vector<PyObject *> all;
+        for (const char *name : {"_global_forward_hooks", "_global_forward_pre_hooks", "_global_backward_hooks", "_global_backward_pre_hooks"})
+            all.push_back(py::object(m.attr(name)).release().ptr());
+        return all;
+    }();
+    if ((PyObject *)Py_TYPE(module.ptr()) != type.ptr()) return false;
+    for (PyObject *name : hooks) {
+        const py::object d = attribute(module, name);
+        if (!PyDict_Check(d.ptr()) || PyDict_GET_SIZE(d.ptr()) != 0) return false;
+    }
+    for (PyObject *d : global_hooks)
+        if (!PyDict_Check(d) || PyDict_GET_SIZE(d) != 0) return false;
+    PyObject **dict = _PyObject_GetDictPtr(module.ptr());
+    return dict == nullptr || *dict == nullptr || PyDict_Contains(*dict, forward_name) == 0;
+}
+
+// TABLinear.forward around its TABConv2d (`conv_type`: that class): (N, F) as N images of one pixel.  None where calling the
+// convolution module is more than its forward, or it takes another layout: the caller then calls it.
+py::object linear_forward(py::handle module, py::handle conv_type, const torch::Tensor &x)
+{
+    static PyObject *const modules_name = interned("_modules"), *const conv_name = interned("conv"), *const format_name = interned("data_format");
+    const py::object conv = item_or_attribute(module, modules_name, conv_name);
+    if (!plain_call(conv, conv_type)) return py::none();
+    const py::object format = attribute(conv, format_name);
+    if (!PyUnicode_Check(format.ptr()) || PyUnicode_CompareWithASCIIString(format.ptr(), "NHWC") != 0) return py::none();
     const Layer l(conv);
     if (x.dim() != 2) throw py::value_error("expected an input of two dimensions, got " + std::to_string(x.dim()));
     const int N = (int)x.size(0);
@@ -455,7 +503,7 @@ torch::Tensor linear_forward(py::handle conv, const torch::Tensor &x)
     const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(X.device());
     const torch::Tensor y = device_empty({N, l.KN}, torch::kFloat32, X);
     run_layer(l, X, false, N, 1, 1, y);
-    return y;
+    return py::cast(y);
 }
 
 // TABPackedChain.forward: packed activations between the layers, in raw blocks of the caching allocator

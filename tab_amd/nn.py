@@ -7,18 +7,11 @@ Inference only (the operators have no backward).
 """
 import torch
 from torch import nn
-from torch.nn.modules.module import _has_any_global_hook
 
 from . import _C, BNN, BTN, TBN, TNN, Quantize, Threshold
 
 _ACT_BITS = {TNN: 2, TBN: 2, BTN: 1, BNN: 1}
 _WEIGHT_BITS = {TNN: 2, TBN: 1, BTN: 2, BNN: 1}
-
-
-def _hooked(module):
-    """Whether calling the module would run more than its forward."""
-    return bool(module._forward_hooks or module._forward_pre_hooks or module._backward_hooks or module._backward_pre_hooks
-                or _has_any_global_hook())
 
 
 def _pair(v):
@@ -84,11 +77,11 @@ class TABLinear(nn.Module):
         return cls(conv)
 
     def forward(self, x):
-        conv = self.conv
-        if type(conv) is TABConv2d and conv.data_format == "NHWC" and not _hooked(conv):
-            return _C.linear_forward(conv, x)
-        N, F = x.shape
-        return conv(x.reshape(N, 1, 1, F)).reshape(N, conv.out_channels)
+        y = _C.linear_forward(self, TABConv2d, x)
+        if y is None:  # the inner layer has hooks, or another layout
+            N, F = x.shape
+            y = self.conv(x.reshape(N, 1, 1, F)).reshape(N, self.conv.out_channels)
+        return y
 
 
 class TABPackedChain(nn.Module):

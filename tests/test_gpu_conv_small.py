@@ -7,7 +7,7 @@ import torch
 import oracle
 import tab_amd
 from helpers import TYPE_NAMES, act_bits, make_layer, weight_bits
-from tab_amd.nn import TABConv2d
+from tab_amd.nn import TABConv2d, TABLinear
 
 pytestmark = pytest.mark.gpu
 
@@ -78,3 +78,16 @@ def test_special_values_and_negative_thresholds():
             assert tab_amd.conv2d_launches(x.cuda(), *args) == 1
             y = tab_amd.Conv2d(x.cuda(), torch.from_numpy(qw_o).cuda(), x_ths.cuda(), torch.from_numpy(btn_o).cuda(), *args)
             assert np.array_equal(y.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("C", [64, 320, 1024, 1088, 2048])
+def test_linear_threshold_inside_the_launch(C):
+    """A linear layer's ternary thresholds, taken from the rows inside the one launch, are those of Threshold to the last bit:
+    rows of fewer and more words than a turn of the sum, counts that leave the last block of sixteen rows partly empty."""
+    for N, KN in ((1, 16), (16, 70), (37, 20)):
+        print(f"[case] linear thresholds N={N} C={C}", flush=True)
+        g = torch.Generator("cpu").manual_seed(C + N)
+        x = torch.randn((N, C), generator=g).cuda()
+        fc = TABLinear.from_float(torch.randn((KN, C), generator=g), tab_amd.TBN)
+        want = tab_amd.Conv2d(x, fc.conv.QW, tab_amd.Threshold(x, N), fc.conv.BTN_W, 1, 0, 0, 1, 1, N, 1, 1, C, KN, 1, 1)
+        assert torch.equal(fc(x), want.view(N, KN))
