@@ -24,14 +24,6 @@
 namespace tab {
 namespace {
 
-// 16 bytes per lane from a buffer straight into LDS: lane i's data lands at dst + 16*i (dst is
-// wave-uniform), an out-of-range offset writes zeros.  In a function of its own because the cast to the
-// LDS address space must not appear in the kernel's body, which the host pass also parses.
-__device__ __forceinline__ void load16_to_lds(__amdgpu_buffer_rsrc_t rsrc, uint32_t *dst, uint32_t byte_offset)
-{
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void *)dst, 16, byte_offset, 0, 0, 0);
-}
-
 // Granules of a row and chunk fetched by neighbouring lanes.
 // (Pairs of one-plane granules, read 8 bytes a lane, measured no faster than single ones.)
 constexpr int granule_run(int per_row, int planes) { return per_row % 4 == 0 ? 4 : (per_row % 2 == 0 && planes == 2 ? 2 : 1); }

@@ -50,6 +50,14 @@ __device__ __forceinline__ Item<PL> load_item(__amdgpu_buffer_rsrc_t rsrc, uint3
     return it;
 }
 
+// 16 bytes per lane from a buffer straight into LDS: lane i's data lands at dst + 16*i (dst is
+// wave-uniform), an out-of-range offset writes zeros.  In a function of its own because the cast to the
+// LDS address space must not appear in the kernel's body, which the host pass also parses.
+__device__ __forceinline__ void load16_to_lds(__amdgpu_buffer_rsrc_t rsrc, uint32_t *dst, uint32_t byte_offset)
+{
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void *)dst, 16, byte_offset, 0, 0, 0);
+}
+
 template <int PL, int ROWS, int Q>
 __device__ __forceinline__ void store_item(uint32_t *lds, const Item<PL> &it, int word, int row)
 {

@@ -6,6 +6,7 @@
 //
 // The tensor is a sequence of "rows" of 64 consecutive channels; row r becomes packed
 // word r (C % 64 == 0) so the whole op is one streaming pass: 256 B in, 8 or 16 B out.
+#include "tab_conv_stage.h"
 #include "tab_pack.h"
 
 namespace tab {
@@ -28,12 +29,11 @@ __device__ __forceinline__ int wave_sum(int v)
 // writes them on the side, since a launch of its own for them costs 1.2-4.8 us before the quantizer: a lane takes the
 // counts with the numbers of `n` rows (or pixels) of its own, of which there are at least as many as items.  At the end of
 // the kernel, so that nothing waits for the argument.  Null: none wanted.
-template <int STRIDE = 1>
 __device__ __forceinline__ void zero_counts(int32_t *btn, long items, long first, int n = 1)
 {
     if (btn == nullptr) return;
     for (int i = 0; i < n; i++)
-        if (first + i * STRIDE < items) btn[first + i * STRIDE] = 0;
+        if (first + i < items) btn[first + i] = 0;
 }
 
 // Fast path, C % 64 == 0 and X 16-byte aligned.
@@ -142,147 +142,135 @@ __global__ __launch_bounds__(64) void quantize_rows64_strided(const floatx4 *__r
     }
 }
 
-// General path (any C, any alignment of x; pixels * PC < 2^31): a group of LP lanes takes one (pixel, word) row of
-// up to 4 * LP channels, lane l the channels l, l + LP, l + 2 LP, l + 3 LP of the word (so a wave-wide load reads
-// runs of 4 * LP bytes, and neighbouring groups neighbouring rows); LP = 16 serves words of up to 64 channels,
-// smaller groups tensors of few channels (LP = 1: a lane per pixel).  Eight rows per group are in flight.  The
-// lanes' compare bits are ORed over the group; unused high bits of a tail word stay 0 (TAB_GEMM.cu:203-206).
-template <int BITS, int LP>
-__global__ __launch_bounds__(kThreads) void quantize_groups(const float *__restrict__ x, const Thresholds ths,
-                                                            uint32_t *__restrict__ q, long rows, long pixels_per_item,
-                                                            int C, int PC, int32_t *btn, long items)
+// Spread the 32 bits of v to the even bits of a 64-bit word.
+__device__ __forceinline__ uint64_t spread_bits(uint32_t v)
 {
-    constexpr int GROUPS = 64 / LP;  // rows per wave-wide load
-    constexpr int U = 8;
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int group = lane / LP, l = lane % LP;
-    const long row0 = ((long)blockIdx.x * kWavesPerBlock + wave) * (GROUPS * U);
-    if (row0 >= rows) return;
-    long row_last = row0 + GROUPS * U - 1;
-    if (row_last > rows - 1) row_last = rows - 1;
-
-    float v[U][4];
-    int channels[U];  // of the row's word
-    long pixel[U];
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-        const long r = row0 + u * GROUPS + group;
-        const uint32_t rc = (uint32_t)(r < rows ? r : rows - 1);  // rows past the end read the last row again (not stored)
-        const uint32_t px = PC == 1 ? rc : rc / (uint32_t)PC;
-        const int c0 = (int)(rc - px * (uint32_t)PC) * kWordBits;
-        channels[u] = C - c0 < kWordBits ? C - c0 : kWordBits;
-        pixel[u] = px;
-        const float *src = x + (long)px * C + c0;
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const int ch = l + LP * e;  // past the word: its last channel again, masked below
-            v[u][e] = __builtin_nontemporal_load(src + (ch < channels[u] ? ch : channels[u] - 1));
-        }
-    }
-
-    const long item_first = (row0 / PC) / pixels_per_item;
-    const bool one_item = ((row_last / PC) / pixels_per_item) == item_first;  // scalar
-    const float t_first = wave_threshold(ths, item_first);
-
-    auto finish = [&](int u, float t) {
-        uint32_t out[4];
-        pack_row_strided<BITS, LP>(v[u], t, l, channels[u], out);
-        const long r = row0 + u * GROUPS + group;
-        if (BITS == 2) {
-            if (r < rows && l == 0) *reinterpret_cast<uintx4 *>(q + r * 4) = uintx4{out[0], out[1], out[2], out[3]};
-        } else {
-            if (r < rows && l == 0) *reinterpret_cast<uintx2 *>(q + r * 2) = uintx2{out[0], out[1]};
-        }
-    };
-    if (one_item) {
-#pragma unroll
-        for (int u = 0; u < U; u++) finish(u, t_first);
-    } else {
-#pragma unroll
-        for (int u = 0; u < U; u++) finish(u, lane_threshold(ths, pixel[u] / pixels_per_item));
-    }
-    if (lane < GROUPS * U) zero_counts<64>(btn, items, row0 + lane, GROUPS * U / 64 > 1 ? GROUPS * U / 64 : 1);
+    uint64_t x = v;
+    x = (x | x << 16) & 0x0000ffff0000ffffull;
+    x = (x | x << 8) & 0x00ff00ff00ff00ffull;
+    x = (x | x << 4) & 0x0f0f0f0f0f0f0f0full;
+    x = (x | x << 2) & 0x3333333333333333ull;
+    return (x | x << 1) & 0x5555555555555555ull;
 }
 
-// Fallback of the general path for tensors of 2^31 rows or more: one wave per (pixel, word); lane i tests channel
-// word*64 + i and the two wave-wide ballots are the packed words, LSB first
-// (onebit[i] = 1 << i, TAB_GEMM.cu:252-258).  Unused high bits of a tail word stay 0
+// General path: any C, any alignment of x, every format (MODE as in compare4).  A workgroup takes a tile of consecutive pixels,
+// whose channels are one contiguous run of x, sends the run to LDS in granules of 16 bytes, and its waves then read the words
+// out of it: LP lanes a word (the smallest power of two that holds it; 64 / LP pixels a read where a pixel is one word), so
+// that one compare makes the bits of a whole read as a wave mask (LSB first; onebit[i] = 1 << i, TAB_GEMM.cu:252-258).  Lane
+// i keeps the word of the wave's pixel i.  Unused high bits of a tail word stay 0
 // (TAB_GEMM.cu:203-206).
-template <int BITS>
-__global__ __launch_bounds__(kThreads) void quantize_ballot(const float *__restrict__ x,
-                                                            const Thresholds ths,
-                                                            uint64_t *__restrict__ q, long pixels,
-                                                            long pixels_per_item, int C, int PC, int32_t *btn, long items)
+// Bound by reading x and by the waits of a tile for its run: the 16-byte loads do not care where pixels begin, and a word costs
+// six to twelve instructions.  With 4-byte loads a lane and row, ORed together over the lanes of a word (one plane / two, before
+// -> now, us): 64x56x56x100 21.5 / 23.1 -> 16.0 / 18.3, x200 38 / 41 -> 27 / 32, 64x112x112x32 31 / 33 -> 18.0 / 18.6, 64x224x224x3
+// 19.3 / 25.0 -> 13.3 / 16.8, 5x37x53x100 5.3 / 5.8 -> 3.9 / 4.0; formats 4 and 5 had one wave per word.
+// Formats 4 and 5 belong to the CPU-only conv types, whose layouts follow from the reference's GEMMs (it has no quantizer for
+// them: TAB_Conv calls Parallel_Binarize_NCHW and Parallel_Ternarize_RTN, TAB_CPU.cpp:522,527, which no file defines):
+// 4, DoReFa 2-bit (DRFGEMM_baseline, TAB_CPU.cpp:345-354): [pixel][ceil(C/64)][2], plane 0 the weight-2 bit and plane 1 the
+//    weight-1 bit of level = (v >= 0.5t) + (v >= 1.5t) + (v >= 2.5t);
+// 5, RTN (RTNGEMM_baseline, TAB_CPU.cpp:364-379; 32 channels per word, 520-521): [pixel][ceil(C/32)], channel c in word c/32
+//    as the field (bit 2*(c%32) = nonzero, bit 2*(c%32)+1 = sign) of the ternarizer's value.
+template <int MODE, int LP>
+__global__ __launch_bounds__(kThreads) void quantize_tile(const float *__restrict__ x, const Thresholds ths, uint64_t *__restrict__ q,
+                                                          long pixels, long pixels_per_item, Div32 div_item, int C, int tile_pixels, int words,
+                                                          int32_t *btn, long items)
 {
-    const int lane = threadIdx.x & 63;
-    const long nwaves = (long)gridDim.x * kWavesPerBlock;
-    const long units = pixels * PC;
-    for (long unit = (long)blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6); unit < units; unit += nwaves) {
-        const long pixel = unit / PC;
-        const int word = (int)(unit - pixel * PC);
-        const long item = pixel / pixels_per_item;
-        const float t = wave_threshold(ths, item);
-        const int c = word * kWordBits + lane;
-        const bool live = c < C;
-        const float v = live ? x[pixel * C + c] : 0.f;
-        if (BITS == 2) {
-            const bool pos = live && (v > t);
-            const bool neg = live && !pos && (v < -t);
-            const uint64_t nz = __ballot(pos || neg);
-            const uint64_t sign = __ballot(neg);
-            if (lane == 0) {
-                q[unit * 2 + 0] = sign;
-                q[unit * 2 + 1] = nz;
-            }
-        } else {
-            const uint64_t neg = __ballot(live && (v < t));
-            if (lane == 0) q[unit] = neg;
-        }
-        if (lane == 0) zero_counts(btn, items, unit);
-    }
-}
+    constexpr int G = 64 / LP;  // rows per read
+    constexpr int U = LP == 64 ? 4 : 2;  // reads in flight
+    extern __shared__ __attribute__((aligned(16))) uint32_t tile[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const long p0 = (long)blockIdx.x * tile_pixels;
+    const int live = pixels - p0 < tile_pixels ? (int)(pixels - p0) : tile_pixels;  // pixels of the tile that exist
+    const int PC = (C + kWordBits - 1) / kWordBits;
+    // words w0 ... of the pixel where one pixel is more than a tile (`words` of them), else all
+    const int w0 = blockIdx.y * words, PW = min(words, PC - w0), channels_here = min(C - w0 * kWordBits, PW * kWordBits);
 
-// Packers of the two CPU-only conv types, whose word layouts follow from the reference's GEMMs (it has
-// no quantizer for them: TAB_Conv calls Parallel_Binarize_NCHW and Parallel_Ternarize_RTN,
-// TAB_CPU.cpp:522,527, which no file defines).  One wave per output word, ballots as above.
-// FORMAT 4, DoReFa 2-bit (DRFGEMM_baseline, TAB_CPU.cpp:345-354): [pixel][ceil(C/64)][2], plane 0 the
-//   weight-2 bit and plane 1 the weight-1 bit of level = (v >= 0.5t) + (v >= 1.5t) + (v >= 2.5t).
-// FORMAT 5, RTN (RTNGEMM_baseline, TAB_CPU.cpp:364-379; 32 channels per word, 520-521):
-//   [pixel][ceil(C/32)], channel c in word c/32 as the field (bit 2*(c%32) = nonzero, bit 2*(c%32)+1 =
-//   sign) of the ternarizer's value; lane j of the wave tests channel j/2 for bit j.
-template <int FORMAT>
-__global__ __launch_bounds__(kThreads) void quantize_ballot_format(const float *__restrict__ x, const Thresholds ths,
-                                                                   uint64_t *__restrict__ q, long pixels,
-                                                                   long pixels_per_item, int C, int PC)
-{
-    const int lane = threadIdx.x & 63;
-    const long nwaves = (long)gridDim.x * kWavesPerBlock;
-    const long units = pixels * PC;
-    for (long unit = (long)blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6); unit < units; unit += nwaves) {
-        const long pixel = unit / PC;
-        const int word = (int)(unit - pixel * PC);
-        const float t = lane_threshold(ths, pixel / pixels_per_item);
-        if (FORMAT == 4) {
-            const int c = word * kWordBits + lane;
-            const bool live = c < C;
-            const float v = live ? x[pixel * C + c] : 0.f;
-            const int level = live ? (int)(v >= 0.5f * t) + (int)(v >= 1.5f * t) + (int)(v >= 2.5f * t) : 0;
-            const uint64_t hi = __ballot(level >> 1), lo = __ballot(level & 1);
-            if (lane == 0) {
-                q[unit * 2 + 0] = hi;
-                q[unit * 2 + 1] = lo;
+    // ---- the run of x, from the 16-byte boundary at or below its start to its last float ----------------------------------
+    const uintptr_t start = (uintptr_t)(x + p0 * C + w0 * kWordBits);
+    const int skew = (int)(start & 15) / 4;  // floats
+    const int floats = (live - 1) * C + channels_here + skew;
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(start & ~(uintptr_t)15), 0, floats * 4, kBufferFlags);
+    for (int i = wave * 64; i * 4 < floats; i += kThreads) load16_to_lds(rsrc, tile + i * 4, (uint32_t)(i + lane) * 16u);
+
+    // ---- thresholds: one for the tile, or a table behind the run ---------------------------------------------------------------
+    auto item_of = [&](long pixel) { return div_item.mul ? (long)div32((uint32_t)pixel, div_item) : pixel / pixels_per_item; };
+    const long item_first = item_of(p0);
+    const bool one_item = item_of(p0 + live - 1) == item_first;
+    float *const th = reinterpret_cast<float *>(tile + ((tile_pixels - 1) * C + channels_here + 3 + 3) / 4 * 4 + 256);
+    const float t_first = wave_threshold(ths, item_first);
+    if (!one_item)
+        for (int i = tid; i < live; i += kThreads) th[i] = lane_threshold(ths, item_of(p0 + i));
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+
+    // ---- words: the wave's pixels of the tile, word after word, 64 pixels at a time; a read takes G of them -------------------------
+    const int share = ((live + 3) / 4 + G - 1) / G * G;
+    const int end = min(live, (wave + 1) * share);
+    const float *const run = reinterpret_cast<const float *>(tile) + skew;
+    const int ch = LP == 64 ? lane : lane % LP;
+    for (int px0 = wave * share; px0 < end; px0 += 64)
+        for (int w = 0; w < PW; w++) {
+            const int channels = min(channels_here - w * kWordBits, kWordBits);
+            const uint64_t exist = __ballot(ch < channels);
+            const float *src = run + px0 * C + w * kWordBits + (lane / LP) * C + min(ch, channels - 1);
+            const int reads = (min(end - px0, 64) + G - 1) / G;
+            uint32_t out[4] = {0, 0, 0, 0};  // of pixel px0 + lane: plane 0 low, high, plane 1 low, high
+            for (int j0 = 0; j0 < reads; j0 += U) {
+                float v[U], t[U];
+#pragma unroll
+                for (int u = 0; u < U; u++) {  // (reads past the tile's last pixel: that of the first, kept by no lane)
+                    const bool past = px0 + (j0 + u) * G + lane / LP >= live;
+                    v[u] = src[past ? 0 : (j0 + u) * G * C];
+                    t[u] = one_item ? t_first : th[past ? 0 : px0 + (j0 + u) * G + lane / LP];
+                }
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    uint64_t m0, m1 = 0;
+                    if (MODE == 1) {
+                        m0 = __ballot(v[u] < t[u]) & exist;
+                    } else if (MODE == 4) {
+                        const uint64_t l1 = __ballot(v[u] >= 0.5f * t[u]), l2 = __ballot(v[u] >= 1.5f * t[u]), l3 = __ballot(v[u] >= 2.5f * t[u]);
+                        // level = number of bounds reached, whatever their order (t may be negative)
+                        m0 = ((l1 & l2) | (l1 & l3) | (l2 & l3)) & exist;
+                        m1 = (l1 ^ l2 ^ l3) & exist;
+                    } else {
+                        const uint64_t pos = __ballot(v[u] > t[u]);
+                        m0 = __ballot(v[u] < -t[u]) & ~pos & exist;
+                        m1 = (pos & exist) | m0;
+                    }
+                    // lane j * G + g keeps the LP bits of the read's pixel g
+                    const bool mine = lane / G == j0 + u;
+                    if (LP == 64) {
+                        out[0] = mine ? (uint32_t)m0 : out[0];
+                        out[1] = mine ? (uint32_t)(m0 >> 32) : out[1];
+                        if (MODE != 1) {
+                            out[2] = mine ? (uint32_t)m1 : out[2];
+                            out[3] = mine ? (uint32_t)(m1 >> 32) : out[3];
+                        }
+                    } else {
+                        const int shift = LP * (lane % G);
+                        constexpr uint32_t bits = LP >= 32 ? ~0u : (1u << (LP & 31)) - 1;
+                        out[0] = mine ? (uint32_t)(m0 >> shift) & bits : out[0];
+                        if (MODE != 1) out[2] = mine ? (uint32_t)(m1 >> shift) & bits : out[2];
+                    }
+                }
             }
-        } else {
-            const int c = word * 32 + (lane >> 1);
-            const bool live = c < C;
-            const float v = live ? x[pixel * C + c] : 0.f;
-            const bool pos = live && (v > t);
-            const bool neg = live && !pos && (v < -t);
-            const uint64_t fields = __ballot((lane & 1) ? neg : (pos || neg));
-            if (lane == 0) q[unit] = fields;
+            if (px0 + lane < end) {
+                const size_t pixel = (size_t)p0 + px0 + lane, at = pixel * PC + w0 + w;
+                if (MODE == 1) {
+                    *reinterpret_cast<uintx2 *>(q + at) = uintx2{out[0], out[1]};
+                } else if (MODE == 5) {
+                    // 32 channels a word: 64 are two words, or one where the last 32 of a pixel do not exist
+                    const int halves = (C + 31) / 32;
+                    uint64_t *dst = q + pixel * halves + 2 * (w0 + w);
+                    dst[0] = spread_bits(out[2]) | spread_bits(out[0]) << 1;
+                    if (2 * (w0 + w) + 1 < halves) dst[1] = spread_bits(out[3]) | spread_bits(out[1]) << 1;
+                } else {
+                    *reinterpret_cast<uintx4 *>(q + 2 * at) = uintx4{out[0], out[1], out[2], out[3]};
+                }
+            }
         }
-    }
+    for (int i = tid; i < live; i += kThreads) zero_counts(btn, items, p0 + i);
 }
 
 // The same quantizers on an NCHW tensor, the layout the reference's CPU quantizers read
@@ -662,28 +650,38 @@ void launch_btn_popcount(const uint64_t *qx, int32_t *btn, long items, long word
                                                                                words_per_item, splits, threads);
 }
 
-template <int LP>
-void launch_quantize_groups_of(const float *x, const Thresholds &ths, int bitwidth, long rows, long pixels_per_item, int C, int PC,
-                               uint32_t *q, int32_t *btn, long items, hipStream_t stream)
+template <int MODE, int LP>
+void launch_quantize_tile_of(const float *x, const Thresholds &ths, long pixels, long pixels_per_item, long items, int C, uint64_t *q,
+                             int32_t *btn, hipStream_t stream)
 {
-    const long per_block = (long)kWavesPerBlock * (64 / LP) * 8;
-    const dim3 grid((unsigned)((rows + per_block - 1) / per_block)), block(kThreads);
-    if (bitwidth == 2)
-        quantize_groups<2, LP><<<grid, block, 0, stream>>>(x, ths, q, rows, pixels_per_item, C, PC, btn, items);
-    else
-        quantize_groups<1, LP><<<grid, block, 0, stream>>>(x, ths, q, rows, pixels_per_item, C, PC, btn, items);
+    // Bytes of x in a tile, measured from 4 to 48 KB on C = 3 ... 700: what a few workgroups a CU keep in flight against the
+    // wait of each for its whole tile.  The pixels are shared by four waves in turns of U reads, so sixteen (a turn of four
+    // each) are worth more than the bytes: C=200 41 us at 8 pixels, 32 at 16, 27 at 32.
+    const int PC = (C + kWordBits - 1) / kWordBits;
+    const long bytes = LP < 64 ? 12 * 1024 : (C <= 128 ? 20 * 1024 : 32 * 1024);
+    const long fit = bytes / (4L * C);
+    // a pixel of more than 3072 channels goes in parts of 64 words
+    const int words = C <= 3072 ? PC : 64;
+    long tile_pixels = C > 3072 ? 1 : (fit >= 16 ? fit / 16 * 16 : (C <= 768 ? 16 : 4));
+    // a tensor of few tiles: smaller ones, down to a read of every wave
+    while (tile_pixels >= 8 && pixels / tile_pixels < 512 && tile_pixels / 2 >= 4 * (64 / LP)) tile_pixels = tile_pixels / 8 * 4;
+    const long run = C > 3072 ? words * kWordBits : tile_pixels * C;
+    const size_t lds = ((size_t)(run + 6) / 4 * 4 + 256 + tile_pixels) * 4;
+    const dim3 grid((unsigned)((pixels + tile_pixels - 1) / tile_pixels), (unsigned)((PC + words - 1) / words));
+    const Div32 div_item = pixels < 0x7fffffffL ? make_div32((uint32_t)pixels_per_item) : Div32{0, 0};
+    quantize_tile<MODE, LP><<<grid, dim3(kThreads), lds, stream>>>(x, ths, q, pixels, pixels_per_item, div_item, C, (int)tile_pixels, words, btn, items);
 }
 
-// The general-path kernel with the smallest group of lanes whose 4 channels a lane cover the widest word.
-void launch_quantize_groups(const float *x, const Thresholds &ths, int bitwidth, long rows, long pixels_per_item, int C, int PC,
-                            uint32_t *q, int32_t *btn, long items, hipStream_t stream)
+// The general path with the fewest lanes a word that hold it.
+template <int MODE>
+void launch_quantize_tile(const float *x, const Thresholds &ths, long pixels, long pixels_per_item, long items, int C, uint64_t *q,
+                          int32_t *btn, hipStream_t stream)
 {
-    const int widest = C < kWordBits ? C : kWordBits;
-    if (widest <= 4) launch_quantize_groups_of<1>(x, ths, bitwidth, rows, pixels_per_item, C, PC, q, btn, items, stream);
-    else if (widest <= 8) launch_quantize_groups_of<2>(x, ths, bitwidth, rows, pixels_per_item, C, PC, q, btn, items, stream);
-    else if (widest <= 16) launch_quantize_groups_of<4>(x, ths, bitwidth, rows, pixels_per_item, C, PC, q, btn, items, stream);
-    else if (widest <= 32) launch_quantize_groups_of<8>(x, ths, bitwidth, rows, pixels_per_item, C, PC, q, btn, items, stream);
-    else launch_quantize_groups_of<16>(x, ths, bitwidth, rows, pixels_per_item, C, PC, q, btn, items, stream);
+    if (C <= 4) launch_quantize_tile_of<MODE, 4>(x, ths, pixels, pixels_per_item, items, C, q, btn, stream);
+    else if (C <= 8) launch_quantize_tile_of<MODE, 8>(x, ths, pixels, pixels_per_item, items, C, q, btn, stream);
+    else if (C <= 16) launch_quantize_tile_of<MODE, 16>(x, ths, pixels, pixels_per_item, items, C, q, btn, stream);
+    else if (C <= 32) launch_quantize_tile_of<MODE, 32>(x, ths, pixels, pixels_per_item, items, C, q, btn, stream);
+    else launch_quantize_tile_of<MODE, 64>(x, ths, pixels, pixels_per_item, items, C, q, btn, stream);
 }
 
 // x: fp32 [items][pixels_per_item][C]; qx: [items*pixels_per_item][PC][bitwidth];
@@ -720,17 +718,10 @@ hipError_t launch_quantize(const float *x, const Thresholds &ths, int bitwidth, 
             else
                 quantize_rows64<1><<<grid, block, 0, stream>>>(x4, ths, q32, rows, words_per_item, div_item, zeroed, items);
         }
-    } else if (pixels * PC < 0x7fffffffL) {
-        launch_quantize_groups(x, ths, bitwidth, pixels * PC, pixels_per_item, C, PC, reinterpret_cast<uint32_t *>(qx), zeroed, items, stream);
+    } else if (bitwidth == 2) {
+        launch_quantize_tile<2>(x, ths, pixels, pixels_per_item, items, C, qx, zeroed, stream);
     } else {
-        const long units = pixels * PC;
-        long blocks = (units + kWavesPerBlock - 1) / kWavesPerBlock;
-        if (blocks > 256 * 32) blocks = 256 * 32;  // grid-stride beyond 32 blocks per CU
-        const dim3 grid((unsigned)blocks), block(kThreads);
-        if (bitwidth == 2)
-            quantize_ballot<2><<<grid, block, 0, stream>>>(x, ths, qx, pixels, pixels_per_item, C, PC, zeroed, items);
-        else
-            quantize_ballot<1><<<grid, block, 0, stream>>>(x, ths, qx, pixels, pixels_per_item, C, PC, zeroed, items);
+        launch_quantize_tile<1>(x, ths, pixels, pixels_per_item, items, C, qx, zeroed, stream);
     }
     if (btn && bitwidth == 2) launch_btn_popcount(qx, btn, items, words_per_item, splits, stream);
     return hipGetLastError();
@@ -775,7 +766,6 @@ hipError_t launch_quantize_format(const float *x, const float *ths_values, int f
                                   uint64_t *qx, hipStream_t stream)
 {
     const Thresholds ths = given_thresholds(ths_values);
-    const int PC = format == 5 ? (C + 31) / 32 : (C + kWordBits - 1) / kWordBits;
     const long pixels = items * pixels_per_item;
     if (format != 4 && format != 5) return hipErrorInvalidValue;
     if ((C % kWordBits == 0) && ((uintptr_t)x % 16 == 0)) {
@@ -800,16 +790,8 @@ hipError_t launch_quantize_format(const float *x, const float *ths_values, int f
         }
         return hipGetLastError();
     }
-    const long units = pixels * PC;
-    long blocks = (units + kWavesPerBlock - 1) / kWavesPerBlock;
-    if (blocks > 256 * 32) blocks = 256 * 32;  // grid-stride beyond 32 blocks per CU
-    const dim3 grid((unsigned)blocks), block(kThreads);
-    if (format == 4)
-        quantize_ballot_format<4><<<grid, block, 0, stream>>>(x, ths, qx, pixels, pixels_per_item, C, PC);
-    else if (format == 5)
-        quantize_ballot_format<5><<<grid, block, 0, stream>>>(x, ths, qx, pixels, pixels_per_item, C, PC);
-    else
-        return hipErrorInvalidValue;
+    if (format == 4) launch_quantize_tile<4>(x, ths, pixels, pixels_per_item, items, C, qx, nullptr, stream);
+    else launch_quantize_tile<5>(x, ths, pixels, pixels_per_item, items, C, qx, nullptr, stream);
     return hipGetLastError();
 }
 
