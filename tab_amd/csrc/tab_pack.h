@@ -33,6 +33,13 @@ __device__ __forceinline__ float wave_threshold(const Thresholds &t, long item)
     return __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint((float)(sum * t.scale))));
 }
 
+// bits = 2 * bits + (a < b), in two instructions: the carry of an addition is the compare's result.  (Select and OR take three
+// to five, which is what bounds a lane that packs bits of its own on small tensors.)
+__device__ __forceinline__ void shift_in_less(uint32_t &bits, const float a, const float b)
+{
+    asm("v_cmp_lt_f32_e32 vcc, %1, %2\n\tv_addc_co_u32_e32 %0, vcc, %0, %0, vcc" : "+v"(bits) : "v"(a), "v"(b) : "vcc");
+}
+
 // OR over the 8 lanes of each half of a 16-lane DPP row; every lane gets the result.
 __device__ __forceinline__ uint32_t or_reduce8(uint32_t v)
 {

@@ -275,143 +275,198 @@ __global__ __launch_bounds__(kThreads) void quantize_tile(const float *__restric
 
 // The same quantizers on an NCHW tensor, the layout the reference's CPU quantizers read
 // (Parallel_Ternarize_NCHWB_to_NHWCB / Parallel_Binarize_NCHW_to_NHWC, TAB_CPU.cpp:20-206), into the same NHWC
-// packed output.  A thread owns VEC consecutive pixels of one image and one 64-channel word: it walks the
-// word's channels, VEC floats per load (consecutive threads read consecutive pixels of one channel plane,
-// so every load instruction is contiguous), and shifts each compare bit into the words it holds in
-// registers: no cross-lane step at all.  Pixels are numbered through all images (VEC divides H*W, so a
-// thread's pixels share an image), which keeps every workgroup full whatever H*W is.
-// grid = ceil(N*H*W / (VEC * 256)) * PC workgroups, the word index fastest: the workgroups that write the PC
-// words of the same pixels run side by side, so their 8- or 16-byte stores meet in L2 as whole lines.
-// The form of one pixel a thread serves tensors too small to fill the chip otherwise: bound by the round trip of its
-// loads, it requests the whole word's 64 channels at once (two batches of 32 took one round trip more).
-template <int BITS, int VEC>
+// packed output.  A thread owns a run of VEC consecutive pixels of one image and a part of a word's channels: each load is
+// VEC floats of one channel plane (consecutive threads read consecutive pixels of the plane, so every load instruction is
+// contiguous), and each compare shifts its bit into the words the thread holds in registers: no cross-lane step at all.
+// An image of H*W pixels is ceil(H*W / VEC) runs; where VEC does not divide H*W the last one is moved back to end with the
+// image and overlaps the one before it (the same words are then written twice).  Planes of odd sizes so take the same 16-byte
+// loads, which need 4-byte alignment only, as even ones: with one pixel a thread 55x55 planes were read at 4 TB/s.
+template <int VEC, bool EVEN = false>
+struct PixelRun {
+    typedef float Vec __attribute__((ext_vector_type(VEC)));
+    typedef Vec VecAnywhere __attribute__((aligned(4)));
+    long n, s, pixel;  // image, first pixel in the image, first pixel counted through all images
+
+    // run `i` counted through all images; past the last one: the last one again, with the same results
+    __device__ __forceinline__ PixelRun(long i, int N, long HW)
+    {
+        if (EVEN) {
+            const long total = N * HW;
+            pixel = i * VEC < total ? i * VEC : total - VEC;
+            n = pixel / HW;
+            s = pixel - n * HW;
+        } else {
+            const long per_image = (HW + VEC - 1) / VEC;
+            const long runs = N * per_image;
+            if (i >= runs) i = runs - 1;
+            n = i / per_image;
+            s = (i - n * per_image) * VEC;
+            if (s > HW - VEC) s = HW - VEC;
+            pixel = n * HW + s;
+        }
+    }
+    template <bool NT = false>
+    __device__ __forceinline__ void load(float (&v)[VEC], const float *src) const
+    {
+        if constexpr (VEC == 1) {
+            v[0] = *src;
+        } else {
+            const VecAnywhere *at = reinterpret_cast<const VecAnywhere *>(src);
+            const Vec w = NT ? __builtin_nontemporal_load(at) : *at;
+#pragma unroll
+            for (int e = 0; e < VEC; e++) v[e] = w[e];
+        }
+    }
+    __device__ __forceinline__ float threshold(const Thresholds &ths) const
+    {
+        const long n_first = (long)__builtin_amdgcn_readfirstlane((int)n);
+        return __all(n == n_first) ? wave_threshold(ths, n_first) : lane_threshold(ths, n);
+    }
+    // pixels [first, last) of a wave's lanes from..to, which follow each other without a gap
+    __device__ __forceinline__ long first(int from = 0) const { return lane_pixel(from); }
+    __device__ __forceinline__ long last(int to = 63) const { return lane_pixel(to) + VEC; }
+    __device__ __forceinline__ long lane_pixel(int lane) const
+    {
+        const uint32_t low = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)pixel, lane);
+        const uint32_t high = (uint32_t)__builtin_amdgcn_readlane((int)((uint64_t)pixel >> 32), lane);
+        return (long)((uint64_t)high << 32 | low);
+    }
+};
+
+//
+// A wave packs 16 channels of 64 runs, all of whose loads it requests at once; the up to four waves of a workgroup that
+// share a word (SPLIT: C > 32 four, C > 16 two) meet in LDS, from where the word is stored, pixels in order over the lanes.
+// With a thread to a whole word, 64 loads and the 200 to 700 instructions of their bits in a row were what a tensor too small
+// to fill the chip waited for, and two loads in three were short of the parallelism a large one needs: N=32 64 x 56 x 56
+// (two planes) 6.1 -> 4.4 us, N=128 64 x 112 x 112 79.9 -> 72.4 (6.0 TB/s), N=64 3 x 112 x 112 16.6 -> 6.7.
+// grid = ceil(runs / (64 * 4 / SPLIT)) * PC workgroups, the word index fastest: the workgroups that write the PC words of the
+// same pixels run side by side, so their 8- or 16-byte stores meet in L2 as whole lines.
+template <int BITS, int VEC, int SPLIT, bool NT = false>
 __global__ __launch_bounds__(kThreads) void quantize_nchw(const float *__restrict__ x, const Thresholds ths,
                                                           uint64_t *__restrict__ q, int N, int C, long HW, int PC, int32_t *btn)
 {
-    typedef float vec_t __attribute__((ext_vector_type(VEC)));
-    constexpr int kInFlight = VEC == 1 ? 64 : 8, kTail = VEC == 1 ? 16 : 8;  // loads of a batch; of a batch of a partial word
+    constexpr int kPart = 16;                       // channels a wave packs of its pixels
+    constexpr int GROUPS = kWavesPerBlock / SPLIT;  // of 64 pixel runs, per workgroup
+    constexpr int SLOTS = 64 * VEC;
+    // Loads are requested in the order in which their bits are shifted in: from the last channel down the bits come out in
+    // place (4.2 -> 3.95 us at 26 MB); runs of four, which overlap cache lines of the planes' ends, are read faster upwards
+    // (24 x 75 x 61 x 47: 7.1 -> 6.7 us).
+    constexpr bool UP = VEC == 4;
+    __shared__ alignas(16) uint16_t parts[GROUPS][SPLIT][BITS][SLOTS];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int part = wave % SPLIT, group = wave / SPLIT;
     const int pc = blockIdx.x % PC;
-    const long total = (long)N * HW;
-    const long mine = ((long)(blockIdx.x / PC) * kThreads + threadIdx.x) * VEC;  // first pixel, counted through all images
-    const bool live = mine < total;
-    const long g0 = live ? mine : total - VEC;  // lanes past the end repeat the last pixels and store nothing
-    const long n = g0 / HW, s0 = g0 - n * HW;
-    const int c0 = pc * kWordBits;
-    const int channels = C - c0 < kWordBits ? C - c0 : kWordBits;
-    const float *src = x + (n * C + c0) * HW + s0;
-    uint64_t sign[VEC], nz[VEC];
+    const PixelRun<VEC> run((blockIdx.x / PC * GROUPS + group) * 64L + lane, N, HW);
+    const int c0 = pc * kWordBits + part * kPart;
+    const int channels = C - c0 < kPart ? C - c0 : kPart;  // zero or less: no such part
+    uint32_t less[VEC], more[VEC];
 #pragma unroll
-    for (int e = 0; e < VEC; e++) sign[e] = nz[e] = 0;
-    float v[kInFlight][VEC];
-    auto load = [&](const int j0, auto count) {
+    for (int e = 0; e < VEC; e++) less[e] = more[e] = 0;
+    if (channels > 0) {
+        const float *src = x + (run.n * C + c0) * HW + run.s;
+        float v[kPart][VEC];
+        if (channels == kPart) {
 #pragma unroll
-        for (int u = 0; u < decltype(count)::value; u++) {
-            const int j = j0 + u < channels ? j0 + u : channels - 1;  // clamped: the bit is masked below
-            if (VEC == 1) {
-                v[u][0] = src[(long)j * HW];  // small tensors, likely cache-resident: plain loads
-            } else {
-                const vec_t w = __builtin_nontemporal_load(reinterpret_cast<const vec_t *>(src + (long)j * HW));
+            for (int i = 0; i < kPart; i++) {
+                const int u = UP ? i : kPart - 1 - i;
+                run.template load<NT>(v[u], src + u * HW);
+            }
+        } else {  // what is left of C: nothing is read twice (a clamped channel number would, past the cache if NT)
 #pragma unroll
-                for (int e = 0; e < VEC; e++) v[u][e] = w[e];
+            for (int u = 0; u < kPart; u++) {
+#pragma unroll
+                for (int e = 0; e < VEC; e++) v[u][e] = 0.f;
+                if (u < channels) run.template load<NT>(v[u], src + u * HW);
             }
         }
-    };
-    float t = 0.f;
-    auto pack = [&](const int j0, auto count) {
+        // the threshold is looked up (or added up) while the channels are in flight
+        const float t = run.threshold(ths);
+        const float low = BITS == 2 ? -t : t;
 #pragma unroll
-        for (int u = 0; u < decltype(count)::value; u++) {
-            const uint64_t bit = j0 + u < channels ? (uint64_t)1 << (j0 + u) : 0;
+        for (int i = 0; i < kPart; i++) {
+            const int u = UP ? i : kPart - 1 - i;
 #pragma unroll
             for (int e = 0; e < VEC; e++) {
-                if (BITS == 2) {
-                    const bool pos = v[u][e] > t;
-                    const bool neg = !pos && (v[u][e] < -t);
-                    if (pos || neg) nz[e] |= bit;
-                    if (neg) sign[e] |= bit;
-                } else {
-                    if (v[u][e] < t) sign[e] |= bit;
-                }
+                shift_in_less(less[e], v[u][e], low);
+                if (BITS == 2) shift_in_less(more[e], t, v[u][e]);
             }
         }
-    };
-    // the threshold is looked up (or added up) while the first batch is in flight
-    auto threshold = [&]() {
-        const long n_first = (long)__builtin_amdgcn_readfirstlane((int)n);
-        t = __all(n == n_first) ? wave_threshold(ths, n_first) : lane_threshold(ths, n);
-    };
-    if (channels == kWordBits) {  // a whole word: unrolled, every bit position a constant
-        using Batch = std::integral_constant<int, kInFlight>;
-        load(0, Batch());
-        threshold();
-        pack(0, Batch());
+        const uint32_t exist = 0xffffu >> (kPart - channels);
 #pragma unroll
-        for (int j0 = kInFlight; j0 < kWordBits; j0 += kInFlight) {
-            load(j0, Batch());
-            pack(j0, Batch());
-        }
-    } else {
-        using Batch = std::integral_constant<int, kTail>;
-        load(0, Batch());
-        threshold();
-        pack(0, Batch());
-        for (int j0 = kTail; j0 < channels; j0 += kTail) {
-            load(j0, Batch());
-            pack(j0, Batch());
+        for (int e = 0; e < VEC; e++) {
+            if (UP) {  // the first channel went in first and stands highest
+                less[e] = __brev(less[e]) >> (32 - kPart);
+                more[e] = __brev(more[e]) >> (32 - kPart);
+            }
+            less[e] &= exist;
+            more[e] &= exist;
         }
     }
-    if (!live) return;
+    typedef uint16_t Bits __attribute__((ext_vector_type(VEC)));
+    Bits sign, nz;
 #pragma unroll
     for (int e = 0; e < VEC; e++) {
-        const long pixel = g0 + e;
-        if (BITS == 2) {
-            q[(pixel * PC + pc) * 2 + 0] = sign[e];
-            q[(pixel * PC + pc) * 2 + 1] = nz[e];
-        } else {
-            q[pixel * PC + pc] = sign[e];
-        }
+        sign[e] = (uint16_t)(BITS == 2 ? less[e] & ~more[e] : less[e]);
+        nz[e] = (uint16_t)(less[e] | more[e]);
     }
-    zero_counts(btn, N, g0, VEC);
+    *reinterpret_cast<Bits *>(&parts[group][part][0][lane * VEC]) = sign;
+    if (BITS == 2) *reinterpret_cast<Bits *>(&parts[group][part][BITS - 1][lane * VEC]) = nz;
+    __syncthreads();
+#pragma unroll
+    for (int s0 = 0; s0 < SLOTS; s0 += 64 * SPLIT) {
+        if (s0 + part * 64 >= SLOTS) break;
+        const int slot = s0 + part * 64 + lane;
+        const long pixel = (VEC == 1 ? run.pixel : run.first() + __shfl((int)(run.pixel - run.first()), slot / VEC, 64)) + slot % VEC;
+        uint64_t word[BITS];
+#pragma unroll
+        for (int b = 0; b < BITS; b++) {
+            word[b] = 0;
+#pragma unroll
+            for (int p = 0; p < SPLIT; p++) word[b] |= (uint64_t)parts[group][p][b][slot] << (kPart * p);
+        }
+        uint64_t *dst = q + (pixel * PC + pc) * BITS;
+#pragma unroll
+        for (int b = 0; b < BITS; b++) dst[b] = word[b];
+    }
+    if (part == 0) zero_counts(btn, N, run.pixel, VEC);
 }
 
 // The NCHW quantizer for PC a multiple of U = 2 or 4 and at least one wave of work per SIMD: a thread packs U
 // neighbouring words of its four pixels, one after the other, and the wave then turns its 256 pixels x U words
 // (x 2 planes) around in LDS, so that a store instruction writes whole runs of the output - U * BITS words per pixel,
 // the entire kilobyte when PC == U - instead of one 8-byte word per lane at the stride of a pixel.  Measured on
-// 256 x 256 x 56 x 56: the loads alone take 120 us; with quantize_nchw's word-per-lane stores 152 us (one plane) /
-// 166 us (two), with this kernel 135-137 / 153 us.
+// 256 x 256 x 56 x 56: 137 us (one plane) / 151 us (two); with quantize_nchw 166 / 187.  Planes of odd sizes
+// (256 x 256 x 55 x 55: 159 -> 146 us, 177 -> 153): EVEN keeps the flat numbering of runs for the others, whose 3 us of 137
+// are the registers that it does without.
 // One wave per workgroup (with four, the 784 workgroups of that tensor load the CUs 4 : 3), 4 KB of LDS, gone through
-// in WPP / 2 rounds of 64 / rounds lanes each.  grid = ceil(N*H*W / 256) * (PC / U), the word group fastest.
-template <int BITS, int U>
-__global__ __launch_bounds__(64) void quantize_nchw_gather(const float *__restrict__ x, const Thresholds ths,
+// in WPP / 2 rounds of 64 / rounds lanes each.  grid = ceil(runs / 64) * (PC / U), the word group fastest.
+// Bits are made by the form and in as many registers as measured best: SHIFT for U = 2.
+template <int BITS, int U, bool EVEN>
+__global__ __launch_bounds__(64, BITS == 1 ? (U == 4 ? 4 : 7) : (U == 4 ? 1 : 4)) void quantize_nchw_gather(const float *__restrict__ x, const Thresholds ths,
                                                                  uint64_t *__restrict__ q, int N, int C, long HW, int PC, int32_t *btn)
 {
     constexpr int VEC = 4, kInFlight = 8;
     constexpr int WPP = U * BITS;      // words a thread packs per pixel, contiguous in q
     constexpr int ROUNDS = WPP / 2;    // 64 / ROUNDS lanes x 4 pixels x WPP words = 512 words a round
     constexpr int LPR = 64 / ROUNDS;
+    constexpr bool SHIFT = U == 2;
     static_assert(U == 2 || U == 4, "one word per thread is quantize_nchw");
-    typedef float vec_t __attribute__((ext_vector_type(VEC)));
     __shared__ __attribute__((aligned(16))) uint64_t stage[512];
     const int groups = PC / U;
     const int pc0 = (blockIdx.x % groups) * U;
     const int lane = threadIdx.x;
-    const long total = (long)N * HW;
-    const long wave_pixel0 = (long)(blockIdx.x / groups) * (64 * VEC);  // below total: the grid is ceil(total / 256) * groups
-    const long mine = wave_pixel0 + lane * VEC;
-    const long g0 = mine < total ? mine : wave_pixel0;  // lanes past the end repeat the wave's first pixels and store nothing
-    const long n = g0 / HW, s0 = g0 - n * HW;
+    const PixelRun<VEC, EVEN> run((long)(blockIdx.x / groups) * 64 + lane, N, HW);
     // The U words are U * 64 consecutive channels: batches of kInFlight channels, the next batch's loads issued before
     // the compares of this one (two register buffers), so the memory pipe never waits for the packing.
     const int cbase = pc0 * kWordBits;
-    const float *src = x + n * C * HW + s0;
+    const float *src = x + run.n * C * HW + run.s;
     auto load = [&](float (&v)[kInFlight][VEC], const int b) {
 #pragma unroll
-        for (int k = 0; k < kInFlight; k++) {
+        for (int i = 0; i < kInFlight; i++) {
+            const int k = SHIFT ? kInFlight - 1 - i : i;  // in the order of use
             int c = cbase + b * kInFlight + k;
             c = c < C ? c : C - 1;  // past the last channel (tail word, prefetch after the last batch): masked in pack() or unused
-            const vec_t w = __builtin_nontemporal_load(reinterpret_cast<const vec_t *>(src + (long)c * HW));
-#pragma unroll
-            for (int e = 0; e < VEC; e++) v[k][e] = w[e];
+            run.template load<true>(v[k], src + (long)c * HW);
         }
     };
     uint64_t words[VEC][WPP];
@@ -419,20 +474,40 @@ __global__ __launch_bounds__(64) void quantize_nchw_gather(const float *__restri
     float t;
     auto pack = [&](const float (&v)[kInFlight][VEC], const int b) {
         uint32_t s[VEC], z[VEC];
-#pragma unroll
-        for (int e = 0; e < VEC; e++) s[e] = z[e] = 0;
-#pragma unroll
-        for (int k = 0; k < kInFlight; k++) {
-            const uint32_t bit = cbase + b * kInFlight + k < C ? 1u << k : 0u;
+        if constexpr (SHIFT) {
+            const int left = C - cbase - b * kInFlight;
+            const uint32_t exist = left >= kInFlight ? (1u << kInFlight) - 1 : left > 0 ? (1u << left) - 1 : 0u;
 #pragma unroll
             for (int e = 0; e < VEC; e++) {
-                if (BITS == 2) {
-                    const bool pos = v[k][e] > t;
-                    const bool neg = !pos && (v[k][e] < -t);
-                    if (pos || neg) z[e] |= bit;
-                    if (neg) s[e] |= bit;
-                } else {
-                    if (v[k][e] < t) s[e] |= bit;
+                uint32_t less = 0, more = 0;
+#pragma unroll
+                for (int k = kInFlight - 1; k >= 0; k--) {
+                    if (BITS == 1) {
+                        shift_in_less(less, v[k][e], t);
+                    } else {
+                        less |= v[k][e] < -t ? 1u << k : 0u;
+                        more |= t < v[k][e] ? 1u << k : 0u;
+                    }
+                }
+                s[e] = (less & ~more) & exist;
+                z[e] = (less | more) & exist;
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < VEC; e++) s[e] = z[e] = 0;
+#pragma unroll
+            for (int k = 0; k < kInFlight; k++) {
+                const uint32_t bit = cbase + b * kInFlight + k < C ? 1u << k : 0u;
+#pragma unroll
+                for (int e = 0; e < VEC; e++) {
+                    if (BITS == 2) {
+                        const bool pos = v[k][e] > t;
+                        const bool neg = !pos && (v[k][e] < -t);
+                        if (pos || neg) z[e] |= bit;
+                        if (neg) s[e] |= bit;
+                    } else {
+                        if (v[k][e] < t) s[e] |= bit;
+                    }
                 }
             }
         }
@@ -446,8 +521,7 @@ __global__ __launch_bounds__(64) void quantize_nchw_gather(const float *__restri
     constexpr int kBatches = kWordBits / kInFlight;  // per word
     float v0[kInFlight][VEC], v1[kInFlight][VEC];
     load(v0, 0);
-    const long n_first = (long)__builtin_amdgcn_readfirstlane((int)n);
-    t = __all(n == n_first) ? wave_threshold(ths, n_first) : lane_threshold(ths, n);
+    t = run.threshold(ths);
 #pragma unroll
     for (int u = 0; u < U; u++) {
 #pragma unroll
@@ -465,31 +539,32 @@ __global__ __launch_bounds__(64) void quantize_nchw_gather(const float *__restri
             if (BITS == 2) words[e][u * BITS + 1] = nz[e];
         }
     }
-    uint64_t *st = stage;
 #pragma unroll
     for (int r = 0; r < ROUNDS; r++) {
+        const long first = run.first(r * LPR);
         __builtin_amdgcn_wave_barrier();
         if (lane / LPR == r) {
-            const int l = lane % LPR;
+            ulonglong2 *dst = reinterpret_cast<ulonglong2 *>(stage + (run.pixel - first) * WPP);
 #pragma unroll
             for (int e = 0; e < VEC; e++)
 #pragma unroll
                 for (int j = 0; j < WPP; j += 2)
-                    *reinterpret_cast<ulonglong2 *>(st + (l * VEC + e) * WPP + j) = make_ulonglong2(words[e][j], words[e][j + 1]);
+                    dst[(e * WPP + j) / 2] = make_ulonglong2(words[e][j], words[e][j + 1]);
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const long last = run.last(r * LPR + LPR - 1);
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const int w = (i * 64 + lane) * 2;  // two words a lane: 1 KB a store instruction
-            const long pixel = wave_pixel0 + r * LPR * VEC + w / WPP;
-            const ulonglong2 pair = *reinterpret_cast<const ulonglong2 *>(st + w);
+            const long pixel = first + w / WPP;
+            const ulonglong2 pair = *reinterpret_cast<const ulonglong2 *>(stage + w);
             // an even word index (PC * BITS, pc0 * BITS and w % WPP are even) into a 16-byte aligned q
-            if (pixel < total) *reinterpret_cast<ulonglong2 *>(q + (pixel * PC + pc0) * BITS + w % WPP) = pair;
+            if (pixel < last) *reinterpret_cast<ulonglong2 *>(q + (pixel * PC + pc0) * BITS + w % WPP) = pair;
         }
     }
-    zero_counts(btn, N, g0, VEC);
+    zero_counts(btn, N, run.pixel, VEC);
 }
 
 // btn[n] = sum over item n of popcount(nonzero-plane word) (BTN_Weight, TAB_GEMM.cu:150-160,
@@ -734,29 +809,40 @@ hipError_t launch_quantize_nchw(const float *x, const Thresholds &ths, int bitwi
     const long words_per_item = HW * PC;
     const int splits = btn && bitwidth == 2 ? count_splits(N, words_per_item) : 1;
     int32_t *zeroed = btn && (bitwidth != 2 || splits > 1) ? btn : nullptr;
-    // four pixels per thread when the planes allow aligned 16-byte loads and the launch still fills the chip
     const long pixels = (long)N * HW;
-    const bool vec4 = HW % 4 == 0 && (uintptr_t)x % 16 == 0 && ((pixels + 4 * kThreads - 1) / (4 * kThreads)) * PC >= 2048;
-    const long per_block = (vec4 ? 4 : 1) * (long)kThreads;
-    const long blocks = (pixels + per_block - 1) / per_block;
-    if (blocks * PC > 0x7fffffffL) return hipErrorInvalidValue;
-    const dim3 grid((unsigned)(blocks * PC)), block(kThreads);
+    const long runs = N * ((HW + 3) / 4);
+    auto launch = [&](auto kernel, long blocks, int threads) {
+        kernel<<<dim3((unsigned)blocks), dim3(threads), 0, stream>>>(x, ths, qx, N, C, HW, PC, zeroed);
+    };
     // PC even, enough pixels for a wave on every SIMD: the form that gathers each wave's output into whole runs
     const int unit = PC % 4 == 0 ? 4 : PC % 2 == 0 ? 2 : 1;
-    const long gather_waves = (pixels + 255) / 256 * (PC / unit);
+    const long gather_waves = (runs + 63) / 64 * (PC / unit);
     if (gather_waves > 0x7fffffffL) return hipErrorInvalidValue;
-    if (HW % 4 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)qx % 16 == 0 && unit > 1 && gather_waves >= 1024) {
-        const dim3 ggrid((unsigned)gather_waves), gblock(64);
-        if (unit == 4 && bitwidth == 2) quantize_nchw_gather<2, 4><<<ggrid, gblock, 0, stream>>>(x, ths, qx, N, C, HW, PC, zeroed);
-        else if (unit == 4) quantize_nchw_gather<1, 4><<<ggrid, gblock, 0, stream>>>(x, ths, qx, N, C, HW, PC, zeroed);
-        else if (bitwidth == 2) quantize_nchw_gather<2, 2><<<ggrid, gblock, 0, stream>>>(x, ths, qx, N, C, HW, PC, zeroed);
-        else quantize_nchw_gather<1, 2><<<ggrid, gblock, 0, stream>>>(x, ths, qx, N, C, HW, PC, zeroed);
-    } else if (vec4) {
-        if (bitwidth == 2) quantize_nchw<2, 4><<<grid, block, 0, stream>>>(x, ths, qx, N, C, HW, PC, zeroed);
-        else quantize_nchw<1, 4><<<grid, block, 0, stream>>>(x, ths, qx, N, C, HW, PC, zeroed);
+    if (HW >= 4 && (uintptr_t)qx % 16 == 0 && unit > 1 && gather_waves >= 1024) {
+        if (unit == 4 && bitwidth == 2) launch(HW % 4 ? quantize_nchw_gather<2, 4, false> : quantize_nchw_gather<2, 4, true>, gather_waves, 64);
+        else if (unit == 4) launch(HW % 4 ? quantize_nchw_gather<1, 4, false> : quantize_nchw_gather<1, 4, true>, gather_waves, 64);
+        else if (bitwidth == 2) launch(HW % 4 ? quantize_nchw_gather<2, 2, false> : quantize_nchw_gather<2, 2, true>, gather_waves, 64);
+        else launch(HW % 4 ? quantize_nchw_gather<1, 2, false> : quantize_nchw_gather<1, 2, true>, gather_waves, 64);
     } else {
-        if (bitwidth == 2) quantize_nchw<2, 1><<<grid, block, 0, stream>>>(x, ths, qx, N, C, HW, PC, zeroed);
-        else quantize_nchw<1, 1><<<grid, block, 0, stream>>>(x, ths, qx, N, C, HW, PC, zeroed);
+        // waves per word: as many as it has parts of 16 channels
+        const int split = C <= 16 ? 1 : C <= 32 ? 2 : 4;
+        // One pixel a thread until four give two waves per SIMD (32 x 64 x 56 x 56: 4.4 us, with four 4.8; 53 MB of 57 x 57
+        // planes: 14.1 us, with four 11.9).
+        const bool four = HW >= 4 && (runs + 63) / 64 * PC * split >= 2048;
+        // Past the caches where the tensor is large next to them and a wave reads whole lines, i.e. its kilobyte of a plane
+        // is not mostly a plane's end: 128 x 64 x 112 x 112 73.6 -> 67.6 us, but 128 x 512 x 28 x 28 38.9 -> 44.5.
+        const bool stream_past = four && split == 4 && pixels * C >= (8L << 20) && HW >= 2048;
+        const int groups = kWavesPerBlock / split;
+        const long blocks = ((four ? runs : pixels) + 64 * groups - 1) / (64 * groups) * PC;
+        if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
+        auto pick = [&](auto one, auto two) { launch(bitwidth == 2 ? two : one, blocks, kThreads); };
+        if (stream_past) pick(quantize_nchw<1, 4, 4, true>, quantize_nchw<2, 4, 4, true>);
+        else if (four && split == 4) pick(quantize_nchw<1, 4, 4>, quantize_nchw<2, 4, 4>);
+        else if (four && split == 2) pick(quantize_nchw<1, 4, 2>, quantize_nchw<2, 4, 2>);
+        else if (four) pick(quantize_nchw<1, 4, 1>, quantize_nchw<2, 4, 1>);
+        else if (split == 4) pick(quantize_nchw<1, 1, 4>, quantize_nchw<2, 1, 4>);
+        else if (split == 2) pick(quantize_nchw<1, 1, 2>, quantize_nchw<2, 1, 2>);
+        else pick(quantize_nchw<1, 1, 1>, quantize_nchw<2, 1, 1>);
     }
     if (btn && bitwidth == 2) launch_btn_popcount(qx, btn, N, words_per_item, splits, stream);
     return hipGetLastError();
