@@ -391,24 +391,24 @@ hipError_t launch_conv_mfma(int type, const ConvArgs &args, int shape, hipStream
 }
 
 // Workgroup tile of the matrix-core kernel: the shape with the lowest predicted duration under a cost model fitted to
-// the measured duration of every shape on some 290 (type, layer) cases (tab_conv_shape_model.h: the ResNet-18 layers at
+// the measured duration of every shape on some 430 (type, layer) cases (tab_conv_shape_model.h: the ResNet-18 layers at
 // N = 16 / 64 / 256, the VGG stack, the 28x28 sweep and layers of other geometries).  What the model's features say:
 // the busiest CU decides (ceil(tiles / CUs) tiles of a shape land on it, and it is refilled when it holds no more), K
 // scales the loop, the size of Y the epilogue (with a price of its own where K is at most nine words and the launch is
 // little but epilogue), and a launch smaller than the chip is as long as one tile.  Features and coefficients are all
 // non-negative, so a prediction is positive and monotone in K, tiles and Y for any geometry; on top of that no prediction
 // is taken below what the matrix cores of the busiest CU need at their peak rate plus a launch.
+// (Types 4 and 5 have coefficients of their own: with those of the types of as many planes, 0 and 3, their choices took 4.2 %
+// more than the best shapes', N=256 7x7x512 of type 5 28.4 us for 22.3.)
 // A shape whose filter tile is at least twice the 64-rounded filter count is no candidate.
 // cost_us (optional): the predicted duration of the chosen shape.
-int conv_mfma_shape(int conv_type, const ConvArgs &a, float *cost_us)
+int conv_mfma_shape(int type, const ConvArgs &a, float *cost_us)
 {
-    // the CPU-only types follow the type with the same planes: 4 like TNN, 5 like BNN
-    const int type = conv_type == 4 ? 0 : (conv_type == 5 ? 3 : conv_type);
     // K of at most nine words and packed output: the kernel with the weights resident in registers, whose epilogue
     // thresholds a pixel's filters inside a lane, runs 1.4-2x faster than the tiled shapes once the launch is a few
     // rounds of waves (N=256 56x56x64->64 3x3: 24 against 38 us) and level with them on small ones; with fp32 output
     // both are bound by writing Y and measure within 5 % of each other, so the tiled shapes keep those launches
-    if (conv_type <= 3 && a.G <= 9 && a.qy != nullptr && (a.M >= 65536 || a.G <= 2)) {
+    if (type <= 3 && a.G <= 9 && a.qy != nullptr && (a.M >= 65536 || a.G <= 2)) {
         if (cost_us) *cost_us = 0.f;
         return 7;
     }
@@ -416,6 +416,7 @@ int conv_mfma_shape(int conv_type, const ConvArgs &a, float *cost_us)
     const long cus = device_compute_units();
     // (packed output ranks the shapes as fp32 output does: the model's terms in Y also stand for what grows with M * KN)
     const float y_mb = (float)a.M * (float)a.KN * 4e-6f;
+    const float words = type == 5 ? 0.5f * (float)a.G : (float)a.G;  // of 64 elements
     int best = 2;
     float best_cost = 0.f;
     bool any = false;
@@ -433,21 +434,21 @@ int conv_mfma_shape(int conv_type, const ConvArgs &a, float *cost_us)
             // that the launch is bound by writing Y, whatever the balance of its last round)
             const long pieces = bm / 64 * (bn / 64);
             const long whole = tiles / cus, quarters = (pieces * (tiles % cus) + cus - 1) / cus;
-            const int planes = type == 0 ? 4 : (type == 3 ? 2 : 3);
+            const int planes = type == 0 || type == 4 ? 4 : (type == 3 || type == 5 ? 2 : 3);
             if (a.G * planes <= 36 || whole == 0 || quarters == 0) continue;  // (an odd number of words per pixel: excluded above)
             if (shape == 11 && a.PC % 4 != 0) continue;                       // the 128x256 tiles take four-word chunks inside a tap
             const float f[kConvShapeFeatures] = {(float)a.G * (float)whole, (float)a.G * (float)quarters, (float)quarters, (float)whole, y_mb, y_mb,
                                                  1.f, 1.f, 0.f};
             for (int k = 0; k < kConvShapeFeatures; k++) cost += kConvShapeCost[type][i][k] * f[k];
-            floor_us = 1.f + (float)(4 * pieces * whole + 4 * quarters) * (float)a.G * (32.f / 4.f / 2400.f);
+            floor_us = 1.f + (float)(4 * pieces * whole + 4 * quarters) * words * (32.f / 4.f / 2400.f);
         } else {
             const float n = (float)((tiles + cus - 1) / cus), rounds = (float)(((tiles + cus - 1) / cus + held - 1) / held);
             const float busy = tiles >= cus ? 1.f : (float)tiles / (float)cus;
             const float f[kConvShapeFeatures] = {(float)a.G * n, (float)a.G * rounds, rounds, n, y_mb, y_mb * busy, busy, 1.f,
                                                  a.G <= 9 ? y_mb : 0.f};
             for (int k = 0; k < kConvShapeFeatures; k++) cost += kConvShapeCost[type][i][k] * f[k];
-            // the busiest CU's n tiles of (bm/32)(bn/32) MFMA tiles x G words, 32 cycles each on four SIMDs at 2.4 GHz, and a launch
-            floor_us = 1.f + n * (float)(bm / 32 * (bn / 32)) * (float)a.G * (32.f / 4.f / 2400.f);
+            // the busiest CU's n tiles of (bm/32)(bn/32) MFMA tiles x words, 32 cycles each on four SIMDs at 2.4 GHz, and a launch
+            floor_us = 1.f + n * (float)(bm / 32 * (bn / 32)) * words * (32.f / 4.f / 2400.f);
         }
         if (cost < floor_us) cost = floor_us;
         if (!any || cost < best_cost) {

@@ -40,7 +40,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 SHAPES = {0: (128, 128, 4), 1: (128, 64, 6), 2: (64, 64, 8), 3: (32, 32, 4), 4: (256, 64, 4), 5: (256, 128, 2), 6: (128, 256, 2),
           8: (64, 64, 4), 9: (128, 128, 2), 10: (128, 128, 4), 11: (128, 256, 2)}
 MIXED = (10, 11)
-PLANES = {0: 4, 1: 3, 2: 3, 3: 2}  # bit planes of activation + weight operand, per type
+PLANES = {0: 4, 1: 3, 2: 3, 3: 2, 4: 4, 5: 2}  # bit planes of activation + weight operand, per type
 IDS = sorted(SHAPES)
 NFEAT = 9
 
@@ -57,7 +57,8 @@ def parse(path):
         t, N, H, W, C, KN, kh, kw, p1, p2, s1, s2 = map(int, m.groups()[:12])
         OH, OW = (H + 2 * p1 - kh + 1) // s1, (W + 2 * p2 - kw + 1) // s2  # TAB_GEMM.cu:354-357
         times = {int(a.split(":")[0]): float(a.split(":")[1]) for a in m.group(13).split()}
-        rows.append(dict(set=which, type=t, M=N * OH * OW, KN=KN, G=kh * kw * ((C + 63) // 64), PC=(C + 63) // 64, times=times,
+        PC = (C + 31) // 32 if t == 5 else (C + 63) // 64  # a word of type 5 holds 32 channels
+        rows.append(dict(set=which, type=t, M=N * OH * OW, KN=KN, G=kh * kw * PC, PC=PC, times=times,
                          name=line.split()[2]))
     return rows
 
@@ -93,7 +94,7 @@ def fit(rows):
 
     coef = {}
     for s in SHAPES:
-        for t in range(4):
+        for t in range(6):
             X = np.array([features(r, s) for r in rows if r["type"] == t and eligible(r, s)])
             y = np.array([r["times"][s] for r in rows if r["type"] == t and eligible(r, s)])
             w = 1.0 / np.maximum(y, 1.0)  # relative error; the latency-bound N=16 set, the benchmark's headline, counts threefold
@@ -160,8 +161,8 @@ def main():
         f.write("constexpr int kConvShapeIds[kConvShapes] = {" + ", ".join(str(i) for i in IDS) + "};\n")
         f.write("// rows x filters of the workgroup tile and workgroups a CU holds (compiled occupancy), per shape\n")
         f.write("constexpr int kConvShapeTile[kConvShapes][3] = {" + ", ".join("{%d, %d, %d}" % SHAPES[s] for s in IDS) + "};\n")
-        f.write("constexpr float kConvShapeCost[4][kConvShapes][kConvShapeFeatures] = {\n")
-        for t in range(4):
+        f.write("constexpr float kConvShapeCost[6][kConvShapes][kConvShapeFeatures] = {\n")
+        for t in range(6):
             f.write("    {\n")
             for s_ in IDS:
                 f.write("        {" + ", ".join(("%.6g" % v if "." in "%.6g" % v or "e" in "%.6g" % v else "%.6g.0" % v) + "f" for v in coef[(t, s_)]) + "},\n")
