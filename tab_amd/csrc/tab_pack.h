@@ -33,12 +33,49 @@ __device__ __forceinline__ float wave_threshold(const Thresholds &t, long item)
     return __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint((float)(sum * t.scale))));
 }
 
-// bits = 2 * bits + (a < b), in two instructions: the carry of an addition is the compare's result.  (Select and OR take three
-// to five, which is what bounds a lane that packs bits of its own on small tensors.)
-__device__ __forceinline__ void shift_in_less(uint32_t &bits, const float a, const float b)
+// Four compares shifted into bits, two instructions each: bits = 2 * bits + (a < b), the carry of an addition being the
+// compare's result.  (Select and OR take three to five, which is what bounds a lane that packs bits of its own on small
+// tensors.)  The compares stand before the additions because a carry read as a scalar mask needs two other instructions
+// between it and the compare that wrote it; the compiler cannot see into the block to put them there.
+#define TAB_SHIFT_IN_LESS4(B0, B1, B2, B3, A0, A1, A2, A3, L0, L1, L2, L3)                                                       \
+    "v_cmp_lt_f32_e64 %[c0], %[" A0 "], %[" L0 "]\n\tv_cmp_lt_f32_e64 %[c1], %[" A1 "], %[" L1 "]\n\t"                            \
+    "v_cmp_lt_f32_e64 %[c2], %[" A2 "], %[" L2 "]\n\tv_cmp_lt_f32_e64 %[c3], %[" A3 "], %[" L3 "]\n\t"                            \
+    "v_addc_co_u32_e64 %[" B0 "], %[c0], %[" B0 "], %[" B0 "], %[c0]\n\tv_addc_co_u32_e64 %[" B1 "], %[c1], %[" B1 "], %[" B1 "], %[c1]\n\t" \
+    "v_addc_co_u32_e64 %[" B2 "], %[c2], %[" B2 "], %[" B2 "], %[c2]\n\tv_addc_co_u32_e64 %[" B3 "], %[c3], %[" B3 "], %[" B3 "], %[c3]"
+
+// into the bits of four pixels
+__device__ __forceinline__ void shift_in_less4(uint32_t (&bits)[4], const float (&a)[4], const float limit)
 {
-    asm("v_cmp_lt_f32_e32 vcc, %1, %2\n\tv_addc_co_u32_e32 %0, vcc, %0, %0, vcc" : "+v"(bits) : "v"(a), "v"(b) : "vcc");
+    uint64_t c0, c1, c2, c3;
+    asm(TAB_SHIFT_IN_LESS4("b0", "b1", "b2", "b3", "a0", "a1", "a2", "a3", "l", "l", "l", "l")
+        : [b0] "+v"(bits[0]), [b1] "+v"(bits[1]), [b2] "+v"(bits[2]), [b3] "+v"(bits[3]), [c0] "=&s"(c0), [c1] "=&s"(c1), [c2] "=&s"(c2), [c3] "=&s"(c3)
+        : [a0] "v"(a[0]), [a1] "v"(a[1]), [a2] "v"(a[2]), [a3] "v"(a[3]), [l] "v"(limit));
 }
+// limit < a
+__device__ __forceinline__ void shift_in_more4(uint32_t (&bits)[4], const float (&a)[4], const float limit)
+{
+    uint64_t c0, c1, c2, c3;
+    asm(TAB_SHIFT_IN_LESS4("b0", "b1", "b2", "b3", "l", "l", "l", "l", "a0", "a1", "a2", "a3")
+        : [b0] "+v"(bits[0]), [b1] "+v"(bits[1]), [b2] "+v"(bits[2]), [b3] "+v"(bits[3]), [c0] "=&s"(c0), [c1] "=&s"(c1), [c2] "=&s"(c2), [c3] "=&s"(c3)
+        : [a0] "v"(a[0]), [a1] "v"(a[1]), [a2] "v"(a[2]), [a3] "v"(a[3]), [l] "v"(limit));
+}
+
+// into the bits of one pixel, a0 first
+__device__ __forceinline__ void shift_in_less4(uint32_t &bits, const float a0, const float a1, const float a2, const float a3, const float limit)
+{
+    uint64_t c0, c1, c2, c3;
+    asm(TAB_SHIFT_IN_LESS4("b", "b", "b", "b", "a0", "a1", "a2", "a3", "l", "l", "l", "l")
+        : [b] "+v"(bits), [c0] "=&s"(c0), [c1] "=&s"(c1), [c2] "=&s"(c2), [c3] "=&s"(c3)
+        : [a0] "v"(a0), [a1] "v"(a1), [a2] "v"(a2), [a3] "v"(a3), [l] "v"(limit));
+}
+__device__ __forceinline__ void shift_in_more4(uint32_t &bits, const float a0, const float a1, const float a2, const float a3, const float limit)
+{
+    uint64_t c0, c1, c2, c3;
+    asm(TAB_SHIFT_IN_LESS4("b", "b", "b", "b", "l", "l", "l", "l", "a0", "a1", "a2", "a3")
+        : [b] "+v"(bits), [c0] "=&s"(c0), [c1] "=&s"(c1), [c2] "=&s"(c2), [c3] "=&s"(c3)
+        : [a0] "v"(a0), [a1] "v"(a1), [a2] "v"(a2), [a3] "v"(a3), [l] "v"(limit));
+}
+#undef TAB_SHIFT_IN_LESS4
 
 // OR over the 8 lanes of each half of a 16-lane DPP row; every lane gets the result.
 __device__ __forceinline__ uint32_t or_reduce8(uint32_t v)

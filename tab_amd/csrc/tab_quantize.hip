@@ -382,13 +382,17 @@ __global__ __launch_bounds__(kThreads) void quantize_nchw(const float *__restric
         // the threshold is looked up (or added up) while the channels are in flight
         const float t = run.threshold(ths);
         const float low = BITS == 2 ? -t : t;
+        if constexpr (VEC == 4) {
 #pragma unroll
-        for (int i = 0; i < kPart; i++) {
-            const int u = UP ? i : kPart - 1 - i;
+            for (int u = 0; u < kPart; u++) {
+                shift_in_less4(less, v[u], low);
+                if (BITS == 2) shift_in_more4(more, v[u], t);
+            }
+        } else {
 #pragma unroll
-            for (int e = 0; e < VEC; e++) {
-                shift_in_less(less[e], v[u][e], low);
-                if (BITS == 2) shift_in_less(more[e], t, v[u][e]);
+            for (int u = kPart - 1; u > 0; u -= 4) {
+                shift_in_less4(less[0], v[u][0], v[u - 1][0], v[u - 2][0], v[u - 3][0], low);
+                if (BITS == 2) shift_in_more4(more[0], v[u][0], v[u - 1][0], v[u - 2][0], v[u - 3][0], t);
             }
         }
         const uint32_t exist = 0xffffu >> (kPart - channels);
@@ -477,20 +481,23 @@ __global__ __launch_bounds__(64, BITS == 1 ? (U == 4 ? 4 : 7) : (U == 4 ? 1 : 4)
         if constexpr (SHIFT) {
             const int left = C - cbase - b * kInFlight;
             const uint32_t exist = left >= kInFlight ? (1u << kInFlight) - 1 : left > 0 ? (1u << left) - 1 : 0u;
+            uint32_t less[VEC] = {0, 0, 0, 0}, more[VEC] = {0, 0, 0, 0};
 #pragma unroll
-            for (int e = 0; e < VEC; e++) {
-                uint32_t less = 0, more = 0;
+            for (int k = kInFlight - 1; k >= 0; k--) {
+                if (BITS == 1) {
+                    shift_in_less4(less, v[k], t);
+                } else {
 #pragma unroll
-                for (int k = kInFlight - 1; k >= 0; k--) {
-                    if (BITS == 1) {
-                        shift_in_less(less, v[k][e], t);
-                    } else {
-                        less |= v[k][e] < -t ? 1u << k : 0u;
-                        more |= t < v[k][e] ? 1u << k : 0u;
+                    for (int e = 0; e < VEC; e++) {
+                        less[e] |= v[k][e] < -t ? 1u << k : 0u;
+                        more[e] |= t < v[k][e] ? 1u << k : 0u;
                     }
                 }
-                s[e] = (less & ~more) & exist;
-                z[e] = (less | more) & exist;
+            }
+#pragma unroll
+            for (int e = 0; e < VEC; e++) {
+                s[e] = (less[e] & ~more[e]) & exist;
+                z[e] = (less[e] | more[e]) & exist;
             }
         } else {
 #pragma unroll
