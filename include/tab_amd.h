@@ -89,6 +89,16 @@ int tab_quantize_nchw(const float *dev_X, const float *dev_ths, int bitwidth, in
                       int64_t *dev_QX, int32_t *dev_BTN, void *stream);
 
 /*
+ * tab_quantize (nchw 0) or tab_quantize_nchw (1) with dev_BTN, in fewer or shorter launches: the quantizer counts while it packs
+ * and leaves the counts of an item's parts in the workspace, so the packed output is not read back for them.
+ *   workspace  tab_quantize_workspace_bytes(...) bytes, 4-byte aligned, free again when the call's work on the stream is
+ *              done; 0 bytes (one plane, small items): NULL will do
+ */
+size_t tab_quantize_workspace_bytes(int bitwidth, int N, int H, int W, int C);
+int tab_quantize_counted(const float *dev_X, const float *dev_ths, int nchw, int bitwidth, int N, int H, int W, int C,
+                         int64_t *dev_QX, int32_t *dev_BTN, void *workspace, size_t workspace_bytes, void *stream);
+
+/*
  * Packers for conv types 4 and 5, activations and weights alike (weights as (N,H,W,C) = (KN,KH,KW,C)).
  * The reference defines the word layouts through DRFGEMM_baseline / RTNGEMM_baseline
  * (TAB_CPU.cpp:332-383) but ships no quantizer for them (TAB_Conv calls Parallel_Binarize_NCHW and

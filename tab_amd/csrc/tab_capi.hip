@@ -128,35 +128,51 @@ int tab_out_extent(int in, int pad, int k, int stride)
     return (in + 2 * pad - k + 1) / stride;
 }
 
-int tab_quantize(const float *dev_X, const float *dev_ths, int bitwidth, int N, int H, int W,
-                 int C, int64_t *dev_QX, int32_t *dev_BTN, void *stream)
+static int quantize_any(const float *dev_X, const float *dev_ths, bool nchw, int bitwidth, int N, int H, int W, int C, int64_t *dev_QX,
+                        int32_t *dev_BTN, int32_t *count_workspace, void *stream)
 {
     if (bitwidth != 1 && bitwidth != 2) return fail(TAB_ERR_BAD_ARGUMENT, "bitwidth must be 1 or 2, got %d", bitwidth);
     if (N < 1 || H < 1 || W < 1 || C < 1) return fail(TAB_ERR_BAD_ARGUMENT, "N, H, W, C must be positive");
     if (!dev_X || !dev_ths || !dev_QX) return fail(TAB_ERR_BAD_ARGUMENT, "null device pointer");  // dev_BTN may be NULL
     if (((uintptr_t)dev_X % 4) || ((uintptr_t)dev_QX % (8 * bitwidth)))
         return fail(TAB_ERR_BAD_ARGUMENT, "X must be aligned to its floats and QX to a whole packed element (%d bytes)", 8 * bitwidth);
-    hipError_t e = tab::launch_quantize(dev_X, tab::given_thresholds(dev_ths), bitwidth, (long)H * W, N, C,
-                                        reinterpret_cast<uint64_t *>(dev_QX), dev_BTN,
-                                        static_cast<hipStream_t>(stream));
+    if (nchw && ((long)N * H * W + 255) / 256 * tab_packed_channels(C) > kMaxIndex)
+        return fail(TAB_ERR_BAD_SHAPE, "tensor too large for one launch (N*H*W/256 * ceil(C/64) workgroups)");
+    const tab::Thresholds ths = tab::given_thresholds(dev_ths);
+    uint64_t *q = reinterpret_cast<uint64_t *>(dev_QX);
+    const hipError_t e =
+        nchw ? tab::launch_quantize_nchw(dev_X, ths, bitwidth, N, C, (long)H * W, q, dev_BTN, count_workspace, static_cast<hipStream_t>(stream))
+             : tab::launch_quantize(dev_X, ths, bitwidth, (long)H * W, N, C, q, dev_BTN, count_workspace, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return device_fail(e, "quantize launch");
     return TAB_OK;
+}
+
+int tab_quantize(const float *dev_X, const float *dev_ths, int bitwidth, int N, int H, int W,
+                 int C, int64_t *dev_QX, int32_t *dev_BTN, void *stream)
+{
+    return quantize_any(dev_X, dev_ths, false, bitwidth, N, H, W, C, dev_QX, dev_BTN, nullptr, stream);
 }
 
 int tab_quantize_nchw(const float *dev_X, const float *dev_ths, int bitwidth, int N, int C, int H, int W,
                       int64_t *dev_QX, int32_t *dev_BTN, void *stream)
 {
-    if (bitwidth != 1 && bitwidth != 2) return fail(TAB_ERR_BAD_ARGUMENT, "bitwidth must be 1 or 2, got %d", bitwidth);
-    if (N < 1 || H < 1 || W < 1 || C < 1) return fail(TAB_ERR_BAD_ARGUMENT, "N, C, H, W must be positive");
-    if (!dev_X || !dev_ths || !dev_QX) return fail(TAB_ERR_BAD_ARGUMENT, "null device pointer");  // dev_BTN may be NULL
-    if (((uintptr_t)dev_X % 4) || ((uintptr_t)dev_QX % (8 * bitwidth)))
-        return fail(TAB_ERR_BAD_ARGUMENT, "X must be aligned to its floats and QX to a whole packed element (%d bytes)", 8 * bitwidth);
-    if (((long)N * H * W + 255) / 256 * tab_packed_channels(C) > kMaxIndex)
-        return fail(TAB_ERR_BAD_SHAPE, "tensor too large for one launch (N*H*W/256 * ceil(C/64) workgroups)");
-    hipError_t e = tab::launch_quantize_nchw(dev_X, tab::given_thresholds(dev_ths), bitwidth, N, C, (long)H * W, reinterpret_cast<uint64_t *>(dev_QX),
-                                             dev_BTN, static_cast<hipStream_t>(stream));
-    if (e != hipSuccess) return device_fail(e, "quantize launch");
-    return TAB_OK;
+    return quantize_any(dev_X, dev_ths, true, bitwidth, N, H, W, C, dev_QX, dev_BTN, nullptr, stream);
+}
+
+size_t tab_quantize_workspace_bytes(int bitwidth, int N, int H, int W, int C)
+{
+    if (N < 1 || H < 1 || W < 1 || C < 1) return 0;
+    return tab::quantize_count_workspace(bitwidth, N, (long)H * W, C);
+}
+
+int tab_quantize_counted(const float *dev_X, const float *dev_ths, int nchw, int bitwidth, int N, int H, int W, int C, int64_t *dev_QX,
+                         int32_t *dev_BTN, void *workspace, size_t workspace_bytes, void *stream)
+{
+    if (!dev_BTN) return fail(TAB_ERR_BAD_ARGUMENT, "null device pointer");
+    const size_t need = tab_quantize_workspace_bytes(bitwidth, N, H, W, C);
+    if (need && (!workspace || workspace_bytes < need || ((uintptr_t)workspace % 4)))
+        return fail(TAB_ERR_WORKSPACE, "workspace must hold %zu bytes (got %zu)", need, workspace_bytes);
+    return quantize_any(dev_X, dev_ths, nchw != 0, bitwidth, N, H, W, C, dev_QX, dev_BTN, need ? static_cast<int32_t *>(workspace) : nullptr, stream);
 }
 
 size_t tab_threshold_workspace_bytes(int N, long per_item)
@@ -375,7 +391,7 @@ static int conv_from_nhwc(const float *dev_X, const int64_t *dev_QW, const tab::
     }
     // stage 1: quantize + pack the activation (TAB_GEMM.cu:419-426); no btn for activations
     hipError_t e = tab::launch_quantize(dev_X, ths, s.abits, (long)H * W, N, C, reinterpret_cast<uint64_t *>(workspace), nullptr,
-                                        static_cast<hipStream_t>(stream));
+                                        nullptr, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return device_fail(e, "quantize launch");
     // stage 2: pad + im2row + GEMM, fused
     return tab_conv2d_packed(reinterpret_cast<const int64_t *>(workspace), dev_QW, dev_btn, type,
@@ -456,8 +472,8 @@ int tab_layer_quantize(const float *dev_X, int nchw, int bitwidth, float act_sca
     if (e != hipSuccess) return device_fail(e, "threshold launch");
     uint64_t *q = reinterpret_cast<uint64_t *>(dev_QX);
     // one pixel per image: NCHW and NHWC are the same memory, and the NHWC quantizers read it along the channels
-    e = nchw && H * W > 1 ? tab::launch_quantize_nchw(dev_X, ths, bitwidth, N, C, (long)H * W, q, nullptr, static_cast<hipStream_t>(stream))
-                          : tab::launch_quantize(dev_X, ths, bitwidth, (long)H * W, N, C, q, nullptr, static_cast<hipStream_t>(stream));
+    e = nchw && H * W > 1 ? tab::launch_quantize_nchw(dev_X, ths, bitwidth, N, C, (long)H * W, q, nullptr, nullptr, static_cast<hipStream_t>(stream))
+                          : tab::launch_quantize(dev_X, ths, bitwidth, (long)H * W, N, C, q, nullptr, nullptr, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return device_fail(e, "quantize launch");
     return TAB_OK;
 }

@@ -209,12 +209,15 @@ struct Thresholds {
 constexpr int kOwnPixelThresholds = -1;  // splits, conv_small only: images of one pixel, the kernel adds up |x| itself
 inline Thresholds given_thresholds(const float *ths) { return Thresholds{ths, 0.0, 0}; }
 
+// count_workspace: quantize_count_workspace bytes for the counts of two planes, or null (they are then taken from the packed
+// output, one launch more)
+size_t quantize_count_workspace(int bitwidth, long items, long pixels_per_item, int C);
 hipError_t launch_quantize(const float *x, const Thresholds &ths, int bitwidth, long pixels_per_item,
-                           long items, int C, uint64_t *qx, int32_t *btn, hipStream_t stream);
+                           long items, int C, uint64_t *qx, int32_t *btn, int32_t *count_workspace, hipStream_t stream);
 
 // The same quantizer reading x as [N][C][H*W] (the CPU path's input layout, TAB_CPU.cpp:20-206); output as above.
 hipError_t launch_quantize_nchw(const float *x, const Thresholds &ths, int bitwidth, int N, int C, long HW, uint64_t *qx,
-                                int32_t *btn, hipStream_t stream);
+                                int32_t *btn, int32_t *count_workspace, hipStream_t stream);
 
 // Packers of the CPU-only conv types: format 4 = DoReFa 2-bit levels, 5 = RTN fields.
 hipError_t launch_quantize_format(const float *x, const float *ths, int format, long pixels_per_item, long items, int C,

@@ -36,6 +36,51 @@ __device__ __forceinline__ void zero_counts(int32_t *btn, long items, long first
         if (first + i < items) btn[first + i] = 0;
 }
 
+// Counts of nonzero values made by the quantizer itself (template parameter COUNT, two planes): each item is cut into
+// `slices` workgroups, a workgroup takes the slice's units (what it quantizes in one go) `slices` apart and stores their
+// count, in btn where an item is one slice, else in a workspace from where count_finish adds the slices up.  Reading the packed
+// output back for the counts instead took a launch of 4.8-9.6 us behind every two-plane quantizer, a third of the whole for
+// tensors of 10-20 MB.
+struct Counts {
+    int32_t *out;  // [items * slices]
+    int slices;
+};
+
+// The sum of `count` over the workgroup, stored by one thread.  scratch: a dword per wave, free to overwrite.
+template <int WAVES>
+__device__ __forceinline__ void store_count(int count, int32_t *out, int32_t *scratch)
+{
+    count = wave_sum(count);
+    if (WAVES == 1) {
+        if (threadIdx.x == 0) *out = count;
+        return;
+    }
+    if ((threadIdx.x & 63) == 0) scratch[threadIdx.x >> 6] = count;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int total = 0;
+#pragma unroll
+        for (int w = 0; w < WAVES; w++) total += scratch[w];
+        *out = total;
+    }
+}
+
+// One workgroup per item; four counts in flight a thread (one wave with a count at a time took 5 us for 700).
+__global__ __launch_bounds__(kThreads) void count_finish(const int32_t *__restrict__ counts, int32_t *__restrict__ btn, int slices)
+{
+    __shared__ int32_t scratch[kWavesPerBlock];
+    const int32_t *src = counts + (long)blockIdx.x * slices;
+    int count = 0;
+    for (int i = threadIdx.x; i < slices; i += 4 * kThreads) {
+        int32_t v[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) v[u] = src[i + u * kThreads < slices ? i + u * kThreads : i];
+#pragma unroll
+        for (int u = 0; u < 4; u++) count += i + u * kThreads < slices ? v[u] : 0;
+    }
+    store_count<kWavesPerBlock>(count, btn + blockIdx.x, scratch);
+}
+
 // Fast path, C % 64 == 0 and X 16-byte aligned.
 // Lane layout: a 16-lane DPP row reads one 64-channel row as 16 float4 (256 B contiguous),
 // a wave reads 4 consecutive rows per load (1 KB contiguous) and keeps kLoadsPerLane loads
@@ -142,6 +187,42 @@ __global__ __launch_bounds__(64) void quantize_rows64_strided(const floatx4 *__r
     }
 }
 
+// quantize_rows64 of two planes with counts (see Counts): a slice is one unit, 4 * LOADS rows of every wave.
+template <int LOADS, bool NT>
+__global__ __launch_bounds__(kThreads) void quantize_rows64_count(const floatx4 *__restrict__ x, const Thresholds ths, uint32_t *__restrict__ q,
+                                                                    long rows_per_item, const Counts counts)
+{
+    constexpr int UNIT = 4 * LOADS * kWavesPerBlock;
+    __shared__ int32_t scratch[kWavesPerBlock];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int sub = lane >> 4, l = lane & 15;
+    const int item = (int)(blockIdx.x / (uint32_t)counts.slices), slice = (int)blockIdx.x - item * counts.slices;
+    const long first = item * rows_per_item;
+    int count = 0;
+    const long at = (long)slice * UNIT + wave * (4 * LOADS);  // of the item's rows
+    if (at < rows_per_item) {
+        floatx4 v[LOADS];
+#pragma unroll
+        for (int u = 0; u < LOADS; u++) {
+            const long r = at + u * 4 + sub;
+            const floatx4 *src = &x[(first + (r < rows_per_item ? r : rows_per_item - 1)) * 16 + l];
+            v[u] = NT ? __builtin_nontemporal_load(src) : *src;
+        }
+        const float t = wave_threshold(ths, item);
+#pragma unroll
+        for (int u = 0; u < LOADS; u++) {
+            const long r = at + u * 4 + sub;
+            uint32_t sign, nz, out[4];
+            compare4<2>(v[u], t, sign, nz);
+            count += r < rows_per_item ? __builtin_popcount(nz) : 0;
+            pack_row<2>(sign, nz, l, out);
+            if (r < rows_per_item && l == 0) *reinterpret_cast<uintx4 *>(q + (first + r) * 4) = uintx4{out[0], out[1], out[2], out[3]};
+        }
+    }
+    store_count<kWavesPerBlock>(count, counts.out + blockIdx.x, scratch);
+}
+
 // Spread the 32 bits of v to the even bits of a 64-bit word.
 __device__ __forceinline__ uint64_t spread_bits(uint32_t v)
 {
@@ -169,21 +250,21 @@ __device__ __forceinline__ uint64_t spread_bits(uint32_t v)
 //    weight-1 bit of level = (v >= 0.5t) + (v >= 1.5t) + (v >= 2.5t);
 // 5, RTN (RTNGEMM_baseline, TAB_CPU.cpp:364-379; 32 channels per word, 520-521): [pixel][ceil(C/32)], channel c in word c/32
 //    as the field (bit 2*(c%32) = nonzero, bit 2*(c%32)+1 = sign) of the ternarizer's value.
+// One tile: `live` pixels from p0 on, `words` words a pixel from w0 on.  Returns how many of the values this lane stored are nonzero
+// (MODE 2).
 template <int MODE, int LP>
-__global__ __launch_bounds__(kThreads) void quantize_tile(const float *__restrict__ x, const Thresholds ths, uint64_t *__restrict__ q,
-                                                          long pixels, long pixels_per_item, Div32 div_item, int C, int tile_pixels, int words,
-                                                          int32_t *btn, long items)
+__device__ __forceinline__ int quantize_one_tile(const float *__restrict__ x, const Thresholds &ths, uint64_t *__restrict__ q, long p0, int live,
+                                                 long pixels_per_item, Div32 div_item, int C, int tile_pixels, int w0, int words)
 {
     constexpr int G = 64 / LP;  // rows per read
     constexpr int U = LP == 64 ? 4 : 2;  // reads in flight
     extern __shared__ __attribute__((aligned(16))) uint32_t tile[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const long p0 = (long)blockIdx.x * tile_pixels;
-    const int live = pixels - p0 < tile_pixels ? (int)(pixels - p0) : tile_pixels;  // pixels of the tile that exist
     const int PC = (C + kWordBits - 1) / kWordBits;
+    int count = 0;
     // words w0 ... of the pixel where one pixel is more than a tile (`words` of them), else all
-    const int w0 = blockIdx.y * words, PW = min(words, PC - w0), channels_here = min(C - w0 * kWordBits, PW * kWordBits);
+    const int PW = min(words, PC - w0), channels_here = min(C - w0 * kWordBits, PW * kWordBits);
 
     // ---- the run of x, from the 16-byte boundary at or below its start to its last float ----------------------------------
     const uintptr_t start = (uintptr_t)(x + p0 * C + w0 * kWordBits);
@@ -267,10 +348,39 @@ __global__ __launch_bounds__(kThreads) void quantize_tile(const float *__restric
                     if (2 * (w0 + w) + 1 < halves) dst[1] = spread_bits(out[3]) | spread_bits(out[1]) << 1;
                 } else {
                     *reinterpret_cast<uintx4 *>(q + 2 * at) = uintx4{out[0], out[1], out[2], out[3]};
+                    if (MODE == 2) count += __builtin_popcount(out[2]) + __builtin_popcount(out[3]);
                 }
             }
         }
-    for (int i = tid; i < live; i += kThreads) zero_counts(btn, items, p0 + i);
+    return count;
+}
+
+template <int MODE, int LP>
+__global__ __launch_bounds__(kThreads) void quantize_tile(const float *__restrict__ x, const Thresholds ths, uint64_t *__restrict__ q,
+                                                          long pixels, long pixels_per_item, Div32 div_item, int C, int tile_pixels, int words,
+                                                          int32_t *btn, long items)
+{
+    const long p0 = (long)blockIdx.x * tile_pixels;
+    const int live = pixels - p0 < tile_pixels ? (int)(pixels - p0) : tile_pixels;  // pixels of the tile that exist
+    quantize_one_tile<MODE, LP>(x, ths, q, p0, live, pixels_per_item, div_item, C, tile_pixels, blockIdx.y * words, words);
+    for (int i = threadIdx.x; i < live; i += kThreads) zero_counts(btn, items, p0 + i);
+}
+
+// The same with counts (see Counts); a unit is a tile of whole pixels.
+template <int LP>
+__global__ __launch_bounds__(kThreads) void quantize_tile_count(const float *__restrict__ x, const Thresholds ths, uint64_t *__restrict__ q,
+                                                                long pixels_per_item, Div32 div_item, int C, int tile_pixels, const Counts counts)
+{
+    __shared__ int32_t scratch[kWavesPerBlock];
+    const int item = (int)(blockIdx.x / (uint32_t)counts.slices), slice = (int)blockIdx.x - item * counts.slices;
+    int count = 0;
+    for (long at = (long)slice * tile_pixels; at < pixels_per_item; at += (long)counts.slices * tile_pixels) {
+        const int live = pixels_per_item - at < tile_pixels ? (int)(pixels_per_item - at) : tile_pixels;
+        if (at >= (long)counts.slices * tile_pixels) __syncthreads();  // the waves have read the tile before
+        count += quantize_one_tile<2, LP>(x, ths, q, item * pixels_per_item + at, live, pixels_per_item, div_item, C, tile_pixels, 0,
+                                          (C + kWordBits - 1) / kWordBits);
+    }
+    store_count<kWavesPerBlock>(count, counts.out + blockIdx.x, scratch);
 }
 
 // The same quantizers on an NCHW tensor, the layout the reference's CPU quantizers read
@@ -286,9 +396,10 @@ struct PixelRun {
     typedef float Vec __attribute__((ext_vector_type(VEC)));
     typedef Vec VecAnywhere __attribute__((aligned(4)));
     long n, s, pixel;  // image, first pixel in the image, first pixel counted through all images
+    int repeated;      // pixels at the run's start that the run before it has too (the per-image numbering only)
 
     // run `i` counted through all images; past the last one: the last one again, with the same results
-    __device__ __forceinline__ PixelRun(long i, int N, long HW)
+    __device__ __forceinline__ PixelRun(long i, int N, long HW) : repeated(0)
     {
         if (EVEN) {
             const long total = N * HW;
@@ -304,6 +415,14 @@ struct PixelRun {
             if (s > HW - VEC) s = HW - VEC;
             pixel = n * HW + s;
         }
+    }
+    // run `i` of image `image`
+    __device__ __forceinline__ PixelRun(long i, long image, long HW, std::true_type)
+    {
+        n = image;
+        s = i * VEC < HW - VEC ? i * VEC : HW - VEC;
+        pixel = n * HW + s;
+        repeated = i * VEC - s < VEC ? (int)(i * VEC - s) : VEC;
     }
     template <bool NT = false>
     __device__ __forceinline__ void load(float (&v)[VEC], const float *src) const
@@ -341,9 +460,10 @@ struct PixelRun {
 // (two planes) 6.1 -> 4.4 us, N=128 64 x 112 x 112 79.9 -> 72.4 (6.0 TB/s), N=64 3 x 112 x 112 16.6 -> 6.7.
 // grid = ceil(runs / (64 * 4 / SPLIT)) * PC workgroups, the word index fastest: the workgroups that write the PC words of the
 // same pixels run side by side, so their 8- or 16-byte stores meet in L2 as whole lines.
-template <int BITS, int VEC, int SPLIT, bool NT = false>
-__global__ __launch_bounds__(kThreads) void quantize_nchw(const float *__restrict__ x, const Thresholds ths,
-                                                          uint64_t *__restrict__ q, int N, int C, long HW, int PC, int32_t *btn)
+// The lane's nonzero values are counted for COUNT (see Counts).
+template <int BITS, int VEC, int SPLIT, bool NT>
+__device__ __forceinline__ int quantize_nchw_unit(const float *__restrict__ x, const Thresholds &ths, uint64_t *__restrict__ q, const PixelRun<VEC> &run,
+                                                  int C, long HW, int PC, int pc)
 {
     constexpr int kPart = 16;                       // channels a wave packs of its pixels
     constexpr int GROUPS = kWavesPerBlock / SPLIT;  // of 64 pixel runs, per workgroup
@@ -355,8 +475,6 @@ __global__ __launch_bounds__(kThreads) void quantize_nchw(const float *__restric
     __shared__ alignas(16) uint16_t parts[GROUPS][SPLIT][BITS][SLOTS];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int part = wave % SPLIT, group = wave / SPLIT;
-    const int pc = blockIdx.x % PC;
-    const PixelRun<VEC> run((blockIdx.x / PC * GROUPS + group) * 64L + lane, N, HW);
     const int c0 = pc * kWordBits + part * kPart;
     const int channels = C - c0 < kPart ? C - c0 : kPart;  // zero or less: no such part
     uint32_t less[VEC], more[VEC];
@@ -432,8 +550,39 @@ __global__ __launch_bounds__(kThreads) void quantize_nchw(const float *__restric
 #pragma unroll
         for (int b = 0; b < BITS; b++) dst[b] = word[b];
     }
-    if (part == 0) zero_counts(btn, N, run.pixel, VEC);
+    int count = 0;
+#pragma unroll
+    for (int e = 0; e < VEC; e++) count += e >= run.repeated ? __builtin_popcount((uint32_t)nz[e]) : 0;
+    return count;
 }
+
+template <int BITS, int VEC, int SPLIT, bool NT = false>
+__global__ __launch_bounds__(kThreads) void quantize_nchw(const float *__restrict__ x, const Thresholds ths,
+                                                          uint64_t *__restrict__ q, int N, int C, long HW, int PC, int32_t *btn)
+{
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const PixelRun<VEC> run((blockIdx.x / PC * (kWavesPerBlock / SPLIT) + wave / SPLIT) * 64L + (threadIdx.x & 63), N, HW);
+    quantize_nchw_unit<BITS, VEC, SPLIT, NT>(x, ths, q, run, C, HW, PC, blockIdx.x % PC);
+    if (wave % SPLIT == 0) zero_counts(btn, N, run.pixel, VEC);
+}
+
+// The same with counts: a unit is 64 * 4 / SPLIT runs and one word.
+template <int VEC, int SPLIT, bool NT = false>
+__global__ __launch_bounds__(kThreads) void quantize_nchw_count(const float *__restrict__ x, const Thresholds ths, uint64_t *__restrict__ q, int C,
+                                                                long HW, int PC, int units, const Counts counts)
+{
+    __shared__ int32_t scratch[kWavesPerBlock];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int item = (int)(blockIdx.x / (uint32_t)counts.slices), slice = (int)blockIdx.x - item * counts.slices;
+    int count = 0;
+    for (int unit = slice; unit < units; unit += counts.slices) {
+        if (unit >= counts.slices) __syncthreads();  // the waves have read the words before
+        const PixelRun<VEC> run((unit / PC * (kWavesPerBlock / SPLIT) + wave / SPLIT) * 64L + (threadIdx.x & 63), item, HW, std::true_type());
+        count += quantize_nchw_unit<2, VEC, SPLIT, NT>(x, ths, q, run, C, HW, PC, unit % PC);
+    }
+    store_count<kWavesPerBlock>(count, counts.out + blockIdx.x, scratch);
+}
+
 
 // The NCHW quantizer for PC a multiple of U = 2 or 4 and at least one wave of work per SIMD: a thread packs U
 // neighbouring words of its four pixels, one after the other, and the wave then turns its 256 pixels x U words
@@ -445,10 +594,12 @@ __global__ __launch_bounds__(kThreads) void quantize_nchw(const float *__restric
 // One wave per workgroup (with four, the 784 workgroups of that tensor load the CUs 4 : 3), 4 KB of LDS, gone through
 // in WPP / 2 rounds of 64 / rounds lanes each.  grid = ceil(runs / 64) * (PC / U), the word group fastest.
 // Bits are made by the form and in as many registers as measured best: SHIFT for U = 2.
-template <int BITS, int U, bool EVEN>
+// COUNT: a wave is a slice of one unit (see Counts).
+template <int BITS, int U, bool EVEN, bool COUNT = false>
 __global__ __launch_bounds__(64, BITS == 1 ? (U == 4 ? 4 : 7) : (U == 4 ? 1 : 4)) void quantize_nchw_gather(const float *__restrict__ x, const Thresholds ths,
                                                                  uint64_t *__restrict__ q, int N, int C, long HW, int PC, int32_t *btn)
 {
+    static_assert(!COUNT || BITS == 2, "counts of two planes");
     constexpr int VEC = 4, kInFlight = 8;
     constexpr int WPP = U * BITS;      // words a thread packs per pixel, contiguous in q
     constexpr int ROUNDS = WPP / 2;    // 64 / ROUNDS lanes x 4 pixels x WPP words = 512 words a round
@@ -457,9 +608,13 @@ __global__ __launch_bounds__(64, BITS == 1 ? (U == 4 ? 4 : 7) : (U == 4 ? 1 : 4)
     static_assert(U == 2 || U == 4, "one word per thread is quantize_nchw");
     __shared__ __attribute__((aligned(16))) uint64_t stage[512];
     const int groups = PC / U;
-    const int pc0 = (blockIdx.x % groups) * U;
+    // COUNT: N is the number of slices of an image
+    const int image = COUNT ? (int)(blockIdx.x / (uint32_t)N) : 0;
+    const int unit = (int)blockIdx.x - image * N * COUNT;
+    const int pc0 = (unit % groups) * U;
     const int lane = threadIdx.x;
-    const PixelRun<VEC, EVEN> run((long)(blockIdx.x / groups) * 64 + lane, N, HW);
+    const PixelRun<VEC, EVEN> run = COUNT ? PixelRun<VEC, EVEN>((long)(unit / groups) * 64 + lane, image, HW, std::true_type())
+                                          : PixelRun<VEC, EVEN>((long)(unit / groups) * 64 + lane, N, HW);
     // The U words are U * 64 consecutive channels: batches of kInFlight channels, the next batch's loads issued before
     // the compares of this one (two register buffers), so the memory pipe never waits for the packing.
     const int cbase = pc0 * kWordBits;
@@ -571,7 +726,16 @@ __global__ __launch_bounds__(64, BITS == 1 ? (U == 4 ? 4 : 7) : (U == 4 ? 1 : 4)
             if (pixel < last) *reinterpret_cast<ulonglong2 *>(q + (pixel * PC + pc0) * BITS + w % WPP) = pair;
         }
     }
-    zero_counts(btn, N, run.pixel, VEC);
+    if (COUNT) {
+        int count = 0;
+#pragma unroll
+        for (int e = 0; e < VEC; e++)
+#pragma unroll
+            for (int u = 0; u < U; u++) count += e >= run.repeated ? __popcll(words[e][u * BITS + BITS - 1]) : 0;
+        store_count<1>(count, btn + blockIdx.x, nullptr);
+    } else {
+        zero_counts(btn, N, run.pixel, VEC);
+    }
 }
 
 // btn[n] = sum over item n of popcount(nonzero-plane word) (BTN_Weight, TAB_GEMM.cu:150-160,
@@ -732,9 +896,21 @@ void launch_btn_popcount(const uint64_t *qx, int32_t *btn, long items, long word
                                                                                words_per_item, splits, threads);
 }
 
+// Where the counts of a two-plane quantizer go: an item of this many units is one slice (a unit takes some 0.7 us, count_finish
+// 2.4), others are slices of one unit each, whose counts need `workspace`; null: none there, the packed output is read back.
+struct CountTarget {
+    int32_t *btn, *workspace;
+};
+constexpr long kOneSliceUnits = 3;
+
+void finish_counts(const CountTarget &target, long items, int slices, hipStream_t stream)
+{
+    if (slices > 1) count_finish<<<dim3((unsigned)items), dim3(kThreads), 0, stream>>>(target.workspace, target.btn, slices);
+}
+
 template <int MODE, int LP>
 void launch_quantize_tile_of(const float *x, const Thresholds &ths, long pixels, long pixels_per_item, long items, int C, uint64_t *q,
-                             int32_t *btn, hipStream_t stream)
+                             int32_t *btn, const CountTarget *counted, hipStream_t stream)
 {
     // Bytes of x in a tile, measured from 4 to 48 KB on C = 3 ... 700: what a few workgroups a CU keep in flight against the
     // wait of each for its whole tile.  The pixels are shared by four waves in turns of U reads, so sixteen (a turn of four
@@ -745,31 +921,49 @@ void launch_quantize_tile_of(const float *x, const Thresholds &ths, long pixels,
     // a pixel of more than 3072 channels goes in parts of 64 words
     const int words = C <= 3072 ? PC : 64;
     long tile_pixels = C > 3072 ? 1 : (fit >= 16 ? fit / 16 * 16 : (C <= 768 ? 16 : 4));
+    const bool one_slice = counted && pixels_per_item <= kOneSliceUnits * tile_pixels;
     // a tensor of few tiles: smaller ones, down to a read of every wave
-    while (tile_pixels >= 8 && pixels / tile_pixels < 512 && tile_pixels / 2 >= 4 * (64 / LP)) tile_pixels = tile_pixels / 8 * 4;
+    while (!one_slice && tile_pixels >= 8 && pixels / tile_pixels < 512 && tile_pixels / 2 >= 4 * (64 / LP)) tile_pixels = tile_pixels / 8 * 4;
     const long run = C > 3072 ? words * kWordBits : tile_pixels * C;
     const size_t lds = ((size_t)(run + 6) / 4 * 4 + 256 + tile_pixels) * 4;
-    const dim3 grid((unsigned)((pixels + tile_pixels - 1) / tile_pixels), (unsigned)((PC + words - 1) / words));
     const Div32 div_item = pixels < 0x7fffffffL ? make_div32((uint32_t)pixels_per_item) : Div32{0, 0};
+    if constexpr (MODE == 2) {
+        if (counted) {
+            const long slices = one_slice ? 1 : (pixels_per_item + tile_pixels - 1) / tile_pixels;
+            quantize_tile_count<LP><<<dim3((unsigned)(items * slices)), dim3(kThreads), lds, stream>>>(
+                x, ths, q, pixels_per_item, div_item, C, (int)tile_pixels, Counts{slices == 1 ? counted->btn : counted->workspace, (int)slices});
+            finish_counts(*counted, items, (int)slices, stream);
+            return;
+        }
+    }
+    const dim3 grid((unsigned)((pixels + tile_pixels - 1) / tile_pixels), (unsigned)((PC + words - 1) / words));
     quantize_tile<MODE, LP><<<grid, dim3(kThreads), lds, stream>>>(x, ths, q, pixels, pixels_per_item, div_item, C, (int)tile_pixels, words, btn, items);
 }
 
 // The general path with the fewest lanes a word that hold it.
 template <int MODE>
 void launch_quantize_tile(const float *x, const Thresholds &ths, long pixels, long pixels_per_item, long items, int C, uint64_t *q,
-                          int32_t *btn, hipStream_t stream)
+                          int32_t *btn, const CountTarget *counted, hipStream_t stream)
 {
-    if (C <= 4) launch_quantize_tile_of<MODE, 4>(x, ths, pixels, pixels_per_item, items, C, q, btn, stream);
-    else if (C <= 8) launch_quantize_tile_of<MODE, 8>(x, ths, pixels, pixels_per_item, items, C, q, btn, stream);
-    else if (C <= 16) launch_quantize_tile_of<MODE, 16>(x, ths, pixels, pixels_per_item, items, C, q, btn, stream);
-    else if (C <= 32) launch_quantize_tile_of<MODE, 32>(x, ths, pixels, pixels_per_item, items, C, q, btn, stream);
-    else launch_quantize_tile_of<MODE, 64>(x, ths, pixels, pixels_per_item, items, C, q, btn, stream);
+    if (C <= 4) launch_quantize_tile_of<MODE, 4>(x, ths, pixels, pixels_per_item, items, C, q, btn, counted, stream);
+    else if (C <= 8) launch_quantize_tile_of<MODE, 8>(x, ths, pixels, pixels_per_item, items, C, q, btn, counted, stream);
+    else if (C <= 16) launch_quantize_tile_of<MODE, 16>(x, ths, pixels, pixels_per_item, items, C, q, btn, counted, stream);
+    else if (C <= 32) launch_quantize_tile_of<MODE, 32>(x, ths, pixels, pixels_per_item, items, C, q, btn, counted, stream);
+    else launch_quantize_tile_of<MODE, 64>(x, ths, pixels, pixels_per_item, items, C, q, btn, counted, stream);
+}
+
+// Counts of every two-plane quantizer in slices: workspace ints at most (a unit holds at least four words).
+size_t quantize_count_workspace(int bitwidth, long items, long pixels_per_item, int C)
+{
+    const long PC = (C + kWordBits - 1) / kWordBits;
+    if (bitwidth != 2 || (pixels_per_item * PC <= 64 && PC <= kOneSliceUnits)) return 0;  // one slice in every form
+    return (size_t)items * (pixels_per_item * PC / 4 + PC + 1) * sizeof(int32_t);
 }
 
 // x: fp32 [items][pixels_per_item][C]; qx: [items*pixels_per_item][PC][bitwidth];
 // btn: [items] or nullptr (then no counts are produced).
 hipError_t launch_quantize(const float *x, const Thresholds &ths, int bitwidth, long pixels_per_item,
-                           long items, int C, uint64_t *qx, int32_t *btn, hipStream_t stream)
+                           long items, int C, uint64_t *qx, int32_t *btn, int32_t *count_workspace, hipStream_t stream)
 {
     const int PC = (C + kWordBits - 1) / kWordBits;
     const long pixels = items * pixels_per_item;
@@ -778,6 +972,28 @@ hipError_t launch_quantize(const float *x, const Thresholds &ths, int bitwidth, 
     // counts that are not stored whole by btn_popcount start at zero
     int32_t *zeroed = btn && (bitwidth != 2 || splits > 1) ? btn : nullptr;
     const bool fast = (C % kWordBits == 0) && ((uintptr_t)x % 16 == 0);
+    const CountTarget target{btn, count_workspace};
+    const bool counted = btn && bitwidth == 2 && items * (words_per_item / 4 + 1) < 0x7fffffffL &&
+                         (count_workspace || (words_per_item <= 64 && PC <= kOneSliceUnits));
+    if (counted && fast) {
+        const floatx4 *x4 = reinterpret_cast<const floatx4 *>(x);
+        uint32_t *q32 = reinterpret_cast<uint32_t *>(qx);
+        auto launch = [&](auto kernel, long rows) {
+            const long slices = (words_per_item + rows - 1) / rows;
+            kernel<<<dim3((unsigned)(items * slices)), dim3(kThreads), 0, stream>>>(
+                x4, ths, q32, words_per_item, Counts{slices == 1 ? btn : count_workspace, (int)slices});
+            finish_counts(target, items, (int)slices, stream);
+        };
+        // (units of 128 rows for streaming and 32 for launches too small to fill the chip, as below)
+        if (words_per_item > 32 && words_per_item <= 128) launch(quantize_rows64_count<8, false>, 128);
+        else if (items * words_per_item <= kSmallLaunchBlocks * 128) launch(quantize_rows64_count<2, false>, 32);
+        else launch(quantize_rows64_count<8, true>, 128);
+        return hipGetLastError();
+    }
+    if (counted && C <= 3072) {
+        launch_quantize_tile<2>(x, ths, pixels, pixels_per_item, items, C, qx, nullptr, &target, stream);
+        return hipGetLastError();
+    }
     if (fast) {
         const long rows = pixels * PC;
         const Div32 div_item = rows < 0x7fffffffL ? make_div32((uint32_t)words_per_item) : Div32{0, 0};
@@ -801,16 +1017,16 @@ hipError_t launch_quantize(const float *x, const Thresholds &ths, int bitwidth, 
                 quantize_rows64<1><<<grid, block, 0, stream>>>(x4, ths, q32, rows, words_per_item, div_item, zeroed, items);
         }
     } else if (bitwidth == 2) {
-        launch_quantize_tile<2>(x, ths, pixels, pixels_per_item, items, C, qx, zeroed, stream);
+        launch_quantize_tile<2>(x, ths, pixels, pixels_per_item, items, C, qx, zeroed, nullptr, stream);
     } else {
-        launch_quantize_tile<1>(x, ths, pixels, pixels_per_item, items, C, qx, zeroed, stream);
+        launch_quantize_tile<1>(x, ths, pixels, pixels_per_item, items, C, qx, zeroed, nullptr, stream);
     }
     if (btn && bitwidth == 2) launch_btn_popcount(qx, btn, items, words_per_item, splits, stream);
     return hipGetLastError();
 }
 
 hipError_t launch_quantize_nchw(const float *x, const Thresholds &ths, int bitwidth, int N, int C, long HW, uint64_t *qx,
-                                int32_t *btn, hipStream_t stream)
+                                int32_t *btn, int32_t *count_workspace, hipStream_t stream)
 {
     const int PC = (C + kWordBits - 1) / kWordBits;
     const long words_per_item = HW * PC;
@@ -818,6 +1034,8 @@ hipError_t launch_quantize_nchw(const float *x, const Thresholds &ths, int bitwi
     int32_t *zeroed = btn && (bitwidth != 2 || splits > 1) ? btn : nullptr;
     const long pixels = (long)N * HW;
     const long runs = N * ((HW + 3) / 4);
+    const bool counted = btn && bitwidth == 2 && (count_workspace || (words_per_item <= 64 && PC <= kOneSliceUnits)) &&
+                         N * (HW / 4 + 1) * PC < 0x7fffffffL;
     auto launch = [&](auto kernel, long blocks, int threads) {
         kernel<<<dim3((unsigned)blocks), dim3(threads), 0, stream>>>(x, ths, qx, N, C, HW, PC, zeroed);
     };
@@ -825,7 +1043,18 @@ hipError_t launch_quantize_nchw(const float *x, const Thresholds &ths, int bitwi
     const int unit = PC % 4 == 0 ? 4 : PC % 2 == 0 ? 2 : 1;
     const long gather_waves = (runs + 63) / 64 * (PC / unit);
     if (gather_waves > 0x7fffffffL) return hipErrorInvalidValue;
-    if (HW >= 4 && (uintptr_t)qx % 16 == 0 && unit > 1 && gather_waves >= 1024) {
+    const long gather_slices = (runs / N + 63) / 64 * (PC / unit);
+    if (HW >= 4 && (uintptr_t)qx % 16 == 0 && unit > 1 && gather_waves >= 1024 && !(counted && gather_slices > 1 && !count_workspace)) {
+        if (counted) {
+            const long slices = gather_slices;
+            auto launch_counted = [&](auto kernel) {
+                kernel<<<dim3((unsigned)(N * slices)), dim3(64), 0, stream>>>(x, ths, qx, (int)slices, C, HW, PC, slices == 1 ? btn : count_workspace);
+            };
+            if (unit == 4) launch_counted(HW % 4 ? quantize_nchw_gather<2, 4, false, true> : quantize_nchw_gather<2, 4, true, true>);
+            else launch_counted(HW % 4 ? quantize_nchw_gather<2, 2, false, true> : quantize_nchw_gather<2, 2, true, true>);
+            finish_counts(CountTarget{btn, count_workspace}, N, (int)slices, stream);
+            return hipGetLastError();
+        }
         if (unit == 4 && bitwidth == 2) launch(HW % 4 ? quantize_nchw_gather<2, 4, false> : quantize_nchw_gather<2, 4, true>, gather_waves, 64);
         else if (unit == 4) launch(HW % 4 ? quantize_nchw_gather<1, 4, false> : quantize_nchw_gather<1, 4, true>, gather_waves, 64);
         else if (bitwidth == 2) launch(HW % 4 ? quantize_nchw_gather<2, 2, false> : quantize_nchw_gather<2, 2, true>, gather_waves, 64);
@@ -835,11 +1064,27 @@ hipError_t launch_quantize_nchw(const float *x, const Thresholds &ths, int bitwi
         const int split = C <= 16 ? 1 : C <= 32 ? 2 : 4;
         // One pixel a thread until four give two waves per SIMD (32 x 64 x 56 x 56: 4.4 us, with four 4.8; 53 MB of 57 x 57
         // planes: 14.1 us, with four 11.9).
-        const bool four = HW >= 4 && (runs + 63) / 64 * PC * split >= 2048;
+        bool four = HW >= 4 && (runs + 63) / 64 * PC * split >= 2048;
         // Past the caches where the tensor is large next to them and a wave reads whole lines, i.e. its kilobyte of a plane
         // is not mostly a plane's end: 128 x 64 x 112 x 112 73.6 -> 67.6 us, but 128 x 512 x 28 x 28 38.9 -> 44.5.
         const bool stream_past = four && split == 4 && pixels * C >= (8L << 20) && HW >= 2048;
         const int groups = kWavesPerBlock / split;
+        // counted: units end with the image, and a last one that is mostly empty weighs more with four
+        const long padded1 = (HW + 64 * groups - 1) / (64 * groups), padded4 = (HW + 256 * groups - 1) / (256 * groups) * 4;
+        if (counted && HW % 4 == 0 && padded1 * 8 < padded4 * 7) four = false;
+        if (counted) {
+            const long units = ((four ? runs / N : HW) + 64 * groups - 1) / (64 * groups) * PC;
+            const int slices = units <= kOneSliceUnits ? 1 : (int)units;
+            auto launch_counted = [&](auto kernel) {
+                kernel<<<dim3((unsigned)(N * slices)), dim3(kThreads), 0, stream>>>(x, ths, qx, C, HW, PC, (int)units,
+                                                                                   Counts{slices == 1 ? btn : count_workspace, slices});
+            };
+            if (stream_past) launch_counted(quantize_nchw_count<4, 4, true>);
+            else if (four) launch_counted(split == 4 ? quantize_nchw_count<4, 4> : split == 2 ? quantize_nchw_count<4, 2> : quantize_nchw_count<4, 1>);
+            else launch_counted(split == 4 ? quantize_nchw_count<1, 4> : split == 2 ? quantize_nchw_count<1, 2> : quantize_nchw_count<1, 1>);
+            finish_counts(CountTarget{btn, count_workspace}, N, slices, stream);
+            return hipGetLastError();
+        }
         const long blocks = ((four ? runs : pixels) + 64 * groups - 1) / (64 * groups) * PC;
         if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
         auto pick = [&](auto one, auto two) { launch(bitwidth == 2 ? two : one, blocks, kThreads); };
@@ -883,8 +1128,8 @@ hipError_t launch_quantize_format(const float *x, const float *ths_values, int f
         }
         return hipGetLastError();
     }
-    if (format == 4) launch_quantize_tile<4>(x, ths, pixels, pixels_per_item, items, C, qx, nullptr, stream);
-    else launch_quantize_tile<5>(x, ths, pixels, pixels_per_item, items, C, qx, nullptr, stream);
+    if (format == 4) launch_quantize_tile<4>(x, ths, pixels, pixels_per_item, items, C, qx, nullptr, nullptr, stream);
+    else launch_quantize_tile<5>(x, ths, pixels, pixels_per_item, items, C, qx, nullptr, nullptr, stream);
     return hipGetLastError();
 }
 

@@ -78,6 +78,19 @@ private:
     void *ptr_;
 };
 
+void quantize_counted(const torch::Tensor &X, const torch::Tensor &thresholds, bool nchw, int bitwidth, int N, int H, int W, int C,
+                      const torch::Tensor &QX, const torch::Tensor &BTN)
+{
+    const hipStream_t stream = current_stream(X);
+    const size_t bytes = tab_quantize_workspace_bytes(bitwidth, N, H, W, C);
+    auto call = [&](void *workspace) {
+        check_status(tab_quantize_counted(X.data_ptr<float>(), thresholds.data_ptr<float>(), nchw, bitwidth, N, H, W, C, QX.data_ptr<int64_t>(),
+                                          BTN.data_ptr<int32_t>(), workspace, bytes, stream));
+    };
+    if (bytes) call(Workspace(bytes, stream).get());
+    else call(nullptr);
+}
+
 }  // namespace
 
 std::vector<torch::Tensor> TAB_Quantize(const torch::Tensor &X, const torch::Tensor &thresholds, int bitwidth, int N,
@@ -97,8 +110,7 @@ std::vector<torch::Tensor> TAB_Quantize(const torch::Tensor &X, const torch::Ten
     const int PC = tab_packed_channels(C);
     auto QX = device_empty({N, H, W, PC, bitwidth}, torch::kInt64, X);
     auto BTN = device_empty({N}, torch::kInt32, X);
-    check_status(tab_quantize(X.data_ptr<float>(), thresholds.data_ptr<float>(), bitwidth, N, H, W, C,
-                              QX.data_ptr<int64_t>(), BTN.data_ptr<int32_t>(), current_stream(X)));
+    quantize_counted(X, thresholds, false, bitwidth, N, H, W, C, QX, BTN);
     return {QX, BTN};
 }
 
@@ -185,8 +197,7 @@ std::vector<torch::Tensor> TAB_QuantizeNCHW(const torch::Tensor &X, const torch:
     const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(X.device());
     auto QX = device_empty({N, H, W, tab_packed_channels(C), bitwidth}, torch::kInt64, X);
     auto BTN = device_empty({N}, torch::kInt32, X);
-    check_status(tab_quantize_nchw(X.data_ptr<float>(), thresholds.data_ptr<float>(), bitwidth, N, C, H, W,
-                                   QX.data_ptr<int64_t>(), BTN.data_ptr<int32_t>(), current_stream(X)));
+    quantize_counted(X, thresholds, true, bitwidth, N, H, W, C, QX, BTN);
     return {QX, BTN};
 }
 
