@@ -190,6 +190,8 @@ hipError_t launch_conv(int type, const ConvArgs &args, hipStream_t stream);
 bool conv_mfma_exact(const ConvArgs &args);
 bool conv_mfma_exact_levels(const ConvArgs &args);  // the same for type 4, whose products reach 9
 int conv_mfma_shape(int type, const ConvArgs &args, float *cost_us = nullptr);
+// At most 32 filters, fp32 output, an even number of words per pixel: the shapes of 64 filters that exist in a form of 32.
+inline bool conv_mfma_narrow(const ConvArgs &a) { return a.KN <= 32 && a.PC % 2 == 0 && a.qy == nullptr; }
 hipError_t launch_conv_mfma(int type, const ConvArgs &args, int shape, hipStream_t stream);
 hipError_t launch_conv_mfma_tnn(const ConvArgs &args, int shape, hipStream_t stream);
 hipError_t launch_conv_mfma_tbn(const ConvArgs &args, int shape, hipStream_t stream);

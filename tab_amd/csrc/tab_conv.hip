@@ -414,6 +414,7 @@ int conv_mfma_shape(int type, const ConvArgs &a, float *cost_us)
     }
     const long kn64 = ((long)a.KN + 63) / 64 * 64;
     const long cus = device_compute_units();
+    const bool narrow = conv_mfma_narrow(a);
     // (packed output ranks the shapes as fp32 output does: the model's terms in Y also stand for what grows with M * KN)
     const float y_mb = (float)a.M * (float)a.KN * 4e-6f;
     const float words = type == 5 ? 0.5f * (float)a.G : (float)a.G;  // of 64 elements
@@ -449,6 +450,10 @@ int conv_mfma_shape(int type, const ConvArgs &a, float *cost_us)
             for (int k = 0; k < kConvShapeFeatures; k++) cost += kConvShapeCost[type][i][k] * f[k];
             // the busiest CU's n tiles of (bm/32)(bn/32) MFMA tiles x words, 32 cycles each on four SIMDs at 2.4 GHz, and a launch
             floor_us = 1.f + n * (float)(bm / 32 * (bn / 32)) * words * (32.f / 4.f / 2400.f);
+        }
+        if (narrow && (shape == 1 || shape == 8)) {  // in their forms of 32 filters: what is above a launch, by a quarter less
+            if (cost > 3.f) cost = 3.f + 0.75f * (cost - 3.f);
+            floor_us = 1.f + 0.5f * (floor_us - 1.f);
         }
         if (cost < floor_us) cost = floor_us;
         if (!any || cost < best_cost) {

@@ -607,6 +607,8 @@ template <int TYPE, int WM, int WN, int TM, int TN, int KCH, int KS = 1, int ARU
 hipError_t launch_mfma_direct(ConvArgs a, hipStream_t stream);
 template <int TYPE, int WM, int WN, int TM, int TN, int KS, int WORDS>
 hipError_t launch_mfma_split(const ConvArgs &a, hipStream_t stream);
+template <int TYPE, int WM, int KS, int WORDS>
+hipError_t launch_mfma_narrow(const ConvArgs &a, hipStream_t stream);
 template <int TYPE>
 hipError_t launch_mfma_tail(ConvArgs a, hipStream_t stream);
 template <int TYPE>
@@ -656,11 +658,11 @@ hipError_t launch_mfma_shape(const ConvArgs &a, hipStream_t stream)
 template <int TYPE>
 hipError_t launch_mfma_regs(const ConvArgs &a, hipStream_t stream);
 
-// shape: 0 = 128x128, 1 = 128x64, 2 = 64x64 (rows x filters per workgroup), 3 = 32x32 with the four
+// shape: 0 = 128x128, 1 = 128x64 (conv_mfma_narrow: 128x32), 2 = 64x64 (rows x filters per workgroup), 3 = 32x32 with the four
 // waves splitting every chunk of four words between them, 4 = 256x64, 5 = 256x128 and 6 = 128x256
 // (eight MFMA tiles per wave: fewer operand expansions per MFMA, half the occupancy), 7 = the register-resident
 // short-K kernel (K of at most nine words; longer K falls back to the shape picked from the launch),
-// 8 = 64x64 with K split over the four waves (each wave 2x2 MFMA tiles over a quarter of every chunk), 9 = 128x128 with K
+// 8 = 64x64 (conv_mfma_narrow: 64x32) with K split over the four waves (each wave 2x2 MFMA tiles over a quarter of every chunk), 9 = 128x128 with K
 // split over two pairs of waves (each wave 2x4 MFMA tiles over half of every chunk); both need an even number of words per
 // pixel and otherwise run as shapes 2 and 0, 10 = 128x128 tiles for the whole rounds of the chip and 64x64 split-K quarters for
 // the rest of the last round (an even number of words per pixel; otherwise shape 0), 11 = the same with whole tiles of 128x256
@@ -684,6 +686,13 @@ hipError_t launch_mfma_type(const ConvArgs &a, int shape, hipStream_t stream)
     }
     if (shape == 8 && a.PC % 2 != 0) shape = 2;
     if (shape == 9 && a.PC % 2 != 0) shape = 0;
+    // Layers of at most 32 filters: half of a 64-filter tile would be work for nothing.  The tiles of 32 filters split K over
+    // two or four waves and keep two 32-row tiles a wave, three operand expansions for two MFMAs (a wave of one row and one
+    // filter tile makes four): N=45 56x56x384->7 3x3 TNN 28.6 us with 128x64, 26.3 with 64x64 split, 20.5 and 20.2 with these.
+    if (conv_mfma_narrow(a)) {
+        if (shape == 1) return launch_mfma_narrow<TYPE, 2, 2, 4>(a, stream);
+        if (shape == 8) return launch_mfma_narrow<TYPE, 1, 4, 2>(a, stream);
+    }
     switch (shape) {
     case 8: return launch_mfma_split<TYPE, 1, 1, 2, 2, 4, 2>(a, stream);
     case 9: return launch_mfma_split<TYPE, 2, 1, 2, 4, 2, 2>(a, stream);

@@ -81,7 +81,7 @@ __device__ __forceinline__ void conv_mfma_direct_tile(const ConvArgs &p, uint32_
     constexpr int A_ITEMS = (A_GRANULES + kConvThreads - 1) / kConvThreads, B_ITEMS = (B_GRANULES + kConvThreads - 1) / kConvThreads;
     constexpr int BUF_DWORDS = 4 * (A_ITEMS + B_ITEMS) * kConvThreads;  // whole wave instructions
     constexpr int A_RUN = ARUN ? ARUN : granule_run(PA, APL), B_RUN = granule_run(PB, BPL);
-    static_assert(BM % 64 == 0 && BN % 64 == 0, "one wave instruction moves 64 / RUN rows of one run");
+    static_assert(BM % (64 / A_RUN) == 0 && BN % (64 / B_RUN) == 0, "one wave instruction moves 64 / RUN rows of one run");
     static_assert(PA % A_RUN == 0, "whole runs");
 
     const int tid = threadIdx.x;
@@ -526,6 +526,7 @@ hipError_t launch_mfma_tail(ConvArgs a, hipStream_t stream)
 template <int TYPE, int WM, int WN, int TM, int TN, int KCH, int KS, int ARUN>
 hipError_t launch_mfma_direct(ConvArgs a, hipStream_t stream)
 {
+    constexpr bool kPackedOut = WN * TN % 2 == 0;  // whole words of packed output
     constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN;
     // words of a run of activation granules, which must not straddle filter taps
     constexpr int A_RUN_WORDS = (ARUN ? ARUN : granule_run(KCH * Planes<TYPE>::A / 2, Planes<TYPE>::A)) * (Planes<TYPE>::A == 1 ? 2 : 1);
@@ -536,7 +537,10 @@ hipError_t launch_mfma_direct(ConvArgs a, hipStream_t stream)
     const long blocks = order_workgroups<Planes<TYPE>::A>(a, (a.KN + BN - 1) / BN);
     if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
     if (a.qy != nullptr) {
-        conv_mfma_direct<TYPE, WM, WN, TM, TN, KCH, true, KS, ARUN><<<dim3((unsigned)blocks), dim3(kConvThreads), 0, stream>>>(pack_conv<TYPE, true>(a));
+        if constexpr (kPackedOut)
+            conv_mfma_direct<TYPE, WM, WN, TM, TN, KCH, true, KS, ARUN><<<dim3((unsigned)blocks), dim3(kConvThreads), 0, stream>>>(pack_conv<TYPE, true>(a));
+        else
+            return hipErrorInvalidValue;
     } else {
         conv_mfma_direct<TYPE, WM, WN, TM, TN, KCH, false, KS, ARUN><<<dim3((unsigned)blocks), dim3(kConvThreads), 0, stream>>>(pack_conv<TYPE, false>(a));
     }
@@ -559,6 +563,13 @@ hipError_t launch_mfma_split(const ConvArgs &a, hipStream_t stream)
     if constexpr (PA % 2 == 0)
         if (granules_per_pixel % 2 == 0) return launch_mfma_direct<TYPE, WM, WN, TM, TN, KCH, KS, 2>(a, stream);
     return launch_mfma_direct<TYPE, WM, WN, TM, TN, KCH, KS, 1>(a, stream);
+}
+
+// 32 filters a workgroup, K split over KS groups of WM waves.
+template <int TYPE, int WM, int KS, int WORDS>
+hipError_t launch_mfma_narrow(const ConvArgs &a, hipStream_t stream)
+{
+    return launch_mfma_split<TYPE, WM, 1, 2, 1, KS, WORDS>(a, stream);
 }
 
 }  // namespace
