@@ -1066,8 +1066,10 @@ hipError_t launch_quantize_nchw(const float *x, const Thresholds &ths, int bitwi
         // planes: 14.1 us, with four 11.9).
         bool four = HW >= 4 && (runs + 63) / 64 * PC * split >= 2048;
         // Past the caches where the tensor is large next to them and a wave reads whole lines, i.e. its kilobyte of a plane
-        // is not mostly a plane's end: 128 x 64 x 112 x 112 73.6 -> 67.6 us, but 128 x 512 x 28 x 28 38.9 -> 44.5.
-        const bool stream_past = four && split == 4 && pixels * C >= (8L << 20) && HW >= 2048;
+        // is not mostly a plane's end: 128 x 64 x 112 x 112 73.6 -> 67.6 us, but 128 x 512 x 28 x 28 38.9 -> 44.5.  Runs that straddle
+        // lines fetch them twice then, from HBM if x is larger than the 256 MB cache: N=64 57x57x64 11.2 -> 10.2, 75x75 17.0 -> 16.5,
+        // but N=40 151x151 (234 MB) 46.2 -> 48.3.
+        const bool stream_past = four && split == 4 && pixels * C >= (8L << 20) && HW >= 2048 && (HW % 4 == 0 || pixels * C < (32L << 20));
         const int groups = kWavesPerBlock / split;
         // counted: units end with the image, and a last one that is mostly empty weighs more with four
         const long padded1 = (HW + 64 * groups - 1) / (64 * groups), padded4 = (HW + 256 * groups - 1) / (256 * groups) * 4;
