@@ -419,7 +419,8 @@ static int conv_from_floats(const float *dev_X, const int64_t *dev_QW, const flo
     }
     rc = check_from_floats(s, type, dev_X, dev_QW, dev_btn, dev_Y, workspace, workspace_bytes, need);
     if (rc != TAB_OK) return rc;
-    if (type > 3) {  // the CPU-only types: their own packers, then the same fused kernel
+    if (type > 3 && !one_launch(type, dev_X, false, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, s)) {
+        // the CPU-only types: their own packers, then the same fused kernel
         hipError_t e = tab::launch_quantize_format(dev_X, dev_ths, type, (long)H * W, N, C, reinterpret_cast<uint64_t *>(workspace),
                                                    static_cast<hipStream_t>(stream));
         if (e != hipSuccess) return device_fail(e, "quantize launch");

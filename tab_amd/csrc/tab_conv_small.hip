@@ -1,4 +1,4 @@
-// Quantize + convolution in one launch for the smallest calls (types 0..3, any kernel, stride and padding): all stages of
+// Quantize + convolution in one launch for the smallest calls (all types, any kernel, stride and padding): all stages of
 // ConvWithCuda_TAB (TAB_GEMM.cu:419-509), the packed activation never reaching memory.
 //
 // Such a call is bound by what a launch costs the host (2.4-2.8 us each) and by the instructions a wave runs one after the
@@ -48,9 +48,12 @@ enum SmallInput {
 template <int TYPE, int INPUT, int PAIRS, bool WLDS>
 __global__ __launch_bounds__(kConvThreads) void conv_small(const SmallConvArgs p)
 {
-    static_assert(TYPE >= 0 && TYPE <= 3, "types 0..3");
-    constexpr int APL = Planes<TYPE>::A, BPL = Planes<TYPE>::B;
-    constexpr int MODE = APL;  // ternary or binary activation
+    // Type 5 goes like the two-plane types, over words of 64 channels: its two words of 32 fields are as long, and where
+    // another lane takes 32 bits of both planes its lane takes a word, low and high half for plane 0 and 1.
+    constexpr bool FIELDS = TYPE == 5;
+    constexpr int APL = FIELDS ? 2 : Planes<TYPE>::A, BPL = FIELDS ? 2 : Planes<TYPE>::B;
+    constexpr int MODE = TYPE > 3 ? TYPE : APL;  // ternary or binary activation, or the type's own format
+    constexpr int kHalf = FIELDS ? 2 : 1, kPlane = FIELDS ? 1 : 2;  // dwords between the halves and the planes of a weight word
     constexpr int FT = 1;      // 16-filter tiles per wave
     // [slot][word][half][plane], then per slot its input pixel (-1: padding) and threshold, per word of K its place in a window
     extern __shared__ __attribute__((aligned(16))) uint32_t act[];
@@ -89,12 +92,12 @@ __global__ __launch_bounds__(kConvThreads) void conv_small(const SmallConvArgs p
         for (int t = 0; t < FT; t++) {
             int f = f0 + t * 16 + r;
             f = f < p.KN ? f : p.KN - 1;  // filters past KN repeat the last one and are never stored
-            const uint32_t *row = qw32 + (size_t)f * G * (2 * BPL) + (q & 1);
+            const uint32_t *row = qw32 + (size_t)f * G * (2 * BPL) + (q & 1) * kHalf;
 #pragma unroll
             for (int j = 0; j < PAIRS; j++) {
                 const int g = 2 * (j0 + j) + (q >> 1), at = (g < G ? g : G - 1) * (2 * BPL);
 #pragma unroll
-                for (int pl = 0; pl < BPL; pl++) raw[j % (WLDS ? 1 : PAIRS)][t][pl] = row[at + 2 * pl];
+                for (int pl = 0; pl < BPL; pl++) raw[j % (WLDS ? 1 : PAIRS)][t][pl] = row[at + kPlane * pl];
             }
         }
     };
@@ -141,7 +144,7 @@ __global__ __launch_bounds__(kConvThreads) void conv_small(const SmallConvArgs p
     }
     const float t_image = own_image ? wave_threshold(p.ths, n0) : 0.f;
     __syncthreads();
-    if constexpr (INPUT == kNhwcWords && APL == 2) {
+    if constexpr (INPUT == kNhwcWords && MODE == 2) {
         if (p.ths.splits == kOwnPixelThresholds) {
             // Images of one pixel: a 16-lane row adds up |x| of its slot's image, in the order of abs_sum_partial (whose 256
             // threads take every 256th float4, i.e. every 16th word: words w, w + 16, ... in turn, then a tree over the four
@@ -256,7 +259,10 @@ __global__ __launch_bounds__(kConvThreads) void conv_small(const SmallConvArgs p
                 }
                 if (r == 0 && at[i] >= 0) {
                     uint32_t *dst = act + at[i];
-                    if (APL == 2) {
+                    if (FIELDS) {
+                        *reinterpret_cast<uintx2 *>(dst) = ok[i] ? uintx2{out[0], out[1]} : uintx2{0, 0};
+                        *reinterpret_cast<uintx2 *>(dst + 2) = ok[i] ? uintx2{out[2], out[3]} : uintx2{0, 0};
+                    } else if (APL == 2) {
                         *reinterpret_cast<uintx2 *>(dst) = ok[i] ? uintx2{out[0], out[2]} : uintx2{0, 0};
                         *reinterpret_cast<uintx2 *>(dst + 2) = ok[i] ? uintx2{out[1], out[3]} : uintx2{0, 0};
                     } else {
@@ -302,9 +308,9 @@ __global__ __launch_bounds__(kConvThreads) void conv_small(const SmallConvArgs p
             for (int t = 0; t < FT; t++) {
                 if constexpr (WLDS) {
                     const int pair = c * PAIRS + j, k = BPL == 1 ? pair : 2 * pair + (q >> 1);
-                    const uint32_t *src = weights + ((k < granules ? k : 0) * 64 + (wave * FT + t) * 16 + r) * 4 + (BPL == 1 ? q : (q & 1));
+                    const uint32_t *src = weights + ((k < granules ? k : 0) * 64 + (wave * FT + t) * 16 + r) * 4 + (BPL == 1 ? q : (q & 1) * kHalf);
 #pragma unroll
-                    for (int pl = 0; pl < BPL; pl++) now[j][t][pl] = src[2 * pl];
+                    for (int pl = 0; pl < BPL; pl++) now[j][t][pl] = src[kPlane * pl];
                 } else {
 #pragma unroll
                     for (int pl = 0; pl < BPL; pl++) now[j][t][pl] = raw[j % (WLDS ? 1 : PAIRS)][t][pl];
@@ -345,10 +351,13 @@ __global__ __launch_bounds__(kConvThreads) void conv_small(const SmallConvArgs p
             const int pl = (int)((uint32_t)px * inv_tc >> 8), pcol = px - pl * tc;
             const int line = line0 + pl, col = col0 + pcol;
             if (f < p.KN && px < tl * tc && line < lines && col < p.OW)
-                p.y[(((size_t)n0 * p.OH + line) * p.OW + col) * p.KN + f] = (TYPE == 0 ? acc[t][i] * 0.25f : acc[t][i]) + bias;
+                p.y[(((size_t)n0 * p.OH + line) * p.OW + col) * p.KN + f] = acc[t][i] * kSumScale<TYPE> + bias;
         }
     }
 }
+
+int small_act_bits(int type) { return type < 2 || type > 3 ? 2 : 1; }
+int small_weight_bits(int type) { return type == 1 || type == 3 ? 1 : 2; }
 
 int small_input(const float *x, bool nchw, int C)
 {
@@ -436,9 +445,10 @@ bool conv_small_supported(int type, const float *x, bool nchw, int N, int H, int
                           int s2, int OH, int OW)
 {
     constexpr float kMostUs = 6.3f;
-    if (type < 0 || type > 3 || KH > 255 || KW > 255 || s1 > 65535 || s2 > 65535 || p1 > 65535 || p2 > 65535 || N > 65535) return false;
+    // (type 5: the two words of every 64 channels exist)
+    if (type < 0 || type > 5 || (type > 3 && nchw) || (type == 5 && (C + 31) / 32 % 2 != 0) || KH > 255 || KW > 255 || s1 > 65535 || s2 > 65535 || p1 > 65535 || p2 > 65535 || N > 65535) return false;
     if ((long)N * H * W * C > (4L << 20) || (long)N * OH * OW > 65535) return false;  // no need to plan for these
-    const int PC = (C + kWordBits - 1) / kWordBits, abits = type < 2 ? 2 : 1, wbits = type == 0 || type == 2 ? 2 : 1;
+    const int PC = (C + kWordBits - 1) / kWordBits, abits = small_act_bits(type), wbits = small_weight_bits(type);
     const SmallPlan s = plan_small(abits, wbits, N, C, KN, KH, KW, s1, s2, OH, OW);
     if (s.lds > 64 * 1024 || (long)s.slots * PC >= 65536 || (long)s.lines_blocks * s.column_blocks >= 65536 || s.filter_groups > 65535 ||
         (size_t)KN * s.words * 16 >= kNoFilter)
@@ -466,7 +476,7 @@ hipError_t launch_conv_small(int type, const float *x, bool nchw, const Threshol
                              int N, int H, int W, int C, int KN, int KH, int KW, int p1, int p2, int s1, int s2, int OH, int OW,
                              hipStream_t stream)
 {
-    const SmallPlan s = plan_small(type < 2 ? 2 : 1, type == 0 || type == 2 ? 2 : 1, N, C, KN, KH, KW, s1, s2, OH, OW);
+    const SmallPlan s = plan_small(small_act_bits(type), small_weight_bits(type), N, C, KN, KH, KW, s1, s2, OH, OW);
     const int PC = (C + kWordBits - 1) / kWordBits;
     SmallConvArgs a;
     a.x = x; a.ths = ths; a.qw = qw; a.btn = btn; a.y = y;
@@ -480,7 +490,8 @@ hipError_t launch_conv_small(int type, const float *x, bool nchw, const Threshol
     const int input = small_input(x, nchw, C);
     auto by_input = [&](auto t) {
         constexpr int TYPE = decltype(t)::value;
-        if (input == kNchw) return launch_small<TYPE, kNchw>(a, s, stream);
+        if constexpr (TYPE <= 3)
+            if (input == kNchw) return launch_small<TYPE, kNchw>(a, s, stream);
         if (input == kNhwcWords) return launch_small<TYPE, kNhwcWords>(a, s, stream);
         return launch_small<TYPE, kNhwcRagged>(a, s, stream);
     };
@@ -489,6 +500,8 @@ hipError_t launch_conv_small(int type, const float *x, bool nchw, const Threshol
     case 1: return by_input(std::integral_constant<int, 1>());
     case 2: return by_input(std::integral_constant<int, 2>());
     case 3: return by_input(std::integral_constant<int, 3>());
+    case 4: return by_input(std::integral_constant<int, 4>());
+    case 5: return by_input(std::integral_constant<int, 5>());
     default: return hipErrorInvalidValue;
     }
 }

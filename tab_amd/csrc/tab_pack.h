@@ -151,44 +151,45 @@ __device__ __forceinline__ void pack_row(uint32_t sign, uint32_t nz, int l, uint
     }
 }
 
-// OR over the LP lanes (a power of two up to 16, aligned inside a DPP row) of a group; every lane gets the result.
-template <int LP>
-__device__ __forceinline__ uint32_t or_reduce_group(uint32_t v)
+// Spread the 32 bits of v to the even bits of a 64-bit word.
+__device__ __forceinline__ uint64_t spread_bits(uint32_t v)
 {
-    if (LP >= 2) v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, true);    // quad_perm [1,0,3,2]
-    if (LP >= 4) v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, true);    // quad_perm [2,3,0,1]
-    if (LP >= 8) v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xF, 0xF, true);   // row_half_mirror
-    if (LP >= 16) v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xF, 0xF, true);  // row_mirror
+    uint64_t x = v;
+    x = (x | x << 16) & 0x0000ffff0000ffffull;
+    x = (x | x << 8) & 0x00ff00ff00ff00ffull;
+    x = (x | x << 4) & 0x0f0f0f0f0f0f0f0full;
+    x = (x | x << 2) & 0x3333333333333333ull;
+    return (x | x << 1) & 0x5555555555555555ull;
+}
+
+// OR over the 16 lanes of a DPP row; every lane gets the result.
+__device__ __forceinline__ uint32_t or_reduce16(uint32_t v)
+{
+    v = or_reduce8(v);
+    v |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xF, 0xF, true);  // row_mirror
     return v;
 }
 
-// The packed element of a word of `channels` channels (at least 64 count as 64) from a group of LP lanes, lane l holding the
-// channels l, l + LP, l + 2 LP, l + 3 LP; every lane of the group gets out[0..1] for MODE 1, out[0..3] for MODE 2.  Bits of
-// channels that do not exist stay 0 (TAB_GEMM.cu:203-206).
-template <int MODE, int LP = 16>
+// The packed element of one pixel's word, of any channel count, from the 16 lanes of a DPP row, lane l holding channels
+// l + 16 * e: what pack_row gives for whole words.  Channels that do not exist stay 0 (TAB_GEMM.cu:203-206).
+template <int MODE>
 __device__ __forceinline__ void pack_row_strided(const float (&v)[4], float t, int l, int channels, uint32_t (&out)[4])
 {
-    uint32_t w[4] = {0, 0, 0, 0};  // sign low, sign high, nonzero low, nonzero high
+    uint32_t w[4] = {0, 0, 0, 0};  // plane 0 low, high, plane 1 low, high
 #pragma unroll
     for (int e = 0; e < 4; e++) {
-        const int ch = l + LP * e;
-        const bool valid = ch < channels;
-        const int half = LP * e >= 32 ? 1 : 0;             // LP * e is 0, 16, 32, 48 when channels reach 32
-        const int shift = l + (LP * e - 32 * half);
-        if (MODE == 2) {
-            const bool pos = v[e] > t;
-            const bool neg = !pos && (v[e] < -t);
-            w[half] |= (uint32_t)(valid && neg) << shift;
-            w[2 + half] |= (uint32_t)(valid && (pos || neg)) << shift;
-        } else {
-            w[half] |= (uint32_t)(valid && (v[e] < t)) << shift;
-        }
+        uint32_t sign, nz;  // bit 0
+        compare4<MODE>(floatx4{v[e], 0.f, 0.f, 0.f}, t, sign, nz);
+        const uint32_t valid = l + 16 * e < channels ? 1u : 0u;
+        w[e / 2] |= (sign & valid) << (l + 16 * (e % 2));
+        if (MODE != 1) w[2 + e / 2] |= (nz & valid) << (l + 16 * (e % 2));
     }
-    out[0] = or_reduce_group<LP>(w[0]);
-    out[1] = LP == 16 ? or_reduce_group<LP>(w[1]) : 0u;
-    if (MODE == 2) {
-        out[2] = or_reduce_group<LP>(w[2]);
-        out[3] = LP == 16 ? or_reduce_group<LP>(w[3]) : 0u;
+#pragma unroll
+    for (int i = 0; i < (MODE == 1 ? 2 : 4); i++) out[i] = or_reduce16(w[i]);
+    if (MODE == 5) {
+        const uint64_t word0 = spread_bits(out[2]) | spread_bits(out[0]) << 1, word1 = spread_bits(out[3]) | spread_bits(out[1]) << 1;
+        out[0] = (uint32_t)word0; out[1] = (uint32_t)(word0 >> 32);
+        out[2] = (uint32_t)word1; out[3] = (uint32_t)(word1 >> 32);
     }
 }
 

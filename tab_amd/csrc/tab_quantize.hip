@@ -223,17 +223,6 @@ __global__ __launch_bounds__(kThreads) void quantize_rows64_count(const floatx4 
     store_count<kWavesPerBlock>(count, counts.out + blockIdx.x, scratch);
 }
 
-// Spread the 32 bits of v to the even bits of a 64-bit word.
-__device__ __forceinline__ uint64_t spread_bits(uint32_t v)
-{
-    uint64_t x = v;
-    x = (x | x << 16) & 0x0000ffff0000ffffull;
-    x = (x | x << 8) & 0x00ff00ff00ff00ffull;
-    x = (x | x << 4) & 0x0f0f0f0f0f0f0f0full;
-    x = (x | x << 2) & 0x3333333333333333ull;
-    return (x | x << 1) & 0x5555555555555555ull;
-}
-
 // General path: any C, any alignment of x, every format (MODE as in compare4).  A workgroup takes a tile of consecutive pixels,
 // whose channels are one contiguous run of x, sends the run to LDS in granules of 16 bytes, and its waves then read the words
 // out of it: LP lanes a word (the smallest power of two that holds it; 64 / LP pixels a read where a pixel is one word), so

@@ -91,3 +91,26 @@ def test_linear_threshold_inside_the_launch(C):
         fc = TABLinear.from_float(torch.randn((KN, C), generator=g), tab_amd.TBN)
         want = tab_amd.Conv2d(x, fc.conv.QW, tab_amd.Threshold(x, N), fc.conv.BTN_W, 1, 0, 0, 1, 1, N, 1, 1, C, KN, 1, 1)
         assert torch.equal(fc(x), want.view(N, KN))
+
+
+@pytest.mark.parametrize("type", [4, 5])
+@pytest.mark.parametrize("case", CASES)
+def test_formats_match_their_two_launches(type, case):
+    """Types 4 and 5 (5: channels whose words of 32 come in pairs), negative and zero thresholds included."""
+    N, H, W, C, KN, KH, KW, p1, p2, s1, s2 = case
+    print(f"[case] one launch type {type} {case}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(C)
+    x = torch.randn((N, H, W, C), device="cuda", generator=g)
+    w = torch.randn((KN, KH, KW, C), device="cuda", generator=g)
+    ths = torch.linspace(-0.1, 0.9, N, device="cuda")
+    QW = tab_amd.QuantizeFormat(w, torch.full((KN,), 0.4, device="cuda"), type, KN, KH, KW, C)
+    btn = torch.zeros(KN, dtype=torch.int32, device="cuda")
+    args = (type, p1, p2, s1, s2, N, H, W, C, KN, KH, KW)
+    if type == 5 and (C + 31) // 32 % 2:
+        assert tab_amd.conv2d_launches(x, *args) == 2
+    want = tab_amd.Conv2dPacked(tab_amd.QuantizeFormat(x, ths, type, N, H, W, C), QW, btn, *args)
+    assert torch.equal(tab_amd.Conv2d(x, QW, ths, btn, *args), want)
+    base = torch.empty(x.numel() + 1, device="cuda")  # aligned to its floats only
+    shifted = base[1:].view(x.shape)
+    shifted.copy_(x)
+    assert torch.equal(tab_amd.Conv2d(shifted, QW, ths, btn, *args), want)
