@@ -350,15 +350,17 @@ static int check_from_floats(const ConvShape &s, int type, const float *dev_X, c
     return check_conv_pointers(s, type, workspace, dev_QW, dev_btn, dev_Y, nullptr);
 }
 
-/* Which kernel takes a call from fp32 in one launch: 0 none, 1 conv1x1_fused, 2 conv_small. */
+/* Which kernel takes a call from fp32 in one launch: 0 none, 1 conv1x1_fused, 2 conv_small.  own_thresholds: each image is one pixel
+ * whose threshold the kernel is to find. */
 static int one_launch(int type, const float *dev_X, bool nchw, int padding1, int padding2, int stride1, int stride2, int N, int H, int W,
-                      int C, int KN, int KH, int KW, const ConvShape &s)
+                      int C, int KN, int KH, int KW, const ConvShape &s, bool own_thresholds = false)
 {
     if (tab::conv_kernel_forced()) return 0;
     const bool small = tab::conv_small_supported(type, dev_X, nchw, N, H, W, C, KN, KH, KW, padding1, padding2, stride1, stride2, s.OH, s.OW);
     // of 1x1 layers both take, conv_small is the sooner one from five words a pixel on (N=64 512->1000 4.8 against 5.4 us),
-    // conv1x1_fused below (64->64 3.8 against 3.0)
-    if (!nchw && !(small && s.PC > 4) && tab::conv1x1_fused_supported(type, dev_X, C, KH, KW, padding1, padding2, s.M, KN)) return 1;
+    // conv1x1_fused below (64->64 3.8 against 3.0), but where the kernel is to find the thresholds itself, which conv_small can
+    // and which is a launch less (N=277 256->55 ternary layer 7.4 -> 5.2)
+    if (!nchw && !(small && (s.PC > 4 || own_thresholds)) && tab::conv1x1_fused_supported(type, dev_X, C, KH, KW, padding1, padding2, s.M, KN)) return 1;
     return small ? 2 : 0;
 }
 
@@ -370,7 +372,8 @@ static int conv_from_nhwc(const float *dev_X, const int64_t *dev_QW, const tab::
 {
     // One launch where it pays (only under the automatic kernel choice: a forced kernel is what the caller wants to see run):
     // a 1x1 convolution without padding, the smallest calls of any kernel.  The packed activation stays in LDS.
-    if (const int one = one_launch(type, dev_X, false, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, s)) {
+    if (const int one = one_launch(type, dev_X, false, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, s,
+                                   ths.splits == tab::kOwnPixelThresholds)) {
         hipError_t e = one == 1 ? tab::launch_conv1x1_fused(type, dev_X, ths, reinterpret_cast<const uint64_t *>(dev_QW), dev_btn, dev_Y, N, H, W,
                                                             C, KN, stride1, stride2, s.OH, s.OW, static_cast<hipStream_t>(stream))
                                 : tab::launch_conv_small(type, dev_X, false, ths, reinterpret_cast<const uint64_t *>(dev_QW), dev_btn, dev_Y, N, H, W,
@@ -491,7 +494,8 @@ int tab_layer_conv2d(const float *dev_X, int nchw, float act_scale, const int64_
     if (rc != TAB_OK) return rc;
     char *sums = static_cast<char *>(workspace) + layer_packed_bytes(s.abits, N, H, W, C);
     const bool planes = nchw && H * W > 1;  // one pixel per image: NCHW and NHWC are the same memory
-    const int one = one_launch(type, dev_X, planes, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, s);
+    const bool own = s.abits == 2 && tab::conv_small_own_thresholds(dev_X, H, W, C, KH, KW, padding1, padding2);
+    const int one = one_launch(type, dev_X, planes, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, s, own);
     if (planes && !one) {
         rc = tab_layer_quantize(dev_X, 1, s.abits, act_scale, N, H, W, C, static_cast<int64_t *>(workspace), sums,
                                 workspace_bytes - layer_packed_bytes(s.abits, N, H, W, C), stream);
@@ -501,7 +505,7 @@ int tab_layer_conv2d(const float *dev_X, int nchw, float act_scale, const int64_
     }
     tab::Thresholds ths;
     hipError_t e = hipSuccess;
-    if (one == 2 && s.abits == 2 && tab::conv_small_own_thresholds(dev_X, H, W, C, KH, KW, padding1, padding2))
+    if (one == 2 && own)
         ths = tab::Thresholds{dev_X, (double)act_scale / (double)C, tab::kOwnPixelThresholds};
     else
         e = own_thresholds(dev_X, s.abits, act_scale, N, (long)H * W * C, sums, &ths, stream);

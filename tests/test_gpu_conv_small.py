@@ -80,7 +80,7 @@ def test_special_values_and_negative_thresholds():
             assert np.array_equal(y.cpu().numpy(), want)
 
 
-@pytest.mark.parametrize("C", [64, 320, 1024, 1088, 2048])
+@pytest.mark.parametrize("C", [64, 128, 256, 320, 1024, 1088, 2048])
 def test_linear_threshold_inside_the_launch(C):
     """A linear layer's ternary thresholds, taken from the rows inside the one launch, are those of Threshold to the last bit:
     rows of fewer and more words than a turn of the sum, counts that leave the last block of sixteen rows partly empty."""
