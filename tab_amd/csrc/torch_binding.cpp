@@ -407,6 +407,8 @@ struct Layer {
         std::tie(s1, s2) = pair_of(m, n_stride);
         std::tie(p1, p2) = pair_of(m, n_padding);
         act_scale = attribute(m, n_scale).cast<double>();
+        // (act_bits and with it the size of a packed activation hold for these types only)
+        TORCH_CHECK(type >= 0 && type <= 3, "conv_type must be 0 (TNN), 1 (TBN), 2 (BTN) or 3 (BNN), got ", type);
     }
 
     int act_bits() const { return type < 2 ? 2 : 1; }
@@ -523,6 +525,11 @@ torch::Tensor chain_forward(const py::list &modules, const py::dict &ternary_thr
     std::vector<Layer> layers;
     layers.reserve(modules.size());
     for (const py::handle m : modules) layers.emplace_back(m);
+    // The module's constructor checks this too, but its list of layers can change afterwards, and the packed activations
+    // between them are raw blocks: no tensor's size would say that the next layer reads more than this one wrote.
+    if (layers.empty()) throw py::index_error("the chain has no layers");
+    for (size_t i = 1; i < layers.size(); i++)
+        TORCH_CHECK(layers[i - 1].KN == layers[i].C, layers[i - 1].KN, " output channels feed a layer with ", layers[i].C, " input channels");
     const Layer &first = layers.front();
     auto [N, H, W, C] = activation_sizes(x, nchw, first.C);
     const torch::Tensor X = plain_input(x);

@@ -1,0 +1,30 @@
+"""Host side of the layer calls (csrc/torch_binding.cpp), without a GPU: what they refuse and which calls they leave to the
+inner module.  A call that gets past these checks ends with the refusal of a CPU tensor."""
+import pytest
+import torch
+
+import tab_amd
+from tab_amd.nn import TABConv2d, TABPackedChain
+
+
+def _layer(C, KN, conv_type=tab_amd.BNN):
+    words = tab_amd.operand_words(conv_type, 1, C)
+    return TABConv2d(torch.zeros(KN, 3, 3, words, dtype=torch.int64), torch.zeros(KN, dtype=torch.int32), conv_type, C, KN, 3, 1, 1)
+
+
+def test_chain_checks_its_layers_on_every_call():
+    """A layer that reads more channels, or more planes, than the one before it wrote would read past the packed activation."""
+    x = torch.zeros(1, 64, 8, 8)
+    chain = TABPackedChain([_layer(64, 64), _layer(64, 64)])
+    with pytest.raises(RuntimeError, match="must be a CUDA tensor"):
+        chain(x)
+    chain.layers[1] = _layer(640, 64)
+    with pytest.raises(RuntimeError, match="64 output channels feed a layer with 640 input channels"):
+        chain(x)
+    chain.layers[1] = _layer(64, 64)
+    chain.layers[1].conv_type = tab_amd.DRF
+    with pytest.raises(RuntimeError, match="conv_type must be"):
+        chain(x)
+    del chain.layers[0], chain.layers[0]
+    with pytest.raises(IndexError):
+        chain(x)
