@@ -473,12 +473,13 @@ torch::Tensor layer_forward(py::handle module, const torch::Tensor &x, bool nchw
     return y;
 }
 
-// Whether calling the module would run more than its forward: hooks of its own, hooks of every module, a forward replaced.
+// Whether calling the module would run more than its forward: hooks of its own, hooks of every module, a forward replaced, a
+// compiled call (Module.compile).
 bool plain_call(py::handle module, py::handle type)
 {
     static PyObject *const hooks[] = {interned("_forward_hooks"), interned("_forward_pre_hooks"), interned("_backward_hooks"),
                                       interned("_backward_pre_hooks")};
-    static PyObject *const forward_name = interned("forward");
+    static PyObject *const forward_name = interned("forward"), *const compiled_name = interned("_compiled_call_impl");
     static const std::vector<PyObject *> global_hooks = [] {
         const py::module_ m = py::module_::import("torch.nn.modules.module");
         std::vector<PyObject *> all;
@@ -493,6 +494,7 @@ bool plain_call(py::handle module, py::handle type)
     }
     for (PyObject *d : global_hooks)
         if (!PyDict_Check(d) || PyDict_GET_SIZE(d) != 0) return false;
+    if (!attribute(module, compiled_name).is_none()) return false;
     PyObject **dict = _PyObject_GetDictPtr(module.ptr());
     return dict == nullptr || *dict == nullptr || PyDict_Contains(*dict, forward_name) == 0;
 }

@@ -4,7 +4,7 @@ import pytest
 import torch
 
 import tab_amd
-from tab_amd.nn import TABConv2d, TABPackedChain
+from tab_amd.nn import TABConv2d, TABLinear, TABPackedChain
 
 
 def _layer(C, KN, conv_type=tab_amd.BNN):
@@ -28,3 +28,20 @@ def test_chain_checks_its_layers_on_every_call():
     del chain.layers[0], chain.layers[0]
     with pytest.raises(IndexError):
         chain(x)
+
+
+def _linear(conv_type=tab_amd.BNN):
+    words = tab_amd.operand_words(conv_type, 1, 64)
+    conv = TABConv2d(torch.zeros(8, 1, 1, words, dtype=torch.int64), torch.zeros(8, dtype=torch.int32), conv_type, 64, 8, 1,
+                     data_format="NHWC")
+    return TABLinear(conv)
+
+
+def test_linear_runs_the_inner_layers_compiled_call(monkeypatch):
+    """Module.compile() replaces what calling the module runs."""
+    fc, x = _linear(), torch.zeros(3, 64)
+    with pytest.raises(RuntimeError, match="must be a CUDA tensor"):
+        fc(x)
+    monkeypatch.setattr(torch, "compile", lambda call, *args, **kwargs: lambda x: torch.full((x.shape[0], 1, 1, 8), 7.0))
+    fc.conv.compile()
+    assert torch.equal(fc(x), torch.full((3, 8), 7.0))
