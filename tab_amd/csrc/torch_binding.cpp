@@ -473,39 +473,50 @@ torch::Tensor layer_forward(py::handle module, const torch::Tensor &x, bool nchw
     return y;
 }
 
-// Whether calling the module would run more than its forward: hooks of its own, hooks of every module, a forward replaced, a
-// compiled call (Module.compile).
-bool plain_call(py::handle module, py::handle type)
+// The class of module a one-call path may stand in for: its methods as they were when the class was made, and the
+// dictionaries of the hooks of every module.
+struct PlainClass {
+    py::object type, forward, call;
+    std::vector<py::object> global_hooks;
+
+    explicit PlainClass(py::object t) : type(t), forward(t.attr("forward")), call(t.attr("__call__"))
+    {
+        const py::module_ m = py::module_::import("torch.nn.modules.module");
+        for (const char *name : {"_global_forward_hooks", "_global_forward_pre_hooks", "_global_backward_hooks", "_global_backward_pre_hooks"})
+            global_hooks.push_back(m.attr(name));
+    }
+};
+
+// Whether calling the module would run more than its forward: another class's or a replaced method, a forward of the
+// module's own, hooks of its own or of every module, a compiled call (Module.compile).
+bool plain_call(py::handle module, const PlainClass &plain)
 {
     static PyObject *const hooks[] = {interned("_forward_hooks"), interned("_forward_pre_hooks"), interned("_backward_hooks"),
                                       interned("_backward_pre_hooks")};
-    static PyObject *const forward_name = interned("forward"), *const compiled_name = interned("_compiled_call_impl");
-    static const std::vector<PyObject *> global_hooks = [] {
-        const py::module_ m = py::module_::import("torch.nn.modules.module");
-        std::vector<PyObject *> all;
-        for (const char *name : {"_global_forward_hooks", "_global_forward_pre_hooks", "_global_backward_hooks", "_global_backward_pre_hooks"})
-            all.push_back(py::object(m.attr(name)).release().ptr());
-        return all;
-    }();
-    if ((PyObject *)Py_TYPE(module.ptr()) != type.ptr()) return false;
+    static PyObject *const forward_name = interned("forward"), *const call_name = interned("__call__"),
+                           *const compiled_name = interned("_compiled_call_impl");
+    PyTypeObject *const type = Py_TYPE(module.ptr());
+    if ((PyObject *)type != plain.type.ptr() || _PyType_Lookup(type, forward_name) != plain.forward.ptr() ||
+        _PyType_Lookup(type, call_name) != plain.call.ptr())
+        return false;
     for (PyObject *name : hooks) {
         const py::object d = attribute(module, name);
         if (!PyDict_Check(d.ptr()) || PyDict_GET_SIZE(d.ptr()) != 0) return false;
     }
-    for (PyObject *d : global_hooks)
-        if (!PyDict_Check(d) || PyDict_GET_SIZE(d) != 0) return false;
+    for (const py::object &d : plain.global_hooks)
+        if (!PyDict_Check(d.ptr()) || PyDict_GET_SIZE(d.ptr()) != 0) return false;
     if (!attribute(module, compiled_name).is_none()) return false;
     PyObject **dict = _PyObject_GetDictPtr(module.ptr());
     return dict == nullptr || *dict == nullptr || PyDict_Contains(*dict, forward_name) == 0;
 }
 
-// TABLinear.forward around its TABConv2d (`conv_type`: that class): (N, F) as N images of one pixel.  None where calling the
+// TABLinear.forward around its TABConv2d (`plain`: that class): (N, F) as N images of one pixel.  None where calling the
 // convolution module is more than its forward, or it takes another layout: the caller then calls it.
-py::object linear_forward(py::handle module, py::handle conv_type, const torch::Tensor &x)
+py::object linear_forward(py::handle module, const PlainClass &plain, const torch::Tensor &x)
 {
     static PyObject *const modules_name = interned("_modules"), *const conv_name = interned("conv"), *const format_name = interned("data_format");
     const py::object conv = item_or_attribute(module, modules_name, conv_name);
-    if (!plain_call(conv, conv_type)) return py::none();
+    if (!plain_call(conv, plain)) return py::none();
     const py::object format = attribute(conv, format_name);
     if (!PyUnicode_Check(format.ptr()) || PyUnicode_CompareWithASCIIString(format.ptr(), "NHWC") != 0) return py::none();
     const Layer l(conv);
@@ -574,6 +585,7 @@ torch::Tensor chain_forward(const py::list &modules, const py::dict &ternary_thr
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
 {
     m.def("layer_forward", &layer_forward, "nn.TABConv2d.forward");
+    py::class_<PlainClass>(m, "PlainClass").def(py::init<py::object>());
     m.def("linear_forward", &linear_forward, "nn.TABLinear.forward");
     m.def("chain_forward", &chain_forward, "nn.TABPackedChain.forward");
     pybind11::register_exception_translator([](std::exception_ptr p) {

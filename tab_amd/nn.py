@@ -61,6 +61,9 @@ class TABConv2d(nn.Module):
                 f"padding={self.padding}, type={names[self.conv_type]}, data_format={self.data_format}")
 
 
+_PLAIN_CONV = _C.PlainClass(TABConv2d)
+
+
 class TABLinear(nn.Module):
     """Fully connected layer as a 1x1 convolution on a 1x1 image ("FC equals to 1x1 conv",
     TAB_CPU.cpp:487-488).  Input (N, in_features), output (N, out_features)."""
@@ -77,8 +80,8 @@ class TABLinear(nn.Module):
         return cls(conv)
 
     def forward(self, x):
-        y = _C.linear_forward(self, TABConv2d, x)
-        if y is None:  # the inner layer has hooks, or another layout
+        y = _C.linear_forward(self, _PLAIN_CONV, x)
+        if y is None:  # calling the inner layer is more than its forward, or it has another layout
             N, F = x.shape
             y = self.conv(x.reshape(N, 1, 1, F)).reshape(N, self.conv.out_channels)
         return y

@@ -45,3 +45,12 @@ def test_linear_runs_the_inner_layers_compiled_call(monkeypatch):
     monkeypatch.setattr(torch, "compile", lambda call, *args, **kwargs: lambda x: torch.full((x.shape[0], 1, 1, 8), 7.0))
     fc.conv.compile()
     assert torch.equal(fc(x), torch.full((3, 8), 7.0))
+
+
+@pytest.mark.parametrize("name", ["forward", "__call__"])
+def test_linear_runs_a_method_replaced_on_the_class(monkeypatch, name):
+    """Tools wrap a class's forward, or every module's __call__, to see the calls pass."""
+    fc = _linear()
+    monkeypatch.setattr(TABConv2d if name == "forward" else torch.nn.Module, name,
+                        lambda self, x: torch.full((x.shape[0], 1, 1, 8), 7.0) if isinstance(self, TABConv2d) else self.forward(x))
+    assert torch.equal(fc(torch.zeros(3, 64)), torch.full((3, 8), 7.0))
