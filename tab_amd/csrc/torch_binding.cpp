@@ -511,9 +511,12 @@ bool plain_call(py::handle module, const PlainClass &plain)
 }
 
 // TABLinear.forward around its TABConv2d (`plain`: that class): (N, F) as N images of one pixel.  None where calling the
-// convolution module is more than its forward, or it takes another layout: the caller then calls it.
-py::object linear_forward(py::handle module, const PlainClass &plain, const torch::Tensor &x)
+// convolution module is more than its forward, it takes another layout, or the input is no tensor (a tracer's proxy): the
+// caller then calls it.
+py::object linear_forward(py::handle module, const PlainClass &plain, py::handle input)
 {
+    if (!THPVariable_Check(input.ptr())) return py::none();
+    const torch::Tensor &x = THPVariable_Unpack(input.ptr());
     static PyObject *const modules_name = interned("_modules"), *const conv_name = interned("conv"), *const format_name = interned("data_format");
     const py::object conv = item_or_attribute(module, modules_name, conv_name);
     if (!plain_call(conv, plain)) return py::none();

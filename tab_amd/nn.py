@@ -81,7 +81,7 @@ class TABLinear(nn.Module):
 
     def forward(self, x):
         y = _C.linear_forward(self, _PLAIN_CONV, x)
-        if y is None:  # calling the inner layer is more than its forward, or it has another layout
+        if y is None:  # calling the inner layer is more than its forward, it has another layout, or x is a tracer's proxy
             N, F = x.shape
             y = self.conv(x.reshape(N, 1, 1, F)).reshape(N, self.conv.out_channels)
         return y

@@ -2,6 +2,7 @@
 inner module.  A call that gets past these checks ends with the refusal of a CPU tensor."""
 import pytest
 import torch
+import torch.fx
 
 import tab_amd
 from tab_amd.nn import TABConv2d, TABLinear, TABPackedChain
@@ -54,3 +55,15 @@ def test_linear_runs_a_method_replaced_on_the_class(monkeypatch, name):
     monkeypatch.setattr(TABConv2d if name == "forward" else torch.nn.Module, name,
                         lambda self, x: torch.full((x.shape[0], 1, 1, 8), 7.0) if isinstance(self, TABConv2d) else self.forward(x))
     assert torch.equal(fc(torch.zeros(3, 64)), torch.full((3, 8), 7.0))
+
+
+def test_linear_traces_down_to_the_inner_layer():
+    """Symbolic tracing with the convolution layer as a leaf: a proxy is no tensor for the one-call path."""
+
+    class Tracer(torch.fx.Tracer):
+        def is_leaf_module(self, module, name):
+            return isinstance(module, TABConv2d) or super().is_leaf_module(module, name)
+
+    graph = Tracer().trace(_linear())
+    assert [n.target for n in graph.nodes if n.op == "call_module"] == ["conv"]
+    assert [n.target for n in graph.nodes if n.op == "call_method"] == ["reshape", "reshape"]
