@@ -109,6 +109,8 @@ int tab_internal_conv_shape(int type, int M, int KN, int G, int PC, int packed, 
  * round of the chip; 0 = the device's compute units.  Small values let small test shapes mix whole tiles and quarters. */
 void tab_internal_set_tail_round(int workgroups) { tab::set_tail_round(workgroups); }
 
+/* Test hook, absent from include/tab_amd.h: the compute units that the rules choosing a kernel count; 0 = the device's. */
+void tab_internal_set_compute_units(int units) { tab::set_compute_units(units); }
 
 int tab_set_conv_kernel(int kernel, int tile)
 {

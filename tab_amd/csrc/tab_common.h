@@ -181,6 +181,7 @@ __device__ __forceinline__ ConvArgs unpack_conv(const ConvParamsOf<PACKED> &k)
 
 // Compute units of the current device (256 on MI355X), looked up once; 256 if the lookup fails.
 int device_compute_units();
+void set_compute_units(int units);  // test hook of the rules that count them (0: the device's)
 
 // Launchers (tab_conv.hip / tab_quantize.hip); they enqueue on `stream` and return the
 // launch status.

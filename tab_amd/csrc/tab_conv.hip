@@ -343,8 +343,13 @@ void force_conv_tile(int tm, int ng)
     g_forced_kernel.store(tm == 0 ? 0 : ((tm << 8) | ((ng + 1) & 0xff)), std::memory_order_relaxed);
 }
 
+std::atomic<int> g_compute_units{0};
+void set_compute_units(int units) { g_compute_units.store(units > 0 ? units : 0, std::memory_order_relaxed); }
+
 int device_compute_units()
 {
+    const int forced = g_compute_units.load(std::memory_order_relaxed);
+    if (forced > 0) return forced;
     static std::atomic<int> cached{0};
     int cus = cached.load(std::memory_order_relaxed);
     if (cus == 0) {

@@ -432,7 +432,7 @@ float small_cost_us(const SmallPlan &s, int abits, int wbits, int PC, int input)
     if (input == kNhwcRagged) passes *= 1.8f;
     if (input == kNchw) passes = (float)((s.slots + 63) / 64 * PC) * (abits == 2 ? 4.f : 3.f);
     const float pairs = (float)((((G + 1) / 2) + s.pairs - 1) / s.pairs * s.pairs) * 0.5f * (float)(abits + wbits);
-    const float more = s.workgroups > 256 ? (float)s.workgroups / 256.f - 1.f : 0.f;  // CUs: 256
+    const float cus = (float)device_compute_units(), more = (float)s.workgroups > cus ? (float)s.workgroups / cus - 1.f : 0.f;
     return 3.7f + 0.075f * passes + 0.062f * pairs + more * (0.033f * passes + 0.044f * pairs + 0.32f);
 }
 
@@ -453,7 +453,7 @@ bool conv_small_supported(int type, const float *x, bool nchw, int N, int H, int
     if (s.lds > 64 * 1024 || (long)s.slots * PC >= 65536 || (long)s.lines_blocks * s.column_blocks >= 65536 || s.filter_groups > 65535 ||
         (size_t)KN * s.words * 16 >= kNoFilter)
         return false;
-    if (KH * KW == 1 && s.workgroups > 256) return false;
+    if (KH * KW == 1 && s.workgroups > device_compute_units()) return false;
     return small_cost_us(s, abits, wbits, PC, small_input(x, nchw, C)) <= kMostUs;
 }
 

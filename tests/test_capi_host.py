@@ -195,3 +195,20 @@ def test_multiply_shift_division_is_exact_below_2_31():
         xs.update(min(k * d + o, top) for k in (1, 2, 3, 7) for o in (-1, 0, 1) if k * d + o >= 0)
         for x in xs:
             assert f(x, d) == x // d, (x, d)
+
+
+def test_one_launch_rule_counts_the_devices_compute_units():
+    """conv_small is taken up to some microseconds of its own, which depend on how many workgroups a CU gets: on a device (or a
+    partition of one) with fewer CUs the same layer is a longer launch."""
+    lib = ctypes.CDLL(_capi.LIB_PATH)
+    three = lambda N: lib.tab_conv2d_launches(ctypes.c_void_p(4096), 3, 1, 1, 1, 1, N, 14, 14, 128, 128, 3, 3)  # noqa: E731
+    one = lambda N: lib.tab_conv2d_launches(ctypes.c_void_p(4096), 3, 0, 0, 1, 1, N, 7, 7, 640, 64, 1, 1)  # noqa: E731
+    try:
+        lib.tab_internal_set_compute_units(256)
+        assert (three(4), one(16)) == (1, 1)
+        lib.tab_internal_set_compute_units(32)
+        assert (three(4), one(16)) == (2, 2)
+        lib.tab_internal_set_compute_units(1024)
+        assert (three(4), one(16)) == (1, 1)
+    finally:
+        lib.tab_internal_set_compute_units(0)
