@@ -588,7 +588,7 @@ template <int BITS, int U, bool EVEN, bool COUNT = false>
 __global__ __launch_bounds__(64, BITS == 1 ? (U == 4 ? 4 : 7) : (U == 4 ? 1 : 4)) void quantize_nchw_gather(const float *__restrict__ x, const Thresholds ths,
                                                                  uint64_t *__restrict__ q, int N, int C, long HW, int PC, int32_t *btn)
 {
-    static_assert(!COUNT || BITS == 2, "counts of two planes");
+    static_assert(!COUNT || (BITS == 2 && !EVEN), "counts of two planes; runs of one image are numbered for any plane size");
     constexpr int VEC = 4, kInFlight = 8;
     constexpr int WPP = U * BITS;      // words a thread packs per pixel, contiguous in q
     constexpr int ROUNDS = WPP / 2;    // 64 / ROUNDS lanes x 4 pixels x WPP words = 512 words a round
@@ -1039,8 +1039,7 @@ hipError_t launch_quantize_nchw(const float *x, const Thresholds &ths, int bitwi
             auto launch_counted = [&](auto kernel) {
                 kernel<<<dim3((unsigned)(N * slices)), dim3(64), 0, stream>>>(x, ths, qx, (int)slices, C, HW, PC, slices == 1 ? btn : count_workspace);
             };
-            if (unit == 4) launch_counted(HW % 4 ? quantize_nchw_gather<2, 4, false, true> : quantize_nchw_gather<2, 4, true, true>);
-            else launch_counted(HW % 4 ? quantize_nchw_gather<2, 2, false, true> : quantize_nchw_gather<2, 2, true, true>);
+            launch_counted(unit == 4 ? quantize_nchw_gather<2, 4, false, true> : quantize_nchw_gather<2, 2, false, true>);
             finish_counts(CountTarget{btn, count_workspace}, N, (int)slices, stream);
             return hipGetLastError();
         }
