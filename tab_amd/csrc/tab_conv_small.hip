@@ -3,10 +3,10 @@
 //
 // Such a call is bound by what a launch costs the host (2.4-2.8 us each) and by the instructions a wave runs one after the
 // other: alone on its SIMD a wave takes some 2.5 ns per instruction, and the chip is mostly idle.  So the work is cut fine:
-// a workgroup owns 16 output pixels (a block of tl lines x tc columns) and 64 * FT filters, and
+// a workgroup owns 16 output pixels (a block of tl lines x tc columns) and 64 filters, and
 //   * its four waves quantize the patch of input pixels that block reads - "slots", row by row, padding included as zero
 //     words (TAB_CPU.cpp:39,155) - into LDS, each input pixel once per workgroup;
-//   * each wave multiplies the 16 pixels with its FT tiles of 16 filters (v_mfma_f32_16x16x128_f8f6f4: two words of K per
+//   * each wave multiplies the 16 pixels with its 16 filters (v_mfma_f32_16x16x128_f8f6f4: two words of K per
 //     instruction, an operand is four lanes' 32 bits of one pixel or filter), the weights straight from global memory,
 //     requested before the activation.
 // A patch is quantized again by the workgroups of the other filters and, at its rim, of the neighbouring blocks; where that
@@ -54,7 +54,6 @@ __global__ __launch_bounds__(kConvThreads) void conv_small(const SmallConvArgs p
     constexpr int APL = FIELDS ? 2 : Planes<TYPE>::A, BPL = FIELDS ? 2 : Planes<TYPE>::B;
     constexpr int MODE = TYPE > 3 ? TYPE : APL;  // ternary or binary activation, or the type's own format
     constexpr int kHalf = FIELDS ? 2 : 1, kPlane = FIELDS ? 1 : 2;  // dwords between the halves and the planes of a weight word
-    constexpr int FT = 1;      // 16-filter tiles per wave
     // [slot][word][half][plane], then per slot its input pixel (-1: padding) and threshold, per word of K its place in a window
     extern __shared__ __attribute__((aligned(16))) uint32_t act[];
 
@@ -83,22 +82,18 @@ __global__ __launch_bounds__(kConvThreads) void conv_small(const SmallConvArgs p
     int *const place_of = reinterpret_cast<int *>(th_of + slots);
     const ExpandConsts consts;
 
-    // ---- weights: filter tile t of this wave, pair of words j: lane (q, r) feeds half q % 2 of word 2j + q / 2 -------------
-    const int f0 = (blockIdx.z * 4 + wave) * 16 * FT;
+    // ---- weights: the wave's filters from f0 on, pair of words j: lane (q, r) feeds half q % 2 of word 2j + q / 2 -----------
+    const int f0 = (blockIdx.z * 4 + wave) * 16;
     const uint32_t *qw32 = reinterpret_cast<const uint32_t *>(p.qw);
-    uint32_t raw[WLDS ? 1 : PAIRS][FT][BPL];
+    uint32_t raw[WLDS ? 1 : PAIRS][BPL];
     auto request_weights = [&](int j0) {
+        const int f = f0 + r < p.KN ? f0 + r : p.KN - 1;  // filters past KN repeat the last one and are never stored
+        const uint32_t *row = qw32 + (size_t)f * G * (2 * BPL) + (q & 1) * kHalf;
 #pragma unroll
-        for (int t = 0; t < FT; t++) {
-            int f = f0 + t * 16 + r;
-            f = f < p.KN ? f : p.KN - 1;  // filters past KN repeat the last one and are never stored
-            const uint32_t *row = qw32 + (size_t)f * G * (2 * BPL) + (q & 1) * kHalf;
+        for (int j = 0; j < PAIRS; j++) {
+            const int g = 2 * (j0 + j) + (q >> 1), at = (g < G ? g : G - 1) * (2 * BPL);
 #pragma unroll
-            for (int j = 0; j < PAIRS; j++) {
-                const int g = 2 * (j0 + j) + (q >> 1), at = (g < G ? g : G - 1) * (2 * BPL);
-#pragma unroll
-                for (int pl = 0; pl < BPL; pl++) raw[j % (WLDS ? 1 : PAIRS)][t][pl] = row[at + kPlane * pl];
-            }
+            for (int pl = 0; pl < BPL; pl++) raw[j % (WLDS ? 1 : PAIRS)][pl] = row[at + kPlane * pl];
         }
     };
     // WLDS: granule k of filter f of the workgroup's 64 at ((k * 64) + f) * 16 bytes: two words of one plane or one of two
@@ -281,13 +276,8 @@ __global__ __launch_bounds__(kConvThreads) void conv_small(const SmallConvArgs p
     const uint32_t inv_tc = (256u + (uint32_t)tc - 1) / (uint32_t)tc;  // i / tc for i below 16
     const int li = (int)((uint32_t)r * inv_tc >> 8), ci = r - li * tc;
     const uint32_t *mine = act + (r < tl * tc ? (li * rs * pw + ci * cs) * stride : 0) + (q & 1) * APL;
-    f32x4v acc[FT];
-    int nonzero[FT];  // BTN: bits set in the nonzero plane of this lane's part of its filter
-#pragma unroll
-    for (int t = 0; t < FT; t++) {
-        acc[t] = f32x4v{0.f, 0.f, 0.f, 0.f};
-        nonzero[t] = 0;
-    }
+    f32x4v acc = {0.f, 0.f, 0.f, 0.f};
+    int nonzero = 0;  // BTN: bits set in the nonzero plane of this lane's part of its filter
     for (int c = 0; c < chunks; c++) {
         uint32_t a[PAIRS][APL];
 #pragma unroll
@@ -301,21 +291,19 @@ __global__ __launch_bounds__(kConvThreads) void conv_small(const SmallConvArgs p
                 a[j][0] = src[0];
             }
         }
-        uint32_t now[PAIRS][FT][BPL];
+        uint32_t now[PAIRS][BPL];
 #pragma unroll
-        for (int j = 0; j < PAIRS; j++)
+        for (int j = 0; j < PAIRS; j++) {
+            if constexpr (WLDS) {
+                const int pair = c * PAIRS + j, k = BPL == 1 ? pair : 2 * pair + (q >> 1);
+                const uint32_t *src = weights + ((k < granules ? k : 0) * 64 + wave * 16 + r) * 4 + (BPL == 1 ? q : (q & 1) * kHalf);
 #pragma unroll
-            for (int t = 0; t < FT; t++) {
-                if constexpr (WLDS) {
-                    const int pair = c * PAIRS + j, k = BPL == 1 ? pair : 2 * pair + (q >> 1);
-                    const uint32_t *src = weights + ((k < granules ? k : 0) * 64 + (wave * FT + t) * 16 + r) * 4 + (BPL == 1 ? q : (q & 1) * kHalf);
+                for (int pl = 0; pl < BPL; pl++) now[j][pl] = src[kPlane * pl];
+            } else {
 #pragma unroll
-                    for (int pl = 0; pl < BPL; pl++) now[j][t][pl] = src[kPlane * pl];
-                } else {
-#pragma unroll
-                    for (int pl = 0; pl < BPL; pl++) now[j][t][pl] = raw[j % (WLDS ? 1 : PAIRS)][t][pl];
-                }
+                for (int pl = 0; pl < BPL; pl++) now[j][pl] = raw[j % (WLDS ? 1 : PAIRS)][pl];
             }
+        }
         if constexpr (!WLDS)
             if (c + 1 < chunks) request_weights((c + 1) * PAIRS);
 #pragma unroll
@@ -323,36 +311,30 @@ __global__ __launch_bounds__(kConvThreads) void conv_small(const SmallConvArgs p
             // (words past K: zeros on both sides, +64 each for binary x binary, which the bias counts)
             const bool live = 2 * (c * PAIRS + j) + (q >> 1) < G;
             const i32x8 af = expand_operand<TYPE, 0>(live ? a[j][0] : 0u, live ? a[j][APL - 1] : 0u, consts);
-#pragma unroll
-            for (int t = 0; t < FT; t++) {
-                const uint32_t b0 = live ? now[j][t][0] : 0u, b1 = live ? now[j][t][BPL - 1] : 0u;
-                const i32x8 bf = expand_operand<TYPE, 1>(b0, b1, consts);
-                if (TYPE == 2) nonzero[t] += __builtin_popcount(b1);
-                acc[t] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(af, bf, acc[t], 4, 4, 0, 0, 0, 0);
-            }
+            const uint32_t b0 = live ? now[j][0] : 0u, b1 = live ? now[j][BPL - 1] : 0u;
+            const i32x8 bf = expand_operand<TYPE, 1>(b0, b1, consts);
+            if (TYPE == 2) nonzero += __builtin_popcount(b1);
+            acc = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(af, bf, acc, 4, 4, 0, 0, 0, 0);
         }
     }
 
     // ---- store: element i of lane (q, r) is pixel 4q + i of the block, filter r of the tile ---------------------------------
     const int padded = chunks * PAIRS * 2;  // words of K multiplied
+    const int f = f0 + r;
+    // BTN btn[f] - popcount(b1 of f), BNN NUM - 64 per word (TAB_GEMM.cu:116, 144)
+    float bias = TYPE == 3 ? (float)(KH * KW * p.C - 64 * padded) : 0.f;
+    if (TYPE == 2) {
+        int total = nonzero + __shfl_xor(nonzero, 16, 64);
+        total += __shfl_xor(total, 32, 64);
+        bias = (float)((f < p.KN ? p.btn[f] : 0) - total);
+    }
 #pragma unroll
-    for (int t = 0; t < FT; t++) {
-        const int f = f0 + t * 16 + r;
-        // BTN btn[f] - popcount(b1 of f), BNN NUM - 64 per word (TAB_GEMM.cu:116, 144)
-        float bias = TYPE == 3 ? (float)(KH * KW * p.C - 64 * padded) : 0.f;
-        if (TYPE == 2) {
-            int total = nonzero[t] + __shfl_xor(nonzero[t], 16, 64);
-            total += __shfl_xor(total, 32, 64);
-            bias = (float)((f < p.KN ? p.btn[f] : 0) - total);
-        }
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int px = 4 * q + i;
-            const int pl = (int)((uint32_t)px * inv_tc >> 8), pcol = px - pl * tc;
-            const int line = line0 + pl, col = col0 + pcol;
-            if (f < p.KN && px < tl * tc && line < lines && col < p.OW)
-                p.y[(((size_t)n0 * p.OH + line) * p.OW + col) * p.KN + f] = acc[t][i] * kSumScale<TYPE> + bias;
-        }
+    for (int i = 0; i < 4; i++) {
+        const int px = 4 * q + i;
+        const int pl = (int)((uint32_t)px * inv_tc >> 8), pcol = px - pl * tc;
+        const int line = line0 + pl, col = col0 + pcol;
+        if (f < p.KN && px < tl * tc && line < lines && col < p.OW)
+            p.y[(((size_t)n0 * p.OH + line) * p.OW + col) * p.KN + f] = acc[i] * kSumScale<TYPE> + bias;
     }
 }
 
