@@ -55,7 +55,7 @@ def test_notebook_flow_matches_oracle():
 def test_extension_equals_ctypes_front_end():
     import TAB_CUDA as TAB
 
-    import tab_amd
+    import capi_calls as capi
 
     g = torch.Generator("cpu").manual_seed(3)
     N, H, W, C, KN = 3, 9, 7, 192, 40
@@ -64,10 +64,10 @@ def test_extension_equals_ctypes_front_end():
     x_ths = (0.7 * x.abs().reshape(N, -1).mean(dim=1)).contiguous()
     w_ths = (0.7 * w.abs().reshape(KN, -1).mean(dim=1)).contiguous()
     QWa, BTNa = TAB.Quantize(w, w_ths, 2, KN, 3, 3, C)
-    QWb, BTNb = tab_amd.Quantize(w, w_ths, 2, KN, 3, 3, C)
+    QWb, BTNb = capi.Quantize(w, w_ths, 2, KN, 3, 3, C)
     assert torch.equal(QWa, QWb) and torch.equal(BTNa, BTNb)
     ya = TAB.Conv2d(x, QWa, x_ths, BTNa, 0, 1, 0, 2, 1, N, H, W, C, KN, 3, 3)
-    yb = tab_amd.Conv2d(x, QWb, x_ths, BTNb, 0, 1, 0, 2, 1, N, H, W, C, KN, 3, 3)
+    yb = capi.Conv2d(x, QWb, x_ths, BTNb, 0, 1, 0, 2, 1, N, H, W, C, KN, 3, 3)
     assert torch.equal(ya, yb)
 
 
@@ -93,11 +93,12 @@ def test_extension_input_checks():
 
 
 def test_every_extension_entry_point_equals_ctypes_front_end():
-    """The pybind module exports everything the ctypes mirror does; each function, called through TAB_CUDA,
-    returns the tensors the mirror returns (same C ABI underneath), and Conv2d takes types 4 and 5 like the
-    reference's CPU binding (TAB_CPU.cpp:577-584, 621-633)."""
+    """Each function of the pybind module, called through TAB_CUDA, returns the tensors that the C ABI call it stands for
+    writes when called through ctypes, and Conv2d takes types 4 and 5 like the reference's CPU binding
+    (TAB_CPU.cpp:577-584, 621-633)."""
     import TAB_CUDA as TAB
 
+    import capi_calls as capi
     import tab_amd
 
     assert {"QuantizeNCHW", "QuantizeFormat", "Threshold", "Conv2dPacked", "Conv2dPackedOut", "TAB_Quantize",
@@ -107,14 +108,14 @@ def test_every_extension_entry_point_equals_ctypes_front_end():
     x = torch.randn([N, H, W, C], generator=g).cuda()
     w = torch.randn([KN, 3, 3, C], generator=g).cuda()
     # Threshold
-    ths_a, ths_b = TAB.Threshold(x, N, 0.7), tab_amd.Threshold(x, N, 0.7)
+    ths_a, ths_b = TAB.Threshold(x, N, 0.7), capi.Threshold(x, N, 0.7)
     assert torch.equal(ths_a, ths_b) and torch.equal(TAB.Threshold(x, N), ths_b)
     w_ths = TAB.Threshold(w, KN, 0.7)
     # QuantizeNCHW
     x_nchw = x.permute(0, 3, 1, 2).contiguous()
     for bits in (1, 2):
         qa, ba = TAB.QuantizeNCHW(x_nchw, ths_a, bits, N, C, H, W)
-        qb, bb = tab_amd.QuantizeNCHW(x_nchw, ths_a, bits, N, C, H, W)
+        qb, bb = capi.QuantizeNCHW(x_nchw, ths_a, bits, N, C, H, W)
         qc, _ = TAB.Quantize(x, ths_a, bits, N, H, W, C)
         assert torch.equal(qa, qb) and torch.equal(ba, bb) and torch.equal(qa, qc)
     zeros = torch.zeros(max(N, KN), device="cuda")
@@ -124,13 +125,13 @@ def test_every_extension_entry_point_equals_ctypes_front_end():
         QW, BTN = TAB.Quantize(w, w_ths if wb == 2 else zeros, wb, KN, 3, 3, C)
         QX, _ = TAB.Quantize(x, ths_a if ab == 2 else zeros, ab, N, H, W, C)
         ya = TAB.Conv2dPacked(QX, QW, BTN, type, 1, 0, 1, 2, N, H, W, C, KN, 3, 3)
-        yb = tab_amd.Conv2dPacked(QX, QW, BTN, type, 1, 0, 1, 2, N, H, W, C, KN, 3, 3)
+        yb = capi.Conv2dPacked(QX, QW, BTN, type, 1, 0, 1, 2, N, H, W, C, KN, 3, 3)
         assert torch.equal(ya, yb) and tuple(ya.shape) == tuple(yb.shape)
         assert torch.equal(ya, TAB.TAB_Conv2d(x, QW, ths_a if ab == 2 else zeros, BTN, type, 1, 0, 1, 2, N, H, W, C, KN, 3, 3))
         out_ths = torch.full((N,), 3.0, device="cuda")
         for out_bits in (1, 2):
             qa = TAB.Conv2dPackedOut(QX, QW, BTN, type, 1, 0, 1, 2, N, H, W, C, KN, 3, 3, out_ths, out_bits)
-            qb = tab_amd.Conv2dPackedOut(QX, QW, BTN, type, 1, 0, 1, 2, N, H, W, C, KN, 3, 3, out_ths, out_bits)
+            qb = capi.Conv2dPackedOut(QX, QW, BTN, type, 1, 0, 1, 2, N, H, W, C, KN, 3, 3, out_ths, out_bits)
             assert torch.equal(qa, qb) and tuple(qa.shape) == tuple(qb.shape)
     # types 4 and 5: packer and Conv2d
     btn = torch.zeros(KN, dtype=torch.int32, device="cuda")
@@ -138,21 +139,21 @@ def test_every_extension_entry_point_equals_ctypes_front_end():
         print(f"[case] TAB_CUDA types of the CPU path type={type}", flush=True)
         xs, ws = (x.abs(), w.abs()) if type == 4 else (x, w)
         x_t, w_t = torch.full((N,), 0.6, device="cuda"), torch.full((KN,), 0.5, device="cuda")
-        QWa, QWb = TAB.QuantizeFormat(ws, w_t, type, KN, 3, 3, C), tab_amd.QuantizeFormat(ws, w_t, type, KN, 3, 3, C)
+        QWa, QWb = TAB.QuantizeFormat(ws, w_t, type, KN, 3, 3, C), capi.QuantizeFormat(ws, w_t, type, KN, 3, 3, C)
         assert torch.equal(QWa, QWb) and tuple(QWa.shape) == tuple(QWb.shape)
         ya = TAB.Conv2d(xs, QWa, x_t, btn, type, 1, 1, 2, 1, N, H, W, C, KN, 3, 3)
-        yb = tab_amd.Conv2d(xs, QWa, x_t, btn, type, 1, 1, 2, 1, N, H, W, C, KN, 3, 3)
+        yb = capi.Conv2d(xs, QWa, x_t, btn, type, 1, 1, 2, 1, N, H, W, C, KN, 3, 3)
         assert torch.equal(ya, yb)
         qw_o = oracle.quantize_format(ws.cpu().numpy(), w_t.cpu().numpy(), type, KN, 3, 3, C)
         want = oracle.conv2d(xs.cpu().numpy(), qw_o, x_t.cpu().numpy(), np.zeros(KN, np.int32), type, 1, 1, 2, 1, N, H, W, C, KN, 3, 3)
         assert np.array_equal(ya.cpu().numpy(), want)
         QX = TAB.QuantizeFormat(xs, x_t, type, N, H, W, C)
         assert torch.equal(TAB.Conv2dPacked(QX, QWa, btn, type, 1, 1, 2, 1, N, H, W, C, KN, 3, 3), ya)
-        # packed output for these types too: both front ends agree with quantizing the fp32 result
+        # packed output for these types too: both sides agree with quantizing the fp32 result
         OH, OW = tab_amd.out_shape(H, W, 3, 3, 1, 1, 2, 1)
         out_t = torch.full((N,), float(ya.abs().median()), device="cuda")
         for out_bits in (1, 2):
             qa = TAB.Conv2dPackedOut(QX, QWa, btn, type, 1, 1, 2, 1, N, H, W, C, KN, 3, 3, out_t, out_bits)
-            qb = tab_amd.Conv2dPackedOut(QX, QWa, btn, type, 1, 1, 2, 1, N, H, W, C, KN, 3, 3, out_t, out_bits)
-            want_q, _ = tab_amd.Quantize(ya.view(N, OH, OW, KN), out_t, out_bits, N, OH, OW, KN)
+            qb = capi.Conv2dPackedOut(QX, QWa, btn, type, 1, 1, 2, 1, N, H, W, C, KN, 3, 3, out_t, out_bits)
+            want_q, _ = capi.Quantize(ya.view(N, OH, OW, KN), out_t, out_bits, N, OH, OW, KN)
             assert torch.equal(qa, qb) and torch.equal(qa.reshape(want_q.shape), want_q)
