@@ -67,7 +67,7 @@ struct ConvArgs {
     int OH, OW;
     int M;         // N*OH*OW
     int G;         // KH*KW*PC, packed words along K per plane
-    int kcw;       // words per K chunk (<= kMaxChunkWords)
+    int kcw;       // words per K chunk (at most the kernel's KCH; 6 bits of ConvParams)
     int nchunks;   // ceil(G / kcw)
     int num;       // KH*KW*C (BNN constant)
     int tiles_m;   // ceil(M / BM)
