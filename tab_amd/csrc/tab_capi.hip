@@ -105,6 +105,19 @@ int tab_internal_conv_shape(int type, int M, int KN, int G, int PC, int packed, 
     return tab::conv_mfma_shape(type, a, cost_us);
 }
 
+/* Test hook, absent from include/tab_amd.h: whether the one-launch kernel of the smallest calls can run a call, and its predicted
+ * duration on the GPU in microseconds with the three numbers it comes from. */
+int tab_internal_conv_small_cost(int type, const float *dev_X, int nchw, int N, int H, int W, int C, int KN, int KH, int KW, int padding1,
+                                 int padding2, int stride1, int stride2, float *cost)
+{
+    float c[4];
+    const int OH = tab_out_extent(H, padding1, KH, stride1), OW = tab_out_extent(W, padding2, KW, stride2);
+    if (OH < 1 || OW < 1 || !tab::conv_small_cost(type, dev_X, nchw != 0, N, H, W, C, KN, KH, KW, padding1, padding2, stride1, stride2, OH, OW, c))
+        return 0;
+    for (int i = 0; i < 4; i++) cost[i] = c[i];
+    return 1;
+}
+
 /* Test hook, absent from include/tab_amd.h: the number of workgroups the mixed launch (TAB_CONV_MATRIX tile 10) counts as one
  * round of the chip; 0 = the device's compute units.  Small values let small test shapes mix whole tiles and quarters. */
 void tab_internal_set_tail_round(int workgroups) { tab::set_tail_round(workgroups); }

@@ -251,6 +251,9 @@ hipError_t launch_conv1x1_fused(int type, const float *x, const Thresholds &ths,
 // Quantize + convolution in one launch for the smallest calls (tab_conv_small.hip); x NHWC or NCHW.
 bool conv_small_supported(int type, const float *x, bool nchw, int N, int H, int W, int C, int KN, int KH, int KW, int p1, int p2, int s1,
                           int s2, int OH, int OW);
+// False where conv_small cannot run the call; cost: the predicted microseconds on the GPU and the three numbers they come from.
+bool conv_small_cost(int type, const float *x, bool nchw, int N, int H, int W, int C, int KN, int KH, int KW, int p1, int p2, int s1, int s2,
+                     int OH, int OW, float (&cost)[4]);
 bool conv_small_in_one_image(int OH, int OW);
 // Images of one pixel (H = W = 1, a 1x1 kernel without padding): conv_small takes kOwnPixelThresholds.
 bool conv_small_own_thresholds(const float *x, int H, int W, int C, int KH, int KW, int p1, int p2);

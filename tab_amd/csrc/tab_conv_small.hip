@@ -403,30 +403,46 @@ hipError_t launch_small(const SmallConvArgs &a, const SmallPlan &s, hipStream_t 
     return hipGetLastError();
 }
 
-// Microseconds a launch takes on the GPU, from 400 launches of random geometry (medians within 10 %; TNN, BTN, ... share
-// the coefficients): a start, a wave's passes over the patch and its pairs of words of K, one after the other, and the same
-// again, at the rate of waves that share a SIMD, for every further workgroup a CU gets.  A two-plane activation costs half
-// as much again to pack, channels that are no whole words nearly twice.
-float small_cost_us(const SmallPlan &s, int abits, int wbits, int PC, int input)
+// What a launch's duration is made of: a wave's passes over the patch, its pairs of words of K, and how many workgroups a CU gets
+// beyond the first, which run at the rate of waves that share a SIMD.  A two-plane activation costs half as much again to pack,
+// channels that are no whole words nearly twice.  Against the measured duration in graph replays (conv_small_timings.txt) the
+// prediction is off by 7 % in the median on 306 NHWC calls (5 % too low on average) and by 19 %, too low, on 64 NCHW ones.
+struct SmallCost {
+    float passes, pairs, more;
+    float us() const { return 3.7f + 0.075f * passes + 0.062f * pairs + more * (0.033f * passes + 0.044f * pairs + 0.32f); }
+};
+
+SmallCost small_cost(const SmallPlan &s, int abits, int wbits, int PC, int input)
 {
-    const int G = s.words;
-    float passes = (float)((s.slots * PC + 63) / 64 * 4) * (abits == 2 ? 1.5f : 1.f);
-    if (input == kNhwcRagged) passes *= 1.8f;
-    if (input == kNchw) passes = (float)((s.slots + 63) / 64 * PC) * (abits == 2 ? 4.f : 3.f);
-    const float pairs = (float)((((G + 1) / 2) + s.pairs - 1) / s.pairs * s.pairs) * 0.5f * (float)(abits + wbits);
-    const float cus = (float)device_compute_units(), more = (float)s.workgroups > cus ? (float)s.workgroups / cus - 1.f : 0.f;
-    return 3.7f + 0.075f * passes + 0.062f * pairs + more * (0.033f * passes + 0.044f * pairs + 0.32f);
+    SmallCost c;
+    c.passes = (float)((s.slots * PC + 63) / 64 * 4) * (abits == 2 ? 1.5f : 1.f);
+    if (input == kNhwcRagged) c.passes *= 1.8f;
+    if (input == kNchw) c.passes = (float)((s.slots + 63) / 64 * PC) * (abits == 2 ? 4.f : 3.f);
+    c.pairs = (float)((((s.words + 1) / 2) + s.pairs - 1) / s.pairs * s.pairs) * 0.5f * (float)(abits + wbits);
+    const float cus = (float)device_compute_units();
+    c.more = (float)s.workgroups > cus ? (float)s.workgroups / cus - 1.f : 0.f;
+    return c;
 }
 
 }  // namespace
 
-// True when conv_small takes the call.  Against the two launches, which cost the host 5 us and the GPU 5 us or more at any
-// size, it pays up to about 6 us of its own (random geometries, time of a call: -10 %; the best choice of every one -12 %).
+// True when conv_small takes the call.  Two launches cost the host 5 us and the GPU 5 us or more at any size; called one after
+// the other from Python, calls on NHWC take 8.4-8.7 us in two launches and 5.3-6.3 in this one where it is taken.  The limit lies
+// between what suits such callers (420 measured calls of random geometry, time as a share of always two launches: 82 % at 5.5 us,
+// 78 % at 6.3, 77 % from 6.6 on; with the better choice of each 76 %) and graph replays, where a launch costs the host nothing
+// (94, 95, 96 and from 8 us on 100 %; 93 %).  tab_amd/tuning/check_conv_small_cost.py prints this from the timings beside it.
 // Of the 1x1 layers it is left those that conv1x1_fused does not take, within one workgroup a CU.
 bool conv_small_supported(int type, const float *x, bool nchw, int N, int H, int W, int C, int KN, int KH, int KW, int p1, int p2, int s1,
                           int s2, int OH, int OW)
 {
     constexpr float kMostUs = 6.3f;
+    float cost[4];
+    return conv_small_cost(type, x, nchw, N, H, W, C, KN, KH, KW, p1, p2, s1, s2, OH, OW, cost) && cost[0] <= kMostUs;
+}
+
+bool conv_small_cost(int type, const float *x, bool nchw, int N, int H, int W, int C, int KN, int KH, int KW, int p1, int p2, int s1, int s2,
+                     int OH, int OW, float (&cost)[4])
+{
     // (type 5: the two words of every 64 channels exist)
     if (type < 0 || type > 5 || (type > 3 && nchw) || (type == 5 && (C + 31) / 32 % 2 != 0) || KH > 255 || KW > 255 || s1 > 65535 || s2 > 65535 || p1 > 65535 || p2 > 65535 || N > 65535) return false;
     if ((long)N * H * W * C > (4L << 20) || (long)N * OH * OW > 65535) return false;  // no need to plan for these
@@ -436,7 +452,12 @@ bool conv_small_supported(int type, const float *x, bool nchw, int N, int H, int
         (size_t)KN * s.words * 16 >= kNoFilter)
         return false;
     if (KH * KW == 1 && s.workgroups > device_compute_units()) return false;
-    return small_cost_us(s, abits, wbits, PC, small_input(x, nchw, C)) <= kMostUs;
+    const SmallCost c = small_cost(s, abits, wbits, PC, small_input(x, nchw, C));
+    cost[0] = c.us();
+    cost[1] = c.passes;
+    cost[2] = c.pairs;
+    cost[3] = c.more;
+    return true;
 }
 
 // A workgroup's outputs lie in one image (then its waves add up an image's partial sums together).
