@@ -361,7 +361,7 @@ def profile_sequence(torch, tab):
     N=256 56x56x64->64 with fp32 and with packed output, the conv kernel of three mid-size layers
     (N=256 7x7x512->512, N=256 14x14x256->256, N=32 14x14x512->512; BNN and TNN), and the conv kernel of the large
     sweep point for all four types: the default (matrix-core) kernel, then the popcount kernel on
-    the same tensors.  Three repetitions each."""
+    the same tensors, and whole calls of the other kinds (other_calls).  Three repetitions each."""
     src = torch.empty(256 * 1024 * 1024 // 4, dtype=torch.float32, device="cuda").normal_()
     dst = torch.empty_like(src)
     for _ in range(3):
@@ -407,8 +407,41 @@ def profile_sequence(torch, tab):
                 L.conv_kernel_only()
         tab.set_conv_kernel(tab.CONV_AUTO, -1)
         del L
+    for call in other_calls(torch, tab):
+        for _ in range(3):
+            call()
+        del call
     torch.cuda.synchronize()
     print("profile sequence done")
+
+
+def other_calls(torch, tab):
+    """Calls whose kernels the layers above do not run: the one-launch kernels, the quantizers of ragged channels and of NCHW with
+    their counts, a layer that takes its threshold from the activation, a packed chain."""
+    from tab_amd import nn as tab_nn
+
+    g = torch.Generator("cuda").manual_seed(5)
+    randn = lambda *shape: torch.randn(shape, generator=g, device="cuda")  # noqa: E731
+    for type, N, layer in ((0, 1, (32, 32, 64, 64, 3, 3, 1, 1, 1, 1)), (2, 128, (28, 28, 256, 512, 1, 1, 0, 0, 2, 2)),
+                           (1, 5, (37, 53, 100, 75, 5, 5, 2, 1, 2, 2)), (0, 32, (56, 56, 256, 256, 3, 3, 1, 1, 1, 1))):
+        yield Layer(tab, torch, type, N, layer, seed=3).conv2d
+    x, w = randn(64, 14, 14, 256).abs(), randn(256, 3, 3, 256).abs()
+    QW, btn = tab.QuantizeFormat(w, tab.Threshold(w, 256), tab.DRF, 256, 3, 3, 256), torch.zeros(256, dtype=torch.int32, device="cuda")
+    ths = tab.Threshold(x, 64)
+    yield lambda: tab.Conv2d(x, QW, ths, btn, tab.DRF, 1, 1, 1, 1, 64, 14, 14, 256, 256, 3, 3)
+    for type, C in ((tab.BNN, 512), (tab.TNN, 256)):
+        fc, rows = tab_nn.TABLinear.from_float(randn(1000, C), type), randn(64, C)
+        yield lambda: fc(rows)
+    for bits, nchw, N, H, W, C in ((2, False, 64, 56, 56, 100), (1, True, 24, 61, 47, 75), (2, True, 256, 56, 56, 256)):
+        t, q_ths = randn(*((N, C, H, W) if nchw else (N, H, W, C))), torch.full((N,), 0.5, device="cuda")
+        yield (lambda: tab.QuantizeNCHW(t, q_ths, bits, N, C, H, W)) if nchw else (lambda: tab.Quantize(t, q_ths, bits, N, H, W, C))
+    conv = tab_nn.TABConv2d.from_float(randn(64, 64, 3, 3), tab.TNN, 1, 1)
+    image = randn(32, 64, 56, 56)
+    yield lambda: conv(image)
+    chain = tab_nn.TABPackedChain([tab_nn.TABConv2d.from_float(randn(KN, C, 3, 3), tab.BNN, s, 1)
+                                   for C, KN, s in ((64, 64, 1), (64, 128, 2), (128, 256, 2), (256, 512, 2))])
+    images = randn(64, 64, 56, 56)
+    yield lambda: chain(images)
 
 
 def timed_steps(torch, run_steps, steps, warmup_steps, reps=HEADLINE_REPS):
@@ -619,7 +652,7 @@ def main():
                    "ms_per_step_min": round(min(times) / args.steps * 1e3, 4),
                    "ms_per_step_max": round(max(times) / args.steps * 1e3, 4),
                    "warmup": f"{args.warmup} steps, then >= 20 ms of replays"},
-        "eager": {**rate(eager_times, args.steps), "note": "same step launched call by call from Python through the ctypes mirror (host-bound)"},
+        "eager": {**rate(eager_times, args.steps), "note": "same step launched call by call from Python through tab_amd.Conv2d (host-bound)"},
         "eager_TAB_CUDA": {**rate(ext_times, args.steps),
                            "note": "same step call by call through the drop-in pybind11 module TAB_CUDA.Conv2d (host-bound)"},
         "one_step_per_graph": {**rate(single_times, args.steps),
