@@ -61,7 +61,7 @@ class TABConv2d(nn.Module):
                 f"padding={self.padding}, type={names[self.conv_type]}, data_format={self.data_format}")
 
 
-_PLAIN_CONV = _C.PlainClass(TABConv2d)
+_PLAIN_CONV = _C.plain_class(TABConv2d)
 
 
 class TABLinear(nn.Module):
