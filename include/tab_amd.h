@@ -72,8 +72,7 @@ int tab_out_extent(int in, int pad, int k, int stride);
  *            for tab_quantize_nchw, 16 bytes for tab_quantize_format); every element is written
  *   dev_BTN  int32 [N]; bitwidth 2: popcount of item n's nonzero plane (TAB_GEMM.cu:150-160,
  *            for every n); bitwidth 1: zeros (TAB_GEMM.cu:283).  NULL: not wanted (an activation's
- *            counts are read by nobody); the launches that produce them are then skipped.  The same
- *            holds for tab_quantize_nchw.
+ *            counts are read by nobody); none are made then.  The same holds for tab_quantize_nchw.
  */
 int tab_quantize(const float *dev_X, const float *dev_ths, int bitwidth, int N, int H, int W,
                  int C, int64_t *dev_QX, int32_t *dev_BTN, void *stream);
@@ -152,8 +151,8 @@ size_t tab_conv2d_workspace_bytes(int type, int N, int H, int W, int C);
  * Types 4 and 5 (CPU-only in the reference, TAB_CPU.cpp:507-614) are accepted too: X goes through
  * tab_quantize_format, dev_QW holds the same format, zero words are the value 0, and Y is
  * DRFGEMM_baseline's / RTNGEMM_baseline's integer as fp32.  Type 4 needs 9 * 64 * K words < 2^24.
- * Launches: the quantizer, then the fused pad + im2row + GEMM kernel; a small 1x1 convolution without
- * padding (64, 128, 256 or 512 channels, types 0..3) quantizes and multiplies in ONE kernel and leaves
+ * Launches: the quantizer, then the fused pad + im2row + GEMM kernel; a 1x1 convolution without padding of a
+ * moderate size (types 0..3) and any call of a few microseconds quantize and multiply in ONE kernel and leave
  * the workspace untouched.  tab_conv2d_launches() says which (1 or 2; 0 on bad arguments), for tools that
  * attribute time per launch; dev_X matters only through its alignment.
  */
@@ -244,7 +243,8 @@ int tab_conv2d_packed_out_const(const int64_t *dev_QX, const int64_t *dev_QW, co
  * tab_conv2d always runs the quantizer and the chosen conv kernel as two launches.
  *   TAB_CONV_AUTO      (tile -1) the library's choice: matrix cores, tile picked from the shape
  *   TAB_CONV_MATRIX    bit planes expanded to FP4 operands of v_mfma_f32_32x32x64_f8f6f4;
- *                      tile 0: 128x128, 1: 128x64, 2: 64x64, 3: 32x32 with K split over the
+ *                      tile 0: 128x128, 1: 128x64 (128x32 for at most 32 filters, fp32 output and an even
+ *                      number of words per pixel; 8 then 64x32), 2: 64x64, 3: 32x32 with K split over the
  *                      four waves, 4: 256x64, 5: 256x128, 6: 128x256, 7: weights resident in registers
  *                      (K of at most nine words; longer K takes the library's choice), 8: 64x64 and
  *                      9: 128x128 with K split over four / two groups of waves inside the workgroup (an

@@ -396,7 +396,7 @@ hipError_t launch_conv_mfma(int type, const ConvArgs &args, int shape, hipStream
 }
 
 // Workgroup tile of the matrix-core kernel: the shape with the lowest predicted duration under a cost model fitted to
-// the measured duration of every shape on some 430 (type, layer) cases (tab_conv_shape_model.h: the ResNet-18 layers at
+// the measured duration of every shape on 420 (type, layer) cases (tab_conv_shape_model.h: the ResNet-18 layers at
 // N = 16 / 64 / 256, the VGG stack, the 28x28 sweep and layers of other geometries).  What the model's features say:
 // the busiest CU decides (ceil(tiles / CUs) tiles of a shape land on it, and it is refilled when it holds no more), K
 // scales the loop, the size of Y the epilogue (with a price of its own where K is at most nine words and the launch is
