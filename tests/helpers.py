@@ -4,10 +4,25 @@ Nothing here restates the oracle's C code: `dequantize_*` and `torch_conv_refere
 through torch.nn.functional.conv2d on {-1,0,+1} tensors, and `brute_*` are per-element
 closed forms in numpy.
 """
+import contextlib
+
 import numpy as np
 import torch
 
 TYPE_NAMES = {0: "TNN", 1: "TBN", 2: "BTN", 3: "BNN", 4: "DRF", 5: "RTN"}
+
+
+@contextlib.contextmanager
+def two_launches():
+    """Conv2d as quantizer and convolution whatever the call's size (small ones are one launch): a kernel choice is held, of
+    the library's own tile."""
+    import tab_amd
+
+    tab_amd.set_conv_kernel(tab_amd.CONV_MATRIX, -1)
+    try:
+        yield
+    finally:
+        tab_amd.set_conv_kernel(tab_amd.CONV_AUTO, -1)
 
 
 def act_bits(type):

@@ -13,7 +13,7 @@ import torch
 
 import oracle
 import tab_amd
-from helpers import TYPE_NAMES, act_bits, make_layer, weight_bits
+from helpers import TYPE_NAMES, act_bits, make_layer, two_launches, weight_bits
 
 pytestmark = pytest.mark.gpu
 
@@ -31,6 +31,10 @@ def _against_oracle(type, N, H, W, C, KN, KH, KW, p1, p2, s1, s2, seed=0, relu=F
     assert np.array_equal(QW.cpu().numpy(), qw_o) and np.array_equal(BTN.cpu().numpy(), btn_o)
     got = y.cpu().numpy()
     assert np.array_equal(got, want), f"max |diff| = {np.abs(got - want).max()}"
+    args = (type, p1, p2, s1, s2, N, H, W, C, KN, KH, KW)
+    if tab_amd.conv2d_launches(x.cuda(), *args) == 1:
+        with two_launches():
+            assert torch.equal(tab_amd.Conv2d(x.cuda(), QW, x_ths.cuda(), BTN, *args), y)
 
 
 def _full_batch_properties(type, N, H, W, C, KN, KH, KW, p1, p2, s1, s2, seed=0, relu=False):

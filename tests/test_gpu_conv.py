@@ -6,7 +6,7 @@ import torch
 
 import oracle
 import tab_amd
-from helpers import TYPE_NAMES, act_bits, make_layer, weight_bits
+from helpers import TYPE_NAMES, act_bits, make_layer, two_launches, weight_bits
 
 pytestmark = pytest.mark.gpu
 
@@ -29,6 +29,10 @@ def _conv_case(type, N, H, W, C, KN, KH, KW, p1, p2, s1, s2, seed=0, relu=False)
     QX, _ = tab_amd.Quantize(x.cuda(), x_ths.cuda(), act_bits(type), N, H, W, C)
     y2 = tab_amd.Conv2dPacked(QX, QW, BTN, type, p1, p2, s1, s2, N, H, W, C, KN, KH, KW)
     assert torch.equal(y, y2)
+    args = (type, p1, p2, s1, s2, N, H, W, C, KN, KH, KW)
+    if tab_amd.conv2d_launches(x.cuda(), *args) == 1:  # and so do quantizer and convolution as two launches
+        with two_launches():
+            assert torch.equal(tab_amd.Conv2d(x.cuda(), QW, x_ths.cuda(), BTN, *args), y)
 
 
 @pytest.mark.parametrize("type", [0, 1, 2, 3])

@@ -7,7 +7,7 @@ import torch
 
 import oracle
 import tab_amd
-from helpers import TYPE_NAMES
+from helpers import TYPE_NAMES, two_launches
 
 pytestmark = pytest.mark.gpu
 
@@ -78,6 +78,10 @@ def test_conv2d_from_floats(type, case):
     assert np.array_equal(QW.cpu().numpy(), qw_o)
     got = y.cpu().numpy()
     assert got.shape == want.shape and np.array_equal(got, want), f"max |diff| = {np.abs(got - want).max()}"
+    with two_launches():  # (small calls are one)
+        y2 = tab_amd.Conv2d(torch.from_numpy(x).cuda(), QW, torch.from_numpy(x_ths).cuda(), btn, type, p1, p2, s1, s2,
+                            N, H, W, C, KN, KH, KW)
+    assert torch.equal(y2, y)
 
 
 KERNELS = [(tab_amd.CONV_MATRIX, t) for t in range(12)] + [(tab_amd.CONV_POPCOUNT, -1)]

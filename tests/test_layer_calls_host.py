@@ -5,6 +5,7 @@ import torch
 import torch.fx
 
 import tab_amd
+from tab_amd import nn as tab_nn
 from tab_amd.nn import TABConv2d, TABLinear, TABPackedChain
 
 
@@ -41,10 +42,11 @@ def _linear(conv_type=tab_amd.BNN):
 def test_linear_runs_the_inner_layers_compiled_call(monkeypatch):
     """Module.compile() replaces what calling the module runs."""
     fc, x = _linear(), torch.zeros(3, 64)
-    with pytest.raises(RuntimeError, match="must be a CUDA tensor"):
-        fc(x)
+    with pytest.raises(RuntimeError, match="must be a CUDA tensor"):  # the one-call path (None: the call is left to the module)
+        tab_nn._C.linear_forward(fc, tab_nn._PLAIN_CONV, x)
     monkeypatch.setattr(torch, "compile", lambda call, *args, **kwargs: lambda x: torch.full((x.shape[0], 1, 1, 8), 7.0))
     fc.conv.compile()
+    assert tab_nn._C.linear_forward(fc, tab_nn._PLAIN_CONV, x) is None
     assert torch.equal(fc(x), torch.full((3, 8), 7.0))
 
 

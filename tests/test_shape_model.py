@@ -73,7 +73,7 @@ def _tuning_script(name):
 
 @pytest.mark.parametrize("timings, cases", [("conv_shape_training_timings.txt", 280), ("conv_narrow_timings.txt", 170)])
 def test_choice_on_the_training_cases_stays_within_the_stated_regret(timings, cases):
-    """The compiled chooser (256 compute units where no device is present, as on the box the timings come from) on the model's
+    """The compiled chooser (256 compute units where no device is present, as an MI355X has) on the model's
     own training cases, and on the layers of at most 32 filters that its rule for those was not fitted to: summed over them,
     the measured duration of its choice is within 2 % of the best measured candidate (1.4 % on either), and no single choice
     is more than 25 % off."""

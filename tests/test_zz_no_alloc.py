@@ -1,15 +1,17 @@
 """tab_conv2d_static (the packed activation in the library's built-in device scratch, no allocation in the call)
 against tab_conv2d (caller-owned workspace) through the C ABI: bit-identical outputs, on calls in a row that
-share the scratch, the later ones with smaller inputs."""
-import ctypes
+share the scratch, the later ones with smaller inputs.  Small calls are one launch that leaves the scratch alone: every
+test also holds a kernel choice, under which they are two launches that go through it."""
+import contextlib
 
 import numpy as np
 import pytest
 import torch
 
-from helpers import make_layer, weight_bits
+from helpers import make_layer, two_launches, weight_bits
 
 pytestmark = pytest.mark.gpu
+launches = pytest.mark.parametrize("launches", [contextlib.nullcontext, two_launches], ids=["own_choice", "two_launches"])
 
 
 def _both(lib, check, type, N, H, W, C, KN, KH, KW, p1, p2, s1, s2, seed, relu=False):
@@ -47,16 +49,19 @@ def _both(lib, check, type, N, H, W, C, KN, KH, KW, p1, p2, s1, s2, seed, relu=F
     return y_static
 
 
+@launches
 @pytest.mark.parametrize("type", [0, 1, 2, 3])
-def test_static_scratch_matches_workspace_on_calls_in_a_row(type):
+def test_static_scratch_matches_workspace_on_calls_in_a_row(type, launches):
     from tab_amd import _capi
 
     lib = _capi.load()
-    # a large call first, then smaller ones that find its packed activation still in the scratch
-    _both(lib, _capi.check, type, 4, 28, 28, 256, 128, 3, 3, 1, 1, 1, 1, seed=10 + type, relu=type in (1, 2))
-    _both(lib, _capi.check, type, 2, 14, 14, 128, 64, 3, 3, 1, 1, 2, 2, seed=20 + type)
-    _both(lib, _capi.check, type, 1, 9, 7, 70, 33, 1, 1, 0, 0, 2, 2, seed=30 + type)   # the strided 1x1 quantizer
-    y = _both(lib, _capi.check, type, 1, 8, 8, 64, 64, 3, 3, 1, 0, 1, 1, seed=40 + type)
+    with launches():
+        # a large call first, then smaller ones that find its packed activation still in the scratch
+        _both(lib, _capi.check, type, 4, 28, 28, 256, 128, 3, 3, 1, 1, 1, 1, seed=10 + type, relu=type in (1, 2))
+        _both(lib, _capi.check, type, 2, 14, 14, 128, 64, 3, 3, 1, 1, 2, 2, seed=20 + type)
+        _both(lib, _capi.check, type, 1, 9, 7, 70, 33, 1, 1, 0, 0, 2, 2, seed=30 + type)
+        _both(lib, _capi.check, type, 1, 9, 7, 192, 33, 1, 1, 0, 0, 2, 2, seed=35 + type)   # the strided 1x1 quantizer
+        y = _both(lib, _capi.check, type, 1, 8, 8, 64, 64, 3, 3, 1, 0, 1, 1, seed=40 + type)
     # and against the oracle, once
     import oracle
 
@@ -66,8 +71,9 @@ def test_static_scratch_matches_workspace_on_calls_in_a_row(type):
     assert np.array_equal(y.cpu().numpy().reshape(want.shape), want)
 
 
+@launches
 @pytest.mark.parametrize("type", [0, 3])
-def test_static_scratch_under_graph_capture(type):
+def test_static_scratch_under_graph_capture(type, launches):
     """The use the entry point is made for: captured into a HIP graph after a first eager call, replayed several times
     with the program's own eager work and synchronisations in between, every replay equal to tab_conv2d's result."""
     import tab_amd
@@ -81,22 +87,24 @@ def test_static_scratch_under_graph_capture(type):
     want = tab_amd.Conv2d(xd, QW, td, BTN, type, 1, 1, 1, 1, N, H, W, C, KN, 3, 3)
     out = torch.zeros_like(want)
     args = (xd.data_ptr(), QW.data_ptr(), td.data_ptr(), BTN.data_ptr(), type, 1, 1, 1, 1, N, H, W, C, KN, 3, 3, out.data_ptr())
-    _capi.check(lib, lib.tab_conv2d_static(*args, torch.cuda.current_stream().cuda_stream))  # address lookup, outside the capture
-    torch.cuda.synchronize()
-    graph = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(graph):
-        _capi.check(lib, lib.tab_conv2d_static(*args, torch.cuda.current_stream().cuda_stream))
-    for replay in range(4):
-        out.fill_(float("nan"))
-        # eager work that reuses the scratch between the replays: a different, smaller call
-        tab_amd.Conv2dStatic(xd[:1].contiguous(), QW, td[:1].contiguous(), BTN, type, 1, 1, 1, 1, 1, H, W, C, KN, 3, 3)
+    with launches():
+        _capi.check(lib, lib.tab_conv2d_static(*args, torch.cuda.current_stream().cuda_stream))  # address lookup, outside the capture
         torch.cuda.synchronize()
-        graph.replay()
-        torch.cuda.synchronize()
-        assert torch.equal(out, want), f"replay {replay}"
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            _capi.check(lib, lib.tab_conv2d_static(*args, torch.cuda.current_stream().cuda_stream))
+        for replay in range(4):
+            out.fill_(float("nan"))
+            # eager work that reuses the scratch between the replays: a different, smaller call
+            tab_amd.Conv2dStatic(xd[:1].contiguous(), QW, td[:1].contiguous(), BTN, type, 1, 1, 1, 1, 1, H, W, C, KN, 3, 3)
+            torch.cuda.synchronize()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, want), f"replay {replay}"
 
 
-def test_static_scratch_formats_4_and_5():
+@launches
+def test_static_scratch_formats_4_and_5(launches):
     import tab_amd
     from tab_amd import _capi
 
@@ -109,7 +117,8 @@ def test_static_scratch_formats_4_and_5():
         QW = tab_amd.QuantizeFormat(w.cuda(), w_ths.cuda(), type, KN, 3, 3, C)
         btn = torch.zeros(KN, dtype=torch.int32, device="cuda")
         want = tab_amd.Conv2d(x.cuda(), QW, x_ths.cuda(), btn, type, 1, 1, 1, 1, N, H, W, C, KN, 3, 3)
-        got = tab_amd.Conv2dStatic(x.cuda(), QW, x_ths.cuda(), btn, type, 1, 1, 1, 1, N, H, W, C, KN, 3, 3)
+        with launches():
+            got = tab_amd.Conv2dStatic(x.cuda(), QW, x_ths.cuda(), btn, type, 1, 1, 1, 1, N, H, W, C, KN, 3, 3)
         torch.cuda.synchronize()
         assert torch.equal(want, got)
 
