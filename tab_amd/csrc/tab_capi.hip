@@ -294,8 +294,9 @@ static int conv_packed(const int64_t *dev_QX, const int64_t *dev_QW, const int32
     // (the cache takes the stores faster than HBM: Y of 190-206 MB 1-11 % sooner); every other Y with non-temporal
     // stores: a smaller one leaves no dirty L2 to flush when the launch ends (7-25 % sooner), a larger one would only
     // push the operands out (Y of 411 MB: 7-28 % sooner).  At 103 MB the two policies measured within 3 %.
+    // A Y of 24 MB or more whose rows are no whole cache lines goes through the caches (tab::ragged_rows_cached).
     const long y_bytes = s.M * (long)KN * 4;
-    a.y_cached = y_bytes >= (128L << 20) && y_bytes <= (240L << 20);
+    a.y_cached = (y_bytes >= (128L << 20) && y_bytes <= (240L << 20)) || tab::ragged_rows_cached(s.M, KN);
     a.div_filter_tiles = tab::make_div32(1);
     hipError_t e = tab::launch_conv(type, a, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return device_fail(e, "conv launch");

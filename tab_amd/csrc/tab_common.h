@@ -50,6 +50,16 @@ __host__ __device__ __forceinline__ uint32_t div32(uint32_t x, Div32 f)
     return (uint32_t)(((uint64_t)x * f.mul) >> f.shift);
 }
 
+// Whether an fp32 Y of M rows of KN filters is written through the caches because its rows are no whole cache lines: a line is
+// then completed by two waves or two tiles, and non-temporal stores send its parts to memory one by one once Y outgrows what the
+// L2s hold (32 MB).  Non-temporal / cached, us: KN = 41 103 MB 83 / 26, KN = 106 115 MB 79 / 28, KN = 70 179 MB 132 / 51, KN = 958 52 MB
+// 55 / 43, KN = 517 31 MB 11.4 / 9.5; one launch of quantizer and 1x1 conv: KN = 70 56 MB 51 / 26, KN = 513 26 MB 12.9 / 10.0, but KN = 100
+// 20 MB 7.4 / 9.2.  At most 32 filters are one wave's own block of contiguous rows (KN = 25 29 MB 28.6 / 29.4).
+__host__ __device__ __forceinline__ bool ragged_rows_cached(long M, int KN)
+{
+    return KN % 32 != 0 && KN > 32 && M * KN >= (6L << 20);
+}
+
 // Arguments of the fused pad + im2row + GEMM kernels; they travel as ConvParams (below).
 struct ConvArgs {
     const uint64_t *qx;  // packed activation [N][H][W][PC][APL]; PC = words per pixel and plane

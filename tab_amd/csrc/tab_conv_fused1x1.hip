@@ -48,7 +48,8 @@ enum FusedInput {
 };
 
 // NP: pairs of words, enough for a pixel's (1, 2 or 4).
-template <int TYPE, int NP, int INPUT>
+// CACHED: Y through the caches (ragged_rows_cached).
+template <int TYPE, int NP, int INPUT, bool CACHED>
 __global__ __launch_bounds__(kConvThreads) void conv1x1_fused(const Fused1x1Args p)
 {
     static_assert(TYPE >= 0 && TYPE <= 3, "types 0..3");
@@ -252,7 +253,7 @@ __global__ __launch_bounds__(kConvThreads) void conv1x1_fused(const Fused1x1Args
 #pragma unroll
             for (int i = 0; i < 4; i++)  // accumulator element 4j+i of lane (kb, r) is pixel 8j+4kb+i, filter n0 + r
                 __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[4 * j + i] + bias), out, lane_off + (uint32_t)(8 * j + i) * row_bytes, 0,
-                                                      kStreamingStore);
+                                                      CACHED ? 0 : kStreamingStore);
     }
 }
 
@@ -263,7 +264,7 @@ int fused_tiles(int PC, long blocks, int KN) { return PC >= 3 && blocks >= 1024 
 
 long fused_blocks(long M, int KN) { return (M + 31) / 32 * ((KN + 127) / 128); }
 
-template <int TYPE, int NP>
+template <int TYPE, int NP, bool CACHED>
 hipError_t launch_fused_rows(const Fused1x1Args &a, hipStream_t stream)
 {
     const int PC = (a.C + kWordBits - 1) / kWordBits;
@@ -271,23 +272,29 @@ hipError_t launch_fused_rows(const Fused1x1Args &a, hipStream_t stream)
     const dim3 grid((unsigned)((a.M + 31) / 32), (unsigned)((a.KN + 128 * tiles - 1) / (128 * tiles)));
     const unsigned lds = 2 * NP * 32 * Planes<TYPE>::A * 8;
     if (a.C % kWordBits != 0 || (uintptr_t)a.x % 16 != 0) {
-        if constexpr (NP == 1) conv1x1_fused<TYPE, NP, kInputRagged><<<grid, dim3(kConvThreads), lds, stream>>>(a);
+        if constexpr (NP == 1) conv1x1_fused<TYPE, NP, kInputRagged, CACHED><<<grid, dim3(kConvThreads), lds, stream>>>(a);
         else return hipErrorInvalidValue;
     } else if (NP >= 2 && PC % 4 == 0) {
-        if constexpr (NP >= 2) conv1x1_fused<TYPE, NP, kInputQuads><<<grid, dim3(kConvThreads), lds, stream>>>(a);
+        if constexpr (NP >= 2) conv1x1_fused<TYPE, NP, kInputQuads, CACHED><<<grid, dim3(kConvThreads), lds, stream>>>(a);
     } else {
-        conv1x1_fused<TYPE, NP, kInputWords><<<grid, dim3(kConvThreads), lds, stream>>>(a);
+        conv1x1_fused<TYPE, NP, kInputWords, CACHED><<<grid, dim3(kConvThreads), lds, stream>>>(a);
     }
     return hipGetLastError();
+}
+
+template <int TYPE, bool CACHED>
+hipError_t launch_fused_words(const Fused1x1Args &a, hipStream_t stream)
+{
+    const int PC = (a.C + kWordBits - 1) / kWordBits;
+    if (PC <= 2) return launch_fused_rows<TYPE, 1, CACHED>(a, stream);
+    if (PC <= 4) return launch_fused_rows<TYPE, 2, CACHED>(a, stream);
+    return launch_fused_rows<TYPE, 4, CACHED>(a, stream);
 }
 
 template <int TYPE>
 hipError_t launch_fused_type(const Fused1x1Args &a, hipStream_t stream)
 {
-    const int PC = (a.C + kWordBits - 1) / kWordBits;
-    if (PC <= 2) return launch_fused_rows<TYPE, 1>(a, stream);
-    if (PC <= 4) return launch_fused_rows<TYPE, 2>(a, stream);
-    return launch_fused_rows<TYPE, 4>(a, stream);
+    return ragged_rows_cached(a.M, a.KN) ? launch_fused_words<TYPE, true>(a, stream) : launch_fused_words<TYPE, false>(a, stream);
 }
 
 }  // namespace
