@@ -133,6 +133,13 @@ int tab_conv2d_launches(const float *dev_X, int type, int padding1, int padding2
 size_t tab_conv2d_workspace_bytes(int type, int N, int H, int W, int C);
 
 /*
+ * The same with room for the weights in the order of the library's fastest kernel for large layers, which the quantizer's launch
+ * then lays out there on every call.  A workspace of tab_conv2d_workspace_bytes() takes every call too, with the kernels that
+ * read the weights where they lie; the results are the same.  0 on bad arguments.
+ */
+size_t tab_conv2d_workspace_bytes_full(int type, int N, int H, int W, int C, int KN, int KH, int KW);
+
+/*
  * Replaces ConvWithCuda_TAB (TAB_GEMM.cu:325-527), the body of
  * TAB_Conv2d(X, QW, thresholds, btn, type, padding1, padding2, stride1, stride2,
  *            N, H, W, C, KN, KH, KW) (TAB_GPU.cpp:34-42).
@@ -223,6 +230,8 @@ int tab_conv2d_packed_out(const int64_t *dev_QX, const int64_t *dev_QW, const in
  *              tab_threshold_workspace_bytes(N, H*W*C) for two planes and none for one
  */
 size_t tab_layer_workspace_bytes(int bitwidth, int N, int H, int W, int C);
+/* The same for tab_layer_conv2d with room for the weights, as tab_conv2d_workspace_bytes_full. */
+size_t tab_layer_workspace_bytes_full(int type, int N, int H, int W, int C, int KN, int KH, int KW);
 int tab_layer_quantize(const float *dev_X, int nchw, int bitwidth, float act_scale, int N, int H, int W, int C,
                        int64_t *dev_QX, void *workspace, size_t workspace_bytes, void *stream);
 int tab_layer_conv2d(const float *dev_X, int nchw, float act_scale, const int64_t *dev_QW, const int32_t *dev_btn,

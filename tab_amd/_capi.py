@@ -26,6 +26,7 @@ SIGNATURES = {
     "tab_threshold_workspace_bytes": (_sz, [_int, ctypes.c_long]),
     "tab_threshold": (_int, [_vp, _int, ctypes.c_long, ctypes.c_float, _vp, _vp, _sz, _vp]),
     "tab_conv2d_workspace_bytes": (_sz, [_int] * 5),
+    "tab_conv2d_workspace_bytes_full": (_sz, [_int] * 8),
     "tab_conv2d": (_int, [_vp] * 4 + [_int] * 12 + [_vp, _vp, _sz, _vp]),
     "tab_conv2d_launches": (_int, [_vp] + [_int] * 12),
     "tab_static_scratch_bytes": (_sz, []),
@@ -34,6 +35,7 @@ SIGNATURES = {
     "tab_conv2d_packed_out": (_int, [_vp] * 3 + [_int] * 12 + [_vp, _int, _vp, _vp]),
     "tab_conv2d_packed_out_const": (_int, [_vp] * 3 + [_int] * 12 + [ctypes.c_float, _int, _vp, _vp]),
     "tab_layer_workspace_bytes": (_sz, [_int] * 5),
+    "tab_layer_workspace_bytes_full": (_sz, [_int] * 8),
     "tab_layer_quantize": (_int, [_vp, _int, _int, ctypes.c_float] + [_int] * 4 + [_vp, _vp, _sz, _vp]),
     "tab_layer_conv2d": (_int, [_vp, _int, ctypes.c_float, _vp, _vp] + [_int] * 12 + [_vp, _vp, _sz, _vp]),
     "tab_set_conv_kernel": (_int, [_int, _int]),

@@ -125,6 +125,10 @@ void tab_internal_set_tail_round(int workgroups) { tab::set_tail_round(workgroup
 /* Test hook, absent from include/tab_amd.h: the compute units that the rules choosing a kernel count; 0 = the device's. */
 void tab_internal_set_compute_units(int units) { tab::set_compute_units(units); }
 
+/* Test hook, absent from include/tab_amd.h: convolutions from fp32 take this shape (12 .. 16) of the kernel that keeps the input
+ * patch in LDS wherever its patch fits; tab_set_conv_kernel ends it. */
+void tab_internal_force_patch(int shape) { tab::force_conv_tile(9, shape); }
+
 int tab_set_conv_kernel(int kernel, int tile)
 {
     static const int popcount_tm[4] = {7, 8, 4, 2};  // 7: the popcount kernel's own choice
@@ -224,6 +228,20 @@ size_t tab_conv2d_workspace_bytes(int type, int N, int H, int W, int C)
     return (size_t)N * H * W * tab_operand_words(type, 0, C) * sizeof(int64_t);
 }
 
+/* Room for a convolution's weights in another kernel's order, aligned. */
+static size_t spare_weight_bytes(int type, int C, int KN, int KH, int KW)
+{
+    const size_t bytes = KH > 1 || KW > 1 ? tab::patch_weight_bytes(type, C, KN, KH, KW) : 0;
+    return bytes ? bytes + 16 : 0;
+}
+
+size_t tab_conv2d_workspace_bytes_full(int type, int N, int H, int W, int C, int KN, int KH, int KW)
+{
+    const size_t need = tab_conv2d_workspace_bytes(type, N, H, W, C);
+    if (need == 0 || KN < 1 || KH < 1 || KW < 1) return 0;
+    return need + spare_weight_bytes(type, C, KN, KH, KW);
+}
+
 int tab_quantize_format(const float *dev_X, const float *dev_ths, int type, int N, int H, int W, int C,
                         int64_t *dev_QX, void *stream)
 {
@@ -249,32 +267,19 @@ static int check_conv_pointers(const ConvShape &s, int type, const void *dev_QX,
     return TAB_OK;
 }
 
-/* Shared body of the packed-activation entry points: Y as fp32 (dev_Y) or thresholded (dev_out_ths per image, or out_th
- * for all of them) and packed (dev_QY). */
-static int conv_packed(const int64_t *dev_QX, const int64_t *dev_QW, const int32_t *dev_btn, int type, int padding1,
-                       int padding2, int stride1, int stride2, int N, int H, int W, int C, int KN, int KH, int KW,
-                       float *dev_Y, const float *dev_out_ths, float out_th, int out_bitwidth, int64_t *dev_QY, void *stream)
+/* The kernels' arguments for fp32 output. */
+static tab::ConvArgs conv_args(const ConvShape &s, int padding1, int padding2, int stride1, int stride2, int N, int H, int W, int C, int KN,
+                               int KH, int KW, const void *dev_QX, const int64_t *dev_QW, const int32_t *dev_btn, float *dev_Y)
 {
-    ConvShape s;
-    int rc = check_conv(type, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, &s);
-    if (rc != TAB_OK) return rc;
-    rc = check_conv_pointers(s, type, dev_QX, dev_QW, dev_btn, dev_Y, dev_QY);
-    if (rc != TAB_OK) return rc;
-    if (dev_QY) {
-        if (out_bitwidth != 1 && out_bitwidth != 2)
-            return fail(TAB_ERR_BAD_ARGUMENT, "out_bitwidth must be 1 or 2, got %d", out_bitwidth);
-        if ((uintptr_t)dev_QY % (8 * out_bitwidth)) return fail(TAB_ERR_BAD_ARGUMENT, "QY must be aligned to a whole packed element");
-    }
-
     tab::ConvArgs a;
-    a.qx = reinterpret_cast<const uint64_t *>(dev_QX);
+    a.qx = static_cast<const uint64_t *>(dev_QX);
     a.qw = reinterpret_cast<const uint64_t *>(dev_QW);
     a.btn = dev_btn;
     a.y = dev_Y;
-    a.qy = reinterpret_cast<uint32_t *>(dev_QY);
-    a.out_ths = dev_out_ths;
-    a.out_th = out_th;
-    a.out_bits = out_bitwidth;
+    a.qy = nullptr;
+    a.out_ths = nullptr;
+    a.out_th = 0.f;
+    a.out_bits = 0;
     a.N = N; a.H = H; a.W = W; a.PC = s.PC;
     a.KN = KN; a.KH = KH; a.KW = KW;
     a.p1 = padding1; a.p2 = padding2; a.s1 = stride1; a.s2 = stride2;
@@ -298,6 +303,31 @@ static int conv_packed(const int64_t *dev_QX, const int64_t *dev_QW, const int32
     const long y_bytes = s.M * (long)KN * 4;
     a.y_cached = (y_bytes >= (128L << 20) && y_bytes <= (240L << 20)) || tab::ragged_rows_cached(s.M, KN);
     a.div_filter_tiles = tab::make_div32(1);
+    return a;
+}
+
+/* Shared body of the packed-activation entry points: Y as fp32 (dev_Y) or thresholded (dev_out_ths per image, or out_th
+ * for all of them) and packed (dev_QY). */
+static int conv_packed(const int64_t *dev_QX, const int64_t *dev_QW, const int32_t *dev_btn, int type, int padding1,
+                       int padding2, int stride1, int stride2, int N, int H, int W, int C, int KN, int KH, int KW,
+                       float *dev_Y, const float *dev_out_ths, float out_th, int out_bitwidth, int64_t *dev_QY, void *stream)
+{
+    ConvShape s;
+    int rc = check_conv(type, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, &s);
+    if (rc != TAB_OK) return rc;
+    rc = check_conv_pointers(s, type, dev_QX, dev_QW, dev_btn, dev_Y, dev_QY);
+    if (rc != TAB_OK) return rc;
+    if (dev_QY) {
+        if (out_bitwidth != 1 && out_bitwidth != 2)
+            return fail(TAB_ERR_BAD_ARGUMENT, "out_bitwidth must be 1 or 2, got %d", out_bitwidth);
+        if ((uintptr_t)dev_QY % (8 * out_bitwidth)) return fail(TAB_ERR_BAD_ARGUMENT, "QY must be aligned to a whole packed element");
+    }
+
+    tab::ConvArgs a = conv_args(s, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, dev_QX, dev_QW, dev_btn, dev_Y);
+    a.qy = reinterpret_cast<uint32_t *>(dev_QY);
+    a.out_ths = dev_out_ths;
+    a.out_th = out_th;
+    a.out_bits = out_bitwidth;
     hipError_t e = tab::launch_conv(type, a, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return device_fail(e, "conv launch");
     return TAB_OK;
@@ -330,6 +360,49 @@ int tab_conv2d_packed_out_const(const int64_t *dev_QX, const int64_t *dev_QW, co
     if (!dev_QY) return fail(TAB_ERR_BAD_ARGUMENT, "null device pointer");
     return conv_packed(dev_QX, dev_QW, dev_btn, type, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW,
                        nullptr, nullptr, out_threshold, out_bitwidth, dev_QY, stream);
+}
+
+/* Test hook, absent from include/tab_amd.h: the shape (12 .. 16) of the kernel that keeps the input patch in LDS which the library would
+ * pick for a convolution from fp32, -1 for another kernel; what[0..2]: words of a chunk, pixels and LDS bytes of its patch. */
+int tab_internal_conv_patch_shape(int type, int padding1, int padding2, int stride1, int stride2, int N, int H, int W, int C, int KN, int KH,
+                                  int KW, int *what, size_t *weight_bytes)
+{
+    ConvShape s;
+    if (check_conv(type, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, &s) != TAB_OK) return -1;
+    const tab::ConvArgs a = conv_args(s, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, nullptr, nullptr, nullptr, nullptr);
+    const tab::PatchPlan plan = tab::conv_patch_plan(type, a);
+    if (plan.shape < 0) return -1;
+    what[0] = plan.kc;
+    what[1] = plan.npix;
+    what[2] = plan.lds_bytes;
+    *weight_bytes = plan.weight_bytes;
+    return plan.shape;
+}
+
+/* Test hook, absent from include/tab_amd.h: the shape that tab_internal_force_patch holds, on an activation already packed; fp32
+ * output to dev_Y, or packed to dev_QY (out_bitwidth planes, one threshold).  what: 1 = lay the weights out in `weights`
+ * (weight_bytes bytes), 2 = convolve with those there, 3 = both. */
+int tab_internal_conv_patch(const int64_t *dev_QX, const int64_t *dev_QW, const int32_t *dev_btn, int type, int padding1, int padding2,
+                            int stride1, int stride2, int N, int H, int W, int C, int KN, int KH, int KW, float *dev_Y, float out_threshold,
+                            int out_bitwidth, int64_t *dev_QY, void *weights, size_t weight_bytes, int what, void *stream)
+{
+    ConvShape s;
+    int rc = check_conv(type, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, &s);
+    if (rc == TAB_OK) rc = check_conv_pointers(s, type, dev_QX, dev_QW, dev_btn, dev_Y, dev_QY);
+    if (rc != TAB_OK) return rc;
+    tab::ConvArgs a = conv_args(s, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, dev_QX, dev_QW, dev_btn, dev_Y);
+    a.qy = reinterpret_cast<uint32_t *>(dev_QY);
+    a.out_th = out_threshold;
+    a.out_bits = out_bitwidth;
+    const tab::PatchPlan plan = tab::conv_patch_plan(type, a);
+    if (plan.shape < 0) return fail(TAB_ERR_BAD_SHAPE, "the patch does not fit");
+    if (!weights || weight_bytes < plan.weight_bytes) return fail(TAB_ERR_WORKSPACE, "weights take %zu bytes", plan.weight_bytes);
+    hipError_t e = hipSuccess;
+    if (what & 1) e = tab::launch_patch_weights(tab::patch_weight_job(type, a, plan, static_cast<uint64_t *>(weights)), static_cast<hipStream_t>(stream));
+    a.qw = static_cast<const uint64_t *>(weights);
+    if (e == hipSuccess && (what & 2)) e = tab::launch_conv_mfma(type, a, plan.shape, static_cast<hipStream_t>(stream));
+    if (e != hipSuccess) return device_fail(e, "conv launch");
+    return TAB_OK;
 }
 
 /* Device address of `scratch` on the current device, looked up on the first call made with that device current. */
@@ -380,11 +453,42 @@ static int one_launch(int type, const float *dev_X, bool nchw, int padding1, int
     return small ? 2 : 0;
 }
 
+/* A convolution of an activation that is still to be quantized: which kernel multiplies it, and where in the workspace (`room`
+ * bytes at `spare`, behind the packed activation) the quantizer's launch leaves the weights in that kernel's order. */
+struct ConvRoute {
+    tab::ConvArgs args;
+    tab::PatchPlan plan;
+    tab::WeightJob job;
+    const tab::WeightJob *weights() const { return plan.shape >= 0 ? &job : nullptr; }
+};
+
+static ConvRoute conv_route(const tab::ConvArgs &args, int type, void *spare, size_t room)
+{
+    ConvRoute r = {args, tab::conv_patch_plan(type, args), {}};
+    char *at = reinterpret_cast<char *>(((uintptr_t)spare + 15) & ~(uintptr_t)15);
+    const size_t lost = (size_t)(at - static_cast<char *>(spare));
+    if (r.plan.shape >= 0 && (room < lost || room - lost < r.plan.weight_bytes)) r.plan.shape = -1;
+    if (r.plan.shape >= 0) r.job = tab::patch_weight_job(type, args, r.plan, reinterpret_cast<uint64_t *>(at));
+    return r;
+}
+
+/* The convolution of a route whose quantizer has been enqueued. */
+static int run_route(const ConvRoute &r, int type, void *stream)
+{
+    tab::ConvArgs a = r.args;
+    if (r.plan.shape >= 0) a.qw = r.job.out;
+    const int shape = r.plan.shape >= 0 ? r.plan.shape : r.plan.tiled;
+    const hipError_t e = shape >= 0 ? tab::launch_conv_mfma(type, a, shape, static_cast<hipStream_t>(stream))
+                                    : tab::launch_conv(type, a, static_cast<hipStream_t>(stream));
+    if (e != hipSuccess) return device_fail(e, "conv launch");
+    return TAB_OK;
+}
+
 /* Quantize an NHWC activation of types 0..3 into the workspace, then the fused conv kernel; small and strided 1x1 layers
- * take their own ways.  The arguments have been checked. */
+ * take their own ways.  The arguments have been checked.  spare, room: of the workspace, behind what the call needs. */
 static int conv_from_nhwc(const float *dev_X, const int64_t *dev_QW, const tab::Thresholds &ths, const int32_t *dev_btn, int type,
                           int padding1, int padding2, int stride1, int stride2, int N, int H, int W, int C, int KN, int KH, int KW,
-                          const ConvShape &s, float *dev_Y, void *workspace, void *stream)
+                          const ConvShape &s, float *dev_Y, void *workspace, void *spare, size_t room, void *stream)
 {
     // One launch where it pays (only under the automatic kernel choice: a forced kernel is what the caller wants to see run):
     // a 1x1 convolution without padding, the smallest calls of any kernel.  The packed activation stays in LDS.
@@ -408,14 +512,14 @@ static int conv_from_nhwc(const float *dev_X, const int64_t *dev_QW, const tab::
         return tab_conv2d_packed(reinterpret_cast<const int64_t *>(workspace), dev_QW, dev_btn, type, 0, 0, 1, 1, N, s.OH,
                                  s.OW, C, KN, 1, 1, dev_Y, stream);
     }
+    const ConvRoute route = conv_route(conv_args(s, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, workspace, dev_QW, dev_btn, dev_Y),
+                                       type, spare, room);
     // stage 1: quantize + pack the activation (TAB_GEMM.cu:419-426); no btn for activations
     hipError_t e = tab::launch_quantize(dev_X, ths, s.abits, (long)H * W, N, C, reinterpret_cast<uint64_t *>(workspace), nullptr,
-                                        nullptr, static_cast<hipStream_t>(stream));
+                                        nullptr, static_cast<hipStream_t>(stream), route.weights());
     if (e != hipSuccess) return device_fail(e, "quantize launch");
     // stage 2: pad + im2row + GEMM, fused
-    return tab_conv2d_packed(reinterpret_cast<const int64_t *>(workspace), dev_QW, dev_btn, type,
-                             padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, dev_Y,
-                             stream);
+    return run_route(route, type, stream);
 }
 
 /* Body of tab_conv2d and tab_conv2d_static (builtin: the library's own scratch). */
@@ -438,16 +542,19 @@ static int conv_from_floats(const float *dev_X, const int64_t *dev_QW, const flo
     }
     rc = check_from_floats(s, type, dev_X, dev_QW, dev_btn, dev_Y, workspace, workspace_bytes, need);
     if (rc != TAB_OK) return rc;
+    void *const spare = static_cast<char *>(workspace) + need;
+    const size_t room = workspace_bytes - need;
     if (type > 3 && !one_launch(type, dev_X, false, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, s)) {
         // the CPU-only types: their own packers, then the same fused kernel
+        const ConvRoute route = conv_route(conv_args(s, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, workspace, dev_QW, dev_btn, dev_Y),
+                                           type, spare, room);
         hipError_t e = tab::launch_quantize_format(dev_X, dev_ths, type, (long)H * W, N, C, reinterpret_cast<uint64_t *>(workspace),
-                                                   static_cast<hipStream_t>(stream));
+                                                   static_cast<hipStream_t>(stream), route.weights());
         if (e != hipSuccess) return device_fail(e, "quantize launch");
-        return tab_conv2d_packed(reinterpret_cast<const int64_t *>(workspace), dev_QW, dev_btn, type, padding1, padding2, stride1,
-                                 stride2, N, H, W, C, KN, KH, KW, dev_Y, stream);
+        return run_route(route, type, stream);
     }
     return conv_from_nhwc(dev_X, dev_QW, tab::given_thresholds(dev_ths), dev_btn, type, padding1, padding2, stride1, stride2, N, H, W, C,
-                          KN, KH, KW, s, dev_Y, workspace, stream);
+                          KN, KH, KW, s, dev_Y, workspace, spare, room, stream);
 }
 
 /* Packed activation bytes of a layer call, rounded up so that the partial sums behind them are aligned. */
@@ -473,8 +580,16 @@ size_t tab_layer_workspace_bytes(int bitwidth, int N, int H, int W, int C)
     return layer_packed_bytes(bitwidth, N, H, W, C) + (bitwidth == 2 ? sums : 0);
 }
 
-int tab_layer_quantize(const float *dev_X, int nchw, int bitwidth, float act_scale, int N, int H, int W, int C, int64_t *dev_QX,
-                       void *workspace, size_t workspace_bytes, void *stream)
+size_t tab_layer_workspace_bytes_full(int type, int N, int H, int W, int C, int KN, int KH, int KW)
+{
+    if (type < 0 || type > 3 || KN < 1 || KH < 1 || KW < 1) return 0;
+    const size_t need = tab_layer_workspace_bytes(type < 2 ? 2 : 1, N, H, W, C);
+    return need ? need + spare_weight_bytes(type, C, KN, KH, KW) : 0;
+}
+
+/* weights: of the convolution that follows, or null. */
+static int layer_quantize(const float *dev_X, int nchw, int bitwidth, float act_scale, int N, int H, int W, int C, int64_t *dev_QX,
+                          void *workspace, size_t workspace_bytes, const tab::WeightJob *weights, void *stream)
 {
     if (bitwidth != 1 && bitwidth != 2) return fail(TAB_ERR_BAD_ARGUMENT, "bitwidth must be 1 or 2, got %d", bitwidth);
     if (N < 1 || H < 1 || W < 1 || C < 1) return fail(TAB_ERR_BAD_ARGUMENT, "N, H, W, C must be positive");
@@ -492,10 +607,16 @@ int tab_layer_quantize(const float *dev_X, int nchw, int bitwidth, float act_sca
     if (e != hipSuccess) return device_fail(e, "threshold launch");
     uint64_t *q = reinterpret_cast<uint64_t *>(dev_QX);
     // one pixel per image: NCHW and NHWC are the same memory, and the NHWC quantizers read it along the channels
-    e = nchw && H * W > 1 ? tab::launch_quantize_nchw(dev_X, ths, bitwidth, N, C, (long)H * W, q, nullptr, nullptr, static_cast<hipStream_t>(stream))
-                          : tab::launch_quantize(dev_X, ths, bitwidth, (long)H * W, N, C, q, nullptr, nullptr, static_cast<hipStream_t>(stream));
+    e = nchw && H * W > 1 ? tab::launch_quantize_nchw(dev_X, ths, bitwidth, N, C, (long)H * W, q, nullptr, nullptr, static_cast<hipStream_t>(stream), weights)
+                          : tab::launch_quantize(dev_X, ths, bitwidth, (long)H * W, N, C, q, nullptr, nullptr, static_cast<hipStream_t>(stream), weights);
     if (e != hipSuccess) return device_fail(e, "quantize launch");
     return TAB_OK;
+}
+
+int tab_layer_quantize(const float *dev_X, int nchw, int bitwidth, float act_scale, int N, int H, int W, int C, int64_t *dev_QX,
+                       void *workspace, size_t workspace_bytes, void *stream)
+{
+    return layer_quantize(dev_X, nchw, bitwidth, act_scale, N, H, W, C, dev_QX, workspace, workspace_bytes, nullptr, stream);
 }
 
 int tab_layer_conv2d(const float *dev_X, int nchw, float act_scale, const int64_t *dev_QW, const int32_t *dev_btn, int type,
@@ -509,15 +630,19 @@ int tab_layer_conv2d(const float *dev_X, int nchw, float act_scale, const int64_
     rc = check_from_floats(s, type, dev_X, dev_QW, dev_btn, dev_Y, workspace, workspace_bytes, tab_layer_workspace_bytes(s.abits, N, H, W, C));
     if (rc != TAB_OK) return rc;
     char *sums = static_cast<char *>(workspace) + layer_packed_bytes(s.abits, N, H, W, C);
+    const size_t need = tab_layer_workspace_bytes(s.abits, N, H, W, C);
+    void *const spare = static_cast<char *>(workspace) + need;
+    const size_t room = workspace_bytes - need;
     const bool planes = nchw && H * W > 1;  // one pixel per image: NCHW and NHWC are the same memory
     const bool own = s.abits == 2 && tab::conv_small_own_thresholds(dev_X, H, W, C, KH, KW, padding1, padding2);
     const int one = one_launch(type, dev_X, planes, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, s, own);
     if (planes && !one) {
-        rc = tab_layer_quantize(dev_X, 1, s.abits, act_scale, N, H, W, C, static_cast<int64_t *>(workspace), sums,
-                                workspace_bytes - layer_packed_bytes(s.abits, N, H, W, C), stream);
+        const ConvRoute route = conv_route(conv_args(s, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, workspace, dev_QW, dev_btn, dev_Y),
+                                           type, spare, room);
+        rc = layer_quantize(dev_X, 1, s.abits, act_scale, N, H, W, C, static_cast<int64_t *>(workspace), sums,
+                            need - layer_packed_bytes(s.abits, N, H, W, C), route.weights(), stream);
         if (rc != TAB_OK) return rc;
-        return tab_conv2d_packed(static_cast<const int64_t *>(workspace), dev_QW, dev_btn, type, padding1, padding2, stride1, stride2,
-                                 N, H, W, C, KN, KH, KW, dev_Y, stream);
+        return run_route(route, type, stream);
     }
     tab::Thresholds ths;
     hipError_t e = hipSuccess;
@@ -540,7 +665,7 @@ int tab_layer_conv2d(const float *dev_X, int nchw, float act_scale, const int64_
         return TAB_OK;
     }
     return conv_from_nhwc(dev_X, dev_QW, ths, dev_btn, type, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, s, dev_Y,
-                          workspace, stream);
+                          workspace, spare, room, stream);
 }
 
 int tab_conv2d(const float *dev_X, const int64_t *dev_QW, const float *dev_ths,

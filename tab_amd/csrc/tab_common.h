@@ -193,6 +193,33 @@ __device__ __forceinline__ ConvArgs unpack_conv(const ConvParamsOf<PACKED> &k)
 int device_compute_units();
 void set_compute_units(int units);  // test hook of the rules that count them (0: the device's)
 
+// The convolution that keeps the input patch of a tile in LDS (tab_conv_mfma_patch.h) reads the weights in an order of its own, in
+// which the quantizer's launch leaves them in the caller's workspace (pack_weights, tab_patch_weights.h): its first `blocks`
+// workgroups do that.  out == null: no such weights wanted.
+struct WeightJob {
+    const uint64_t *qw;
+    uint64_t *out;
+    int KN;
+    uint32_t pc_taps;    // PC | KH * KW << 16
+    uint32_t blocks;
+    uint32_t kc_planes;  // words of a chunk | bit planes << 8
+};
+static_assert(sizeof(WeightJob) == 32, "quantizers take it beside at most 80 bytes of arguments");
+
+// A convolution's plan for that kernel: shape < 0 where another kernel takes it, of which `tiled` is the shape if it has been looked
+// up (else -1).
+struct PatchPlan {
+    int shape, kc, npix, lds_bytes, tiled;
+    size_t weight_bytes;
+};
+constexpr int kPatchShape = 12;  // shapes (of launch_conv_mfma) from here on are that kernel's
+// The plan of the automatic choice (or of the test hook's); fp32 output.
+PatchPlan conv_patch_plan(int type, const ConvArgs &args);
+// Bytes that hold the weights of any plan for these sizes.
+size_t patch_weight_bytes(int type, int C, int KN, int KH, int KW);
+WeightJob patch_weight_job(int type, const ConvArgs &args, const PatchPlan &plan, uint64_t *out);
+hipError_t launch_patch_weights(const WeightJob &job, hipStream_t stream);  // the job in a launch of its own
+
 // Launchers (tab_conv.hip / tab_quantize.hip); they enqueue on `stream` and return the
 // launch status.
 hipError_t launch_conv(int type, const ConvArgs &args, hipStream_t stream);
@@ -226,15 +253,16 @@ inline Thresholds given_thresholds(const float *ths) { return Thresholds{ths, 0.
 // output, one launch more)
 size_t quantize_count_workspace(int bitwidth, long items, long pixels_per_item, int C);
 hipError_t launch_quantize(const float *x, const Thresholds &ths, int bitwidth, long pixels_per_item,
-                           long items, int C, uint64_t *qx, int32_t *btn, int32_t *count_workspace, hipStream_t stream);
+                           long items, int C, uint64_t *qx, int32_t *btn, int32_t *count_workspace, hipStream_t stream,
+                           const WeightJob *weights = nullptr);  // weights: with btn == null only
 
 // The same quantizer reading x as [N][C][H*W] (the CPU path's input layout, TAB_CPU.cpp:20-206); output as above.
 hipError_t launch_quantize_nchw(const float *x, const Thresholds &ths, int bitwidth, int N, int C, long HW, uint64_t *qx,
-                                int32_t *btn, int32_t *count_workspace, hipStream_t stream);
+                                int32_t *btn, int32_t *count_workspace, hipStream_t stream, const WeightJob *weights = nullptr);
 
 // Packers of the CPU-only conv types: format 4 = DoReFa 2-bit levels, 5 = RTN fields.
 hipError_t launch_quantize_format(const float *x, const float *ths, int format, long pixels_per_item, long items, int C,
-                                  uint64_t *qx, hipStream_t stream);
+                                  uint64_t *qx, hipStream_t stream, const WeightJob *weights = nullptr);
 
 // Quantize only the pixels (oh*s1, ow*s2) of every image into a compact [N][OH][OW][PC] activation
 // (what a 1x1 convolution with stride and no padding reads).

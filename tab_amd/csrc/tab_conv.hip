@@ -13,8 +13,11 @@
 // one k-slice with 128-bit LDS reads (A reads broadcast over the 16 tx lanes, B reads are
 // 256 B contiguous per 16 lanes).  The inner loop is pure VALU: XOR/AND + v_bcnt_u32_b32
 // with the count accumulated in the instruction's addend.
+#include "tab_conv_patch.h"
+#include "tab_conv_patch_model.h"
 #include "tab_conv_shape_model.h"
 #include "tab_conv_stage.h"
+#include "tab_patch_weights.h"
 
 #include <atomic>
 
@@ -473,9 +476,78 @@ int conv_mfma_shape(int type, const ConvArgs &a, float *cost_us)
     return best;
 }
 
+// The kernel that keeps the input patch in LDS, against the tiled one that conv_mfma_shape picks: the shape with the lowest predicted
+// duration, if that is 7 % below what the tiled kernel is predicted to take (tab_conv_patch_model.h; both are linear forms with
+// non-negative coefficients, fitted to 1944 measured launches: over them the choices take 0.93 of the tiled kernels' time, the
+// better one of each 0.915).  Not for 1x1 kernels, which read every pixel for one tap only, nor for at most 32 filters, half of
+// whose tiles would be work for nothing, nor for launches below 128 tiles of 64x64, which last as long as one tile's chain of waits
+// (no win below 49 such tiles, one in eight from there to 120).  Measured, tiled / patch, conv kernel alone in the kernel trace:
+// N=64 14x14x256 levels 13.6 / 10.6 us, N=256 28x28x512->512 BNN 224 / 196, N=32 56x56x64 TNN 10.3 / 8.5.
+PatchPlan conv_patch_plan(int type, const ConvArgs &a)
+{
+    PatchPlan plan = {-1, 0, 0, 0, -1, 0};
+    const Forced forced = forced_kernel();
+    if (type > 4 || !conv_mfma_exact(a) || (type == 4 && !conv_mfma_exact_levels(a))) return plan;
+    int npix, lds_bytes;
+    auto weigh = [&](int shape, int kc) {
+        plan.shape = shape;
+        plan.kc = kc;
+        plan.npix = npix;
+        plan.lds_bytes = lds_bytes;
+        const long tiles = (a.KN + 31) / 32, pairs = (long)((a.PC + kc - 1) / kc) * patch_pairs(a.KH * a.KW, kc);
+        plan.weight_bytes = (size_t)(tiles * pairs) * 512 * (type == 0 || type == 2 || type == 4 ? 2 : 1);
+        return plan;
+    };
+    if (forced.tm == 9 && forced.ng >= kPatchShape) {  // the test hook
+        const int i = forced.ng - kPatchShape;
+        const int kc = i < kPatchShapes ? patch_chunk(a, kPatchTile[i].rows, patch_most_words(kPatchTile[i].wave_tiles), &npix, &lds_bytes) : 0;
+        return kc ? weigh(forced.ng, kc) : plan;
+    }
+    if (a.qy != nullptr || (forced.tm != 0 && !(forced.tm == 9 && forced.ng < 0))) return plan;
+    const long kn64 = ((long)a.KN + 63) / 64;
+    if (a.KH * a.KW == 1 || a.KN <= 32 || ((long)a.M + 63) / 64 * kn64 < 128) return plan;
+    float tiled_us = 0.f;
+    plan.tiled = conv_mfma_shape(type, a, &tiled_us);
+    float t[kTiledFeatures];
+    tiled_features(a, tiled_us, t);
+    float limit = 0.f;
+    for (int k = 0; k < kTiledFeatures; k++) limit += kTiledCost[type][k] * t[k];
+    limit *= 0.93f;
+    const uint32_t cus = (uint32_t)device_compute_units();
+    for (int i = 0; i < kPatchShapes; i++) {
+        if (kPatchTile[i].filters >= 128 * kn64) continue;
+        const int kc = patch_chunk(a, kPatchTile[i].rows, patch_most_words(kPatchTile[i].wave_tiles), &npix, &lds_bytes);
+        if (kc == 0) continue;
+        float f[kPatchFeatures], us = 0.5f;  // the weights' part of the quantizer's launch (measured 0.1-0.8)
+        patch_features(a, i, kc, npix, lds_bytes, cus, f);
+        for (int k = 0; k < kPatchFeatures; k++) us += kPatchCost[type][i][k] * f[k];
+        if (us < limit) {
+            limit = us;
+            weigh(kPatchShape + i, kc);
+        }
+    }
+    return plan;
+}
+
+size_t patch_weight_bytes(int type, int C, int KN, int KH, int KW)
+{
+    if (type > 4 || KN <= 0) return 0;
+    const size_t PC = (size_t)(C + kWordBits - 1) / kWordBits, taps = (size_t)KH * KW;
+    // (of four words at most one is padding, of two taps one)
+    return ((size_t)KN + 31) / 32 * (((taps + 1) * (PC + 1) + 1) / 2) * 512 * (type == 0 || type == 2 || type == 4 ? 2 : 1);
+}
+
+WeightJob patch_weight_job(int type, const ConvArgs &a, const PatchPlan &plan, uint64_t *out)
+{
+    const int planes = type == 0 || type == 2 || type == 4 ? 2 : 1;
+    const long items = (long)(plan.weight_bytes / 8 / planes);  // 64 lanes a run
+    return WeightJob{a.qw, out, a.KN, (uint32_t)a.PC | (uint32_t)(a.KH * a.KW) << 16, (uint32_t)((items + 255) / 256), (uint32_t)plan.kc | (uint32_t)planes << 8};
+}
+
 hipError_t launch_conv(int type, const ConvArgs &args, hipStream_t stream)
 {
-    const Forced forced = forced_kernel();
+    Forced forced = forced_kernel();
+    if (forced.tm == 9 && forced.ng >= kPatchShape) forced.ng = -1;  // (the weights here are in their public order)
     const int force_tm = forced.tm, force_ng = forced.ng;
     if (args.qy != nullptr) {  // packed output exists in the matrix-core kernel's 64-wide shapes only
         if (!conv_mfma_exact(args)) return hipErrorInvalidValue;

@@ -613,6 +613,9 @@ template <int TYPE>
 hipError_t launch_mfma_tail(ConvArgs a, hipStream_t stream);
 template <int TYPE>
 hipError_t launch_mfma_tail_wide(ConvArgs a, hipStream_t stream);
+// Tiles whose input patch stays in LDS (tab_conv_mfma_patch.h).
+template <int TYPE, int WM, int WN, int TM, int TN>
+hipError_t launch_patch(const ConvArgs &a, hipStream_t stream);
 
 template <int TYPE, int WM, int WN, int TM, int TN, int KCH, int KS = 1>
 hipError_t launch_mfma_intap(const ConvArgs &a, hipStream_t stream)
@@ -666,7 +669,8 @@ hipError_t launch_mfma_regs(const ConvArgs &a, hipStream_t stream);
 // split over two pairs of waves (each wave 2x4 MFMA tiles over half of every chunk); both need an even number of words per
 // pixel and otherwise run as shapes 2 and 0, 10 = 128x128 tiles for the whole rounds of the chip and 64x64 split-K quarters for
 // the rest of the last round (an even number of words per pixel; otherwise shape 0), 11 = the same with whole tiles of 128x256
-// (words per pixel in fours; otherwise shape 6)
+// (words per pixel in fours; otherwise shape 6); 12 .. 16 = the kernel that keeps the input patch in LDS, on weights laid out for
+// it (ConvArgs::qw then points to those): 256x128, 128x128, 128x64, 64x64, 256x64; refused where its patch does not fit
 template <int TYPE>
 hipError_t launch_mfma_type(const ConvArgs &a, int shape, hipStream_t stream)
 {
@@ -683,6 +687,18 @@ hipError_t launch_mfma_type(const ConvArgs &a, int shape, hipStream_t stream)
     if (shape == 10) {
         if (a.PC % 2 == 0) return launch_mfma_tail<TYPE>(a, stream);
         shape = 0;
+    }
+    if (shape >= kPatchShape) {
+        if constexpr (TYPE <= 4) {
+            switch (shape) {
+            case 12: return launch_patch<TYPE, 2, 2, 4, 2>(a, stream);
+            case 13: return launch_patch<TYPE, 1, 4, 4, 1>(a, stream);
+            case 14: return launch_patch<TYPE, 2, 2, 2, 1>(a, stream);
+            case 15: return launch_patch<TYPE, 2, 2, 1, 1>(a, stream);
+            case 16: return launch_patch<TYPE, 4, 1, 2, 2>(a, stream);
+            }
+        }
+        return hipErrorInvalidValue;
     }
     if (shape == 8 && a.PC % 2 != 0) shape = 2;
     if (shape == 9 && a.PC % 2 != 0) shape = 0;

@@ -575,4 +575,5 @@ hipError_t launch_mfma_narrow(const ConvArgs &a, hipStream_t stream)
 }  // namespace
 }  // namespace tab
 
+#include "tab_conv_mfma_patch.h"
 #include "tab_conv_mfma_regs.h"

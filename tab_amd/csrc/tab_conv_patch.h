@@ -1,0 +1,90 @@
+// Geometry of the convolution that keeps its input patch in LDS (tab_conv_mfma_patch.h), as the host counts it: what fits, and
+// in how many chunks.
+#pragma once
+#include "tab_common.h"
+
+namespace tab {
+
+template <int KC> constexpr int kPatchItems = KC == 4 ? 2 : 3;  // pixels of the patch a thread fetches at most, KC words of each
+constexpr int kPatchLdsBytes = 64 * 1024;                       // of a workgroup
+constexpr int kPatchThreads = 256;
+
+// Words of a chunk at most: waves of eight MFMA tiles have no registers for four.
+constexpr int patch_most_words(int tiles_per_wave) { return tiles_per_wave >= 8 ? 2 : 4; }
+
+// Pixels of the patch of `rows` consecutive output pixels at most, wherever they begin on a multiple of `rows` (a power of two);
+// kPatchPixels + 1 for any number above it.  (32-bit arithmetic: this runs in every call.)
+constexpr int kPatchPixels = kPatchItems<1> * kPatchThreads;
+inline int patch_pixels(const ConvArgs &a, int rows)
+{
+    const int64_t wide = (int64_t)(a.OW - 1) * a.s2 + a.KW;
+    if (wide > kPatchPixels || a.KH > kPatchPixels || a.s1 > kPatchPixels) return kPatchPixels + 1;
+    const int PW = (int)wide;
+    // output lines touched: the run may begin at any multiple of gcd(rows, OW) of a line
+    const int low = a.OW & -a.OW, g = low < rows ? low : rows;
+    const int lines_out = (a.OW - g + rows - 1) / a.OW + 1;
+    const int crossings = a.OH >= lines_out ? (lines_out > 1 ? 1 : 0) : (lines_out - 1 + a.OH - 1) / a.OH;  // from an image's last line to the next one's first
+    const int across = a.KH > a.s1 ? a.KH - a.s1 : 0;
+    const int lines = (lines_out - 1) * a.s1 + crossings * across + a.KH;
+    return lines > kPatchPixels || lines * PW > kPatchPixels ? kPatchPixels + 1 : lines * PW;
+}
+
+// Words of a chunk and bytes of LDS; 0 when the patch does not fit.
+inline int patch_chunk(const ConvArgs &a, int rows, int most, int *npix, int *lds_bytes)
+{
+    const int pixels = patch_pixels(a, rows);
+    if (pixels > kPatchPixels || (int64_t)(a.OH - 1) * a.s1 + a.KH + pixels >= 65536) return 0;
+    for (int kc = a.PC == 1 ? 1 : most; kc >= 1; kc >>= 1) {
+        // of four words at most one is padding, and of three words none
+        if ((kc == 4 && a.PC % 4 != 0 && a.PC % 4 != 3) || (kc == 2 && a.PC == 3)) continue;
+        const int planes = pixels + (kc == 1 ? 1 : 0);
+        const int bytes = planes * 32 * kc * (a.PC > kc ? 2 : 1);
+        if (bytes > kPatchLdsBytes || (kc == 4 && pixels > kPatchItems<4> * kPatchThreads)) continue;
+        *npix = planes;
+        *lds_bytes = bytes < 4096 ? 4096 : bytes;
+        return kc;
+    }
+    return 0;
+}
+
+// The kernel's shapes: rows and filters of a workgroup's tile, MFMA tiles of a wave, workgroups a CU holds by their registers.
+struct PatchTile { int rows, filters, wave_tiles, held; };
+constexpr int kPatchShapes = 5;
+constexpr PatchTile kPatchTile[kPatchShapes] = {{256, 128, 8, 2}, {128, 128, 4, 3}, {128, 64, 2, 4}, {64, 64, 1, 4}, {256, 64, 4, 3}};
+
+// What the predicted durations (tab_conv_patch_model.h) are linear in; the fit script states the same.
+constexpr int kPatchFeatures = 13, kTiledFeatures = 10;
+
+// A launch of shape i: the busiest CU holds n tiles in so many rounds; its loop, its patches, its chunks and its output.
+inline void patch_features(const ConvArgs &a, int i, int kc, int npix, int lds_bytes, uint32_t cus, float (&f)[kPatchFeatures])
+{
+    const PatchTile &tile = kPatchTile[i];
+    const int taps = a.KH * a.KW;
+    const float chunks = (float)((a.PC + kc - 1) / kc);
+    const float K = chunks * (float)(kc == 1 ? (taps + 1) / 2 * 2 : taps * kc);  // words multiplied
+    const uint32_t tiles_m = ((uint32_t)a.M + (uint32_t)tile.rows - 1) / (uint32_t)tile.rows, tiles_n = ((uint32_t)a.KN + (uint32_t)tile.filters - 1) / (uint32_t)tile.filters;
+    const uint64_t tiles = (uint64_t)tiles_m * tiles_n;
+    const int by_lds = 160 * 1024 / lds_bytes, held = tile.held < by_lds ? tile.held : by_lds;
+    const uint64_t busiest = tiles <= 0xffffffffu ? ((uint32_t)tiles + cus - 1) / cus : (tiles + cus - 1) / cus;
+    const float n = (float)busiest, rounds = (float)((busiest + (uint32_t)held - 1) / (uint32_t)held);
+    const float busy = tiles < cus ? (float)tiles / (float)cus : 1.f;
+    const float y_mb = (float)a.M * (float)a.KN * 4e-6f;
+    const float patch = (float)npix * (float)kc * chunks * 1e-3f;  // words expanded a tile
+    const float values[kPatchFeatures] = {1.f, busy, K * n, K * rounds, n, rounds, y_mb, y_mb * busy, patch * n, patch * rounds, chunks * rounds,
+                                          (float)tiles / (float)cus, a.KN % 32 ? y_mb : 0.f};
+    for (int k = 0; k < kPatchFeatures; k++) f[k] = values[k];
+}
+
+// The tiled kernel that conv_mfma_shape picks, which predicts `us` for it: that prediction was fitted to even words per pixel, whole
+// lines of Y and launches like the benchmark's.
+inline void tiled_features(const ConvArgs &a, float us, float (&f)[kTiledFeatures])
+{
+    const float G = (float)a.G, y_mb = (float)a.M * (float)a.KN * 4e-6f;
+    const float products = (float)a.M * (float)((a.KN + 63) / 64 * 64) * G * 1e-9f;
+    const bool odd = a.PC % 2 != 0;
+    const float values[kTiledFeatures] = {1.f, us, y_mb, products, odd ? products : 0.f, odd ? us : 0.f, 0.1f * G, odd ? 0.1f * G : 0.f,
+                                          (float)a.M * G * 1e-6f, a.KN % 32 ? y_mb : 0.f};
+    for (int k = 0; k < kTiledFeatures; k++) f[k] = values[k];
+}
+
+}  // namespace tab

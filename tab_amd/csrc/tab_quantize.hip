@@ -8,13 +8,14 @@
 // word r (C % 64 == 0) so the whole op is one streaming pass: 256 B in, 8 or 16 B out.
 #include "tab_conv_stage.h"
 #include "tab_pack.h"
+#include "tab_quantize_rows.h"
+#include "tab_patch_weights.h"
 
 namespace tab {
 namespace {
 
 constexpr int kThreads = 256;
 constexpr int kWavesPerBlock = kThreads / 64;
-constexpr int kLoadsPerLane = 8;                // float4 loads in flight per lane
 constexpr int kRowsPerWave = 4 * kLoadsPerLane; // each wave-wide float4 load covers 4 rows
 constexpr long kSmallLaunchBlocks = 512;        // at or below this many 128-row workgroups a launch is latency-bound
 
@@ -81,69 +82,25 @@ __global__ __launch_bounds__(kThreads) void count_finish(const int32_t *__restri
     store_count<kWavesPerBlock>(count, btn + blockIdx.x, scratch);
 }
 
-// Fast path, C % 64 == 0 and X 16-byte aligned.
-// Lane layout: a 16-lane DPP row reads one 64-channel row as 16 float4 (256 B contiguous),
-// a wave reads 4 consecutive rows per load (1 KB contiguous) and keeps kLoadsPerLane loads
-// in flight; pack_row turns the compare bits of the row's lanes into its packed element.
-// BITS = 1 or 2 (the reference's bit widths), or the format of conv type 4 or 5; LOADS = 8 (128 rows per
-// workgroup) for streaming, 2 for launches too small to fill the chip.
+// The streaming path (tab_quantize_rows.h).
 template <int BITS, int LOADS = kLoadsPerLane>
-__global__ __launch_bounds__(kThreads) void quantize_rows64(const floatx4 *__restrict__ x,
-                                                            const Thresholds ths,
-                                                            uint32_t *__restrict__ q, long rows,
+__global__ __launch_bounds__(kThreads) void quantize_rows64(const floatx4 *__restrict__ x, const Thresholds ths, uint32_t *__restrict__ q, long rows,
                                                             long rows_per_item, Div32 div_item, int32_t *btn, long items)
 {
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // scalar: so are row0 and the item test below
-    const int sub = lane >> 4;  // which of the 4 rows of a load
-    const int l = lane & 15;    // float4 within the row
-    const long row0 = ((long)blockIdx.x * kWavesPerBlock + wave) * (4 * LOADS);
-    if (row0 >= rows) return;
-    long row_last = row0 + (4 * LOADS) - 1;
-    if (row_last > rows - 1) row_last = rows - 1;
+    quantize_rows64_block<BITS, LOADS>(x, ths, q, rows, rows_per_item, div_item, blockIdx.x);
+    const long row = (long)blockIdx.x * (4 * LOADS * kWavesPerBlock) + (threadIdx.x >> 6) * (4 * LOADS) + (threadIdx.x & 63);
+    if ((threadIdx.x & 63) < 4 * LOADS) zero_counts(btn, items, row);
+}
 
-    floatx4 v[LOADS];
-#pragma unroll
-    for (int u = 0; u < LOADS; u++) {
-        const long r = row0 + u * 4 + sub;
-        // rows past the end read the last row again (not stored): straight-line loads, no branch per load
-        const floatx4 *src = &x[(r < rows ? r : rows - 1) * 16 + l];
-        // a small tensor is likely to sit in the caches (it was just written, or is read again): plain loads;
-        // a large one streams past them: non-temporal loads (plain ones are 8-11 % slower at 400 MB and more)
-        v[u] = LOADS == 2 ? *src : __builtin_nontemporal_load(src);
-    }
-
-    // The wave's items (scalar; div_item.mul == 0 says that rows reach 2^31 and the division takes 64 bits): with the
-    // short division the threshold is in flight together with the loads of x instead of behind a long one.
-    const long item_first = div_item.mul ? (long)div32((uint32_t)row0, div_item) : row0 / rows_per_item;
-    const long item_last = div_item.mul ? (long)div32((uint32_t)row_last, div_item) : row_last / rows_per_item;
-    const bool one_item = item_last == item_first;
-    const float t_first = wave_threshold(ths, item_first);
-
-    auto finish = [&](int u, float t) {
-        const long r = row0 + u * 4 + sub;
-        uint32_t sign, nz, out[4];
-        compare4<BITS>(v[u], t, sign, nz);
-        pack_row<BITS>(sign, nz, l, out);  // lane 0 stores the whole element (8 or 16 bytes) at once
-        if (BITS != 1) {
-            if (r < rows && l == 0) *reinterpret_cast<uintx4 *>(q + r * 4) = uintx4{out[0], out[1], out[2], out[3]};
-        } else {
-            if (r < rows && l == 0) *reinterpret_cast<uintx2 *>(q + r * 2) = uintx2{out[0], out[1]};
-        }
-    };
-    // two copies of the loop under a scalar branch: the common one has no load but x in flight, so each load is
-    // waited for on its own
-    if (one_item) {
-#pragma unroll
-        for (int u = 0; u < LOADS; u++) finish(u, t_first);
-    } else {
-#pragma unroll
-        for (int u = 0; u < LOADS; u++) {
-            const long r = row0 + u * 4 + sub;
-            finish(u, lane_threshold(ths, (r < rows ? r : rows - 1) / rows_per_item));
-        }
-    }
-    if (lane < 4 * LOADS) zero_counts(btn, items, row0 + lane);
+// Beside a convolution's weights, which the first workgroups lay out (kernels of their own: with the code for the weights in every
+// quantizer the short ones took 2-4 % longer).
+template <int BITS, int LOADS = kLoadsPerLane>
+__global__ __launch_bounds__(kThreads) void quantize_rows64_weights(const floatx4 *__restrict__ x, const Thresholds ths, uint32_t *__restrict__ q,
+                                                                    long rows, long rows_per_item, Div32 div_item, const WeightJob job)
+{
+    uint32_t block = blockIdx.x;
+    if (pack_weights(job, block)) return;
+    quantize_rows64_block<BITS, LOADS>(x, ths, q, rows, rows_per_item, div_item, block);
 }
 
 // The same row quantizer for a 1x1 convolution with stride and no padding, which reads only the
@@ -221,6 +178,13 @@ __global__ __launch_bounds__(kThreads) void quantize_rows64_count(const floatx4 
         }
     }
     store_count<kWavesPerBlock>(count, counts.out + blockIdx.x, scratch);
+}
+
+// A convolution's weights alone.
+__global__ __launch_bounds__(kThreads) void patch_weights(const WeightJob job)
+{
+    uint32_t block = blockIdx.x;
+    pack_weights(job, block);
 }
 
 // General path: any C, any alignment of x, every format (MODE as in compare4).  A workgroup takes a tile of consecutive pixels,
@@ -353,6 +317,20 @@ __global__ __launch_bounds__(kThreads) void quantize_tile(const float *__restric
     const int live = pixels - p0 < tile_pixels ? (int)(pixels - p0) : tile_pixels;  // pixels of the tile that exist
     quantize_one_tile<MODE, LP>(x, ths, q, p0, live, pixels_per_item, div_item, C, tile_pixels, blockIdx.y * words, words);
     for (int i = threadIdx.x; i < live; i += kThreads) zero_counts(btn, items, p0 + i);
+}
+
+// Without counts, beside a convolution's weights.
+template <int MODE, int LP>
+__global__ __launch_bounds__(kThreads) void quantize_tile_weights(const float *__restrict__ x, const Thresholds ths, uint64_t *__restrict__ q,
+                                                                  long pixels, long pixels_per_item, Div32 div_item, int C, int tile_pixels,
+                                                                  int words, const WeightJob job)
+{
+    uint32_t block = blockIdx.x;
+    if (blockIdx.y != 0 && block < job.blocks) return;  // (the grid's other parts of a pixel)
+    if (pack_weights(job, block)) return;
+    const long p0 = (long)block * tile_pixels;
+    const int live = pixels - p0 < tile_pixels ? (int)(pixels - p0) : tile_pixels;  // pixels of the tile that exist
+    quantize_one_tile<MODE, LP>(x, ths, q, p0, live, pixels_per_item, div_item, C, tile_pixels, blockIdx.y * words, words);
 }
 
 // The same with counts (see Counts); a unit is a tile of whole pixels.
@@ -555,6 +533,18 @@ __global__ __launch_bounds__(kThreads) void quantize_nchw(const float *__restric
     if (wave % SPLIT == 0) zero_counts(btn, N, run.pixel, VEC);
 }
 
+// Beside a convolution's weights.
+template <int BITS, int VEC, int SPLIT, bool NT = false>
+__global__ __launch_bounds__(kThreads) void quantize_nchw_weights(const float *__restrict__ x, const Thresholds ths, uint64_t *__restrict__ q, int N,
+                                                                  int C, long HW, int PC, const WeightJob job)
+{
+    uint32_t block = blockIdx.x;
+    if (pack_weights(job, block)) return;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const PixelRun<VEC> run((block / PC * (kWavesPerBlock / SPLIT) + wave / SPLIT) * 64L + (threadIdx.x & 63), N, HW);
+    quantize_nchw_unit<BITS, VEC, SPLIT, NT>(x, ths, q, run, C, HW, PC, block % PC);
+}
+
 // The same with counts: a unit is 64 * 4 / SPLIT runs and one word.
 template <int VEC, int SPLIT, bool NT = false>
 __global__ __launch_bounds__(kThreads) void quantize_nchw_count(const float *__restrict__ x, const Thresholds ths, uint64_t *__restrict__ q, int C,
@@ -584,9 +574,11 @@ __global__ __launch_bounds__(kThreads) void quantize_nchw_count(const float *__r
 // in WPP / 2 rounds of 64 / rounds lanes each.  grid = ceil(runs / 64) * (PC / U), the word group fastest.
 // Bits are made by the form and in as many registers as measured best: SHIFT for U = 2.
 // COUNT: a wave is a slice of one unit (see Counts).
-template <int BITS, int U, bool EVEN, bool COUNT = false>
+// WEIGHTS: a convolution's weights beside (then without counts).
+template <int BITS, int U, bool EVEN, bool COUNT = false, bool WEIGHTS = false>
 __global__ __launch_bounds__(64, BITS == 1 ? (U == 4 ? 4 : 7) : (U == 4 ? 1 : 4)) void quantize_nchw_gather(const float *__restrict__ x, const Thresholds ths,
-                                                                 uint64_t *__restrict__ q, int N, int C, long HW, int PC, int32_t *btn)
+                                                                 uint64_t *__restrict__ q, int N, int C, long HW, int PC,
+                                                                 typename std::conditional<WEIGHTS, WeightJob, int32_t *>::type extra)
 {
     static_assert(!COUNT || (BITS == 2 && !EVEN), "counts of two planes; runs of one image are numbered for any plane size");
     constexpr int VEC = 4, kInFlight = 8;
@@ -596,10 +588,15 @@ __global__ __launch_bounds__(64, BITS == 1 ? (U == 4 ? 4 : 7) : (U == 4 ? 1 : 4)
     constexpr bool SHIFT = U == 2;
     static_assert(U == 2 || U == 4, "one word per thread is quantize_nchw");
     __shared__ __attribute__((aligned(16))) uint64_t stage[512];
+    uint32_t block = blockIdx.x;
+    if constexpr (WEIGHTS)
+        if (pack_weights(extra, block)) return;
+    int32_t *btn = nullptr;
+    if constexpr (!WEIGHTS) btn = extra;
     const int groups = PC / U;
     // COUNT: N is the number of slices of an image
-    const int image = COUNT ? (int)(blockIdx.x / (uint32_t)N) : 0;
-    const int unit = (int)blockIdx.x - image * N * COUNT;
+    const int image = COUNT ? (int)(block / (uint32_t)N) : 0;
+    const int unit = (int)block - image * N * COUNT;
     const int pc0 = (unit % groups) * U;
     const int lane = threadIdx.x;
     const PixelRun<VEC, EVEN> run = COUNT ? PixelRun<VEC, EVEN>((long)(unit / groups) * 64 + lane, image, HW, std::true_type())
@@ -899,7 +896,7 @@ void finish_counts(const CountTarget &target, long items, int slices, hipStream_
 
 template <int MODE, int LP>
 void launch_quantize_tile_of(const float *x, const Thresholds &ths, long pixels, long pixels_per_item, long items, int C, uint64_t *q,
-                             int32_t *btn, const CountTarget *counted, hipStream_t stream)
+                             int32_t *btn, const CountTarget *counted, const WeightJob *weights, hipStream_t stream)
 {
     // Bytes of x in a tile, measured from 4 to 48 KB on C = 3 ... 700: what a few workgroups a CU keep in flight against the
     // wait of each for its whole tile.  The pixels are shared by four waves in turns of U reads, so sixteen (a turn of four
@@ -926,19 +923,24 @@ void launch_quantize_tile_of(const float *x, const Thresholds &ths, long pixels,
         }
     }
     const dim3 grid((unsigned)((pixels + tile_pixels - 1) / tile_pixels), (unsigned)((PC + words - 1) / words));
+    if (weights) {
+        quantize_tile_weights<MODE, LP><<<dim3(grid.x + weights->blocks, grid.y), dim3(kThreads), lds, stream>>>(
+            x, ths, q, pixels, pixels_per_item, div_item, C, (int)tile_pixels, words, *weights);
+        return;
+    }
     quantize_tile<MODE, LP><<<grid, dim3(kThreads), lds, stream>>>(x, ths, q, pixels, pixels_per_item, div_item, C, (int)tile_pixels, words, btn, items);
 }
 
 // The general path with the fewest lanes a word that hold it.
 template <int MODE>
 void launch_quantize_tile(const float *x, const Thresholds &ths, long pixels, long pixels_per_item, long items, int C, uint64_t *q,
-                          int32_t *btn, const CountTarget *counted, hipStream_t stream)
+                          int32_t *btn, const CountTarget *counted, const WeightJob *weights, hipStream_t stream)
 {
-    if (C <= 4) launch_quantize_tile_of<MODE, 4>(x, ths, pixels, pixels_per_item, items, C, q, btn, counted, stream);
-    else if (C <= 8) launch_quantize_tile_of<MODE, 8>(x, ths, pixels, pixels_per_item, items, C, q, btn, counted, stream);
-    else if (C <= 16) launch_quantize_tile_of<MODE, 16>(x, ths, pixels, pixels_per_item, items, C, q, btn, counted, stream);
-    else if (C <= 32) launch_quantize_tile_of<MODE, 32>(x, ths, pixels, pixels_per_item, items, C, q, btn, counted, stream);
-    else launch_quantize_tile_of<MODE, 64>(x, ths, pixels, pixels_per_item, items, C, q, btn, counted, stream);
+    if (C <= 4) launch_quantize_tile_of<MODE, 4>(x, ths, pixels, pixels_per_item, items, C, q, btn, counted, weights, stream);
+    else if (C <= 8) launch_quantize_tile_of<MODE, 8>(x, ths, pixels, pixels_per_item, items, C, q, btn, counted, weights, stream);
+    else if (C <= 16) launch_quantize_tile_of<MODE, 16>(x, ths, pixels, pixels_per_item, items, C, q, btn, counted, weights, stream);
+    else if (C <= 32) launch_quantize_tile_of<MODE, 32>(x, ths, pixels, pixels_per_item, items, C, q, btn, counted, weights, stream);
+    else launch_quantize_tile_of<MODE, 64>(x, ths, pixels, pixels_per_item, items, C, q, btn, counted, weights, stream);
 }
 
 // Counts of every two-plane quantizer in slices: workspace ints at most (a unit holds at least four words).
@@ -949,10 +951,24 @@ size_t quantize_count_workspace(int bitwidth, long items, long pixels_per_item, 
     return (size_t)items * (pixels_per_item * PC / 4 + PC + 1) * sizeof(int32_t);
 }
 
+hipError_t launch_rows64_weights(const float *x, const Thresholds &ths, int format, long rows, long rows_per_item, Div32 div_item, uint64_t *qx,
+                                 const WeightJob &job, hipStream_t stream)
+{
+    auto launch = [&](auto kernel, long rows_per_block) {
+        kernel<<<dim3((unsigned)((rows + rows_per_block - 1) / rows_per_block) + job.blocks), dim3(kThreads), 0, stream>>>(
+            reinterpret_cast<const floatx4 *>(x), ths, reinterpret_cast<uint32_t *>(qx), rows, rows_per_item, div_item, job);
+    };
+    // (sizes of workgroups as in launch_quantize)
+    if (rows <= kSmallLaunchBlocks * 128) launch(format == 4 ? quantize_rows64_weights<4, 2> : format == 2 ? quantize_rows64_weights<2, 2> : quantize_rows64_weights<1, 2>, 32);
+    else launch(format == 4 ? quantize_rows64_weights<4> : format == 2 ? quantize_rows64_weights<2> : quantize_rows64_weights<1>, 128);
+    return hipGetLastError();
+}
+
 // x: fp32 [items][pixels_per_item][C]; qx: [items*pixels_per_item][PC][bitwidth];
 // btn: [items] or nullptr (then no counts are produced).
 hipError_t launch_quantize(const float *x, const Thresholds &ths, int bitwidth, long pixels_per_item,
-                           long items, int C, uint64_t *qx, int32_t *btn, int32_t *count_workspace, hipStream_t stream)
+                           long items, int C, uint64_t *qx, int32_t *btn, int32_t *count_workspace, hipStream_t stream,
+                           const WeightJob *weights)
 {
     const int PC = (C + kWordBits - 1) / kWordBits;
     const long pixels = items * pixels_per_item;
@@ -980,7 +996,7 @@ hipError_t launch_quantize(const float *x, const Thresholds &ths, int bitwidth, 
         return hipGetLastError();
     }
     if (counted && C <= 3072) {
-        launch_quantize_tile<2>(x, ths, pixels, pixels_per_item, items, C, qx, nullptr, &target, stream);
+        launch_quantize_tile<2>(x, ths, pixels, pixels_per_item, items, C, qx, nullptr, &target, nullptr, stream);
         return hipGetLastError();
     }
     if (fast) {
@@ -990,6 +1006,7 @@ hipError_t launch_quantize(const float *x, const Thresholds &ths, int bitwidth, 
         const dim3 block(kThreads);
         const floatx4 *x4 = reinterpret_cast<const floatx4 *>(x);
         uint32_t *q32 = reinterpret_cast<uint32_t *>(qx);
+        if (weights) return launch_rows64_weights(x, ths, bitwidth, rows, words_per_item, div_item, qx, *weights, stream);
         if (blocks <= kSmallLaunchBlocks) {
             // a tensor too small to fill the chip with 128-row workgroups: 32 rows per workgroup, two loads per lane
             // (3.1 MB of fp32: 5.5 -> 4.2 us)
@@ -1006,16 +1023,22 @@ hipError_t launch_quantize(const float *x, const Thresholds &ths, int bitwidth, 
                 quantize_rows64<1><<<grid, block, 0, stream>>>(x4, ths, q32, rows, words_per_item, div_item, zeroed, items);
         }
     } else if (bitwidth == 2) {
-        launch_quantize_tile<2>(x, ths, pixels, pixels_per_item, items, C, qx, zeroed, nullptr, stream);
+        launch_quantize_tile<2>(x, ths, pixels, pixels_per_item, items, C, qx, zeroed, nullptr, weights, stream);
     } else {
-        launch_quantize_tile<1>(x, ths, pixels, pixels_per_item, items, C, qx, zeroed, nullptr, stream);
+        launch_quantize_tile<1>(x, ths, pixels, pixels_per_item, items, C, qx, zeroed, nullptr, weights, stream);
     }
     if (btn && bitwidth == 2) launch_btn_popcount(qx, btn, items, words_per_item, splits, stream);
     return hipGetLastError();
 }
 
+hipError_t launch_patch_weights(const WeightJob &job, hipStream_t stream)
+{
+    patch_weights<<<dim3(job.blocks), dim3(kThreads), 0, stream>>>(job);
+    return hipGetLastError();
+}
+
 hipError_t launch_quantize_nchw(const float *x, const Thresholds &ths, int bitwidth, int N, int C, long HW, uint64_t *qx,
-                                int32_t *btn, int32_t *count_workspace, hipStream_t stream)
+                                int32_t *btn, int32_t *count_workspace, hipStream_t stream, const WeightJob *weights)
 {
     const int PC = (C + kWordBits - 1) / kWordBits;
     const long words_per_item = HW * PC;
@@ -1027,6 +1050,11 @@ hipError_t launch_quantize_nchw(const float *x, const Thresholds &ths, int bitwi
                          N * (HW / 4 + 1) * PC < 0x7fffffffL;
     auto launch = [&](auto kernel, long blocks, int threads) {
         kernel<<<dim3((unsigned)blocks), dim3(threads), 0, stream>>>(x, ths, qx, N, C, HW, PC, zeroed);
+    };
+    auto launch_weights = [&](auto kernel, long blocks, int threads) {
+        WeightJob job = *weights;
+        job.blocks *= kThreads / threads;
+        kernel<<<dim3((unsigned)blocks + job.blocks), dim3(threads), 0, stream>>>(x, ths, qx, N, C, HW, PC, job);
     };
     // PC even, enough pixels for a wave on every SIMD: the form that gathers each wave's output into whole runs
     const int unit = PC % 4 == 0 ? 4 : PC % 2 == 0 ? 2 : 1;
@@ -1043,10 +1071,18 @@ hipError_t launch_quantize_nchw(const float *x, const Thresholds &ths, int bitwi
             finish_counts(CountTarget{btn, count_workspace}, N, (int)slices, stream);
             return hipGetLastError();
         }
-        if (unit == 4 && bitwidth == 2) launch(HW % 4 ? quantize_nchw_gather<2, 4, false> : quantize_nchw_gather<2, 4, true>, gather_waves, 64);
-        else if (unit == 4) launch(HW % 4 ? quantize_nchw_gather<1, 4, false> : quantize_nchw_gather<1, 4, true>, gather_waves, 64);
-        else if (bitwidth == 2) launch(HW % 4 ? quantize_nchw_gather<2, 2, false> : quantize_nchw_gather<2, 2, true>, gather_waves, 64);
-        else launch(HW % 4 ? quantize_nchw_gather<1, 2, false> : quantize_nchw_gather<1, 2, true>, gather_waves, 64);
+        auto pick = [&](auto even, auto any, auto even_weights, auto any_weights) {
+            if (weights) launch_weights(HW % 4 ? any_weights : even_weights, gather_waves, 64);
+            else launch(HW % 4 ? any : even, gather_waves, 64);
+        };
+        if (unit == 4 && bitwidth == 2)
+            pick(quantize_nchw_gather<2, 4, true>, quantize_nchw_gather<2, 4, false>, quantize_nchw_gather<2, 4, true, false, true>, quantize_nchw_gather<2, 4, false, false, true>);
+        else if (unit == 4)
+            pick(quantize_nchw_gather<1, 4, true>, quantize_nchw_gather<1, 4, false>, quantize_nchw_gather<1, 4, true, false, true>, quantize_nchw_gather<1, 4, false, false, true>);
+        else if (bitwidth == 2)
+            pick(quantize_nchw_gather<2, 2, true>, quantize_nchw_gather<2, 2, false>, quantize_nchw_gather<2, 2, true, false, true>, quantize_nchw_gather<2, 2, false, false, true>);
+        else
+            pick(quantize_nchw_gather<1, 2, true>, quantize_nchw_gather<1, 2, false>, quantize_nchw_gather<1, 2, true, false, true>, quantize_nchw_gather<1, 2, false, false, true>);
     } else {
         // waves per word: as many as it has parts of 16 channels
         const int split = C <= 16 ? 1 : C <= 32 ? 2 : 4;
@@ -1077,21 +1113,28 @@ hipError_t launch_quantize_nchw(const float *x, const Thresholds &ths, int bitwi
         }
         const long blocks = ((four ? runs : pixels) + 64 * groups - 1) / (64 * groups) * PC;
         if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
-        auto pick = [&](auto one, auto two) { launch(bitwidth == 2 ? two : one, blocks, kThreads); };
-        if (stream_past) pick(quantize_nchw<1, 4, 4, true>, quantize_nchw<2, 4, 4, true>);
-        else if (four && split == 4) pick(quantize_nchw<1, 4, 4>, quantize_nchw<2, 4, 4>);
-        else if (four && split == 2) pick(quantize_nchw<1, 4, 2>, quantize_nchw<2, 4, 2>);
-        else if (four) pick(quantize_nchw<1, 4, 1>, quantize_nchw<2, 4, 1>);
-        else if (split == 4) pick(quantize_nchw<1, 1, 4>, quantize_nchw<2, 1, 4>);
-        else if (split == 2) pick(quantize_nchw<1, 1, 2>, quantize_nchw<2, 1, 2>);
-        else pick(quantize_nchw<1, 1, 1>, quantize_nchw<2, 1, 1>);
+        auto form = [&](auto vec, auto parts, auto past) {
+            constexpr int VEC = decltype(vec)::value, PARTS = decltype(parts)::value;
+            constexpr bool PAST = decltype(past)::value;
+            if (weights) launch_weights(bitwidth == 2 ? quantize_nchw_weights<2, VEC, PARTS, PAST> : quantize_nchw_weights<1, VEC, PARTS, PAST>, blocks, kThreads);
+            else launch(bitwidth == 2 ? quantize_nchw<2, VEC, PARTS, PAST> : quantize_nchw<1, VEC, PARTS, PAST>, blocks, kThreads);
+        };
+        using std::integral_constant;
+        auto parts = [&](auto vec) {
+            if (split == 4) form(vec, integral_constant<int, 4>(), std::false_type());
+            else if (split == 2) form(vec, integral_constant<int, 2>(), std::false_type());
+            else form(vec, integral_constant<int, 1>(), std::false_type());
+        };
+        if (stream_past) form(integral_constant<int, 4>(), integral_constant<int, 4>(), std::true_type());
+        else if (four) parts(integral_constant<int, 4>());
+        else parts(integral_constant<int, 1>());
     }
     if (btn && bitwidth == 2) launch_btn_popcount(qx, btn, N, words_per_item, splits, stream);
     return hipGetLastError();
 }
 
 hipError_t launch_quantize_format(const float *x, const float *ths_values, int format, long pixels_per_item, long items, int C,
-                                  uint64_t *qx, hipStream_t stream)
+                                  uint64_t *qx, hipStream_t stream, const WeightJob *weights)
 {
     const Thresholds ths = given_thresholds(ths_values);
     const long pixels = items * pixels_per_item;
@@ -1105,6 +1148,7 @@ hipError_t launch_quantize_format(const float *x, const float *ths_values, int f
         uint32_t *q32 = reinterpret_cast<uint32_t *>(qx);
         const long rows_per_item = pixels_per_item * (C / kWordBits);
         const Div32 div_item = rows < 0x7fffffffL ? make_div32((uint32_t)rows_per_item) : Div32{0, 0};
+        if (weights && format == 4) return launch_rows64_weights(x, ths, format, rows, rows_per_item, div_item, qx, *weights, stream);
         if (blocks <= kSmallLaunchBlocks) {  // too small to fill the chip: 32 rows per workgroup, as in launch_quantize
             const dim3 small((unsigned)((rows + 8 * kWavesPerBlock - 1) / (8 * kWavesPerBlock)));
             if (format == 4)
@@ -1118,8 +1162,8 @@ hipError_t launch_quantize_format(const float *x, const float *ths_values, int f
         }
         return hipGetLastError();
     }
-    if (format == 4) launch_quantize_tile<4>(x, ths, pixels, pixels_per_item, items, C, qx, nullptr, nullptr, stream);
-    else launch_quantize_tile<5>(x, ths, pixels, pixels_per_item, items, C, qx, nullptr, nullptr, stream);
+    if (format == 4) launch_quantize_tile<4>(x, ths, pixels, pixels_per_item, items, C, qx, nullptr, nullptr, weights, stream);
+    else launch_quantize_tile<5>(x, ths, pixels, pixels_per_item, items, C, qx, nullptr, nullptr, weights, stream);
     return hipGetLastError();
 }
 

@@ -169,7 +169,7 @@ torch::Tensor TAB_Conv2d(const torch::Tensor &X, const torch::Tensor &QW, const 
     const auto [OH, OW] = check_conv_from_floats(X, QW, thresholds, btn, type, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW);
     const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(X.device());
     auto Y = device_empty({N, KN, OH, OW}, torch::kFloat32, X);
-    const size_t ws_bytes = tab_conv2d_workspace_bytes(type, N, H, W, C);
+    const size_t ws_bytes = tab_conv2d_workspace_bytes_full(type, N, H, W, C, KN, KH, KW);
     const hipStream_t stream = current_stream(X);
     const Workspace ws(ws_bytes, stream);
     check_status(tab_conv2d(X.data_ptr<float>(), QW.data_ptr<int64_t>(), thresholds.data_ptr<float>(),
@@ -453,7 +453,7 @@ torch::Tensor layer_output(const torch::Tensor &X, bool nchw, int64_t N, int64_t
 void run_layer(const Layer &l, const torch::Tensor &X, bool nchw, int N, int H, int W, const torch::Tensor &y)
 {
     const hipStream_t stream = current_stream(X);
-    const size_t ws_bytes = tab_layer_workspace_bytes(l.act_bits(), N, H, W, l.C);
+    const size_t ws_bytes = tab_layer_workspace_bytes_full(l.type, N, H, W, l.C, l.KN, l.KH, l.KW);
     const Workspace ws(ws_bytes, stream);
     check_status(tab_layer_conv2d(X.data_ptr<float>(), nchw, (float)l.act_scale, l.QW.data_ptr<int64_t>(), l.btn.data_ptr<int32_t>(),
                                   l.type, l.p1, l.p2, l.s1, l.s2, N, H, W, l.C, l.KN, l.KH, l.KW, y.data_ptr<float>(), ws.get(),

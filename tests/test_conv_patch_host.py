@@ -1,0 +1,95 @@
+"""The convolution that keeps its input patch in LDS, host side: the patch the plan allots holds what every tile of the launch reads
+(by brute force over the tiles), the workspace's room holds the weights of every plan, and the rule that takes a call there, on its
+measured launches, is within what its comment states."""
+import ctypes
+import importlib.util
+import os
+import random
+
+import numpy as np
+import pytest
+
+from tab_amd import _capi
+
+TUNING = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "tab_amd", "tuning")
+ROWS = {12: 256, 13: 128, 14: 128, 15: 64, 16: 256}
+
+
+@pytest.fixture(scope="module")
+def lib():
+    lib = ctypes.CDLL(_capi.LIB_PATH)
+    lib.tab_internal_conv_patch_shape.argtypes = [ctypes.c_int] * 12 + [ctypes.POINTER(ctypes.c_int), ctypes.POINTER(ctypes.c_size_t)]
+    for f in (lib.tab_conv2d_workspace_bytes_full, lib.tab_conv2d_workspace_bytes, lib.tab_layer_workspace_bytes_full, lib.tab_layer_workspace_bytes):
+        f.restype = ctypes.c_size_t
+    yield lib
+    lib.tab_set_conv_kernel(0, -1)
+
+
+def plan(lib, type, p1, p2, s1, s2, N, H, W, C, KN, KH, KW):
+    what, size = (ctypes.c_int * 3)(), ctypes.c_size_t()
+    shape = lib.tab_internal_conv_patch_shape(type, p1, p2, s1, s2, N, H, W, C, KN, KH, KW, what, ctypes.byref(size))
+    return shape, what[0], what[1], what[2], size.value
+
+
+def test_every_tile_fits_its_patch_and_every_plan_its_room(lib):
+    rng, planned = random.Random(3), 0
+    for _ in range(4000):
+        KH, KW, s1, s2 = rng.randint(1, 7), rng.randint(1, 7), rng.choice((1, 1, 2, 3, 9)), rng.choice((1, 1, 2, 3))
+        p1, p2 = rng.randint(0, KH), rng.randint(0, KW)
+        H, W = rng.randint(max(1, KH - 2 * p1), 40), rng.randint(max(1, KW - 2 * p2), 60)
+        N, C, KN, type = rng.randint(1, 12), rng.choice((3, 64, 100, 128, 192, 256, 320, 448, 512, 1000)), rng.randint(1, 300), rng.randint(0, 4)
+        OH, OW = (H + 2 * p1 - KH + 1) // s1, (W + 2 * p2 - KW + 1) // s2
+        if OH < 1 or OW < 1:
+            continue
+        shape = rng.choice(tuple(ROWS))
+        lib.tab_internal_force_patch(shape)
+        got, kc, npix, lds, weights = plan(lib, type, p1, p2, s1, s2, N, H, W, C, KN, KH, KW)
+        if got < 0:
+            continue
+        assert got == shape
+        planned += 1
+        PH, PW, PC = (OH - 1) * s1 + KH, (OW - 1) * s2 + KW, (C + 63) // 64
+        line = lambda m: m // (OH * OW) * PH + m % (OH * OW) // OW * s1  # noqa: E731
+        M, rows = N * OH * OW, ROWS[shape]
+        need = max((line(min(m0 + rows, M) - 1) + KH - line(m0)) * PW for m0 in range(0, M, rows))
+        chunks = -(-PC // kc)
+        assert need + (kc == 1) <= npix <= (2 if kc == 4 else 3) * 256 + (kc == 1)
+        assert npix * 32 * kc * (2 if chunks > 1 else 1) <= lds <= 64 * 1024
+        planes = 2 if type in (0, 2, 4) else 1
+        pairs = (KH * KW + 1) // 2 if kc == 1 else KH * KW * kc // 2
+        assert weights == -(-KN // 32) * chunks * pairs * 512 * planes
+        a = (type, N, H, W, C)
+        if KH * KW > 1:
+            assert lib.tab_conv2d_workspace_bytes_full(*a, KN, KH, KW) >= lib.tab_conv2d_workspace_bytes(*a) + weights + 15
+            if type < 4:
+                bits = 2 if type < 2 else 1
+                assert lib.tab_layer_workspace_bytes_full(*a, KN, KH, KW) >= lib.tab_layer_workspace_bytes(bits, N, H, W, C) + weights + 15
+    assert planned > 1500
+
+
+def test_sizes_of_refused_arguments(lib):
+    assert lib.tab_conv2d_workspace_bytes_full(7, 1, 1, 1, 1, 1, 3, 3) == 0 and lib.tab_conv2d_workspace_bytes_full(0, 1, 1, 1, 1, 0, 3, 3) == 0
+    assert lib.tab_layer_workspace_bytes_full(4, 1, 1, 1, 1, 1, 3, 3) == 0
+    for type in range(6):  # one tap, or type 5: no room beyond the packed activation
+        KH = 1 if type < 5 else 3
+        assert lib.tab_conv2d_workspace_bytes_full(type, 2, 9, 9, 100, 64, KH, KH) == lib.tab_conv2d_workspace_bytes(type, 2, 9, 9, 100)
+
+
+def test_the_rule_on_its_measured_launches(lib):
+    """The compiled choices (256 compute units where no device is present) against the tiled kernels' times: within what the rule's
+    comment states, and no single choice more than a quarter off."""
+    spec = importlib.util.spec_from_file_location("fit", os.path.join(TUNING, "fit_conv_patch_model.py"))
+    fit = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(fit)
+    lib.tab_set_conv_kernel(0, -1)
+    rows = [r for r in fit.parse(fit.DATA) if fit.eligible(r)]
+    assert len(rows) > 1500
+    chosen = []
+    for r in rows:
+        shape, kc, npix, lds, _ = plan(lib, r["type"], r["p1"], r["p2"], r["s"], r["s"], r["N"], r["H"], r["W"], r["C"], r["KN"], r["KH"], r["KW"])
+        if shape >= 0:
+            assert fit.patch_features(r, shape) is not None and fit.chunk(r, shape) == (kc, npix, lds), r
+        chosen.append(shape if shape >= 0 else None)
+    geometric, total, best_geometric, best_total, worst = fit.regret(rows, chosen)
+    assert geometric < 0.96 and total < 0.94 and geometric < 1.02 * best_geometric and worst < 1.3, (geometric, total, worst)
+    assert np.mean([c is not None for c in chosen]) > 0.2

@@ -1,0 +1,129 @@
+"""The convolution that keeps its input patch in LDS, every shape forced on whole calls, layers (NHWC and NCHW) and packed activations,
+against the tiled kernel of 64x64: chunks of one, two and four words, one and several of them, odd words per pixel, an odd number of taps,
+tiles that span images and lines, rows past M, filters past a tile, strides, asymmetric padding, arbitrary weight bits, packed output."""
+import ctypes
+
+import pytest
+import torch
+
+import tab_amd
+from tab_amd import _capi
+from tab_amd import nn as tab_nn
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = range(12, 17)
+CASES = [
+    # N, H, W, C, KN, KH, KW, p1, p2, s1, s2
+    (2, 14, 14, 128, 64, 3, 3, 1, 1, 1, 1), (3, 7, 7, 64, 70, 3, 3, 1, 1, 1, 1), (2, 13, 11, 192, 130, 3, 3, 1, 0, 1, 1),
+    (3, 9, 10, 256, 40, 5, 5, 2, 2, 2, 2), (1, 30, 31, 100, 75, 3, 3, 1, 1, 1, 1), (5, 6, 7, 320, 33, 2, 3, 0, 1, 1, 2),
+    (9, 23, 23, 832, 49, 3, 3, 1, 1, 1, 1), (1, 56, 56, 64, 65, 3, 3, 1, 1, 1, 1), (2, 8, 12, 3, 35, 1, 7, 0, 3, 1, 1),
+    (2, 17, 3, 448, 99, 3, 3, 1, 1, 2, 1), (7, 1, 9, 130, 31, 1, 2, 0, 1, 1, 1), (3, 20, 20, 70, 256, 3, 3, 2, 3, 3, 1),
+]
+
+
+@pytest.fixture(scope="module")
+def lib():
+    return ctypes.CDLL(_capi.LIB_PATH)
+
+
+@pytest.fixture(autouse=True)
+def automatic_kernel():
+    yield
+    tab_amd.set_conv_kernel()
+
+
+def weights(type, g, KN, KH, KW, C):
+    w = torch.randn((KN, KH, KW, C), device="cuda", generator=g)
+    ths = tab_amd.Threshold(w, KN)
+    if type == 4:
+        return tab_amd.QuantizeFormat(w, ths, 4, KN, KH, KW, C), torch.zeros(KN, dtype=torch.int32, device="cuda")
+    return tab_amd.Quantize(w, ths, 2 if type in (0, 2) else 1, KN, KH, KW, C)
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_calls_and_layers(case, lib):
+    N, H, W, C, KN, KH, KW, p1, p2, s1, s2 = case
+    print(f"[case] patch {case}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(KN + C)
+    x = torch.randn((N, H, W, C), device="cuda", generator=g)
+    ths = tab_amd.Threshold(x, N)
+    for type in range(5):
+        QW, btn = weights(type, g, KN, KH, KW, C)
+        run = lambda: tab_amd.Conv2d(x, QW, ths, btn, type, p1, p2, s1, s2, N, H, W, C, KN, KH, KW)  # noqa: E731
+        layers = []
+        if type < 4:
+            w = torch.randn((KN, C, KH, KW), device="cuda", generator=g)
+            for layout in ("NHWC", "NCHW"):
+                layer = tab_nn.TABConv2d.from_float(w, type, (s1, s2), (p1, p2), data_format=layout)
+                layers.append((layer, x if layout == "NHWC" else x.permute(0, 3, 1, 2).contiguous()))
+        tab_amd.set_conv_kernel(tab_amd.CONV_MATRIX, 2)
+        want = [run()] + [layer(a) for layer, a in layers]
+        for shape in SHAPES:
+            lib.tab_internal_force_patch(shape)
+            got = [run()] + [layer(a) for layer, a in layers]
+            assert all(torch.equal(y, z) for y, z in zip(got, want)), (type, shape)
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_arbitrary_bits_and_packed_output(case, lib):
+    N, H, W, C, KN, KH, KW, p1, p2, s1, s2 = case
+    print(f"[case] patch, arbitrary bits {case}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(KN + W)
+    OH, OW = (H + 2 * p1 - KH + 1) // s1, (W + 2 * p2 - KW + 1) // s2
+    bits = lambda *shape: torch.randint(-2**63, 2**63 - 1, shape, device="cuda", generator=g, dtype=torch.int64)  # noqa: E731
+    room = torch.empty((((KN + 31) // 32) * ((KH * KW + 1) * ((C + 63) // 64 + 1) // 2 + 1) * 1024,), dtype=torch.uint8, device="cuda")
+    fitted = 0
+    for type in range(5):
+        QX, QW = bits(N * H * W * tab_amd.operand_words(type, 0, C)), bits(KN * KH * KW * tab_amd.operand_words(type, 1, C))
+        btn = torch.randint(0, 99, (KN,), device="cuda", generator=g, dtype=torch.int32)
+        a = (QX, QW, btn, type, p1, p2, s1, s2, N, H, W, C, KN, KH, KW)
+        for planes in (0, 1, 2):
+            tab_amd.set_conv_kernel(tab_amd.CONV_MATRIX, 2)
+            want = tab_amd.Conv2dPacked(*a) if planes == 0 else tab_amd.Conv2dPackedOut(*a, torch.full((N,), 3.0, device="cuda"), planes)
+            for shape in SHAPES:
+                lib.tab_internal_force_patch(shape)
+                got = torch.empty_like(want)
+                p = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+                status = lib.tab_internal_conv_patch(p(QX), p(QW), p(btn), *a[3:], p(got) if planes == 0 else None, ctypes.c_float(3.0), planes,
+                                                     None if planes == 0 else p(got), p(room), ctypes.c_size_t(room.numel()), 3,
+                                                     ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+                if status == 0:  # (else the patch does not fit LDS)
+                    fitted += 1
+                    assert torch.equal(got, want), (type, planes, shape)
+    assert fitted >= 15
+
+
+def test_a_small_workspace_and_the_built_in_scratch(lib):
+    """A workspace of tab_conv2d_workspace_bytes takes the kernels that read the weights where they lie; the built-in scratch has room
+    for them; a capture replays with both."""
+    N, H, W, C, KN = 64, 14, 14, 256, 256
+    g = torch.Generator(device="cuda").manual_seed(5)
+    x, ths = torch.randn((N, H, W, C), device="cuda", generator=g), torch.full((N,), 0.5, device="cuda")
+    QW, btn = weights(0, g, KN, 3, 3, C)
+    lib.tab_internal_force_patch(14)
+    lib.tab_conv2d_workspace_bytes.restype = ctypes.c_size_t
+    size = lib.tab_conv2d_workspace_bytes(0, N, H, W, C)
+    ws, y = torch.empty(size, dtype=torch.uint8, device="cuda"), torch.empty((N, KN, H, W), device="cuda")
+    p = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+
+    def call():
+        assert lib.tab_conv2d(p(x), p(QW), p(ths), p(btn), 0, 1, 1, 1, 1, N, H, W, C, KN, 3, 3, p(y), p(ws), ctypes.c_size_t(size),
+                              ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+
+    call()
+    a = (x, QW, ths, btn, 0, 1, 1, 1, 1, N, H, W, C, KN, 3, 3)
+    want = tab_amd.Conv2d(*a)
+    assert torch.equal(y, want) and torch.equal(tab_amd.Conv2dStatic(*a), want)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = tab_amd.Conv2d(*a)
+        call()
+    for seed in range(3):
+        x.copy_(torch.randn((N, H, W, C), device="cuda", generator=torch.Generator(device="cuda").manual_seed(seed)))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, y)
+        tab_amd.set_conv_kernel(tab_amd.CONV_MATRIX, 2)
+        assert torch.equal(out, tab_amd.Conv2d(*a))
+        lib.tab_internal_force_patch(14)
