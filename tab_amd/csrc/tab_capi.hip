@@ -647,7 +647,7 @@ int tab_layer_conv2d(const float *dev_X, int nchw, float act_scale, const int64_
     tab::Thresholds ths;
     hipError_t e = hipSuccess;
     if (one == 2 && own)
-        ths = tab::Thresholds{dev_X, (double)act_scale / (double)C, tab::kOwnPixelThresholds};
+        ths = tab::Thresholds{dev_X, (double)act_scale / (double)C, tab::kOwnPixelThresholds, 0};
     else
         e = own_thresholds(dev_X, s.abits, act_scale, N, (long)H * W * C, sums, &ths, stream);
     if (e != hipSuccess) return device_fail(e, "threshold launch");

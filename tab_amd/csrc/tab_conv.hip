@@ -541,7 +541,9 @@ WeightJob patch_weight_job(int type, const ConvArgs &a, const PatchPlan &plan, u
 {
     const int planes = type == 0 || type == 2 || type == 4 ? 2 : 1;
     const long items = (long)(plan.weight_bytes / 8 / planes);  // 64 lanes a run
-    return WeightJob{a.qw, out, a.KN, (uint32_t)a.PC | (uint32_t)(a.KH * a.KW) << 16, (uint32_t)((items + 255) / 256), (uint32_t)plan.kc | (uint32_t)planes << 8};
+    return WeightJob{a.qw, out, a.KN, (uint32_t)a.PC | (uint32_t)(a.KH * a.KW) << 16,
+                     (uint32_t)((items + 255) / 256 + 7) / 8 * 8,  // whole groups of eight: the quantizer's workgroups stay on their XCDs
+                     (uint32_t)plan.kc | (uint32_t)planes << 8};
 }
 
 hipError_t launch_conv(int type, const ConvArgs &args, hipStream_t stream)

@@ -87,7 +87,7 @@ template <int BITS, int LOADS = kLoadsPerLane>
 __global__ __launch_bounds__(kThreads) void quantize_rows64(const floatx4 *__restrict__ x, const Thresholds ths, uint32_t *__restrict__ q, long rows,
                                                             long rows_per_item, Div32 div_item, int32_t *btn, long items)
 {
-    quantize_rows64_block<BITS, LOADS>(x, ths, q, rows, rows_per_item, div_item, blockIdx.x);
+    quantize_rows64_block<BITS, LOADS>(x, ths, q, rows, rows_per_item, div_item, in_eighths(blockIdx.x, ths.eighth));
     const long row = (long)blockIdx.x * (4 * LOADS * kWavesPerBlock) + (threadIdx.x >> 6) * (4 * LOADS) + (threadIdx.x & 63);
     if ((threadIdx.x & 63) < 4 * LOADS) zero_counts(btn, items, row);
 }
@@ -100,7 +100,7 @@ __global__ __launch_bounds__(kThreads) void quantize_rows64_weights(const floatx
 {
     uint32_t block = blockIdx.x;
     if (pack_weights(job, block)) return;
-    quantize_rows64_block<BITS, LOADS>(x, ths, q, rows, rows_per_item, div_item, block);
+    quantize_rows64_block<BITS, LOADS>(x, ths, q, rows, rows_per_item, div_item, in_eighths(block, ths.eighth));
 }
 
 // The same row quantizer for a 1x1 convolution with stride and no padding, which reads only the
@@ -313,7 +313,7 @@ __global__ __launch_bounds__(kThreads) void quantize_tile(const float *__restric
                                                           long pixels, long pixels_per_item, Div32 div_item, int C, int tile_pixels, int words,
                                                           int32_t *btn, long items)
 {
-    const long p0 = (long)blockIdx.x * tile_pixels;
+    const long p0 = (long)in_eighths(blockIdx.x, ths.eighth) * tile_pixels;
     const int live = pixels - p0 < tile_pixels ? (int)(pixels - p0) : tile_pixels;  // pixels of the tile that exist
     quantize_one_tile<MODE, LP>(x, ths, q, p0, live, pixels_per_item, div_item, C, tile_pixels, blockIdx.y * words, words);
     for (int i = threadIdx.x; i < live; i += kThreads) zero_counts(btn, items, p0 + i);
@@ -328,7 +328,7 @@ __global__ __launch_bounds__(kThreads) void quantize_tile_weights(const float *_
     uint32_t block = blockIdx.x;
     if (blockIdx.y != 0 && block < job.blocks) return;  // (the grid's other parts of a pixel)
     if (pack_weights(job, block)) return;
-    const long p0 = (long)block * tile_pixels;
+    const long p0 = (long)in_eighths(block, ths.eighth) * tile_pixels;
     const int live = pixels - p0 < tile_pixels ? (int)(pixels - p0) : tile_pixels;  // pixels of the tile that exist
     quantize_one_tile<MODE, LP>(x, ths, q, p0, live, pixels_per_item, div_item, C, tile_pixels, blockIdx.y * words, words);
 }
@@ -528,8 +528,9 @@ __global__ __launch_bounds__(kThreads) void quantize_nchw(const float *__restric
                                                           uint64_t *__restrict__ q, int N, int C, long HW, int PC, int32_t *btn)
 {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const PixelRun<VEC> run((blockIdx.x / PC * (kWavesPerBlock / SPLIT) + wave / SPLIT) * 64L + (threadIdx.x & 63), N, HW);
-    quantize_nchw_unit<BITS, VEC, SPLIT, NT>(x, ths, q, run, C, HW, PC, blockIdx.x % PC);
+    const uint32_t block = in_eighths(blockIdx.x, ths.eighth);
+    const PixelRun<VEC> run((block / PC * (kWavesPerBlock / SPLIT) + wave / SPLIT) * 64L + (threadIdx.x & 63), N, HW);
+    quantize_nchw_unit<BITS, VEC, SPLIT, NT>(x, ths, q, run, C, HW, PC, block % PC);
     if (wave % SPLIT == 0) zero_counts(btn, N, run.pixel, VEC);
 }
 
@@ -540,6 +541,7 @@ __global__ __launch_bounds__(kThreads) void quantize_nchw_weights(const float *_
 {
     uint32_t block = blockIdx.x;
     if (pack_weights(job, block)) return;
+    block = in_eighths(block, ths.eighth);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const PixelRun<VEC> run((block / PC * (kWavesPerBlock / SPLIT) + wave / SPLIT) * 64L + (threadIdx.x & 63), N, HW);
     quantize_nchw_unit<BITS, VEC, SPLIT, NT>(x, ths, q, run, C, HW, PC, block % PC);
@@ -593,6 +595,7 @@ __global__ __launch_bounds__(64, BITS == 1 ? (U == 4 ? 4 : 7) : (U == 4 ? 1 : 4)
         if (pack_weights(extra, block)) return;
     int32_t *btn = nullptr;
     if constexpr (!WEIGHTS) btn = extra;
+    if constexpr (!COUNT) block = in_eighths(block, ths.eighth);
     const int groups = PC / U;
     // COUNT: N is the number of slices of an image
     const int image = COUNT ? (int)(block / (uint32_t)N) : 0;
@@ -779,12 +782,14 @@ __global__ __launch_bounds__(kCountThreads) void btn_popcount(const ulonglong2 *
 // partials in index order in fp64.
 // An item of one slice is finished here: `out` gets its threshold, not its sum.
 __global__ __launch_bounds__(kThreads) void abs_sum_partial(const float *__restrict__ x, float *__restrict__ out,
-                                                            long per_item, int splits, double scale_over_count)
+                                                            long per_item, int splits, double scale_over_count, int eighth, int kept)
 {
     constexpr int kLoads = 4;  // in flight per lane
     __shared__ float wave_part[kWavesPerBlock];
-    const long item = blockIdx.x / splits;
-    const int split = blockIdx.x % splits;
+    const uint32_t block = in_eighths(blockIdx.x, eighth);
+    const bool keep = (int)(blockIdx.x >> 3) >= kept;  // uniform
+    const long item = block / (uint32_t)splits;
+    const int split = (int)(block % (uint32_t)splits);
     const long slice = ((per_item + splits - 1) / splits + 3) & ~3L;  // multiple of 4 elements
     const long begin = split * slice;
     long end = begin + slice;
@@ -798,14 +803,18 @@ __global__ __launch_bounds__(kThreads) void abs_sum_partial(const float *__restr
             sum += (__builtin_fabsf(v[0]) + __builtin_fabsf(v[1])) + (__builtin_fabsf(v[2]) + __builtin_fabsf(v[3]));
         };
         long i = threadIdx.x;
-        for (; i + (kLoads - 1) * kThreads < n4; i += kLoads * kThreads) {
-            floatx4 v[kLoads];
+        auto stream = [&](auto load) {
+            for (; i + (kLoads - 1) * kThreads < n4; i += kLoads * kThreads) {
+                floatx4 v[kLoads];
 #pragma unroll
-            for (int u = 0; u < kLoads; u++) v[u] = __builtin_nontemporal_load(&src4[i + u * kThreads]);
+                for (int u = 0; u < kLoads; u++) v[u] = load(&src4[i + u * kThreads]);
 #pragma unroll
-            for (int u = 0; u < kLoads; u++) add(v[u]);
-        }
-        for (; i < n4; i += kThreads) add(__builtin_nontemporal_load(&src4[i]));
+                for (int u = 0; u < kLoads; u++) add(v[u]);
+            }
+            for (; i < n4; i += kThreads) add(load(&src4[i]));
+        };
+        if (keep) stream([](const floatx4 *p) { return *p; });
+        else stream([](const floatx4 *p) { return __builtin_nontemporal_load(p); });
         for (i = begin + n4 * 4 + threadIdx.x; i < end; i += kThreads) sum += __builtin_fabsf(src[i]);
     } else {
         for (long i = begin + threadIdx.x; i < end; i += kThreads) sum += __builtin_fabsf(src[i]);
@@ -818,7 +827,7 @@ __global__ __launch_bounds__(kThreads) void abs_sum_partial(const float *__restr
         float total = 0.f;
 #pragma unroll
         for (int w = 0; w < kWavesPerBlock; w++) total += wave_part[w];
-        out[blockIdx.x] = splits == 1 ? (float)((double)total * scale_over_count) : total;
+        out[block] = splits == 1 ? (float)((double)total * scale_over_count) : total;
     }
 }
 
@@ -846,7 +855,14 @@ hipError_t launch_abs_sums(const float *x, long items, long per_item, float scal
     source->values = partial;
     source->scale = (double)scale / (double)per_item;
     source->splits = splits == 1 ? 0 : splits;
-    abs_sum_partial<<<dim3((unsigned)(items * splits)), dim3(kThreads), 0, stream>>>(x, partial, per_item, splits, source->scale);
+    // The quantizer that follows reads x again, backwards in eighths: what it begins with, 24 MB, is read through the L2s here, the rest
+    // past them (plain loads stream 8-11 % slower from 400 MB on).  Two passes over 25.7 MB (NCHW, N=32 56x56x64): 7.0 + 7.0 -> 5.6 +
+    // 5.6 us; over 103 MB (N=64 56x56x128): 9.5 + 22.6 -> 8.8 + 17.2.
+    source->eighth = -1;
+    const long blocks = items * splits, share = blocks / 8, bytes = items * per_item * 4;
+    const long kept = bytes <= (24L << 20) ? 0 : share - (long)((double)share * (24L << 20) / (double)bytes);
+    abs_sum_partial<<<dim3((unsigned)blocks), dim3(kThreads), 0, stream>>>(x, partial, per_item, splits, source->scale, blocks < 64 ? 0 : (int)share,
+                                                                         (int)kept);
     return hipGetLastError();
 }
 
@@ -925,10 +941,10 @@ void launch_quantize_tile_of(const float *x, const Thresholds &ths, long pixels,
     const dim3 grid((unsigned)((pixels + tile_pixels - 1) / tile_pixels), (unsigned)((PC + words - 1) / words));
     if (weights) {
         quantize_tile_weights<MODE, LP><<<dim3(grid.x + weights->blocks, grid.y), dim3(kThreads), lds, stream>>>(
-            x, ths, q, pixels, pixels_per_item, div_item, C, (int)tile_pixels, words, *weights);
+            x, grid.y == 1 ? ordered(ths, grid.x) : ordered(ths, 0), q, pixels, pixels_per_item, div_item, C, (int)tile_pixels, words, *weights);
         return;
     }
-    quantize_tile<MODE, LP><<<grid, dim3(kThreads), lds, stream>>>(x, ths, q, pixels, pixels_per_item, div_item, C, (int)tile_pixels, words, btn, items);
+    quantize_tile<MODE, LP><<<grid, dim3(kThreads), lds, stream>>>(x, grid.y == 1 ? ordered(ths, grid.x) : ordered(ths, 0), q, pixels, pixels_per_item, div_item, C, (int)tile_pixels, words, btn, items);
 }
 
 // The general path with the fewest lanes a word that hold it.
@@ -956,7 +972,7 @@ hipError_t launch_rows64_weights(const float *x, const Thresholds &ths, int form
 {
     auto launch = [&](auto kernel, long rows_per_block) {
         kernel<<<dim3((unsigned)((rows + rows_per_block - 1) / rows_per_block) + job.blocks), dim3(kThreads), 0, stream>>>(
-            reinterpret_cast<const floatx4 *>(x), ths, reinterpret_cast<uint32_t *>(qx), rows, rows_per_item, div_item, job);
+            reinterpret_cast<const floatx4 *>(x), ordered(ths, (rows + rows_per_block - 1) / rows_per_block), reinterpret_cast<uint32_t *>(qx), rows, rows_per_item, div_item, job);
     };
     // (sizes of workgroups as in launch_quantize)
     if (rows <= kSmallLaunchBlocks * 128) launch(format == 4 ? quantize_rows64_weights<4, 2> : format == 2 ? quantize_rows64_weights<2, 2> : quantize_rows64_weights<1, 2>, 32);
@@ -1012,15 +1028,15 @@ hipError_t launch_quantize(const float *x, const Thresholds &ths, int bitwidth, 
             // (3.1 MB of fp32: 5.5 -> 4.2 us)
             const dim3 grid((unsigned)((rows + 8 * kWavesPerBlock - 1) / (8 * kWavesPerBlock)));
             if (bitwidth == 2)
-                quantize_rows64<2, 2><<<grid, block, 0, stream>>>(x4, ths, q32, rows, words_per_item, div_item, zeroed, items);
+                quantize_rows64<2, 2><<<grid, block, 0, stream>>>(x4, ordered(ths, grid.x), q32, rows, words_per_item, div_item, zeroed, items);
             else
-                quantize_rows64<1, 2><<<grid, block, 0, stream>>>(x4, ths, q32, rows, words_per_item, div_item, zeroed, items);
+                quantize_rows64<1, 2><<<grid, block, 0, stream>>>(x4, ordered(ths, grid.x), q32, rows, words_per_item, div_item, zeroed, items);
         } else {
             const dim3 grid((unsigned)blocks);
             if (bitwidth == 2)
-                quantize_rows64<2><<<grid, block, 0, stream>>>(x4, ths, q32, rows, words_per_item, div_item, zeroed, items);
+                quantize_rows64<2><<<grid, block, 0, stream>>>(x4, ordered(ths, grid.x), q32, rows, words_per_item, div_item, zeroed, items);
             else
-                quantize_rows64<1><<<grid, block, 0, stream>>>(x4, ths, q32, rows, words_per_item, div_item, zeroed, items);
+                quantize_rows64<1><<<grid, block, 0, stream>>>(x4, ordered(ths, grid.x), q32, rows, words_per_item, div_item, zeroed, items);
         }
     } else if (bitwidth == 2) {
         launch_quantize_tile<2>(x, ths, pixels, pixels_per_item, items, C, qx, zeroed, nullptr, weights, stream);
@@ -1049,12 +1065,12 @@ hipError_t launch_quantize_nchw(const float *x, const Thresholds &ths, int bitwi
     const bool counted = btn && bitwidth == 2 && (count_workspace || (words_per_item <= 64 && PC <= kOneSliceUnits)) &&
                          N * (HW / 4 + 1) * PC < 0x7fffffffL;
     auto launch = [&](auto kernel, long blocks, int threads) {
-        kernel<<<dim3((unsigned)blocks), dim3(threads), 0, stream>>>(x, ths, qx, N, C, HW, PC, zeroed);
+        kernel<<<dim3((unsigned)blocks), dim3(threads), 0, stream>>>(x, ordered(ths, blocks), qx, N, C, HW, PC, zeroed);
     };
     auto launch_weights = [&](auto kernel, long blocks, int threads) {
         WeightJob job = *weights;
         job.blocks *= kThreads / threads;
-        kernel<<<dim3((unsigned)blocks + job.blocks), dim3(threads), 0, stream>>>(x, ths, qx, N, C, HW, PC, job);
+        kernel<<<dim3((unsigned)blocks + job.blocks), dim3(threads), 0, stream>>>(x, ordered(ths, blocks), qx, N, C, HW, PC, job);
     };
     // PC even, enough pixels for a wave on every SIMD: the form that gathers each wave's output into whole runs
     const int unit = PC % 4 == 0 ? 4 : PC % 2 == 0 ? 2 : 1;
