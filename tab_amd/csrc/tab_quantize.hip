@@ -17,6 +17,11 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kWavesPerBlock = kThreads / 64;
 constexpr int kRowsPerWave = 4 * kLoadsPerLane; // each wave-wide float4 load covers 4 rows
+// LDS that the streaming launches of quantize_rows64 ask for and do not use: seven workgroups on a CU, where registers would let eight.
+// Their reads then follow each other more closely in memory: 822 MB of one plane 136.6 -> 134.1 us, of two 148.0 -> 145.8; six are as fast
+// there, but 54 MB, 1636 workgroups, are a second round for them (10.4 -> 11.1).
+constexpr int kStreamLds = 22 << 10;
+
 constexpr long kSmallLaunchBlocks = 512;        // at or below this many 128-row workgroups a launch is latency-bound
 
 __device__ __forceinline__ int wave_sum(int v)
@@ -166,7 +171,7 @@ __global__ __launch_bounds__(kThreads) void quantize_rows64_count(const floatx4 
             const floatx4 *src = &x[(first + (r < rows_per_item ? r : rows_per_item - 1)) * 16 + l];
             v[u] = NT ? __builtin_nontemporal_load(src) : *src;
         }
-        const float t = wave_threshold(ths, item);
+        const float t = given_threshold(ths, item);
 #pragma unroll
         for (int u = 0; u < LOADS; u++) {
             const long r = at + u * 4 + sub;
@@ -233,7 +238,12 @@ __device__ __forceinline__ int quantize_one_tile(const float *__restrict__ x, co
     float *const th = reinterpret_cast<float *>(tile + ((tile_pixels - 1) * C + channels_here + 3 + 3) / 4 * 4 + 256);
     const float t_first = wave_threshold(ths, item_first);
     if (!one_item)
-        for (int i = tid; i < live; i += kThreads) th[i] = lane_threshold(ths, item_of(p0 + i));
+        for (int i0 = wave * 64; i0 < live; i0 += kThreads) {
+            const long item = item_of(p0 + min(i0 + lane, live - 1));
+            const long first = item_of(p0 + i0), last = item_of(p0 + min(i0 + 63, live - 1));
+            const float t = MODE == 2 && ths.splits > 0 ? span_threshold(ths, item, first, last, request_threshold(ths, first)) : given_threshold(ths, item);
+            if (i0 + lane < live) th[i0 + lane] = t;
+        }
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
 
@@ -403,10 +413,20 @@ struct PixelRun {
             for (int e = 0; e < VEC; e++) v[e] = w[e];
         }
     }
-    __device__ __forceinline__ float threshold(const Thresholds &ths) const
+    // the thread's threshold in two steps (every lane active): the partial sums of the wave's first image are requested before the pixels.
+    // OWN: it may have to be added up (layers of two planes); ONE: the workgroup has one image
+    template <bool OWN>
+    __device__ __forceinline__ floatx4 request(const Thresholds &ths) const
     {
-        const long n_first = (long)__builtin_amdgcn_readfirstlane((int)n);
-        return __all(n == n_first) ? wave_threshold(ths, n_first) : lane_threshold(ths, n);
+        return OWN && ths.splits > 0 ? request_threshold(ths, (long)__builtin_amdgcn_readfirstlane((int)n)) : floatx4{};
+    }
+    template <bool OWN, bool ONE>
+    __device__ __forceinline__ float threshold(const Thresholds &ths, const floatx4 requested) const
+    {
+        if (ONE) return given_threshold(ths, n);
+        const long n_first = (long)__builtin_amdgcn_readfirstlane((int)n), n_last = (long)__builtin_amdgcn_readlane((int)n, 63);
+        if (OWN && ths.splits > 0) return span_threshold(ths, n, n_first, n_last, requested);
+        return n_last == n_first ? given_threshold(ths, n_first) : given_threshold(ths, n);
     }
     // pixels [first, last) of a wave's lanes from..to, which follow each other without a gap
     __device__ __forceinline__ long first(int from = 0) const { return lane_pixel(from); }
@@ -428,7 +448,7 @@ struct PixelRun {
 // grid = ceil(runs / (64 * 4 / SPLIT)) * PC workgroups, the word index fastest: the workgroups that write the PC words of the
 // same pixels run side by side, so their 8- or 16-byte stores meet in L2 as whole lines.
 // The lane's nonzero values are counted for COUNT (see Counts).
-template <int BITS, int VEC, int SPLIT, bool NT>
+template <int BITS, int VEC, int SPLIT, bool NT, bool COUNT = false>
 __device__ __forceinline__ int quantize_nchw_unit(const float *__restrict__ x, const Thresholds &ths, uint64_t *__restrict__ q, const PixelRun<VEC> &run,
                                                   int C, long HW, int PC, int pc)
 {
@@ -449,6 +469,7 @@ __device__ __forceinline__ int quantize_nchw_unit(const float *__restrict__ x, c
     for (int e = 0; e < VEC; e++) less[e] = more[e] = 0;
     if (channels > 0) {
         const float *src = x + (run.n * C + c0) * HW + run.s;
+        const floatx4 requested = run.template request<BITS == 2 && !COUNT>(ths);
         float v[kPart][VEC];
         if (channels == kPart) {
 #pragma unroll
@@ -464,8 +485,8 @@ __device__ __forceinline__ int quantize_nchw_unit(const float *__restrict__ x, c
                 if (u < channels) run.template load<NT>(v[u], src + u * HW);
             }
         }
-        // the threshold is looked up (or added up) while the channels are in flight
-        const float t = run.threshold(ths);
+        // the threshold is added up while the channels are in flight
+        const float t = run.template threshold<BITS == 2 && !COUNT, COUNT>(ths, requested);
         const float low = BITS == 2 ? -t : t;
         if constexpr (VEC == 4) {
 #pragma unroll
@@ -559,7 +580,7 @@ __global__ __launch_bounds__(kThreads) void quantize_nchw_count(const float *__r
     for (int unit = slice; unit < units; unit += counts.slices) {
         if (unit >= counts.slices) __syncthreads();  // the waves have read the words before
         const PixelRun<VEC> run((unit / PC * (kWavesPerBlock / SPLIT) + wave / SPLIT) * 64L + (threadIdx.x & 63), item, HW, std::true_type());
-        count += quantize_nchw_unit<2, VEC, SPLIT, NT>(x, ths, q, run, C, HW, PC, unit % PC);
+        count += quantize_nchw_unit<2, VEC, SPLIT, NT, true>(x, ths, q, run, C, HW, PC, unit % PC);
     }
     store_count<kWavesPerBlock>(count, counts.out + blockIdx.x, scratch);
 }
@@ -671,8 +692,9 @@ __global__ __launch_bounds__(64, BITS == 1 ? (U == 4 ? 4 : 7) : (U == 4 ? 1 : 4)
     };
     constexpr int kBatches = kWordBits / kInFlight;  // per word
     float v0[kInFlight][VEC], v1[kInFlight][VEC];
+    const floatx4 requested = run.template request<BITS == 2 && !COUNT>(ths);
     load(v0, 0);
-    t = run.threshold(ths);
+    t = run.template threshold<BITS == 2 && !COUNT, COUNT>(ths, requested);
 #pragma unroll
     for (int u = 0; u < U; u++) {
 #pragma unroll
@@ -970,13 +992,13 @@ size_t quantize_count_workspace(int bitwidth, long items, long pixels_per_item, 
 hipError_t launch_rows64_weights(const float *x, const Thresholds &ths, int format, long rows, long rows_per_item, Div32 div_item, uint64_t *qx,
                                  const WeightJob &job, hipStream_t stream)
 {
-    auto launch = [&](auto kernel, long rows_per_block) {
-        kernel<<<dim3((unsigned)((rows + rows_per_block - 1) / rows_per_block) + job.blocks), dim3(kThreads), 0, stream>>>(
+    auto launch = [&](auto kernel, long rows_per_block, int lds) {
+        kernel<<<dim3((unsigned)((rows + rows_per_block - 1) / rows_per_block) + job.blocks), dim3(kThreads), lds, stream>>>(
             reinterpret_cast<const floatx4 *>(x), ordered(ths, (rows + rows_per_block - 1) / rows_per_block), reinterpret_cast<uint32_t *>(qx), rows, rows_per_item, div_item, job);
     };
     // (sizes of workgroups as in launch_quantize)
-    if (rows <= kSmallLaunchBlocks * 128) launch(format == 4 ? quantize_rows64_weights<4, 2> : format == 2 ? quantize_rows64_weights<2, 2> : quantize_rows64_weights<1, 2>, 32);
-    else launch(format == 4 ? quantize_rows64_weights<4> : format == 2 ? quantize_rows64_weights<2> : quantize_rows64_weights<1>, 128);
+    if (rows <= kSmallLaunchBlocks * 128) launch(format == 4 ? quantize_rows64_weights<4, 2> : format == 2 ? quantize_rows64_weights<2, 2> : quantize_rows64_weights<1, 2>, 32, 0);
+    else launch(format == 4 ? quantize_rows64_weights<4> : format == 2 ? quantize_rows64_weights<2> : quantize_rows64_weights<1>, 128, kStreamLds);
     return hipGetLastError();
 }
 
@@ -999,16 +1021,16 @@ hipError_t launch_quantize(const float *x, const Thresholds &ths, int bitwidth, 
     if (counted && fast) {
         const floatx4 *x4 = reinterpret_cast<const floatx4 *>(x);
         uint32_t *q32 = reinterpret_cast<uint32_t *>(qx);
-        auto launch = [&](auto kernel, long rows) {
+        auto launch = [&](auto kernel, long rows, int lds) {
             const long slices = (words_per_item + rows - 1) / rows;
-            kernel<<<dim3((unsigned)(items * slices)), dim3(kThreads), 0, stream>>>(
+            kernel<<<dim3((unsigned)(items * slices)), dim3(kThreads), lds, stream>>>(
                 x4, ths, q32, words_per_item, Counts{slices == 1 ? btn : count_workspace, (int)slices});
             finish_counts(target, items, (int)slices, stream);
         };
         // (units of 128 rows for streaming and 32 for launches too small to fill the chip, as below)
-        if (words_per_item > 32 && words_per_item <= 128) launch(quantize_rows64_count<8, false>, 128);
-        else if (items * words_per_item <= kSmallLaunchBlocks * 128) launch(quantize_rows64_count<2, false>, 32);
-        else launch(quantize_rows64_count<8, true>, 128);
+        if (words_per_item > 32 && words_per_item <= 128) launch(quantize_rows64_count<8, false>, 128, 0);
+        else if (items * words_per_item <= kSmallLaunchBlocks * 128) launch(quantize_rows64_count<2, false>, 32, 0);
+        else launch(quantize_rows64_count<8, true>, 128, kStreamLds);
         return hipGetLastError();
     }
     if (counted && C <= 3072) {
@@ -1034,9 +1056,9 @@ hipError_t launch_quantize(const float *x, const Thresholds &ths, int bitwidth, 
         } else {
             const dim3 grid((unsigned)blocks);
             if (bitwidth == 2)
-                quantize_rows64<2><<<grid, block, 0, stream>>>(x4, ordered(ths, grid.x), q32, rows, words_per_item, div_item, zeroed, items);
+                quantize_rows64<2><<<grid, block, kStreamLds, stream>>>(x4, ordered(ths, grid.x), q32, rows, words_per_item, div_item, zeroed, items);
             else
-                quantize_rows64<1><<<grid, block, 0, stream>>>(x4, ordered(ths, grid.x), q32, rows, words_per_item, div_item, zeroed, items);
+                quantize_rows64<1><<<grid, block, kStreamLds, stream>>>(x4, ordered(ths, grid.x), q32, rows, words_per_item, div_item, zeroed, items);
         }
     } else if (bitwidth == 2) {
         launch_quantize_tile<2>(x, ths, pixels, pixels_per_item, items, C, qx, zeroed, nullptr, weights, stream);
@@ -1172,9 +1194,9 @@ hipError_t launch_quantize_format(const float *x, const float *ths_values, int f
             else
                 quantize_rows64<5, 2><<<small, block, 0, stream>>>(x4, ths, q32, rows, rows_per_item, div_item, nullptr, 0);
         } else if (format == 4) {
-            quantize_rows64<4><<<grid, block, 0, stream>>>(x4, ths, q32, rows, rows_per_item, div_item, nullptr, 0);
+            quantize_rows64<4><<<grid, block, kStreamLds, stream>>>(x4, ths, q32, rows, rows_per_item, div_item, nullptr, 0);
         } else {
-            quantize_rows64<5><<<grid, block, 0, stream>>>(x4, ths, q32, rows, rows_per_item, div_item, nullptr, 0);
+            quantize_rows64<5><<<grid, block, kStreamLds, stream>>>(x4, ths, q32, rows, rows_per_item, div_item, nullptr, 0);
         }
         return hipGetLastError();
     }

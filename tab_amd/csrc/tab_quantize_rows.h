@@ -29,45 +29,51 @@ __device__ __forceinline__ void quantize_rows64_block(const floatx4 *__restrict_
     long row_last = row0 + (4 * LOADS) - 1;
     if (row_last > rows - 1) row_last = rows - 1;
 
+    // The wave's items (scalar; div_item.mul == 0 says that rows reach 2^31 and the division takes 64 bits).  Partial sums are
+    // requested before x.
+    const long item_first = div_item.mul ? (long)div32((uint32_t)row0, div_item) : row0 / rows_per_item;
+    const long item_last = div_item.mul ? (long)div32((uint32_t)row_last, div_item) : row_last / rows_per_item;
+    const bool own = BITS == 2 && ths.splits > 0;
+    const floatx4 requested = own ? request_threshold(ths, item_first) : floatx4{};
+    // x and q from the wave's row on: 32-bit offsets from a scalar address leave registers for one more wave per SIMD
+    const floatx4 *const src = x + row0 * 16;
+    uint32_t *const dst = q + row0 * (BITS != 1 ? 4 : 2);
+    const uint32_t live = (uint32_t)(row_last - row0) + 1;
     floatx4 v[LOADS];
 #pragma unroll
     for (int u = 0; u < LOADS; u++) {
-        const long r = row0 + u * 4 + sub;
         // rows past the end read the last row again (not stored): straight-line loads, no branch per load
-        const floatx4 *src = &x[(r < rows ? r : rows - 1) * 16 + l];
+        const floatx4 *at = &src[min((uint32_t)(u * 4 + sub), live - 1) * 16 + l];
         // a small tensor is likely to sit in the caches (it was just written, or is read again): plain loads;
         // a large one streams past them: non-temporal loads (plain ones are 8-11 % slower at 400 MB and more)
-        v[u] = LOADS == 2 ? *src : __builtin_nontemporal_load(src);
+        v[u] = LOADS == 2 ? *at : __builtin_nontemporal_load(at);
     }
-
-    // The wave's items (scalar; div_item.mul == 0 says that rows reach 2^31 and the division takes 64 bits): with the
-    // short division the threshold is in flight together with the loads of x instead of behind a long one.
-    const long item_first = div_item.mul ? (long)div32((uint32_t)row0, div_item) : row0 / rows_per_item;
-    const long item_last = div_item.mul ? (long)div32((uint32_t)row_last, div_item) : row_last / rows_per_item;
-    const bool one_item = item_last == item_first;
-    const float t_first = wave_threshold(ths, item_first);
+    const float t_first = own ? finish_threshold(ths, item_first, requested) : given_threshold(ths, item_first);
+    const float t_last = item_last == item_first ? t_first : wave_threshold(ths, item_last);
 
     auto finish = [&](int u, float t) {
-        const long r = row0 + u * 4 + sub;
+        const uint32_t r = u * 4 + sub;
         uint32_t sign, nz, out[4];
         compare4<BITS>(v[u], t, sign, nz);
         pack_row<BITS>(sign, nz, l, out);  // lane 0 stores the whole element (8 or 16 bytes) at once
         if (BITS != 1) {
-            if (r < rows && l == 0) *reinterpret_cast<uintx4 *>(q + r * 4) = uintx4{out[0], out[1], out[2], out[3]};
+            if (r < live && l == 0) *reinterpret_cast<uintx4 *>(dst + r * 4) = uintx4{out[0], out[1], out[2], out[3]};
         } else {
-            if (r < rows && l == 0) *reinterpret_cast<uintx2 *>(q + r * 2) = uintx2{out[0], out[1]};
+            if (r < live && l == 0) *reinterpret_cast<uintx2 *>(dst + r * 2) = uintx2{out[0], out[1]};
         }
     };
     // two copies of the loop under a scalar branch: the common one has no load but x in flight, so each load is
     // waited for on its own
-    if (one_item) {
+    if (item_last <= item_first + 1) {
+        const uint32_t border = item_last == item_first ? 4 * LOADS : (uint32_t)(item_last * rows_per_item - row0);  // where the second begins
 #pragma unroll
-        for (int u = 0; u < LOADS; u++) finish(u, t_first);
-    } else {
+        for (int u = 0; u < LOADS; u++) finish(u, (uint32_t)(u * 4 + sub) < border ? t_first : t_last);
+    } else {  // items of fewer rows than the wave: their thresholds are given (partial sums are those of 64 rows and more)
+        const uint32_t before = (uint32_t)(row0 - item_first * rows_per_item);  // rows of the first item in front of the wave
 #pragma unroll
         for (int u = 0; u < LOADS; u++) {
-            const long r = row0 + u * 4 + sub;
-            finish(u, lane_threshold(ths, (r < rows ? r : rows - 1) / rows_per_item));
+            const uint32_t at = before + min((uint32_t)(u * 4 + sub), live - 1);
+            finish(u, ths.values == nullptr ? 0.f : ths.values[item_first + at / (uint32_t)rows_per_item]);
         }
     }
 }

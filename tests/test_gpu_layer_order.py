@@ -3,6 +3,7 @@ add the thresholds up in waves that may hold the ends of several images: against
 import pytest
 import torch
 
+import oracle
 import tab_amd
 from tab_amd.nn import TABConv2d
 
@@ -32,3 +33,20 @@ def test_layer_in_cache_order(size, nchw):
         want = tab_amd.Conv2dPacked(q, layer.QW, layer.BTN_W, conv_type, k // 2, k // 2, 1, 1, N, H, W, C, 130, k, k).view(N, H, W, 130)
         for _ in range(2):
             assert torch.equal(layer(given), want.permute(0, 3, 1, 2) if nchw else want), conv_type
+
+
+# N, H, W, C: waves of 32 rows (the larger half) and of 8 that hold one image, two and many, the last of them short
+GIVEN = [(41000, 1, 1, 64), (9001, 1, 5, 64), (1400, 31, 1, 64), (1250, 3, 11, 64), (700, 3, 7, 192), (90, 1, 7, 64), (33, 1, 1, 64), (11, 3, 3, 128)]
+
+
+@pytest.mark.parametrize("size", GIVEN)
+def test_given_thresholds_of_images_within_a_wave(size):
+    N, H, W, C = size
+    print(f"[case] given thresholds {size}", flush=True)
+    g = torch.Generator().manual_seed(N)
+    x = torch.randn((N, H, W, C), generator=g)
+    ths = torch.rand(N, generator=g)
+    for bits in (1, 2):
+        want, _ = oracle.quantize(x.numpy(), ths.numpy(), bits, N, H, W, C)
+        q = tab_amd.QuantizeActivation(x.cuda(), ths.cuda(), bits, N, H, W, C)
+        assert torch.equal(q.cpu().flatten(), torch.from_numpy(want).flatten().view(q.dtype)), bits
