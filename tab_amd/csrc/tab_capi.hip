@@ -651,8 +651,8 @@ int tab_layer_conv2d(const float *dev_X, int nchw, float act_scale, const int64_
     else
         e = own_thresholds(dev_X, s.abits, act_scale, N, (long)H * W * C, sums, &ths, stream);
     if (e != hipSuccess) return device_fail(e, "threshold launch");
-    if (ths.splits > 4 && (one == 1 || (one == 2 && !tab::conv_small_in_one_image(s.OH, s.OW)))) {
-        // these one-launch kernels look thresholds up lane by lane: with many partial sums an item they are added first
+    if (ths.splits > 4 && one == 2 && !tab::conv_small_in_one_image(s.OH, s.OW)) {
+        // this one-launch kernel looks thresholds up lane by lane: with many partial sums an item they are added first
         float *values = reinterpret_cast<float *>(sums + tab_threshold_workspace_bytes(N, (long)H * W * C));
         e = tab::launch_threshold_values(ths, N, values, static_cast<hipStream_t>(stream));
         if (e != hipSuccess) return device_fail(e, "threshold launch");

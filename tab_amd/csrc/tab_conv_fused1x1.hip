@@ -49,7 +49,7 @@ enum FusedInput {
 
 // NP: pairs of words, enough for a pixel's (1, 2 or 4).
 // CACHED: Y through the caches (ragged_rows_cached).
-template <int TYPE, int NP, int INPUT, bool CACHED>
+template <int TYPE, int NP, int INPUT, bool CACHED, bool OWN>
 __global__ __launch_bounds__(kConvThreads) void conv1x1_fused(const Fused1x1Args p)
 {
     static_assert(TYPE >= 0 && TYPE <= 3, "types 0..3");
@@ -65,7 +65,7 @@ __global__ __launch_bounds__(kConvThreads) void conv1x1_fused(const Fused1x1Args
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int r = lane & 31, kb = lane >> 5;
     const int sub = lane >> 4, l = lane & 15;
-    const int m0 = blockIdx.x * 32;
+    const int m0 = (int)(OWN ? in_eighths(blockIdx.x, p.ths.eighth) : blockIdx.x) * 32;
     const int PC = (p.C + kWordBits - 1) / kWordBits;
     const int tiles = (int)(p.shifts_tiles >> 12);
     const int live = p.M - m0 < 32 ? p.M - m0 : 32;
@@ -83,6 +83,23 @@ __global__ __launch_bounds__(kConvThreads) void conv1x1_fused(const Fused1x1Args
     constexpr bool HANDED = INPUT != kInputWords;
     int n = 0;
     const size_t in_offset = HANDED ? place_of(m0 + r, n) : 0;
+    // OWN: thresholds from the layer's own sums: the wave adds up those of its pixels' first and last image, requested before x.  (In a
+    // launch of its own it took 2 to 3 us: N=8 56x56x64->256 12.2 -> 10.4, one image of 56x56x64->64 11.2 -> 8.3.  A form of its own,
+    // since the code that is not run costs the calls with given thresholds 2 %.)
+    int n_first = 0, n_last = 0;
+    floatx4 requested = {};
+    if (OWN) {
+        if (HANDED) {
+            n_first = __builtin_amdgcn_readfirstlane(n);
+            n_last = __builtin_amdgcn_readlane(n, 31);
+        } else {
+            place_of(m0, n_first);
+            place_of(m0 + live - 1, n_last);
+            n_first = __builtin_amdgcn_readfirstlane(n_first);
+            n_last = __builtin_amdgcn_readfirstlane(n_last);
+        }
+        requested = request_threshold(p.ths, n_first);
+    }
 
     // ---- activation: row = pixel * PC + word of the tile; load i of the wave takes the rows (4*i + wave) * WIDE ... ------
     // (ragged: load i is word i % WORDS of the pixel 4 * (i / WORDS) + wave.  Code that runs once costs its instructions: with
@@ -112,7 +129,8 @@ __global__ __launch_bounds__(kConvThreads) void conv1x1_fused(const Fused1x1Args
                 off_lane = l * 16;
                 int image;
                 off = place_of(m0 + pixel, image);
-                th_row[i % (HANDED ? 1 : LOADS)] = lane_threshold(p.ths, image);
+                th_row[i % (HANDED ? 1 : LOADS)] = OWN ? (n_last - n_first > 1 ? lane_threshold(p.ths, image) : image == n_first ? 0.f : 1.f)
+                                                       : given_threshold(p.ths, image);
             } else {
                 const int row = last_row(row_of(i));
                 pixel = pixel_of(row);
@@ -125,7 +143,14 @@ __global__ __launch_bounds__(kConvThreads) void conv1x1_fused(const Fused1x1Args
             for (int e = 0; e < WIDE; e++) v[i][e] = w[e % 4];
         }
     }
-    const float th = HANDED ? lane_threshold(p.ths, n) : 0.f;
+    float th = 0.f;
+    if (HANDED) {
+        th = OWN ? span_threshold(p.ths, n, n_first, n_last, requested) : given_threshold(p.ths, n);
+    } else if (OWN && n_last - n_first <= 1) {
+        const float t_first = finish_threshold(p.ths, n_first, requested), t_last = n_last == n_first ? t_first : wave_threshold(p.ths, n_last);
+#pragma unroll
+        for (int i = 0; i < (HANDED ? 1 : LOADS); i++) th_row[i] = th_row[i] == 0.f ? t_first : t_last;
+    }
 
     // ---- weights: filter tile t of this wave --------------------------------------------------------
     const int n_wave = (blockIdx.y * 4 + wave) * tiles * 32;  // first filter of the wave
@@ -264,7 +289,7 @@ int fused_tiles(int PC, long blocks, int KN) { return PC >= 3 && blocks >= 1024 
 
 long fused_blocks(long M, int KN) { return (M + 31) / 32 * ((KN + 127) / 128); }
 
-template <int TYPE, int NP, bool CACHED>
+template <int TYPE, int NP, bool CACHED, bool OWN>
 hipError_t launch_fused_rows(const Fused1x1Args &a, hipStream_t stream)
 {
     const int PC = (a.C + kWordBits - 1) / kWordBits;
@@ -272,29 +297,32 @@ hipError_t launch_fused_rows(const Fused1x1Args &a, hipStream_t stream)
     const dim3 grid((unsigned)((a.M + 31) / 32), (unsigned)((a.KN + 128 * tiles - 1) / (128 * tiles)));
     const unsigned lds = 2 * NP * 32 * Planes<TYPE>::A * 8;
     if (a.C % kWordBits != 0 || (uintptr_t)a.x % 16 != 0) {
-        if constexpr (NP == 1) conv1x1_fused<TYPE, NP, kInputRagged, CACHED><<<grid, dim3(kConvThreads), lds, stream>>>(a);
+        if constexpr (NP == 1) conv1x1_fused<TYPE, NP, kInputRagged, CACHED, OWN><<<grid, dim3(kConvThreads), lds, stream>>>(a);
         else return hipErrorInvalidValue;
     } else if (NP >= 2 && PC % 4 == 0) {
-        if constexpr (NP >= 2) conv1x1_fused<TYPE, NP, kInputQuads, CACHED><<<grid, dim3(kConvThreads), lds, stream>>>(a);
+        if constexpr (NP >= 2) conv1x1_fused<TYPE, NP, kInputQuads, CACHED, OWN><<<grid, dim3(kConvThreads), lds, stream>>>(a);
     } else {
-        conv1x1_fused<TYPE, NP, kInputWords, CACHED><<<grid, dim3(kConvThreads), lds, stream>>>(a);
+        conv1x1_fused<TYPE, NP, kInputWords, CACHED, OWN><<<grid, dim3(kConvThreads), lds, stream>>>(a);
     }
     return hipGetLastError();
 }
 
-template <int TYPE, bool CACHED>
+template <int TYPE, bool CACHED, bool OWN>
 hipError_t launch_fused_words(const Fused1x1Args &a, hipStream_t stream)
 {
     const int PC = (a.C + kWordBits - 1) / kWordBits;
-    if (PC <= 2) return launch_fused_rows<TYPE, 1, CACHED>(a, stream);
-    if (PC <= 4) return launch_fused_rows<TYPE, 2, CACHED>(a, stream);
-    return launch_fused_rows<TYPE, 4, CACHED>(a, stream);
+    if (PC <= 2) return launch_fused_rows<TYPE, 1, CACHED, OWN>(a, stream);
+    if (PC <= 4) return launch_fused_rows<TYPE, 2, CACHED, OWN>(a, stream);
+    return launch_fused_rows<TYPE, 4, CACHED, OWN>(a, stream);
 }
 
 template <int TYPE>
 hipError_t launch_fused_type(const Fused1x1Args &a, hipStream_t stream)
 {
-    return ragged_rows_cached(a.M, a.KN) ? launch_fused_words<TYPE, true>(a, stream) : launch_fused_words<TYPE, false>(a, stream);
+    const bool cached = ragged_rows_cached(a.M, a.KN);
+    if constexpr (Planes<TYPE>::A == 2)
+        if (a.ths.splits > 0) return cached ? launch_fused_words<TYPE, true, true>(a, stream) : launch_fused_words<TYPE, false, true>(a, stream);
+    return cached ? launch_fused_words<TYPE, true, false>(a, stream) : launch_fused_words<TYPE, false, false>(a, stream);
 }
 
 }  // namespace
@@ -319,9 +347,10 @@ hipError_t launch_conv1x1_fused(int type, const float *x, const Thresholds &ths,
                                 int H, int W, int C, int KN, int s1, int s2, int OH, int OW, hipStream_t stream)
 {
     Fused1x1Args a;
-    a.x = x; a.ths = ths; a.qw = qw; a.btn = btn; a.y = y;
+    a.x = x; a.qw = qw; a.btn = btn; a.y = y;
     a.H = H; a.W = W; a.C = C; a.KN = KN; a.s1 = s1; a.s2 = s2; a.pixels = OH * OW; a.OW = OW;
     a.M = N * OH * OW;
+    a.ths = ordered(ths, (a.M + 31) / 32);
     const Div32 by_pixels = make_div32((uint32_t)a.pixels), by_ow = make_div32((uint32_t)OW);
     a.mul_pixels = by_pixels.mul;
     a.mul_ow = by_ow.mul;

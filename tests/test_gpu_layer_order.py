@@ -35,6 +35,26 @@ def test_layer_in_cache_order(size, nchw):
             assert torch.equal(layer(given), want.permute(0, 3, 1, 2) if nchw else want), conv_type
 
 
+# N, H, W, C, KN, stride: one launch, whose tiles of 32 pixels hold one image, two and several; every form of input; tiles from the 64th on
+ONE_LAUNCH = [(1, 56, 57, 64, 64, 1), (5, 23, 22, 128, 40, 1), (70, 8, 8, 64, 130, 1), (33, 8, 9, 64, 70, 2), (41, 8, 8, 128, 33, 3), (9, 13, 12, 256, 64, 2),
+              (31, 7, 7, 192, 96, 1), (23, 7, 7, 512, 100, 1), (6, 15, 14, 512, 64, 3), (17, 9, 10, 70, 48, 1), (35, 7, 7, 100, 65, 2)]
+
+
+@pytest.mark.parametrize("case", ONE_LAUNCH)
+def test_one_launch_adds_up_thresholds(case):
+    N, H, W, C, KN, stride = case
+    print(f"[case] one launch, own thresholds {case}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(C + N)
+    x = torch.randn((N, H, W, C), device="cuda", generator=g) * torch.logspace(-2, 2, N, device="cuda")[torch.randperm(N, device="cuda", generator=g)].view(N, 1, 1, 1)
+    ths = tab_amd.Threshold(x, N, 0.6)
+    q = tab_amd.QuantizeActivation(x, ths, 2, N, H, W, C)
+    for conv_type in (0, 1):
+        w = torch.randn((KN, C, 1, 1), device="cuda", generator=g)
+        layer = TABConv2d.from_float(w, conv_type, stride, 0, act_scale=0.6, data_format="NHWC")
+        want = tab_amd.Conv2dPacked(q, layer.QW, layer.BTN_W, conv_type, 0, 0, stride, stride, N, H, W, C, KN, 1, 1)
+        assert torch.equal(layer(x).flatten(), want.flatten()), conv_type
+
+
 # N, H, W, C: waves of 32 rows (the larger half) and of 8 that hold one image, two and many, the last of them short
 GIVEN = [(41000, 1, 1, 64), (9001, 1, 5, 64), (1400, 31, 1, 64), (1250, 3, 11, 64), (700, 3, 7, 192), (90, 1, 7, 64), (33, 1, 1, 64), (11, 3, 3, 128)]
 
