@@ -88,24 +88,24 @@ __global__ __launch_bounds__(kThreads) void count_finish(const int32_t *__restri
 }
 
 // The streaming path (tab_quantize_rows.h).
-template <int BITS, int LOADS = kLoadsPerLane>
+template <int BITS, int LOADS = kLoadsPerLane, bool OWN = false>
 __global__ __launch_bounds__(kThreads) void quantize_rows64(const floatx4 *__restrict__ x, const Thresholds ths, uint32_t *__restrict__ q, long rows,
                                                             long rows_per_item, Div32 div_item, int32_t *btn, long items)
 {
-    quantize_rows64_block<BITS, LOADS>(x, ths, q, rows, rows_per_item, div_item, in_eighths(blockIdx.x, ths.eighth));
+    quantize_rows64_block<BITS, LOADS, OWN>(x, ths, q, rows, rows_per_item, div_item, in_eighths(blockIdx.x, ths.eighth));
     const long row = (long)blockIdx.x * (4 * LOADS * kWavesPerBlock) + (threadIdx.x >> 6) * (4 * LOADS) + (threadIdx.x & 63);
     if ((threadIdx.x & 63) < 4 * LOADS) zero_counts(btn, items, row);
 }
 
 // Beside a convolution's weights, which the first workgroups lay out (kernels of their own: with the code for the weights in every
 // quantizer the short ones took 2-4 % longer).
-template <int BITS, int LOADS = kLoadsPerLane>
+template <int BITS, int LOADS = kLoadsPerLane, bool OWN = false>
 __global__ __launch_bounds__(kThreads) void quantize_rows64_weights(const floatx4 *__restrict__ x, const Thresholds ths, uint32_t *__restrict__ q,
                                                                     long rows, long rows_per_item, Div32 div_item, const WeightJob job)
 {
     uint32_t block = blockIdx.x;
     if (pack_weights(job, block)) return;
-    quantize_rows64_block<BITS, LOADS>(x, ths, q, rows, rows_per_item, div_item, in_eighths(block, ths.eighth));
+    quantize_rows64_block<BITS, LOADS, OWN>(x, ths, q, rows, rows_per_item, div_item, in_eighths(block, ths.eighth));
 }
 
 // The same row quantizer for a 1x1 convolution with stride and no padding, which reads only the
@@ -997,8 +997,11 @@ hipError_t launch_rows64_weights(const float *x, const Thresholds &ths, int form
             reinterpret_cast<const floatx4 *>(x), ordered(ths, (rows + rows_per_block - 1) / rows_per_block), reinterpret_cast<uint32_t *>(qx), rows, rows_per_item, div_item, job);
     };
     // (sizes of workgroups as in launch_quantize)
-    if (rows <= kSmallLaunchBlocks * 128) launch(format == 4 ? quantize_rows64_weights<4, 2> : format == 2 ? quantize_rows64_weights<2, 2> : quantize_rows64_weights<1, 2>, 32, 0);
-    else launch(format == 4 ? quantize_rows64_weights<4> : format == 2 ? quantize_rows64_weights<2> : quantize_rows64_weights<1>, 128, kStreamLds);
+    const bool own = ths.splits > 0;
+    if (rows <= kSmallLaunchBlocks * 128)
+        launch(format == 4 ? quantize_rows64_weights<4, 2> : format == 1 ? quantize_rows64_weights<1, 2> : own ? quantize_rows64_weights<2, 2, true> : quantize_rows64_weights<2, 2>, 32, 0);
+    else
+        launch(format == 4 ? quantize_rows64_weights<4> : format == 1 ? quantize_rows64_weights<1> : own ? quantize_rows64_weights<2, 8, true> : quantize_rows64_weights<2>, 128, kStreamLds);
     return hipGetLastError();
 }
 
@@ -1049,16 +1052,12 @@ hipError_t launch_quantize(const float *x, const Thresholds &ths, int bitwidth, 
             // a tensor too small to fill the chip with 128-row workgroups: 32 rows per workgroup, two loads per lane
             // (3.1 MB of fp32: 5.5 -> 4.2 us)
             const dim3 grid((unsigned)((rows + 8 * kWavesPerBlock - 1) / (8 * kWavesPerBlock)));
-            if (bitwidth == 2)
-                quantize_rows64<2, 2><<<grid, block, 0, stream>>>(x4, ordered(ths, grid.x), q32, rows, words_per_item, div_item, zeroed, items);
-            else
-                quantize_rows64<1, 2><<<grid, block, 0, stream>>>(x4, ordered(ths, grid.x), q32, rows, words_per_item, div_item, zeroed, items);
+            auto kernel = bitwidth == 1 ? quantize_rows64<1, 2> : ths.splits > 0 ? quantize_rows64<2, 2, true> : quantize_rows64<2, 2>;
+            kernel<<<grid, block, 0, stream>>>(x4, ordered(ths, grid.x), q32, rows, words_per_item, div_item, zeroed, items);
         } else {
             const dim3 grid((unsigned)blocks);
-            if (bitwidth == 2)
-                quantize_rows64<2><<<grid, block, kStreamLds, stream>>>(x4, ordered(ths, grid.x), q32, rows, words_per_item, div_item, zeroed, items);
-            else
-                quantize_rows64<1><<<grid, block, kStreamLds, stream>>>(x4, ordered(ths, grid.x), q32, rows, words_per_item, div_item, zeroed, items);
+            auto kernel = bitwidth == 1 ? quantize_rows64<1> : ths.splits > 0 ? quantize_rows64<2, 8, true> : quantize_rows64<2>;
+            kernel<<<grid, block, kStreamLds, stream>>>(x4, ordered(ths, grid.x), q32, rows, words_per_item, div_item, zeroed, items);
         }
     } else if (bitwidth == 2) {
         launch_quantize_tile<2>(x, ths, pixels, pixels_per_item, items, C, qx, zeroed, nullptr, weights, stream);

@@ -16,7 +16,8 @@ constexpr int kLoadsPerLane = 8;   // float4 loads in flight per lane
 // BITS = 1 or 2 (the reference's bit widths), or the format of conv type 4 or 5; LOADS = 8 (128 rows per
 // workgroup) for streaming, 2 for launches too small to fill the chip.
 // block: the workgroup's number among those that quantize.
-template <int BITS, int LOADS>
+// OWN: thresholds are partial sums to be added up (a form of its own: the code that is not run costs calls with given thresholds 2 to 4 %).
+template <int BITS, int LOADS, bool OWN>
 __device__ __forceinline__ void quantize_rows64_block(const floatx4 *__restrict__ x, const Thresholds &ths, uint32_t *__restrict__ q, long rows,
                                                       long rows_per_item, Div32 div_item, uint32_t block)
 {
@@ -33,8 +34,7 @@ __device__ __forceinline__ void quantize_rows64_block(const floatx4 *__restrict_
     // requested before x.
     const long item_first = div_item.mul ? (long)div32((uint32_t)row0, div_item) : row0 / rows_per_item;
     const long item_last = div_item.mul ? (long)div32((uint32_t)row_last, div_item) : row_last / rows_per_item;
-    const bool own = BITS == 2 && ths.splits > 0;
-    const floatx4 requested = own ? request_threshold(ths, item_first) : floatx4{};
+    const floatx4 requested = OWN ? request_threshold(ths, item_first) : floatx4{};
     // x and q from the wave's row on: 32-bit offsets from a scalar address leave registers for one more wave per SIMD
     const floatx4 *const src = x + row0 * 16;
     uint32_t *const dst = q + row0 * (BITS != 1 ? 4 : 2);
@@ -48,8 +48,8 @@ __device__ __forceinline__ void quantize_rows64_block(const floatx4 *__restrict_
         // a large one streams past them: non-temporal loads (plain ones are 8-11 % slower at 400 MB and more)
         v[u] = LOADS == 2 ? *at : __builtin_nontemporal_load(at);
     }
-    const float t_first = own ? finish_threshold(ths, item_first, requested) : given_threshold(ths, item_first);
-    const float t_last = item_last == item_first ? t_first : wave_threshold(ths, item_last);
+    const float t_first = OWN ? finish_threshold(ths, item_first, requested) : given_threshold(ths, item_first);
+    const float t_last = item_last == item_first ? t_first : OWN ? wave_threshold(ths, item_last) : given_threshold(ths, item_last);
 
     auto finish = [&](int u, float t) {
         const uint32_t r = u * 4 + sub;
@@ -68,12 +68,12 @@ __device__ __forceinline__ void quantize_rows64_block(const floatx4 *__restrict_
         const uint32_t border = item_last == item_first ? 4 * LOADS : (uint32_t)(item_last * rows_per_item - row0);  // where the second begins
 #pragma unroll
         for (int u = 0; u < LOADS; u++) finish(u, (uint32_t)(u * 4 + sub) < border ? t_first : t_last);
-    } else {  // items of fewer rows than the wave: their thresholds are given (partial sums are those of 64 rows and more)
+    } else if (!OWN) {  // items of fewer rows than the wave (partial sums are those of 64 rows and more)
         const uint32_t before = (uint32_t)(row0 - item_first * rows_per_item);  // rows of the first item in front of the wave
 #pragma unroll
         for (int u = 0; u < LOADS; u++) {
             const uint32_t at = before + min((uint32_t)(u * 4 + sub), live - 1);
-            finish(u, ths.values == nullptr ? 0.f : ths.values[item_first + at / (uint32_t)rows_per_item]);
+            finish(u, given_threshold(ths, item_first + at / (uint32_t)rows_per_item));
         }
     }
 }
