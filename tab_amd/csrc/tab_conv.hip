@@ -412,27 +412,25 @@ hipError_t launch_conv_mfma(int type, const ConvArgs &args, int shape, hipStream
 // cost_us (optional): the predicted duration of the chosen shape.
 int conv_mfma_shape(int type, const ConvArgs &a, float *cost_us)
 {
-    // K of at most nine words and packed output: the kernel with the weights resident in registers, whose epilogue
-    // thresholds a pixel's filters inside a lane, runs 1.4-2x faster than the tiled shapes once the launch is a few
-    // rounds of waves (N=256 56x56x64->64 3x3: 24 against 38 us) and level with them on small ones; with fp32 output
-    // both are bound by writing Y and measure within 5 % of each other, so the tiled shapes keep those launches
-    if (type <= 3 && a.G <= 9 && a.qy != nullptr && (a.M >= 65536 || a.G <= 2)) {
-        if (cost_us) *cost_us = 0.f;
-        return 7;
-    }
     const long kn64 = ((long)a.KN + 63) / 64 * 64;
     const long cus = device_compute_units();
     const bool narrow = conv_mfma_narrow(a);
-    // (packed output ranks the shapes as fp32 output does: the model's terms in Y also stand for what grows with M * KN)
+    // Packed output has a ranking of its own: with the one of fp32 output, and the kernel with the weights in registers wherever K is at
+    // most nine words and M at least 65536, 743 random layers took 6 % more than the best shapes' time; with this one 1.5 %.
+    // (types 4 and 5 are ranked as with fp32 output: they were not measured)
+    const bool packed = a.qy != nullptr && type <= 3;
     const float y_mb = (float)a.M * (float)a.KN * 4e-6f;
     const float words = type == 5 ? 0.5f * (float)a.G : (float)a.G;  // of 64 elements
     int best = 2;
     float best_cost = 0.f;
     bool any = false;
-    for (int i = 0; i < kConvShapes; i++) {
-        const int shape = kConvShapeIds[i];
-        const int bm = kConvShapeTile[i][0], bn = kConvShapeTile[i][1], held = kConvShapeTile[i][2];
+    for (int i = 0; i < (packed ? kConvPackedShapes : kConvShapes); i++) {
+        const int shape = packed ? kConvPackedIds[i] : kConvShapeIds[i];
+        const int *const tile = packed ? kConvPackedTile[i] : kConvShapeTile[i];
+        const float *const coefficients = packed ? kConvPackedCost[type][i] : kConvShapeCost[type][i];
+        const int bm = tile[0], bn = tile[1], held = tile[2];
         if (bn >= 2 * kn64) continue;
+        if (shape == 7 && a.G > 9) continue;
         if (shape == 3 && a.qy != nullptr) continue;        // the packed epilogues need tiles 64 filters wide
         if (shape >= 8 && a.PC % 2 != 0) continue;          // the split-K shapes move whole pairs of words inside a tap
         const long tiles = (long)((a.M + bm - 1) / bm) * ((a.KN + bn - 1) / bn);
@@ -448,14 +446,14 @@ int conv_mfma_shape(int type, const ConvArgs &a, float *cost_us)
             if (shape == 11 && a.PC % 4 != 0) continue;                       // the 128x256 tiles take four-word chunks inside a tap
             const float f[kConvShapeFeatures] = {(float)a.G * (float)whole, (float)a.G * (float)quarters, (float)quarters, (float)whole, y_mb, y_mb,
                                                  1.f, 1.f, 0.f};
-            for (int k = 0; k < kConvShapeFeatures; k++) cost += kConvShapeCost[type][i][k] * f[k];
+            for (int k = 0; k < kConvShapeFeatures; k++) cost += coefficients[k] * f[k];
             floor_us = 1.f + (float)(4 * pieces * whole + 4 * quarters) * words * (32.f / 4.f / 2400.f);
         } else {
             const float n = (float)((tiles + cus - 1) / cus), rounds = (float)(((tiles + cus - 1) / cus + held - 1) / held);
             const float busy = tiles >= cus ? 1.f : (float)tiles / (float)cus;
             const float f[kConvShapeFeatures] = {(float)a.G * n, (float)a.G * rounds, rounds, n, y_mb, y_mb * busy, busy, 1.f,
                                                  a.G <= 9 ? y_mb : 0.f};
-            for (int k = 0; k < kConvShapeFeatures; k++) cost += kConvShapeCost[type][i][k] * f[k];
+            for (int k = 0; k < kConvShapeFeatures; k++) cost += coefficients[k] * f[k];
             // the busiest CU's n tiles of (bm/32)(bn/32) MFMA tiles x words, 32 cycles each on four SIMDs at 2.4 GHz, and a launch
             floor_us = 1.f + n * (float)(bm / 32 * (bn / 32)) * words * (32.f / 4.f / 2400.f);
         }

@@ -27,6 +27,12 @@ whose predictions can cross or go negative where nothing was measured).  A shape
 (64-rounded) filter count is not a candidate.  The script prints the regret of the model's choice against the best measured shape:
 fitted on everything, and with each set held out in turn.
 
+Packed output has coefficients of its own, for types 0..3, from conv_packed_timings.txt (743 random layers): an epilogue that
+writes a bit per filter and pixel favours wider tiles than one that writes a float, and with the coefficients of fp32 output the
+choices took 6 % more than the best shapes' (with its own 1.6 % fitted, 1.7 % with an eighth of the layers held out in turn).  There the
+kernel with the weights resident in registers (shape 7, a wave per 64 pixels x 64 filters, four to a workgroup) competes with the
+tiles where K is at most nine words, and 32x32 tiles do not exist.
+
     python tab_amd/tuning/fit_conv_shape_model.py        # needs numpy only"""
 import collections
 import os
@@ -43,6 +49,8 @@ MIXED = (10, 11)
 PLANES = {0: 4, 1: 3, 2: 3, 3: 2, 4: 4, 5: 2}  # bit planes of activation + weight operand, per type
 IDS = sorted(SHAPES)
 NFEAT = 9
+PACKED_SHAPES = {**{s: v for s, v in SHAPES.items() if s != 3}, 7: (256, 64, 2)}
+PACKED_IDS = sorted(PACKED_SHAPES)
 
 
 def parse(path):
@@ -63,6 +71,46 @@ def parse(path):
     return rows
 
 
+def parse_packed(path):
+    rows = []
+    for line in open(path):
+        m = re.match(r"type (\d) out (\d) N(\d+)_(\d+)x(\d+)x(\d+)->(\d+)_k(\d+)x(\d+)_p(\d)\.(\d)_s(\d) \| (.*)", line)
+        if not m:
+            continue
+        t, _, N, H, W, C, KN, kh, kw, p1, p2, s = map(int, m.groups()[:12])
+        times = {int(a.split(":")[0]): float(a.split(":")[1]) for a in m.group(13).split()}
+        PC = (C + 63) // 64
+        r = dict(set="packed", type=t, M=N * ((H + 2 * p1 - kh + 1) // s) * ((W + 2 * p2 - kw + 1) // s), KN=KN, G=kh * kw * PC, PC=PC, times=times,
+                 name=line.split()[4])
+        r["times"] = {s: v for s, v in times.items() if packed_eligible(r, s)}
+        rows.append(r)
+    return [r for r in rows if r["times"]]
+
+
+def packed_eligible(r, s):
+    return r["G"] <= 9 if s == 7 else s != 3 and eligible(r, s)
+
+
+def packed_fit(rows):
+    from scipy.optimize import nnls
+
+    coef = {}
+    for s in PACKED_IDS:
+        for t in range(4):
+            some = [r for r in rows if r["type"] == t and s in r["times"]]
+            y = np.array([r["times"][s] for r in some])
+            coef[(t, s)] = nnls(np.array([features(r, s) for r in some]) / y[:, None], np.ones(len(y)))[0]
+    return coef
+
+
+def packed_choose(coef, r):
+    return min(r["times"], key=lambda s: (float(coef[(r["type"], s)] @ np.array(features(r, s))), s))
+
+
+def packed_regret(rows, choices):
+    return sum(r["times"][c] for r, c in zip(rows, choices)) / sum(min(r["times"].values()) for r in rows) - 1
+
+
 def mixed_rounds(r, s):
     BM, BN, _ = SHAPES[s]
     tiles = -(-r["M"] // BM) * -(-r["KN"] // BN)
@@ -77,7 +125,7 @@ def eligible(r, s):
 
 
 def features(r, s):
-    BM, BN, held = SHAPES[s]
+    BM, BN, held = PACKED_SHAPES[s] if s == 7 else SHAPES[s]
     Y = r["M"] * r["KN"] * 4e-6
     if s in MIXED:
         whole, quarters = mixed_rounds(r, s)
@@ -140,6 +188,16 @@ def main():
                 held_best += best_time(r)
     print(f"{len(rows)} cases; regret of the model's choice, fitted on all: {total:.2%} ({', '.join(f'{k} {v:.1%}' for k, v in sorted(per.items()))})")
     print(f"each set held out of the fit in turn: {held_chosen / held_best - 1:.2%} ({', '.join(f'{k} {v:.1%}' for k, v in sorted(held.items()))})")
+    packed = parse_packed(os.path.join(HERE, "conv_packed_timings.txt"))
+    packed_coef = packed_fit(packed)
+    packed_all = packed_regret(packed, [packed_choose(packed_coef, r) for r in packed])
+    choices = [None] * len(packed)
+    for k in range(8):
+        c = packed_fit([r for i, r in enumerate(packed) if i % 8 != k])
+        for i in range(k, len(packed), 8):
+            choices[i] = packed_choose(c, packed[i])
+    packed_held = packed_regret(packed, choices)
+    print(f"packed output, {len(packed)} cases: {packed_all:.2%}; an eighth held out in turn: {packed_held:.2%}")
     out = os.path.join(os.path.dirname(HERE), "csrc", "tab_conv_shape_model.h")
     import datetime
     import subprocess
@@ -166,6 +224,19 @@ def main():
             f.write("    {\n")
             for s_ in IDS:
                 f.write("        {" + ", ".join(("%.6g" % v if "." in "%.6g" % v or "e" in "%.6g" % v else "%.6g.0" % v) + "f" for v in coef[(t, s_)]) + "},\n")
+            f.write("    },\n")
+        f.write("};\n\n")
+        f.write("// The same for packed output, types 0..3, from tab_amd/tuning/conv_packed_timings.txt; shape 7 is the kernel with the weights in\n")
+        f.write(f"// registers (K of at most nine words).  Regret over the {len(packed)} fitted cases: {packed_all:.2%}; with an eighth of them held out in\n")
+        f.write(f"// turn: {packed_held:.2%}.\n")
+        f.write(f"constexpr int kConvPackedShapes = {len(PACKED_IDS)};\n")
+        f.write("constexpr int kConvPackedIds[kConvPackedShapes] = {" + ", ".join(str(i) for i in PACKED_IDS) + "};\n")
+        f.write("constexpr int kConvPackedTile[kConvPackedShapes][3] = {" + ", ".join("{%d, %d, %d}" % PACKED_SHAPES[s] for s in PACKED_IDS) + "};\n")
+        f.write("constexpr float kConvPackedCost[4][kConvPackedShapes][kConvShapeFeatures] = {\n")
+        for t in range(4):
+            f.write("    {\n")
+            for s_ in PACKED_IDS:
+                f.write("        {" + ", ".join(("%.6g" % v if "." in "%.6g" % v or "e" in "%.6g" % v else "%.6g.0" % v) + "f" for v in packed_coef[(t, s_)]) + "},\n")
             f.write("    },\n")
         f.write("};\n\n}  // namespace tab\n")
     print("wrote", out)
