@@ -125,7 +125,7 @@ void tab_internal_set_tail_round(int workgroups) { tab::set_tail_round(workgroup
 /* Test hook, absent from include/tab_amd.h: the compute units that the rules choosing a kernel count; 0 = the device's. */
 void tab_internal_set_compute_units(int units) { tab::set_compute_units(units); }
 
-/* Test hook, absent from include/tab_amd.h: convolutions from fp32 take this shape (12 .. 16) of the kernel that keeps the input
+/* Test hook, absent from include/tab_amd.h: convolutions from fp32 take this shape (12 .. 18) of the kernel that keeps the input
  * patch in LDS wherever its patch fits; tab_set_conv_kernel ends it. */
 void tab_internal_force_patch(int shape) { tab::force_conv_tile(9, shape); }
 
@@ -362,7 +362,7 @@ int tab_conv2d_packed_out_const(const int64_t *dev_QX, const int64_t *dev_QW, co
                        nullptr, nullptr, out_threshold, out_bitwidth, dev_QY, stream);
 }
 
-/* Test hook, absent from include/tab_amd.h: the shape (12 .. 16) of the kernel that keeps the input patch in LDS which the library would
+/* Test hook, absent from include/tab_amd.h: the shape (12 .. 18) of the kernel that keeps the input patch in LDS which the library would
  * pick for a convolution from fp32, -1 for another kernel; what[0..2]: words of a chunk, pixels and LDS bytes of its patch. */
 int tab_internal_conv_patch_shape(int type, int padding1, int padding2, int stride1, int stride2, int N, int H, int W, int C, int KN, int KH,
                                   int KW, int *what, size_t *weight_bytes)

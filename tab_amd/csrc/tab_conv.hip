@@ -476,11 +476,12 @@ int conv_mfma_shape(int type, const ConvArgs &a, float *cost_us)
 
 // The kernel that keeps the input patch in LDS, against the tiled one that conv_mfma_shape picks: the shape with the lowest predicted
 // duration, if that is 7 % below what the tiled kernel is predicted to take (tab_conv_patch_model.h; both are linear forms with
-// non-negative coefficients, fitted to 1944 measured launches: over them the choices take 0.93 of the tiled kernels' time, the
-// better one of each 0.915).  Not for 1x1 kernels, which read every pixel for one tap only, nor for at most 32 filters, half of
+// non-negative coefficients, fitted to 1970 measured launches: over them the choices take 0.946 of the tiled kernels' time, in
+// total 0.907, the better one of each 0.931 and 0.893).  Not for 1x1 kernels, which read every pixel for one tap only, nor for at most 32 filters, half of
 // whose tiles would be work for nothing, nor for launches below 128 tiles of 64x64, which last as long as one tile's chain of waits
 // (no win below 49 such tiles, one in eight from there to 120).  Measured, tiled / patch, conv kernel alone in the kernel trace:
-// N=64 14x14x256 levels 13.6 / 10.6 us, N=256 28x28x512->512 BNN 224 / 196, N=32 56x56x64 TNN 10.3 / 8.5.
+// N=64 14x14x256 levels 13.6 / 10.6 us, N=256 28x28x512->512 BNN 224 / 196, N=32 56x56x64 TNN 10.3 / 8.5,
+// N=32 56x56x256->256 TNN 41.5 / 35 (64x256 tiles).
 PatchPlan conv_patch_plan(int type, const ConvArgs &a)
 {
     PatchPlan plan = {-1, 0, 0, 0, -1, 0};

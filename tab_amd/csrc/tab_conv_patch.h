@@ -48,9 +48,14 @@ inline int patch_chunk(const ConvArgs &a, int rows, int most, int *npix, int *ld
 }
 
 // The kernel's shapes: rows and filters of a workgroup's tile, MFMA tiles of a wave, workgroups a CU holds by their registers.
+// What bounds the loop of a wide launch is the operands' way out of LDS, TM reads of 1 KB for TM * TN multiplications of a wave, and the
+// patch, which each tile of the filters fetches and expands again: 64 rows x 256 filters, waves of 2 x 2 MFMA tiles, read half as much per
+// multiplication as 128 x 128 with waves of 4 x 1 and a patch once for 256 filters (N=32 56x56x256->256 TNN 36.6 -> 33.1 us, conv kernel
+// alone; N=256 14x14x256->512 stride 2 16.2 -> 13.7).  64 x 128 tiles, waves of 2 x 1, leave launches of few tiles a better last round than
+// 128 x 64 (N=64 56x56x64->128 stride 2 8.9 -> 8.4).  128 x 128 with waves of 2 x 2 and 128 x 256 won nowhere by more than 3 %.
 struct PatchTile { int rows, filters, wave_tiles, held; };
-constexpr int kPatchShapes = 5;
-constexpr PatchTile kPatchTile[kPatchShapes] = {{256, 128, 8, 2}, {128, 128, 4, 3}, {128, 64, 2, 4}, {64, 64, 1, 4}, {256, 64, 4, 3}};
+constexpr int kPatchShapes = 7;
+constexpr PatchTile kPatchTile[kPatchShapes] = {{256, 128, 8, 2}, {128, 128, 4, 3}, {128, 64, 2, 4}, {64, 64, 1, 4}, {256, 64, 4, 3}, {64, 256, 4, 3}, {64, 128, 2, 4}};
 
 // What the predicted durations (tab_conv_patch_model.h) are linear in; the fit script states the same.
 constexpr int kPatchFeatures = 13, kTiledFeatures = 10;

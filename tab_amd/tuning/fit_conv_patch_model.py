@@ -1,6 +1,6 @@
 """Coefficients of the rule that takes a convolution to the kernel that keeps its input patch in LDS (tab_conv_patch_model.h), by
 non-negative least squares of the relative error on conv_patch_timings.txt: the conv kernel alone, in graph replays, on random
-packed operands, as the tiled kernels run it by their own choice ("tiled") and in the patch kernel's shapes 12 .. 16.
+packed operands, as the tiled kernels run it by their own choice ("tiled") and in the patch kernel's shapes 12 .. 18.
 
     python tab_amd/tuning/fit_conv_patch_model.py            fit on everything, write the header
     python tab_amd/tuning/fit_conv_patch_model.py --check    fit on one half of the geometries, regret on the other
@@ -16,7 +16,8 @@ from scipy.optimize import nnls
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(os.path.dirname(HERE), "csrc")
 DATA = os.path.join(HERE, "conv_patch_timings.txt")
-SHAPES = {12: (256, 128, 8, 2), 13: (128, 128, 4, 3), 14: (128, 64, 2, 4), 15: (64, 64, 1, 4), 16: (256, 64, 4, 3)}  # kPatchTile
+SHAPES = {12: (256, 128, 8, 2), 13: (128, 128, 4, 3), 14: (128, 64, 2, 4), 15: (64, 64, 1, 4), 16: (256, 64, 4, 3),
+          17: (64, 256, 4, 3), 18: (64, 128, 2, 4)}  # kPatchTile
 CUS, ITEMS, LDS = 256, {1: 3, 2: 3, 4: 2}, 64 * 1024
 MARGIN, WEIGHTS_US = 0.93, 0.5  # the weights' part of the quantizer's launch, measured 0.1-0.8 us
 
@@ -134,7 +135,7 @@ def write_header(tiled, patch):
 
     with open(os.path.join(CSRC, "tab_conv_patch_model.h"), "w") as f:
         f.write("// Written by tab_amd/tuning/fit_conv_patch_model.py from conv_patch_timings.txt: microseconds, linear in patch_features and\n"
-                "// tiled_features (tab_conv_patch.h), per type 0 .. 4 and, for the patch kernel, shape 12 .. 16.\n#pragma once\n"
+                "// tiled_features (tab_conv_patch.h), per type 0 .. 4 and, for the patch kernel, shape 12 .. 18.\n#pragma once\n"
                 "#include \"tab_conv_patch.h\"\n\nnamespace tab {\n\n")
         f.write("constexpr float kTiledCost[5][kTiledFeatures] = {\n" + "".join("    {%s},\n" % rows_of(tiled[t]) for t in range(5)) + "};\n\n")
         f.write("constexpr float kPatchCost[5][kPatchShapes][kPatchFeatures] = {\n")

@@ -12,7 +12,7 @@ import pytest
 from tab_amd import _capi
 
 TUNING = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "tab_amd", "tuning")
-ROWS = {12: 256, 13: 128, 14: 128, 15: 64, 16: 256}
+ROWS = {12: 256, 13: 128, 14: 128, 15: 64, 16: 256, 17: 64, 18: 64}
 
 
 @pytest.fixture(scope="module")

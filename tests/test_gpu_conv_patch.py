@@ -12,7 +12,7 @@ from tab_amd import nn as tab_nn
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = range(12, 17)
+SHAPES = range(12, 19)
 CASES = [
     # N, H, W, C, KN, KH, KW, p1, p2, s1, s2
     (2, 14, 14, 128, 64, 3, 3, 1, 1, 1, 1), (3, 7, 7, 64, 70, 3, 3, 1, 1, 1, 1), (2, 13, 11, 192, 130, 3, 3, 1, 0, 1, 1),
