@@ -418,7 +418,13 @@ int conv_mfma_shape(int type, const ConvArgs &a, float *cost_us)
     // Packed output has a ranking of its own: with the one of fp32 output, and the kernel with the weights in registers wherever K is at
     // most nine words and M at least 65536, 743 random layers took 6 % more than the best shapes' time; with this one 1.5 %.
     // (types 4 and 5 are ranked as with fp32 output: they were not measured)
-    const bool packed = a.qy != nullptr && type <= 3;
+    // Below 128 tiles of 64x64, where none of those layers lies, the ranking of fp32 output stays (one image of 41x41x192 through four
+    // layers: 26.1 us with it, 26.7 with the other), and weights in registers for K of at most two words.
+    const bool packed = a.qy != nullptr && type <= 3 && (long)((a.M + 63) / 64) * (kn64 / 64) >= 128;
+    if (a.qy != nullptr && type <= 3 && !packed && a.G <= 2) {
+        if (cost_us) *cost_us = 0.f;
+        return 7;
+    }
     const float y_mb = (float)a.M * (float)a.KN * 4e-6f;
     const float words = type == 5 ? 0.5f * (float)a.G : (float)a.G;  // of 64 elements
     int best = 2;
