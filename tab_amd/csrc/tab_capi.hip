@@ -379,21 +379,17 @@ int tab_internal_conv_patch_shape(int type, int padding1, int padding2, int stri
     return plan.shape;
 }
 
-/* Test hook, absent from include/tab_amd.h: the shape that tab_internal_force_patch holds, on an activation already packed; fp32
- * output to dev_Y, or packed to dev_QY (out_bitwidth planes, one threshold).  what: 1 = lay the weights out in `weights`
- * (weight_bytes bytes), 2 = convolve with those there, 3 = both. */
+/* Test hook, absent from include/tab_amd.h: the shape that tab_internal_force_patch holds, on an activation already packed.
+ * what: 1 = lay the weights out in `weights` (weight_bytes bytes), 2 = convolve with those there, 3 = both. */
 int tab_internal_conv_patch(const int64_t *dev_QX, const int64_t *dev_QW, const int32_t *dev_btn, int type, int padding1, int padding2,
-                            int stride1, int stride2, int N, int H, int W, int C, int KN, int KH, int KW, float *dev_Y, float out_threshold,
-                            int out_bitwidth, int64_t *dev_QY, void *weights, size_t weight_bytes, int what, void *stream)
+                            int stride1, int stride2, int N, int H, int W, int C, int KN, int KH, int KW, float *dev_Y, void *weights,
+                            size_t weight_bytes, int what, void *stream)
 {
     ConvShape s;
     int rc = check_conv(type, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, &s);
-    if (rc == TAB_OK) rc = check_conv_pointers(s, type, dev_QX, dev_QW, dev_btn, dev_Y, dev_QY);
+    if (rc == TAB_OK) rc = check_conv_pointers(s, type, dev_QX, dev_QW, dev_btn, dev_Y, nullptr);
     if (rc != TAB_OK) return rc;
     tab::ConvArgs a = conv_args(s, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, dev_QX, dev_QW, dev_btn, dev_Y);
-    a.qy = reinterpret_cast<uint32_t *>(dev_QY);
-    a.out_th = out_threshold;
-    a.out_bits = out_bitwidth;
     const tab::PatchPlan plan = tab::conv_patch_plan(type, a);
     if (plan.shape < 0) return fail(TAB_ERR_BAD_SHAPE, "the patch does not fit");
     if (!weights || weight_bytes < plan.weight_bytes) return fail(TAB_ERR_WORKSPACE, "weights take %zu bytes", plan.weight_bytes);

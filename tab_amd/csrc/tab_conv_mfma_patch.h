@@ -45,15 +45,15 @@ __device__ __forceinline__ Item<PL> load_item_at(__amdgpu_buffer_rsrc_t rsrc, ui
 
 // ConvParams with other contents where this kernel has no use for the usual ones: G = pixels of the patch (the stride between
 // planes), nchunks = KH, the magics of PC and KW = those of PW and PH.
-template <int TYPE, int WM, int WN, int TM, int TN, int KC, bool PACKED>
+template <int TYPE, int WM, int WN, int TM, int TN, int KC>
 __global__ __launch_bounds__(kConvThreads) __attribute__((amdgpu_waves_per_eu(TM * TN >= 8 ? 2 : (TM * TN >= 4 ? 3 : 4))))
-void conv_mfma_patch(const ConvParamsOf<PACKED> k)
+void conv_mfma_patch(const ConvParams k)
 {
     static_assert(WM * WN * 64 == kConvThreads, "four waves");
     constexpr int APL = Planes<TYPE>::A, BPL = Planes<TYPE>::B;
     constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN;
     constexpr int NM = TM * TN;
-    ConvArgs p = unpack_conv<TYPE, PACKED, BM, BN>(k);
+    ConvArgs p = unpack_conv<TYPE, false, BM, BN>(k);
     const int npix = p.G, KH = p.nchunks;
     const int taps = KH * p.KW;
     const int PW = (p.OW - 1) * p.s2 + p.KW, PH = (p.OH - 1) * p.s1 + KH;
@@ -227,8 +227,7 @@ void conv_mfma_patch(const ConvParamsOf<PACKED> k)
     };
     auto multiply = [&](int i, int set) {
         const int mt = i / TN, nt = i % TN;
-        acc[mt][nt] = PACKED ? __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(bf[set][nt], af[set][mt], acc[mt][nt], 4, 4, 0, 0, 0, 0)
-                             : __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(af[set][mt], bf[set][nt], acc[mt][nt], 4, 4, 0, 0, 0, 0);
+        acc[mt][nt] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(af[set][mt], bf[set][nt], acc[mt][nt], 4, 4, 0, 0, 0, 0);
     };
 
     // byte offset of the tap to come in a plane, and its column
@@ -325,12 +324,7 @@ void conv_mfma_patch(const ConvParamsOf<PACKED> k)
     }
     scale_sums<TYPE>(acc);
     const int wave_m0 = m0 + wm * (32 * TM), wave_n0 = n0 + wn * (32 * TN);
-    if constexpr (PACKED) {
-        if (TYPE == 2) __syncthreads();  // BTN hands its biases round through LDS: not before every wave has read its last operands
-        conv_mfma_epilogue_packed<TYPE, TM, TN, KC>(p, acc, b_nonzero, wave_m0, wave_n0, lane, lds + wave * (32 * TN), p.G);
-    } else {
-        conv_mfma_epilogue<TYPE, TM, TN, KC, 1>(p, acc, b_nonzero, wave_m0, wave_n0, lane, 0, nullptr, p.G);
-    }
+    conv_mfma_epilogue<TYPE, TM, TN, KC, 1>(p, acc, b_nonzero, wave_m0, wave_n0, lane, 0, nullptr, p.G);
 }
 
 template <int TYPE, int WM, int WN, int TM, int TN, int KC>
@@ -344,20 +338,14 @@ hipError_t launch_patch_chunk(ConvArgs a, int npix, int lds_bytes, hipStream_t s
     a.div_kw = make_fastdiv((uint32_t)((a.OH - 1) * a.s1 + a.KH));
     a.G = npix;
     a.nchunks = a.KH;
-    if (a.qy != nullptr) {
-        if constexpr (WN * TN % 2 == 0)
-            conv_mfma_patch<TYPE, WM, WN, TM, TN, KC, true><<<dim3((unsigned)blocks), dim3(kConvThreads), lds_bytes, stream>>>(pack_conv<TYPE, true>(a));
-        else
-            return hipErrorInvalidValue;
-    } else {
-        conv_mfma_patch<TYPE, WM, WN, TM, TN, KC, false><<<dim3((unsigned)blocks), dim3(kConvThreads), lds_bytes, stream>>>(pack_conv<TYPE, false>(a));
-    }
+    conv_mfma_patch<TYPE, WM, WN, TM, TN, KC><<<dim3((unsigned)blocks), dim3(kConvThreads), lds_bytes, stream>>>(pack_conv<TYPE, false>(a));
     return hipGetLastError();
 }
 
 template <int TYPE, int WM, int WN, int TM, int TN>
 hipError_t launch_patch(const ConvArgs &a, hipStream_t stream)
 {
+    if (a.qy != nullptr) return hipErrorInvalidValue;  // fp32 output only: packed output comes without room for the weights
     int npix = 0, lds_bytes = 0;
     constexpr int MOST = patch_most_words(TM * TN);
     switch (patch_chunk(a, 32 * WM * TM, MOST, &npix, &lds_bytes)) {
