@@ -375,19 +375,21 @@ struct PixelRun {
     long n, s, pixel;  // image, first pixel in the image, first pixel counted through all images
     int repeated;      // pixels at the run's start that the run before it has too (the per-image numbering only)
 
-    // run `i` counted through all images; past the last one: the last one again, with the same results
-    __device__ __forceinline__ PixelRun(long i, int N, long HW) : repeated(0)
+    // run `i` counted through all images; past the last one: the last one again, with the same results.  by_image divides by
+    // the pixels of an image (EVEN) or its runs; mul == 0 says that they reach 2^31 and the division takes 64 bits, which every
+    // wave waits for before it can request a pixel
+    __device__ __forceinline__ PixelRun(long i, int N, long HW, Div32 by_image) : repeated(0)
     {
         if (EVEN) {
             const long total = N * HW;
             pixel = i * VEC < total ? i * VEC : total - VEC;
-            n = pixel / HW;
+            n = by_image.mul ? (long)div32((uint32_t)pixel, by_image) : pixel / HW;
             s = pixel - n * HW;
         } else {
             const long per_image = (HW + VEC - 1) / VEC;
             const long runs = N * per_image;
             if (i >= runs) i = runs - 1;
-            n = i / per_image;
+            n = by_image.mul ? (long)div32((uint32_t)i, by_image) : i / per_image;
             s = (i - n * per_image) * VEC;
             if (s > HW - VEC) s = HW - VEC;
             pixel = n * HW + s;
@@ -546,11 +548,11 @@ __device__ __forceinline__ int quantize_nchw_unit(const float *__restrict__ x, c
 
 template <int BITS, int VEC, int SPLIT, bool NT = false>
 __global__ __launch_bounds__(kThreads) void quantize_nchw(const float *__restrict__ x, const Thresholds ths,
-                                                          uint64_t *__restrict__ q, int N, int C, long HW, int PC, int32_t *btn)
+                                                          uint64_t *__restrict__ q, int N, int C, long HW, int PC, Div32 by_image, int32_t *btn)
 {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t block = in_eighths(blockIdx.x, ths.eighth);
-    const PixelRun<VEC> run((block / PC * (kWavesPerBlock / SPLIT) + wave / SPLIT) * 64L + (threadIdx.x & 63), N, HW);
+    const PixelRun<VEC> run((block / PC * (kWavesPerBlock / SPLIT) + wave / SPLIT) * 64L + (threadIdx.x & 63), N, HW, by_image);
     quantize_nchw_unit<BITS, VEC, SPLIT, NT>(x, ths, q, run, C, HW, PC, block % PC);
     if (wave % SPLIT == 0) zero_counts(btn, N, run.pixel, VEC);
 }
@@ -558,13 +560,13 @@ __global__ __launch_bounds__(kThreads) void quantize_nchw(const float *__restric
 // Beside a convolution's weights.
 template <int BITS, int VEC, int SPLIT, bool NT = false>
 __global__ __launch_bounds__(kThreads) void quantize_nchw_weights(const float *__restrict__ x, const Thresholds ths, uint64_t *__restrict__ q, int N,
-                                                                  int C, long HW, int PC, const WeightJob job)
+                                                                  int C, long HW, int PC, Div32 by_image, const WeightJob job)
 {
     uint32_t block = blockIdx.x;
     if (pack_weights(job, block)) return;
     block = in_eighths(block, ths.eighth);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const PixelRun<VEC> run((block / PC * (kWavesPerBlock / SPLIT) + wave / SPLIT) * 64L + (threadIdx.x & 63), N, HW);
+    const PixelRun<VEC> run((block / PC * (kWavesPerBlock / SPLIT) + wave / SPLIT) * 64L + (threadIdx.x & 63), N, HW, by_image);
     quantize_nchw_unit<BITS, VEC, SPLIT, NT>(x, ths, q, run, C, HW, PC, block % PC);
 }
 
@@ -600,7 +602,7 @@ __global__ __launch_bounds__(kThreads) void quantize_nchw_count(const float *__r
 // WEIGHTS: a convolution's weights beside (then without counts).
 template <int BITS, int U, bool EVEN, bool COUNT = false, bool WEIGHTS = false>
 __global__ __launch_bounds__(64, BITS == 1 ? (U == 4 ? 4 : 7) : (U == 4 ? 1 : 4)) void quantize_nchw_gather(const float *__restrict__ x, const Thresholds ths,
-                                                                 uint64_t *__restrict__ q, int N, int C, long HW, int PC,
+                                                                 uint64_t *__restrict__ q, int N, int C, long HW, int PC, Div32 by_image,
                                                                  typename std::conditional<WEIGHTS, WeightJob, int32_t *>::type extra)
 {
     static_assert(!COUNT || (BITS == 2 && !EVEN), "counts of two planes; runs of one image are numbered for any plane size");
@@ -624,7 +626,7 @@ __global__ __launch_bounds__(64, BITS == 1 ? (U == 4 ? 4 : 7) : (U == 4 ? 1 : 4)
     const int pc0 = (unit % groups) * U;
     const int lane = threadIdx.x;
     const PixelRun<VEC, EVEN> run = COUNT ? PixelRun<VEC, EVEN>((long)(unit / groups) * 64 + lane, image, HW, std::true_type())
-                                          : PixelRun<VEC, EVEN>((long)(unit / groups) * 64 + lane, N, HW);
+                                          : PixelRun<VEC, EVEN>((long)(unit / groups) * 64 + lane, N, HW, by_image);
     // The U words are U * 64 consecutive channels: batches of kInFlight channels, the next batch's loads issued before
     // the compares of this one (two register buffers), so the memory pipe never waits for the packing.
     const int cbase = pc0 * kWordBits;
@@ -1085,13 +1087,14 @@ hipError_t launch_quantize_nchw(const float *x, const Thresholds &ths, int bitwi
     const long runs = N * ((HW + 3) / 4);
     const bool counted = btn && bitwidth == 2 && (count_workspace || (words_per_item <= 64 && PC <= kOneSliceUnits)) &&
                          N * (HW / 4 + 1) * PC < 0x7fffffffL;
-    auto launch = [&](auto kernel, long blocks, int threads) {
-        kernel<<<dim3((unsigned)blocks), dim3(threads), 0, stream>>>(x, ordered(ths, blocks), qx, N, C, HW, PC, zeroed);
+    auto by_image = [&](long per_image) { return N * per_image < 0x7fffffffL ? make_div32((uint32_t)per_image) : Div32{0, 0}; };
+    auto launch = [&](auto kernel, long blocks, int threads, long per_image) {
+        kernel<<<dim3((unsigned)blocks), dim3(threads), 0, stream>>>(x, ordered(ths, blocks), qx, N, C, HW, PC, by_image(per_image), zeroed);
     };
-    auto launch_weights = [&](auto kernel, long blocks, int threads) {
+    auto launch_weights = [&](auto kernel, long blocks, int threads, long per_image) {
         WeightJob job = *weights;
         job.blocks *= kThreads / threads;
-        kernel<<<dim3((unsigned)blocks + job.blocks), dim3(threads), 0, stream>>>(x, ordered(ths, blocks), qx, N, C, HW, PC, job);
+        kernel<<<dim3((unsigned)blocks + job.blocks), dim3(threads), 0, stream>>>(x, ordered(ths, blocks), qx, N, C, HW, PC, by_image(per_image), job);
     };
     // PC even, enough pixels for a wave on every SIMD: the form that gathers each wave's output into whole runs
     const int unit = PC % 4 == 0 ? 4 : PC % 2 == 0 ? 2 : 1;
@@ -1102,15 +1105,16 @@ hipError_t launch_quantize_nchw(const float *x, const Thresholds &ths, int bitwi
         if (counted) {
             const long slices = gather_slices;
             auto launch_counted = [&](auto kernel) {
-                kernel<<<dim3((unsigned)(N * slices)), dim3(64), 0, stream>>>(x, ths, qx, (int)slices, C, HW, PC, slices == 1 ? btn : count_workspace);
+                kernel<<<dim3((unsigned)(N * slices)), dim3(64), 0, stream>>>(x, ths, qx, (int)slices, C, HW, PC, Div32{0, 0}, slices == 1 ? btn : count_workspace);
             };
             launch_counted(unit == 4 ? quantize_nchw_gather<2, 4, false, true> : quantize_nchw_gather<2, 2, false, true>);
             finish_counts(CountTarget{btn, count_workspace}, N, (int)slices, stream);
             return hipGetLastError();
         }
         auto pick = [&](auto even, auto any, auto even_weights, auto any_weights) {
-            if (weights) launch_weights(HW % 4 ? any_weights : even_weights, gather_waves, 64);
-            else launch(HW % 4 ? any : even, gather_waves, 64);
+            const long per_image = HW % 4 ? (HW + 3) / 4 : HW;  // runs, or pixels
+            if (weights) launch_weights(HW % 4 ? any_weights : even_weights, gather_waves, 64, per_image);
+            else launch(HW % 4 ? any : even, gather_waves, 64, per_image);
         };
         if (unit == 4 && bitwidth == 2)
             pick(quantize_nchw_gather<2, 4, true>, quantize_nchw_gather<2, 4, false>, quantize_nchw_gather<2, 4, true, false, true>, quantize_nchw_gather<2, 4, false, false, true>);
@@ -1153,8 +1157,8 @@ hipError_t launch_quantize_nchw(const float *x, const Thresholds &ths, int bitwi
         auto form = [&](auto vec, auto parts, auto past) {
             constexpr int VEC = decltype(vec)::value, PARTS = decltype(parts)::value;
             constexpr bool PAST = decltype(past)::value;
-            if (weights) launch_weights(bitwidth == 2 ? quantize_nchw_weights<2, VEC, PARTS, PAST> : quantize_nchw_weights<1, VEC, PARTS, PAST>, blocks, kThreads);
-            else launch(bitwidth == 2 ? quantize_nchw<2, VEC, PARTS, PAST> : quantize_nchw<1, VEC, PARTS, PAST>, blocks, kThreads);
+            if (weights) launch_weights(bitwidth == 2 ? quantize_nchw_weights<2, VEC, PARTS, PAST> : quantize_nchw_weights<1, VEC, PARTS, PAST>, blocks, kThreads, (HW + VEC - 1) / VEC);
+            else launch(bitwidth == 2 ? quantize_nchw<2, VEC, PARTS, PAST> : quantize_nchw<1, VEC, PARTS, PAST>, blocks, kThreads, (HW + VEC - 1) / VEC);
         };
         using std::integral_constant;
         auto parts = [&](auto vec) {
