@@ -481,7 +481,7 @@ int conv_mfma_shape(int type, const ConvArgs &a, float *cost_us)
 }
 
 // The kernel that keeps the input patch in LDS, against the tiled one that conv_mfma_shape picks: the shape with the lowest predicted
-// duration, if that is 7 % below what the tiled kernel is predicted to take (tab_conv_patch_model.h; both are linear forms with
+// duration, if that is 7 % (15 % where the tiled kernels fill the chip best) below what the tiled kernel is predicted to take (tab_conv_patch_model.h; both are linear forms with
 // non-negative coefficients, fitted to 1970 measured launches: over them the choices take 0.946 of the tiled kernels' time, in
 // total 0.907, the better one of each 0.931 and 0.893).  Not for 1x1 kernels, which read every pixel for one tap only, nor for at most 32 filters, half of
 // whose tiles would be work for nothing, nor for launches below 128 tiles of 64x64, which last as long as one tile's chain of waits
@@ -510,15 +510,18 @@ PatchPlan conv_patch_plan(int type, const ConvArgs &a)
     }
     if (a.qy != nullptr || (forced.tm != 0 && !(forced.tm == 9 && forced.ng < 0))) return plan;
     const long kn64 = ((long)a.KN + 63) / 64;
-    if (a.KH * a.KW == 1 || a.KN <= 32 || ((long)a.M + 63) / 64 * kn64 < 128) return plan;
+    const long tiles64 = ((long)a.M + 63) / 64 * kn64;
+    if (a.KH * a.KW == 1 || a.KN <= 32 || tiles64 < 128) return plan;
     float tiled_us = 0.f;
     plan.tiled = conv_mfma_shape(type, a, &tiled_us);
     float t[kTiledFeatures];
     tiled_features(a, tiled_us, t);
     float limit = 0.f;
     for (int k = 0; k < kTiledFeatures; k++) limit += kTiledCost[type][k] * t[k];
-    limit *= 0.93f;
+    // From one and a half to two tiles of 64x64 a CU the tiled kernels fill the chip best and the predictions are least certain: of the
+    // choices between 7 and 15 % half were slower (N=36 14x14x256 TNN 10.3 -> 11.6 us a call), none above.
     const uint32_t cus = (uint32_t)device_compute_units();
+    limit *= tiles64 * 2 >= 3 * (long)cus && tiles64 <= 2 * (long)cus ? 0.85f : 0.93f;
     for (int i = 0; i < kPatchShapes; i++) {
         if (kPatchTile[i].filters >= 128 * kn64) continue;
         const int kc = patch_chunk(a, kPatchTile[i].rows, patch_most_words(kPatchTile[i].wave_tiles), &npix, &lds_bytes);

@@ -19,7 +19,7 @@ DATA = os.path.join(HERE, "conv_patch_timings.txt")
 SHAPES = {12: (256, 128, 8, 2), 13: (128, 128, 4, 3), 14: (128, 64, 2, 4), 15: (64, 64, 1, 4), 16: (256, 64, 4, 3),
           17: (64, 256, 4, 3), 18: (64, 128, 2, 4)}  # kPatchTile
 CUS, ITEMS, LDS = 256, {1: 3, 2: 3, 4: 2}, 64 * 1024
-MARGIN, WEIGHTS_US = 0.93, 0.5  # the weights' part of the quantizer's launch, measured 0.1-0.8 us
+MARGIN, NARROW_MARGIN, WEIGHTS_US = 0.93, 0.85, 0.5  # the weights' part of the quantizer's launch, measured 0.1-0.8 us
 
 
 def parse(path):
@@ -114,7 +114,9 @@ def fit(rows, predict):
 
 
 def choose(r, tiled, patch, predict):
-    limit, best = MARGIN * float(tiled[r["type"]] @ tiled_features(r, predict(r))), None
+    tiles64 = (r["M"] + 63) // 64 * ((r["KN"] + 63) // 64)
+    margin = NARROW_MARGIN if 3 * CUS <= 2 * tiles64 <= 4 * CUS else MARGIN
+    limit, best = margin * float(tiled[r["type"]] @ tiled_features(r, predict(r))), None
     for s in SHAPES:
         f = patch_features(r, s)
         if f is not None and WEIGHTS_US + float(patch[r["type"], s] @ f) < limit:
