@@ -92,7 +92,7 @@ template <int BITS, int LOADS = kLoadsPerLane, bool OWN = false>
 __global__ __launch_bounds__(kThreads) void quantize_rows64(const floatx4 *__restrict__ x, const Thresholds ths, uint32_t *__restrict__ q, long rows,
                                                             long rows_per_item, Div32 div_item, int32_t *btn, long items)
 {
-    quantize_rows64_block<BITS, LOADS, OWN>(x, ths, q, rows, rows_per_item, div_item, in_eighths(blockIdx.x, ths.eighth));
+    quantize_rows64_block<BITS, LOADS, OWN>(x, ths, q, rows, rows_per_item, div_item, OWN ? in_eighths(blockIdx.x, ths.eighth) : blockIdx.x);
     const long row = (long)blockIdx.x * (4 * LOADS * kWavesPerBlock) + (threadIdx.x >> 6) * (4 * LOADS) + (threadIdx.x & 63);
     if ((threadIdx.x & 63) < 4 * LOADS) zero_counts(btn, items, row);
 }
@@ -105,7 +105,7 @@ __global__ __launch_bounds__(kThreads) void quantize_rows64_weights(const floatx
 {
     uint32_t block = blockIdx.x;
     if (pack_weights(job, block)) return;
-    quantize_rows64_block<BITS, LOADS, OWN>(x, ths, q, rows, rows_per_item, div_item, in_eighths(block, ths.eighth));
+    quantize_rows64_block<BITS, LOADS, OWN>(x, ths, q, rows, rows_per_item, div_item, OWN ? in_eighths(block, ths.eighth) : block);
 }
 
 // The same row quantizer for a 1x1 convolution with stride and no padding, which reads only the

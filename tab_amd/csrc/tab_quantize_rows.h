@@ -31,10 +31,17 @@ __device__ __forceinline__ void quantize_rows64_block(const floatx4 *__restrict_
     if (row_last > rows - 1) row_last = rows - 1;
 
     // The wave's items (scalar; div_item.mul == 0 says that rows reach 2^31 and the division takes 64 bits).  Partial sums are
-    // requested before x.
-    const long item_first = div_item.mul ? (long)div32((uint32_t)row0, div_item) : row0 / rows_per_item;
-    const long item_last = div_item.mul ? (long)div32((uint32_t)row_last, div_item) : row_last / rows_per_item;
-    const floatx4 requested = OWN ? request_threshold(ths, item_first) : floatx4{};
+    // requested before x, whose loads do not wait for the division otherwise.
+    long item_first = 0, item_last = 0;
+    auto find_items = [&] {
+        item_first = div_item.mul ? (long)div32((uint32_t)row0, div_item) : row0 / rows_per_item;
+        item_last = div_item.mul ? (long)div32((uint32_t)row_last, div_item) : row_last / rows_per_item;
+    };
+    floatx4 requested = {};
+    if (OWN) {
+        find_items();
+        requested = request_threshold(ths, item_first);
+    }
     // x and q from the wave's row on: 32-bit offsets from a scalar address leave registers for one more wave per SIMD
     const floatx4 *const src = x + row0 * 16;
     uint32_t *const dst = q + row0 * (BITS != 1 ? 4 : 2);
@@ -48,6 +55,7 @@ __device__ __forceinline__ void quantize_rows64_block(const floatx4 *__restrict_
         // a large one streams past them: non-temporal loads (plain ones are 8-11 % slower at 400 MB and more)
         v[u] = LOADS == 2 ? *at : __builtin_nontemporal_load(at);
     }
+    if (!OWN) find_items();
     const float t_first = OWN ? finish_threshold(ths, item_first, requested) : given_threshold(ths, item_first);
     const float t_last = item_last == item_first ? t_first : OWN ? wave_threshold(ths, item_last) : given_threshold(ths, item_last);
 
@@ -62,10 +70,13 @@ __device__ __forceinline__ void quantize_rows64_block(const floatx4 *__restrict_
             if (r < live && l == 0) *reinterpret_cast<uintx2 *>(dst + r * 2) = uintx2{out[0], out[1]};
         }
     };
-    // two copies of the loop under a scalar branch: the common one has no load but x in flight, so each load is
+    // copies of the loop under scalar branches: the common one has no load but x in flight, so each load is
     // waited for on its own
-    if (item_last <= item_first + 1) {
-        const uint32_t border = item_last == item_first ? 4 * LOADS : (uint32_t)(item_last * rows_per_item - row0);  // where the second begins
+    if (item_last == item_first) {
+#pragma unroll
+        for (int u = 0; u < LOADS; u++) finish(u, t_first);
+    } else if (item_last == item_first + 1) {
+        const uint32_t border = (uint32_t)(item_last * rows_per_item - row0);  // where the second begins
 #pragma unroll
         for (int u = 0; u < LOADS; u++) finish(u, (uint32_t)(u * 4 + sub) < border ? t_first : t_last);
     } else if (!OWN) {  // items of fewer rows than the wave (partial sums are those of 64 rows and more)
