@@ -76,7 +76,7 @@ __global__ __launch_bounds__(kConvThreads) __attribute__((amdgpu_waves_per_eu(2,
         if (w >= p.G) tap_kh[w] = 1 << 29;  // a word past K: no row is in range
     }
     const int tiles = (p.M + 31) >> 5;
-    const int waves = (int)gridDim.x * (kConvThreads / 64);
+    const int waves = (int)p.div_tiles_m.mul;  // of a column of the grid (gridDim would add 256 bytes of hidden arguments)
 
     // two tiles of activation in registers: the one being multiplied and the next one in flight (a second tile in
     // flight measured no faster and cost a wave per SIMD in registers)
@@ -348,7 +348,9 @@ hipError_t launch_mfma_regs_tile(ConvArgs a, hipStream_t stream)
     const int cap = (held + tiles_n - 1) / tiles_n;
     a.kcw = G;
     a.nchunks = 1;
-    conv_mfma_regs<TYPE, G, TN, OUT><<<dim3(regs_grid_x(tiles, cap < 1 ? 1 : cap), (unsigned)tiles_n), dim3(kConvThreads), 0, stream>>>(pack_conv<TYPE, (OUT >= kOutBits1)>(a));
+    const unsigned grid_x = regs_grid_x(tiles, cap < 1 ? 1 : cap);
+    a.div_tiles_m = Div32{grid_x * (kConvThreads / 64), 31};  // not a divisor here
+    conv_mfma_regs<TYPE, G, TN, OUT><<<dim3(grid_x, (unsigned)tiles_n), dim3(kConvThreads), 0, stream>>>(pack_conv<TYPE, (OUT >= kOutBits1)>(a));
     return hipGetLastError();
 }
 

@@ -15,6 +15,9 @@ namespace {
 // The two planes of a word travel as the pair words of the operand (ternary_dword, level_dword in tab_conv_mfma.h), which leaves 6
 // instructions of the 10 for the conv kernel.
 // True for the workgroups of the job (uniform); `block` is the workgroup's number, made the one among the others.
+// THREADS: of a workgroup; blockDim would add 256 bytes of hidden arguments to every quantizer, past the 120 from which a launch takes
+// longer (ConvParams).
+template <int THREADS>
 __device__ __forceinline__ bool pack_weights(const WeightJob &job, uint32_t &block)
 {
     if (block >= job.blocks) {
@@ -24,7 +27,7 @@ __device__ __forceinline__ bool pack_weights(const WeightJob &job, uint32_t &blo
     const int kc = (int)(job.kc_planes & 255u), planes = (int)(job.kc_planes >> 8);
     const int PC = (int)(job.pc_taps & 0xffffu), taps = (int)(job.pc_taps >> 16);
     const int pairs = patch_pairs(taps, kc), chunks = (PC + kc - 1) / kc;
-    const uint32_t item = block * blockDim.x + threadIdx.x;
+    const uint32_t item = block * THREADS + threadIdx.x;
     const int lane = (int)(item & 63u), r = lane & 31, kb = lane >> 5;
     const uint32_t run = item >> 6, chunk_run = run / (uint32_t)pairs;
     const int j = (int)(run - chunk_run * (uint32_t)pairs), tile = (int)(chunk_run / (uint32_t)chunks), c = (int)chunk_run - tile * chunks;

@@ -104,7 +104,7 @@ __global__ __launch_bounds__(kThreads) void quantize_rows64_weights(const floatx
                                                                     long rows, long rows_per_item, Div32 div_item, const WeightJob job)
 {
     uint32_t block = blockIdx.x;
-    if (pack_weights(job, block)) return;
+    if (pack_weights<kThreads>(job, block)) return;
     quantize_rows64_block<BITS, LOADS, OWN>(x, ths, q, rows, rows_per_item, div_item, OWN ? in_eighths(block, ths.eighth) : block);
 }
 
@@ -189,7 +189,7 @@ __global__ __launch_bounds__(kThreads) void quantize_rows64_count(const floatx4 
 __global__ __launch_bounds__(kThreads) void patch_weights(const WeightJob job)
 {
     uint32_t block = blockIdx.x;
-    pack_weights(job, block);
+    pack_weights<kThreads>(job, block);
 }
 
 // General path: any C, any alignment of x, every format (MODE as in compare4).  A workgroup takes a tile of consecutive pixels,
@@ -337,7 +337,7 @@ __global__ __launch_bounds__(kThreads) void quantize_tile_weights(const float *_
 {
     uint32_t block = blockIdx.x;
     if (blockIdx.y != 0 && block < job.blocks) return;  // (the grid's other parts of a pixel)
-    if (pack_weights(job, block)) return;
+    if (pack_weights<kThreads>(job, block)) return;
     const long p0 = (long)in_eighths(block, ths.eighth) * tile_pixels;
     const int live = pixels - p0 < tile_pixels ? (int)(pixels - p0) : tile_pixels;  // pixels of the tile that exist
     quantize_one_tile<MODE, LP>(x, ths, q, p0, live, pixels_per_item, div_item, C, tile_pixels, blockIdx.y * words, words);
@@ -563,7 +563,7 @@ __global__ __launch_bounds__(kThreads) void quantize_nchw_weights(const float *_
                                                                   int C, long HW, int PC, Div32 by_image, const WeightJob job)
 {
     uint32_t block = blockIdx.x;
-    if (pack_weights(job, block)) return;
+    if (pack_weights<kThreads>(job, block)) return;
     block = in_eighths(block, ths.eighth);
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const PixelRun<VEC> run((block / PC * (kWavesPerBlock / SPLIT) + wave / SPLIT) * 64L + (threadIdx.x & 63), N, HW, by_image);
@@ -615,7 +615,7 @@ __global__ __launch_bounds__(64, BITS == 1 ? (U == 4 ? 4 : 7) : (U == 4 ? 1 : 4)
     __shared__ __attribute__((aligned(16))) uint64_t stage[512];
     uint32_t block = blockIdx.x;
     if constexpr (WEIGHTS)
-        if (pack_weights(extra, block)) return;
+        if (pack_weights<64>(extra, block)) return;
     int32_t *btn = nullptr;
     if constexpr (!WEIGHTS) btn = extra;
     if constexpr (!COUNT) block = in_eighths(block, ths.eighth);
