@@ -458,9 +458,10 @@ struct ConvRoute {
     const tab::WeightJob *weights() const { return plan.shape >= 0 ? &job : nullptr; }
 };
 
-static ConvRoute conv_route(const tab::ConvArgs &args, int type, void *spare, size_t room)
+/* plan: already made, or null. */
+static ConvRoute conv_route(const tab::ConvArgs &args, int type, const tab::PatchPlan *plan, void *spare, size_t room)
 {
-    ConvRoute r = {args, tab::conv_patch_plan(type, args), {}};
+    ConvRoute r = {args, plan ? *plan : tab::conv_patch_plan(type, args), {}};
     char *at = reinterpret_cast<char *>(((uintptr_t)spare + 15) & ~(uintptr_t)15);
     const size_t lost = (size_t)(at - static_cast<char *>(spare));
     if (r.plan.shape >= 0 && (room < lost || room - lost < r.plan.weight_bytes)) r.plan.shape = -1;
@@ -484,7 +485,7 @@ static int run_route(const ConvRoute &r, int type, void *stream)
  * take their own ways.  The arguments have been checked.  spare, room: of the workspace, behind what the call needs. */
 static int conv_from_nhwc(const float *dev_X, const int64_t *dev_QW, const tab::Thresholds &ths, const int32_t *dev_btn, int type,
                           int padding1, int padding2, int stride1, int stride2, int N, int H, int W, int C, int KN, int KH, int KW,
-                          const ConvShape &s, float *dev_Y, void *workspace, void *spare, size_t room, void *stream)
+                          const ConvShape &s, float *dev_Y, void *workspace, const tab::PatchPlan *plan, void *spare, size_t room, void *stream)
 {
     // One launch where it pays (only under the automatic kernel choice: a forced kernel is what the caller wants to see run):
     // a 1x1 convolution without padding, the smallest calls of any kernel.  The packed activation stays in LDS.
@@ -509,7 +510,7 @@ static int conv_from_nhwc(const float *dev_X, const int64_t *dev_QW, const tab::
                                  s.OW, C, KN, 1, 1, dev_Y, stream);
     }
     const ConvRoute route = conv_route(conv_args(s, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, workspace, dev_QW, dev_btn, dev_Y),
-                                       type, spare, room);
+                                       type, plan, spare, room);
     // stage 1: quantize + pack the activation (TAB_GEMM.cu:419-426); no btn for activations
     hipError_t e = tab::launch_quantize(dev_X, ths, s.abits, (long)H * W, N, C, reinterpret_cast<uint64_t *>(workspace), nullptr,
                                         nullptr, static_cast<hipStream_t>(stream), route.weights());
@@ -521,7 +522,7 @@ static int conv_from_nhwc(const float *dev_X, const int64_t *dev_QW, const tab::
 /* Body of tab_conv2d and tab_conv2d_static (builtin: the library's own scratch). */
 static int conv_from_floats(const float *dev_X, const int64_t *dev_QW, const float *dev_ths, const int32_t *dev_btn, int type,
                             int padding1, int padding2, int stride1, int stride2, int N, int H, int W, int C, int KN, int KH,
-                            int KW, float *dev_Y, void *workspace, size_t workspace_bytes, bool builtin, void *stream)
+                            int KW, float *dev_Y, void *workspace, size_t workspace_bytes, bool builtin, const tab::PatchPlan *plan, void *stream)
 {
     ConvShape s;
     int rc = check_conv(type, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, &s);
@@ -543,14 +544,14 @@ static int conv_from_floats(const float *dev_X, const int64_t *dev_QW, const flo
     if (type > 3 && !one_launch(type, dev_X, false, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, s)) {
         // the CPU-only types: their own packers, then the same fused kernel
         const ConvRoute route = conv_route(conv_args(s, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, workspace, dev_QW, dev_btn, dev_Y),
-                                           type, spare, room);
+                                           type, plan, spare, room);
         hipError_t e = tab::launch_quantize_format(dev_X, dev_ths, type, (long)H * W, N, C, reinterpret_cast<uint64_t *>(workspace),
                                                    static_cast<hipStream_t>(stream), route.weights());
         if (e != hipSuccess) return device_fail(e, "quantize launch");
         return run_route(route, type, stream);
     }
     return conv_from_nhwc(dev_X, dev_QW, tab::given_thresholds(dev_ths), dev_btn, type, padding1, padding2, stride1, stride2, N, H, W, C,
-                          KN, KH, KW, s, dev_Y, workspace, spare, room, stream);
+                          KN, KH, KW, s, dev_Y, workspace, plan, spare, room, stream);
 }
 
 /* Packed activation bytes of a layer call, rounded up so that the partial sums behind them are aligned. */
@@ -615,9 +616,9 @@ int tab_layer_quantize(const float *dev_X, int nchw, int bitwidth, float act_sca
     return layer_quantize(dev_X, nchw, bitwidth, act_scale, N, H, W, C, dev_QX, workspace, workspace_bytes, nullptr, stream);
 }
 
-int tab_layer_conv2d(const float *dev_X, int nchw, float act_scale, const int64_t *dev_QW, const int32_t *dev_btn, int type,
-                     int padding1, int padding2, int stride1, int stride2, int N, int H, int W, int C, int KN, int KH, int KW,
-                     float *dev_Y, void *workspace, size_t workspace_bytes, void *stream)
+int tab_internal_layer_conv2d(const float *dev_X, int nchw, float act_scale, const int64_t *dev_QW, const int32_t *dev_btn, int type,
+                              int padding1, int padding2, int stride1, int stride2, int N, int H, int W, int C, int KN, int KH, int KW,
+                              float *dev_Y, void *workspace, size_t workspace_bytes, const tab::PatchPlan *plan, void *stream)
 {
     if (type > 3) return fail(TAB_ERR_BAD_ARGUMENT, "type must be 0 (TNN), 1 (TBN), 2 (BTN) or 3 (BNN), got %d", type);
     ConvShape s;
@@ -634,7 +635,7 @@ int tab_layer_conv2d(const float *dev_X, int nchw, float act_scale, const int64_
     const int one = one_launch(type, dev_X, planes, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, s, own);
     if (planes && !one) {
         const ConvRoute route = conv_route(conv_args(s, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, workspace, dev_QW, dev_btn, dev_Y),
-                                           type, spare, room);
+                                           type, plan, spare, room);
         rc = layer_quantize(dev_X, 1, s.abits, act_scale, N, H, W, C, static_cast<int64_t *>(workspace), sums,
                             need - layer_packed_bytes(s.abits, N, H, W, C), route.weights(), stream);
         if (rc != TAB_OK) return rc;
@@ -661,7 +662,36 @@ int tab_layer_conv2d(const float *dev_X, int nchw, float act_scale, const int64_
         return TAB_OK;
     }
     return conv_from_nhwc(dev_X, dev_QW, ths, dev_btn, type, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, s, dev_Y,
-                          workspace, spare, room, stream);
+                          workspace, plan, spare, room, stream);
+}
+
+int tab_layer_conv2d(const float *dev_X, int nchw, float act_scale, const int64_t *dev_QW, const int32_t *dev_btn, int type,
+                     int padding1, int padding2, int stride1, int stride2, int N, int H, int W, int C, int KN, int KH, int KW,
+                     float *dev_Y, void *workspace, size_t workspace_bytes, void *stream)
+{
+    return tab_internal_layer_conv2d(dev_X, nchw, act_scale, dev_QW, dev_btn, type, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW,
+                                     dev_Y, workspace, workspace_bytes, nullptr, stream);
+}
+
+size_t tab_internal_conv_plan(int type, int padding1, int padding2, int stride1, int stride2, int N, int H, int W, int C, int KN, int KH, int KW,
+                              tab::PatchPlan *plan)
+{
+    *plan = {-1, 0, 0, 0, -1, 0};
+    ConvShape s;
+    if (stride1 < 1 || stride2 < 1 ||
+        !tab::conv_patch_considered(type, (long)N * tab_out_extent(H, padding1, KH, stride1) * tab_out_extent(W, padding2, KW, stride2), KN, KH, KW) ||
+        check_conv(type, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, &s) != TAB_OK)
+        return 0;
+    *plan = tab::conv_patch_plan(type, conv_args(s, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, nullptr, nullptr, nullptr, nullptr));
+    return plan->shape >= 0 ? plan->weight_bytes + 16 : 0;
+}
+
+int tab_internal_conv2d(const float *dev_X, const int64_t *dev_QW, const float *dev_ths, const int32_t *dev_btn, int type, int padding1,
+                        int padding2, int stride1, int stride2, int N, int H, int W, int C, int KN, int KH, int KW, float *dev_Y,
+                        void *workspace, size_t workspace_bytes, const tab::PatchPlan *plan, void *stream)
+{
+    return conv_from_floats(dev_X, dev_QW, dev_ths, dev_btn, type, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW,
+                            dev_Y, workspace, workspace_bytes, false, plan, stream);
 }
 
 int tab_conv2d(const float *dev_X, const int64_t *dev_QW, const float *dev_ths,
@@ -670,7 +700,7 @@ int tab_conv2d(const float *dev_X, const int64_t *dev_QW, const float *dev_ths,
                void *workspace, size_t workspace_bytes, void *stream)
 {
     return conv_from_floats(dev_X, dev_QW, dev_ths, dev_btn, type, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW,
-                            dev_Y, workspace, workspace_bytes, false, stream);
+                            dev_Y, workspace, workspace_bytes, false, nullptr, stream);
 }
 
 int tab_conv2d_launches(const float *dev_X, int type, int padding1, int padding2, int stride1, int stride2, int N, int H, int W,
@@ -688,7 +718,7 @@ int tab_conv2d_static(const float *dev_X, const int64_t *dev_QW, const float *de
                       float *dev_Y, void *stream)
 {
     return conv_from_floats(dev_X, dev_QW, dev_ths, dev_btn, type, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW,
-                            dev_Y, nullptr, 0, true, stream);
+                            dev_Y, nullptr, 0, true, nullptr, stream);
 }
 
 }  // extern "C"

@@ -6,6 +6,8 @@
 #include <string.h>
 #include <type_traits>
 
+#include "tab_route.h"
+
 namespace tab {
 
 constexpr int kWordBits = 64;  // channels per packed int64 word (CNTBITS, TAB_GEMM.cuh:10)
@@ -206,13 +208,9 @@ struct WeightJob {
 };
 static_assert(sizeof(WeightJob) == 32, "quantizers take it beside at most 80 bytes of arguments");
 
-// A convolution's plan for that kernel: shape < 0 where another kernel takes it, of which `tiled` is the shape if it has been looked
-// up (else -1).
-struct PatchPlan {
-    int shape, kc, npix, lds_bytes, tiled;
-    size_t weight_bytes;
-};
 constexpr int kPatchShape = 12;  // shapes (of launch_conv_mfma) from here on are that kernel's
+// Whether a call of these sizes may go there at all: the launches for which the plan is worked out.
+bool conv_patch_considered(int type, long M, int KN, int KH, int KW);
 // The plan of the automatic choice (or of the test hook's); fp32 output.
 PatchPlan conv_patch_plan(int type, const ConvArgs &args);
 // Bytes that hold the weights of any plan for these sizes.

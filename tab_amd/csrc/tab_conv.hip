@@ -488,11 +488,19 @@ int conv_mfma_shape(int type, const ConvArgs &a, float *cost_us)
 // (no win below 49 such tiles, one in eight from there to 120).  Measured, tiled / patch, conv kernel alone in the kernel trace:
 // N=64 14x14x256 levels 13.6 / 10.6 us, N=256 28x28x512->512 BNN 224 / 196, N=32 56x56x64 TNN 10.3 / 8.5,
 // N=32 56x56x256->256 TNN 41.5 / 35 (64x256 tiles).
+bool conv_patch_considered(int type, long M, int KN, int KH, int KW)
+{
+    if (type > 4) return false;
+    const Forced forced = forced_kernel();
+    if (forced.tm == 9 && forced.ng >= kPatchShape) return true;  // the test hook
+    return (forced.tm == 0 || (forced.tm == 9 && forced.ng < 0)) && KH * KW > 1 && KN > 32 && (M + 63) / 64 * (((long)KN + 63) / 64) >= 128;
+}
+
 PatchPlan conv_patch_plan(int type, const ConvArgs &a)
 {
     PatchPlan plan = {-1, 0, 0, 0, -1, 0};
     const Forced forced = forced_kernel();
-    if (type > 4 || !conv_mfma_exact(a) || (type == 4 && !conv_mfma_exact_levels(a))) return plan;
+    if (!conv_patch_considered(type, a.M, a.KN, a.KH, a.KW) || !conv_mfma_exact(a) || (type == 4 && !conv_mfma_exact_levels(a))) return plan;
     int npix, lds_bytes;
     auto weigh = [&](int shape, int kc) {
         plan.shape = shape;
@@ -508,10 +516,9 @@ PatchPlan conv_patch_plan(int type, const ConvArgs &a)
         const int kc = i < kPatchShapes ? patch_chunk(a, kPatchTile[i].rows, patch_most_words(kPatchTile[i].wave_tiles), &npix, &lds_bytes) : 0;
         return kc ? weigh(forced.ng, kc) : plan;
     }
-    if (a.qy != nullptr || (forced.tm != 0 && !(forced.tm == 9 && forced.ng < 0))) return plan;
+    if (a.qy != nullptr) return plan;
     const long kn64 = ((long)a.KN + 63) / 64;
     const long tiles64 = ((long)a.M + 63) / 64 * kn64;
-    if (a.KH * a.KW == 1 || a.KN <= 32 || tiles64 < 128) return plan;
     float tiled_us = 0.f;
     plan.tiled = conv_mfma_shape(type, a, &tiled_us);
     float t[kTiledFeatures];

@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "../../include/tab_amd.h"
+#include "tab_route.h"
 
 // CHECK_INPUT of the reference (TAB_GPU.cpp:7-9)
 #define CHECK_CUDA(x) TORCH_CHECK(x.device().is_cuda(), #x " must be a CUDA tensor")
@@ -169,12 +170,14 @@ torch::Tensor TAB_Conv2d(const torch::Tensor &X, const torch::Tensor &QW, const 
     const auto [OH, OW] = check_conv_from_floats(X, QW, thresholds, btn, type, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW);
     const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(X.device());
     auto Y = device_empty({N, KN, OH, OW}, torch::kFloat32, X);
-    const size_t ws_bytes = tab_conv2d_workspace_bytes_full(type, N, H, W, C, KN, KH, KW);
+    tab::PatchPlan plan;
+    const size_t ws_bytes = tab_conv2d_workspace_bytes(type, N, H, W, C) +
+                            tab_internal_conv_plan(type, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, &plan);
     const hipStream_t stream = current_stream(X);
     const Workspace ws(ws_bytes, stream);
-    check_status(tab_conv2d(X.data_ptr<float>(), QW.data_ptr<int64_t>(), thresholds.data_ptr<float>(),
-                            btn.data_ptr<int32_t>(), type, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH,
-                            KW, Y.data_ptr<float>(), ws.get(), ws_bytes, stream));
+    check_status(tab_internal_conv2d(X.data_ptr<float>(), QW.data_ptr<int64_t>(), thresholds.data_ptr<float>(),
+                                     btn.data_ptr<int32_t>(), type, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH,
+                                     KW, Y.data_ptr<float>(), ws.get(), ws_bytes, &plan, stream));
     return Y;
 }
 
@@ -453,11 +456,13 @@ torch::Tensor layer_output(const torch::Tensor &X, bool nchw, int64_t N, int64_t
 void run_layer(const Layer &l, const torch::Tensor &X, bool nchw, int N, int H, int W, const torch::Tensor &y)
 {
     const hipStream_t stream = current_stream(X);
-    const size_t ws_bytes = tab_layer_workspace_bytes_full(l.type, N, H, W, l.C, l.KN, l.KH, l.KW);
+    tab::PatchPlan plan;
+    const size_t ws_bytes = tab_layer_workspace_bytes(l.act_bits(), N, H, W, l.C) +
+                            tab_internal_conv_plan(l.type, l.p1, l.p2, l.s1, l.s2, N, H, W, l.C, l.KN, l.KH, l.KW, &plan);
     const Workspace ws(ws_bytes, stream);
-    check_status(tab_layer_conv2d(X.data_ptr<float>(), nchw, (float)l.act_scale, l.QW.data_ptr<int64_t>(), l.btn.data_ptr<int32_t>(),
-                                  l.type, l.p1, l.p2, l.s1, l.s2, N, H, W, l.C, l.KN, l.KH, l.KW, y.data_ptr<float>(), ws.get(),
-                                  ws_bytes, stream));
+    check_status(tab_internal_layer_conv2d(X.data_ptr<float>(), nchw, (float)l.act_scale, l.QW.data_ptr<int64_t>(), l.btn.data_ptr<int32_t>(),
+                                           l.type, l.p1, l.p2, l.s1, l.s2, N, H, W, l.C, l.KN, l.KH, l.KW, y.data_ptr<float>(), ws.get(),
+                                           ws_bytes, &plan, stream));
 }
 
 // TABConv2d.forward

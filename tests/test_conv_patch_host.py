@@ -75,6 +75,24 @@ def test_sizes_of_refused_arguments(lib):
         assert lib.tab_conv2d_workspace_bytes_full(type, 2, 9, 9, 100, 64, KH, KH) == lib.tab_conv2d_workspace_bytes(type, 2, 9, 9, 100)
 
 
+def test_the_front_end_asks_for_the_room_of_the_plan(lib):
+    """tab_internal_conv_plan, what the PyTorch front end allocates by: the weights' room where the rule takes a call to this kernel, else
+    none (the room of every plan for every call moved the blocks of the calls behind it, which then ran slower)."""
+    lib.tab_set_conv_kernel(0, -1)
+    lib.tab_internal_conv_plan.restype, plan_of = ctypes.c_size_t, (ctypes.c_byte * 64)()
+    seen = set()
+    for type in range(6):
+        for N in (1, 16, 36, 256):
+            for H, C, KN, KH, p, s in ((56, 64, 64, 3, 1, 1), (28, 128, 128, 3, 1, 1), (14, 256, 256, 3, 1, 1), (7, 512, 512, 3, 1, 1),
+                                       (56, 64, 128, 3, 1, 2), (56, 64, 128, 1, 0, 2), (40, 100, 75, 5, 2, 1), (9, 64, 64, 11, 0, 1)):
+                a = (type, p, p, s, s, N, H, H, C, KN, KH, KH)
+                shape, _, _, _, weights = plan(lib, *a)
+                assert lib.tab_internal_conv_plan(*a, plan_of) == (weights + 16 if shape >= 0 else 0), a
+                assert ctypes.c_int.from_buffer(plan_of).value == shape
+                seen.add(shape >= 0)
+    assert seen == {False, True}
+
+
 def test_the_rule_on_its_measured_launches(lib):
     """The compiled choices (256 compute units where no device is present) against the tiled kernels' times: within what the rule's
     comment states, and no single choice more than a quarter off."""

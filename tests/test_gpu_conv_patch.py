@@ -125,3 +125,22 @@ def test_a_small_workspace_and_the_built_in_scratch(lib):
         tab_amd.set_conv_kernel(tab_amd.CONV_MATRIX, 2)
         assert torch.equal(out, tab_amd.Conv2d(*a))
         lib.tab_internal_force_patch(14)
+
+
+@pytest.mark.parametrize("N", [16, 64])
+def test_calls_allocate_the_room_they_use(N, lib):
+    """Y, the packed activation and, where the rule takes the call to this kernel (N = 64), its weights: nothing else."""
+    H, C, KN, type = 14, 256, 256, 4
+    g = torch.Generator(device="cuda").manual_seed(6)
+    x, ths = torch.randn((N, H, H, C), device="cuda", generator=g).abs(), torch.full((N,), 0.5, device="cuda")
+    QW, btn = weights(type, g, KN, 3, 3, C)
+    what, size = (ctypes.c_int * 3)(), ctypes.c_size_t(0)
+    shape = lib.tab_internal_conv_patch_shape(type, 1, 1, 1, 1, N, H, H, C, KN, 3, 3, what, ctypes.byref(size))
+    assert (shape >= 0) == (N == 64)
+    room = lambda n: (n + 511) // 512 * 512  # noqa: E731
+    want = room(N * H * H * KN * 4) + room(N * H * H * tab_amd.operand_words(type, 0, C) * 8 + (size.value + 16 if shape >= 0 else 0))
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    y = tab_amd.Conv2d(x, QW, ths, btn, type, 1, 1, 1, 1, N, H, H, C, KN, 3, 3)
+    assert torch.cuda.max_memory_allocated() - before == want, y.shape
