@@ -152,7 +152,8 @@ size_t tab_conv2d_workspace_bytes_full(int type, int N, int H, int W, int C, int
  *           16-byte aligned (the kernels store four floats at a time); every element is written
  *   workspace / workspace_bytes: device scratch of at least tab_conv2d_workspace_bytes()
  *           bytes, 16-byte aligned; owned by the caller, reusable once the stream has
- *           passed this call
+ *           passed this call.  All workspace_bytes of it are the call's to write: pass the
+ *           size that is free for it, not that of a larger buffer it lies in
  * Padded taps read all-zero words: value 0 for ternary, +1 for binary activations
  * (TAB_CPU.cpp:39,155); BNN's constant is KH*KW*C (TAB_GEMM.cu:509).
  * Types 4 and 5 (CPU-only in the reference, TAB_CPU.cpp:507-614) are accepted too: X goes through
@@ -227,7 +228,7 @@ int tab_conv2d_packed_out(const int64_t *dev_QX, const int64_t *dev_QW, const in
  * zeros, and the quantizer adds up an image's partial sums itself.
  *   nchw       0: dev_X is fp32 [N][H][W][C]; otherwise [N][C][H][W]
  *   workspace  tab_layer_workspace_bytes(bitwidth of the activation, ...), 16-byte aligned; tab_layer_quantize takes
- *              tab_threshold_workspace_bytes(N, H*W*C) for two planes and none for one
+ *              tab_threshold_workspace_bytes(N, H*W*C) for two planes and none for one; all workspace_bytes are the call's to write
  */
 size_t tab_layer_workspace_bytes(int bitwidth, int N, int H, int W, int C);
 /* The same for tab_layer_conv2d with room for the weights, as tab_conv2d_workspace_bytes_full. */

@@ -127,6 +127,31 @@ def test_a_small_workspace_and_the_built_in_scratch(lib):
         lib.tab_internal_force_patch(14)
 
 
+@pytest.mark.parametrize("full", [False, True])
+def test_nothing_behind_the_workspace_is_written(full, lib):
+    """The call writes inside the workspace_bytes it is given: of the packed activation alone, and with room for the weights."""
+    N, H, C, KN = 64, 14, 192, 70
+    g = torch.Generator(device="cuda").manual_seed(9)
+    x, ths = torch.randn((N, H, H, C), device="cuda", generator=g), torch.full((N,), 0.5, device="cuda")
+    y, p = torch.empty((N, H, H, KN), device="cuda"), lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    for f in (lib.tab_conv2d_workspace_bytes, lib.tab_conv2d_workspace_bytes_full, lib.tab_layer_workspace_bytes, lib.tab_layer_workspace_bytes_full):
+        f.restype = ctypes.c_size_t
+    for type in range(5):
+        QW, btn = weights(type, g, KN, 3, 3, C)
+        a = (type, N, H, H, C)
+        sizes = [lib.tab_conv2d_workspace_bytes_full(*a, KN, 3, 3) if full else lib.tab_conv2d_workspace_bytes(*a)]
+        if type < 4:
+            sizes.append(lib.tab_layer_workspace_bytes_full(*a, KN, 3, 3) if full else lib.tab_layer_workspace_bytes(2 if type < 2 else 1, N, H, H, C))
+        for layer, size in enumerate(sizes):
+            buffer = torch.full((size + 4096,), 0xA5, dtype=torch.uint8, device="cuda")
+            room, sizes_of = ctypes.c_size_t(size), (type, 1, 1, 1, 1, N, H, H, C, KN, 3, 3)
+            lib.tab_internal_force_patch(18)
+            status = (lib.tab_layer_conv2d(p(x), 0, ctypes.c_float(0.7), p(QW), p(btn), *sizes_of, p(y), p(buffer), room, stream) if layer else
+                      lib.tab_conv2d(p(x), p(QW), p(ths), p(btn), *sizes_of, p(y), p(buffer), room, stream))
+            assert status == 0 and bool((buffer[size:] == 0xA5).all()), (type, layer)
+
+
 @pytest.mark.parametrize("N", [16, 64])
 def test_calls_allocate_the_room_they_use(N, lib):
     """Y, the packed activation and, where the rule takes the call to this kernel (N = 64), its weights: nothing else."""
