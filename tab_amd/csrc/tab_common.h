@@ -197,7 +197,7 @@ void set_compute_units(int units);  // test hook of the rules that count them (0
 
 // The convolution that keeps the input patch of a tile in LDS (tab_conv_mfma_patch.h) reads the weights in an order of its own, in
 // which the quantizer's launch leaves them in the caller's workspace (pack_weights, tab_patch_weights.h): its first `blocks`
-// workgroups do that.  out == null: no such weights wanted.
+// workgroups do that.
 struct WeightJob {
     const uint64_t *qw;
     uint64_t *out;

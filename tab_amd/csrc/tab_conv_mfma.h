@@ -670,7 +670,8 @@ hipError_t launch_mfma_regs(const ConvArgs &a, hipStream_t stream);
 // pixel and otherwise run as shapes 2 and 0, 10 = 128x128 tiles for the whole rounds of the chip and 64x64 split-K quarters for
 // the rest of the last round (an even number of words per pixel; otherwise shape 0), 11 = the same with whole tiles of 128x256
 // (words per pixel in fours; otherwise shape 6); 12 .. 18 = the kernel that keeps the input patch in LDS, on weights laid out for
-// it (ConvArgs::qw then points to those): 256x128, 128x128, 128x64, 64x64, 256x64; refused where its patch does not fit
+// it (ConvArgs::qw then points to those): 256x128, 128x128, 128x64, 64x64, 256x64, 64x256, 64x128; refused where its patch does not
+// fit
 template <int TYPE>
 hipError_t launch_mfma_type(const ConvArgs &a, int shape, hipStream_t stream)
 {

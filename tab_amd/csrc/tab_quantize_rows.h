@@ -1,5 +1,5 @@
-// The streaming quantizer of whole words, by the workgroup: quantize_rows64 (tab_quantize.hip) and the convolutions that quantize
-// their successor's activation on the side (tab_conv_mfma_patch.h).
+// The streaming quantizer of whole words, by the workgroup: the body of quantize_rows64 and of quantize_rows64_weights, which lays a
+// convolution's weights out beside it (tab_quantize.hip).
 #pragma once
 #include "tab_pack.h"
 

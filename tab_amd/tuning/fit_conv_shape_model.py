@@ -29,7 +29,7 @@ fitted on everything, and with each set held out in turn.
 
 Packed output has coefficients of its own, for types 0..3, from conv_packed_timings.txt (743 random layers): an epilogue that
 writes a bit per filter and pixel favours wider tiles than one that writes a float, and with the coefficients of fp32 output the
-choices took 6 % more than the best shapes' (with its own 1.6 % fitted, 1.7 % with an eighth of the layers held out in turn).  There the
+choices took 6 % more than the best shapes' (with its own 1.5 % fitted, 1.7 % with an eighth of the layers held out in turn).  There the
 kernel with the weights resident in registers (shape 7, a wave per 64 pixels x 64 filters, four to a workgroup) competes with the
 tiles where K is at most nine words, and 32x32 tiles do not exist.
 
