@@ -481,19 +481,23 @@ int conv_mfma_shape(int type, const ConvArgs &a, float *cost_us)
 }
 
 // The kernel that keeps the input patch in LDS, against the tiled one that conv_mfma_shape picks: the shape with the lowest predicted
-// duration, if that is 7 % (15 % where the tiled kernels fill the chip best) below what the tiled kernel is predicted to take (tab_conv_patch_model.h; both are linear forms with
-// non-negative coefficients, fitted to 1970 measured launches: over them the choices take 0.946 of the tiled kernels' time, in
-// total 0.907, the better one of each 0.931 and 0.893).  Not for 1x1 kernels, which read every pixel for one tap only, nor for at most 32 filters, half of
-// whose tiles would be work for nothing, nor for launches below 128 tiles of 64x64, which last as long as one tile's chain of waits
-// (no win below 49 such tiles, one in eight from there to 120).  Measured, tiled / patch, conv kernel alone in the kernel trace:
-// N=64 14x14x256 levels 13.6 / 10.6 us, N=256 28x28x512->512 BNN 224 / 196, N=32 56x56x64 TNN 10.3 / 8.5,
-// N=32 56x56x256->256 TNN 41.5 / 35 (64x256 tiles).
+// duration, if that is 1.5 % and 0.1 us below what the call through the tiled kernel is predicted to take (tab_conv_patch_model.h; both are
+// linear forms with non-negative coefficients, fitted to the whole calls of 3970 random layers).  On 10756 further layers: 0.967 of the
+// tiled kernels' time (in total 0.952; the better one of each 0.959 and 0.945), of 3607 choices 95 more than 2 % slower, 25 more than
+// 5 %, 7 more than 8 %, the worst 15 %.  (Fitted to convolutions replayed on the same operands, weights in the L2s, 294 of those layers were more than
+// 5 % slower, the worst 1.6 times.)
+// Not for 1x1 kernels, which read every pixel for one tap only, nor for at most 32 filters, half of whose tiles would be work for nothing,
+// nor for launches of fewer 64x64 tiles than compute units, which last as long as one tile's chain of waits (from half as many on, 129
+// of 2709 layers gained more than 3 %, none that a fit could tell from the others).  Measured, whole calls, tiled / patch: N=64 14x14x256
+// levels 16.2 / 14.4 us, N=256 28x28x512->512 BNN 247 / 228, N=32 56x56x256->256 TNN 59.6 / 54.1 (64x256 tiles).  Each shape is the
+// best one of some launches, from 256x128 tiles (59 of those 10756, by 2 % in the median) to 128x64 (1373, 1.5 %).
 bool conv_patch_considered(int type, long M, int KN, int KH, int KW)
 {
     if (type > 4) return false;
     const Forced forced = forced_kernel();
     if (forced.tm == 9 && forced.ng >= kPatchShape) return true;  // the test hook
-    return (forced.tm == 0 || (forced.tm == 9 && forced.ng < 0)) && KH * KW > 1 && KN > 32 && (M + 63) / 64 * (((long)KN + 63) / 64) >= 128;
+    return (forced.tm == 0 || (forced.tm == 9 && forced.ng < 0)) && KH * KW > 1 && KN > 32 &&
+           (M + 63) / 64 * (((long)KN + 63) / 64) >= device_compute_units();
 }
 
 PatchPlan conv_patch_plan(int type, const ConvArgs &a)
@@ -508,7 +512,7 @@ PatchPlan conv_patch_plan(int type, const ConvArgs &a)
         plan.npix = npix;
         plan.lds_bytes = lds_bytes;
         const long tiles = (a.KN + 31) / 32, pairs = (long)((a.PC + kc - 1) / kc) * patch_pairs(a.KH * a.KW, kc);
-        plan.weight_bytes = (size_t)(tiles * pairs) * 512 * (type == 0 || type == 2 || type == 4 ? 2 : 1);
+        plan.weight_bytes = (size_t)(tiles * pairs) * 512 * patch_weight_planes(type);
         return plan;
     };
     if (forced.tm == 9 && forced.ng >= kPatchShape) {  // the test hook
@@ -517,24 +521,21 @@ PatchPlan conv_patch_plan(int type, const ConvArgs &a)
         return kc ? weigh(forced.ng, kc) : plan;
     }
     if (a.qy != nullptr) return plan;
-    const long kn64 = ((long)a.KN + 63) / 64;
-    const long tiles64 = ((long)a.M + 63) / 64 * kn64;
     float tiled_us = 0.f;
     plan.tiled = conv_mfma_shape(type, a, &tiled_us);
     float t[kTiledFeatures];
-    tiled_features(a, tiled_us, t);
+    tiled_features(a, type, tiled_us, t);
     float limit = 0.f;
     for (int k = 0; k < kTiledFeatures; k++) limit += kTiledCost[type][k] * t[k];
-    // From one and a half to two tiles of 64x64 a CU the tiled kernels fill the chip best and the predictions are least certain: of the
-    // choices between 7 and 15 % half were slower (N=36 14x14x256 TNN 10.3 -> 11.6 us a call), none above.
+    limit = 0.985f * limit - 0.1f;
+    const long kn64 = ((long)a.KN + 63) / 64;
     const uint32_t cus = (uint32_t)device_compute_units();
-    limit *= tiles64 * 2 >= 3 * (long)cus && tiles64 <= 2 * (long)cus ? 0.85f : 0.93f;
     for (int i = 0; i < kPatchShapes; i++) {
         if (kPatchTile[i].filters >= 128 * kn64) continue;
         const int kc = patch_chunk(a, kPatchTile[i].rows, patch_most_words(kPatchTile[i].wave_tiles), &npix, &lds_bytes);
         if (kc == 0) continue;
-        float f[kPatchFeatures], us = 0.5f;  // the weights' part of the quantizer's launch (measured 0.1-0.8)
-        patch_features(a, i, kc, npix, lds_bytes, cus, f);
+        float f[kPatchFeatures], us = 0.f;
+        patch_features(a, type, i, kc, npix, lds_bytes, cus, f);
         for (int k = 0; k < kPatchFeatures; k++) us += kPatchCost[type][i][k] * f[k];
         if (us < limit) {
             limit = us;
@@ -549,12 +550,12 @@ size_t patch_weight_bytes(int type, int C, int KN, int KH, int KW)
     if (type > 4 || KN <= 0) return 0;
     const size_t PC = (size_t)(C + kWordBits - 1) / kWordBits, taps = (size_t)KH * KW;
     // (of four words at most one is padding, of two taps one)
-    return ((size_t)KN + 31) / 32 * (((taps + 1) * (PC + 1) + 1) / 2) * 512 * (type == 0 || type == 2 || type == 4 ? 2 : 1);
+    return ((size_t)KN + 31) / 32 * (((taps + 1) * (PC + 1) + 1) / 2) * 512 * patch_weight_planes(type);
 }
 
 WeightJob patch_weight_job(int type, const ConvArgs &a, const PatchPlan &plan, uint64_t *out)
 {
-    const int planes = type == 0 || type == 2 || type == 4 ? 2 : 1;
+    const int planes = patch_weight_planes(type);
     const long items = (long)(plan.weight_bytes / 8 / planes);  // 64 lanes a run
     return WeightJob{a.qw, out, a.KN, (uint32_t)a.PC | (uint32_t)(a.KH * a.KW) << 16,
                      (uint32_t)((items + 255) / 256 + 7) / 8 * 8,  // whole groups of eight: the quantizer's workgroups stay on their XCDs

@@ -9,6 +9,9 @@ template <int KC> constexpr int kPatchItems = KC == 4 ? 2 : 3;  // pixels of the
 constexpr int kPatchLdsBytes = 64 * 1024;                       // of a workgroup
 constexpr int kPatchThreads = 256;
 
+// Bit planes of the weights.
+inline int patch_weight_planes(int type) { return type == 0 || type == 2 || type == 4 ? 2 : 1; }
+
 // Words of a chunk at most: waves of eight MFMA tiles have no registers for four.
 constexpr int patch_most_words(int tiles_per_wave) { return tiles_per_wave >= 8 ? 2 : 4; }
 
@@ -58,37 +61,44 @@ constexpr int kPatchShapes = 7;
 constexpr PatchTile kPatchTile[kPatchShapes] = {{256, 128, 8, 2}, {128, 128, 4, 3}, {128, 64, 2, 4}, {64, 64, 1, 4}, {256, 64, 4, 3}, {64, 256, 4, 3}, {64, 128, 2, 4}};
 
 // What the predicted durations (tab_conv_patch_model.h) are linear in; the fit script states the same.
-constexpr int kPatchFeatures = 13, kTiledFeatures = 10;
+constexpr int kPatchFeatures = 18, kTiledFeatures = 14;
 
-// A launch of shape i: the busiest CU holds n tiles in so many rounds; its loop, its patches, its chunks and its output.
-inline void patch_features(const ConvArgs &a, int i, int kc, int npix, int lds_bytes, uint32_t cus, float (&f)[kPatchFeatures])
+// A call through shape i: the busiest CU holds n tiles in so many rounds; its loop, its patches, its chunks and its output.  Then what the
+// convolution replayed on the same operands does not show: laying out the weights, and fetching them where they are in no L2 yet, pair
+// after pair of words (N=64 7x7x512->512 TNN, 36 pairs: 11.0 us replayed, 15.1 behind its quantizer).  One word a pixel leaves little
+// but output; and rows of Y that end inside a cache line are written in parts until they go through the caches.
+inline void patch_features(const ConvArgs &a, int type, int i, int kc, int npix, int lds_bytes, uint32_t cus, float (&f)[kPatchFeatures])
 {
     const PatchTile &tile = kPatchTile[i];
     const int taps = a.KH * a.KW;
     const float chunks = (float)((a.PC + kc - 1) / kc);
-    const float K = chunks * (float)(kc == 1 ? (taps + 1) / 2 * 2 : taps * kc);  // words multiplied
+    const float pairs = chunks * (float)(kc == 1 ? (taps + 1) / 2 : taps * kc / 2), K = 2.f * pairs;  // words multiplied
     const uint32_t tiles_m = ((uint32_t)a.M + (uint32_t)tile.rows - 1) / (uint32_t)tile.rows, tiles_n = ((uint32_t)a.KN + (uint32_t)tile.filters - 1) / (uint32_t)tile.filters;
     const uint64_t tiles = (uint64_t)tiles_m * tiles_n;
     const int by_lds = 160 * 1024 / lds_bytes, held = tile.held < by_lds ? tile.held : by_lds;
     const uint64_t busiest = tiles <= 0xffffffffu ? ((uint32_t)tiles + cus - 1) / cus : (tiles + cus - 1) / cus;
     const float n = (float)busiest, rounds = (float)((busiest + (uint32_t)held - 1) / (uint32_t)held);
     const float busy = tiles < cus ? (float)tiles / (float)cus : 1.f;
-    const float y_mb = (float)a.M * (float)a.KN * 4e-6f;
+    const float y_mb = (float)a.M * (float)a.KN * 4e-6f, ragged = a.KN % 32 ? y_mb : 0.f;
     const float patch = (float)npix * (float)kc * chunks * 1e-3f;  // words expanded a tile
+    const float weights = (float)((a.KN + 31) / 32) * pairs * (patch_weight_planes(type) == 2 ? 1024e-6f : 512e-6f);
     const float values[kPatchFeatures] = {1.f, busy, K * n, K * rounds, n, rounds, y_mb, y_mb * busy, patch * n, patch * rounds, chunks * rounds,
-                                          (float)tiles / (float)cus, a.KN % 32 ? y_mb : 0.f};
+                                          (float)tiles / (float)cus, ragged, weights, 0.01f * pairs, a.PC == 1 ? 1.f : 0.f, a.PC == 1 ? y_mb : 0.f,
+                                          ragged_rows_cached(a.M, a.KN) ? 0.f : ragged};
     for (int k = 0; k < kPatchFeatures; k++) f[k] = values[k];
 }
 
-// The tiled kernel that conv_mfma_shape picks, which predicts `us` for it: that prediction was fitted to even words per pixel, whole
-// lines of Y and launches like the benchmark's.
-inline void tiled_features(const ConvArgs &a, float us, float (&f)[kTiledFeatures])
+// The call through the tiled kernel that conv_mfma_shape picks, which predicts `us` for its convolution: that prediction was fitted to even
+// words per pixel, whole lines of Y and launches like the benchmark's.
+inline void tiled_features(const ConvArgs &a, int type, float us, float (&f)[kTiledFeatures])
 {
     const float G = (float)a.G, y_mb = (float)a.M * (float)a.KN * 4e-6f;
     const float products = (float)a.M * (float)((a.KN + 63) / 64 * 64) * G * 1e-9f;
-    const bool odd = a.PC % 2 != 0;
+    const bool odd = a.PC % 2 != 0, one = a.PC == 1;
+    const float ragged = a.KN % 32 ? y_mb : 0.f;
     const float values[kTiledFeatures] = {1.f, us, y_mb, products, odd ? products : 0.f, odd ? us : 0.f, 0.1f * G, odd ? 0.1f * G : 0.f,
-                                          (float)a.M * G * 1e-6f, a.KN % 32 ? y_mb : 0.f};
+                                          (float)a.M * G * 1e-6f, ragged, (float)a.KN * G * (float)patch_weight_planes(type) * 8e-6f,
+                                          one ? 1.f : 0.f, one ? us : 0.f, one && ragged_rows_cached(a.M, a.KN) ? ragged : 0.f};
     for (int k = 0; k < kTiledFeatures; k++) f[k] = values[k];
 }
 

@@ -6,7 +6,6 @@ import importlib.util
 import os
 import random
 
-import numpy as np
 import pytest
 
 from tab_amd import _capi
@@ -93,21 +92,26 @@ def test_the_front_end_asks_for_the_room_of_the_plan(lib):
     assert seen == {False, True}
 
 
-def test_the_rule_on_its_measured_launches(lib):
-    """The compiled choices (256 compute units where no device is present) against the tiled kernels' times: within what the rule's
-    comment states, and no single choice more than a quarter off."""
+def test_the_rule_on_its_measured_calls(lib):
+    """The compiled choices (256 compute units where no device is present) against the tiled kernels' times, whole calls: the figures that
+    the rule's fit states, and none beyond."""
     spec = importlib.util.spec_from_file_location("fit", os.path.join(TUNING, "fit_conv_patch_model.py"))
     fit = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(fit)
     lib.tab_set_conv_kernel(0, -1)
     rows = [r for r in fit.parse(fit.DATA) if fit.eligible(r)]
-    assert len(rows) > 1500
+    assert len(rows) > 3900
     chosen = []
     for r in rows:
         shape, kc, npix, lds, _ = plan(lib, r["type"], r["p1"], r["p2"], r["s"], r["s"], r["N"], r["H"], r["W"], r["C"], r["KN"], r["KH"], r["KW"])
         if shape >= 0:
             assert fit.patch_features(r, shape) is not None and fit.chunk(r, shape) == (kc, npix, lds), r
         chosen.append(shape if shape >= 0 else None)
-    geometric, total, best_geometric, best_total, worst = fit.regret(rows, chosen)
-    assert geometric < 0.96 and total < 0.94 and geometric < 1.02 * best_geometric and worst < 1.3, (geometric, total, worst)
-    assert np.mean([c is not None for c in chosen]) > 0.2
+    geometric, total, _, _, each = fit.regret(rows, chosen)
+    stated = fit.stated(rows, chosen)
+    # (to the last digit of what the script prints: float arithmetic may turn a call or two on the border)
+    assert geometric < 0.9628 and total < 0.9447 and each.max() < 1.10, stated
+    assert (each > 1.02).sum() <= 29 and (each > 1.05).sum() <= 9 and (each > 1.08).sum() <= 3, stated
+    assert len({c for c in chosen if c is not None}) == len(ROWS), stated  # every shape has launches of its own
+    # launches of fewer tiles than compute units are not looked at
+    assert plan(lib, 0, 1, 1, 1, 1, 16, 14, 14, 256, 256, 3, 3)[0] < 0 and plan(lib, 0, 1, 1, 1, 1, 64, 14, 14, 256, 256, 3, 3)[0] >= 0
