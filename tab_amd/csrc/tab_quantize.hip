@@ -963,10 +963,12 @@ void launch_quantize_tile_of(const float *x, const Thresholds &ths, long pixels,
         }
     }
     const dim3 grid((unsigned)((pixels + tile_pixels - 1) / tile_pixels), (unsigned)((PC + words - 1) / words));
-    if (weights) {
-        quantize_tile_weights<MODE, LP><<<dim3(grid.x + weights->blocks, grid.y), dim3(kThreads), lds, stream>>>(
-            x, grid.y == 1 ? ordered(ths, grid.x) : ordered(ths, 0), q, pixels, pixels_per_item, div_item, C, (int)tile_pixels, words, *weights);
-        return;
+    if constexpr (MODE != 5) {  // (type 5 has no kernel that reads its weights in another order)
+        if (weights) {
+            quantize_tile_weights<MODE, LP><<<dim3(grid.x + weights->blocks, grid.y), dim3(kThreads), lds, stream>>>(
+                x, grid.y == 1 ? ordered(ths, grid.x) : ordered(ths, 0), q, pixels, pixels_per_item, div_item, C, (int)tile_pixels, words, *weights);
+            return;
+        }
     }
     quantize_tile<MODE, LP><<<grid, dim3(kThreads), lds, stream>>>(x, grid.y == 1 ? ordered(ths, grid.x) : ordered(ths, 0), q, pixels, pixels_per_item, div_item, C, (int)tile_pixels, words, btn, items);
 }
