@@ -41,8 +41,25 @@ def weights(type, g, KN, KH, KW, C):
     return tab_amd.Quantize(w, ths, 2 if type in (0, 2) else 1, KN, KH, KW, C)
 
 
+def fitting(lib, type, sizes):
+    """(the shape that the test hook holds, its weights' bytes) where the patch of these sizes fits it, else (-1, 0)."""
+    what, size = (ctypes.c_int * 3)(), ctypes.c_size_t(0)
+    shape = lib.tab_internal_conv_patch_shape(type, *sizes, what, ctypes.byref(size))
+    return (shape, size.value) if shape >= 0 else (-1, 0)
+
+
+def requested(call):
+    """(the call's result, the most bytes it has asked the allocator for)."""
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_stats()["requested_bytes.all.current"]
+    y = call()
+    return y, torch.cuda.memory_stats()["requested_bytes.all.peak"] - before
+
+
 @pytest.mark.parametrize("case", CASES)
 def test_calls_and_layers(case, lib):
+    """That the kernel ran shows in the memory a call asks for: room for its weights, which no other kernel is given, and only where the
+    patch fits.  (The quantizer lays them out there exactly when this kernel follows; test_the_weights_are_laid_out_behind_the_activation.)"""
     N, H, W, C, KN, KH, KW, p1, p2, s1, s2 = case
     print(f"[case] patch {case}", flush=True)
     g = torch.Generator(device="cuda").manual_seed(KN + C)
@@ -58,11 +75,16 @@ def test_calls_and_layers(case, lib):
                 layer = tab_nn.TABConv2d.from_float(w, type, (s1, s2), (p1, p2), data_format=layout)
                 layers.append((layer, x if layout == "NHWC" else x.permute(0, 3, 1, 2).contiguous()))
         tab_amd.set_conv_kernel(tab_amd.CONV_MATRIX, 2)
-        want = [run()] + [layer(a) for layer, a in layers]
+        calls = [run] + [lambda layer=layer, a=a: layer(a) for layer, a in layers]
+        want = [requested(call) for call in calls]
         for shape in SHAPES:
             lib.tab_internal_force_patch(shape)
-            got = [run()] + [layer(a) for layer, a in layers]
-            assert all(torch.equal(y, z) for y, z in zip(got, want)), (type, shape)
+            fits, room = fitting(lib, type, (p1, p2, s1, s2, N, H, W, C, KN, KH, KW))
+            assert fits in (shape, -1)
+            for call, (y, least) in zip(calls, want):
+                z, more = requested(call)
+                assert torch.equal(z, y), (type, shape)
+                assert more == least + (room + 16 if fits == shape else 0), (type, shape)
 
 
 @pytest.mark.parametrize("case", CASES)
@@ -125,6 +147,54 @@ def test_a_small_workspace_and_the_built_in_scratch(lib):
         tab_amd.set_conv_kernel(tab_amd.CONV_MATRIX, 2)
         assert torch.equal(out, tab_amd.Conv2d(*a))
         lib.tab_internal_force_patch(14)
+
+
+@pytest.mark.parametrize("case", CASES)
+def test_the_weights_are_laid_out_behind_the_activation(case, lib):
+    """What a call or a layer leaves behind its packed activation: the weights in the order of the shape in force, as a launch of their own
+    lays them out, where the patch fits; nothing where it does not, or where the workspace has no room for them.  The output is right either
+    way, and the kernels read the weights in two different orders: so it came from the kernel that the workspace shows."""
+    N, H, W, C, KN, KH, KW, p1, p2, s1, s2 = case
+    print(f"[case] patch, weights laid out {case}", flush=True)
+    sizes = (p1, p2, s1, s2, N, H, W, C, KN, KH, KW)
+    g = torch.Generator(device="cuda").manual_seed(KN + H)
+    x = torch.randn((N, H, W, C), device="cuda", generator=g)
+    x_nchw, ths = x.permute(0, 3, 1, 2).contiguous(), tab_amd.Threshold(x, N)
+    stream, p = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream), lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    for f in (lib.tab_conv2d_workspace_bytes, lib.tab_conv2d_workspace_bytes_full, lib.tab_layer_workspace_bytes, lib.tab_layer_workspace_bytes_full):
+        f.restype = ctypes.c_size_t
+    for type in range(5):
+        QW, btn = weights(type, g, KN, KH, KW, C)
+        y = torch.empty_like(tab_amd.Conv2d(x, QW, ths, btn, type, *sizes))
+        need, full = lib.tab_conv2d_workspace_bytes(type, N, H, W, C), lib.tab_conv2d_workspace_bytes_full(type, N, H, W, C, KN, KH, KW)
+        calls = [(need, full, lambda ws, n: lib.tab_conv2d(p(x), p(QW), p(ths), p(btn), type, *sizes, p(y), p(ws), ctypes.c_size_t(n), stream))]
+        if type < 4:
+            need, full = lib.tab_layer_workspace_bytes(2 if type < 2 else 1, N, H, W, C), lib.tab_layer_workspace_bytes_full(type, N, H, W, C, KN, KH, KW)
+            for nchw, a in ((0, x), (1, x_nchw)):
+                calls.append((need, full, lambda ws, n, nchw=nchw, a=a: lib.tab_layer_conv2d(p(a), nchw, ctypes.c_float(0.7), p(QW), p(btn), type, *sizes,
+                                                                                              p(y), p(ws), ctypes.c_size_t(n), stream)))
+        want = []
+        tab_amd.set_conv_kernel(tab_amd.CONV_MATRIX, 2)
+        for need, _, call in calls:
+            ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+            assert call(ws, need) == 0
+            want.append(y.clone())
+        for shape in SHAPES:
+            lib.tab_internal_force_patch(shape)
+            fits, room = fitting(lib, type, sizes)
+            alone = torch.empty(max(room, 16), dtype=torch.uint8, device="cuda")
+            if fits == shape:
+                assert lib.tab_internal_conv_patch(p(x), p(QW), p(btn), type, *sizes, p(y), p(alone), ctypes.c_size_t(room), 1, stream) == 0
+            for (need, full, call), right in zip(calls, want):
+                assert (need + 15) // 16 * 16 + room <= full
+                for size in (need, full):
+                    ws = torch.full((full,), 0xA5, dtype=torch.uint8, device="cuda")
+                    assert call(ws, size) == 0 and torch.equal(y, right), (type, shape)
+                    at = (need + 15) // 16 * 16
+                    if fits == shape and size == full:
+                        assert torch.equal(ws[at:at + room], alone), (type, shape)
+                        at += room
+                    assert bool((ws[at:] == 0xA5).all()), (type, shape)
 
 
 @pytest.mark.parametrize("full", [False, True])
