@@ -40,8 +40,7 @@ struct Div32 {
 };
 inline Div32 make_div32(uint32_t d)
 {
-    uint32_t s = 0;
-    while (((uint64_t)1 << s) < d) s++;
+    const uint32_t s = d > 1 ? 32u - (uint32_t)__builtin_clz(d - 1) : 0u;
     Div32 f;
     f.shift = 31 + s;
     f.mul = (uint32_t)((((uint64_t)1 << (31 + s)) / d) + 1);

@@ -410,53 +410,49 @@ hipError_t launch_conv_mfma(int type, const ConvArgs &args, int shape, hipStream
 // more than the best shapes', N=256 7x7x512 of type 5 28.4 us for 22.3.)
 // A shape whose filter tile is at least twice the 64-rounded filter count is no candidate.
 // cost_us (optional): the predicted duration of the chosen shape.
-int conv_mfma_shape(int type, const ConvArgs &a, float *cost_us)
+// (Host time of every call of two launches, 8.5 us at N=16 28x28x128: the loop over a table's shapes is unrolled, so that tile counts are
+// shifts, and counts are divided in 32 bits where they fit: 72-163 -> 34-87 ns.)
+template <bool PACKED>
+static int conv_mfma_ranked(int type, const ConvArgs &a, float *cost_us)
 {
     const long kn64 = ((long)a.KN + 63) / 64 * 64;
-    const long cus = device_compute_units();
+    const uint32_t cus = (uint32_t)device_compute_units();
     const bool narrow = conv_mfma_narrow(a);
-    // Packed output has a ranking of its own: with the one of fp32 output, and the kernel with the weights in registers wherever K is at
-    // most nine words and M at least 65536, 743 random layers took 6 % more than the best shapes' time; with this one 1.5 %.
-    // (types 4 and 5 are ranked as with fp32 output: they were not measured)
-    // Below 128 tiles of 64x64, where none of those layers lies, the ranking of fp32 output stays (one image of 41x41x192 through four
-    // layers: 26.1 us with it, 26.7 with the other), and weights in registers for K of at most two words.
-    const bool packed = a.qy != nullptr && type <= 3 && (long)((a.M + 63) / 64) * (kn64 / 64) >= 128;
-    if (a.qy != nullptr && type <= 3 && !packed && a.G <= 2) {
-        if (cost_us) *cost_us = 0.f;
-        return 7;
-    }
     const float y_mb = (float)a.M * (float)a.KN * 4e-6f;
     const float words = type == 5 ? 0.5f * (float)a.G : (float)a.G;  // of 64 elements
     int best = 2;
     float best_cost = 0.f;
     bool any = false;
-    for (int i = 0; i < (packed ? kConvPackedShapes : kConvShapes); i++) {
-        const int shape = packed ? kConvPackedIds[i] : kConvShapeIds[i];
-        const int *const tile = packed ? kConvPackedTile[i] : kConvShapeTile[i];
-        const float *const coefficients = packed ? kConvPackedCost[type][i] : kConvShapeCost[type][i];
-        const int bm = tile[0], bn = tile[1], held = tile[2];
+#pragma unroll
+    for (int i = 0; i < (PACKED ? kConvPackedShapes : kConvShapes); i++) {
+        const int shape = PACKED ? kConvPackedIds[i] : kConvShapeIds[i];
+        const int bm = PACKED ? kConvPackedTile[i][0] : kConvShapeTile[i][0], bn = PACKED ? kConvPackedTile[i][1] : kConvShapeTile[i][1];
+        const int held = PACKED ? kConvPackedTile[i][2] : kConvShapeTile[i][2];
+        const float *const coefficients = PACKED ? kConvPackedCost[type & 3][i] : kConvShapeCost[type][i];
         if (bn >= 2 * kn64) continue;
         if (shape == 7 && a.G > 9) continue;
         if (shape == 3 && a.qy != nullptr) continue;        // the packed epilogues need tiles 64 filters wide
         if (shape >= 8 && a.PC % 2 != 0) continue;          // the split-K shapes move whole pairs of words inside a tap
-        const long tiles = (long)((a.M + bm - 1) / bm) * ((a.KN + bn - 1) / bn);
+        const uint64_t tiles = (uint64_t)(((uint32_t)a.M + bm - 1) / bm) * (((uint32_t)a.KN + bn - 1) / bn);
+        const uint64_t whole = tiles < 1u << 31 ? (uint32_t)tiles / cus : tiles / cus, rest = tiles - whole * cus;
         float cost = 0.f, floor_us;
         if (shape == 10 || shape == 11) {
             // the mixed launches: whole tiles on every CU, then 64x64 quarter tiles (four to a 128x128 tile, eight to a
             // 128x256 one); candidates where they have both and K words x bit planes of the two operands exceed 36 (below
             // that the launch is bound by writing Y, whatever the balance of its last round)
-            const long pieces = bm / 64 * (bn / 64);
-            const long whole = tiles / cus, quarters = (pieces * (tiles % cus) + cus - 1) / cus;
+            const int pieces = bm / 64 * (bn / 64);
+            const uint32_t quarters = (uint32_t)(pieces * (uint32_t)rest + cus - 1) / cus;
             const int planes = type == 0 || type == 4 ? 4 : (type == 3 || type == 5 ? 2 : 3);
             if (a.G * planes <= 36 || whole == 0 || quarters == 0) continue;  // (an odd number of words per pixel: excluded above)
             if (shape == 11 && a.PC % 4 != 0) continue;                       // the 128x256 tiles take four-word chunks inside a tap
             const float f[kConvShapeFeatures] = {(float)a.G * (float)whole, (float)a.G * (float)quarters, (float)quarters, (float)whole, y_mb, y_mb,
                                                  1.f, 1.f, 0.f};
             for (int k = 0; k < kConvShapeFeatures; k++) cost += coefficients[k] * f[k];
-            floor_us = 1.f + (float)(4 * pieces * whole + 4 * quarters) * words * (32.f / 4.f / 2400.f);
+            floor_us = 1.f + (float)(4 * (uint64_t)pieces * whole + 4 * quarters) * words * (32.f / 4.f / 2400.f);
         } else {
-            const float n = (float)((tiles + cus - 1) / cus), rounds = (float)(((tiles + cus - 1) / cus + held - 1) / held);
-            const float busy = tiles >= cus ? 1.f : (float)tiles / (float)cus;
+            const uint64_t busiest = whole + (rest != 0);
+            const float n = (float)busiest, rounds = (float)((busiest + (uint64_t)held - 1) / (uint64_t)held);
+            const float busy = whole != 0 ? 1.f : (float)tiles / (float)cus;
             const float f[kConvShapeFeatures] = {(float)a.G * n, (float)a.G * rounds, rounds, n, y_mb, y_mb * busy, busy, 1.f,
                                                  a.G <= 9 ? y_mb : 0.f};
             for (int k = 0; k < kConvShapeFeatures; k++) cost += coefficients[k] * f[k];
@@ -478,6 +474,22 @@ int conv_mfma_shape(int type, const ConvArgs &a, float *cost_us)
     }
     if (cost_us) *cost_us = best_cost;
     return best;
+}
+
+int conv_mfma_shape(int type, const ConvArgs &a, float *cost_us)
+{
+    // Packed output has a ranking of its own: with the one of fp32 output, and the kernel with the weights in registers wherever K is at
+    // most nine words and M at least 65536, 743 random layers took 6 % more than the best shapes' time; with this one 1.5 %.
+    // (types 4 and 5 are ranked as with fp32 output: they were not measured)
+    // Below 128 tiles of 64x64, where none of those layers lies, the ranking of fp32 output stays (one image of 41x41x192 through four
+    // layers: 26.1 us with it, 26.7 with the other), and weights in registers for K of at most two words.
+    if (a.qy == nullptr || type > 3) return conv_mfma_ranked<false>(type, a, cost_us);
+    if ((long)((a.M + 63) / 64) * (((long)a.KN + 63) / 64) >= 128) return conv_mfma_ranked<true>(type, a, cost_us);
+    if (a.G <= 2) {
+        if (cost_us) *cost_us = 0.f;
+        return 7;
+    }
+    return conv_mfma_ranked<false>(type, a, cost_us);
 }
 
 // The kernel that keeps the input patch in LDS, against the tiled one that conv_mfma_shape picks: the shape with the lowest predicted
@@ -505,20 +517,16 @@ PatchPlan conv_patch_plan(int type, const ConvArgs &a)
     PatchPlan plan = {-1, 0, 0, 0, -1, 0};
     const Forced forced = forced_kernel();
     if (!conv_patch_considered(type, a.M, a.KN, a.KH, a.KW) || !conv_mfma_exact(a) || (type == 4 && !conv_mfma_exact_levels(a))) return plan;
-    int npix, lds_bytes;
-    auto weigh = [&](int shape, int kc) {
-        plan.shape = shape;
-        plan.kc = kc;
-        plan.npix = npix;
-        plan.lds_bytes = lds_bytes;
-        const long tiles = (a.KN + 31) / 32, pairs = (long)((a.PC + kc - 1) / kc) * patch_pairs(a.KH * a.KW, kc);
-        plan.weight_bytes = (size_t)(tiles * pairs) * 512 * patch_weight_planes(type);
-        return plan;
+    auto take = [&](int i, const PatchFit &fit) {
+        const size_t tiles = ((size_t)a.KN + 31) / 32;
+        plan = PatchPlan{kPatchShape + i, fit.kc, fit.npix, fit.lds_bytes, plan.tiled, tiles * (size_t)fit.pairs * 512 * patch_weight_planes(type)};
     };
+    auto fit_of = [&](int i) { return patch_fit(a, kPatchTile[i].rows, patch_most_words(kPatchTile[i].wave_tiles)); };
     if (forced.tm == 9 && forced.ng >= kPatchShape) {  // the test hook
         const int i = forced.ng - kPatchShape;
-        const int kc = i < kPatchShapes ? patch_chunk(a, kPatchTile[i].rows, patch_most_words(kPatchTile[i].wave_tiles), &npix, &lds_bytes) : 0;
-        return kc ? weigh(forced.ng, kc) : plan;
+        const PatchFit fit = i < kPatchShapes ? fit_of(i) : PatchFit{};
+        if (fit.kc) take(i, fit);
+        return plan;
     }
     if (a.qy != nullptr) return plan;
     float tiled_us = 0.f;
@@ -529,19 +537,18 @@ PatchPlan conv_patch_plan(int type, const ConvArgs &a)
     for (int k = 0; k < kTiledFeatures; k++) limit += kTiledCost[type][k] * t[k];
     limit = 0.985f * limit - 0.1f;
     const long kn64 = ((long)a.KN + 63) / 64;
-    const uint32_t cus = (uint32_t)device_compute_units();
-    for (int i = 0; i < kPatchShapes; i++) {
-        if (kPatchTile[i].filters >= 128 * kn64) continue;
-        const int kc = patch_chunk(a, kPatchTile[i].rows, patch_most_words(kPatchTile[i].wave_tiles), &npix, &lds_bytes);
-        if (kc == 0) continue;
-        float f[kPatchFeatures], us = 0.f;
-        patch_features(a, type, i, kc, npix, lds_bytes, cus, f);
-        for (int k = 0; k < kPatchFeatures; k++) us += kPatchCost[type][i][k] * f[k];
-        if (us < limit) {
-            limit = us;
-            weigh(kPatchShape + i, kc);
+    const PatchCall call = patch_call(a, type, (uint32_t)device_compute_units());
+    PatchFit fits[kPatchShapes];
+    for (int i = 0; i < kPatchShapes; i++) fits[i] = kPatchTwins.of[i] < i ? fits[kPatchTwins.of[i]] : fit_of(i);
+    float us[kPatchColumns];
+    patch_durations(call, fits, kPatchCost[type], us);
+    int best = -1;
+    for (int i = 0; i < kPatchShapes; i++)
+        if (us[i] < limit && kPatchTile[i].filters < 128 * kn64) {
+            limit = us[i];
+            best = i;
         }
-    }
+    if (best >= 0) take(best, fits[best]);
     return plan;
 }
 

@@ -346,14 +346,14 @@ template <int TYPE, int WM, int WN, int TM, int TN>
 hipError_t launch_patch(const ConvArgs &a, hipStream_t stream)
 {
     if (a.qy != nullptr) return hipErrorInvalidValue;  // fp32 output only: packed output comes without room for the weights
-    int npix = 0, lds_bytes = 0;
     constexpr int MOST = patch_most_words(TM * TN);
-    switch (patch_chunk(a, 32 * WM * TM, MOST, &npix, &lds_bytes)) {
+    const PatchFit fit = patch_fit(a, 32 * WM * TM, MOST);
+    switch (fit.kc) {
     case 4:
-        if constexpr (MOST == 4) return launch_patch_chunk<TYPE, WM, WN, TM, TN, 4>(a, npix, lds_bytes, stream);
+        if constexpr (MOST == 4) return launch_patch_chunk<TYPE, WM, WN, TM, TN, 4>(a, fit.npix, fit.lds_bytes, stream);
         return hipErrorInvalidValue;
-    case 2: return launch_patch_chunk<TYPE, WM, WN, TM, TN, 2>(a, npix, lds_bytes, stream);
-    case 1: return launch_patch_chunk<TYPE, WM, WN, TM, TN, 1>(a, npix, lds_bytes, stream);
+    case 2: return launch_patch_chunk<TYPE, WM, WN, TM, TN, 2>(a, fit.npix, fit.lds_bytes, stream);
+    case 1: return launch_patch_chunk<TYPE, WM, WN, TM, TN, 1>(a, fit.npix, fit.lds_bytes, stream);
     default: return hipErrorInvalidValue;
     }
 }

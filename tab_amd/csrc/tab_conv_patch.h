@@ -2,11 +2,13 @@
 // in how many chunks.
 #pragma once
 #include "tab_common.h"
+#include "tab_patch_weights.h"
 
 namespace tab {
 
 template <int KC> constexpr int kPatchItems = KC == 4 ? 2 : 3;  // pixels of the patch a thread fetches at most, KC words of each
 constexpr int kPatchLdsBytes = 64 * 1024;                       // of a workgroup
+constexpr int kCuLdsBytes = 160 * 1024;
 constexpr int kPatchThreads = 256;
 
 // Bit planes of the weights.
@@ -32,22 +34,26 @@ inline int patch_pixels(const ConvArgs &a, int rows)
     return lines > kPatchPixels || lines * PW > kPatchPixels ? kPatchPixels + 1 : lines * PW;
 }
 
-// Words of a chunk and bytes of LDS; 0 when the patch does not fit.
-inline int patch_chunk(const ConvArgs &a, int rows, int most, int *npix, int *lds_bytes)
+// What a patch takes: words of a chunk (0: it does not fit), pixels, bytes of LDS, workgroups that a CU's LDS holds (at most 4, which is
+// all that registers leave), chunks, and pairs of words multiplied (patch_pairs of every chunk).
+struct PatchFit { int kc, npix, lds_bytes, by_lds, chunks, pairs; };
+
+// The patch of `rows` output pixels in the most words a chunk, up to `most`, that fit.
+inline PatchFit patch_fit(const ConvArgs &a, int rows, int most)
 {
     const int pixels = patch_pixels(a, rows);
-    if (pixels > kPatchPixels || (int64_t)(a.OH - 1) * a.s1 + a.KH + pixels >= 65536) return 0;
+    if (pixels > kPatchPixels || (int64_t)(a.OH - 1) * a.s1 + a.KH + pixels >= 65536) return PatchFit{};
     for (int kc = a.PC == 1 ? 1 : most; kc >= 1; kc >>= 1) {
         // of four words at most one is padding, and of three words none
         if ((kc == 4 && a.PC % 4 != 0 && a.PC % 4 != 3) || (kc == 2 && a.PC == 3)) continue;
         const int planes = pixels + (kc == 1 ? 1 : 0);
         const int bytes = planes * 32 * kc * (a.PC > kc ? 2 : 1);
         if (bytes > kPatchLdsBytes || (kc == 4 && pixels > kPatchItems<4> * kPatchThreads)) continue;
-        *npix = planes;
-        *lds_bytes = bytes < 4096 ? 4096 : bytes;
-        return kc;
+        const int lds_bytes = bytes < 4096 ? 4096 : bytes;
+        const int chunks = kc == 4 ? (a.PC + 3) >> 2 : kc == 2 ? (a.PC + 1) >> 1 : a.PC;
+        return PatchFit{kc, planes, lds_bytes, 2 + (lds_bytes * 3 <= kCuLdsBytes) + (lds_bytes * 4 <= kCuLdsBytes), chunks, chunks * patch_pairs(a.KH * a.KW, kc)};
     }
-    return 0;
+    return PatchFit{};
 }
 
 // The kernel's shapes: rows and filters of a workgroup's tile, MFMA tiles of a wave, workgroups a CU holds by their registers.
@@ -60,32 +66,75 @@ struct PatchTile { int rows, filters, wave_tiles, held; };
 constexpr int kPatchShapes = 7;
 constexpr PatchTile kPatchTile[kPatchShapes] = {{256, 128, 8, 2}, {128, 128, 4, 3}, {128, 64, 2, 4}, {64, 64, 1, 4}, {256, 64, 4, 3}, {64, 256, 4, 3}, {64, 128, 2, 4}};
 
+// The first shape with the same patch.
+struct PatchTwins { int of[kPatchShapes]; };
+constexpr PatchTwins patch_twins()
+{
+    PatchTwins t = {};
+    for (int i = 0; i < kPatchShapes; i++)
+        for (int j = i; j >= 0; j--)
+            if (kPatchTile[j].rows == kPatchTile[i].rows && patch_most_words(kPatchTile[j].wave_tiles) == patch_most_words(kPatchTile[i].wave_tiles)) t.of[i] = j;
+    return t;
+}
+constexpr PatchTwins kPatchTwins = patch_twins();
+
 // What the predicted durations (tab_conv_patch_model.h) are linear in; the fit script states the same.
 constexpr int kPatchFeatures = 18, kTiledFeatures = 14;
+constexpr int kPatchColumns = 8;  // kPatchShapes and a spare one: two vectors of four
 
 // A call through shape i: the busiest CU holds n tiles in so many rounds; its loop, its patches, its chunks and its output.  Then what the
 // convolution replayed on the same operands does not show: laying out the weights, and fetching them where they are in no L2 yet, pair
 // after pair of words (N=64 7x7x512->512 TNN, 36 pairs: 11.0 us replayed, 15.1 behind its quantizer).  One word a pixel leaves little
 // but output; and rows of Y that end inside a cache line are written in parts until they go through the caches.
-inline void patch_features(const ConvArgs &a, int type, int i, int kc, int npix, int lds_bytes, uint32_t cus, float (&f)[kPatchFeatures])
+// What the shapes share is worked out once, and four shapes' sums at a time: calls of two short launches wait for the host (N=16 28x28x128
+// TNN 8.5 us of it a call), so the rule's time is theirs (with the tiled kernels' ranking 340 -> 210 ns, shapes one after the other before).
+struct PatchCall {
+    uint32_t M, KN, cus;
+    float y_mb, ragged, one, one_y_mb, ragged_uncached;
+    float weights_mb;  // of a pair of words
+};
+inline PatchCall patch_call(const ConvArgs &a, int type, uint32_t cus)
 {
-    const PatchTile &tile = kPatchTile[i];
-    const int taps = a.KH * a.KW;
-    const float chunks = (float)((a.PC + kc - 1) / kc);
-    const float pairs = chunks * (float)(kc == 1 ? (taps + 1) / 2 : taps * kc / 2), K = 2.f * pairs;  // words multiplied
-    const uint32_t tiles_m = ((uint32_t)a.M + (uint32_t)tile.rows - 1) / (uint32_t)tile.rows, tiles_n = ((uint32_t)a.KN + (uint32_t)tile.filters - 1) / (uint32_t)tile.filters;
-    const uint64_t tiles = (uint64_t)tiles_m * tiles_n;
-    const int by_lds = 160 * 1024 / lds_bytes, held = tile.held < by_lds ? tile.held : by_lds;
-    const uint64_t busiest = tiles <= 0xffffffffu ? ((uint32_t)tiles + cus - 1) / cus : (tiles + cus - 1) / cus;
-    const float n = (float)busiest, rounds = (float)((busiest + (uint32_t)held - 1) / (uint32_t)held);
-    const float busy = tiles < cus ? (float)tiles / (float)cus : 1.f;
     const float y_mb = (float)a.M * (float)a.KN * 4e-6f, ragged = a.KN % 32 ? y_mb : 0.f;
-    const float patch = (float)npix * (float)kc * chunks * 1e-3f;  // words expanded a tile
-    const float weights = (float)((a.KN + 31) / 32) * pairs * (patch_weight_planes(type) == 2 ? 1024e-6f : 512e-6f);
-    const float values[kPatchFeatures] = {1.f, busy, K * n, K * rounds, n, rounds, y_mb, y_mb * busy, patch * n, patch * rounds, chunks * rounds,
-                                          (float)tiles / (float)cus, ragged, weights, 0.01f * pairs, a.PC == 1 ? 1.f : 0.f, a.PC == 1 ? y_mb : 0.f,
-                                          ragged_rows_cached(a.M, a.KN) ? 0.f : ragged};
-    for (int k = 0; k < kPatchFeatures; k++) f[k] = values[k];
+    return PatchCall{(uint32_t)a.M, (uint32_t)a.KN, cus, y_mb, ragged, a.PC == 1 ? 1.f : 0.f, a.PC == 1 ? y_mb : 0.f,
+                     ragged_rows_cached(a.M, a.KN) ? 0.f : ragged, (float)((a.KN + 31) / 32) * (patch_weight_planes(type) == 2 ? 1024e-6f : 512e-6f)};
+}
+// The durations in the shapes whose patch fits (kc > 0); infinity in the others.  Column by column: the sums of all shapes go on at once.
+inline void patch_durations(const PatchCall &c, const PatchFit (&fits)[kPatchShapes], const float (&cost)[kPatchFeatures][kPatchColumns],
+                            float (&us)[kPatchColumns])
+{
+    float n[kPatchColumns], rounds[kPatchColumns], all[kPatchColumns], chunks[kPatchColumns], pairs[kPatchColumns], words[kPatchColumns];
+    n[kPatchShapes] = rounds[kPatchShapes] = all[kPatchShapes] = chunks[kPatchShapes] = pairs[kPatchShapes] = words[kPatchShapes] = 0.f;
+    us[kPatchShapes] = 0.f;
+#pragma unroll
+    for (int i = 0; i < kPatchShapes; i++) {
+        const PatchTile &tile = kPatchTile[i];
+        const PatchFit &fit = fits[i];
+        // M is below 2^31 and a filter's row of Y below 16 MB: fewer than 2^41 tiles
+        const uint64_t tiles = (uint64_t)((c.M + (uint32_t)tile.rows - 1) / (uint32_t)tile.rows) * ((c.KN + (uint32_t)tile.filters - 1) / (uint32_t)tile.filters);
+        const uint64_t busiest = tiles < 1u << 31 ? ((uint32_t)tiles + c.cus - 1) / c.cus : (tiles + c.cus - 1) / c.cus;
+        const int held = tile.held < fit.by_lds ? tile.held : fit.by_lds;
+        n[i] = (float)busiest;
+        rounds[i] = (float)(held == 3 ? (busiest + 2) / 3 : (busiest + (uint64_t)held - 1) >> (held >> 1));
+        all[i] = (float)tiles;
+        chunks[i] = (float)fit.chunks;
+        pairs[i] = (float)fit.pairs;
+        words[i] = (float)(fit.npix * fit.kc);
+        us[i] = fit.kc ? 0.f : INFINITY;
+    }
+    using Four = float __attribute__((ext_vector_type(4)));
+    for (int i = 0; i < kPatchColumns; i += 4) {
+        auto four = [i](const float *p) { return Four{p[i], p[i + 1], p[i + 2], p[i + 3]}; };
+        const Four vn = four(n), vrounds = four(rounds), vchunks = four(chunks), vpairs = four(pairs);
+        const Four load = four(all) * (1.f / (float)c.cus), busy = __builtin_elementwise_min(load, Four{1.f, 1.f, 1.f, 1.f});
+        const Four K = 2.f * vpairs, patch = four(words) * vchunks * 1e-3f;  // words multiplied; words expanded a tile
+        auto of = [&](int k) { return four(cost[k]); };
+        const Four sum = (of(0) + of(1) * busy + of(2) * (K * vn) + of(3) * (K * vrounds) + of(4) * vn + of(5) * vrounds) +
+                         (of(6) * c.y_mb + of(7) * (c.y_mb * busy) + of(8) * (patch * vn) + of(9) * (patch * vrounds) + of(10) * (vchunks * vrounds) + of(11) * load) +
+                         (of(12) * c.ragged + of(13) * (c.weights_mb * vpairs) + of(14) * (0.01f * vpairs) + of(15) * c.one + of(16) * c.one_y_mb +
+                          of(17) * c.ragged_uncached);
+        for (int j = 0; j < 4; j++) us[i + j] += sum[j];
+    }
 }
 
 // The call through the tiled kernel that conv_mfma_shape picks, which predicts `us` for its convolution: that prediction was fitted to even

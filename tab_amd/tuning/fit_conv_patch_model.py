@@ -191,9 +191,10 @@ def write_header(tiled, patch):
                 "// share, linear in patch_features and tiled_features (tab_conv_patch.h), per type 0 .. 4 and, for the patch kernel, shape 12 .. 18.\n"
                 "#pragma once\n#include \"tab_conv_patch.h\"\n\nnamespace tab {\n\n")
         f.write("constexpr float kTiledCost[5][kTiledFeatures] = {\n" + "".join("    {%s},\n" % rows_of(tiled[t]) for t in range(5)) + "};\n\n")
-        f.write("constexpr float kPatchCost[5][kPatchShapes][kPatchFeatures] = {\n")
+        f.write("// (a row per feature, its columns the shapes and a last one of zeros: the host adds the shapes' sums up side by side)\n"
+                "constexpr float kPatchCost[5][kPatchFeatures][kPatchColumns] = {\n")
         for t in range(5):
-            f.write("    {\n" + "".join("        {%s},\n" % rows_of(patch[t, s]) for s in SHAPES) + "    },\n")
+            f.write("    {\n" + "".join("        {%s, 0.f},\n" % rows_of([patch[t, s][k] for s in SHAPES]) for k in range(PATCH_FEATURES)) + "    },\n")
         f.write("};\n\n}  // namespace tab\n")
 
 
