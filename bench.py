@@ -423,7 +423,8 @@ def other_calls(torch, tab):
     g = torch.Generator("cuda").manual_seed(5)
     randn = lambda *shape: torch.randn(shape, generator=g, device="cuda")  # noqa: E731
     for type, N, layer in ((0, 1, (32, 32, 64, 64, 3, 3, 1, 1, 1, 1)), (2, 128, (28, 28, 256, 512, 1, 1, 0, 0, 2, 2)),
-                           (1, 5, (37, 53, 100, 75, 5, 5, 2, 1, 2, 2)), (0, 32, (56, 56, 256, 256, 3, 3, 1, 1, 1, 1))):
+                           (1, 5, (37, 53, 100, 75, 5, 5, 2, 1, 2, 2)), (0, 32, (56, 56, 256, 256, 3, 3, 1, 1, 1, 1)),
+                           (3, 256, (28, 28, 512, 512, 3, 3, 1, 0, 1, 1))):
         yield Layer(tab, torch, type, N, layer, seed=3).conv2d
     x, w = randn(64, 14, 14, 256).abs(), randn(256, 3, 3, 256).abs()
     QW, btn = tab.QuantizeFormat(w, tab.Threshold(w, 256), tab.DRF, 256, 3, 3, 256), torch.zeros(256, dtype=torch.int32, device="cuda")
