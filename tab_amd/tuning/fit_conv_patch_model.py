@@ -188,7 +188,8 @@ def write_header(tiled, patch):
 
     with open(os.path.join(CSRC, "tab_conv_patch_model.h"), "w") as f:
         f.write("// Written by tab_amd/tuning/fit_conv_patch_model.py from conv_patch_timings.txt: microseconds up to a summand that both sides\n"
-                "// share, linear in patch_features and tiled_features (tab_conv_patch.h), per type 0 .. 4 and, for the patch kernel, shape 12 .. 18.\n"
+                "// share, linear in the terms of patch_durations and in tiled_features (tab_conv_patch.h), per type 0 .. 4 and, for the patch\n"
+                "// kernel, shape 12 .. 18.\n"
                 "#pragma once\n#include \"tab_conv_patch.h\"\n\nnamespace tab {\n\n")
         f.write("constexpr float kTiledCost[5][kTiledFeatures] = {\n" + "".join("    {%s},\n" % rows_of(tiled[t]) for t in range(5)) + "};\n\n")
         f.write("// (a row per feature, its columns the shapes and a last one of zeros: the host adds the shapes' sums up side by side)\n"
