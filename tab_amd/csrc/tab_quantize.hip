@@ -92,7 +92,7 @@ template <int BITS, int LOADS = kLoadsPerLane, bool OWN = false>
 __global__ __launch_bounds__(kThreads) void quantize_rows64(const floatx4 *__restrict__ x, const Thresholds ths, uint32_t *__restrict__ q, long rows,
                                                             long rows_per_item, Div32 div_item, int32_t *btn, long items)
 {
-    quantize_rows64_block<BITS, LOADS, OWN>(x, ths, q, rows, rows_per_item, div_item, OWN ? in_eighths(blockIdx.x, ths.eighth) : blockIdx.x);
+    quantize_rows_block<BITS, LOADS, OWN>(WholeRows{}, x, ths, q, rows, rows_per_item, div_item, OWN ? in_eighths(blockIdx.x, ths.eighth) : blockIdx.x);
     const long row = (long)blockIdx.x * (4 * LOADS * kWavesPerBlock) + (threadIdx.x >> 6) * (4 * LOADS) + (threadIdx.x & 63);
     if ((threadIdx.x & 63) < 4 * LOADS) zero_counts(btn, items, row);
 }
@@ -105,10 +105,34 @@ __global__ __launch_bounds__(kThreads) void quantize_rows64_weights(const floatx
 {
     uint32_t block = blockIdx.x;
     if (pack_weights<kThreads>(job, block)) return;
-    quantize_rows64_block<BITS, LOADS, OWN>(x, ths, q, rows, rows_per_item, div_item, OWN ? in_eighths(block, ths.eighth) : block);
+    quantize_rows_block<BITS, LOADS, OWN>(WholeRows{}, x, ths, q, rows, rows_per_item, div_item, OWN ? in_eighths(block, ths.eighth) : block);
 }
 
-// The same row quantizer for a 1x1 convolution with stride and no padding, which reads only the
+// The same for any channel count and any alignment of x.  Bound like quantize_rows64 by reading x, and by the lanes that a pixel's last
+// row leaves without channels.  A tile of pixels sent through LDS, which took these tensors before, waited for its whole run and went
+// over the pixels of a wave word after word (one plane / two, before -> now, us): C=100 2 MB 4.3 / 4.7 -> 2.4 / 2.5, 8 MB 4.6 / 5.2 -> 3.0 / 3.3, 60
+// MB 13.0 / 14.9 -> 11.3 / 12.7, 300 MB 54.6 / 57.7 -> 49.6 / 54.5 (6.0 TB/s); C=494 8 MB 7.1 / 8.4 -> 2.9 / 3.1; C=1000 2 MB 8.2 / 9.8 -> 2.4 / 2.5,
+// 300 MB 121 / 147 -> 49 / 53.  32 rows a workgroup or 128 as for whole rows (C=100, 8 MB 3.0 / 4.0, 20 MB 5.8 / 5.8, 60 MB 12.4 / 11.3).
+template <int BITS, int LOADS = kLoadsPerLane, bool OWN = false>
+__global__ __launch_bounds__(kThreads) void quantize_rows_ragged(const floatx4 *__restrict__ x, const Thresholds ths, uint32_t *__restrict__ q, long rows,
+                                                                 long rows_per_item, Div32 div_item, int32_t *btn, long items, const RaggedRows ragged)
+{
+    quantize_rows_block<BITS, LOADS, OWN>(ragged, x, ths, q, rows, rows_per_item, div_item, OWN ? in_eighths(blockIdx.x, ths.eighth) : blockIdx.x);
+    const long row = (long)blockIdx.x * (4 * LOADS * kWavesPerBlock) + (threadIdx.x >> 6) * (4 * LOADS) + (threadIdx.x & 63);
+    if ((threadIdx.x & 63) < 4 * LOADS) zero_counts(btn, items, row);
+}
+
+template <int BITS, int LOADS = kLoadsPerLane, bool OWN = false>
+__global__ __launch_bounds__(kThreads) void quantize_rows_ragged_weights(const floatx4 *__restrict__ x, const Thresholds ths, uint32_t *__restrict__ q,
+                                                                         long rows, long rows_per_item, Div32 div_item, const RaggedRows ragged,
+                                                                         const WeightJob job)
+{
+    uint32_t block = blockIdx.x;
+    if (pack_weights<kThreads>(job, block)) return;
+    quantize_rows_block<BITS, LOADS, OWN>(ragged, x, ths, q, rows, rows_per_item, div_item, OWN ? in_eighths(block, ths.eighth) : block);
+}
+
+// The row quantizer for a 1x1 convolution with stride and no padding, which reads only the
 // pixels (oh*s1, ow*s2): one wave per 4*LOADS consecutive words of one output line (n, oh); the packed
 // result is the compact [N][OH][OW][PC] activation, i.e. what the conv reads with stride 1.
 // grid = (ceil(OW*PC / (4*LOADS)), N*OH), one wave per workgroup; OW*PC < 65536 (fastdiv range).
@@ -149,40 +173,55 @@ __global__ __launch_bounds__(64) void quantize_rows64_strided(const floatx4 *__r
     }
 }
 
-// quantize_rows64 of two planes with counts (see Counts): a slice is one unit, 4 * LOADS rows of every wave.
-template <int LOADS, bool NT>
-__global__ __launch_bounds__(kThreads) void quantize_rows64_count(const floatx4 *__restrict__ x, const Thresholds ths, uint32_t *__restrict__ q,
-                                                                    long rows_per_item, const Counts counts)
+// Two planes with counts (see Counts): a slice is one unit, 4 * LOADS rows of every wave.
+template <int LOADS, bool NT, class Rows>
+__device__ __forceinline__ void quantize_rows_counted(const Rows kind, const floatx4 *__restrict__ x, const Thresholds &ths, uint32_t *__restrict__ q,
+                                                      long rows_per_item, const Counts &counts, int32_t *scratch)
 {
     constexpr int UNIT = 4 * LOADS * kWavesPerBlock;
-    __shared__ int32_t scratch[kWavesPerBlock];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int sub = lane >> 4, l = lane & 15;
     const int item = (int)(blockIdx.x / (uint32_t)counts.slices), slice = (int)blockIdx.x - item * counts.slices;
-    const long first = item * rows_per_item;
     int count = 0;
     const long at = (long)slice * UNIT + wave * (4 * LOADS);  // of the item's rows
     if (at < rows_per_item) {
-        floatx4 v[LOADS];
-#pragma unroll
-        for (int u = 0; u < LOADS; u++) {
-            const long r = at + u * 4 + sub;
-            const floatx4 *src = &x[(first + (r < rows_per_item ? r : rows_per_item - 1)) * 16 + l];
-            v[u] = NT ? __builtin_nontemporal_load(src) : *src;
-        }
+        const long first = item * rows_per_item + at;
+        const uint32_t live = (uint32_t)(rows_per_item - at < 4 * LOADS ? rows_per_item - at : 4 * LOADS);
+        RowLoads<LOADS> held;
+        load_rows<NT>(kind, x, first, live, sub, l, held);
         const float t = given_threshold(ths, item);
 #pragma unroll
         for (int u = 0; u < LOADS; u++) {
-            const long r = at + u * 4 + sub;
+            const uint32_t r = u * 4 + sub;
             uint32_t sign, nz, out[4];
-            compare4<2>(v[u], t, sign, nz);
-            count += r < rows_per_item ? __builtin_popcount(nz) : 0;
+            compare4<2>(held.v[u], t, sign, nz);
+            if (std::is_same<Rows, RaggedRows>::value) {
+                sign &= held.exist[u];
+                nz &= held.exist[u];
+            }
+            count += r < live ? __builtin_popcount(nz) : 0;
             pack_row<2>(sign, nz, l, out);
-            if (r < rows_per_item && l == 0) *reinterpret_cast<uintx4 *>(q + (first + r) * 4) = uintx4{out[0], out[1], out[2], out[3]};
+            if (r < live && l == 0) *reinterpret_cast<uintx4 *>(q + (first + r) * 4) = uintx4{out[0], out[1], out[2], out[3]};
         }
     }
     store_count<kWavesPerBlock>(count, counts.out + blockIdx.x, scratch);
+}
+
+template <int LOADS, bool NT>
+__global__ __launch_bounds__(kThreads) void quantize_rows64_count(const floatx4 *__restrict__ x, const Thresholds ths, uint32_t *__restrict__ q,
+                                                                  long rows_per_item, const Counts counts)
+{
+    __shared__ int32_t scratch[kWavesPerBlock];
+    quantize_rows_counted<LOADS, NT>(WholeRows{}, x, ths, q, rows_per_item, counts, scratch);
+}
+
+template <int LOADS, bool NT>
+__global__ __launch_bounds__(kThreads) void quantize_rows_ragged_count(const floatx4 *__restrict__ x, const Thresholds ths, uint32_t *__restrict__ q,
+                                                                       long rows_per_item, const Counts counts, const RaggedRows ragged)
+{
+    __shared__ int32_t scratch[kWavesPerBlock];
+    quantize_rows_counted<LOADS, NT>(ragged, x, ths, q, rows_per_item, counts, scratch);
 }
 
 // A convolution's weights alone.
@@ -192,42 +231,40 @@ __global__ __launch_bounds__(kThreads) void patch_weights(const WeightJob job)
     pack_weights<kThreads>(job, block);
 }
 
-// General path: any C, any alignment of x, every format (MODE as in compare4).  A workgroup takes a tile of consecutive pixels,
+// Up to 32 channels, any alignment of x, every format (MODE as in compare4), where a row of 16 lanes a pixel would be mostly empty: a
+// workgroup takes a tile of consecutive pixels,
 // whose channels are one contiguous run of x, sends the run to LDS in granules of 16 bytes, and its waves then read the words
-// out of it: LP lanes a word (the smallest power of two that holds it; 64 / LP pixels a read where a pixel is one word), so
+// out of it: LP lanes a word (the smallest power of two that holds it; 64 / LP pixels a read), so
 // that one compare makes the bits of a whole read as a wave mask (LSB first; onebit[i] = 1 << i, TAB_GEMM.cu:252-258).  Lane
 // i keeps the word of the wave's pixel i.  Unused high bits of a tail word stay 0
 // (TAB_GEMM.cu:203-206).
 // Bound by reading x and by the waits of a tile for its run: the 16-byte loads do not care where pixels begin, and a word costs
-// six to twelve instructions.  With 4-byte loads a lane and row, ORed together over the lanes of a word (one plane / two, before
-// -> now, us): 64x56x56x100 21.5 / 23.1 -> 16.0 / 18.3, x200 38 / 41 -> 27 / 32, 64x112x112x32 31 / 33 -> 18.0 / 18.6, 64x224x224x3
-// 19.3 / 25.0 -> 13.3 / 16.8, 5x37x53x100 5.3 / 5.8 -> 3.9 / 4.0; formats 4 and 5 had one wave per word.
+// six to twelve instructions.  Against 4-byte loads a lane and row, ORed together over the lanes of a word (one plane / two, us):
+// 64x112x112x32 31 / 33 -> 18.0 / 18.6, 64x224x224x3 19.3 / 25.0 -> 13.3 / 16.8; 60 MB against rows of 16 lanes (quantize_rows_ragged):
+// C=5 68 / 85 -> 16.5 / 20.7, C=27 15.2 / 18.3 -> 11.8 / 13.2.
 // Formats 4 and 5 belong to the CPU-only conv types, whose layouts follow from the reference's GEMMs (it has no quantizer for
 // them: TAB_Conv calls Parallel_Binarize_NCHW and Parallel_Ternarize_RTN, TAB_CPU.cpp:522,527, which no file defines):
 // 4, DoReFa 2-bit (DRFGEMM_baseline, TAB_CPU.cpp:345-354): [pixel][ceil(C/64)][2], plane 0 the weight-2 bit and plane 1 the
 //    weight-1 bit of level = (v >= 0.5t) + (v >= 1.5t) + (v >= 2.5t);
 // 5, RTN (RTNGEMM_baseline, TAB_CPU.cpp:364-379; 32 channels per word, 520-521): [pixel][ceil(C/32)], channel c in word c/32
 //    as the field (bit 2*(c%32) = nonzero, bit 2*(c%32)+1 = sign) of the ternarizer's value.
-// One tile: `live` pixels from p0 on, `words` words a pixel from w0 on.  Returns how many of the values this lane stored are nonzero
-// (MODE 2).
+// One tile: `live` pixels from p0 on.  Returns how many of the values this lane stored are nonzero (MODE 2).
 template <int MODE, int LP>
 __device__ __forceinline__ int quantize_one_tile(const float *__restrict__ x, const Thresholds &ths, uint64_t *__restrict__ q, long p0, int live,
-                                                 long pixels_per_item, Div32 div_item, int C, int tile_pixels, int w0, int words)
+                                                 long pixels_per_item, Div32 div_item, int C, int tile_pixels)
 {
+    static_assert(LP <= 32, "a word of 32 bits or less");
     constexpr int G = 64 / LP;  // rows per read
-    constexpr int U = LP == 64 ? 4 : 2;  // reads in flight
+    constexpr int U = 2;        // reads in flight
     extern __shared__ __attribute__((aligned(16))) uint32_t tile[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int PC = (C + kWordBits - 1) / kWordBits;
     int count = 0;
-    // words w0 ... of the pixel where one pixel is more than a tile (`words` of them), else all
-    const int PW = min(words, PC - w0), channels_here = min(C - w0 * kWordBits, PW * kWordBits);
 
     // ---- the run of x, from the 16-byte boundary at or below its start to its last float ----------------------------------
-    const uintptr_t start = (uintptr_t)(x + p0 * C + w0 * kWordBits);
+    const uintptr_t start = (uintptr_t)(x + p0 * C);
     const int skew = (int)(start & 15) / 4;  // floats
-    const int floats = (live - 1) * C + channels_here + skew;
+    const int floats = live * C + skew;
     const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(start & ~(uintptr_t)15), 0, floats * 4, kBufferFlags);
     for (int i = wave * 64; i * 4 < floats; i += kThreads) load16_to_lds(rsrc, tile + i * 4, (uint32_t)(i + lane) * 16u);
 
@@ -235,7 +272,7 @@ __device__ __forceinline__ int quantize_one_tile(const float *__restrict__ x, co
     auto item_of = [&](long pixel) { return div_item.mul ? (long)div32((uint32_t)pixel, div_item) : pixel / pixels_per_item; };
     const long item_first = item_of(p0);
     const bool one_item = item_of(p0 + live - 1) == item_first;
-    float *const th = reinterpret_cast<float *>(tile + ((tile_pixels - 1) * C + channels_here + 3 + 3) / 4 * 4 + 256);
+    float *const th = reinterpret_cast<float *>(tile + (tile_pixels * C + 3 + 3) / 4 * 4 + 256);
     const float t_first = wave_threshold(ths, item_first);
     if (!one_item)
         for (int i0 = wave * 64; i0 < live; i0 += kThreads) {
@@ -247,85 +284,70 @@ __device__ __forceinline__ int quantize_one_tile(const float *__restrict__ x, co
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
 
-    // ---- words: the wave's pixels of the tile, word after word, 64 pixels at a time; a read takes G of them -------------------------
+    // ---- words: the wave's pixels of the tile, 64 at a time; a read takes G of them -------------------------------------------------
     const int share = ((live + 3) / 4 + G - 1) / G * G;
     const int end = min(live, (wave + 1) * share);
     const float *const run = reinterpret_cast<const float *>(tile) + skew;
-    const int ch = LP == 64 ? lane : lane % LP;
-    for (int px0 = wave * share; px0 < end; px0 += 64)
-        for (int w = 0; w < PW; w++) {
-            const int channels = min(channels_here - w * kWordBits, kWordBits);
-            const uint64_t exist = __ballot(ch < channels);
-            const float *src = run + px0 * C + w * kWordBits + (lane / LP) * C + min(ch, channels - 1);
-            const int reads = (min(end - px0, 64) + G - 1) / G;
-            uint32_t out[4] = {0, 0, 0, 0};  // of pixel px0 + lane: plane 0 low, high, plane 1 low, high
-            for (int j0 = 0; j0 < reads; j0 += U) {
-                float v[U], t[U];
+    const int ch = lane % LP;
+    const uint64_t exist = __ballot(ch < C);
+    for (int px0 = wave * share; px0 < end; px0 += 64) {
+        const float *src = run + px0 * C + (lane / LP) * C + min(ch, C - 1);
+        const int reads = (min(end - px0, 64) + G - 1) / G;
+        uint32_t out0 = 0, out1 = 0;  // the planes' low halves of pixel px0 + lane; the high ones are zero
+        for (int j0 = 0; j0 < reads; j0 += U) {
+            float v[U], t[U];
 #pragma unroll
-                for (int u = 0; u < U; u++) {  // (reads past the tile's last pixel: that of the first, kept by no lane)
-                    const bool past = px0 + (j0 + u) * G + lane / LP >= live;
-                    v[u] = src[past ? 0 : (j0 + u) * G * C];
-                    t[u] = one_item ? t_first : th[past ? 0 : px0 + (j0 + u) * G + lane / LP];
-                }
-#pragma unroll
-                for (int u = 0; u < U; u++) {
-                    uint64_t m0, m1 = 0;
-                    if (MODE == 1) {
-                        m0 = __ballot(v[u] < t[u]) & exist;
-                    } else if (MODE == 4) {
-                        const uint64_t l1 = __ballot(v[u] >= 0.5f * t[u]), l2 = __ballot(v[u] >= 1.5f * t[u]), l3 = __ballot(v[u] >= 2.5f * t[u]);
-                        // level = number of bounds reached, whatever their order (t may be negative)
-                        m0 = ((l1 & l2) | (l1 & l3) | (l2 & l3)) & exist;
-                        m1 = (l1 ^ l2 ^ l3) & exist;
-                    } else {
-                        const uint64_t pos = __ballot(v[u] > t[u]);
-                        m0 = __ballot(v[u] < -t[u]) & ~pos & exist;
-                        m1 = (pos & exist) | m0;
-                    }
-                    // lane j * G + g keeps the LP bits of the read's pixel g
-                    const bool mine = lane / G == j0 + u;
-                    if (LP == 64) {
-                        out[0] = mine ? (uint32_t)m0 : out[0];
-                        out[1] = mine ? (uint32_t)(m0 >> 32) : out[1];
-                        if (MODE != 1) {
-                            out[2] = mine ? (uint32_t)m1 : out[2];
-                            out[3] = mine ? (uint32_t)(m1 >> 32) : out[3];
-                        }
-                    } else {
-                        const int shift = LP * (lane % G);
-                        constexpr uint32_t bits = LP >= 32 ? ~0u : (1u << (LP & 31)) - 1;
-                        out[0] = mine ? (uint32_t)(m0 >> shift) & bits : out[0];
-                        if (MODE != 1) out[2] = mine ? (uint32_t)(m1 >> shift) & bits : out[2];
-                    }
-                }
+            for (int u = 0; u < U; u++) {  // (reads past the tile's last pixel: that of the first, kept by no lane)
+                const bool past = px0 + (j0 + u) * G + lane / LP >= live;
+                v[u] = src[past ? 0 : (j0 + u) * G * C];
+                t[u] = one_item ? t_first : th[past ? 0 : px0 + (j0 + u) * G + lane / LP];
             }
-            if (px0 + lane < end) {
-                const size_t pixel = (size_t)p0 + px0 + lane, at = pixel * PC + w0 + w;
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                uint64_t m0, m1 = 0;
                 if (MODE == 1) {
-                    *reinterpret_cast<uintx2 *>(q + at) = uintx2{out[0], out[1]};
-                } else if (MODE == 5) {
-                    // 32 channels a word: 64 are two words, or one where the last 32 of a pixel do not exist
-                    const int halves = (C + 31) / 32;
-                    uint64_t *dst = q + pixel * halves + 2 * (w0 + w);
-                    dst[0] = spread_bits(out[2]) | spread_bits(out[0]) << 1;
-                    if (2 * (w0 + w) + 1 < halves) dst[1] = spread_bits(out[3]) | spread_bits(out[1]) << 1;
+                    m0 = __ballot(v[u] < t[u]) & exist;
+                } else if (MODE == 4) {
+                    const uint64_t l1 = __ballot(v[u] >= 0.5f * t[u]), l2 = __ballot(v[u] >= 1.5f * t[u]), l3 = __ballot(v[u] >= 2.5f * t[u]);
+                    // level = number of bounds reached, whatever their order (t may be negative)
+                    m0 = ((l1 & l2) | (l1 & l3) | (l2 & l3)) & exist;
+                    m1 = (l1 ^ l2 ^ l3) & exist;
                 } else {
-                    *reinterpret_cast<uintx4 *>(q + 2 * at) = uintx4{out[0], out[1], out[2], out[3]};
-                    if (MODE == 2) count += __builtin_popcount(out[2]) + __builtin_popcount(out[3]);
+                    const uint64_t pos = __ballot(v[u] > t[u]);
+                    m0 = __ballot(v[u] < -t[u]) & ~pos & exist;
+                    m1 = (pos & exist) | m0;
                 }
+                // lane j * G + g keeps the LP bits of the read's pixel g
+                const bool mine = lane / G == j0 + u;
+                const int shift = LP * (lane % G);
+                constexpr uint32_t bits = LP >= 32 ? ~0u : (1u << (LP & 31)) - 1;
+                out0 = mine ? (uint32_t)(m0 >> shift) & bits : out0;
+                if (MODE != 1) out1 = mine ? (uint32_t)(m1 >> shift) & bits : out1;
             }
         }
+        if (px0 + lane < end) {
+            const size_t pixel = (size_t)p0 + px0 + lane;
+            if (MODE == 1) {
+                *reinterpret_cast<uintx2 *>(q + pixel) = uintx2{out0, 0};
+            } else if (MODE == 5) {
+                q[pixel] = spread_bits(out1) | spread_bits(out0) << 1;  // one word of 32 fields
+            } else {
+                *reinterpret_cast<uintx4 *>(q + 2 * pixel) = uintx4{out0, 0, out1, 0};
+                if (MODE == 2) count += __builtin_popcount(out1);
+            }
+        }
+    }
     return count;
 }
 
 template <int MODE, int LP>
 __global__ __launch_bounds__(kThreads) void quantize_tile(const float *__restrict__ x, const Thresholds ths, uint64_t *__restrict__ q,
-                                                          long pixels, long pixels_per_item, Div32 div_item, int C, int tile_pixels, int words,
+                                                          long pixels, long pixels_per_item, Div32 div_item, int C, int tile_pixels,
                                                           int32_t *btn, long items)
 {
     const long p0 = (long)in_eighths(blockIdx.x, ths.eighth) * tile_pixels;
     const int live = pixels - p0 < tile_pixels ? (int)(pixels - p0) : tile_pixels;  // pixels of the tile that exist
-    quantize_one_tile<MODE, LP>(x, ths, q, p0, live, pixels_per_item, div_item, C, tile_pixels, blockIdx.y * words, words);
+    quantize_one_tile<MODE, LP>(x, ths, q, p0, live, pixels_per_item, div_item, C, tile_pixels);
     for (int i = threadIdx.x; i < live; i += kThreads) zero_counts(btn, items, p0 + i);
 }
 
@@ -333,14 +355,13 @@ __global__ __launch_bounds__(kThreads) void quantize_tile(const float *__restric
 template <int MODE, int LP>
 __global__ __launch_bounds__(kThreads) void quantize_tile_weights(const float *__restrict__ x, const Thresholds ths, uint64_t *__restrict__ q,
                                                                   long pixels, long pixels_per_item, Div32 div_item, int C, int tile_pixels,
-                                                                  int words, const WeightJob job)
+                                                                  const WeightJob job)
 {
     uint32_t block = blockIdx.x;
-    if (blockIdx.y != 0 && block < job.blocks) return;  // (the grid's other parts of a pixel)
     if (pack_weights<kThreads>(job, block)) return;
     const long p0 = (long)in_eighths(block, ths.eighth) * tile_pixels;
     const int live = pixels - p0 < tile_pixels ? (int)(pixels - p0) : tile_pixels;  // pixels of the tile that exist
-    quantize_one_tile<MODE, LP>(x, ths, q, p0, live, pixels_per_item, div_item, C, tile_pixels, blockIdx.y * words, words);
+    quantize_one_tile<MODE, LP>(x, ths, q, p0, live, pixels_per_item, div_item, C, tile_pixels);
 }
 
 // The same with counts (see Counts); a unit is a tile of whole pixels.
@@ -354,8 +375,7 @@ __global__ __launch_bounds__(kThreads) void quantize_tile_count(const float *__r
     for (long at = (long)slice * tile_pixels; at < pixels_per_item; at += (long)counts.slices * tile_pixels) {
         const int live = pixels_per_item - at < tile_pixels ? (int)(pixels_per_item - at) : tile_pixels;
         if (at >= (long)counts.slices * tile_pixels) __syncthreads();  // the waves have read the tile before
-        count += quantize_one_tile<2, LP>(x, ths, q, item * pixels_per_item + at, live, pixels_per_item, div_item, C, tile_pixels, 0,
-                                          (C + kWordBits - 1) / kWordBits);
+        count += quantize_one_tile<2, LP>(x, ths, q, item * pixels_per_item + at, live, pixels_per_item, div_item, C, tile_pixels);
     }
     store_count<kWavesPerBlock>(count, counts.out + blockIdx.x, scratch);
 }
@@ -938,20 +958,13 @@ template <int MODE, int LP>
 void launch_quantize_tile_of(const float *x, const Thresholds &ths, long pixels, long pixels_per_item, long items, int C, uint64_t *q,
                              int32_t *btn, const CountTarget *counted, const WeightJob *weights, hipStream_t stream)
 {
-    // Bytes of x in a tile, measured from 4 to 48 KB on C = 3 ... 700: what a few workgroups a CU keep in flight against the
-    // wait of each for its whole tile.  The pixels are shared by four waves in turns of U reads, so sixteen (a turn of four
-    // each) are worth more than the bytes: C=200 41 us at 8 pixels, 32 at 16, 27 at 32.
-    const int PC = (C + kWordBits - 1) / kWordBits;
-    const long bytes = LP < 64 ? 12 * 1024 : (C <= 128 ? 20 * 1024 : 32 * 1024);
-    const long fit = bytes / (4L * C);
-    // a pixel of more than 3072 channels goes in parts of 64 words
-    const int words = C <= 3072 ? PC : 64;
-    long tile_pixels = C > 3072 ? 1 : (fit >= 16 ? fit / 16 * 16 : (C <= 768 ? 16 : 4));
+    // 12 KB of x a tile, measured from 4 to 48 KB on C = 3 ... 32: what a few workgroups a CU keep in flight against the
+    // wait of each for its whole tile.
+    long tile_pixels = 12 * 1024 / (4L * C) / 16 * 16;
     const bool one_slice = counted && pixels_per_item <= kOneSliceUnits * tile_pixels;
     // a tensor of few tiles: smaller ones, down to a read of every wave
     while (!one_slice && tile_pixels >= 8 && pixels / tile_pixels < 512 && tile_pixels / 2 >= 4 * (64 / LP)) tile_pixels = tile_pixels / 8 * 4;
-    const long run = C > 3072 ? words * kWordBits : tile_pixels * C;
-    const size_t lds = ((size_t)(run + 6) / 4 * 4 + 256 + tile_pixels) * 4;
+    const size_t lds = ((size_t)(tile_pixels * C + 6) / 4 * 4 + 256 + tile_pixels) * 4;
     const Div32 div_item = pixels < 0x7fffffffL ? make_div32((uint32_t)pixels_per_item) : Div32{0, 0};
     if constexpr (MODE == 2) {
         if (counted) {
@@ -962,18 +975,18 @@ void launch_quantize_tile_of(const float *x, const Thresholds &ths, long pixels,
             return;
         }
     }
-    const dim3 grid((unsigned)((pixels + tile_pixels - 1) / tile_pixels), (unsigned)((PC + words - 1) / words));
+    const unsigned tiles = (unsigned)((pixels + tile_pixels - 1) / tile_pixels);
     if constexpr (MODE != 5) {  // (type 5 has no kernel that reads its weights in another order)
         if (weights) {
-            quantize_tile_weights<MODE, LP><<<dim3(grid.x + weights->blocks, grid.y), dim3(kThreads), lds, stream>>>(
-                x, grid.y == 1 ? ordered(ths, grid.x) : ordered(ths, 0), q, pixels, pixels_per_item, div_item, C, (int)tile_pixels, words, *weights);
+            quantize_tile_weights<MODE, LP><<<dim3(tiles + weights->blocks), dim3(kThreads), lds, stream>>>(
+                x, ordered(ths, tiles), q, pixels, pixels_per_item, div_item, C, (int)tile_pixels, *weights);
             return;
         }
     }
-    quantize_tile<MODE, LP><<<grid, dim3(kThreads), lds, stream>>>(x, grid.y == 1 ? ordered(ths, grid.x) : ordered(ths, 0), q, pixels, pixels_per_item, div_item, C, (int)tile_pixels, words, btn, items);
+    quantize_tile<MODE, LP><<<dim3(tiles), dim3(kThreads), lds, stream>>>(x, ordered(ths, tiles), q, pixels, pixels_per_item, div_item, C, (int)tile_pixels, btn, items);
 }
 
-// The general path with the fewest lanes a word that hold it.
+// Up to 32 channels with the fewest lanes a word that hold it.
 template <int MODE>
 void launch_quantize_tile(const float *x, const Thresholds &ths, long pixels, long pixels_per_item, long items, int C, uint64_t *q,
                           int32_t *btn, const CountTarget *counted, const WeightJob *weights, hipStream_t stream)
@@ -981,8 +994,7 @@ void launch_quantize_tile(const float *x, const Thresholds &ths, long pixels, lo
     if (C <= 4) launch_quantize_tile_of<MODE, 4>(x, ths, pixels, pixels_per_item, items, C, q, btn, counted, weights, stream);
     else if (C <= 8) launch_quantize_tile_of<MODE, 8>(x, ths, pixels, pixels_per_item, items, C, q, btn, counted, weights, stream);
     else if (C <= 16) launch_quantize_tile_of<MODE, 16>(x, ths, pixels, pixels_per_item, items, C, q, btn, counted, weights, stream);
-    else if (C <= 32) launch_quantize_tile_of<MODE, 32>(x, ths, pixels, pixels_per_item, items, C, q, btn, counted, weights, stream);
-    else launch_quantize_tile_of<MODE, 64>(x, ths, pixels, pixels_per_item, items, C, q, btn, counted, weights, stream);
+    else launch_quantize_tile_of<MODE, 32>(x, ths, pixels, pixels_per_item, items, C, q, btn, counted, weights, stream);
 }
 
 // Counts of every two-plane quantizer in slices: workspace ints at most (a unit holds at least four words).
@@ -993,19 +1005,53 @@ size_t quantize_count_workspace(int bitwidth, long items, long pixels_per_item, 
     return (size_t)items * (pixels_per_item * PC / 4 + PC + 1) * sizeof(int32_t);
 }
 
-hipError_t launch_rows64_weights(const float *x, const Thresholds &ths, int format, long rows, long rows_per_item, Div32 div_item, uint64_t *qx,
-                                 const WeightJob &job, hipStream_t stream)
+// Which path packs an NHWC tensor: a pixel of up to 32 channels leaves half of a row's 16 lanes and more without work, and tiles are as soon
+// or sooner at every size (tile / rows, one plane, us: C=32 0.6 MB 2.5 / 2.5, 9.6 MB 3.8 / 4.2; C=16 1.2 MB 2.8 / 2.8, 9.6 MB 3.8 / 4.9; C=5 1.2
+// MB 3.0 / 3.8, 60 MB 16.5 / 51); from 33 on rows are (C=33 2 MB 3.4 / 2.4, 150 MB 30.9 / 27.6).
+enum class Path { whole, ragged, tile };
+Path quantize_path(const float *x, int C)
 {
-    auto launch = [&](auto kernel, long rows_per_block, int lds) {
-        kernel<<<dim3((unsigned)((rows + rows_per_block - 1) / rows_per_block) + job.blocks), dim3(kThreads), lds, stream>>>(
-            reinterpret_cast<const floatx4 *>(x), ordered(ths, (rows + rows_per_block - 1) / rows_per_block), reinterpret_cast<uint32_t *>(qx), rows, rows_per_item, div_item, job);
-    };
-    // (sizes of workgroups as in launch_quantize)
-    const bool own = ths.splits > 0;
-    if (rows <= kSmallLaunchBlocks * 128)
-        launch(format == 4 ? quantize_rows64_weights<4, 2> : format == 1 ? quantize_rows64_weights<1, 2> : own ? quantize_rows64_weights<2, 2, true> : quantize_rows64_weights<2, 2>, 32, 0);
-    else
-        launch(format == 4 ? quantize_rows64_weights<4> : format == 1 ? quantize_rows64_weights<1> : own ? quantize_rows64_weights<2, 8, true> : quantize_rows64_weights<2>, 128, kStreamLds);
+    if (C % kWordBits == 0 && (uintptr_t)x % 16 == 0) return Path::whole;
+    return C > 32 ? Path::ragged : Path::tile;
+}
+
+// Rows of 64 channels without counts.  A launch too small to fill the chip with 128 rows a workgroup takes 32, two loads a lane (3.1 MB
+// of fp32: 5.5 -> 4.2 us).
+template <int FORMAT>
+hipError_t launch_rows(Path path, const float *x, const Thresholds &ths, long pixels, long pixels_per_item, long items, int C, uint64_t *qx,
+                       int32_t *zeroed, const WeightJob *weights, hipStream_t stream)
+{
+    constexpr bool SUMS = FORMAT == 2;      // thresholds as partial sums
+    constexpr bool BESIDE = FORMAT != 5;    // (type 5 has no kernel that reads its weights in another order)
+    const long PC = (C + kWordBits - 1) / kWordBits, rows = pixels * PC, rows_per_item = pixels_per_item * PC;
+    const Div32 div_item = rows < 0x7fffffffL ? make_div32((uint32_t)rows_per_item) : Div32{0, 0};
+    const bool few = rows <= kSmallLaunchBlocks * 128, own = SUMS && ths.splits > 0;
+    const long blocks = (rows + (few ? 31 : 127)) / (few ? 32 : 128);
+    const Thresholds t = ordered(ths, blocks);
+    const dim3 grid((unsigned)(blocks + (weights ? weights->blocks : 0)));
+    const int lds = few ? 0 : kStreamLds;
+    const floatx4 *x4 = reinterpret_cast<const floatx4 *>(x);
+    uint32_t *q32 = reinterpret_cast<uint32_t *>(qx);
+    if (path == Path::whole) {
+        if (BESIDE && weights) {
+            auto kernel = few ? own ? quantize_rows64_weights<BESIDE ? FORMAT : 1, 2, SUMS> : quantize_rows64_weights<BESIDE ? FORMAT : 1, 2>
+                              : own ? quantize_rows64_weights<BESIDE ? FORMAT : 1, 8, SUMS> : quantize_rows64_weights<BESIDE ? FORMAT : 1>;
+            kernel<<<grid, dim3(kThreads), lds, stream>>>(x4, t, q32, rows, rows_per_item, div_item, *weights);
+        } else {
+            auto kernel = few ? own ? quantize_rows64<FORMAT, 2, SUMS> : quantize_rows64<FORMAT, 2> : own ? quantize_rows64<FORMAT, 8, SUMS> : quantize_rows64<FORMAT>;
+            kernel<<<grid, dim3(kThreads), lds, stream>>>(x4, t, q32, rows, rows_per_item, div_item, zeroed, items);
+        }
+    } else {
+        const RaggedRows ragged{C, make_div32((uint32_t)PC)};
+        if (BESIDE && weights) {
+            auto kernel = few ? own ? quantize_rows_ragged_weights<BESIDE ? FORMAT : 1, 2, SUMS> : quantize_rows_ragged_weights<BESIDE ? FORMAT : 1, 2>
+                              : own ? quantize_rows_ragged_weights<BESIDE ? FORMAT : 1, 8, SUMS> : quantize_rows_ragged_weights<BESIDE ? FORMAT : 1>;
+            kernel<<<grid, dim3(kThreads), lds, stream>>>(x4, t, q32, rows, rows_per_item, div_item, ragged, *weights);
+        } else {
+            auto kernel = few ? own ? quantize_rows_ragged<FORMAT, 2, SUMS> : quantize_rows_ragged<FORMAT, 2> : own ? quantize_rows_ragged<FORMAT, 8, SUMS> : quantize_rows_ragged<FORMAT>;
+            kernel<<<grid, dim3(kThreads), lds, stream>>>(x4, t, q32, rows, rows_per_item, div_item, zeroed, items, ragged);
+        }
+    }
     return hipGetLastError();
 }
 
@@ -1021,53 +1067,41 @@ hipError_t launch_quantize(const float *x, const Thresholds &ths, int bitwidth, 
     const int splits = btn && bitwidth == 2 ? count_splits(items, words_per_item) : 1;
     // counts that are not stored whole by btn_popcount start at zero
     int32_t *zeroed = btn && (bitwidth != 2 || splits > 1) ? btn : nullptr;
-    const bool fast = (C % kWordBits == 0) && ((uintptr_t)x % 16 == 0);
+    const Path path = quantize_path(x, C);
     const CountTarget target{btn, count_workspace};
     const bool counted = btn && bitwidth == 2 && items * (words_per_item / 4 + 1) < 0x7fffffffL &&
                          (count_workspace || (words_per_item <= 64 && PC <= kOneSliceUnits));
-    if (counted && fast) {
+    if (counted && path != Path::tile) {
         const floatx4 *x4 = reinterpret_cast<const floatx4 *>(x);
         uint32_t *q32 = reinterpret_cast<uint32_t *>(qx);
-        auto launch = [&](auto kernel, long rows, int lds) {
+        auto launch = [&](auto whole, auto ragged, long rows, int lds) {
             const long slices = (words_per_item + rows - 1) / rows;
-            kernel<<<dim3((unsigned)(items * slices)), dim3(kThreads), lds, stream>>>(
-                x4, ths, q32, words_per_item, Counts{slices == 1 ? btn : count_workspace, (int)slices});
+            const dim3 grid((unsigned)(items * slices));
+            const Counts counts{slices == 1 ? btn : count_workspace, (int)slices};
+            if (path == Path::whole) whole<<<grid, dim3(kThreads), lds, stream>>>(x4, ths, q32, words_per_item, counts);
+            else ragged<<<grid, dim3(kThreads), lds, stream>>>(x4, ths, q32, words_per_item, counts, RaggedRows{C, make_div32((uint32_t)PC)});
             finish_counts(target, items, (int)slices, stream);
         };
-        // (units of 128 rows for streaming and 32 for launches too small to fill the chip, as below)
-        if (words_per_item > 32 && words_per_item <= 128) launch(quantize_rows64_count<8, false>, 128, 0);
-        else if (items * words_per_item <= kSmallLaunchBlocks * 128) launch(quantize_rows64_count<2, false>, 32, 0);
-        else launch(quantize_rows64_count<8, true>, 128, kStreamLds);
+        // (units of 128 rows for streaming and 32 for launches too small to fill the chip, as above)
+        if (words_per_item > 32 && words_per_item <= 128) launch(quantize_rows64_count<8, false>, quantize_rows_ragged_count<8, false>, 128, 0);
+        else if (items * words_per_item <= kSmallLaunchBlocks * 128) launch(quantize_rows64_count<2, false>, quantize_rows_ragged_count<2, false>, 32, 0);
+        else launch(quantize_rows64_count<8, true>, quantize_rows_ragged_count<8, true>, 128, kStreamLds);
         return hipGetLastError();
     }
-    if (counted && C <= 3072) {
+    if (counted) {
         launch_quantize_tile<2>(x, ths, pixels, pixels_per_item, items, C, qx, nullptr, &target, nullptr, stream);
         return hipGetLastError();
     }
-    if (fast) {
-        const long rows = pixels * PC;
-        const Div32 div_item = rows < 0x7fffffffL ? make_div32((uint32_t)words_per_item) : Div32{0, 0};
-        const long blocks = (rows + kRowsPerWave * kWavesPerBlock - 1) / (kRowsPerWave * kWavesPerBlock);
-        const dim3 block(kThreads);
-        const floatx4 *x4 = reinterpret_cast<const floatx4 *>(x);
-        uint32_t *q32 = reinterpret_cast<uint32_t *>(qx);
-        if (weights) return launch_rows64_weights(x, ths, bitwidth, rows, words_per_item, div_item, qx, *weights, stream);
-        if (blocks <= kSmallLaunchBlocks) {
-            // a tensor too small to fill the chip with 128-row workgroups: 32 rows per workgroup, two loads per lane
-            // (3.1 MB of fp32: 5.5 -> 4.2 us)
-            const dim3 grid((unsigned)((rows + 8 * kWavesPerBlock - 1) / (8 * kWavesPerBlock)));
-            auto kernel = bitwidth == 1 ? quantize_rows64<1, 2> : ths.splits > 0 ? quantize_rows64<2, 2, true> : quantize_rows64<2, 2>;
-            kernel<<<grid, block, 0, stream>>>(x4, ordered(ths, grid.x), q32, rows, words_per_item, div_item, zeroed, items);
-        } else {
-            const dim3 grid((unsigned)blocks);
-            auto kernel = bitwidth == 1 ? quantize_rows64<1> : ths.splits > 0 ? quantize_rows64<2, 8, true> : quantize_rows64<2>;
-            kernel<<<grid, block, kStreamLds, stream>>>(x4, ordered(ths, grid.x), q32, rows, words_per_item, div_item, zeroed, items);
-        }
+    hipError_t e = hipSuccess;
+    if (path != Path::tile) {
+        if (bitwidth == 2) e = launch_rows<2>(path, x, ths, pixels, pixels_per_item, items, C, qx, zeroed, weights, stream);
+        else e = launch_rows<1>(path, x, ths, pixels, pixels_per_item, items, C, qx, zeroed, weights, stream);
     } else if (bitwidth == 2) {
         launch_quantize_tile<2>(x, ths, pixels, pixels_per_item, items, C, qx, zeroed, nullptr, weights, stream);
     } else {
         launch_quantize_tile<1>(x, ths, pixels, pixels_per_item, items, C, qx, zeroed, nullptr, weights, stream);
     }
+    if (e != hipSuccess) return e;
     if (btn && bitwidth == 2) launch_btn_popcount(qx, btn, items, words_per_item, splits, stream);
     return hipGetLastError();
 }
@@ -1182,29 +1216,10 @@ hipError_t launch_quantize_format(const float *x, const float *ths_values, int f
     const Thresholds ths = given_thresholds(ths_values);
     const long pixels = items * pixels_per_item;
     if (format != 4 && format != 5) return hipErrorInvalidValue;
-    if ((C % kWordBits == 0) && ((uintptr_t)x % 16 == 0)) {
-        // whole 64-channel rows: the streaming kernel; a row is 16 bytes of either format
-        const long rows = pixels * (C / kWordBits);
-        const long blocks = (rows + kRowsPerWave * kWavesPerBlock - 1) / (kRowsPerWave * kWavesPerBlock);
-        const dim3 grid((unsigned)blocks), block(kThreads);
-        const floatx4 *x4 = reinterpret_cast<const floatx4 *>(x);
-        uint32_t *q32 = reinterpret_cast<uint32_t *>(qx);
-        const long rows_per_item = pixels_per_item * (C / kWordBits);
-        const Div32 div_item = rows < 0x7fffffffL ? make_div32((uint32_t)rows_per_item) : Div32{0, 0};
-        if (weights && format == 4) return launch_rows64_weights(x, ths, format, rows, rows_per_item, div_item, qx, *weights, stream);
-        if (blocks <= kSmallLaunchBlocks) {  // too small to fill the chip: 32 rows per workgroup, as in launch_quantize
-            const dim3 small((unsigned)((rows + 8 * kWavesPerBlock - 1) / (8 * kWavesPerBlock)));
-            if (format == 4)
-                quantize_rows64<4, 2><<<small, block, 0, stream>>>(x4, ths, q32, rows, rows_per_item, div_item, nullptr, 0);
-            else
-                quantize_rows64<5, 2><<<small, block, 0, stream>>>(x4, ths, q32, rows, rows_per_item, div_item, nullptr, 0);
-        } else if (format == 4) {
-            quantize_rows64<4><<<grid, block, kStreamLds, stream>>>(x4, ths, q32, rows, rows_per_item, div_item, nullptr, 0);
-        } else {
-            quantize_rows64<5><<<grid, block, kStreamLds, stream>>>(x4, ths, q32, rows, rows_per_item, div_item, nullptr, 0);
-        }
-        return hipGetLastError();
-    }
+    const Path path = quantize_path(x, C);
+    if (path != Path::tile)  // a row is 16 bytes of either format
+        return format == 4 ? launch_rows<4>(path, x, ths, pixels, pixels_per_item, items, C, qx, nullptr, weights, stream)
+                           : launch_rows<5>(path, x, ths, pixels, pixels_per_item, items, C, qx, nullptr, nullptr, stream);
     if (format == 4) launch_quantize_tile<4>(x, ths, pixels, pixels_per_item, items, C, qx, nullptr, nullptr, weights, stream);
     else launch_quantize_tile<5>(x, ths, pixels, pixels_per_item, items, C, qx, nullptr, nullptr, weights, stream);
     return hipGetLastError();
