@@ -254,8 +254,8 @@ int tab_conv2d_packed_out_const(const int64_t *dev_QX, const int64_t *dev_QW, co
  *   TAB_CONV_AUTO      (tile -1) the library's choice: matrix cores, tile picked from the shape
  *   TAB_CONV_MATRIX    bit planes expanded to FP4 operands of v_mfma_f32_32x32x64_f8f6f4;
  *                      tile 0: 128x128, 1: 128x64 (128x32 for at most 32 filters, fp32 output and an even
- *                      number of words per pixel; 8 then 64x32), 2: 64x64, 3: 32x32 with K split over the
- *                      four waves, 4: 256x64, 5: 256x128, 6: 128x256, 7: weights resident in registers
+ *                      number of words per pixel; 8 then 64x32), 2: 64x64, 3: 32x32, 64x32 or 32x64
+ *                      with K split over the waves of a workgroup, 4: 256x64, 5: 256x128, 6: 128x256, 7: weights resident in registers
  *                      (K of at most nine words; longer K takes the library's choice), 8: 64x64 and
  *                      9: 128x128 with K split over four / two groups of waves inside the workgroup (an
  *                      even number of words per pixel; otherwise tiles 2 and 0), 10: 128x128 for the

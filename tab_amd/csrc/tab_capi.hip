@@ -105,6 +105,15 @@ int tab_internal_conv_shape(int type, int M, int KN, int G, int PC, int packed, 
     return tab::conv_mfma_shape(type, a, cost_us);
 }
 
+/* Test hook, absent from include/tab_amd.h: the shape of a launch of fp32 output, the one above or one (19 .. 22) of the kernel that splits K
+ * over the waves of a workgroup. */
+int tab_internal_conv_launch_shape(int type, int M, int KN, int G, int PC)
+{
+    tab::ConvArgs a = {};
+    a.M = M; a.KN = KN; a.G = G; a.PC = PC;
+    return tab::conv_fp32_shape(type, a);
+}
+
 /* Test hook, absent from include/tab_amd.h: whether the one-launch kernel of the smallest calls can run a call, and its predicted
  * duration on the GPU in microseconds with the three numbers it comes from. */
 int tab_internal_conv_small_cost(int type, const float *dev_X, int nchw, int N, int H, int W, int C, int KN, int KH, int KW, int padding1,
@@ -126,7 +135,7 @@ void tab_internal_set_tail_round(int workgroups) { tab::set_tail_round(workgroup
 void tab_internal_set_compute_units(int units) { tab::set_compute_units(units); }
 
 /* Test hook, absent from include/tab_amd.h: convolutions from fp32 take this shape (12 .. 18) of the kernel that keeps the input
- * patch in LDS wherever its patch fits; tab_set_conv_kernel ends it. */
+ * patch in LDS wherever its patch fits, or this one (19 .. 22) of the kernel that splits K over waves; tab_set_conv_kernel ends it. */
 void tab_internal_force_patch(int shape) { tab::force_conv_tile(9, shape); }
 
 int tab_set_conv_kernel(int kernel, int tile)

@@ -208,6 +208,7 @@ struct WeightJob {
 static_assert(sizeof(WeightJob) == 32, "quantizers take it beside at most 80 bytes of arguments");
 
 constexpr int kPatchShape = 12;  // shapes (of launch_conv_mfma) from here on are that kernel's
+constexpr int kWavesShape = 19;  // and from here on those of the kernel that splits K over the waves of a workgroup
 // Whether a call of these sizes may go there at all: the launches for which the plan is worked out.
 bool conv_patch_considered(int type, long M, int KN, int KH, int KW);
 // The plan of the automatic choice (or of the test hook's); fp32 output.
@@ -228,6 +229,10 @@ int conv_mfma_shape(int type, const ConvArgs &args, float *cost_us = nullptr);
 // At most 32 filters, fp32 output, an even number of words per pixel: the shapes of 64 filters that exist in a form of 32.
 inline bool conv_mfma_narrow(const ConvArgs &a) { return a.KN <= 32 && a.PC % 2 == 0 && a.qy == nullptr; }
 hipError_t launch_conv_mfma(int type, const ConvArgs &args, int shape, hipStream_t stream);
+// Of the kernel that splits K over the waves of a workgroup (tab_conv_mfma_waves.h): the shape with the lowest predicted duration.
+int conv_waves_shape(int type, const ConvArgs &args, float *cost_us);
+// The shape of a launch of fp32 output: that kernel's, or the one that conv_mfma_shape picks.
+int conv_fp32_shape(int type, const ConvArgs &args);
 hipError_t launch_conv_mfma_tnn(const ConvArgs &args, int shape, hipStream_t stream);
 hipError_t launch_conv_mfma_tbn(const ConvArgs &args, int shape, hipStream_t stream);
 hipError_t launch_conv_mfma_btn(const ConvArgs &args, int shape, hipStream_t stream);

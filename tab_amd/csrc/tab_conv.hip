@@ -492,6 +492,76 @@ int conv_mfma_shape(int type, const ConvArgs &a, float *cost_us)
     return conv_mfma_ranked<false>(type, a, cost_us);
 }
 
+// The kernel that splits K over the waves of a workgroup (tab_conv_mfma_waves.h): its shape with the lowest predicted duration, and whether
+// that is 2 % below what the tiled kernel is predicted to take and below 12 us (tab_conv_waves_model.h: linear forms with non-negative
+// coefficients, fitted to the calls of 1900 random layers).  32x32 tiles it takes wherever conv_mfma_shape ranks them first, in 0.74 of the time of
+// the kernel that ranking was made with, in which four waves shared chunks of K in LDS.  Held out of the fit by quarters, where other tiles
+// are ranked first: quantizer and convolution 0.922 of the tiled kernels' time, the better of each 0.902; of 668 choices 30 more than 2 % slower,
+// 15 more than 5 %, the worst 13 % (up to 20 us: 0.917, the worst 36 %: long rows of the activation of all waves of a CU
+// push each other out of its cache).  Convolution behind its quantizer, tiled / this, us: N=4 7x7x512->512 BNN 4.7 / 3.1, N=16 5.8 / 4.2, N=16
+// 14x14x256->256 4.9 / 4.3, TNN 6.2 / 5.4, N=16 14x14x256->512 stride 2 4.6 / 3.4; N=32 56x56x64->64 7.3 / 9.3 stays with the tiles.
+struct WavesTile { int rows, filters, waves, held; };
+constexpr int kWavesShapes = 4, kWavesFeatures = 10;
+constexpr WavesTile kWavesTile[kWavesShapes] = {{32, 32, 8, 4}, {32, 32, 4, 8}, {64, 32, 4, 4}, {32, 64, 4, 4}};
+constexpr float kWavesLimitUs = 12.f, kWavesMargin = 0.98f;
+}  // namespace tab
+#include "tab_conv_waves_model.h"
+namespace tab {
+
+int conv_waves_shape(int type, const ConvArgs &a, float *cost_us)
+{
+    const uint32_t cus = (uint32_t)device_compute_units();
+    const float G = (float)a.G, y_mb = (float)a.M * (float)a.KN * 4e-6f;
+    const float weights_mb = (float)a.KN * G * (type == 0 || type == 2 || type == 4 ? 16e-6f : 8e-6f);
+    const int words = a.PC % 2 == 0 && type != 0 && type != 4 ? 2 : 1;  // kWavesOneWord
+    const int units = (a.G + 2 * words - 1) / (2 * words);
+    int best = 0;
+    float best_us = 0.f;
+#pragma unroll
+    for (int i = 0; i < kWavesShapes; i++) {
+        const WavesTile tile = kWavesTile[i];
+        const uint64_t tiles = (uint64_t)(((uint32_t)a.M + tile.rows - 1) / tile.rows) * (((uint32_t)a.KN + tile.filters - 1) / tile.filters);
+        const uint64_t busiest = tiles < 1u << 31 ? ((uint32_t)tiles + cus - 1) / cus : (tiles + cus - 1) / cus;
+        const float load = (float)tiles / (float)cus, n = (float)busiest, rounds = (float)((busiest + tile.held - 1) / tile.held);
+        const float f[kWavesFeatures] = {1.f, (float)((units + tile.waves - 1) / tile.waves * words), load < 1.f ? load : 1.f, n, n * G, load, load * G,
+                                         rounds, y_mb, weights_mb};
+        float us = 0.f;
+        for (int k = 0; k < kWavesFeatures; k++) us += kWavesCost[type][i][k] * f[k];
+        if (i == 0 || us < best_us) {
+            best = i;
+            best_us = us;
+        }
+    }
+    if (cost_us) *cost_us = best_us;
+    return kWavesShape + best;
+}
+
+// That kernel's shape or `tiled`, which conv_mfma_shape picked at a price of `tiled_us`.
+static int conv_waves_or(int type, const ConvArgs &a, int tiled, float tiled_us)
+{
+    if (a.qy != nullptr) return tiled;
+    if (tiled == 3) return conv_waves_shape(type, a, nullptr);
+    if ((long)((a.M + 31) / 32) * ((a.KN + 31) / 32) > 48L * device_compute_units()) return tiled;  // (far above the limit)
+    float us = 0.f;
+    const int shape = conv_waves_shape(type, a, &us);
+    const float G = 0.1f * (float)a.G, y_mb = (float)a.M * (float)a.KN * 4e-6f;
+    const float weights_mb = (float)a.KN * (float)a.G * (type == 0 || type == 2 || type == 4 ? 16e-6f : 8e-6f);
+    const bool odd = a.PC % 2 != 0, one = a.PC == 1;
+    const float f[kWavesFeatures] = {1.f, tiled_us, y_mb, odd ? tiled_us : 0.f, G, odd ? G : 0.f, weights_mb, a.KN % 32 ? y_mb : 0.f, one ? 1.f : 0.f,
+                                     one ? tiled_us : 0.f};
+    float limit = 0.f;
+    for (int k = 0; k < kWavesFeatures; k++) limit += kWavesTiledCost[type][k] * f[k];
+    limit *= kWavesMargin;
+    return us < (limit < kWavesLimitUs ? limit : kWavesLimitUs) ? shape : tiled;
+}
+
+int conv_fp32_shape(int type, const ConvArgs &a)
+{
+    float us = 0.f;
+    const int tiled = conv_mfma_shape(type, a, &us);
+    return conv_waves_or(type, a, tiled, us);
+}
+
 // The kernel that keeps the input patch in LDS, against the tiled one that conv_mfma_shape picks: the shape with the lowest predicted
 // duration, if that is 1.5 % and 0.1 us below what the call through the tiled kernel is predicted to take (tab_conv_patch_model.h; both are
 // linear forms with non-negative coefficients, fitted to the whole calls of 3970 random layers).  On 10756 further layers: 0.967 of the
@@ -503,11 +573,13 @@ int conv_mfma_shape(int type, const ConvArgs &a, float *cost_us)
 // of 2709 layers gained more than 3 %, none that a fit could tell from the others).  Measured, whole calls, tiled / patch: N=64 14x14x256
 // levels 16.2 / 14.4 us, N=256 28x28x512->512 BNN 247 / 228, N=32 56x56x256->256 TNN 59.6 / 54.1 (64x256 tiles).  Each shape is the
 // best one of some launches, from 256x128 tiles (59 of those 10756, by 2 % in the median) to 128x64 (1373, 1.5 %).
+static bool forced_patch(const Forced &forced) { return forced.tm == 9 && forced.ng >= kPatchShape && forced.ng < kWavesShape; }
+
 bool conv_patch_considered(int type, long M, int KN, int KH, int KW)
 {
     if (type > 4) return false;
     const Forced forced = forced_kernel();
-    if (forced.tm == 9 && forced.ng >= kPatchShape) return true;  // the test hook
+    if (forced_patch(forced)) return true;  // the test hook
     return (forced.tm == 0 || (forced.tm == 9 && forced.ng < 0)) && KH * KW > 1 && KN > 32 &&
            (M + 63) / 64 * (((long)KN + 63) / 64) >= device_compute_units();
 }
@@ -522,7 +594,7 @@ PatchPlan conv_patch_plan(int type, const ConvArgs &a)
         plan = PatchPlan{kPatchShape + i, fit.kc, fit.npix, fit.lds_bytes, plan.tiled, tiles * (size_t)fit.pairs * 512 * patch_weight_planes(type)};
     };
     auto fit_of = [&](int i) { return patch_fit(a, kPatchTile[i].rows, patch_most_words(kPatchTile[i].wave_tiles)); };
-    if (forced.tm == 9 && forced.ng >= kPatchShape) {  // the test hook
+    if (forced_patch(forced)) {  // the test hook
         const int i = forced.ng - kPatchShape;
         const PatchFit fit = i < kPatchShapes ? fit_of(i) : PatchFit{};
         if (fit.kc) take(i, fit);
@@ -549,6 +621,7 @@ PatchPlan conv_patch_plan(int type, const ConvArgs &a)
             best = i;
         }
     if (best >= 0) take(best, fits[best]);
+    else plan.tiled = conv_waves_or(type, a, plan.tiled, tiled_us);
     return plan;
 }
 
@@ -572,19 +645,19 @@ WeightJob patch_weight_job(int type, const ConvArgs &a, const PatchPlan &plan, u
 hipError_t launch_conv(int type, const ConvArgs &args, hipStream_t stream)
 {
     Forced forced = forced_kernel();
-    if (forced.tm == 9 && forced.ng >= kPatchShape) forced.ng = -1;  // (the weights here are in their public order)
+    if (forced_patch(forced)) forced.ng = -1;  // (the weights here are in their public order)
     const int force_tm = forced.tm, force_ng = forced.ng;
     if (args.qy != nullptr) {  // packed output exists in the matrix-core kernel's 64-wide shapes only
         if (!conv_mfma_exact(args)) return hipErrorInvalidValue;
         const int shape = (force_tm == 9 && force_ng >= 0 && force_ng != 3 && force_ng <= 11) ? force_ng : conv_mfma_shape(type, args);
         return launch_conv_mfma(type, args, shape, stream);
     }
-    if (force_tm == 9) return launch_conv_mfma(type, args, force_ng < 0 ? conv_mfma_shape(type, args) : force_ng, stream);
+    if (force_tm == 9) return launch_conv_mfma(type, args, force_ng < 0 ? conv_fp32_shape(type, args) : force_ng, stream);
     // default path: matrix cores; the popcount kernel takes over when K is too long for exact fp32
     // accumulation (and when a benchmark forces one of its tiles)
-    if (force_tm == 0 && conv_mfma_exact(args)) return launch_conv_mfma(type, args, conv_mfma_shape(type, args), stream);
+    if (force_tm == 0 && conv_mfma_exact(args)) return launch_conv_mfma(type, args, conv_fp32_shape(type, args), stream);
     // types 4 and 5 exist on the matrix cores only
-    if (type > 3) return launch_conv_mfma(type, args, conv_mfma_shape(type, args), stream);
+    if (type > 3) return launch_conv_mfma(type, args, conv_fp32_shape(type, args), stream);
     switch (type) {
     case 0: return launch_type<0>(args, stream);
     case 1: return launch_type<1>(args, stream);

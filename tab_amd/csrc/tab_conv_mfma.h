@@ -22,7 +22,7 @@
 // Tiling: 256 threads = WM x WN waves, each wave TM x TN MFMA tiles of 32x32.  In the kernel of this file
 // operands are staged in LDS through registers exactly as for the popcount kernel (tab_conv_stage.h), and
 // per 64-bit word a lane reads the 32-bit half lane/32 selects of its row (A) or column (B), lane%32; it
-// serves chunks of K that cross filter taps and the k-split shape.  Chunks inside one tap take the kernel
+// serves chunks of K that cross filter taps.  Chunks inside one tap take the kernel
 // of tab_conv_mfma_direct.h, which shares the expansions and the epilogue defined here.
 #pragma once
 #include "tab_conv_stage.h"
@@ -193,12 +193,11 @@ __device__ __forceinline__ i32x8 expand_operand(uint32_t p0, uint32_t p1, const 
 
 // Epilogue shared by the matrix-core kernels: accumulator element 4*j + i of lane (kb, r) is
 // C[8*j + 4*kb + i][r] of the wave's 32x32 tile (mt, nt).  b_nonzero: BTN, bits set in the nonzero plane of
-// the k-positions this lane multiplied, per filter tile; partial: KS * 17 * 64 floats of LDS when the KS
-// waves of the workgroup hold partial sums of one tile; padded: words of K the kernel multiplied, K rounded up to whole
+// the k-positions this lane multiplied, per filter tile; padded: words of K the kernel multiplied, K rounded up to whole
 // chunks (the words past K are zeros, which add +64 each for binary x binary: the BNN bias counts them).
-template <int TYPE, int TM, int TN, int KCH, int KS>
+template <int TYPE, int TM, int TN>
 __device__ __forceinline__ void conv_mfma_epilogue(const ConvArgs &p, f32x16 (&acc)[TM][TN], int (&b_nonzero)[TN], int wave_m0,
-                                                   int wave_n0, int lane, int ks, float *partial, int padded)
+                                                   int wave_n0, int lane, int padded)
 {
     const int r = lane & 31, kb = lane >> 5;
     // btn of this lane's filters (BTN); loaded here rather than before the loop because the registers they would hold
@@ -208,33 +207,6 @@ __device__ __forceinline__ void conv_mfma_epilogue(const ConvArgs &p, f32x16 (&a
     for (int nt = 0; nt < TN; nt++) {
         const int col = wave_n0 + nt * 32 + r;
         btn_col[nt] = (TYPE == 2 && col < p.KN) ? p.btn[col] : 0;
-    }
-    if (KS > 1) {
-        // the KS waves hold partial sums of the same tile: exchange them through LDS; wave ks
-        // finishes rows 8*ks .. 8*ks+7
-#pragma unroll
-        for (int e = 0; e < 16; e++) partial[(ks * 17 + e) * 64 + lane] = acc[0][0][e];
-        partial[(ks * 17 + 16) * 64 + lane] = (float)b_nonzero[0];
-        __syncthreads();
-        float sum[5];
-#pragma unroll
-        for (int e = 0; e < 5; e++) {
-            sum[e] = 0.f;
-            const int src = e < 4 ? 4 * ks + e : 16;
-#pragma unroll
-            for (int k = 0; k < KS; k++) sum[e] += partial[(k * 17 + src) * 64 + lane];
-        }
-        const int col = wave_n0 + r;
-        const bool col_ok = col < p.KN;
-        float bias = 0.f;
-        if (TYPE == 2) bias = (float)btn_col[0] - (sum[4] + __shfl_xor(sum[4], 32, 64));
-        if (TYPE == 3) bias = (float)(p.num - 64 * padded);
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int m = wave_m0 + 8 * ks + 4 * kb + i;
-            if (col_ok && m < p.M) __builtin_nontemporal_store(sum[i] + bias, &p.y[(size_t)m * p.KN + col]);
-        }
-        return;
     }
     // Y is written once and read by nobody here: non-temporal stores keep it from pushing the operands out of L2
     // (N=256 28x28x512->512: HBM reads 30-78 MB -> 15-31 MB, 1.1-1.3 x the operands' size, and 2-4 % less time);
@@ -441,42 +413,36 @@ constexpr int mfma_waves_per_eu(int wm, int tm, int tn, int lds_bytes)
     const int by_registers = tm * tn > 4 ? 2 : (wm * tm > 4 ? 3 : 4);
     return waves_by_lds(lds_bytes) < by_registers ? waves_by_lds(lds_bytes) : by_registers;
 }
-template <int TYPE, int WM, int WN, int TM, int TN, int KCH, bool INTAP, int KS>
+template <int TYPE, int WM, int WN, int TM, int TN, int KCH>
 constexpr int conv_mfma_lds_bytes()
 {
-    constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN;
-    using Stager = typename std::conditional<INTAP, TapStager<TYPE, BM, BN, INTAP ? KCH : 2>, TileStager<TYPE, BM, BN, KCH>>::type;
-    return 4 * (2 * (Stager::A_DWORDS + Stager::B_DWORDS) + (KS > 1 ? KS * 17 * 64 : 1));
+    using Stager = TileStager<TYPE, 32 * WM * TM, 32 * WN * TN, KCH>;
+    return 4 * 2 * (Stager::A_DWORDS + Stager::B_DWORDS);
 }
 
 // PACKED: packed output (p.qy): the weights are the first MFMA operand and the epilogue packs inside a lane.
-template <int TYPE, int WM, int WN, int TM, int TN, int KCH, bool INTAP, int KS = 1, bool PACKED = false>
+template <int TYPE, int WM, int WN, int TM, int TN, int KCH, bool PACKED = false>
 __global__ __launch_bounds__(kConvThreads)
-__attribute__((amdgpu_waves_per_eu(mfma_waves_per_eu(WM, TM, TN, conv_mfma_lds_bytes<TYPE, WM, WN, TM, TN, KCH, INTAP, KS>())))) void conv_mfma(const ConvParamsOf<PACKED> k)
+__attribute__((amdgpu_waves_per_eu(mfma_waves_per_eu(WM, TM, TN, conv_mfma_lds_bytes<TYPE, WM, WN, TM, TN, KCH>())))) void conv_mfma(const ConvParamsOf<PACKED> k)
 {
     const ConvArgs p = unpack_conv<TYPE, PACKED, 32 * WM * TM, 32 * WN * TN>(k);
-    static_assert(WM * WN * KS * 64 == kConvThreads, "four waves");
-    static_assert(!PACKED || KS == 1, "packed output: whole tiles per wave");
-    static_assert(KCH % KS == 0 && (KS == 1 || (TM == 1 && TN == 1)), "k-split waves share one 32x32 tile");
-    constexpr int WPW = KCH / KS;  // words of a chunk each wave multiplies
+    static_assert(WM * WN * 64 == kConvThreads, "four waves");
     constexpr int APL = Planes<TYPE>::A, BPL = Planes<TYPE>::B;
-    static_assert(TYPE != 5 || WPW % 2 == 0, "type 5 multiplies two words per MFMA");
-    constexpr int STEPS = TYPE == 5 ? WPW / 2 : WPW;  // MFMAs per tile pair and chunk
+    static_assert(TYPE != 5 || KCH % 2 == 0, "type 5 multiplies two words per MFMA");
+    constexpr int STEPS = TYPE == 5 ? KCH / 2 : KCH;  // MFMAs per tile pair and chunk
     constexpr int ASL = TYPE == 5 ? 2 : APL, BSL = TYPE == 5 ? 2 : BPL;
     constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN;
-    using Stager = typename std::conditional<INTAP, TapStager<TYPE, BM, BN, INTAP ? KCH : 2>, TileStager<TYPE, BM, BN, KCH>>::type;
+    using Stager = TileStager<TYPE, BM, BN, KCH>;
     constexpr int A_STRIDE = Stager::A_STRIDE, B_STRIDE = Stager::B_STRIDE;
     constexpr int Q = Stager::Q, A_DWORDS = Stager::A_DWORDS, B_DWORDS = Stager::B_DWORDS;
 
     __shared__ __attribute__((aligned(16))) uint32_t lds[2 * (A_DWORDS + B_DWORDS)];
-    __shared__ float partial[KS > 1 ? KS * 17 * 64 : 1];  // k-split: 16 accumulators + the BTN count per lane
 
     const int tid = threadIdx.x;
     const int wave = tid >> 6, lane = tid & 63;
     const int r = lane & 31;   // row of an A tile / column of a B tile
     const int kb = lane >> 5;  // which 32-bit half of the word this lane feeds
-    const int ks = wave / (WM * WN);  // which words of every chunk this wave takes
-    const int wm = (wave % (WM * WN)) % WM, wn = (wave % (WM * WN)) / WM;
+    const int wm = wave % WM, wn = wave / WM;
     int tile_m, tile_n;
     if (!tile_of_workgroup(p, tile_m, tile_n)) return;
     const int m0 = tile_m * BM, n0 = tile_n * BN;
@@ -517,13 +483,13 @@ __attribute__((amdgpu_waves_per_eu(mfma_waves_per_eu(WM, TM, TN, conv_mfma_lds_b
         auto read_step = [&](int w) {
 #pragma unroll
             for (int sl = 0; sl < ASL; sl++) {
-                const int slice = TYPE == 5 ? 2 * (ks + KS * (2 * w + kb)) + sl : sl * Q + 2 * (ks + KS * w) + kb;
+                const int slice = TYPE == 5 ? 2 * (2 * w + kb) + sl : sl * Q + 2 * w + kb;
 #pragma unroll
                 for (int mt = 0; mt < TM; mt++) a_w[w][sl][mt] = la[slice * A_STRIDE + mt * 32];
             }
 #pragma unroll
             for (int sl = 0; sl < BSL; sl++) {
-                const int slice = TYPE == 5 ? 2 * (ks + KS * (2 * w + kb)) + sl : sl * Q + 2 * (ks + KS * w) + kb;
+                const int slice = TYPE == 5 ? 2 * (2 * w + kb) + sl : sl * Q + 2 * w + kb;
 #pragma unroll
                 for (int nt = 0; nt < TN; nt++) b_w[w][sl][nt] = lb[slice * B_STRIDE + nt * 32];
             }
@@ -565,7 +531,7 @@ __attribute__((amdgpu_waves_per_eu(mfma_waves_per_eu(WM, TM, TN, conv_mfma_lds_b
     if constexpr (PACKED)  // (the chunk loop ends on a barrier: the operand buffers are free for BTN's exchange of biases)
         conv_mfma_epilogue_packed<TYPE, TM, TN, KCH>(p, acc, b_nonzero, wave_m0, wave_n0, lane, lds + wave * (32 * TN), p.nchunks * KCH);
     else
-        conv_mfma_epilogue<TYPE, TM, TN, KCH, KS>(p, acc, b_nonzero, wave_m0, wave_n0, lane, ks, partial, p.nchunks * KCH);
+        conv_mfma_epilogue<TYPE, TM, TN>(p, acc, b_nonzero, wave_m0, wave_n0, lane, p.nchunks * KCH);
 }
 
 // Chunk length for G words: 1..4, the one with the least padded work (a barrier is priced as half a
@@ -580,7 +546,7 @@ inline int mfma_chunk_words(int G)
     return best;
 }
 
-template <int TYPE, int WM, int WN, int TM, int TN, int KCH, bool INTAP, int KS = 1>
+template <int TYPE, int WM, int WN, int TM, int TN, int KCH>
 hipError_t launch_mfma_tile(ConvArgs a, hipStream_t stream)
 {
     constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN;
@@ -589,20 +555,15 @@ hipError_t launch_mfma_tile(ConvArgs a, hipStream_t stream)
     a.tiles_m = (a.M + BM - 1) / BM;
     const long blocks = order_workgroups<Planes<TYPE>::A>(a, (a.KN + BN - 1) / BN);
     if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
-    if (a.qy != nullptr) {
-        if constexpr (KS == 1)
-            conv_mfma<TYPE, WM, WN, TM, TN, KCH, INTAP, KS, true><<<dim3((unsigned)blocks), dim3(kConvThreads), 0, stream>>>(pack_conv<TYPE, true>(a));
-        else
-            return hipErrorInvalidValue;  // no packed output from the k-split 32x32 shape
-    } else {
-        conv_mfma<TYPE, WM, WN, TM, TN, KCH, INTAP, KS><<<dim3((unsigned)blocks), dim3(kConvThreads), 0, stream>>>(pack_conv<TYPE, false>(a));
-    }
+    if (a.qy != nullptr)
+        conv_mfma<TYPE, WM, WN, TM, TN, KCH, true><<<dim3((unsigned)blocks), dim3(kConvThreads), 0, stream>>>(pack_conv<TYPE, true>(a));
+    else
+        conv_mfma<TYPE, WM, WN, TM, TN, KCH><<<dim3((unsigned)blocks), dim3(kConvThreads), 0, stream>>>(pack_conv<TYPE, false>(a));
     return hipGetLastError();
 }
 
 // Chunks of whole word pairs that stay inside a filter tap (PC even) go from global memory straight into LDS
-// (tab_conv_mfma_direct.h), measured 2-14 % faster than staging them through registers; the k-split shape keeps the piece stager of the kernel
-// above (its chunks are too short to split into pairs of words per wave, and it measured no better).
+// (tab_conv_mfma_direct.h), measured 2-14 % faster than staging them through registers.
 template <int TYPE, int WM, int WN, int TM, int TN, int KCH, int KS = 1, int ARUN = 0>
 hipError_t launch_mfma_direct(ConvArgs a, hipStream_t stream);
 template <int TYPE, int WM, int WN, int TM, int TN, int KS, int WORDS>
@@ -617,15 +578,6 @@ hipError_t launch_mfma_tail_wide(ConvArgs a, hipStream_t stream);
 template <int TYPE, int WM, int WN, int TM, int TN>
 hipError_t launch_patch(const ConvArgs &a, hipStream_t stream);
 
-template <int TYPE, int WM, int WN, int TM, int TN, int KCH, int KS = 1>
-hipError_t launch_mfma_intap(const ConvArgs &a, hipStream_t stream)
-{
-    if constexpr (KS == 1)
-        return launch_mfma_direct<TYPE, WM, WN, TM, TN, KCH>(a, stream);
-    else
-        return launch_mfma_tile<TYPE, WM, WN, TM, TN, KCH, true, KS>(a, stream);
-}
-
 // LONG: the launch is small enough to be latency-bound, so prefer few long chunks (fewer serial
 // fetch round trips) over a small LDS footprint.
 template <int TYPE, int WM, int WN, int TM, int TN, bool LONG = false>
@@ -633,26 +585,26 @@ hipError_t launch_mfma_shape(const ConvArgs &a, hipStream_t stream)
 {
     // whole word pairs inside one tap (PC even) load LDS directly
     if constexpr (LONG) {
-        if (a.PC % 4 == 0 && a.G % 12 == 0) return launch_mfma_intap<TYPE, WM, WN, TM, TN, 12>(a, stream);
-        if (a.PC % 8 == 0) return launch_mfma_intap<TYPE, WM, WN, TM, TN, 8>(a, stream);
+        if (a.PC % 4 == 0 && a.G % 12 == 0) return launch_mfma_direct<TYPE, WM, WN, TM, TN, 12>(a, stream);
+        if (a.PC % 8 == 0) return launch_mfma_direct<TYPE, WM, WN, TM, TN, 8>(a, stream);
     }
-    if (a.PC % 4 == 0) return launch_mfma_intap<TYPE, WM, WN, TM, TN, 4>(a, stream);
+    if (a.PC % 4 == 0) return launch_mfma_direct<TYPE, WM, WN, TM, TN, 4>(a, stream);
     // PC = 2, 6, 10 ...: chunks of six words across taps rather than one pair of words per barrier (+5-13 %),
     // unless two two-plane operands would push the big tiles' LDS past four workgroups per CU
     if constexpr (LONG || Planes<TYPE>::A + Planes<TYPE>::B <= 3)
-        if (a.PC % 2 == 0 && a.G % 6 == 0) return launch_mfma_intap<TYPE, WM, WN, TM, TN, 6>(a, stream);
+        if (a.PC % 2 == 0 && a.G % 6 == 0) return launch_mfma_direct<TYPE, WM, WN, TM, TN, 6>(a, stream);
     if constexpr (LONG && TYPE != 5)
-        if (a.G % 9 == 0) return launch_mfma_tile<TYPE, WM, WN, TM, TN, 9, false>(a, stream);
-    if (a.PC % 2 == 0) return launch_mfma_intap<TYPE, WM, WN, TM, TN, 2>(a, stream);
+        if (a.G % 9 == 0) return launch_mfma_tile<TYPE, WM, WN, TM, TN, 9>(a, stream);
+    if (a.PC % 2 == 0) return launch_mfma_direct<TYPE, WM, WN, TM, TN, 2>(a, stream);
     if constexpr (TYPE == 5) {  // whole pairs of words per chunk
-        if ((a.G + 1) / 2 % 2 == 0) return launch_mfma_tile<TYPE, WM, WN, TM, TN, 4, false>(a, stream);
-        return launch_mfma_tile<TYPE, WM, WN, TM, TN, 2, false>(a, stream);
+        if ((a.G + 1) / 2 % 2 == 0) return launch_mfma_tile<TYPE, WM, WN, TM, TN, 4>(a, stream);
+        return launch_mfma_tile<TYPE, WM, WN, TM, TN, 2>(a, stream);
     } else {
         switch (mfma_chunk_words(a.G)) {
-        case 1: return launch_mfma_tile<TYPE, WM, WN, TM, TN, 1, false>(a, stream);
-        case 2: return launch_mfma_tile<TYPE, WM, WN, TM, TN, 2, false>(a, stream);
-        case 3: return launch_mfma_tile<TYPE, WM, WN, TM, TN, 3, false>(a, stream);
-        default: return launch_mfma_tile<TYPE, WM, WN, TM, TN, 4, false>(a, stream);
+        case 1: return launch_mfma_tile<TYPE, WM, WN, TM, TN, 1>(a, stream);
+        case 2: return launch_mfma_tile<TYPE, WM, WN, TM, TN, 2>(a, stream);
+        case 3: return launch_mfma_tile<TYPE, WM, WN, TM, TN, 3>(a, stream);
+        default: return launch_mfma_tile<TYPE, WM, WN, TM, TN, 4>(a, stream);
         }
     }
 }
@@ -660,9 +612,12 @@ hipError_t launch_mfma_shape(const ConvArgs &a, hipStream_t stream)
 // The short-K kernel with the weights resident in registers (tab_conv_mfma_regs.h), types 0..3.
 template <int TYPE>
 hipError_t launch_mfma_regs(const ConvArgs &a, hipStream_t stream);
+// K split over the waves of a workgroup, operands straight into registers (tab_conv_mfma_waves.h).
+template <int TYPE, int WAVES, int TM, int TN>
+hipError_t launch_waves(const ConvArgs &a, hipStream_t stream);
 
-// shape: 0 = 128x128, 1 = 128x64 (conv_mfma_narrow: 128x32), 2 = 64x64 (rows x filters per workgroup), 3 = 32x32 with the four
-// waves splitting every chunk of four words between them, 4 = 256x64, 5 = 256x128 and 6 = 128x256
+// shape: 0 = 128x128, 1 = 128x64 (conv_mfma_narrow: 128x32), 2 = 64x64 (rows x filters per workgroup), 3 = the best of
+// 19 .. 22, 4 = 256x64, 5 = 256x128 and 6 = 128x256
 // (eight MFMA tiles per wave: fewer operand expansions per MFMA, half the occupancy), 7 = the register-resident
 // short-K kernel (K of at most nine words; longer K falls back to the shape picked from the launch),
 // 8 = 64x64 (conv_mfma_narrow: 64x32) with K split over the four waves (each wave 2x2 MFMA tiles over a quarter of every chunk), 9 = 128x128 with K
@@ -671,7 +626,8 @@ hipError_t launch_mfma_regs(const ConvArgs &a, hipStream_t stream);
 // the rest of the last round (an even number of words per pixel; otherwise shape 0), 11 = the same with whole tiles of 128x256
 // (words per pixel in fours; otherwise shape 6); 12 .. 18 = the kernel that keeps the input patch in LDS, on weights laid out for
 // it (ConvArgs::qw then points to those): 256x128, 128x128, 128x64, 64x64, 256x64, 64x256, 64x128; refused where its patch does not
-// fit
+// fit; 19 .. 22 = K split over the waves of a workgroup, operands straight into registers (fp32 output only): 32x32 in eight waves, in four,
+// 64x32 and 32x64 in four
 template <int TYPE>
 hipError_t launch_mfma_type(const ConvArgs &a, int shape, hipStream_t stream)
 {
@@ -689,7 +645,8 @@ hipError_t launch_mfma_type(const ConvArgs &a, int shape, hipStream_t stream)
         if (a.PC % 2 == 0) return launch_mfma_tail<TYPE>(a, stream);
         shape = 0;
     }
-    if (shape >= kPatchShape) {
+    if (shape == 3) shape = conv_waves_shape(TYPE, a, nullptr);
+    if (shape >= kPatchShape && shape < kWavesShape) {
         if constexpr (TYPE <= 4) {
             switch (shape) {
             case 12: return launch_patch<TYPE, 2, 2, 4, 2>(a, stream);
@@ -721,20 +678,10 @@ hipError_t launch_mfma_type(const ConvArgs &a, int shape, hipStream_t stream)
     case 4: return launch_mfma_shape<TYPE, 4, 1, 2, 2>(a, stream);
     case 5: return launch_mfma_shape<TYPE, 2, 2, 4, 2>(a, stream);
     case 6: return launch_mfma_shape<TYPE, 2, 2, 2, 4>(a, stream);
-    case 3:
-        // these launches are latency-bound: few long chunks (three or six words per wave) beat many short ones
-        if constexpr (TYPE != 5) {
-            if (a.G % 24 == 0) return launch_mfma_tile<TYPE, 1, 1, 1, 1, 24, false, 4>(a, stream);
-            if (a.G % 12 == 0) return launch_mfma_tile<TYPE, 1, 1, 1, 1, 12, false, 4>(a, stream);
-        }
-        if (a.PC % 8 == 0) return launch_mfma_intap<TYPE, 1, 1, 1, 1, 8, 4>(a, stream);
-        if constexpr (TYPE == 5) {  // two words per wave and chunk at least
-            return launch_mfma_tile<TYPE, 1, 1, 1, 1, 8, false, 4>(a, stream);
-        } else {
-            if (a.PC % 4 == 0) return launch_mfma_intap<TYPE, 1, 1, 1, 1, 4, 4>(a, stream);
-            if (a.G > 4) return launch_mfma_tile<TYPE, 1, 1, 1, 1, 12, false, 4>(a, stream);
-            return launch_mfma_tile<TYPE, 1, 1, 1, 1, 4, false, 4>(a, stream);
-        }
+    case 19: return launch_waves<TYPE, 8, 1, 1>(a, stream);
+    case 20: return launch_waves<TYPE, 4, 1, 1>(a, stream);
+    case 21: return launch_waves<TYPE, 4, 2, 1>(a, stream);
+    case 22: return launch_waves<TYPE, 4, 1, 2>(a, stream);
     default: return hipErrorInvalidValue;
     }
 }

@@ -395,7 +395,7 @@ __device__ __forceinline__ void conv_mfma_direct_tile(const ConvArgs &p, uint32_
                 if constexpr (PACKED)
                     conv_mfma_epilogue_packed<TYPE, 1, 1, KCH>(p, sum, nonzero, wave_m0 + mt * 32, wave_n0 + nt * 32, lane, exchange, nchunks * KCH);
                 else
-                    conv_mfma_epilogue<TYPE, 1, 1, KCH, 1>(p, sum, nonzero, wave_m0 + mt * 32, wave_n0 + nt * 32, lane, 0, nullptr, nchunks * KCH);
+                    conv_mfma_epilogue<TYPE, 1, 1>(p, sum, nonzero, wave_m0 + mt * 32, wave_n0 + nt * 32, lane, nchunks * KCH);
             }
             if (round + 1 < NT / RT) __syncthreads();  // the parts are read before the next round overwrites them
         }
@@ -405,7 +405,7 @@ __device__ __forceinline__ void conv_mfma_direct_tile(const ConvArgs &p, uint32_
         if (TYPE == 2) __syncthreads();
         conv_mfma_epilogue_packed<TYPE, TM, TN, KCH>(p, acc, b_nonzero, wave_m0, wave_n0, lane, lds + wave * (32 * TN), nchunks * KCH);
     } else {
-        conv_mfma_epilogue<TYPE, TM, TN, KCH, 1>(p, acc, b_nonzero, wave_m0, wave_n0, lane, 0, nullptr, nchunks * KCH);
+        conv_mfma_epilogue<TYPE, TM, TN>(p, acc, b_nonzero, wave_m0, wave_n0, lane, nchunks * KCH);
     }
 }
 
@@ -576,4 +576,5 @@ hipError_t launch_mfma_narrow(const ConvArgs &a, hipStream_t stream)
 }  // namespace tab
 
 #include "tab_conv_mfma_patch.h"
+#include "tab_conv_mfma_waves.h"
 #include "tab_conv_mfma_regs.h"

@@ -325,7 +325,7 @@ void conv_mfma_patch(const ConvParams k)
     }
     scale_sums<TYPE>(acc);
     const int wave_m0 = m0 + wm * (32 * TM), wave_n0 = n0 + wn * (32 * TN);
-    conv_mfma_epilogue<TYPE, TM, TN, KC, 1>(p, acc, b_nonzero, wave_m0, wave_n0, lane, 0, nullptr, p.G);
+    conv_mfma_epilogue<TYPE, TM, TN>(p, acc, b_nonzero, wave_m0, wave_n0, lane, p.G);
 }
 
 template <int TYPE, int WM, int WN, int TM, int TN, int KC>

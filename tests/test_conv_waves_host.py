@@ -1,0 +1,45 @@
+"""The rule that takes a convolution to the kernel that splits K over waves, on the host: the library's choices on the measured layers are the
+fit script's, with the regret that its comment states."""
+import ctypes
+import importlib.util
+import os
+
+import numpy as np
+
+from tab_amd import _capi
+
+SCRIPT = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "tab_amd", "tuning", "fit_conv_waves_model.py")
+
+
+def test_choices_on_the_measured_layers():
+    spec = importlib.util.spec_from_file_location("fit_conv_waves_model", SCRIPT)
+    fit = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(fit)
+    rows = fit.parse()
+    assert len(rows) >= 1900
+    fit.tiled_choice(rows)
+    coefficients = fit.fit(rows)
+    f = ctypes.CDLL(_capi.LIB_PATH).tab_internal_conv_launch_shape
+    differ, taken, best, alone = 0, [], [], []
+    for r in rows:
+        shape = f(r["type"], r["M"], r["KN"], r["G"], r["PC"])
+        assert shape in fit.SHAPES or shape == r["shape"] != 3
+        differ += (shape if shape in fit.SHAPES else "tiled") != fit.choose(r, coefficients)
+        if r["tiled"] is None:
+            alone.append(r["times"][shape] / min(r["times"].values()))
+        else:
+            call = r["quantizer"] + r["tiled"]
+            taken.append((r["quantizer"] + r["times"].get(shape, r["tiled"])) / call)
+            best.append((r["quantizer"] + min(r["tiled"], *r["times"].values())) / call)
+    assert differ <= 3  # (coefficients of six digits)
+    assert np.exp(np.mean(np.log(taken))) < 0.925 and np.exp(np.mean(np.log(best))) > 0.90 and max(taken) < 1.14
+    assert np.exp(np.mean(np.log(alone))) < 1.005
+
+
+def test_packed_output_and_large_launches_stay_with_the_tiles():
+    f = ctypes.CDLL(_capi.LIB_PATH).tab_internal_conv_launch_shape
+    tiled = ctypes.CDLL(_capi.LIB_PATH).tab_internal_conv_shape
+    for type in range(6):
+        for M, KN, G, PC in ((2**31 - 600, 1, 9, 1), (2**31 - 600, 4096, 65535, 65535), (200704, 64, 9, 1), (1, 1, 1, 1), (1, 4096, 65534, 65534)):
+            shape = f(type, M, KN, G, PC)
+            assert 0 <= shape <= 22 and (M < 1000 or shape == tiled(type, M, KN, G, PC, 0, None)), (type, M, KN, G, PC, shape)
