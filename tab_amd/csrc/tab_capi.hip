@@ -617,9 +617,14 @@ static int layer_quantize(const float *dev_X, int nchw, int bitwidth, float act_
     if (need && (!workspace || workspace_bytes < need || ((uintptr_t)workspace % 4)))
         return fail(TAB_ERR_WORKSPACE, "workspace must hold %zu bytes (got %zu)", need, workspace_bytes);
     tab::Thresholds ths;
+    uint64_t *q = reinterpret_cast<uint64_t *>(dev_QX);
+    if (bitwidth == 2 && !weights && tab::quantize_items_supported(true, nchw && H * W > 1, N, (long)H * W, C)) {
+        const hipError_t e = tab::launch_quantize_own(dev_X, act_scale, nchw && H * W > 1, N, (long)H * W, C, q, static_cast<hipStream_t>(stream));
+        if (e != hipSuccess) return device_fail(e, "quantize launch");
+        return TAB_OK;
+    }
     hipError_t e = own_thresholds(dev_X, bitwidth, act_scale, N, per_item, workspace, &ths, stream);
     if (e != hipSuccess) return device_fail(e, "threshold launch");
-    uint64_t *q = reinterpret_cast<uint64_t *>(dev_QX);
     // one pixel per image: NCHW and NHWC are the same memory, and the NHWC quantizers read it along the channels
     e = nchw && H * W > 1 ? tab::launch_quantize_nchw(dev_X, ths, bitwidth, N, C, (long)H * W, q, nullptr, nullptr, static_cast<hipStream_t>(stream), weights)
                           : tab::launch_quantize(dev_X, ths, bitwidth, (long)H * W, N, C, q, nullptr, nullptr, static_cast<hipStream_t>(stream), weights);
@@ -657,6 +662,16 @@ int tab_internal_layer_conv2d(const float *dev_X, int nchw, float act_scale, con
                             need - layer_packed_bytes(s.abits, N, H, W, C), route.weights(), stream);
         if (rc != TAB_OK) return rc;
         return run_route(route, type, stream);
+    }
+    // small images of ternary activations, thresholds and quantizer in one launch; not where only the pixels at a stride are quantized
+    if (!one && s.abits == 2 && !(KH == 1 && KW == 1 && (stride1 > 1 || stride2 > 1)) && tab::quantize_items_supported(true, false, N, (long)H * W, C)) {
+        const ConvRoute route = conv_route(conv_args(s, padding1, padding2, stride1, stride2, N, H, W, C, KN, KH, KW, workspace, dev_QW, dev_btn, dev_Y),
+                                           type, plan, spare, room);
+        if (!route.weights()) {
+            rc = layer_quantize(dev_X, 0, s.abits, act_scale, N, H, W, C, static_cast<int64_t *>(workspace), sums,
+                                need - layer_packed_bytes(s.abits, N, H, W, C), nullptr, stream);
+            return rc != TAB_OK ? rc : run_route(route, type, stream);
+        }
     }
     tab::Thresholds ths;
     hipError_t e = hipSuccess;

@@ -281,6 +281,13 @@ hipError_t launch_quantize(const float *x, const Thresholds &ths, int bitwidth, 
 hipError_t launch_quantize_nchw(const float *x, const Thresholds &ths, int bitwidth, int N, int C, long HW, uint64_t *qx,
                                 int32_t *btn, int32_t *count_workspace, hipStream_t stream, const WeightJob *weights = nullptr);
 
+// Small items of two planes, a workgroup each (tab_quantize_item.hip): with given thresholds and the counts (btn), or with thresholds
+// that it finds itself, scale * mean|x|, as launch_threshold would to the last bit.  own: which of the two.
+bool quantize_items_supported(bool own, bool nchw, long items, long pixels, int C);
+hipError_t launch_quantize_items(const float *x, const Thresholds &ths, bool nchw, long items, long pixels, int C, uint64_t *qx, int32_t *btn,
+                                 hipStream_t stream);
+hipError_t launch_quantize_own(const float *x, float scale, bool nchw, long items, long pixels, int C, uint64_t *qx, hipStream_t stream);
+
 // Packers of the CPU-only conv types: format 4 = DoReFa 2-bit levels, 5 = RTN fields.
 hipError_t launch_quantize_format(const float *x, const float *ths, int format, long pixels_per_item, long items, int C,
                                   uint64_t *qx, hipStream_t stream, const WeightJob *weights = nullptr);

@@ -1071,6 +1071,9 @@ hipError_t launch_quantize(const float *x, const Thresholds &ths, int bitwidth, 
     const CountTarget target{btn, count_workspace};
     const bool counted = btn && bitwidth == 2 && items * (words_per_item / 4 + 1) < 0x7fffffffL &&
                          (count_workspace || (words_per_item <= 64 && PC <= kOneSliceUnits));
+    // an item of several slices, or whose counts would be read back (words_per_item <= 128: one slice, no second launch)
+    if (btn && bitwidth == 2 && words_per_item > (counted ? 128 : 0) && quantize_items_supported(false, false, items, pixels_per_item, C))
+        return launch_quantize_items(x, ths, false, items, pixels_per_item, C, qx, btn, stream);
     if (counted && path != Path::tile) {
         const floatx4 *x4 = reinterpret_cast<const floatx4 *>(x);
         uint32_t *q32 = reinterpret_cast<uint32_t *>(qx);
@@ -1123,6 +1126,9 @@ hipError_t launch_quantize_nchw(const float *x, const Thresholds &ths, int bitwi
     const long runs = N * ((HW + 3) / 4);
     const bool counted = btn && bitwidth == 2 && (count_workspace || (words_per_item <= 64 && PC <= kOneSliceUnits)) &&
                          N * (HW / 4 + 1) * PC < 0x7fffffffL;
+    // an item of several slices (64 pixels and a word each at least), or whose counts would be read back
+    if (btn && bitwidth == 2 && (!counted || (HW + 63) / 64 * PC > kOneSliceUnits) && quantize_items_supported(false, true, N, HW, C))
+        return launch_quantize_items(x, ths, true, N, HW, C, qx, btn, stream);
     auto by_image = [&](long per_image) { return N * per_image < 0x7fffffffL ? make_div32((uint32_t)per_image) : Div32{0, 0}; };
     auto launch = [&](auto kernel, long blocks, int threads, long per_image) {
         kernel<<<dim3((unsigned)blocks), dim3(threads), 0, stream>>>(x, ordered(ths, blocks), qx, N, C, HW, PC, by_image(per_image), zeroed);
