@@ -493,17 +493,19 @@ int conv_mfma_shape(int type, const ConvArgs &a, float *cost_us)
 }
 
 // The kernel that splits K over the waves of a workgroup (tab_conv_mfma_waves.h): its shape with the lowest predicted duration, and whether
-// that is 2 % below what the tiled kernel is predicted to take and below 12 us (tab_conv_waves_model.h: linear forms with non-negative
-// coefficients, fitted to the calls of 1900 random layers).  32x32 tiles it takes wherever conv_mfma_shape ranks them first, in 0.74 of the time of
-// the kernel that ranking was made with, in which four waves shared chunks of K in LDS.  Held out of the fit by quarters, where other tiles
-// are ranked first: quantizer and convolution 0.922 of the tiled kernels' time, the better of each 0.902; of 668 choices 30 more than 2 % slower,
-// 15 more than 5 %, the worst 13 % (up to 20 us: 0.917, the worst 36 %: long rows of the activation of all waves of a CU
-// push each other out of its cache).  Convolution behind its quantizer, tiled / this, us: N=4 7x7x512->512 BNN 4.7 / 3.1, N=16 5.8 / 4.2, N=16
-// 14x14x256->256 4.9 / 4.3, TNN 6.2 / 5.4, N=16 14x14x256->512 stride 2 4.6 / 3.4; N=32 56x56x64->64 7.3 / 9.3 stays with the tiles.
+// that is 2 % below what the tiled kernel is predicted to take, below it by a fifth of what it takes above 4 us besides, and below 12 us
+// (tab_conv_waves_model.h: linear forms with non-negative coefficients, fitted to the calls of 1900 random layers and of 800 of residual and
+// other networks' sizes).  32x32 tiles it takes wherever conv_mfma_shape ranks them first, in 0.74 of the time of the kernel that ranking
+// was made with, in which four waves shared chunks of K in LDS.  Held out of the fit by quarters, where other tiles are ranked first: quantizer
+// and convolution 0.932 of the tiled kernels' time, the better of each 0.913; of 833 choices 21 more than 2 % slower, 9 more than 5 %, the
+// worst 12 %.  (Fitted to the random layers alone, without the fifth and without a price for pixels of whole cache lines: 64 and 36, N=16
+// 14x14x512 of type 5 22 %, N=64 7x7x512->512 TNN 31 % slower.  Those pixels' loads read the same bytes of 32 lines, a half more time than others.)
+// Convolution behind its quantizer, tiled / this, us: N=4 7x7x512->512 BNN 4.7 / 3.1, N=16 5.8 / 4.2, N=16 14x14x256->256 4.9 / 4.3, TNN 6.2 / 5.4, N=16 14x14x256->512 stride 2 4.6 / 3.4; N=32 56x56x64->64 7.3 / 9.3 and N=64 7x7x512->512 TNN 11.6 / 15.2
+// stay with the tiles.
 struct WavesTile { int rows, filters, waves, held; };
-constexpr int kWavesShapes = 4, kWavesFeatures = 10;
+constexpr int kWavesShapes = 4, kWavesFeatures = 11, kWavesTiledFeatures = 10;
 constexpr WavesTile kWavesTile[kWavesShapes] = {{32, 32, 8, 4}, {32, 32, 4, 8}, {64, 32, 4, 4}, {32, 64, 4, 4}};
-constexpr float kWavesLimitUs = 12.f, kWavesMargin = 0.98f;
+constexpr float kWavesLimitUs = 12.f, kWavesMargin = 0.98f, kWavesDoubtUs = 4.f, kWavesDoubt = 0.2f;
 }  // namespace tab
 #include "tab_conv_waves_model.h"
 namespace tab {
@@ -514,6 +516,7 @@ int conv_waves_shape(int type, const ConvArgs &a, float *cost_us)
     const float G = (float)a.G, y_mb = (float)a.M * (float)a.KN * 4e-6f;
     const float weights_mb = (float)a.KN * G * (type == 0 || type == 2 || type == 4 ? 16e-6f : 8e-6f);
     const int words = a.PC % 2 == 0 && type != 0 && type != 4 ? 2 : 1;  // kWavesOneWord
+    const float lines = a.PC * (type <= 1 || type == 4 ? 16 : 8) % 128 == 0 ? G : 0.f;  // a pixel is whole cache lines
     const int units = (a.G + 2 * words - 1) / (2 * words);
     int best = 0;
     float best_us = 0.f;
@@ -524,7 +527,7 @@ int conv_waves_shape(int type, const ConvArgs &a, float *cost_us)
         const uint64_t busiest = tiles < 1u << 31 ? ((uint32_t)tiles + cus - 1) / cus : (tiles + cus - 1) / cus;
         const float load = (float)tiles / (float)cus, n = (float)busiest, rounds = (float)((busiest + tile.held - 1) / tile.held);
         const float f[kWavesFeatures] = {1.f, (float)((units + tile.waves - 1) / tile.waves * words), load < 1.f ? load : 1.f, n, n * G, load, load * G,
-                                         rounds, y_mb, weights_mb};
+                                         rounds, y_mb, weights_mb, n * lines};
         float us = 0.f;
         for (int k = 0; k < kWavesFeatures; k++) us += kWavesCost[type][i][k] * f[k];
         if (i == 0 || us < best_us) {
@@ -547,12 +550,13 @@ static int conv_waves_or(int type, const ConvArgs &a, int tiled, float tiled_us)
     const float G = 0.1f * (float)a.G, y_mb = (float)a.M * (float)a.KN * 4e-6f;
     const float weights_mb = (float)a.KN * (float)a.G * (type == 0 || type == 2 || type == 4 ? 16e-6f : 8e-6f);
     const bool odd = a.PC % 2 != 0, one = a.PC == 1;
-    const float f[kWavesFeatures] = {1.f, tiled_us, y_mb, odd ? tiled_us : 0.f, G, odd ? G : 0.f, weights_mb, a.KN % 32 ? y_mb : 0.f, one ? 1.f : 0.f,
-                                     one ? tiled_us : 0.f};
+    const float f[kWavesTiledFeatures] = {1.f, tiled_us, y_mb, odd ? tiled_us : 0.f, G, odd ? G : 0.f, weights_mb,
+                                          a.KN % 32 ? y_mb : 0.f, one ? 1.f : 0.f, one ? tiled_us : 0.f};
     float limit = 0.f;
-    for (int k = 0; k < kWavesFeatures; k++) limit += kWavesTiledCost[type][k] * f[k];
+    for (int k = 0; k < kWavesTiledFeatures; k++) limit += kWavesTiledCost[type][k] * f[k];
     limit *= kWavesMargin;
-    return us < (limit < kWavesLimitUs ? limit : kWavesLimitUs) ? shape : tiled;
+    const float doubt = us > kWavesDoubtUs ? kWavesDoubt * (us - kWavesDoubtUs) : 0.f;
+    return us < kWavesLimitUs && us + doubt < limit ? shape : tiled;
 }
 
 int conv_fp32_shape(int type, const ConvArgs &a)

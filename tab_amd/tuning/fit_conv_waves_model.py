@@ -1,5 +1,6 @@
 """Coefficients of the rule that takes a convolution with fp32 output to the kernel that splits K over the waves of a workgroup
-(tab_conv_waves_model.h), from conv_waves_timings.txt: random layers of at most 5000 tiles of 32x32 that take two launches, as the tiled kernels
+(tab_conv_waves_model.h), from conv_waves_timings.txt: 1900 random layers and 800 of residual and other networks' sizes, of at most 5000 tiles of
+32x32, that take two launches, as the tiled kernels
 run them by their own choice ("tiled"; left out where that was their 32x32 shape, whose place this kernel takes) and in this kernel's shapes
 19 .. 22.
 
@@ -7,15 +8,18 @@ A timing is that of a quantizer and the convolution behind it on three sets of i
 quantizer's alone ("quantizer").
 
 Model, per (type, shape): duration ~ c . f, non-negative least squares of the relative error, with the features
-    f = [1, steps, busy, n, n * G, load, load * G, rounds, Y, W]
+    f = [1, steps, busy, n, n * G, load, load * G, rounds, Y, W, n * G * lines]
     load   = ceil(M / BM) * ceil(KN / BN) / CUs      workgroups a CU gets
     n      = ceil(load), busy = min(1, load)         the busiest CU's; the share of the CUs that have work at all
     rounds = ceil(n / workgroups a CU holds)
     steps  = words of K of the longest wave          its chain of loads, expansions and multiplications
+    lines  = pixels of whole cache lines: a load's lanes then read the same bytes of different lines
     G      = KH*KW*PC words of K, Y = 4*M*KN bytes / 1e6, W = bytes of the weights / 1e6 (fetched from behind the L2s)
 and for the tiled kernels, with the duration `us` that conv_mfma_shape predicts (fitted to convolutions replayed on the same operands)
     f = [1, us, Y, us * odd, G / 10, G / 10 * odd, W, Y * ragged, one, us * one]
     odd, one: an odd number of words a pixel, a single one; ragged: KN is no multiple of 32
+
+What is predicted to take more than 4 us has to gain more, a fifth of what is above: the predictions that are far too low lie there.
 
     python tab_amd/tuning/fit_conv_waves_model.py            fit on everything, write the header
     python tab_amd/tuning/fit_conv_waves_model.py --check    fit on three quarters of the layers in turn, regret on the fourth
@@ -33,8 +37,7 @@ ROOT = os.path.dirname(os.path.dirname(HERE))
 DATA = os.path.join(HERE, "conv_waves_timings.txt")
 HEADER = os.path.join(ROOT, "tab_amd", "csrc", "tab_conv_waves_model.h")
 SHAPES = {19: (32, 32, 8, 4), 20: (32, 32, 4, 8), 21: (64, 32, 4, 4), 22: (32, 64, 4, 4)}  # kWavesTile
-CUS, LIMIT_US, MARGIN = 256, 12.0, 0.98
-FEATURES = 10
+CUS, LIMIT_US, MARGIN, DOUBT_US, DOUBT = 256, 12.0, 0.98, 4.0, 0.2
 
 
 def parse(path=DATA):
@@ -65,7 +68,8 @@ def features(r, shape):
     units = -(-r["G"] // (2 * words))
     tiles = -(-r["M"] // bm) * -(-r["KN"] // bn)
     load, n = tiles / CUS, -(-tiles // CUS)
-    return [1.0, -(-units // waves) * words, min(1.0, load), n, n * r["G"], load, load * r["G"], -(-n // held), y, w]
+    lines = r["PC"] * (16 if r["type"] in (0, 1, 4) else 8) % 128 == 0
+    return [1.0, -(-units // waves) * words, min(1.0, load), n, n * r["G"], load, load * r["G"], -(-n // held), y, w, n * r["G"] * lines]
 
 
 def tiled_features(r, us):
@@ -104,7 +108,7 @@ def choose(r, coefficients):
     if r["shape"] == 3:
         return best
     tiled = float(coefficients[r["type"], "tiled"] @ np.array(tiled_features(r, r["us"])))
-    return best if us[best] < LIMIT_US and us[best] < MARGIN * tiled else "tiled"
+    return best if us[best] < LIMIT_US and us[best] + DOUBT * max(0.0, us[best] - DOUBT_US) < MARGIN * tiled else "tiled"
 
 
 def report(rows, choices, what):
@@ -143,7 +147,7 @@ def main():
         f.write("constexpr float kWavesCost[6][kWavesShapes][kWavesFeatures] = {\n")
         for t in range(6):
             f.write("    {\n" + "".join("        %s,\n" % row(coefficients[t, s]) for s in SHAPES) + "    },\n")
-        f.write("};\n\nconstexpr float kWavesTiledCost[6][kWavesFeatures] = {\n" + "".join("    %s,\n" % row(coefficients[t, "tiled"]) for t in range(6)) + "};\n\n}  // namespace tab\n")
+        f.write("};\n\nconstexpr float kWavesTiledCost[6][kWavesTiledFeatures] = {\n" + "".join("    %s,\n" % row(coefficients[t, "tiled"]) for t in range(6)) + "};\n\n}  // namespace tab\n")
 
 
 if __name__ == "__main__":
