@@ -540,8 +540,10 @@ int conv_waves_shape(int type, const ConvArgs &a, float *cost_us)
 }
 
 // That kernel's shape or `tiled`, which conv_mfma_shape picked at a price of `tiled_us`.
-static int conv_waves_or(int type, const ConvArgs &a, int tiled, float tiled_us)
+// gain_us (optional): what that kernel is predicted to take less.
+static int conv_waves_or(int type, const ConvArgs &a, int tiled, float tiled_us, float *gain_us = nullptr)
 {
+    if (gain_us) *gain_us = 0.f;
     if (a.qy != nullptr) return tiled;
     if (tiled == 3) return conv_waves_shape(type, a, nullptr);
     if ((long)((a.M + 31) / 32) * ((a.KN + 31) / 32) > 48L * device_compute_units()) return tiled;  // (far above the limit)
@@ -554,6 +556,7 @@ static int conv_waves_or(int type, const ConvArgs &a, int tiled, float tiled_us)
                                           a.KN % 32 ? y_mb : 0.f, one ? 1.f : 0.f, one ? tiled_us : 0.f};
     float limit = 0.f;
     for (int k = 0; k < kWavesTiledFeatures; k++) limit += kWavesTiledCost[type][k] * f[k];
+    if (gain_us) *gain_us = limit - us;
     limit *= kWavesMargin;
     const float doubt = us > kWavesDoubtUs ? kWavesDoubt * (us - kWavesDoubtUs) : 0.f;
     return us < kWavesLimitUs && us + doubt < limit ? shape : tiled;
@@ -568,15 +571,17 @@ int conv_fp32_shape(int type, const ConvArgs &a)
 
 // The kernel that keeps the input patch in LDS, against the tiled one that conv_mfma_shape picks: the shape with the lowest predicted
 // duration, if that is 1.5 % and 0.1 us below what the call through the tiled kernel is predicted to take (tab_conv_patch_model.h; both are
-// linear forms with non-negative coefficients, fitted to the whole calls of 3970 random layers).  On 10756 further layers: 0.967 of the
-// tiled kernels' time (in total 0.952; the better one of each 0.959 and 0.945), of 3607 choices 95 more than 2 % slower, 25 more than
-// 5 %, 7 more than 8 %, the worst 15 %.  (Fitted to convolutions replayed on the same operands, weights in the L2s, 294 of those layers were more than
-// 5 % slower, the worst 1.6 times.)
+// linear forms with non-negative coefficients, fitted to the whole calls of 3970 random layers, those that choices slowed down by more than 5 %
+// counted threefold).  Those calls take 0.951 of the tiled kernels' time (in total 0.935; the better one of each 0.945 and 0.930), of 1826 choices
+// 27 are more than 2 % slower, the worst 4.8 %; on halves held out of the fit 0.952, 47, 11 more than 5 %, the worst 27 %.  (Fitted to
+// convolutions replayed on the same operands, weights in the L2s, a tenth of such layers were more than 5 % slower, the worst 1.6 times.)
+// Where the tiled kernel's place is the split-K kernel's (conv_waves_or), that one is taken if it is predicted to gain half a microsecond more
+// than the patch: of 599 of those layers 187 where the rules want both, patch 0.896 of the tiled time, split K 0.859, the choice 0.858.
 // Not for 1x1 kernels, which read every pixel for one tap only, nor for at most 32 filters, half of whose tiles would be work for nothing,
 // nor for launches of fewer 64x64 tiles than compute units, which last as long as one tile's chain of waits (from half as many on, 129
 // of 2709 layers gained more than 3 %, none that a fit could tell from the others).  Measured, whole calls, tiled / patch: N=64 14x14x256
-// levels 16.2 / 14.4 us, N=256 28x28x512->512 BNN 247 / 228, N=32 56x56x256->256 TNN 59.6 / 54.1 (64x256 tiles).  Each shape is the
-// best one of some launches, from 256x128 tiles (59 of those 10756, by 2 % in the median) to 128x64 (1373, 1.5 %).
+// levels 16.2 / 13.2 us, N=256 28x28x512->512 BNN 247 / 223, N=32 56x56x256->256 TNN 59.6 / 52.7 (64x256 tiles).  Each shape is the
+// best one of some launches.
 static bool forced_patch(const Forced &forced) { return forced.tm == 9 && forced.ng >= kPatchShape && forced.ng < kWavesShape; }
 
 bool conv_patch_considered(int type, long M, int KN, int KH, int KW)
@@ -607,10 +612,15 @@ PatchPlan conv_patch_plan(int type, const ConvArgs &a)
     if (a.qy != nullptr) return plan;
     float tiled_us = 0.f;
     plan.tiled = conv_mfma_shape(type, a, &tiled_us);
+    if (plan.tiled == 3) {  // K split over waves then: of 19 such layers the patch was faster on none
+        plan.tiled = conv_waves_shape(type, a, nullptr);
+        return plan;
+    }
     float t[kTiledFeatures];
     tiled_features(a, type, tiled_us, t);
     float limit = 0.f;
     for (int k = 0; k < kTiledFeatures; k++) limit += kTiledCost[type][k] * t[k];
+    const float tiled_call_us = limit;
     limit = 0.985f * limit - 0.1f;
     const long kn64 = ((long)a.KN + 63) / 64;
     const PatchCall call = patch_call(a, type, (uint32_t)device_compute_units());
@@ -624,8 +634,10 @@ PatchPlan conv_patch_plan(int type, const ConvArgs &a)
             limit = us[i];
             best = i;
         }
-    if (best >= 0) take(best, fits[best]);
-    else plan.tiled = conv_waves_or(type, a, plan.tiled, tiled_us);
+    float waves_gain_us = 0.f;
+    const int other = conv_waves_or(type, a, plan.tiled, tiled_us, &waves_gain_us);
+    if (best >= 0 && (other < kWavesShape || waves_gain_us <= tiled_call_us - us[best] + 0.5f)) take(best, fits[best]);
+    else plan.tiled = other;
     return plan;
 }
 

@@ -44,6 +44,9 @@ __device__ __forceinline__ Item<PL> load_item_at(__amdgpu_buffer_rsrc_t rsrc, ui
     return it;
 }
 
+// Workgroups of the first round, four a CU; those behind them find the weights in the L2.
+constexpr uint32_t kFirstWorkgroups = 1024;
+
 // ConvParams with other contents where this kernel has no use for the usual ones: G = pixels of the patch (the stride between
 // planes), nchunks = KH, the magics of PC and KW = those of PW and PH.
 template <int TYPE, int WM, int WN, int TM, int TN, int KC>
@@ -265,9 +268,17 @@ void conv_mfma_patch(const ConvParams k)
     load_patch(words, 0);
     fetch_b(cur);
     fetch_b(nxt);
+    // The weights come from behind the L2 of whichever XCD wrote them, two pairs of words ahead of the MFMAs: the first workgroups of a launch
+    // would wait for every pair.  While they wait for the patch, eight neighbours ask for a cache line of their filters each, an eighth of them.
+    // Whole calls, us: N=64 14x14x256 levels 14.8 / 14.1 (64x128 tiles 14.6 / 13.8), N=32 20x20x192 5x5 TBN in 64x128 tiles 22.5 / 18.6, N=32
+    // 14x14x512->512 20.5 / 18.0; 64 layers 3 % in 64x128 tiles, 2 in 128x64, none in 256x128.  All lines by every workgroup, or before the patch's
+    // addresses, gained half of that.
+    const uint32_t touched = __builtin_amdgcn_raw_buffer_load_b32(
+        b_rsrc, blockIdx.x < kFirstWorkgroups ? (uint32_t)(tid * 8 + (tile_m & 7)) * 128u : kNoData, 0, 0);
     if (KC == 1 && tid < 4)  // the pixel of zeros, in both planes of both buffers
         *reinterpret_cast<u32x4 *>(base + (nchunks > 1 ? (uint32_t)(tid >> 1) * buffer : 0u) + (uint32_t)(tid & 1) * plane + zero_pixel) = u32x4{0, 0, 0, 0};
     write_patch(words, 0);
+    asm volatile("" ::"v"(touched));
     __syncthreads();
     place_pair(0, 0);
     read_a(0, 0);

@@ -13,6 +13,8 @@ and every shape take beyond the best of them, over the tiled kernel's time, all 
 more.  The durations themselves, with the quantizer's as a form in bytes, join in at a tenth of the weight, which gives the predictions
 their scale; they are the convolution's up to a summand that all share.
 
+Where conv_mfma_shape ranks 32x32 tiles first, the kernel that splits K over waves ran in their place ("tiled"): the patch was never faster.
+
     python tab_amd/tuning/fit_conv_patch_model.py            fit on everything, write the header
     python tab_amd/tuning/fit_conv_patch_model.py --check    fit on one half of the geometries, regret on the other
 """
@@ -32,6 +34,7 @@ SHAPES = {12: (256, 128, 8, 2), 13: (128, 128, 4, 3), 14: (128, 64, 2, 4), 15: (
 CUS, ITEMS, LDS = 256, {1: 3, 2: 3, 4: 2}, 64 * 1024
 MARGIN, MARGIN_US = 0.985, 0.1  # what the patch kernel has to be predicted below: MARGIN of the tiled kernel's duration, less MARGIN_US
 PATCH_FEATURES, TILED_FEATURES = 18, 14  # kPatchFeatures, kTiledFeatures
+ROUNDS, SLOWER = 5, 1.05
 BORDER, SCALE = 0.1, 0.1  # a difference of the share BORDER of a call weighs 0.7 of one that is none; a duration SCALE
 
 
@@ -102,10 +105,10 @@ def tiled_prediction():
     f = lib.tab_internal_conv_shape
     f.restype, f.argtypes = ctypes.c_int, [ctypes.c_int] * 6 + [ctypes.POINTER(ctypes.c_float)]
 
-    def predict(r):
+    def predict(r, shape=False):
         cost = ctypes.c_float()
-        f(r["type"], r["M"], r["KN"], r["G"], r["PC"], 0, ctypes.byref(cost))
-        return cost.value
+        chosen = f(r["type"], r["M"], r["KN"], r["G"], r["PC"], 0, ctypes.byref(cost))
+        return chosen if shape else cost.value
 
     return predict
 
@@ -123,13 +126,13 @@ def quantizer_features(r):
     return np.array([1, x, x * ragged, ragged, r["N"] * r["H"] * r["W"] * r["PC"] * 8e-6 * (2 if r["type"] in (0, 1, 4) else 1)])
 
 
-def fit(rows, predict):
+def fit_weighted(rows, predict, emphasis):
     tiled, patch = {}, {}
     at = {s: TILED_FEATURES + k * PATCH_FEATURES for k, s in enumerate(SHAPES)}
     quantizer = TILED_FEATURES + len(SHAPES) * PATCH_FEATURES
     for t in range(5):
         A, b = [], []
-        for r in rows:
+        for r, emphasised in zip(rows, emphasis):
             if r["type"] != t:
                 continue
             kernels = []  # (duration, its form)
@@ -144,7 +147,7 @@ def fit(rows, predict):
             for i, (us, form) in enumerate(kernels):
                 if i != best:
                     difference = (us - kernels[best][0]) / r["tiled"]
-                    weight = (1 + (difference / BORDER) ** 2) ** -0.5
+                    weight = (1 + (difference / BORDER) ** 2) ** -0.5 * emphasised
                     A.append(weight * (form - kernels[best][1]) / r["tiled"])
                     b.append(weight * difference)
                 whole = form.copy()
@@ -158,7 +161,19 @@ def fit(rows, predict):
     return tiled, patch
 
 
+def fit(rows, predict):
+    """Calls that the choices slow down by more than SLOWER count threefold in the next of ROUNDS fits."""
+    emphasis = np.ones(len(rows))
+    for _ in range(ROUNDS):
+        fitted = fit_weighted(rows, predict, emphasis)
+        each = regret(rows, [choose(r, *fitted, predict) for r in rows])[4]
+        emphasis[each > SLOWER] *= 3
+    return fitted
+
+
 def choose(r, tiled, patch, predict):
+    if predict(r, True) == 3:
+        return None
     limit, best = MARGIN * float(tiled[r["type"]] @ tiled_features(r, predict(r))) - MARGIN_US, None
     for s in SHAPES:
         f = patch_features(r, s)
