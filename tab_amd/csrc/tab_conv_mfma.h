@@ -247,13 +247,44 @@ __device__ __forceinline__ void conv_mfma_epilogue(const ConvArgs &p, f32x16 (&a
     }
 }
 
+// The signs of a lane's 16 values of a tile, value 4j+i as bit 8j+i: the bits move in from the right, one instruction each.  With the
+// difference to the threshold that makes two a value, where comparing, selecting the bit and adding it (and BNN's bias) made four; packed
+// layers of short K are bound by such instructions: us, N=64 56x56x64->64 BNN 9.55 / 8.89, N=31 97x82x64->128 TBN 19.7 / 17.2, N=1 512->1024
+// 15x15 6.82 / 6.65; of 60 layers none slower.
+template <class F>
+__device__ __forceinline__ uint32_t sign_bits(F value)
+{
+    uint32_t bits = 0;
+#pragma unroll
+    for (int j = 3; j >= 0; j--) {
+        if (j < 3) bits <<= 4;
+#pragma unroll
+        for (int i = 3; i >= 0; i--) bits = __builtin_amdgcn_alignbit(bits, __float_as_uint(value(4 * j + i)), 31);
+    }
+    return bits;
+}
+
+// v + this is negative where v < th: a sum that is not zero has the sign of the exact one, one that is zero is +0 (never -0, whatever
+// the zeros' signs), and a th that is no number is above nothing.
+__device__ __forceinline__ float below_threshold(float th) { return th == th ? 0.f - th : __builtin_inff(); }
+
+// v > th, or not and v < -th.
+template <class F>
+__device__ __forceinline__ void ternary_bits(F value, float th, uint32_t &sign, uint32_t &nonzero)
+{
+    const float t = th == th ? 0.f + th : __builtin_inff();
+    const uint32_t pos = sign_bits([&](int e) { return t - value(e); }), neg = sign_bits([&](int e) { return value(e) + t; });
+    sign = neg & ~pos;
+    nonzero = pos | neg;
+}
+
 // Packed output for a kernel that multiplied with the weights as the FIRST MFMA operand: accumulator element 4j+i of
 // lane (kb, r) is then filter 8j+4kb+i of filter tile nt and pixel r of row tile mt, i.e. a lane holds 16 filters of ONE
 // pixel.  It thresholds them against that pixel's threshold (a per-lane constant) exactly as the quantizer would
 // threshold them as the next layer's NHWC activation (item = image, channel = filter; TAB_GEMM.cu:184-192, 231) into 16
 // bits, and the other half-wave's lane of the same pixel supplies the other 16 of the 32-bit half word: no ballot and
 // no cross-lane deposit per value (packing by wave ballot, with the activation as the first operand, costs about 13 vector
-// instructions per pair of rows, this 2-3 per value).  The per-filter bias of BTN (btn - nonzero weights, known per lane = filter after the loop) is
+// instructions per pair of rows, this two per value).  The per-filter bias of BTN (btn - nonzero weights, known per lane = filter after the loop) is
 // handed to the lanes that need it through `exchange`, 32*TN dwords of LDS private to the wave.
 template <int TYPE, int TM, int TN, int KCH>
 __device__ __forceinline__ void conv_mfma_epilogue_packed(const ConvArgs &p, f32x16 (&acc)[TM][TN], int (&b_nonzero)[TN], int wave_m0,
@@ -298,30 +329,21 @@ __device__ __forceinline__ void conv_mfma_epilogue_packed(const ConvArgs &p, f32
             int n = (int)div32((uint32_t)(wave_m0 + mt * 32 + r), p.div_pixels);
             n = n < p.N ? n : p.N - 1;  // rows past M are computed but not stored
             const float th = p.out_ths ? p.out_ths[n] : p.out_th;
+            // BNN: whole numbers of less than 2^23, which are below th where they are below the whole number above it, and with one bias
+            const float below = OUT_BITS == 1 ? (TYPE == 3 ? bias[0][0] - __builtin_fminf(__builtin_fmaxf(__builtin_ceilf(th), -0x1p23f), 0x1p23f) : below_threshold(th)) : 0.f;
             uint32_t sign_half[TN], nz_half[TN];
 #pragma unroll
             for (int nt = 0; nt < TN; nt++) {
-                uint32_t sg = 0, nz = 0;
-#pragma unroll
-                for (int j = 0; j < 4; j++)
-#pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        const float v = (TYPE == 2 || TYPE == 3) ? acc[mt][nt][4 * j + i] + bias[nt][4 * j + i] : acc[mt][nt][4 * j + i];
-                        const uint32_t bit = 1u << (8 * j + i);  // shifted by 4*kb below
-                        if (OUT_BITS == 1) {
-                            sg |= v < th ? bit : 0u;
-                        } else {
-                            const bool pos = v > th, neg = !pos && v < -th;
-                            sg |= neg ? bit : 0u;
-                            nz |= (pos || neg) ? bit : 0u;
-                        }
-                    }
+                auto value = [&](int e) { return (TYPE == 2 || TYPE == 3) ? acc[mt][nt][e] + bias[nt][e] : acc[mt][nt][e]; };
+                uint32_t sg, nz = 0;
+                if (OUT_BITS == 1) sg = sign_bits([&](int e) { return (TYPE == 3 ? acc[mt][nt][e] : value(e)) + below; });
+                else ternary_bits(value, th, sg, nz);
                 const int cols_left = p.KN - (wave_n0 + nt * 32);  // filters of this tile that exist: tail bits stay zero
                 const uint32_t live = cols_left >= 32 ? 0xffffffffu : (cols_left <= 0 ? 0u : (1u << cols_left) - 1u);
                 sg <<= 4 * kb;
                 nz <<= 4 * kb;
                 sign_half[nt] = (sg | (uint32_t)__shfl_xor((int)sg, 32, 64)) & live;
-                nz_half[nt] = (nz | (uint32_t)__shfl_xor((int)nz, 32, 64)) & live;
+                if (OUT_BITS == 2) nz_half[nt] = (nz | (uint32_t)__shfl_xor((int)nz, 32, 64)) & live;
             }
             // the lower half-wave stores; a word past the last one and the upper half-wave get an offset out of range
             const uint32_t row_off = (uint32_t)(mt * 32 + r) * row_bytes;

@@ -244,25 +244,14 @@ __global__ __launch_bounds__(kConvThreads) __attribute__((amdgpu_waves_per_eu(2,
             // The values of pixel m are thresholded exactly as the quantizer would threshold them as the next
             // layer's NHWC activation (TAB_GEMM.cu:184-192, 231); this lane holds filters 8j+4kb+i of every tile,
             // the other half-wave's lane of the same pixel the rest of each 32-bit half.
-            const float th = th_cur;
+            const float th = th_cur, below = below_threshold(th);
             uint32_t sign_half[TN], nz_half[TN];
 #pragma unroll
             for (int nt = 0; nt < TN; nt++) {
-                uint32_t sg = 0, nz = 0;
-#pragma unroll
-                for (int j = 0; j < 4; j++)
-#pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        const float v = acc[nt][4 * j + i];
-                        const uint32_t bit = 1u << (8 * j + i);  // shifted by 4*kb below
-                        if (OUT == kOutBits1) {
-                            sg |= v < th ? bit : 0u;
-                        } else {
-                            const bool pos = v > th, neg = !pos && v < -th;
-                            sg |= neg ? bit : 0u;
-                            nz |= (pos || neg) ? bit : 0u;
-                        }
-                    }
+                uint32_t sg, nz = 0;
+                auto value = [&](int e) { return acc[nt][e]; };
+                if (OUT == kOutBits1) sg = sign_bits([&](int e) { return acc[nt][e] + below; });
+                else ternary_bits(value, th, sg, nz);
                 sg <<= 4 * kb;
                 nz <<= 4 * kb;
                 sign_half[nt] = (sg | (uint32_t)__shfl_xor((int)sg, 32, 64)) & live_cols[nt];
