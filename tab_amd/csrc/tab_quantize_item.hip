@@ -4,7 +4,7 @@
 // With slices of an item in workgroups of their own, the sums of |x| or the counts take a launch before or behind the quantizer: 2.4 us on
 // the GPU and 2.8 of the host, more than a small item's reading.  Here a workgroup reads its item once for the sum, all loads requested at
 // once, and a second time, out of the L2, to pack it.  Bound by what one CU reads, some 40 GB/s of latency and 64 bytes a cycle, hence the
-// limits: items of 26 K values with their counts, of 12 K with their thresholds.  Quantizer and counts in two launches / here, graph replays,
+// limits: items of 24 K values with their counts, of 12 K with their thresholds.  Quantizer and counts in two launches / here, graph replays,
 // us: 136 14x14x64 5.3 / 4.2 (NCHW 6.1 / 4.0), 256 7x7x512 9.1 / 7.6, 79 25x15x64 5.5 / 4.7, but 16 14x14x256 (49 K) 4.8 / 6.5; sums and quantizer:
 // 91 rows of 576 4.6 / 3.7, 153 of 5376 5.4 / 4.3, 2000 of 700 12.3 / 7.2, but 79 25x15x64 (23 K) 6.1 / 6.9.  Called one after the other such
 // quantizers take 7.6 us in two launches, which is the host's time, and 5.0 in one; a ternary linear layer of 2048 inputs 11.4 in three, 8.5 in two.
@@ -16,6 +16,9 @@ namespace tab {
 namespace {
 
 constexpr int kSumThreads = 256;  // of a slice of |x|, as in abs_sum_partial
+
+// Waves that share 64 pixels of an item's channels (NCHW), sixteen channels each.
+__host__ __device__ __forceinline__ int plane_parts_log(int C) { return C > 32 ? 2 : (C > 16 ? 1 : 0); }
 
 // scale * the sum of |x|: slices and their sums as abs_sum_partial makes them, to the last bit the same, a slice to four waves.
 template <int WAVES>
@@ -74,7 +77,11 @@ __device__ __forceinline__ float item_threshold(const float *__restrict__ src, l
     return __uint_as_float((uint32_t)__builtin_amdgcn_readfirstlane((int)__float_as_uint(t)));
 }
 
-struct PlaneRows {};  // x as [C][pixels]
+// x as [C][pixels]; 1 << PARTS_LOG waves share 64 pixels of a word
+template <int PARTS_LOG> struct PlaneRows { static constexpr int kPartsLog = PARTS_LOG; };
+
+template <class Rows> constexpr bool is_planes = false;
+template <int PARTS_LOG> constexpr bool is_planes<PlaneRows<PARTS_LOG>> = true;
 
 // OWN: ths has the number of slices and the scale of the thresholds to be found, else the thresholds.  btn: the counts, or null.
 template <int WAVES, class Rows, bool OWN>
@@ -89,10 +96,9 @@ __device__ __forceinline__ void quantize_one_item(const Rows kind, const float *
     if (OWN) __syncthreads();
     const int PC = (C + kWordBits - 1) / kWordBits;
     int count = 0;
-    if constexpr (std::is_same<Rows, PlaneRows>::value) {
-        // four waves share 64 pixels of a word, a lane sixteen channels of its pixel
-        uint16_t(*const parts)[4][2][64] = reinterpret_cast<uint16_t(*)[4][2][64]>(scratch);
-        constexpr int PARTS = 4, GROUPS = WAVES / PARTS;
+    if constexpr (is_planes<Rows>) {  // a lane takes sixteen channels of its pixel
+        constexpr int PARTS = 1 << Rows::kPartsLog, GROUPS = WAVES / PARTS;
+        uint16_t(*const halves)[2][64] = reinterpret_cast<uint16_t(*)[2][64]>(scratch);  // of a wave
         const int part = wave % PARTS, group = wave / PARTS;
         const int pixel_groups = (pixels + 63) / 64, tasks = pixel_groups * PC;
         uint64_t *const dst = q + (long)item * pixels * PC * 2;
@@ -115,14 +121,18 @@ __device__ __forceinline__ void quantize_one_item(const Rows kind, const float *
             const uint32_t exist = channels <= 0 ? 0u : 0xffffu >> (16 - channels);
             less &= exist;
             more &= exist;
-            parts[group][part][0][lane] = (uint16_t)(less & ~more);
-            parts[group][part][1][lane] = (uint16_t)(less | more);
             count += pixel < pixels ? __builtin_popcount(less | more) : 0;
+            if (PARTS == 1) {
+                if (task < tasks && pixel < pixels) *reinterpret_cast<uintx4 *>(dst + (long)pixel * 2) = uintx4{less & ~more, 0u, less | more, 0u};
+                continue;
+            }
+            halves[wave][0][lane] = (uint16_t)(less & ~more);
+            halves[wave][1][lane] = (uint16_t)(less | more);
             __syncthreads();
             if (part < 2 && task < tasks && pixel < pixels) {  // a wave a plane
                 uint64_t word = 0;
 #pragma unroll
-                for (int p = 0; p < PARTS; p++) word |= (uint64_t)parts[group][p][part][lane] << (16 * p);
+                for (int p = 0; p < PARTS; p++) word |= (uint64_t)halves[wave - part + p][part][lane] << (16 * p);
                 dst[((long)pixel * PC + pc) * 2 + part] = word;
             }
             if (task0 + GROUPS < tasks) __syncthreads();
@@ -172,16 +182,29 @@ __global__ __launch_bounds__(64 * WAVES) void quantize_items(const float *__rest
     quantize_one_item<WAVES, Rows, OWN>(kind, x, ths, q, btn, pixels, C, (int)blockIdx.x);
 }
 
-constexpr long kCountedItem = 26 * 1024, kOwnItem = 12 * 1024;  // values at most
-constexpr long kFewWaves = 4096;                                // values from which an item takes sixteen waves
+// An item's values at most, words NHWC as 64 of them; NCHW pieces of 64 pixels and 16 channels, of which sixteen waves take a round.
+constexpr long kCountedItem = 24 * 1024, kOwnItem = 12 * 1024, kCountedPieces = 32, kOwnPieces = 16;
+constexpr long kFewWaves = 4096;  // values up to which an item takes four waves
+constexpr long kManyItems = 256;  // items from which two of sixteen waves share a CU (300 10x10x96 NCHW with thresholds: 8.0 in two launches, 9.6)
+
+inline long item_pieces(long pixels, int C) { return (pixels + 63) / 64 * ((C + kWordBits - 1) / kWordBits) << plane_parts_log(C); }
+inline bool four_waves(bool nchw, long items, long pixels, int C)
+{
+    return pixels * C <= kFewWaves && (!nchw || item_pieces(pixels, C) <= (items > kManyItems ? 16 : 4));
+}
 
 }  // namespace
 
 bool quantize_items_supported(bool own, bool nchw, long items, long pixels, int C)
 {
-    // Up to 32 channels NHWC goes by tiles (a row of 16 lanes a pixel would be mostly empty); NCHW leaves two of four waves without
-    // channels, which the sums do not make up for (46 21x21x27: 6.2 us in two launches, 7.1 in one).
-    return (C > 32 || (nchw && !own)) && pixels <= kCountedItem / C && pixels * C <= (own ? kOwnItem : kCountedItem) && items < 0x7fffffffL;
+    if (pixels > kCountedItem / C || items >= 0x7fffffffL) return false;
+    if (nchw) {
+        // (few channels leave the sums nothing to make up for: 46 21x21x27, thresholds and quantizer, 6.2 us in two launches, 7.1 in one)
+        return own ? C > 32 && pixels * C <= kOwnItem && item_pieces(pixels, C) <= kOwnPieces && (items <= kManyItems || four_waves(true, items, pixels, C))
+                   : item_pieces(pixels, C) <= kCountedPieces;
+    }
+    // (up to 32 channels go by tiles: a row of 16 lanes a pixel would be mostly empty)
+    return C > 32 && pixels * ((C + kWordBits - 1) / kWordBits) * kWordBits <= (own ? kOwnItem : kCountedItem);
 }
 
 hipError_t launch_quantize_items(const float *x, const Thresholds &ths, bool nchw, long items, long pixels, int C, uint64_t *qx, int32_t *btn, hipStream_t stream)
@@ -194,10 +217,12 @@ hipError_t launch_quantize_items(const float *x, const Thresholds &ths, bool nch
             auto kernel = ths.splits > 0 ? quantize_items<WAVES, Rows, true> : quantize_items<WAVES, Rows, false>;
             kernel<<<dim3((unsigned)items), dim3(64 * WAVES), 0, stream>>>(x, ths, qx, btn, (int)pixels, C, kind);
         };
-        if (pixels * C <= kFewWaves) of(std::integral_constant<int, 4>());
+        if (four_waves(nchw, items, pixels, C)) of(std::integral_constant<int, 4>());
         else of(std::integral_constant<int, 16>());
     };
-    if (nchw) launch(PlaneRows{});
+    if (nchw && plane_parts_log(C) == 0) launch(PlaneRows<0>{});
+    else if (nchw && plane_parts_log(C) == 1) launch(PlaneRows<1>{});
+    else if (nchw) launch(PlaneRows<2>{});
     else if (C % kWordBits == 0 && (uintptr_t)x % 16 == 0) launch(WholeRows{});
     else launch(RaggedRows{C, make_div32((uint32_t)((C + kWordBits - 1) / kWordBits))});
     return hipGetLastError();
