@@ -461,7 +461,8 @@ __attribute__((amdgpu_waves_per_eu(mfma_waves_per_eu(WM, TM, TN, conv_mfma_lds_b
     __shared__ __attribute__((aligned(16))) uint32_t lds[2 * (A_DWORDS + B_DWORDS)];
 
     const int tid = threadIdx.x;
-    const int wave = tid >> 6, lane = tid & 63;
+    // (scalar: the epilogue's descriptors of the wave's rows take a loop over the lanes otherwise; N=158 46x46x64->27 BNN call 34.5 -> 29.0 us)
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int r = lane & 31;   // row of an A tile / column of a B tile
     const int kb = lane >> 5;  // which 32-bit half of the word this lane feeds
     const int wm = wave % WM, wn = wave / WM;
