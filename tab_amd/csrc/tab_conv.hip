@@ -496,10 +496,10 @@ int conv_mfma_shape(int type, const ConvArgs &a, float *cost_us)
 // that is 2 % below what the tiled kernel is predicted to take, below it by a fifth of what it takes above 4 us besides, and below 12 us
 // (tab_conv_waves_model.h: linear forms with non-negative coefficients, fitted to the calls of 1900 random layers and of 800 of residual and
 // other networks' sizes).  32x32 tiles it takes wherever conv_mfma_shape ranks them first, in 0.74 of the time of the kernel that ranking
-// was made with, in which four waves shared chunks of K in LDS.  Held out of the fit by quarters, where other tiles are ranked first: quantizer
-// and convolution 0.932 of the tiled kernels' time, the better of each 0.913; of 833 choices 21 more than 2 % slower, 9 more than 5 %, the
-// worst 12 %.  (Fitted to the random layers alone, without the fifth and without a price for pixels of whole cache lines: 64 and 36, N=16
-// 14x14x512 of type 5 22 %, N=64 7x7x512->512 TNN 31 % slower.  Those pixels' loads read the same bytes of 32 lines, a half more time than others.)
+// was made with, in which four waves shared chunks of K in LDS.  Of the other layers, quantizer and convolution take 0.944 of the tiled kernels'
+// time, the better of each 0.925; of 669 choices 13 are more than 2 % slower, the worst 4.8 % (held out of the fit by quarters 0.945, 25, 9.3 %).
+// (Fitted to the random layers alone, without the fifth and without a price for pixels of whole cache lines, N=16 14x14x512 of type 5 came out
+// 22 %, N=64 7x7x512->512 TNN 31 % slower.  Those pixels' loads read the same bytes of 32 lines, a half more time than others.)
 // Convolution behind its quantizer, tiled / this, us: N=4 7x7x512->512 BNN 4.7 / 3.1, N=16 5.8 / 4.2, N=16 14x14x256->256 4.9 / 4.3, TNN 6.2 / 5.4, N=16 14x14x256->512 stride 2 4.6 / 3.4; N=32 56x56x64->64 7.3 / 9.3 and N=64 7x7x512->512 TNN 11.6 / 15.2
 // stay with the tiles.
 struct WavesTile { int rows, filters, waves, held; };
@@ -572,11 +572,11 @@ int conv_fp32_shape(int type, const ConvArgs &a)
 // The kernel that keeps the input patch in LDS, against the tiled one that conv_mfma_shape picks: the shape with the lowest predicted
 // duration, if that is 1.5 % and 0.1 us below what the call through the tiled kernel is predicted to take (tab_conv_patch_model.h; both are
 // linear forms with non-negative coefficients, fitted to the whole calls of 3970 random layers, those that choices slowed down by more than 5 %
-// counted threefold).  Those calls take 0.951 of the tiled kernels' time (in total 0.935; the better one of each 0.945 and 0.930), of 1826 choices
-// 27 are more than 2 % slower, the worst 4.8 %; on halves held out of the fit 0.952, 47, 11 more than 5 %, the worst 27 %.  (Fitted to
+// counted threefold).  Those calls take 0.965 of the tiled kernels' time (in total 0.955; the better one of each 0.957 and 0.945), of 1313 choices
+// 30 are more than 2 % slower, the worst 4.6 %; on halves held out of the fit 0.966, 61, 21 more than 5 %, the worst 32 %.  (Fitted to
 // convolutions replayed on the same operands, weights in the L2s, a tenth of such layers were more than 5 % slower, the worst 1.6 times.)
 // Where the tiled kernel's place is the split-K kernel's (conv_waves_or), that one is taken if it is predicted to gain half a microsecond more
-// than the patch: of 599 of those layers 187 where the rules want both, patch 0.896 of the tiled time, split K 0.859, the choice 0.858.
+// than the patch: of 599 of those layers 187 where the rules want both, patch 0.896 of the tiled time, split K 0.859, the choice 0.858 (an odd number of words' tiles since faster).
 // Not for 1x1 kernels, which read every pixel for one tap only, nor for at most 32 filters, half of whose tiles would be work for nothing,
 // nor for launches of fewer 64x64 tiles than compute units, which last as long as one tile's chain of waits (from half as many on, 129
 // of 2709 layers gained more than 3 %, none that a fit could tell from the others).  Measured, whole calls, tiled / patch: N=64 14x14x256

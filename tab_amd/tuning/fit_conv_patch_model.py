@@ -13,6 +13,8 @@ and every shape take beyond the best of them, over the tiled kernel's time, all 
 more.  The durations themselves, with the quantizer's as a form in bytes, join in at a tenth of the weight, which gives the predictions
 their scale; they are the convolution's up to a summand that all share.
 
+The tiled kernel has become faster since for odd numbers of words a pixel; the fit takes its later times (conv_patch_tiled_timings.txt).
+
 Where conv_mfma_shape ranks 32x32 tiles first, the kernel that splits K over waves ran in their place ("tiled"): the patch was never faster.
 
     python tab_amd/tuning/fit_conv_patch_model.py            fit on everything, write the header
@@ -29,6 +31,7 @@ from scipy.optimize import nnls
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(os.path.dirname(HERE), "csrc")
 DATA = os.path.join(HERE, "conv_patch_timings.txt")
+TILED = os.path.join(HERE, "conv_patch_tiled_timings.txt")  # later times of the tiled kernel, where it has become faster
 SHAPES = {12: (256, 128, 8, 2), 13: (128, 128, 4, 3), 14: (128, 64, 2, 4), 15: (64, 64, 1, 4), 16: (256, 64, 4, 3),
           17: (64, 256, 4, 3), 18: (64, 128, 2, 4)}  # kPatchTile
 CUS, ITEMS, LDS = 256, {1: 3, 2: 3, 4: 2}, 64 * 1024
@@ -38,8 +41,12 @@ ROUNDS, SLOWER = 5, 1.05
 BORDER, SCALE = 0.1, 0.1  # a difference of the share BORDER of a call weighs 0.7 of one that is none; a duration SCALE
 
 
+def key(r):
+    return tuple(r[k] for k in ("type", "N", "H", "W", "C", "KN", "KH", "KW", "p1", "p2", "s"))
+
+
 def parse(path):
-    rows = []
+    rows, later = [], {} if path == TILED else {key(r): r["tiled"] for r in parse(TILED)}
     pattern = re.compile(r"type (\d) N(\d+)_(\d+)x(\d+)x(\d+)->(\d+)_k(\d+)x(\d+)_p(\d+)\.(\d+)_s(\d+) \| (.*)")
     for line in open(path):
         m = pattern.match(line)
@@ -50,6 +57,7 @@ def parse(path):
             r["G"], r["planes"] = r["KH"] * r["KW"] * r["PC"], 2 if r["type"] in (0, 2, 4) else 1
             times = dict(t.split(":") for t in m.group(12).split())
             r["tiled"] = float(times.pop("tiled"))
+            r["now"] = min(r["tiled"], later.get(key(r), r["tiled"]))
             r["times"] = {int(k): float(v) for k, v in times.items()}  # (those above 1.5 times the tiled kernel's were left out)
             rows.append(r)
     return rows
@@ -142,13 +150,13 @@ def fit_weighted(rows, predict, emphasis):
                     form[:TILED_FEATURES] = tiled_features(r, predict(r))
                 else:
                     form[at[s]:at[s] + PATCH_FEATURES] = patch_features(r, s)
-                kernels.append((r["tiled"] if s is None else r["times"][s], form))
+                kernels.append((r["now"] if s is None else r["times"][s], form))
             best = min(range(len(kernels)), key=lambda i: kernels[i][0])
             for i, (us, form) in enumerate(kernels):
                 if i != best:
-                    difference = (us - kernels[best][0]) / r["tiled"]
+                    difference = (us - kernels[best][0]) / r["now"]
                     weight = (1 + (difference / BORDER) ** 2) ** -0.5 * emphasised
-                    A.append(weight * (form - kernels[best][1]) / r["tiled"])
+                    A.append(weight * (form - kernels[best][1]) / r["now"])
                     b.append(weight * difference)
                 whole = form.copy()
                 whole[quantizer:] = quantizer_features(r)
@@ -166,7 +174,7 @@ def fit(rows, predict):
     emphasis = np.ones(len(rows))
     for _ in range(ROUNDS):
         fitted = fit_weighted(rows, predict, emphasis)
-        each = regret(rows, [choose(r, *fitted, predict) for r in rows])[4]
+        each = regret(rows, [choose(r, *fitted, predict) for r in rows], "now")[4]
         emphasis[each > SLOWER] *= 3
     return fitted
 
@@ -182,16 +190,17 @@ def choose(r, tiled, patch, predict):
     return best
 
 
-def regret(rows, chosen):
-    """(geometric mean, total) of the chosen and of the best times over the tiled ones, and every choice's over the tiled one."""
-    tiled = np.array([r["tiled"] for r in rows])
-    got = np.array([r["tiled"] if c is None else r["times"].get(c, 1.5 * r["tiled"]) for r, c in zip(rows, chosen)])
-    best = np.array([min([r["tiled"]] + list(r["times"].values())) for r in rows])
+def regret(rows, chosen, base="tiled"):
+    """(geometric mean, total) of the chosen and of the best times over the tiled ones, and every choice's over the tiled one.
+    base: the tiled kernel's times with the patch's ("tiled") or its later ones ("now")."""
+    tiled = np.array([r[base] for r in rows])
+    got = np.array([r["now"] if c is None else r["times"].get(c, 1.5 * r["now"]) for r, c in zip(rows, chosen)])
+    best = np.array([min([r["now"]] + list(r["times"].values())) for r in rows])
     return np.exp(np.log(got / tiled).mean()), got.sum() / tiled.sum(), np.exp(np.log(best / tiled).mean()), best.sum() / tiled.sum(), got / tiled
 
 
-def stated(rows, chosen):
-    geometric, total, best_geometric, best_total, each = regret(rows, chosen)
+def stated(rows, chosen, base="tiled"):
+    geometric, total, best_geometric, best_total, each = regret(rows, chosen, base)
     return ("chosen / tiled %.3f (geometric) %.3f (total), best %.3f %.3f; %d of %d in the patch kernel, more than 2 / 5 / 8 %% slower there "
             "%d / %d / %d, worst %.3f" % (geometric, total, best_geometric, best_total, sum(c is not None for c in chosen), len(rows),
                                          (each > 1.02).sum(), (each > 1.05).sum(), (each > 1.08).sum(), each.max()))
@@ -221,8 +230,9 @@ if __name__ == "__main__":
         for h in (0, 1):
             fitted = fit([r for r, x in zip(data, half) if x != h], predicted)
             held_out = [r for r, x in zip(data, half) if x == h]
-            print("held out:", stated(held_out, [choose(r, *fitted, predicted) for r in held_out]))
+            print("held out:", stated(held_out, [choose(r, *fitted, predicted) for r in held_out], "now"))
     else:
         fitted = fit(data, predicted)
         write_header(*fitted)
-        print(stated(data, [choose(r, *fitted, predicted) for r in data]))
+        for base in ("tiled", "now"):
+            print(base + ":", stated(data, [choose(r, *fitted, predicted) for r in data], base))

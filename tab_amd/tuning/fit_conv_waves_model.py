@@ -38,6 +38,7 @@ DATA = os.path.join(HERE, "conv_waves_timings.txt")
 HEADER = os.path.join(ROOT, "tab_amd", "csrc", "tab_conv_waves_model.h")
 SHAPES = {19: (32, 32, 8, 4), 20: (32, 32, 4, 8), 21: (64, 32, 4, 4), 22: (32, 64, 4, 4)}  # kWavesTile
 CUS, LIMIT_US, MARGIN, DOUBT_US, DOUBT = 256, 12.0, 0.98, 4.0, 0.2
+ROUNDS, SLOWER = 4, 1.05
 
 
 def parse(path=DATA):
@@ -87,17 +88,29 @@ def tiled_choice(rows):
         r["us"] = us.value
 
 
-def fit(rows):
-    def solve(x, y):
-        return nnls(np.array(x) / np.array(y)[:, None], np.ones(len(y)))[0]
+def fit_weighted(rows, emphasis):
+    def solve(x, y, w):
+        return nnls(np.array(x) / np.array(y)[:, None] * np.array(w)[:, None], np.array(w))[0]
 
     coefficients = {}
     for t in range(6):
-        some = [r for r in rows if r["type"] == t]
+        some = [(r, w) for r, w in zip(rows, emphasis) if r["type"] == t]
         for s in SHAPES:
-            coefficients[t, s] = solve([features(r, s) for r in some], [r["times"][s] for r in some])
-        some = [r for r in some if r["tiled"] is not None]
-        coefficients[t, "tiled"] = solve([tiled_features(r, r["us"]) for r in some], [r["tiled"] for r in some])
+            coefficients[t, s] = solve([features(r, s) for r, _ in some], [r["times"][s] for r, _ in some], [w for _, w in some])
+        some = [(r, w) for r, w in some if r["tiled"] is not None]
+        coefficients[t, "tiled"] = solve([tiled_features(r, r["us"]) for r, _ in some], [r["tiled"] for r, _ in some], [w for _, w in some])
+    return coefficients
+
+
+def fit(rows):
+    """Calls that the choices slow down by more than SLOWER count threefold in the next of ROUNDS fits."""
+    emphasis = np.ones(len(rows))
+    for _ in range(ROUNDS):
+        coefficients = fit_weighted(rows, emphasis)
+        for i, r in enumerate(rows):
+            c = choose(r, coefficients)
+            if c != "tiled" and r["tiled"] is not None and r["quantizer"] + r["times"][c] > SLOWER * (r["quantizer"] + r["tiled"]):
+                emphasis[i] *= 3
     return coefficients
 
 
