@@ -566,32 +566,83 @@ __device__ __forceinline__ int quantize_nchw_unit(const float *__restrict__ x, c
     return count;
 }
 
-template <int BITS, int VEC, int SPLIT, bool NT = false>
-__global__ __launch_bounds__(kThreads) void quantize_nchw(const float *__restrict__ x, const Thresholds ths,
-                                                          uint64_t *__restrict__ q, int N, int C, long HW, int PC, Div32 by_image, int32_t *btn)
+// Waves that a last word of few channels takes in place of four; 0: as many as the others.
+__host__ __device__ __forceinline__ int last_word_waves(int C, int PC)
+{
+    const int channels = C - (PC - 1) * kWordBits;
+    return PC == 1 || channels > 32 ? 0 : (channels <= 16 ? 1 : 2);
+}
+
+// Which word of which run the wave of a workgroup's unit `block` packs, and how many waves share it.  With four waves on a last word of up to 32
+// channels two or three of them would have none and hold a place on the CU for as long as the others' loads take; and with PC even every
+// second CU would get such words only.  So a workgroup takes the last words of four (or two) groups of runs, behind the other words of those
+// (LAST).  us, one plane: 24 61x47 of 75 channels 7.4 -> 6.4, 128 28x28 of 75 8.9 -> 7.5, 64 56x56 of 200 34.0 -> 32.6.
+struct PlaneUnit {
+    long run;  // of the wave's first lane
+    int pc, split;
+};
+template <int SPLIT, bool LAST>
+__device__ __forceinline__ PlaneUnit plane_unit(uint32_t block, int C, int PC, int wave)
+{
+    if (LAST) {
+        const int last = last_word_waves(C, PC);
+        const uint32_t groups = 4 / last, others = PC - 1, units = groups * others + 1, first = block / units * groups, in = block % units;
+        if (in == units - 1) return {(long)(first + wave / last) * 64, PC - 1, last};
+        return {(long)(first + in / others) * 64, (int)(in % others), SPLIT};
+    }
+    return {((long)(block / (uint32_t)PC) * (kWavesPerBlock / SPLIT) + wave / SPLIT) * 64, (int)(block % (uint32_t)PC), SPLIT};
+}
+// Units of `groups` groups of 64 runs with the last words apart (last: their waves), if those are no more than without, groups * PC: few groups
+// fill a unit of four groups' last words badly, and the workspace of counts has room for that many.
+inline long plane_units(long groups, int PC, int &last)
+{
+    if (last) {
+        const long of_last = 4 / last, units = (groups + of_last - 1) / of_last * (of_last * (PC - 1) + 1);
+        if (units <= groups * PC) return units;
+        last = 0;
+    }
+    return groups * PC;
+}
+
+template <int BITS, int VEC, int SPLIT, bool NT, bool LAST, bool COUNT = false>
+__device__ __forceinline__ int quantize_nchw_unit_of(const float *__restrict__ x, const Thresholds &ths, uint64_t *__restrict__ q, const PixelRun<VEC> &run,
+                                                     const PlaneUnit unit, int C, long HW, int PC)
+{
+    if (LAST && unit.split == 1) return quantize_nchw_unit<BITS, VEC, 1, NT, COUNT>(x, ths, q, run, C, HW, PC, unit.pc);
+    if (LAST && unit.split == 2) return quantize_nchw_unit<BITS, VEC, 2, NT, COUNT>(x, ths, q, run, C, HW, PC, unit.pc);
+    return quantize_nchw_unit<BITS, VEC, SPLIT, NT, COUNT>(x, ths, q, run, C, HW, PC, unit.pc);
+}
+
+template <int BITS, int VEC, int SPLIT, bool NT, bool LAST>
+__device__ __forceinline__ void quantize_nchw_block(const float *__restrict__ x, const Thresholds &ths, uint64_t *__restrict__ q, int N, int C, long HW, int PC,
+                                                    Div32 by_image, uint32_t block, int32_t *btn)
 {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t block = in_eighths(blockIdx.x, ths.eighth);
-    const PixelRun<VEC> run((block / PC * (kWavesPerBlock / SPLIT) + wave / SPLIT) * 64L + (threadIdx.x & 63), N, HW, by_image);
-    quantize_nchw_unit<BITS, VEC, SPLIT, NT>(x, ths, q, run, C, HW, PC, block % PC);
+    const PlaneUnit unit = plane_unit<SPLIT, LAST>(block, C, PC, wave);
+    const PixelRun<VEC> run(unit.run + (threadIdx.x & 63), N, HW, by_image);
+    quantize_nchw_unit_of<BITS, VEC, SPLIT, NT, LAST>(x, ths, q, run, unit, C, HW, PC);
     if (wave % SPLIT == 0) zero_counts(btn, N, run.pixel, VEC);
 }
 
+template <int BITS, int VEC, int SPLIT, bool NT = false, bool LAST = false>
+__global__ __launch_bounds__(kThreads) void quantize_nchw(const float *__restrict__ x, const Thresholds ths,
+                                                          uint64_t *__restrict__ q, int N, int C, long HW, int PC, Div32 by_image, int32_t *btn)
+{
+    quantize_nchw_block<BITS, VEC, SPLIT, NT, LAST>(x, ths, q, N, C, HW, PC, by_image, in_eighths(blockIdx.x, ths.eighth), btn);
+}
+
 // Beside a convolution's weights.
-template <int BITS, int VEC, int SPLIT, bool NT = false>
+template <int BITS, int VEC, int SPLIT, bool NT = false, bool LAST = false>
 __global__ __launch_bounds__(kThreads) void quantize_nchw_weights(const float *__restrict__ x, const Thresholds ths, uint64_t *__restrict__ q, int N,
                                                                   int C, long HW, int PC, Div32 by_image, const WeightJob job)
 {
     uint32_t block = blockIdx.x;
     if (pack_weights<kThreads>(job, block)) return;
-    block = in_eighths(block, ths.eighth);
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const PixelRun<VEC> run((block / PC * (kWavesPerBlock / SPLIT) + wave / SPLIT) * 64L + (threadIdx.x & 63), N, HW, by_image);
-    quantize_nchw_unit<BITS, VEC, SPLIT, NT>(x, ths, q, run, C, HW, PC, block % PC);
+    quantize_nchw_block<BITS, VEC, SPLIT, NT, LAST>(x, ths, q, N, C, HW, PC, by_image, in_eighths(block, ths.eighth), nullptr);
 }
 
 // The same with counts: a unit is 64 * 4 / SPLIT runs and one word.
-template <int VEC, int SPLIT, bool NT = false>
+template <int VEC, int SPLIT, bool NT = false, bool LAST = false>
 __global__ __launch_bounds__(kThreads) void quantize_nchw_count(const float *__restrict__ x, const Thresholds ths, uint64_t *__restrict__ q, int C,
                                                                 long HW, int PC, int units, const Counts counts)
 {
@@ -601,8 +652,9 @@ __global__ __launch_bounds__(kThreads) void quantize_nchw_count(const float *__r
     int count = 0;
     for (int unit = slice; unit < units; unit += counts.slices) {
         if (unit >= counts.slices) __syncthreads();  // the waves have read the words before
-        const PixelRun<VEC> run((unit / PC * (kWavesPerBlock / SPLIT) + wave / SPLIT) * 64L + (threadIdx.x & 63), item, HW, std::true_type());
-        count += quantize_nchw_unit<2, VEC, SPLIT, NT, true>(x, ths, q, run, C, HW, PC, unit % PC);
+        const PlaneUnit of = plane_unit<SPLIT, LAST>((uint32_t)unit, C, PC, wave);
+        const PixelRun<VEC> run(of.run + (threadIdx.x & 63), item, HW, std::true_type());
+        count += quantize_nchw_unit_of<2, VEC, SPLIT, NT, LAST, true>(x, ths, q, run, of, C, HW, PC);
     }
     store_count<kWavesPerBlock>(count, counts.out + blockIdx.x, scratch);
 }
@@ -1138,12 +1190,16 @@ hipError_t launch_quantize_nchw(const float *x, const Thresholds &ths, int bitwi
         job.blocks *= kThreads / threads;
         kernel<<<dim3((unsigned)blocks + job.blocks), dim3(threads), 0, stream>>>(x, ordered(ths, blocks), qx, N, C, HW, PC, by_image(per_image), job);
     };
-    // PC even, enough pixels for a wave on every SIMD: the form that gathers each wave's output into whole runs
+    // PC even, enough pixels for a wave on every SIMD: the form that gathers each wave's output into whole runs, unless its last word is mostly
+    // empty: a thread would go through that one as long as through the others (us, one plane, gathered / by units: 96 61x47 of 75 channels 24.5 /
+    // 18.5, 256 57x57 of 80 68.6 / 53, 200 60x60 of 72 47.1 / 42.1, 128 56x56 of 90 29.4 / 28.3)
     const int unit = PC % 4 == 0 ? 4 : PC % 2 == 0 ? 2 : 1;
+    // (four words of two planes are half a cache line a pixel, which the last word then reaches later: 100 40x40 of 210 31.4 us, 32.5 with it apart)
+    int last = bitwidth == 2 && PC >= 4 ? 0 : last_word_waves(C, PC);
     const long gather_waves = (runs + 63) / 64 * (PC / unit);
     if (gather_waves > 0x7fffffffL) return hipErrorInvalidValue;
     const long gather_slices = (runs / N + 63) / 64 * (PC / unit);
-    if (HW >= 4 && (uintptr_t)qx % 16 == 0 && unit > 1 && gather_waves >= 1024 && !(counted && gather_slices > 1 && !count_workspace)) {
+    if (HW >= 4 && (uintptr_t)qx % 16 == 0 && unit > 1 && gather_waves >= 1024 && !last && !(counted && gather_slices > 1 && !count_workspace)) {
         if (counted) {
             const long slices = gather_slices;
             auto launch_counted = [&](auto kernel) {
@@ -1182,25 +1238,32 @@ hipError_t launch_quantize_nchw(const float *x, const Thresholds &ths, int bitwi
         const long padded1 = (HW + 64 * groups - 1) / (64 * groups), padded4 = (HW + 256 * groups - 1) / (256 * groups) * 4;
         if (counted && HW % 4 == 0 && padded1 * 8 < padded4 * 7) four = false;
         if (counted) {
-            const long units = ((four ? runs / N : HW) + 64 * groups - 1) / (64 * groups) * PC;
+            const long units = plane_units(((four ? runs / N : HW) + 64 * groups - 1) / (64 * groups), PC, last);
             const int slices = units <= kOneSliceUnits ? 1 : (int)units;
             auto launch_counted = [&](auto kernel) {
                 kernel<<<dim3((unsigned)(N * slices)), dim3(kThreads), 0, stream>>>(x, ths, qx, C, HW, PC, (int)units,
                                                                                    Counts{slices == 1 ? btn : count_workspace, slices});
             };
-            if (stream_past) launch_counted(quantize_nchw_count<4, 4, true>);
+            if (stream_past) launch_counted(last ? quantize_nchw_count<4, 4, true, true> : quantize_nchw_count<4, 4, true>);
+            else if (last) launch_counted(four ? quantize_nchw_count<4, 4, false, true> : quantize_nchw_count<1, 4, false, true>);
             else if (four) launch_counted(split == 4 ? quantize_nchw_count<4, 4> : split == 2 ? quantize_nchw_count<4, 2> : quantize_nchw_count<4, 1>);
             else launch_counted(split == 4 ? quantize_nchw_count<1, 4> : split == 2 ? quantize_nchw_count<1, 2> : quantize_nchw_count<1, 1>);
             finish_counts(CountTarget{btn, count_workspace}, N, slices, stream);
             return hipGetLastError();
         }
-        const long blocks = ((four ? runs : pixels) + 64 * groups - 1) / (64 * groups) * PC;
+        const long blocks = plane_units(((four ? runs : pixels) + 64 * groups - 1) / (64 * groups), PC, last);
         if (blocks > 0x7fffffffL) return hipErrorInvalidValue;
-        auto form = [&](auto vec, auto parts, auto past) {
+        auto form_of = [&](auto vec, auto parts, auto past, auto with_last) {
             constexpr int VEC = decltype(vec)::value, PARTS = decltype(parts)::value;
-            constexpr bool PAST = decltype(past)::value;
-            if (weights) launch_weights(bitwidth == 2 ? quantize_nchw_weights<2, VEC, PARTS, PAST> : quantize_nchw_weights<1, VEC, PARTS, PAST>, blocks, kThreads, (HW + VEC - 1) / VEC);
-            else launch(bitwidth == 2 ? quantize_nchw<2, VEC, PARTS, PAST> : quantize_nchw<1, VEC, PARTS, PAST>, blocks, kThreads, (HW + VEC - 1) / VEC);
+            constexpr bool PAST = decltype(past)::value, LAST = decltype(with_last)::value;
+            if (weights) launch_weights(bitwidth == 2 ? quantize_nchw_weights<2, VEC, PARTS, PAST, LAST> : quantize_nchw_weights<1, VEC, PARTS, PAST, LAST>, blocks, kThreads, (HW + VEC - 1) / VEC);
+            else launch(bitwidth == 2 ? quantize_nchw<2, VEC, PARTS, PAST, LAST> : quantize_nchw<1, VEC, PARTS, PAST, LAST>, blocks, kThreads, (HW + VEC - 1) / VEC);
+        };
+        auto form = [&](auto vec, auto parts, auto past) {
+            if constexpr (decltype(parts)::value == 4) {
+                if (last) return form_of(vec, parts, past, std::true_type());
+            }
+            form_of(vec, parts, past, std::false_type());
         };
         using std::integral_constant;
         auto parts = [&](auto vec) {
