@@ -493,19 +493,19 @@ int conv_mfma_shape(int type, const ConvArgs &a, float *cost_us)
 }
 
 // The kernel that splits K over the waves of a workgroup (tab_conv_mfma_waves.h): its shape with the lowest predicted duration, and whether
-// that is 2 % below what the tiled kernel is predicted to take, below it by a fifth of what it takes above 4 us besides, and below 12 us
-// (tab_conv_waves_model.h: linear forms with non-negative coefficients, fitted to the calls of 1900 random layers and of 800 of residual and
-// other networks' sizes).  32x32 tiles it takes wherever conv_mfma_shape ranks them first, in 0.74 of the time of the kernel that ranking
-// was made with, in which four waves shared chunks of K in LDS.  Of the other layers, quantizer and convolution take 0.944 of the tiled kernels'
-// time, the better of each 0.925; of 669 choices 13 are more than 2 % slower, the worst 4.8 % (held out of the fit by quarters 0.945, 25, 9.3 %).
-// (Fitted to the random layers alone, without the fifth and without a price for pixels of whole cache lines, N=16 14x14x512 of type 5 came out
-// 22 %, N=64 7x7x512->512 TNN 31 % slower.  Those pixels' loads read the same bytes of 32 lines, a half more time than others.)
-// Convolution behind its quantizer, tiled / this, us: N=4 7x7x512->512 BNN 4.7 / 3.1, N=16 5.8 / 4.2, N=16 14x14x256->256 4.9 / 4.3, TNN 6.2 / 5.4, N=16 14x14x256->512 stride 2 4.6 / 3.4; N=32 56x56x64->64 7.3 / 9.3 and N=64 7x7x512->512 TNN 11.6 / 15.2
-// stay with the tiles.
+// that is 2 % below what the tiled kernel is predicted to take and below 12 us (tab_conv_waves_model.h: linear forms with non-negative
+// coefficients, fitted to the calls of 1900 random layers and of 800 of residual and other networks' sizes, those that choices slowed down by
+// more than 5 % counted threefold).  32x32 tiles it takes wherever conv_mfma_shape ranks them first, in 0.74 of the time of the kernel that ranking
+// was made with, in which four waves shared chunks of K in LDS.  Of the other layers, quantizer and convolution take 0.943 of the tiled kernels'
+// time, the better of each 0.925; of 715 choices 11 are more than 2 % slower, the worst 4.5 % (held out of the fit by quarters 0.943, 30, 8.7 %).
+// (Fitted to the random layers alone and without a price for pixels of whole cache lines, N=16 14x14x512 of type 5 came out 22 %, N=64
+// 7x7x512->512 TNN 31 % slower.  Those pixels' loads read the same bytes of 32 lines, a half more time than others.)  Convolution behind its
+// quantizer, tiled / this, us: N=4 7x7x512->512 BNN 4.7 / 3.1, N=16 5.8 / 4.2, N=16 14x14x256->256 TNN 6.2 / 5.4, 14x14x256->512 stride 2 BNN 4.6 / 3.4;
+// N=32 56x56x64->64 7.3 / 9.3 and N=64 7x7x512->512 TNN 11.6 / 15.2 stay with the tiles.
 struct WavesTile { int rows, filters, waves, held; };
 constexpr int kWavesShapes = 4, kWavesFeatures = 11, kWavesTiledFeatures = 10;
 constexpr WavesTile kWavesTile[kWavesShapes] = {{32, 32, 8, 4}, {32, 32, 4, 8}, {64, 32, 4, 4}, {32, 64, 4, 4}};
-constexpr float kWavesLimitUs = 12.f, kWavesMargin = 0.98f, kWavesDoubtUs = 4.f, kWavesDoubt = 0.2f;
+constexpr float kWavesLimitUs = 12.f, kWavesMargin = 0.98f;
 }  // namespace tab
 #include "tab_conv_waves_model.h"
 namespace tab {
@@ -558,8 +558,7 @@ static int conv_waves_or(int type, const ConvArgs &a, int tiled, float tiled_us,
     for (int k = 0; k < kWavesTiledFeatures; k++) limit += kWavesTiledCost[type][k] * f[k];
     if (gain_us) *gain_us = limit - us;
     limit *= kWavesMargin;
-    const float doubt = us > kWavesDoubtUs ? kWavesDoubt * (us - kWavesDoubtUs) : 0.f;
-    return us < kWavesLimitUs && us + doubt < limit ? shape : tiled;
+    return us < (limit < kWavesLimitUs ? limit : kWavesLimitUs) ? shape : tiled;
 }
 
 int conv_fp32_shape(int type, const ConvArgs &a)

@@ -273,7 +273,8 @@ void conv_mfma_patch(const ConvParams k)
     // Whole calls, us: N=64 14x14x256 levels 14.8 / 14.1 (64x128 tiles 14.6 / 13.8), N=32 20x20x192 5x5 TBN in 64x128 tiles 22.5 / 18.6, N=32
     // 14x14x512->512 20.5 / 18.0; 64 layers 3 % in 64x128 tiles, 2 in 128x64, none in 256x128.  All lines by every workgroup, or before the patch's
     // addresses, gained half of that.
-    const uint32_t touched = __builtin_amdgcn_raw_buffer_load_b32(
+    // (Waves of eight tiles have the time: N=256 28x28x512->512 BNN 225.0 without, 226.3 with.)
+    const uint32_t touched = TM * TN >= 8 ? 0u : __builtin_amdgcn_raw_buffer_load_b32(
         b_rsrc, blockIdx.x < kFirstWorkgroups ? (uint32_t)(tid * 8 + (tile_m & 7)) * 128u : kNoData, 0, 0);
     if (KC == 1 && tid < 4)  // the pixel of zeros, in both planes of both buffers
         *reinterpret_cast<u32x4 *>(base + (nchunks > 1 ? (uint32_t)(tid >> 1) * buffer : 0u) + (uint32_t)(tid & 1) * plane + zero_pixel) = u32x4{0, 0, 0, 0};

@@ -19,8 +19,6 @@ and for the tiled kernels, with the duration `us` that conv_mfma_shape predicts 
     f = [1, us, Y, us * odd, G / 10, G / 10 * odd, W, Y * ragged, one, us * one]
     odd, one: an odd number of words a pixel, a single one; ragged: KN is no multiple of 32
 
-What is predicted to take more than 4 us has to gain more, a fifth of what is above: the predictions that are far too low lie there.
-
     python tab_amd/tuning/fit_conv_waves_model.py            fit on everything, write the header
     python tab_amd/tuning/fit_conv_waves_model.py --check    fit on three quarters of the layers in turn, regret on the fourth
 """
@@ -37,7 +35,7 @@ ROOT = os.path.dirname(os.path.dirname(HERE))
 DATA = os.path.join(HERE, "conv_waves_timings.txt")
 HEADER = os.path.join(ROOT, "tab_amd", "csrc", "tab_conv_waves_model.h")
 SHAPES = {19: (32, 32, 8, 4), 20: (32, 32, 4, 8), 21: (64, 32, 4, 4), 22: (32, 64, 4, 4)}  # kWavesTile
-CUS, LIMIT_US, MARGIN, DOUBT_US, DOUBT = 256, 12.0, 0.98, 4.0, 0.2
+CUS, LIMIT_US, MARGIN = 256, 12.0, 0.98
 ROUNDS, SLOWER = 4, 1.05
 
 
@@ -121,7 +119,7 @@ def choose(r, coefficients):
     if r["shape"] == 3:
         return best
     tiled = float(coefficients[r["type"], "tiled"] @ np.array(tiled_features(r, r["us"])))
-    return best if us[best] < LIMIT_US and us[best] + DOUBT * max(0.0, us[best] - DOUBT_US) < MARGIN * tiled else "tiled"
+    return best if us[best] < LIMIT_US and us[best] < MARGIN * tiled else "tiled"
 
 
 def report(rows, choices, what):

@@ -32,7 +32,7 @@ def test_choices_on_the_measured_layers():
             taken.append((r["quantizer"] + r["times"].get(shape, r["tiled"])) / call)
             best.append((r["quantizer"] + min(r["tiled"], *r["times"].values())) / call)
     assert differ <= 3  # (coefficients of six digits)
-    assert np.exp(np.mean(np.log(taken))) < 0.945 and np.exp(np.mean(np.log(best))) > 0.92 and max(taken) < 1.05  # fitted: 0.9437, 0.9249, 1.048
+    assert np.exp(np.mean(np.log(taken))) < 0.945 and np.exp(np.mean(np.log(best))) > 0.92 and max(taken) < 1.05  # fitted: 0.9427, 0.9249, 1.045
     assert np.exp(np.mean(np.log(alone))) < 1.005
 
 
