@@ -593,7 +593,7 @@ def main():
     record_gbs = conv_bytes / record_ms / 1e6
     step_bytes = sum(layer_bytes(N, l.layer) for l in layers)
     fused_layers = sum(1 for l in layers if l.launches() == 1)
-    roofline = {"kernel": f"the {len(layers)} conv-side launches of one step: {len(layers) - fused_layers}x conv_mfma_direct<BNN> / conv_mfma<BNN> "
+    roofline = {"kernel": f"the {len(layers)} conv-side launches of one step: {len(layers) - fused_layers}x conv_mfma_direct<BNN> / conv_mfma<BNN> / conv_mfma_waves<BNN> "
                           f"and {fused_layers}x conv1x1_fused<BNN> (v_mfma_f32_32x32x64_f8f6f4, FP4 operands)",
                 "bound": "hbm" if hbm_bound else "mfma",
                 "achieved": round(record_gbs if hbm_bound else record_tops, 2),
