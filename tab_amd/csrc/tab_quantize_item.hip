@@ -4,7 +4,7 @@
 // With slices of an item in workgroups of their own, the sums of |x| or the counts take a launch before or behind the quantizer: 2.4 us on
 // the GPU and 2.8 of the host, more than a small item's reading.  Here a workgroup reads its item once for the sum, all loads requested at
 // once, and a second time, out of the L2, to pack it.  Bound by what one CU reads, some 40 GB/s of latency and 64 bytes a cycle, hence the
-// limits: items of 24 K values with their counts, of 12 K with their thresholds.  Quantizer and counts in two launches / here, graph replays,
+// limits: items of 26 K values with their counts (24 K of ragged rows: 300 14x14x96 10.9 / 11.5), of 12 K with their thresholds.  Quantizer and counts in two launches / here, graph replays,
 // us: 136 14x14x64 5.3 / 4.2 (NCHW 6.1 / 4.0), 256 7x7x512 9.1 / 7.6, 79 25x15x64 5.5 / 4.7, but 16 14x14x256 (49 K) 4.8 / 6.5; sums and quantizer:
 // 91 rows of 576 4.6 / 3.7, 153 of 5376 5.4 / 4.3, 2000 of 700 12.3 / 7.2, but 79 25x15x64 (23 K) 6.1 / 6.9.  Called one after the other such
 // quantizers take 7.6 us in two launches, which is the host's time, and 5.0 in one; a ternary linear layer of 2048 inputs 11.4 in three, 8.5 in two.
@@ -183,7 +183,7 @@ __global__ __launch_bounds__(64 * WAVES) void quantize_items(const float *__rest
 }
 
 // An item's values at most, words NHWC as 64 of them; NCHW pieces of 64 pixels and 16 channels, of which sixteen waves take a round.
-constexpr long kCountedItem = 24 * 1024, kOwnItem = 12 * 1024, kCountedPieces = 32, kOwnPieces = 16;
+constexpr long kCountedItem = 26 * 1024, kCountedRagged = 24 * 1024, kOwnItem = 12 * 1024, kCountedPieces = 32, kOwnPieces = 16;
 constexpr long kFewWaves = 4096;  // values up to which an item takes four waves
 constexpr long kManyItems = 256;  // items from which two of sixteen waves share a CU (300 10x10x96 NCHW with thresholds: 8.0 in two launches, 9.6)
 
@@ -204,7 +204,8 @@ bool quantize_items_supported(bool own, bool nchw, long items, long pixels, int 
                    : item_pieces(pixels, C) <= kCountedPieces;
     }
     // (up to 32 channels go by tiles: a row of 16 lanes a pixel would be mostly empty)
-    return C > 32 && pixels * ((C + kWordBits - 1) / kWordBits) * kWordBits <= (own ? kOwnItem : kCountedItem);
+    return C > 32 && pixels * ((C + kWordBits - 1) / kWordBits) * kWordBits <=
+                         (own ? kOwnItem : C % kWordBits ? kCountedRagged : kCountedItem);
 }
 
 hipError_t launch_quantize_items(const float *x, const Thresholds &ths, bool nchw, long items, long pixels, int C, uint64_t *qx, int32_t *btn, hipStream_t stream)

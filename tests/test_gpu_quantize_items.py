@@ -11,8 +11,8 @@ from tab_amd import _capi
 
 pytestmark = pytest.mark.gpu
 
-# N, H, W, C: one pixel; 4096 values (four waves) and past; 12288 (the most with thresholds) and past; 24576
-# (the most with counts) and past, channels filled up to whole words; NCHW 32 pieces of 64 pixels and 16 channels (counts), 16 (thresholds), more than 256 items
+# N, H, W, C: one pixel; 4096 values (four waves) and past; 12288 (the most with thresholds) and past; 26624
+# (the most with counts; 24576 in ragged rows) and past, channels filled up to whole words; NCHW 32 pieces of 64 pixels and 16 channels (counts), 16 (thresholds), more than 256 items
 CASES = [(5, 1, 1, 33), (3, 1, 1, 4096), (2, 1, 1, 4100), (7, 8, 8, 64), (3, 5, 13, 63), (2, 12, 16, 64), (2, 3, 43, 95), (3, 64, 3, 64), (4, 11, 17, 65),
          (300, 3, 3, 70), (2, 13, 32, 64), (3, 26, 16, 64), (2, 417, 1, 64), (2, 384, 1, 64), (2, 385, 1, 64), (2, 16, 12, 65), (2, 193, 1, 65), (2, 32, 64, 10), (2, 2049, 1, 10), (3, 32, 32, 20),
          (2, 1025, 1, 20), (2, 8, 64, 48), (2, 3, 171, 48), (300, 4, 4, 96), (257, 5, 13, 33), (2, 6, 13, 321), (1, 2, 3, 4099), (2, 1, 5, 2100)]
