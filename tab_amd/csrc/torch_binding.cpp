@@ -596,8 +596,9 @@ torch::Tensor chain_forward(const py::list &modules, const py::dict &ternary_thr
 namespace {
 
 // The operators that a program calls in its inner loop, taken as arrays of arguments: pybind11's dispatch of sixteen arguments costs 0.42 us,
-// this 0.09, of the 4.7 us a call of one launch takes the host.  Anything but tensors and plain ints in their places, and any call that
-// fails, goes through the pybind11 function of the same name, so that conversions and errors are its own.
+// this 0.09, of the 4.7 us a call of one launch takes the host.  Anything but tensors and plain ints in their places goes through the pybind11
+// function of the same name, so that conversions and their errors are its own.  An operator is entered once: what it throws after it may have
+// launched or allocated reaches the caller, translated as pybind11 would.
 template <size_t TENSORS, size_t INTS>
 bool plain_arguments(PyObject *const *args, Py_ssize_t count, const torch::Tensor *(&tensors)[TENSORS], int (&ints)[INTS])
 {
@@ -646,14 +647,16 @@ PyObject *fast_call(PyObject *, PyObject *const *args, Py_ssize_t count, PyObjec
 {
     const torch::Tensor *tensors[TENSORS];
     int ints[INTS];
-    if (keywords == nullptr && plain_arguments(args, count, tensors, ints)) {
-        try {
-            return wrapped(call_plain<OPERATOR>(tensors, ints, std::make_index_sequence<TENSORS>(), std::make_index_sequence<INTS>()));
-        } catch (...) {
-            // the general function meets the same failure and says so
-        }
+    if (keywords != nullptr || !plain_arguments(args, count, tensors, ints))
+        return PyObject_Vectorcall(general<OPERATOR>, args, (size_t)count, keywords);
+    try {
+        return wrapped(call_plain<OPERATOR>(tensors, ints, std::make_index_sequence<TENSORS>(), std::make_index_sequence<INTS>()));
+    } catch (py::error_already_set &e) {
+        e.restore();
+    } catch (...) {
+        py::detail::try_translate_exceptions();
     }
-    return PyObject_Vectorcall(general<OPERATOR>, args, (size_t)count, keywords);
+    return nullptr;
 }
 
 // Puts the fast form of an operator in the place of the pybind11 functions of these names.

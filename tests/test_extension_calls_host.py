@@ -33,3 +33,31 @@ def test_arguments(name):
             f(*args)
     with pytest.raises(TypeError, match="incompatible function arguments"):
         f(*([X] * tensors + numbers[1:]), stride=1)
+
+
+class Watched(torch.Tensor):
+    """A tensor whose device an operator has to ask for in Python, where it can be told that it is elsewhere, or fail."""
+    asked, fails = 0, False
+
+    @staticmethod
+    def __new__(cls):
+        return torch.Tensor._make_wrapper_subclass(cls, (1, 8, 8, 64), dtype=torch.float32, device="cpu", dispatch_device=True)
+
+    @classmethod
+    def __torch_dispatch__(cls, func, types, args=(), kwargs=None):
+        assert func is torch.ops.prim.device.default, func
+        cls.asked += 1
+        if cls.fails:
+            raise KeyError("device of a watched tensor")
+        return torch.device("cpu")
+
+
+@pytest.mark.parametrize("fails, error, words", [(False, RuntimeError, "must be a CUDA tensor"), (True, KeyError, "device of a watched tensor")])
+@pytest.mark.parametrize("name", CALLS)
+def test_an_operator_is_entered_once(name, fails, error, words):
+    """Whatever an operator throws reaches the caller: a second try through the general function would launch, allocate and ask again."""
+    tensors, ints = CALLS[name]
+    x, Watched.fails, Watched.asked = Watched(), fails, 0
+    with pytest.raises(error, match=words):
+        getattr(_C, name)(x, *[X] * (tensors - 1), *[1] * ints)
+    assert Watched.asked == 1
