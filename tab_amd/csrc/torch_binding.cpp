@@ -633,8 +633,8 @@ PyObject *wrapped(std::vector<torch::Tensor> &&ys)
     return list;
 }
 
-// The pybind11 function of an operator, looked up when the module is made (and kept as long as the process).
-template <auto OPERATOR> PyObject *general = nullptr;
+// The pybind11 function of an operator under one of its names, looked up when the module is made (and kept as long as the process).
+template <auto OPERATOR, int ALIAS> PyObject *general = nullptr;
 
 template <auto OPERATOR, size_t... T, size_t... I>
 auto call_plain(const torch::Tensor *const *tensors, const int *ints, std::index_sequence<T...>, std::index_sequence<I...>)
@@ -642,13 +642,13 @@ auto call_plain(const torch::Tensor *const *tensors, const int *ints, std::index
     return OPERATOR(*tensors[T]..., ints[I]...);
 }
 
-template <auto OPERATOR, size_t TENSORS, size_t INTS>
+template <auto OPERATOR, size_t TENSORS, size_t INTS, int ALIAS>
 PyObject *fast_call(PyObject *, PyObject *const *args, Py_ssize_t count, PyObject *keywords)
 {
     const torch::Tensor *tensors[TENSORS];
     int ints[INTS];
     if (keywords != nullptr || !plain_arguments(args, count, tensors, ints))
-        return PyObject_Vectorcall(general<OPERATOR>, args, (size_t)count, keywords);
+        return PyObject_Vectorcall(general<OPERATOR, ALIAS>, args, (size_t)count, keywords);
     try {
         return wrapped(call_plain<OPERATOR>(tensors, ints, std::make_index_sequence<TENSORS>(), std::make_index_sequence<INTS>()));
     } catch (py::error_already_set &e) {
@@ -659,18 +659,16 @@ PyObject *fast_call(PyObject *, PyObject *const *args, Py_ssize_t count, PyObjec
     return nullptr;
 }
 
-// Puts the fast form of an operator in the place of the pybind11 functions of these names.
-template <auto OPERATOR, size_t TENSORS, size_t INTS>
-void make_fast(py::module_ &m, std::initializer_list<const char *> names)
+// Puts the fast form of an operator in the place of the pybind11 function of this name.
+template <auto OPERATOR, size_t TENSORS, size_t INTS, int ALIAS = 0>
+void make_fast(py::module_ &m, const char *name)
 {
-    static std::vector<std::unique_ptr<PyMethodDef>> definitions;
-    general<OPERATOR> = py::object(m.attr(*names.begin())).release().ptr();
-    for (const char *name : names) {
-        const char *const doc = PyUnicode_AsUTF8(py::object(py::handle(general<OPERATOR>).attr("__doc__")).release().ptr());
-        definitions.push_back(std::make_unique<PyMethodDef>(PyMethodDef{
-            name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&fast_call<OPERATOR, TENSORS, INTS>)), METH_FASTCALL | METH_KEYWORDS, doc}));
-        m.attr(name) = py::reinterpret_steal<py::object>(PyCFunction_NewEx(definitions.back().get(), nullptr, py::str(m.attr("__name__")).ptr()));
-    }
+    static PyMethodDef definition;
+    general<OPERATOR, ALIAS> = py::object(m.attr(name)).release().ptr();
+    const char *const doc = PyUnicode_AsUTF8(py::object(py::handle(general<OPERATOR, ALIAS>).attr("__doc__")).release().ptr());
+    definition = PyMethodDef{name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&fast_call<OPERATOR, TENSORS, INTS, ALIAS>)),
+                             METH_FASTCALL | METH_KEYWORDS, doc};
+    m.attr(name) = py::reinterpret_steal<py::object>(PyCFunction_NewEx(&definition, nullptr, py::str(m.attr("__name__")).ptr()));
 }
 
 }  // namespace
@@ -701,8 +699,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     m.def("Conv2dStatic", &TAB_Conv2dStatic, "Conv2d with the packed activation in the library's built-in scratch");
     m.def("Conv2dPacked", &TAB_Conv2dPacked, "Conv2d on an already packed activation");
     m.def("Conv2dPackedOut", &TAB_Conv2dPackedOut, "Conv2dPacked with the output quantized and packed in the epilogue");
-    make_fast<&TAB_Conv2d, 4, 12>(m, {"Conv2d", "TAB_Conv2d"});
-    make_fast<&TAB_Quantize, 2, 5>(m, {"Quantize", "TAB_Quantize"});
-    make_fast<&TAB_QuantizeNCHW, 2, 5>(m, {"QuantizeNCHW"});
-    make_fast<&TAB_Conv2dPacked, 3, 12>(m, {"Conv2dPacked"});
+    make_fast<&TAB_Conv2d, 4, 12>(m, "Conv2d");
+    make_fast<&TAB_Conv2d, 4, 12, 1>(m, "TAB_Conv2d");
+    make_fast<&TAB_Quantize, 2, 5>(m, "Quantize");
+    make_fast<&TAB_Quantize, 2, 5, 1>(m, "TAB_Quantize");
+    make_fast<&TAB_QuantizeNCHW, 2, 5>(m, "QuantizeNCHW");
+    make_fast<&TAB_Conv2dPacked, 3, 12>(m, "Conv2dPacked");
 }

@@ -61,3 +61,9 @@ def test_an_operator_is_entered_once(name, fails, error, words):
     with pytest.raises(error, match=words):
         getattr(_C, name)(x, *[X] * (tensors - 1), *[1] * ints)
     assert Watched.asked == 1
+
+
+@pytest.mark.parametrize("name", CALLS)
+def test_errors_name_the_function_that_was_called(name):
+    with pytest.raises(TypeError, match=rf"^{name}\(\): incompatible function arguments"):
+        getattr(_C, name)(1)
