@@ -634,9 +634,8 @@ PatchPlan conv_patch_plan(int type, const ConvArgs &a)
             best = i;
         }
     float waves_gain_us = 0.f;
-    const int other = conv_waves_or(type, a, plan.tiled, tiled_us, &waves_gain_us);
-    if (best >= 0 && (other < kWavesShape || waves_gain_us <= tiled_call_us - us[best] + 0.5f)) take(best, fits[best]);
-    else plan.tiled = other;
+    plan.tiled = conv_waves_or(type, a, plan.tiled, tiled_us, &waves_gain_us);  // (also where the weights then find no room)
+    if (best >= 0 && (plan.tiled < kWavesShape || waves_gain_us <= tiled_call_us - us[best] + 0.5f)) take(best, fits[best]);
     return plan;
 }
 

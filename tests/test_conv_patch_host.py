@@ -115,3 +115,21 @@ def test_the_rule_on_its_measured_calls(lib):
     assert len({c for c in chosen if c is not None}) == len(ROWS), stated  # every shape has launches of its own
     # launches of fewer tiles than compute units are not looked at
     assert plan(lib, 0, 1, 1, 1, 1, 16, 14, 14, 256, 256, 3, 3)[0] < 0 and plan(lib, 0, 1, 1, 1, 1, 64, 14, 14, 256, 256, 3, 3)[0] >= 0
+
+
+def test_a_plan_without_its_room_leaves_the_kernel_of_calls_without_any(lib):
+    """PatchPlan.tiled, what runs where the workspace cannot hold the weights: the kernel that launch_conv takes."""
+    lib.tab_set_conv_kernel(0, -1)
+    lib.tab_internal_conv_plan.restype, plan_of = ctypes.c_size_t, (ctypes.c_int * 16)()
+    planned, split = 0, 0
+    for type in range(5):
+        for N, H, C, KN, K in ((16, 14, 64, 512, 3), (36, 14, 256, 256, 3), (64, 14, 256, 256, 3), (64, 7, 512, 512, 3), (64, 14, 128, 320, 3),
+                               (16, 28, 128, 128, 3), (20, 20, 192, 200, 5), (64, 11, 320, 320, 3), (256, 28, 512, 512, 3), (100, 7, 256, 320, 3)):
+            lib.tab_internal_conv_plan(type, K // 2, K // 2, 1, 1, N, H, H, C, KN, K, K, plan_of)
+            if plan_of[0] < 0:
+                continue
+            PC = (C + 63) // 64
+            want = lib.tab_internal_conv_launch_shape(type, N * H * H, KN, K * K * PC, PC)
+            assert plan_of[4] == want, (type, N, H, C, KN, K)
+            planned, split = planned + 1, split + (want >= 19)
+    assert planned > 15 and split >= 2, (planned, split)
