@@ -114,6 +114,10 @@ int tab_internal_conv_launch_shape(int type, int M, int KN, int G, int PC)
     return tab::conv_fp32_shape(type, a);
 }
 
+/* Test hook, absent from include/tab_amd.h: whether items of two planes take a workgroup each (own: with thresholds of their own, else with
+ * counts). */
+int tab_internal_quantize_items(int own, int nchw, long items, long pixels, int C) { return tab::quantize_items_supported(own, nchw, items, pixels, C); }
+
 /* Test hook, absent from include/tab_amd.h: whether the one-launch kernel of the smallest calls can run a call, and its predicted
  * duration on the GPU in microseconds with the three numbers it comes from. */
 int tab_internal_conv_small_cost(int type, const float *dev_X, int nchw, int N, int H, int W, int C, int KN, int KH, int KW, int padding1,

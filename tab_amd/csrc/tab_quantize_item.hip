@@ -3,10 +3,11 @@
 //
 // With slices of an item in workgroups of their own, the sums of |x| or the counts take a launch before or behind the quantizer: 2.4 us on
 // the GPU and 2.8 of the host, more than a small item's reading.  Here a workgroup reads its item once for the sum, all loads requested at
-// once, and a second time, out of the L2, to pack it.  Bound by what one CU reads, some 40 GB/s of latency and 64 bytes a cycle, hence the
-// limits: items of 26 K values with their counts (24 K of ragged rows: 300 14x14x96 10.9 / 11.5), of 12 K with their thresholds.  Quantizer and counts in two launches / here, graph replays,
-// us: 136 14x14x64 5.3 / 4.2 (NCHW 6.1 / 4.0), 256 7x7x512 9.1 / 7.6, 79 25x15x64 5.5 / 4.7, but 16 14x14x256 (49 K) 4.8 / 6.5; sums and quantizer:
-// 91 rows of 576 4.6 / 3.7, 153 of 5376 5.4 / 4.3, 2000 of 700 12.3 / 7.2, but 79 25x15x64 (23 K) 6.1 / 6.9.  Called one after the other such
+// once, and a second time, out of the L2, to pack it.  Bound by the latency of one CU's reads and their 64 bytes a cycle, hence the
+// limits: items of 26 K values with their counts (24 K of ragged rows: 300 14x14x96 10.9 / 11.5), of 12 K with their thresholds, and not too many of
+// them (quantize_items_supported).  Quantizer and counts in two launches / here, graph replays,
+// us: 136 14x14x64 5.3 / 4.2 (NCHW 6.1 / 4.0), 256 7x7x512 9.4 / 8.1, 79 25x15x64 5.5 / 4.7, but 16 14x14x256 (49 K) 4.8 / 6.5; sums and quantizer:
+// 91 rows of 576 4.6 / 3.7, 153 of 5376 5.4 / 4.3, 2000 of 2000 11.0 / 8.4, but 79 25x15x64 (23 K) 6.1 / 6.9.  Called one after the other such
 // quantizers take 7.6 us in two launches, which is the host's time, and 5.0 in one; a ternary linear layer of 2048 inputs 11.4 in three, 8.5 in two.
 #include "tab_pack.h"
 #include "tab_patch_weights.h"
@@ -185,27 +186,48 @@ __global__ __launch_bounds__(64 * WAVES) void quantize_items(const float *__rest
 // An item's values at most, words NHWC as 64 of them; NCHW pieces of 64 pixels and 16 channels, of which sixteen waves take a round.
 constexpr long kCountedItem = 26 * 1024, kCountedRagged = 24 * 1024, kOwnItem = 12 * 1024, kCountedPieces = 32, kOwnPieces = 16;
 constexpr long kFewWaves = 4096;  // values up to which an item takes four waves
-constexpr long kManyItems = 256;  // items from which two of sixteen waves share a CU (300 10x10x96 NCHW with thresholds: 8.0 in two launches, 9.6)
 
 inline long item_pieces(long pixels, int C) { return (pixels + 63) / 64 * ((C + kWordBits - 1) / kWordBits) << plane_parts_log(C); }
 inline bool four_waves(bool nchw, long items, long pixels, int C)
 {
-    return pixels * C <= kFewWaves && (!nchw || item_pieces(pixels, C) <= (items > kManyItems ? 16 : 4));
+    // (from more items than CUs on two of sixteen waves share a CU: 300 10x10x96 NCHW with thresholds 8.0 in two launches, 9.6)
+    return pixels * C <= kFewWaves && (!nchw || item_pieces(pixels, C) <= (items > device_compute_units() ? 16 : 4));
 }
 
 }  // namespace
 
+// Where this kernel is the sooner one, of the calls it can take: 1177 measured ones of 0.3 to 500 MB (quantize_items_timings.txt).
+// The limits on the items are those of a workgroup's cost: four waves start 0.7 a nanosecond, whatever they read, and sixteen, two of which a CU
+// holds, are as slow as what one CU reads as soon as there are several rounds of them; the two launches stream.  Two launches / here, us: own
+// thresholds 16384 rows of 8192 values 160 / 242, 46875 of 128 46 / 71, 8000 7x7x128 67 / 111, counts 2200 7x7x300 29.6 / 42.6, 2200 NCHW 14x14x128
+// 43.5 / 50.3.  These rules take 0.884 of the two launches' time, the better of both ways 0.879 (all of them here: 0.967); of 683 choices one is more than
+// 2 % slower, by 13.
 bool quantize_items_supported(bool own, bool nchw, long items, long pixels, int C)
 {
     if (pixels > kCountedItem / C || items >= 0x7fffffffL) return false;
+    const long values = pixels * C, units = device_compute_units();
+    const bool four = four_waves(nchw, items, pixels, C);
     if (nchw) {
+        const long pieces = item_pieces(pixels, C);
         // (few channels leave the sums nothing to make up for: 46 21x21x27, thresholds and quantizer, 6.2 us in two launches, 7.1 in one)
-        return own ? C > 32 && pixels * C <= kOwnItem && item_pieces(pixels, C) <= kOwnPieces && (items <= kManyItems || four_waves(true, items, pixels, C))
-                   : item_pieces(pixels, C) <= kCountedPieces;
+        if (own)  // past a round, items that fill their lanes
+            return C > 32 && values <= kOwnItem && pieces <= kOwnPieces &&
+                   (items <= units || (four && (values >= 320 * pieces || (pieces <= 8 && items <= 4 * units))));
+        if (four || pieces > kCountedPieces) return pieces <= kCountedPieces;
+        if (pieces <= 8) return false;  // half of the waves would have nothing to do
+        // Planes shorter than a wave: the other kernels take four pixels a thread only of planes of whole fours, and once x is
+        // past the caches they read each cache line several times.  Other planes: as long as the other kernels have too few waves.
+        if (pixels % 4 != 0 && pixels > 2 && pixels < 64) return true;
+        return items * values <= 7L << 20 || (pixels <= 64 && items * values > 80L << 20);
     }
     // (up to 32 channels go by tiles: a row of 16 lanes a pixel would be mostly empty)
-    return C > 32 && pixels * ((C + kWordBits - 1) / kWordBits) * kWordBits <=
-                         (own ? kOwnItem : C % kWordBits ? kCountedRagged : kCountedItem);
+    const long rows = pixels * ((C + kWordBits - 1) / kWordBits);
+    if (C <= 32 || rows * kWordBits > (own ? kOwnItem : C % kWordBits ? kCountedRagged : kCountedItem)) return false;
+    if (!own) return C % kWordBits ? items <= units && (rows <= 256 || 4 * items > units) : items * values <= 16L << 20;
+    if (!four) return items <= 2 * units && values % 4 == 0;  // (an item between two multiples of four values is summed a value a load)
+    if (C % kWordBits == 0) return values >= 768 || items <= 6 * values;
+    if (values < 1024) return 2 * items <= 5 * values;
+    return items <= 32 * units || (values % 4 == 0 && values >= 1792);
 }
 
 hipError_t launch_quantize_items(const float *x, const Thresholds &ths, bool nchw, long items, long pixels, int C, uint64_t *qx, int32_t *btn, hipStream_t stream)

@@ -1,0 +1,41 @@
+"""The rules that pick a quantizer's form, on the host: the library's choices on measured calls of both forms, with the regret that the rules'
+comments state."""
+import ctypes
+import os
+import re
+
+import numpy as np
+import pytest
+
+from tab_amd import _capi
+
+TUNING = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "tab_amd", "tuning")
+
+
+def geometric(ratios):
+    return float(np.exp(np.mean(np.log(ratios))))
+
+
+def parse(name, pattern):
+    with open(os.path.join(TUNING, name)) as f:
+        for line in f:
+            m = re.match(pattern, line)
+            if m:
+                yield m.groups()
+
+
+def test_items_by_workgroups():
+    f = ctypes.CDLL(_capi.LIB_PATH).tab_internal_quantize_items
+    f.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_long, ctypes.c_long, ctypes.c_int]
+    taken, best, chosen = [], [], 0
+    for kind, layout, N, H, W, C, two, one in parse("quantize_items_timings.txt", r"(own|counts) (NHWC|NCHW) (\d+)x(\d+)x(\d+)x(\d+) \| (\S+) (\S+)"):
+        two, one = float(two), float(one)
+        items = bool(f(kind == "own", layout == "NCHW", int(N), int(H) * int(W), int(C)))
+        taken.append((one if items else two) / two)
+        best.append(min(one, two) / two)
+        chosen += items
+    slower = np.array(taken)
+    stated = (len(taken), chosen, geometric(taken), geometric(best), sorted(slower)[-3:])
+    assert len(taken) > 1150 and 650 < chosen < 720, stated
+    assert geometric(taken) < 0.885 and geometric(best) > 0.878, stated  # fitted: 0.8838, 0.8792
+    assert (slower > 1.02).sum() <= 1 and slower.max() < 1.14, stated
