@@ -118,6 +118,13 @@ int tab_internal_conv_launch_shape(int type, int M, int KN, int G, int PC)
  * counts). */
 int tab_internal_quantize_items(int own, int nchw, long items, long pixels, int C) { return tab::quantize_items_supported(own, nchw, items, pixels, C); }
 
+/* Test hook, absent from include/tab_amd.h: the form of an NCHW quantizer: -1 gathered words, else the waves of a last word apart, 0 of none. */
+int tab_internal_plane_form(int bitwidth, long N, long HW, int C)
+{
+    const tab::PlaneForm form = tab::plane_form(bitwidth, N, HW, C);
+    return form.gather ? -1 : form.last;
+}
+
 /* Test hook, absent from include/tab_amd.h: whether the one-launch kernel of the smallest calls can run a call, and its predicted
  * duration on the GPU in microseconds with the three numbers it comes from. */
 int tab_internal_conv_small_cost(int type, const float *dev_X, int nchw, int N, int H, int W, int C, int KN, int KH, int KW, int padding1,

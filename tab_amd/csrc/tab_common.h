@@ -281,6 +281,13 @@ hipError_t launch_quantize(const float *x, const Thresholds &ths, int bitwidth, 
 hipError_t launch_quantize_nchw(const float *x, const Thresholds &ths, int bitwidth, int N, int C, long HW, uint64_t *qx,
                                 int32_t *btn, int32_t *count_workspace, hipStream_t stream, const WeightJob *weights = nullptr);
 
+// Of an NCHW tensor: whether the form that gathers words takes it (`unit` a thread), else the waves of a last word apart, or 0.
+struct PlaneForm {
+    bool gather;
+    int unit, last;
+};
+PlaneForm plane_form(int bitwidth, long N, long HW, int C);
+
 // Small items of two planes, a workgroup each (tab_quantize_item.hip): with given thresholds and the counts (btn), or with thresholds
 // that it finds itself, scale * mean|x|, as launch_threshold would to the last bit.  own: which of the two.
 bool quantize_items_supported(bool own, bool nchw, long items, long pixels, int C);

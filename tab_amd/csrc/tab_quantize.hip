@@ -1167,6 +1167,27 @@ hipError_t launch_patch_weights(const WeightJob &job, hipStream_t stream)
     return hipGetLastError();
 }
 
+// Words of an NCHW tensor whose pixels have several: whether the form that gathers each wave's output into whole runs of them takes it (PC even,
+// enough pixels for a wave on every SIMD), `unit` words a thread, and else how many waves a last word of at most 32 channels takes, apart from the
+// others (0: as many as those).  1500 measured calls (quantize_last_words_timings.txt), gathered or all words alike / by this rule, us:
+//   * A thread of the gathering form goes through such a last word as long as through the others.  With two words a thread (PC = 2, 6, 10 ..)
+//     units are the sooner form then: one plane 46 80x80 of 80 24.6 / 20.0, 3287 7x7 of 348 61.2 / 51.1.  With four the form's whole lines are worth
+//     more (120 56x56 of 209 62.5 in units, 58.5; 45 64x64 of 453 69.8, 62.6), unless planes are not whole fours, of which units read no less:
+//     1263 of 205 pixels and 224 channels 55.4 / 51.2; at more than four words only where they are shorter than a wave.
+//   * Last words apart are half of PC = 2's work: 5 % from 4 MB of one plane on, 10 % from 30, of two planes 2 % from 6 MB; a third to an
+//     eighth, 2 % from 40 MB on, one plane only.  Below that a launch is as long as its longest wave, which such a unit makes 0.1 us later (2 47x61 of
+//     261 4.04, 3.88), and four words of two planes are half a cache line a pixel, which the last word then reaches later.
+// All of them: 0.977 of the forms' time that know no such words, the best form of each 0.969, 15 more than 3 % slower, the worst 9; units with the last
+// words apart everywhere 0.990, 395 more than 3 % slower, the worst 44.
+PlaneForm plane_form(int bitwidth, long N, long HW, int C)
+{
+    const int PC = (C + kWordBits - 1) / kWordBits, few = last_word_waves(C, PC), unit = PC % 4 == 0 ? 4 : PC % 2 == 0 ? 2 : 1;
+    const long gather_waves = (N * ((HW + 3) / 4) + 63) / 64 * (PC / unit), values = N * HW * C;
+    const bool units = few && (unit == 2 ? bitwidth == 1 || PC == 2 : bitwidth == 1 && HW % 4 != 0 && (PC == 4 || HW < 64));
+    const bool apart = PC == 2 ? values >= (bitwidth == 1 ? 1L << 20 : 3L << 19) : bitwidth == 1 && PC <= 8 && values >= 10L << 20;
+    return {HW >= 4 && unit > 1 && gather_waves >= 1024 && !units, unit, apart ? few : 0};
+}
+
 hipError_t launch_quantize_nchw(const float *x, const Thresholds &ths, int bitwidth, int N, int C, long HW, uint64_t *qx,
                                 int32_t *btn, int32_t *count_workspace, hipStream_t stream, const WeightJob *weights)
 {
@@ -1190,16 +1211,13 @@ hipError_t launch_quantize_nchw(const float *x, const Thresholds &ths, int bitwi
         job.blocks *= kThreads / threads;
         kernel<<<dim3((unsigned)blocks + job.blocks), dim3(threads), 0, stream>>>(x, ordered(ths, blocks), qx, N, C, HW, PC, by_image(per_image), job);
     };
-    // PC even, enough pixels for a wave on every SIMD: the form that gathers each wave's output into whole runs, unless its last word is mostly
-    // empty: a thread would go through that one as long as through the others (us, one plane, gathered / by units: 96 61x47 of 75 channels 24.5 /
-    // 18.5, 256 57x57 of 80 68.6 / 53, 200 60x60 of 72 47.1 / 42.1, 128 56x56 of 90 29.4 / 28.3)
-    const int unit = PC % 4 == 0 ? 4 : PC % 2 == 0 ? 2 : 1;
-    // (four words of two planes are half a cache line a pixel, which the last word then reaches later: 100 40x40 of 210 31.4 us, 32.5 with it apart)
-    int last = bitwidth == 2 && PC >= 4 ? 0 : last_word_waves(C, PC);
+    const PlaneForm words = plane_form(bitwidth, N, HW, C);
+    const int unit = words.unit;
+    int last = words.last;
     const long gather_waves = (runs + 63) / 64 * (PC / unit);
     if (gather_waves > 0x7fffffffL) return hipErrorInvalidValue;
     const long gather_slices = (runs / N + 63) / 64 * (PC / unit);
-    if (HW >= 4 && (uintptr_t)qx % 16 == 0 && unit > 1 && gather_waves >= 1024 && !last && !(counted && gather_slices > 1 && !count_workspace)) {
+    if (words.gather && (uintptr_t)qx % 16 == 0 && !(counted && gather_slices > 1 && !count_workspace)) {
         if (counted) {
             const long slices = gather_slices;
             auto launch_counted = [&](auto kernel) {

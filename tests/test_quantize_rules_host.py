@@ -39,3 +39,25 @@ def test_items_by_workgroups():
     assert len(taken) > 1150 and 650 < chosen < 720, stated
     assert geometric(taken) < 0.885 and geometric(best) > 0.878, stated  # fitted: 0.8838, 0.8792
     assert (slower > 1.02).sum() <= 1 and slower.max() < 1.14, stated
+
+
+def test_last_words():
+    f = ctypes.CDLL(_capi.LIB_PATH).tab_internal_plane_form
+    f.argtypes = [ctypes.c_int, ctypes.c_long, ctypes.c_long, ctypes.c_int]
+    taken, apart, best = [], [], []
+    for bits, N, H, W, C, alike, last, units in parse("quantize_last_words_timings.txt", r"planes (\d) (\d+)x(\d+)x(\d+)x(\d+) \| (\S+) (\S+) (\S+)"):
+        alike, last, units = float(alike), float(last), float(units)
+        form = f(int(bits), int(N), int(H) * int(W), int(C))
+        assert form in (-1, 0, 1, 2)
+        PC = (int(C) + 63) // 64
+        unit = 4 if PC % 4 == 0 else 2 if PC % 2 == 0 else 1
+        large = unit > 1 and (int(N) * ((int(H) * int(W) + 3) // 4) + 63) // 64 * (PC // unit) >= 1024  # (else "alike" is "units" timed twice)
+        assert form >= 0 or large
+        taken.append((last if form > 0 else units if large and form == 0 else alike) / alike)
+        apart.append(form > 0)
+        best.append(min(alike, last, units) / alike)
+    slower = np.array(taken)
+    stated = (len(taken), sum(apart), geometric(taken), geometric(best), (slower > 1.03).sum(), (slower > 1.05).sum(), slower.max())
+    assert len(taken) == 1500 and 480 < sum(apart) < 500, stated
+    assert geometric(taken) < 0.978 and geometric(best) > 0.969, stated  # fitted: 0.9771, 0.9693
+    assert (slower > 1.03).sum() <= 15 and (slower > 1.05).sum() <= 7 and slower.max() < 1.1, stated
