@@ -200,8 +200,8 @@ inline bool four_waves(bool nchw, long items, long pixels, int C)
 // The limits on the items are those of a workgroup's cost: four waves start 0.7 a nanosecond, whatever they read, and sixteen, two of which a CU
 // holds, are as slow as what one CU reads as soon as there are several rounds of them; the two launches stream.  Two launches / here, us: own
 // thresholds 16384 rows of 8192 values 160 / 242, 46875 of 128 46 / 71, 8000 7x7x128 67 / 111, counts 2200 7x7x300 29.6 / 42.6, 2200 NCHW 14x14x128
-// 43.5 / 50.3.  These rules take 0.884 of the two launches' time, the better of both ways 0.879 (all of them here: 0.967); of 683 choices one is more than
-// 2 % slower, by 13.
+// 43.5 / 50.3.  These rules take 0.882 of the two launches' time, the better of both ways 0.879 (all of them here: 0.967); of 702 choices four are more than
+// 2 % slower, the worst 13.
 bool quantize_items_supported(bool own, bool nchw, long items, long pixels, int C)
 {
     if (pixels > kCountedItem / C || items >= 0x7fffffffL) return false;
@@ -214,16 +214,16 @@ bool quantize_items_supported(bool own, bool nchw, long items, long pixels, int 
             return C > 32 && values <= kOwnItem && pieces <= kOwnPieces &&
                    (items <= units || (four && (values >= 320 * pieces || (pieces <= 8 && items <= 4 * units))));
         if (four || pieces > kCountedPieces) return pieces <= kCountedPieces;
-        if (pieces <= 8) return false;  // half of the waves would have nothing to do
+        if (pieces <= (items > units ? 12 : 8)) return false;  // waves would have nothing to do
         // Planes shorter than a wave: the other kernels take four pixels a thread only of planes of whole fours, and once x is
         // past the caches they read each cache line several times.  Other planes: as long as the other kernels have too few waves.
         if (pixels % 4 != 0 && pixels > 2 && pixels < 64) return true;
-        return items * values <= 7L << 20 || (pixels <= 64 && items * values > 80L << 20);
+        return items * values <= 8L << 20 || (pixels <= 64 && items * values > 80L << 20);
     }
     // (up to 32 channels go by tiles: a row of 16 lanes a pixel would be mostly empty)
     const long rows = pixels * ((C + kWordBits - 1) / kWordBits);
     if (C <= 32 || rows * kWordBits > (own ? kOwnItem : C % kWordBits ? kCountedRagged : kCountedItem)) return false;
-    if (!own) return C % kWordBits ? items <= units && (rows <= 256 || 4 * items > units) : items * values <= 16L << 20;
+    if (!own) return C % kWordBits ? items <= units && (rows <= 256 || 4 * items > units) : items * values <= 24L << 20;
     if (!four) return items <= 2 * units && values % 4 == 0;  // (an item between two multiples of four values is summed a value a load)
     if (C % kWordBits == 0) return values >= 768 || items <= 6 * values;
     if (values < 1024) return 2 * items <= 5 * values;

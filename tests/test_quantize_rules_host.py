@@ -37,8 +37,8 @@ def test_items_by_workgroups():
     slower = np.array(taken)
     stated = (len(taken), chosen, geometric(taken), geometric(best), sorted(slower)[-3:])
     assert len(taken) > 1150 and 650 < chosen < 720, stated
-    assert geometric(taken) < 0.885 and geometric(best) > 0.878, stated  # fitted: 0.8838, 0.8792
-    assert (slower > 1.02).sum() <= 1 and slower.max() < 1.14, stated
+    assert geometric(taken) < 0.883 and geometric(best) > 0.879, stated  # fitted: 0.8824, 0.8792
+    assert (slower > 1.02).sum() <= 4 and (slower > 1.05).sum() <= 2 and slower.max() < 1.14, stated
 
 
 def test_last_words():
