@@ -114,6 +114,9 @@ int tab_internal_conv_launch_shape(int type, int M, int KN, int G, int PC)
     return tab::conv_fp32_shape(type, a);
 }
 
+/* Test hook, absent from include/tab_amd.h: workgroups a CU of a packed layer of short K. */
+int tab_internal_regs_on_cu(int G, int tiles, int tiles_n, int most, int cus) { return tab::regs_on_cu(G, tiles, tiles_n, most, cus); }
+
 /* Test hook, absent from include/tab_amd.h: whether items of two planes take a workgroup each (own: with thresholds of their own, else with
  * counts). */
 int tab_internal_quantize_items(int own, int nchw, long items, long pixels, int C) { return tab::quantize_items_supported(own, nchw, items, pixels, C); }

@@ -229,6 +229,39 @@ int conv_mfma_shape(int type, const ConvArgs &args, float *cost_us = nullptr);
 // At most 32 filters, fp32 output, an even number of words per pixel: the shapes of 64 filters that exist in a form of 32.
 inline bool conv_mfma_narrow(const ConvArgs &a) { return a.KN <= 32 && a.PC % 2 == 0 && a.qy == nullptr; }
 hipError_t launch_conv_mfma(int type, const ConvArgs &args, int shape, hipStream_t stream);
+// Of the kernel with the weights in registers (tab_conv_mfma_regs.h): workgroups along M for `tiles` 32-pixel tiles: one tile per wave while
+// the launch is small; from `cap` workgroups on, the fewest rounds with the waves evenly loaded.
+inline unsigned regs_grid_x(int tiles, int cap)
+{
+    const int wanted = (tiles + 3) / 4;
+    if (wanted <= cap) return (unsigned)wanted;
+    const int rounds = (tiles + 4 * cap - 1) / (4 * cap);
+    return (unsigned)(((tiles + rounds - 1) / rounds + 3) / 4);
+}
+// Packed output: how many of its workgroups a CU is to get, of `most` that fit.  As many as fit is not the soonest way: every workgroup expands its
+// weights first, and the rounds of more waves divide the tiles more roughly.  What the busiest CU takes, in turns of its waves: rounds, each of
+// its workgroups' turns and a wait that they do not hide (the longer of turns with few words), and the expansions; fewer only where that gains
+// 2 %.  819 measured layers of 6 to 150 us (regs_workgroups_timings.txt): 0.967 of the time with as many as fit, the best count 0.958; seven more than
+// 3 % slower, the worst 6 %.  Packing by comparisons, whose registers left room for fewer / by signs and as many as fit / this, us: one plane N=34
+// 71x48x256->64 BTN 6.5 / 8.4 / 6.5, N=219 18x38x256->256 BNN 14.6 / 16.3 / 13.8, N=73 48x44x256->512 21.4 / 23.5 / 20.3, N=53 47x43x64->512 13.4 / 11.9 / 8.4.
+inline int regs_on_cu(int G, int tiles, int tiles_n, int most, int cus)
+{
+    const int full = most < 4 ? most : 4;
+    int best = full;
+    float full_cost = 0.f, best_cost = 0.f;
+    for (int n = full; n >= 2; n--) {
+        const int cap = n * cus / tiles_n < 1 ? 1 : n * cus / tiles_n;
+        const unsigned grid = regs_grid_x(tiles, cap) * (unsigned)tiles_n;
+        const int rounds = ((tiles + 3) / 4 + cap - 1) / cap, busiest = (int)((grid + (unsigned)cus - 1) / (unsigned)cus);
+        const float cost = (float)rounds * ((float)busiest + 0.2f + 0.3f / (float)G) + (float)busiest;
+        if (n == full) full_cost = best_cost = cost;
+        if (cost < best_cost) {
+            best = n;
+            best_cost = cost;
+        }
+    }
+    return best_cost < 0.98f * full_cost ? best : full;
+}
 // Of the kernel that splits K over the waves of a workgroup (tab_conv_mfma_waves.h): the shape with the lowest predicted duration.
 int conv_waves_shape(int type, const ConvArgs &args, float *cost_us);
 // The shape of a launch of fp32 output: that kernel's, or the one that conv_mfma_shape picks.

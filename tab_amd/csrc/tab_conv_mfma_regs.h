@@ -310,16 +310,6 @@ __global__ __launch_bounds__(kConvThreads) __attribute__((amdgpu_waves_per_eu(2,
     }
 }
 
-// Workgroups along M for `tiles` 32-pixel tiles: one tile per wave while the launch is small; from `cap` workgroups on,
-// the fewest rounds with the waves evenly loaded.
-inline unsigned regs_grid_x(int tiles, int cap)
-{
-    const int wanted = (tiles + 3) / 4;
-    if (wanted <= cap) return (unsigned)wanted;
-    const int rounds = (tiles + 4 * cap - 1) / (4 * cap);
-    return (unsigned)(((tiles + rounds - 1) / rounds + 3) / 4);
-}
-
 template <int TYPE, int G, int TN, int OUT>
 hipError_t launch_mfma_regs_tile(ConvArgs a, hipStream_t stream)
 {
@@ -339,7 +329,14 @@ hipError_t launch_mfma_regs_tile(ConvArgs a, hipStream_t stream)
         resident.store(held, std::memory_order_relaxed);
     }
     const int tiles = (a.M + 31) / 32;
-    const int cap = (held + tiles_n - 1) / tiles_n;
+    int cap = (held + tiles_n - 1) / tiles_n;
+    if (OUT >= kOutBits1) {
+        // (of four words and 128 filters in one plane a BNN layer's third workgroup only slows the others down: us, three / two a CU, N=153
+        // 30x53x256->512 29.0 / 26.1, N=129 51x80x256->128 18.2 / 16.9)
+        const int cus = device_compute_units(), fit = held / cus;
+        const int on_cu = regs_on_cu(G, tiles, tiles_n, TYPE == 3 && G == 4 && TN == 4 && OUT == kOutBits1 && fit > 2 ? 2 : fit, cus);
+        cap = on_cu * cus / tiles_n;
+    }
     a.kcw = G;
     a.nchunks = 1;
     const unsigned grid_x = regs_grid_x(tiles, cap < 1 ? 1 : cap);
