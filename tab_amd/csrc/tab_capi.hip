@@ -114,6 +114,15 @@ int tab_internal_conv_launch_shape(int type, int M, int KN, int G, int PC)
     return tab::conv_fp32_shape(type, a);
 }
 
+/* Test hook, absent from include/tab_amd.h: what the kernel that splits K over waves is predicted to gain over the tiled ones, in microseconds;
+ * infinity where those of 32x32 rank first, -infinity where it is not taken. */
+float tab_internal_conv_waves_gain(int type, int M, int KN, int G, int PC)
+{
+    tab::ConvArgs a = {};
+    a.M = M; a.KN = KN; a.G = G; a.PC = PC;
+    return tab::conv_waves_gain(type, a);
+}
+
 /* Test hook, absent from include/tab_amd.h: workgroups a CU of a packed layer of short K. */
 int tab_internal_regs_on_cu(int G, int tiles, int tiles_n, int most, int cus) { return tab::regs_on_cu(G, tiles, tiles_n, most, cus); }
 

@@ -266,6 +266,8 @@ inline int regs_on_cu(int G, int tiles, int tiles_n, int most, int cus)
 int conv_waves_shape(int type, const ConvArgs &args, float *cost_us);
 // The shape of a launch of fp32 output: that kernel's, or the one that conv_mfma_shape picks.
 int conv_fp32_shape(int type, const ConvArgs &args);
+// What that kernel is predicted to gain over the tiles, microseconds: infinity where it has their place by rank, -infinity where it is not taken.
+float conv_waves_gain(int type, const ConvArgs &args);
 hipError_t launch_conv_mfma_tnn(const ConvArgs &args, int shape, hipStream_t stream);
 hipError_t launch_conv_mfma_tbn(const ConvArgs &args, int shape, hipStream_t stream);
 hipError_t launch_conv_mfma_btn(const ConvArgs &args, int shape, hipStream_t stream);

@@ -561,6 +561,13 @@ static int conv_waves_or(int type, const ConvArgs &a, int tiled, float tiled_us,
     return us < (limit < kWavesLimitUs ? limit : kWavesLimitUs) ? shape : tiled;
 }
 
+float conv_waves_gain(int type, const ConvArgs &a)
+{
+    float us = 0.f, gain = 0.f;
+    const int tiled = conv_mfma_shape(type, a, &us);
+    return conv_waves_or(type, a, tiled, us, &gain) >= kWavesShape ? (tiled == 3 ? INFINITY : gain) : -INFINITY;
+}
+
 int conv_fp32_shape(int type, const ConvArgs &a)
 {
     float us = 0.f;
@@ -570,12 +577,16 @@ int conv_fp32_shape(int type, const ConvArgs &a)
 
 // The kernel that keeps the input patch in LDS, against the tiled one that conv_mfma_shape picks: the shape with the lowest predicted
 // duration, if that is 1.5 % and 0.1 us below what the call through the tiled kernel is predicted to take (tab_conv_patch_model.h; both are
-// linear forms with non-negative coefficients, fitted to the whole calls of 3970 random layers, those that choices slowed down by more than 5 %
-// counted threefold).  Those calls take 0.965 of the tiled kernels' time (in total 0.955; the better one of each 0.957 and 0.945), of 1313 choices
-// 30 are more than 2 % slower, the worst 4.6 %; on halves held out of the fit 0.966, 61, 21 more than 5 %, the worst 32 %.  (Fitted to
+// linear forms with non-negative coefficients, fitted to the whole calls of 8169 layers, a quarter of them long K on few tiles and rows of Y that
+// end inside a cache line, where a fit to 3970 had gone wrong: N=24 104x104x7->348 BNN 119 us through the tiles it chose, 78 here).  Those calls take 0.955 of
+// the time without this kernel (in total 0.934; the better one of each 0.949 and 0.927), of 2821 choices 116 are more than 2 % slower, 33 more than
+// 5 %, the worst 18 %; on thirds held out of the fit 0.956, 141, 48, 18 %; on 1499 layers measured after it 0.956 (0.960 before, best 0.949), of 499
+// choices 19 more than 2 % slower, five 5 %, the worst 10 % (33 % before), and 15 calls more than 10 % above the best kernel (37).  (Fitted to
 // convolutions replayed on the same operands, weights in the L2s, a tenth of such layers were more than 5 % slower, the worst 1.6 times.)
-// Where the tiled kernel's place is the split-K kernel's (conv_waves_or), that one is taken if it is predicted to gain half a microsecond more
-// than the patch: of 599 of those layers 187 where the rules want both, patch 0.896 of the tiled time, split K 0.859, the choice 0.858 (an odd number of words' tiles since faster).
+// Where the tiled kernel's place is the split-K kernel's (conv_waves_or), the patch is taken if it is predicted to gain as much: of 995 such layers
+// it is in 52, 0.999 of the split-K kernel's time, the better one of each 0.997.
+// Long K on few tiles, more than 192 words on less than 1.4 to 2 tiles of 64x64 a CU, stays with the others: the weights come from behind the L2s once, and
+// nothing hides them (N=4 54x64x888->128 7x7 TBN 73 us in tile 8, 114 here).
 // Not for 1x1 kernels, which read every pixel for one tap only, nor for at most 32 filters, half of whose tiles would be work for nothing,
 // nor for launches of fewer 64x64 tiles than compute units, which last as long as one tile's chain of waits (from half as many on, 129
 // of 2709 layers gained more than 3 %, none that a fit could tell from the others).  Measured, whole calls, tiled / patch: N=64 14x14x256
@@ -615,14 +626,18 @@ PatchPlan conv_patch_plan(int type, const ConvArgs &a)
         plan.tiled = conv_waves_shape(type, a, nullptr);
         return plan;
     }
+    const long kn64 = ((long)a.KN + 63) / 64, cus = device_compute_units();
+    float waves_gain_us = 0.f;
+    const int tiled = plan.tiled;
+    plan.tiled = conv_waves_or(type, a, tiled, tiled_us, &waves_gain_us);  // (also where the weights then find no room)
+    if (a.G > 192 && ((long)a.M + 63) / 64 * kn64 * 512 < cus * (512 + a.G)) return plan;
     float t[kTiledFeatures];
-    tiled_features(a, type, tiled_us, t);
+    tiled_features(a, type, tiled, tiled_us, t);
     float limit = 0.f;
     for (int k = 0; k < kTiledFeatures; k++) limit += kTiledCost[type][k] * t[k];
     const float tiled_call_us = limit;
     limit = 0.985f * limit - 0.1f;
-    const long kn64 = ((long)a.KN + 63) / 64;
-    const PatchCall call = patch_call(a, type, (uint32_t)device_compute_units());
+    const PatchCall call = patch_call(a, type, (uint32_t)cus);
     PatchFit fits[kPatchShapes];
     for (int i = 0; i < kPatchShapes; i++) fits[i] = kPatchTwins.of[i] < i ? fits[kPatchTwins.of[i]] : fit_of(i);
     float us[kPatchColumns];
@@ -633,9 +648,7 @@ PatchPlan conv_patch_plan(int type, const ConvArgs &a)
             limit = us[i];
             best = i;
         }
-    float waves_gain_us = 0.f;
-    plan.tiled = conv_waves_or(type, a, plan.tiled, tiled_us, &waves_gain_us);  // (also where the weights then find no room)
-    if (best >= 0 && (plan.tiled < kWavesShape || waves_gain_us <= tiled_call_us - us[best] + 0.5f)) take(best, fits[best]);
+    if (best >= 0 && (plan.tiled < kWavesShape || waves_gain_us <= tiled_call_us - us[best])) take(best, fits[best]);
     return plan;
 }
 

@@ -79,7 +79,7 @@ constexpr PatchTwins patch_twins()
 constexpr PatchTwins kPatchTwins = patch_twins();
 
 // What the predicted durations (tab_conv_patch_model.h) are linear in; the fit script states the same.
-constexpr int kPatchFeatures = 18, kTiledFeatures = 14;
+constexpr int kPatchFeatures = 21, kTiledFeatures = 32;
 constexpr int kPatchColumns = 8;  // kPatchShapes and a spare one: two vectors of four
 
 // A call through shape i: the busiest CU holds n tiles in so many rounds; its loop, its patches, its chunks and its output.  Then what the
@@ -90,14 +90,15 @@ constexpr int kPatchColumns = 8;  // kPatchShapes and a spare one: two vectors o
 // TNN 8.5 us of it a call), so the rule's time is theirs (with the tiled kernels' ranking 340 -> 210 ns, shapes one after the other before).
 struct PatchCall {
     uint32_t M, KN, cus;
-    float y_mb, ragged, one, one_y_mb, ragged_uncached;
+    float y_mb, ragged, one, one_y_mb, ragged_uncached, beyond, ragged_beyond;
     float weights_mb;  // of a pair of words
 };
+inline float y_beyond_mb(float y_mb) { return y_mb > 256.f ? y_mb - 256.f : 0.f; }
 inline PatchCall patch_call(const ConvArgs &a, int type, uint32_t cus)
 {
-    const float y_mb = (float)a.M * (float)a.KN * 4e-6f, ragged = a.KN % 32 ? y_mb : 0.f;
+    const float y_mb = (float)a.M * (float)a.KN * 4e-6f, ragged = a.KN % 32 ? y_mb : 0.f, beyond = y_beyond_mb(y_mb);
     return PatchCall{(uint32_t)a.M, (uint32_t)a.KN, cus, y_mb, ragged, a.PC == 1 ? 1.f : 0.f, a.PC == 1 ? y_mb : 0.f,
-                     ragged_rows_cached(a.M, a.KN) ? 0.f : ragged, (float)((a.KN + 31) / 32) * (patch_weight_planes(type) == 2 ? 1024e-6f : 512e-6f)};
+                     ragged_rows_cached(a.M, a.KN) ? 0.f : ragged, beyond, a.KN % 32 ? beyond : 0.f, (float)((a.KN + 31) / 32) * (patch_weight_planes(type) == 2 ? 1024e-6f : 512e-6f)};
 }
 // The durations in the shapes whose patch fits (kc > 0); infinity in the others.  Column by column: the sums of all shapes go on at once.
 inline void patch_durations(const PatchCall &c, const PatchFit (&fits)[kPatchShapes], const float (&cost)[kPatchFeatures][kPatchColumns],
@@ -132,23 +133,31 @@ inline void patch_durations(const PatchCall &c, const PatchFit (&fits)[kPatchSha
         const Four sum = (of(0) + of(1) * busy + of(2) * (K * vn) + of(3) * (K * vrounds) + of(4) * vn + of(5) * vrounds) +
                          (of(6) * c.y_mb + of(7) * (c.y_mb * busy) + of(8) * (patch * vn) + of(9) * (patch * vrounds) + of(10) * (vchunks * vrounds) + of(11) * load) +
                          (of(12) * c.ragged + of(13) * (c.weights_mb * vpairs) + of(14) * (0.01f * vpairs) + of(15) * c.one + of(16) * c.one_y_mb +
-                          of(17) * c.ragged_uncached);
+                          of(17) * c.ragged_uncached) +
+                         (of(18) * c.beyond + of(19) * c.ragged_beyond + of(20) * (c.weights_mb * vpairs / __builtin_elementwise_max(load, Four{1.f, 1.f, 1.f, 1.f})));
         for (int j = 0; j < 4; j++) us[i + j] += sum[j];
     }
 }
 
-// The call through the tiled kernel that conv_mfma_shape picks, which predicts `us` for its convolution: that prediction was fitted to even
-// words per pixel, whole lines of Y and launches like the benchmark's.
-inline void tiled_features(const ConvArgs &a, int type, float us, float (&f)[kTiledFeatures])
+// The call through the tiled kernel, of the shape that conv_mfma_shape picks, which predicts `us` for its convolution: that prediction was fitted to
+// even words per pixel, whole lines of Y and launches like the benchmark's.  Each shape has its own measure of it; chunks of K are single pairs of
+// words where a pixel's words are no multiple of four and K none of six (launch_mfma_shape), which long K feels (N=22 24x18x128->128 5x5 BTN
+// tiled 15.5 us, patch 10.1).
+constexpr int kTiledShapes[] = {0, 1, 2, 4, 5, 6, 8, 9, 10, 11};
+inline void tiled_features(const ConvArgs &a, int type, int shape, float us, float (&f)[kTiledFeatures])
 {
-    const float G = (float)a.G, y_mb = (float)a.M * (float)a.KN * 4e-6f;
+    const float G = (float)a.G, y_mb = (float)a.M * (float)a.KN * 4e-6f, beyond = y_beyond_mb(y_mb);
     const float products = (float)a.M * (float)((a.KN + 63) / 64 * 64) * G * 1e-9f;
-    const bool odd = a.PC % 2 != 0, one = a.PC == 1;
-    const float ragged = a.KN % 32 ? y_mb : 0.f;
-    const float values[kTiledFeatures] = {1.f, us, y_mb, products, odd ? products : 0.f, odd ? us : 0.f, 0.1f * G, odd ? 0.1f * G : 0.f,
-                                          (float)a.M * G * 1e-6f, ragged, (float)a.KN * G * (float)patch_weight_planes(type) * 8e-6f,
-                                          one ? 1.f : 0.f, one ? us : 0.f, one && ragged_rows_cached(a.M, a.KN) ? ragged : 0.f};
-    for (int k = 0; k < kTiledFeatures; k++) f[k] = values[k];
+    const bool odd = a.PC % 2 != 0, one = a.PC == 1, pairs = a.PC % 2 == 0 && a.PC % 4 != 0 && a.G % 6 != 0;
+    const float ragged = a.KN % 32 ? y_mb : 0.f, ragged_beyond = a.KN % 32 ? beyond : 0.f;
+    const bool cached = a.M * (long)a.KN >= (6L << 20);  // (ragged_rows_cached of 33 filters and more)
+    const float uncached = cached ? 0.f : ragged;
+    const float values[22] = {1.f, us, y_mb, products, odd ? products : 0.f, odd ? us : 0.f, 0.1f * G, odd ? 0.1f * G : 0.f,
+                              (float)a.M * G * 1e-6f, ragged, (float)a.KN * G * (float)patch_weight_planes(type) * 8e-6f,
+                              one ? 1.f : 0.f, one ? us : 0.f, one && cached ? ragged : 0.f, pairs ? us : 0.f, pairs ? 0.1f * G : 0.f,
+                              beyond, ragged_beyond, one ? beyond : 0.f, one ? ragged_beyond : 0.f, uncached, uncached > 12.f && shape != 2 ? uncached - 12.f : 0.f};
+    for (int k = 0; k < 22; k++) f[k] = values[k];
+    for (int k = 22; k < kTiledFeatures; k++) f[k] = kTiledShapes[k - 22] == shape ? us : 0.f;
 }
 
 }  // namespace tab

@@ -13,12 +13,12 @@ and every shape take beyond the best of them, over the tiled kernel's time, all 
 more.  The durations themselves, with the quantizer's as a form in bytes, join in at a tenth of the weight, which gives the predictions
 their scale; they are the convolution's up to a summand that all share.
 
-The tiled kernel has become faster since for odd numbers of words a pixel; the fit takes its later times (conv_patch_tiled_timings.txt).
-
-Where conv_mfma_shape ranks 32x32 tiles first, the kernel that splits K over waves ran in their place ("tiled"): the patch was never faster.
+All times are of one build and one session.  "waves": the kernel that splits K over waves, where its rule takes the call from the tiled ones.  Where
+conv_mfma_shape ranks 32x32 tiles first there is no tiled kernel and the patch is not looked at; elsewhere the choice is between the two as
+conv_patch_plan makes it.
 
     python tab_amd/tuning/fit_conv_patch_model.py            fit on everything, write the header
-    python tab_amd/tuning/fit_conv_patch_model.py --check    fit on one half of the geometries, regret on the other
+    python tab_amd/tuning/fit_conv_patch_model.py --check    fit on two thirds of the geometries, regret on the other third
 """
 import ctypes
 import os
@@ -31,22 +31,17 @@ from scipy.optimize import nnls
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(os.path.dirname(HERE), "csrc")
 DATA = os.path.join(HERE, "conv_patch_timings.txt")
-TILED = os.path.join(HERE, "conv_patch_tiled_timings.txt")  # later times of the tiled kernel, where it has become faster
 SHAPES = {12: (256, 128, 8, 2), 13: (128, 128, 4, 3), 14: (128, 64, 2, 4), 15: (64, 64, 1, 4), 16: (256, 64, 4, 3),
           17: (64, 256, 4, 3), 18: (64, 128, 2, 4)}  # kPatchTile
 CUS, ITEMS, LDS = 256, {1: 3, 2: 3, 4: 2}, 64 * 1024
 MARGIN, MARGIN_US = 0.985, 0.1  # what the patch kernel has to be predicted below: MARGIN of the tiled kernel's duration, less MARGIN_US
-PATCH_FEATURES, TILED_FEATURES = 18, 14  # kPatchFeatures, kTiledFeatures
-ROUNDS, SLOWER = 5, 1.05
+PATCH_FEATURES, TILED_FEATURES = 21, 32  # kPatchFeatures, kTiledFeatures
+TILED_SHAPES = (0, 1, 2, 4, 5, 6, 8, 9, 10, 11)  # kTiledShapes
 BORDER, SCALE = 0.1, 0.1  # a difference of the share BORDER of a call weighs 0.7 of one that is none; a duration SCALE
 
 
-def key(r):
-    return tuple(r[k] for k in ("type", "N", "H", "W", "C", "KN", "KH", "KW", "p1", "p2", "s"))
-
-
 def parse(path):
-    rows, later = [], {} if path == TILED else {key(r): r["tiled"] for r in parse(TILED)}
+    rows = []
     pattern = re.compile(r"type (\d) N(\d+)_(\d+)x(\d+)x(\d+)->(\d+)_k(\d+)x(\d+)_p(\d+)\.(\d+)_s(\d+) \| (.*)")
     for line in open(path):
         m = pattern.match(line)
@@ -56,9 +51,9 @@ def parse(path):
             r["M"], r["PC"] = r["N"] * r["OH"] * r["OW"], (r["C"] + 63) // 64
             r["G"], r["planes"] = r["KH"] * r["KW"] * r["PC"], 2 if r["type"] in (0, 2, 4) else 1
             times = dict(t.split(":") for t in m.group(12).split())
-            r["tiled"] = float(times.pop("tiled"))
-            r["now"] = min(r["tiled"], later.get(key(r), r["tiled"]))
-            r["times"] = {int(k): float(v) for k, v in times.items()}  # (those above 1.5 times the tiled kernel's were left out)
+            r["tiled"], r["waves"] = (float(times.pop(k, "nan")) for k in ("tiled", "waves"))
+            r["without"] = r["tiled"] if np.isnan(r["waves"]) else r["waves"]  # the call without the patch kernel
+            r["times"] = {int(k): float(v) for k, v in times.items()}  # (those above 1.7 times the tiled kernel's were left out)
             rows.append(r)
     return rows
 
@@ -104,8 +99,10 @@ def patch_features(r, shape):
     patch = npix * kc * chunks * 1e-3
     weights = -(-r["KN"] // 32) * pairs * 512e-6 * r["planes"]
     ragged, uncached = r["KN"] % 32 != 0, r["M"] * r["KN"] < 6 << 20
+    beyond = max(0.0, y - 256)
     return np.array([1, busy, K * n, K * rounds, n, rounds, y, y * busy, patch * n, patch * rounds, chunks * rounds, tiles / CUS,
-                     y * ragged, weights, 0.01 * pairs, r["PC"] == 1, y * (r["PC"] == 1), y * (ragged and uncached)])
+                     y * ragged, weights, 0.01 * pairs, r["PC"] == 1, y * (r["PC"] == 1), y * (ragged and uncached), beyond, beyond * ragged,
+                     weights / max(1, tiles / CUS)])
 
 
 def tiled_prediction():
@@ -121,12 +118,21 @@ def tiled_prediction():
     return predict
 
 
-def tiled_features(r, us):
+def waves_gain(r):
+    f = ctypes.CDLL(os.path.join(os.path.dirname(HERE), "lib", "libtab_amd.so")).tab_internal_conv_waves_gain
+    f.restype = ctypes.c_float
+    return f(r["type"], r["M"], r["KN"], r["G"], r["PC"])
+
+
+def tiled_features(r, us, shape):
     y, odd, one = r["M"] * r["KN"] * 4e-6, r["PC"] % 2, r["PC"] == 1
-    ragged, cached = r["KN"] % 32 != 0, r["M"] * r["KN"] >= 6 << 20
+    ragged, cached, beyond = r["KN"] % 32 != 0, r["M"] * r["KN"] >= 6 << 20, max(0.0, y - 256)
+    pairs = r["PC"] % 4 == 2 and r["G"] % 6 != 0
     products = r["M"] * (-(-r["KN"] // 64) * 64) * r["G"] * 1e-9
     return np.array([1, us, y, products, odd * products, odd * us, 0.1 * r["G"], odd * 0.1 * r["G"], r["M"] * r["G"] * 1e-6,
-                     y * ragged, r["KN"] * r["G"] * r["planes"] * 8e-6, one, us * one, y * (one and ragged and cached)])
+                     y * ragged, r["KN"] * r["G"] * r["planes"] * 8e-6, one, us * one, y * (one and ragged and cached), us * pairs, 0.1 * r["G"] * pairs,
+                     beyond, beyond * ragged, beyond * one, beyond * (ragged and one), y * (ragged and not cached),
+                     max(0.0, y - 12) * (ragged and not cached and shape != 2)] + [us * (shape == s) for s in TILED_SHAPES])
 
 
 def quantizer_features(r):
@@ -134,29 +140,40 @@ def quantizer_features(r):
     return np.array([1, x, x * ragged, ragged, r["N"] * r["H"] * r["W"] * r["PC"] * 8e-6 * (2 if r["type"] in (0, 1, 4) else 1)])
 
 
-def fit_weighted(rows, predict, emphasis):
+def prepared(rows):
+    """The forms of every row, worked out once."""
+    predict = tiled_prediction()
+    for r in rows:
+        shape = predict(r, True)
+        r["tiled form"] = None if shape == 3 else tiled_features(r, predict(r), shape)
+        r["forms"] = {s: patch_features(r, s) for s in SHAPES}
+        r["waves gain"] = waves_gain(r)
+    return rows
+
+
+def fit(rows):
     tiled, patch = {}, {}
     at = {s: TILED_FEATURES + k * PATCH_FEATURES for k, s in enumerate(SHAPES)}
     quantizer = TILED_FEATURES + len(SHAPES) * PATCH_FEATURES
     for t in range(5):
         A, b = [], []
-        for r, emphasised in zip(rows, emphasis):
-            if r["type"] != t:
+        for r in rows:
+            if r["type"] != t or r["tiled form"] is None:
                 continue
             kernels = []  # (duration, its form)
-            for s in [None] + [s for s in SHAPES if s in r["times"] and patch_features(r, s) is not None]:
+            for s in [None] + [s for s in SHAPES if s in r["times"] and r["forms"][s] is not None]:
                 form = np.zeros(quantizer + 5)
                 if s is None:
-                    form[:TILED_FEATURES] = tiled_features(r, predict(r))
+                    form[:TILED_FEATURES] = r["tiled form"]
                 else:
-                    form[at[s]:at[s] + PATCH_FEATURES] = patch_features(r, s)
-                kernels.append((r["now"] if s is None else r["times"][s], form))
+                    form[at[s]:at[s] + PATCH_FEATURES] = r["forms"][s]
+                kernels.append((r["tiled"] if s is None else r["times"][s], form))
             best = min(range(len(kernels)), key=lambda i: kernels[i][0])
             for i, (us, form) in enumerate(kernels):
                 if i != best:
-                    difference = (us - kernels[best][0]) / r["now"]
-                    weight = (1 + (difference / BORDER) ** 2) ** -0.5 * emphasised
-                    A.append(weight * (form - kernels[best][1]) / r["now"])
+                    difference = (us - kernels[best][0]) / r["tiled"]
+                    weight = (1 + (difference / BORDER) ** 2) ** -0.5
+                    A.append(weight * (form - kernels[best][1]) / r["tiled"])
                     b.append(weight * difference)
                 whole = form.copy()
                 whole[quantizer:] = quantizer_features(r)
@@ -169,41 +186,32 @@ def fit_weighted(rows, predict, emphasis):
     return tiled, patch
 
 
-def fit(rows, predict):
-    """Calls that the choices slow down by more than SLOWER count threefold in the next of ROUNDS fits."""
-    emphasis = np.ones(len(rows))
-    for _ in range(ROUNDS):
-        fitted = fit_weighted(rows, predict, emphasis)
-        each = regret(rows, [choose(r, *fitted, predict) for r in rows], "now")[4]
-        emphasis[each > SLOWER] *= 3
-    return fitted
-
-
-def choose(r, tiled, patch, predict):
-    if predict(r, True) == 3:
+def choose(r, tiled, patch):
+    if r["tiled form"] is None or (r["G"] > 192 and -(-r["M"] // 64) * -(-r["KN"] // 64) < CUS * (1 + r["G"] / 512)):
         return None
-    limit, best = MARGIN * float(tiled[r["type"]] @ tiled_features(r, predict(r))) - MARGIN_US, None
+    call = float(tiled[r["type"]] @ r["tiled form"])
+    limit, best = MARGIN * call - MARGIN_US, None
     for s in SHAPES:
-        f = patch_features(r, s)
+        f = r["forms"][s]
         if f is not None and float(patch[r["type"], s] @ f) < limit:
             limit, best = float(patch[r["type"], s] @ f), s
-    return best
+    return best if best and r["waves gain"] <= call - limit else None
 
 
-def regret(rows, chosen, base="tiled"):
-    """(geometric mean, total) of the chosen and of the best times over the tiled ones, and every choice's over the tiled one.
-    base: the tiled kernel's times with the patch's ("tiled") or its later ones ("now")."""
-    tiled = np.array([r[base] for r in rows])
-    got = np.array([r["now"] if c is None else r["times"].get(c, 1.5 * r["now"]) for r, c in zip(rows, chosen)])
-    best = np.array([min([r["now"]] + list(r["times"].values())) for r in rows])
-    return np.exp(np.log(got / tiled).mean()), got.sum() / tiled.sum(), np.exp(np.log(best / tiled).mean()), best.sum() / tiled.sum(), got / tiled
+def regret(rows, chosen):
+    """(geometric mean, total) of the chosen and of the best times over those without the patch kernel, and every choice's."""
+    without = np.array([r["without"] for r in rows])
+    got = np.array([r["without"] if c is None else r["times"].get(c, 1.7 * r["without"]) for r, c in zip(rows, chosen)])
+    best = np.array([min([r["without"]] + list(r["times"].values())) for r in rows])
+    return np.exp(np.log(got / without).mean()), got.sum() / without.sum(), np.exp(np.log(best / without).mean()), best.sum() / without.sum(), got / without, got / best
 
 
-def stated(rows, chosen, base="tiled"):
-    geometric, total, best_geometric, best_total, each = regret(rows, chosen, base)
-    return ("chosen / tiled %.3f (geometric) %.3f (total), best %.3f %.3f; %d of %d in the patch kernel, more than 2 / 5 / 8 %% slower there "
-            "%d / %d / %d, worst %.3f" % (geometric, total, best_geometric, best_total, sum(c is not None for c in chosen), len(rows),
-                                         (each > 1.02).sum(), (each > 1.05).sum(), (each > 1.08).sum(), each.max()))
+def stated(rows, chosen):
+    geometric, total, best_geometric, best_total, each, missed = regret(rows, chosen)
+    return ("chosen / without %.4f (geometric) %.4f (total), best %.4f %.4f; %d of %d in the patch kernel, more than 2 / 5 / 8 %% slower there "
+            "%d / %d / %d, worst %.3f; more than 5 / 10 %% above the best %d / %d" % (
+                geometric, total, best_geometric, best_total, sum(c is not None for c in chosen), len(rows), (each > 1.02).sum(),
+                (each > 1.05).sum(), (each > 1.08).sum(), each.max(), (missed > 1.05).sum(), (missed > 1.1).sum()))
 
 
 def write_header(tiled, patch):
@@ -224,15 +232,12 @@ def write_header(tiled, patch):
 
 
 if __name__ == "__main__":
-    data, predicted = [r for r in parse(DATA) if eligible(r)], tiled_prediction()
+    data = prepared([r for r in parse(DATA) if eligible(r)])
     if "--check" in sys.argv:
-        half = [(7 * r["N"] + 3 * r["H"] + 5 * r["W"] + 11 * r["C"] + r["KN"]) % 2 for r in data]
-        for h in (0, 1):
-            fitted = fit([r for r, x in zip(data, half) if x != h], predicted)
-            held_out = [r for r, x in zip(data, half) if x == h]
-            print("held out:", stated(held_out, [choose(r, *fitted, predicted) for r in held_out], "now"))
+        part = [(7 * r["N"] + 3 * r["H"] + 5 * r["W"] + 11 * r["C"] + r["KN"]) % 3 for r in data]
+        fitted = [fit([r for r, x in zip(data, part) if x != h]) for h in range(3)]
+        print("held out:", stated(data, [choose(r, *fitted[h]) for r, h in zip(data, part)]))
     else:
-        fitted = fit(data, predicted)
+        fitted = fit(data)
         write_header(*fitted)
-        for base in ("tiled", "now"):
-            print(base + ":", stated(data, [choose(r, *fitted, predicted) for r in data], base))
+        print(stated(data, [choose(r, *fitted) for r in data]))

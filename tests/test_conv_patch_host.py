@@ -93,25 +93,26 @@ def test_the_front_end_asks_for_the_room_of_the_plan(lib):
 
 
 def test_the_rule_on_its_measured_calls(lib):
-    """The compiled choices (256 compute units where no device is present) against the tiled kernels' times, whole calls: the figures that
-    the rule's fit states, and none beyond."""
+    """The compiled choices (256 compute units where no device is present) against the calls without this kernel, whole calls: the script's
+    own choices, with the figures that its fit states, and none beyond."""
     spec = importlib.util.spec_from_file_location("fit", os.path.join(TUNING, "fit_conv_patch_model.py"))
     fit = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(fit)
     lib.tab_set_conv_kernel(0, -1)
     rows = [r for r in fit.parse(fit.DATA) if fit.eligible(r)]
-    assert len(rows) > 3900
+    assert len(rows) > 8100
     chosen = []
     for r in rows:
         shape, kc, npix, lds, _ = plan(lib, r["type"], r["p1"], r["p2"], r["s"], r["s"], r["N"], r["H"], r["W"], r["C"], r["KN"], r["KH"], r["KW"])
         if shape >= 0:
             assert fit.patch_features(r, shape) is not None and fit.chunk(r, shape) == (kc, npix, lds), r
         chosen.append(shape if shape >= 0 else None)
-    geometric, total, _, _, each = fit.regret(rows, chosen)
+    geometric, total, _, _, each, missed = fit.regret(rows, chosen)
     stated = fit.stated(rows, chosen)
     # (to the last digit of what the script prints: float arithmetic may turn a call or two on the border)
-    assert geometric < 0.9628 and total < 0.9447 and each.max() < 1.10, stated
-    assert (each > 1.02).sum() <= 29 and (each > 1.05).sum() <= 9 and (each > 1.08).sum() <= 3, stated
+    assert geometric < 0.9554 and total < 0.9337 and each.max() < 1.18, stated
+    assert (each > 1.02).sum() <= 118 and (each > 1.05).sum() <= 34 and (each > 1.08).sum() <= 14, stated
+    assert (missed > 1.05).sum() <= 350 and (missed > 1.1).sum() <= 91, stated
     assert len({c for c in chosen if c is not None}) == len(ROWS), stated  # every shape has launches of its own
     # launches of fewer tiles than compute units are not looked at
     assert plan(lib, 0, 1, 1, 1, 1, 16, 14, 14, 256, 256, 3, 3)[0] < 0 and plan(lib, 0, 1, 1, 1, 1, 64, 14, 14, 256, 256, 3, 3)[0] >= 0
@@ -124,7 +125,7 @@ def test_a_plan_without_its_room_leaves_the_kernel_of_calls_without_any(lib):
     planned, split = 0, 0
     for type in range(5):
         for N, H, C, KN, K in ((16, 14, 64, 512, 3), (36, 14, 256, 256, 3), (64, 14, 256, 256, 3), (64, 7, 512, 512, 3), (64, 14, 128, 320, 3),
-                               (16, 28, 128, 128, 3), (20, 20, 192, 200, 5), (64, 11, 320, 320, 3), (256, 28, 512, 512, 3), (100, 7, 256, 320, 3)):
+                               (16, 28, 128, 128, 3), (20, 20, 192, 200, 5), (64, 14, 192, 256, 3), (256, 28, 512, 512, 3), (50, 14, 192, 192, 3)):
             lib.tab_internal_conv_plan(type, K // 2, K // 2, 1, 1, N, H, H, C, KN, K, K, plan_of)
             if plan_of[0] < 0:
                 continue
