@@ -191,9 +191,10 @@ def choose(r, tiled, patch):
         return None
     call = float(tiled[r["type"]] @ r["tiled form"])
     limit, best = MARGIN * call - MARGIN_US, None
+    wide = r["KN"] > 64 and r["M"] * r["KN"] * 4e-6 > 150
     for s in SHAPES:
         f = r["forms"][s]
-        if f is not None and float(patch[r["type"], s] @ f) < limit:
+        if f is not None and not (s == 15 and wide) and float(patch[r["type"], s] @ f) < limit:
             limit, best = float(patch[r["type"], s] @ f), s
     return best if best and r["waves gain"] <= call - limit else None
 

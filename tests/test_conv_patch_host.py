@@ -110,9 +110,9 @@ def test_the_rule_on_its_measured_calls(lib):
     geometric, total, _, _, each, missed = fit.regret(rows, chosen)
     stated = fit.stated(rows, chosen)
     # (to the last digit of what the script prints: float arithmetic may turn a call or two on the border)
-    assert geometric < 0.9554 and total < 0.9337 and each.max() < 1.18, stated
-    assert (each > 1.02).sum() <= 118 and (each > 1.05).sum() <= 34 and (each > 1.08).sum() <= 14, stated
-    assert (missed > 1.05).sum() <= 350 and (missed > 1.1).sum() <= 91, stated
+    assert geometric < 0.9555 and total < 0.9340 and each.max() < 1.18, stated
+    assert (each > 1.02).sum() <= 112 and (each > 1.05).sum() <= 32 and (each > 1.08).sum() <= 14, stated
+    assert (missed > 1.05).sum() <= 357 and (missed > 1.1).sum() <= 91, stated
     assert len({c for c in chosen if c is not None}) == len(ROWS), stated  # every shape has launches of its own
     # launches of fewer tiles than compute units are not looked at
     assert plan(lib, 0, 1, 1, 1, 1, 16, 14, 14, 256, 256, 3, 3)[0] < 0 and plan(lib, 0, 1, 1, 1, 1, 64, 14, 14, 256, 256, 3, 3)[0] >= 0
