@@ -178,14 +178,22 @@ __device__ __forceinline__ void compare4(const floatx4 v, const float t, uint32_
 // MODE 5: the row is two words of 32 two-bit fields (TAB_CPU.cpp:364-379); the lane's four fields
 // (8 bits, even bit = nonzero, odd bit = sign) go to byte l%4 of the low (l%8 < 4) or high half of the
 // word lanes 0-7 (channels 0-31) or lanes 8-15 (channels 32-63) build: (word 0 low, high, word 1 low, high).
-template <int MODE>
+// MASKED: the bits have been masked, so that the compiler cannot put the compares' results in their places by itself: they are spread.
+template <int MODE, bool MASKED = false>
 __device__ __forceinline__ void pack_row(uint32_t sign, uint32_t nz, int l, uint32_t (&out)[4])
 {
     if (MODE == 5) {
         uint32_t fields = 0;
+        if (MASKED) {
+            uint32_t both = nz | sign << 16;
+            both = (both | both << 2) & 0x00330033u;
+            both = (both | both << 1) & 0x00550055u;
+            fields = both | both >> 15;
+        } else {
 #pragma unroll
-        for (int i = 0; i < 4; i++) fields |= (((nz >> i) & 1u) | (((sign >> i) & 1u) << 1)) << (2 * i);
-        const uint32_t placed = fields << (8 * (l & 3));
+            for (int i = 0; i < 4; i++) fields |= (((nz >> i) & 1u) | (((sign >> i) & 1u) << 1)) << (2 * i);
+        }
+        const uint32_t placed = (fields & 0xffu) << (8 * (l & 3));
         const uint32_t lo = or_reduce8((l & 4) ? 0u : placed), hi = or_reduce8((l & 4) ? placed : 0u);
         out[0] = lo; out[1] = hi; out[2] = rotate_row8(lo); out[3] = rotate_row8(hi);
         return;

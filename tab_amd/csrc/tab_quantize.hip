@@ -113,6 +113,8 @@ __global__ __launch_bounds__(kThreads) void quantize_rows64_weights(const floatx
 // over the pixels of a wave word after word (one plane / two, before -> now, us): C=100 2 MB 4.3 / 4.7 -> 2.4 / 2.5, 8 MB 4.6 / 5.2 -> 3.0 / 3.3, 60
 // MB 13.0 / 14.9 -> 11.3 / 12.7, 300 MB 54.6 / 57.7 -> 49.6 / 54.5 (6.0 TB/s); C=494 8 MB 7.1 / 8.4 -> 2.9 / 3.1; C=1000 2 MB 8.2 / 9.8 -> 2.4 / 2.5,
 // 300 MB 121 / 147 -> 49 / 53.  32 rows a workgroup or 128 as for whole rows (C=100, 8 MB 3.0 / 4.0, 20 MB 5.8 / 5.8, 60 MB 12.4 / 11.3).
+// Format 5 is the one bound by its instructions: with the addresses of its words from the wave's first and its fields spread two operations at a time 120 MB
+// of C=33 take 30.8 us, 36.1 without, 33.6 by tiles.
 template <int BITS, int LOADS = kLoadsPerLane, bool OWN = false>
 __global__ __launch_bounds__(kThreads) void quantize_rows_ragged(const floatx4 *__restrict__ x, const Thresholds ths, uint32_t *__restrict__ q, long rows,
                                                                  long rows_per_item, Div32 div_item, int32_t *btn, long items, const RaggedRows ragged)

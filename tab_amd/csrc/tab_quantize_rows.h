@@ -26,6 +26,7 @@ template <int LOADS>
 struct RowLoads {
     floatx4 v[LOADS];
     uint32_t exist[LOADS], pixel[LOADS];
+    bool one_word[LOADS];  // of 32 channels: the last 32 of the row do not exist
     long first_pixel;
 };
 
@@ -63,6 +64,7 @@ __device__ __forceinline__ void load_rows(const RaggedRows ragged, const floatx4
         const uint32_t row = word0 + min((uint32_t)(u * 4 + sub), live - 1), pixel = div32(row, ragged.div_pc), word = row - pixel * PC;
         const int here = (int)(C - word * 64u) - 4 * l;
         rows.pixel[u] = pixel;
+        rows.one_word[u] = C - word * 64u <= 32u;
         rows.exist[u] = here >= 4 ? 15u : here > 0 ? (1u << here) - 1u : 0u;
         const uint32_t offset = begins(pixel, word) + 16u * (uint32_t)l;
         const u32x4 w = NT ? __builtin_amdgcn_raw_buffer_load_b128(rsrc, offset, 0, kStreamingStore) : __builtin_amdgcn_raw_buffer_load_b128(rsrc, offset, 0, 0);
@@ -119,15 +121,13 @@ __device__ __forceinline__ void quantize_rows_block(const Rows kind, const float
             sign &= held.exist[u];
             nz &= held.exist[u];
         }
-        pack_row<BITS>(sign, nz, l, out);  // lane 0 stores the whole element (8 or 16 bytes) at once
+        pack_row<BITS, RAGGED>(sign, nz, l, out);  // lane 0 stores the whole element (8 or 16 bytes) at once
         if constexpr (RAGGED && BITS == 5) {
             // 32 channels a word: a row is two words, or one where the last 32 channels of the pixel do not exist
-            const uint32_t C = (uint32_t)kind.C;
-            const bool odd = (C & 63u) - 1u < 32u;  // 1 .. 32 channels in the last row
+            const bool odd = ((uint32_t)kind.C & 63u) - 1u < 32u;  // 1 .. 32 channels in the last row
+            uint32_t *const at = q + 2 * (2 * row0 - (odd ? held.first_pixel : 0)) + 2u * (2u * r - (odd ? held.pixel[u] : 0u));
             if (r < live && l == 0) {
-                const long row = row0 + r, pixel = held.first_pixel + held.pixel[u];
-                uint32_t *at = q + 2 * (2 * row - (odd ? pixel : 0));
-                if (odd && row == (pixel + 1) * (long)((C + 63u) >> 6) - 1) *reinterpret_cast<uintx2 *>(at) = uintx2{out[0], out[1]};
+                if (held.one_word[u]) *reinterpret_cast<uintx2 *>(at) = uintx2{out[0], out[1]};
                 else *reinterpret_cast<PackedPair *>(at) = PackedPair{out[0], out[1], out[2], out[3]};
             }
         } else if (BITS != 1) {
