@@ -105,12 +105,13 @@ int tab_internal_conv_shape(int type, int M, int KN, int G, int PC, int packed, 
     return tab::conv_mfma_shape(type, a, cost_us);
 }
 
-/* Test hook, absent from include/tab_amd.h: the shape of a launch of fp32 output, the one above or one (19 .. 22) of the kernel that splits K
+/* Test hook, absent from include/tab_amd.h: the shape of a launch, the one above or, of fp32 output, one (19 .. 22) of the kernel that splits K
  * over the waves of a workgroup. */
-int tab_internal_conv_launch_shape(int type, int M, int KN, int G, int PC)
+int tab_internal_conv_launch_shape(int type, int M, int KN, int G, int PC, int packed)
 {
     tab::ConvArgs a = {};
     a.M = M; a.KN = KN; a.G = G; a.PC = PC;
+    a.qy = packed ? reinterpret_cast<uint32_t *>(&a) : nullptr;  // only tested against null
     return tab::conv_fp32_shape(type, a);
 }
 

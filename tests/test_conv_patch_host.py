@@ -130,7 +130,7 @@ def test_a_plan_without_its_room_leaves_the_kernel_of_calls_without_any(lib):
             if plan_of[0] < 0:
                 continue
             PC = (C + 63) // 64
-            want = lib.tab_internal_conv_launch_shape(type, N * H * H, KN, K * K * PC, PC)
+            want = lib.tab_internal_conv_launch_shape(type, N * H * H, KN, K * K * PC, PC, 0)
             assert plan_of[4] == want, (type, N, H, C, KN, K)
             planned, split = planned + 1, split + (want >= 19)
     assert planned > 15 and split >= 2, (planned, split)

@@ -22,7 +22,7 @@ def test_choices_on_the_measured_layers():
     f = ctypes.CDLL(_capi.LIB_PATH).tab_internal_conv_launch_shape
     differ, taken, best, alone = 0, [], [], []
     for r in rows:
-        shape = f(r["type"], r["M"], r["KN"], r["G"], r["PC"])
+        shape = f(r["type"], r["M"], r["KN"], r["G"], r["PC"], 0)
         assert shape in fit.SHAPES or shape == r["shape"] != 3
         differ += (shape if shape in fit.SHAPES else "tiled") != fit.choose(r, coefficients)
         if r["tiled"] is None:
@@ -40,6 +40,9 @@ def test_packed_output_and_large_launches_stay_with_the_tiles():
     f = ctypes.CDLL(_capi.LIB_PATH).tab_internal_conv_launch_shape
     tiled = ctypes.CDLL(_capi.LIB_PATH).tab_internal_conv_shape
     for type in range(6):
-        for M, KN, G, PC in ((2**31 - 600, 1, 9, 1), (2**31 - 600, 4096, 65535, 65535), (200704, 64, 9, 1), (1, 1, 1, 1), (1, 4096, 65534, 65534)):
-            shape = f(type, M, KN, G, PC)
-            assert 0 <= shape <= 22 and (M < 1000 or shape == tiled(type, M, KN, G, PC, 0, None)), (type, M, KN, G, PC, shape)
+        for M, KN, G, PC in ((2**31 - 600, 1, 9, 1), (2**31 - 600, 4096, 65535, 65535), (200704, 64, 9, 1)):
+            assert f(type, M, KN, G, PC, 0) == tiled(type, M, KN, G, PC, 0, None), (type, M, KN, G, PC)
+        # few tiles: the split kernel for fp32 output, never for packed
+        for M, KN, G, PC in ((1, 1, 1, 1), (1, 4096, 65534, 65534), (196, 512, 72, 8), (784, 512, 72, 8)):
+            assert 19 <= f(type, M, KN, G, PC, 0) <= 22, (type, M, KN, G, PC)
+            assert f(type, M, KN, G, PC, 1) == tiled(type, M, KN, G, PC, 1, None) < 12, (type, M, KN, G, PC)

@@ -1,5 +1,5 @@
-"""The general quantizer (quantize_tile) at the edges of its tiles: lanes per word, words per pixel, pixels in parts, tiles
-that span items, views aligned to their floats only; all formats, against the oracle."""
+"""The quantizer of up to 32 channels (quantize_tile) at the edges of its tiles: lanes per word, tiles that span items, several hundred tiles, views
+aligned to their floats only; and, from 33 channels on, the rows that take the wider pixels; all formats, against the oracle."""
 import numpy as np
 import pytest
 import torch
@@ -9,11 +9,11 @@ import tab_amd
 
 pytestmark = pytest.mark.gpu
 
-# N, H, W, C: each lane count's first and last channel count, tails of one channel, 3072 and beyond (parts of 64 words), items
-# of one pixel, tensors of one read and of several hundred tiles
+# N, H, W, C: each lane count's first and last channel count, tails of one channel, items of one pixel, tensors of one read and of several hundred
+# tiles (more than 512, which keep their full size)
 CASES = [(1, 1, 1, 1), (3, 5, 7, 4), (2, 9, 9, 5), (7, 3, 3, 8), (2, 8, 8, 9), (5, 4, 4, 16), (2, 7, 7, 17), (70, 1, 1, 32),
          (3, 6, 5, 33), (2, 10, 10, 63), (130, 1, 1, 65), (2, 3, 5, 129), (3, 4, 4, 333), (5, 1, 1, 3071), (2, 1, 2, 3073),
-         (2, 1, 1, 8250), (9, 40, 41, 100)]
+         (2, 1, 1, 8250), (9, 40, 41, 100), (9, 90, 91, 27), (2, 300, 301, 13), (7, 150, 151, 4)]
 
 
 @pytest.mark.parametrize("case", CASES)
