@@ -577,16 +577,15 @@ int conv_fp32_shape(int type, const ConvArgs &a)
 
 // The kernel that keeps the input patch in LDS, against the tiled one that conv_mfma_shape picks: the shape with the lowest predicted
 // duration, if that is 1.5 % and 0.1 us below what the call through the tiled kernel is predicted to take (tab_conv_patch_model.h; both are
-// linear forms with non-negative coefficients, fitted to the whole calls of 8169 layers, a quarter of them long K on few tiles and rows of Y that
-// end inside a cache line, where a fit to 3970 had gone wrong: N=24 104x104x7->348 BNN 119 us through the tiles it chose, 78 here).  Those calls take 0.955 of
-// the time without this kernel (in total 0.934; the better one of each 0.949 and 0.927), of 2815 choices 110 are more than 2 % slower, 31 more than
-// 5 %, the worst 18 %; on thirds held out of the fit 0.956, 136, 45, 18 %; on 1499 layers measured after it 0.956 (0.960 before, best 0.949), of 499
-// choices 19 more than 2 % slower, five 5 %, the worst 10 % (33 % before), and 15 calls more than 10 % above the best kernel (37).  (Fitted to
+// linear forms with non-negative coefficients, fitted to the whole calls of 11068 layers, among them long K on few tiles, rows of Y that end inside a cache line
+// and launches of 30 to 400 us, where a fit to 3970 had gone wrong: N=24 104x104x7->348 BNN 119 us through the tiles it chose, 78 here).  Those calls take 0.944
+// of the time without this kernel (in total 0.914; the better one of each 0.937 and 0.907; the earlier fit 0.949, 0.921); of 4459 choices 149 are more than 2 % slower,
+// 34 more than 5 %, the worst 18 % (61 %), and 113 calls are more than 10 % above the best kernel (341).  On thirds held out of the fit 0.944, 164, 47, 18 %, 124;
+// on 1500 layers measured after it 0.938 (the earlier fit 0.940, best 0.922), of 644 choices 18 more than 2 % slower, six 5 %, the worst 10 %.  (Fitted to
 // convolutions replayed on the same operands, weights in the L2s, a tenth of such layers were more than 5 % slower, the worst 1.6 times.)
-// Where the tiled kernel's place is the split-K kernel's (conv_waves_or), the patch is taken if it is predicted to gain as much: of 995 such layers
-// it is in 52, 0.999 of the split-K kernel's time, the better one of each 0.997.
-// Long K on few tiles, more than 192 words on less than 1.4 to 2 tiles of 64x64 a CU, stays with the others: the weights come from behind the L2s once, and
-// nothing hides them (N=4 54x64x888->128 7x7 TBN 73 us in tile 8, 114 here).
+// Where the tiled kernel's place is the split-K kernel's (conv_waves_or), the patch is taken if it is predicted to gain as much.
+// Long K on few tiles, more than 192 words for more than 256 filters or more than 448 on less than 1.4 to 2 tiles of 64x64 a CU, stays with the others: the
+// weights come from behind the L2s once, and nothing hides them (N=4 54x64x888->128 7x7 TBN 73 us in tile 8, 114 here).
 // Nor does more than 150 MB of Y in rows of more than 64 filters go by 64x64 tiles, which write 256 bytes of a row at a time: timed between other kernels
 // they are as soon as the others, call after call they are not (N=172 30x32x64->512 BNN 69 us, 64x128 tiles 67; N=72 54x35x64->448 BTN 54.4, 128x64 45.8).
 // Not for 1x1 kernels, which read every pixel for one tap only, nor for at most 32 filters, half of whose tiles would be work for nothing,
@@ -632,7 +631,7 @@ PatchPlan conv_patch_plan(int type, const ConvArgs &a)
     float waves_gain_us = 0.f;
     const int tiled = plan.tiled;
     plan.tiled = conv_waves_or(type, a, tiled, tiled_us, &waves_gain_us);  // (also where the weights then find no room)
-    if (a.G > 192 && ((long)a.M + 63) / 64 * kn64 * 512 < cus * (512 + a.G)) return plan;
+    if (a.G > 192 && (a.KN > 256 || a.G > 448) && ((long)a.M + 63) / 64 * kn64 * 512 < cus * (512 + a.G)) return plan;
     float t[kTiledFeatures];
     tiled_features(a, type, tiled, tiled_us, t);
     float limit = 0.f;

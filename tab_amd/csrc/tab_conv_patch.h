@@ -79,10 +79,11 @@ constexpr PatchTwins patch_twins()
 constexpr PatchTwins kPatchTwins = patch_twins();
 
 // What the predicted durations (tab_conv_patch_model.h) are linear in; the fit script states the same.
-constexpr int kPatchFeatures = 21, kTiledFeatures = 32;
+constexpr int kPatchFeatures = 26, kTiledFeatures = 32;
 constexpr int kPatchColumns = 8;  // kPatchShapes and a spare one: two vectors of four
 
-// A call through shape i: the busiest CU holds n tiles in so many rounds; its loop, its patches, its chunks and its output.  Then what the
+// A call through shape i: the busiest CU holds n tiles in so many rounds, the mean one its load of them; its loop, its patches, its chunks and its output, the
+// activation read by every tile of filters, the weights by every tile of rows.  Then what the
 // convolution replayed on the same operands does not show: laying out the weights, and fetching them where they are in no L2 yet, pair
 // after pair of words (N=64 7x7x512->512 TNN, 36 pairs: 11.0 us replayed, 15.1 behind its quantizer).  One word a pixel leaves little
 // but output; and rows of Y that end inside a cache line are written in parts until they go through the caches.
@@ -92,27 +93,32 @@ struct PatchCall {
     uint32_t M, KN, cus;
     float y_mb, ragged, one, one_y_mb, ragged_uncached, beyond, ragged_beyond;
     float weights_mb;  // of a pair of words
+    float x_mb;        // the packed activation
 };
 inline float y_beyond_mb(float y_mb) { return y_mb > 256.f ? y_mb - 256.f : 0.f; }
 inline PatchCall patch_call(const ConvArgs &a, int type, uint32_t cus)
 {
     const float y_mb = (float)a.M * (float)a.KN * 4e-6f, ragged = a.KN % 32 ? y_mb : 0.f, beyond = y_beyond_mb(y_mb);
     return PatchCall{(uint32_t)a.M, (uint32_t)a.KN, cus, y_mb, ragged, a.PC == 1 ? 1.f : 0.f, a.PC == 1 ? y_mb : 0.f,
-                     ragged_rows_cached(a.M, a.KN) ? 0.f : ragged, beyond, a.KN % 32 ? beyond : 0.f, (float)((a.KN + 31) / 32) * (patch_weight_planes(type) == 2 ? 1024e-6f : 512e-6f)};
+                     ragged_rows_cached(a.M, a.KN) ? 0.f : ragged, beyond, a.KN % 32 ? beyond : 0.f, (float)((a.KN + 31) / 32) * (patch_weight_planes(type) == 2 ? 1024e-6f : 512e-6f),
+                     (float)((long)a.N * a.H * a.W) * (float)a.PC * (type == 0 || type == 1 || type == 4 ? 16e-6f : 8e-6f)};
 }
 // The durations in the shapes whose patch fits (kc > 0); infinity in the others.  Column by column: the sums of all shapes go on at once.
 inline void patch_durations(const PatchCall &c, const PatchFit (&fits)[kPatchShapes], const float (&cost)[kPatchFeatures][kPatchColumns],
                             float (&us)[kPatchColumns])
 {
-    float n[kPatchColumns], rounds[kPatchColumns], all[kPatchColumns], chunks[kPatchColumns], pairs[kPatchColumns], words[kPatchColumns];
-    n[kPatchShapes] = rounds[kPatchShapes] = all[kPatchShapes] = chunks[kPatchShapes] = pairs[kPatchShapes] = words[kPatchShapes] = 0.f;
+    float n[kPatchColumns], rounds[kPatchColumns], all[kPatchColumns], chunks[kPatchColumns], pairs[kPatchColumns], words[kPatchColumns], down[kPatchColumns], across[kPatchColumns];
+    n[kPatchShapes] = rounds[kPatchShapes] = all[kPatchShapes] = chunks[kPatchShapes] = pairs[kPatchShapes] = words[kPatchShapes] = down[kPatchShapes] = across[kPatchShapes] = 0.f;
     us[kPatchShapes] = 0.f;
 #pragma unroll
     for (int i = 0; i < kPatchShapes; i++) {
         const PatchTile &tile = kPatchTile[i];
         const PatchFit &fit = fits[i];
         // M is below 2^31 and a filter's row of Y below 16 MB: fewer than 2^41 tiles
-        const uint64_t tiles = (uint64_t)((c.M + (uint32_t)tile.rows - 1) / (uint32_t)tile.rows) * ((c.KN + (uint32_t)tile.filters - 1) / (uint32_t)tile.filters);
+        const uint32_t row_tiles = (c.M + (uint32_t)tile.rows - 1) / (uint32_t)tile.rows, filter_tiles = (c.KN + (uint32_t)tile.filters - 1) / (uint32_t)tile.filters;
+        const uint64_t tiles = (uint64_t)row_tiles * filter_tiles;
+        down[i] = (float)row_tiles;
+        across[i] = (float)filter_tiles;
         const uint64_t busiest = tiles < 1u << 31 ? ((uint32_t)tiles + c.cus - 1) / c.cus : (tiles + c.cus - 1) / c.cus;
         const int held = tile.held < fit.by_lds ? tile.held : fit.by_lds;
         n[i] = (float)busiest;
@@ -134,7 +140,9 @@ inline void patch_durations(const PatchCall &c, const PatchFit (&fits)[kPatchSha
                          (of(6) * c.y_mb + of(7) * (c.y_mb * busy) + of(8) * (patch * vn) + of(9) * (patch * vrounds) + of(10) * (vchunks * vrounds) + of(11) * load) +
                          (of(12) * c.ragged + of(13) * (c.weights_mb * vpairs) + of(14) * (0.01f * vpairs) + of(15) * c.one + of(16) * c.one_y_mb +
                           of(17) * c.ragged_uncached) +
-                         (of(18) * c.beyond + of(19) * c.ragged_beyond + of(20) * (c.weights_mb * vpairs / __builtin_elementwise_max(load, Four{1.f, 1.f, 1.f, 1.f})));
+                         (of(18) * c.beyond + of(19) * c.ragged_beyond + of(20) * (c.weights_mb * vpairs / __builtin_elementwise_max(load, Four{1.f, 1.f, 1.f, 1.f}))) +
+                         (of(21) * (K * load) + of(22) * (patch * load) + of(23) * (vchunks * load) + of(24) * (c.x_mb * four(across)) +
+                          of(25) * (0.01f * c.weights_mb * vpairs * four(down)));
         for (int j = 0; j < 4; j++) us[i + j] += sum[j];
     }
 }

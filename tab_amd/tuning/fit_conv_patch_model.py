@@ -13,7 +13,7 @@ and every shape take beyond the best of them, over the tiled kernel's time, all 
 more.  The durations themselves, with the quantizer's as a form in bytes, join in at a tenth of the weight, which gives the predictions
 their scale; they are the convolution's up to a summand that all share.
 
-All times are of one build and one session.  "waves": the kernel that splits K over waves, where its rule takes the call from the tiled ones.  Where
+All times are of one session.  "waves": the kernel that splits K over waves, where its rule takes the call from the tiled ones.  Where
 conv_mfma_shape ranks 32x32 tiles first there is no tiled kernel and the patch is not looked at; elsewhere the choice is between the two as
 conv_patch_plan makes it.
 
@@ -35,7 +35,7 @@ SHAPES = {12: (256, 128, 8, 2), 13: (128, 128, 4, 3), 14: (128, 64, 2, 4), 15: (
           17: (64, 256, 4, 3), 18: (64, 128, 2, 4)}  # kPatchTile
 CUS, ITEMS, LDS = 256, {1: 3, 2: 3, 4: 2}, 64 * 1024
 MARGIN, MARGIN_US = 0.985, 0.1  # what the patch kernel has to be predicted below: MARGIN of the tiled kernel's duration, less MARGIN_US
-PATCH_FEATURES, TILED_FEATURES = 21, 32  # kPatchFeatures, kTiledFeatures
+PATCH_FEATURES, TILED_FEATURES = 26, 32  # kPatchFeatures, kTiledFeatures
 TILED_SHAPES = (0, 1, 2, 4, 5, 6, 8, 9, 10, 11)  # kTiledShapes
 BORDER, SCALE = 0.1, 0.1  # a difference of the share BORDER of a call weighs 0.7 of one that is none; a duration SCALE
 
@@ -89,10 +89,12 @@ def patch_features(r, shape):
         return None
     kc, npix, lds = got
     rows, filters, _, held = SHAPES[shape]
+    x = r["N"] * r["H"] * r["W"] * r["PC"] * (16e-6 if r["type"] in (0, 1, 4) else 8e-6)
     taps, chunks = r["KH"] * r["KW"], -(-r["PC"] // kc)
     pairs = chunks * ((taps + 1) // 2 if kc == 1 else taps * kc // 2)
     K = 2 * pairs
-    tiles = -(-r["M"] // rows) * -(-r["KN"] // filters)
+    down, across = -(-r["M"] // rows), -(-r["KN"] // filters)
+    tiles, load = down * across, down * across / CUS
     held = min(held, 160 * 1024 // lds)
     n = -(-tiles // CUS)
     rounds, busy, y = -(-n // held), min(1.0, tiles / CUS), r["M"] * r["KN"] * 4e-6
@@ -102,7 +104,7 @@ def patch_features(r, shape):
     beyond = max(0.0, y - 256)
     return np.array([1, busy, K * n, K * rounds, n, rounds, y, y * busy, patch * n, patch * rounds, chunks * rounds, tiles / CUS,
                      y * ragged, weights, 0.01 * pairs, r["PC"] == 1, y * (r["PC"] == 1), y * (ragged and uncached), beyond, beyond * ragged,
-                     weights / max(1, tiles / CUS)])
+                     weights / max(1, load), K * load, patch * load, chunks * load, x * across, 0.01 * weights * down])
 
 
 def tiled_prediction():
@@ -187,7 +189,8 @@ def fit(rows):
 
 
 def choose(r, tiled, patch):
-    if r["tiled form"] is None or (r["G"] > 192 and -(-r["M"] // 64) * -(-r["KN"] // 64) < CUS * (1 + r["G"] / 512)):
+    tiles = -(-r["M"] // 64) * -(-r["KN"] // 64)
+    if r["tiled form"] is None or (r["G"] > 192 and (r["KN"] > 256 or r["G"] > 448) and tiles < CUS * (1 + r["G"] / 512)):
         return None
     call = float(tiled[r["type"]] @ r["tiled form"])
     limit, best = MARGIN * call - MARGIN_US, None

@@ -3,6 +3,7 @@
 measured launches, is within what its comment states."""
 import ctypes
 import importlib.util
+import itertools
 import os
 import random
 
@@ -100,7 +101,7 @@ def test_the_rule_on_its_measured_calls(lib):
     spec.loader.exec_module(fit)
     lib.tab_set_conv_kernel(0, -1)
     rows = [r for r in fit.parse(fit.DATA) if fit.eligible(r)]
-    assert len(rows) > 8100
+    assert len(rows) > 11000
     chosen = []
     for r in rows:
         shape, kc, npix, lds, _ = plan(lib, r["type"], r["p1"], r["p2"], r["s"], r["s"], r["N"], r["H"], r["W"], r["C"], r["KN"], r["KH"], r["KW"])
@@ -110,9 +111,9 @@ def test_the_rule_on_its_measured_calls(lib):
     geometric, total, _, _, each, missed = fit.regret(rows, chosen)
     stated = fit.stated(rows, chosen)
     # (to the last digit of what the script prints: float arithmetic may turn a call or two on the border)
-    assert geometric < 0.9555 and total < 0.9340 and each.max() < 1.18, stated
-    assert (each > 1.02).sum() <= 112 and (each > 1.05).sum() <= 32 and (each > 1.08).sum() <= 14, stated
-    assert (missed > 1.05).sum() <= 357 and (missed > 1.1).sum() <= 91, stated
+    assert geometric < 0.9438 and total < 0.9140 and each.max() < 1.18, stated
+    assert (each > 1.02).sum() <= 151 and (each > 1.05).sum() <= 35 and (each > 1.08).sum() <= 18, stated
+    assert (missed > 1.05).sum() <= 483 and (missed > 1.1).sum() <= 114, stated
     assert len({c for c in chosen if c is not None}) == len(ROWS), stated  # every shape has launches of its own
     # launches of fewer tiles than compute units are not looked at
     assert plan(lib, 0, 1, 1, 1, 1, 16, 14, 14, 256, 256, 3, 3)[0] < 0 and plan(lib, 0, 1, 1, 1, 1, 64, 14, 14, 256, 256, 3, 3)[0] >= 0
@@ -124,8 +125,7 @@ def test_a_plan_without_its_room_leaves_the_kernel_of_calls_without_any(lib):
     lib.tab_internal_conv_plan.restype, plan_of = ctypes.c_size_t, (ctypes.c_int * 16)()
     planned, split = 0, 0
     for type in range(5):
-        for N, H, C, KN, K in ((16, 14, 64, 512, 3), (36, 14, 256, 256, 3), (64, 14, 256, 256, 3), (64, 7, 512, 512, 3), (64, 14, 128, 320, 3),
-                               (16, 28, 128, 128, 3), (20, 20, 192, 200, 5), (64, 14, 192, 256, 3), (256, 28, 512, 512, 3), (50, 14, 192, 192, 3)):
+        for N, H, C, KN, K in itertools.product((12, 20, 28, 36, 50, 64, 100, 256), (9, 11, 14, 18, 20, 28), (64, 128, 192, 320, 512), (64, 128, 192, 256, 320, 512), (3, 5)):
             lib.tab_internal_conv_plan(type, K // 2, K // 2, 1, 1, N, H, H, C, KN, K, K, plan_of)
             if plan_of[0] < 0:
                 continue
@@ -133,4 +133,4 @@ def test_a_plan_without_its_room_leaves_the_kernel_of_calls_without_any(lib):
             want = lib.tab_internal_conv_launch_shape(type, N * H * H, KN, K * K * PC, PC, 0)
             assert plan_of[4] == want, (type, N, H, C, KN, K)
             planned, split = planned + 1, split + (want >= 19)
-    assert planned > 15 and split >= 2, (planned, split)
+    assert planned > 1000 and split >= 20, (planned, split)
