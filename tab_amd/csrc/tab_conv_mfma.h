@@ -250,7 +250,8 @@ __device__ __forceinline__ void conv_mfma_epilogue(const ConvArgs &p, f32x16 (&a
 // The signs of a lane's 16 values of a tile, value 4j+i as bit 8j+i: the bits move in from the right, one instruction each.  With the
 // difference to the threshold that makes two a value, where comparing, selecting the bit and adding it (and BNN's bias) made four; packed
 // layers of short K are bound by such instructions: us, N=64 56x56x64->64 BNN 9.55 / 8.89, N=31 97x82x64->128 TBN 19.7 / 17.2, N=1 512->1024
-// 15x15 6.82 / 6.65; of 60 layers none slower (BNN of nine words in conv_mfma_regs, which keeps the comparisons, aside).
+// 15x15 6.82 / 6.65.  Of 20 layers in every shape and type none of four and more words is slower; of one word, one plane and 64x64 tiles, which the library
+// takes for types 4 and 5 only, N=256 56x56x64->64 18.7 / 20.6.  The kernel with the weights in registers: tab_conv_mfma_regs.h.
 template <class F>
 __device__ __forceinline__ uint32_t sign_bits(F value)
 {

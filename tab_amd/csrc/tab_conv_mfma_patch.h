@@ -44,7 +44,8 @@ __device__ __forceinline__ Item<PL> load_item_at(__amdgpu_buffer_rsrc_t rsrc, ui
     return it;
 }
 
-// Workgroups of the first round, four a CU; those behind them find the weights in the L2.
+// Workgroups of the first round, four a CU of 256; those behind them find the weights in the L2.  On a part of the chip with fewer CUs more than the
+// first round ask for lines, which are then at hand: a hint, on which no result depends.
 constexpr uint32_t kFirstWorkgroups = 1024;
 
 // ConvParams with other contents where this kernel has no use for the usual ones: G = pixels of the patch (the stride between

@@ -470,7 +470,8 @@ struct PixelRun {
 // to fill the chip waited for, and two loads in three were short of the parallelism a large one needs: N=32 64 x 56 x 56
 // (two planes) 6.1 -> 4.4 us, N=128 64 x 112 x 112 79.9 -> 72.4 (6.0 TB/s), N=64 3 x 112 x 112 16.6 -> 6.7.
 // grid = ceil(runs / (64 * 4 / SPLIT)) * PC workgroups, the word index fastest: the workgroups that write the PC words of the
-// same pixels run side by side, so their 8- or 16-byte stores meet in L2 as whole lines.
+// same pixels run side by side, so their 8- or 16-byte stores meet in L2 as whole lines.  Where last words have waves of their own (LAST), plane_units
+// units in the order of plane_unit: those of four or two groups of runs, word after word, then one for the last words of all of these groups.
 // The lane's nonzero values are counted for COUNT (see Counts).
 template <int BITS, int VEC, int SPLIT, bool NT, bool COUNT = false>
 __device__ __forceinline__ int quantize_nchw_unit(const float *__restrict__ x, const Thresholds &ths, uint64_t *__restrict__ q, const PixelRun<VEC> &run,
@@ -643,7 +644,7 @@ __global__ __launch_bounds__(kThreads) void quantize_nchw_weights(const float *_
     quantize_nchw_block<BITS, VEC, SPLIT, NT, LAST>(x, ths, q, N, C, HW, PC, by_image, in_eighths(block, ths.eighth), nullptr);
 }
 
-// The same with counts: a unit is 64 * 4 / SPLIT runs and one word.
+// The same with counts: a unit is what plane_unit gives a workgroup, 64 * 4 / SPLIT runs and one word, or the last words of several groups of runs.
 template <int VEC, int SPLIT, bool NT = false, bool LAST = false>
 __global__ __launch_bounds__(kThreads) void quantize_nchw_count(const float *__restrict__ x, const Thresholds ths, uint64_t *__restrict__ q, int C,
                                                                 long HW, int PC, int units, const Counts counts)
