@@ -115,6 +115,14 @@ int tab_internal_conv_launch_shape(int type, int M, int KN, int G, int PC, int p
     return tab::conv_fp32_shape(type, a);
 }
 
+/* Test hook, absent from include/tab_amd.h: the shape (19 .. 22) of the kernel that splits K over waves for a launch that is to go there. */
+int tab_internal_conv_waves_shape(int type, int M, int KN, int G, int PC)
+{
+    tab::ConvArgs a = {};
+    a.M = M; a.KN = KN; a.G = G; a.PC = PC;
+    return tab::conv_waves_shape(type, a, nullptr);
+}
+
 /* Test hook, absent from include/tab_amd.h: what the kernel that splits K over waves is predicted to gain over the tiled ones, in microseconds;
  * infinity where those of 32x32 rank first, -infinity where it is not taken. */
 float tab_internal_conv_waves_gain(int type, int M, int KN, int G, int PC)

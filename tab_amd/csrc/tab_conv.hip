@@ -530,6 +530,7 @@ int conv_waves_shape(int type, const ConvArgs &a, float *cost_us)
                                          rounds, y_mb, weights_mb, n * lines};
         float us = 0.f;
         for (int k = 0; k < kWavesFeatures; k++) us += kWavesCost[type][i][k] * f[k];
+        if (tiles * (uint64_t)(64 * tile.waves) > 0xffffffffull) us = INFINITY;  // the threads a launch may have
         if (i == 0 || us < best_us) {
             best = i;
             best_us = us;

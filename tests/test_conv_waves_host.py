@@ -46,3 +46,14 @@ def test_packed_output_and_large_launches_stay_with_the_tiles():
         for M, KN, G, PC in ((1, 1, 1, 1), (1, 4096, 65534, 65534), (196, 512, 72, 8), (784, 512, 72, 8)):
             assert 19 <= f(type, M, KN, G, PC, 0) <= 22, (type, M, KN, G, PC)
             assert f(type, M, KN, G, PC, 1) == tiled(type, M, KN, G, PC, 1, None) < 12, (type, M, KN, G, PC)
+
+
+def test_large_launches_have_no_more_threads_than_a_launch_may():
+    """A forced tile 3 on an output of 34 GB and more: eight waves a tile of 32x32 would be 2^32 threads."""
+    f = ctypes.CDLL(_capi.LIB_PATH).tab_internal_conv_waves_shape
+    threads = {19: (32, 32, 512), 20: (32, 32, 256), 21: (64, 32, 256), 22: (32, 64, 256)}
+    for type in range(6):
+        for M in (2**23, 2**28 - 32, 2**28, 2**28 + 2**27):
+            for G, PC in ((1, 1), (9, 1), (72, 8), (575, 64), (4608, 512)):
+                rows, filters, each = threads[f(type, M, 32, G, PC)]
+                assert -(-M // rows) * -(-32 // filters) * each < 2**32, (type, M, G)
